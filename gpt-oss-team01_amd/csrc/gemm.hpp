@@ -48,6 +48,7 @@ struct GemmParams {
   int tile_block;      // grouped problems, > 1: the row tiles of a block are walked together, column
                        // tile by column tile (needs xcd_bounds); 0 or 1 = every row tile on its own
   int dense_rows;      // rows of the dense problem when tiles == nullptr
+  int max_tile_rows;   // no tile of the list has more rows (0: unknown)
   int N, K;
   int n_col_tiles;     // gemm_col_tiles(N)
   GluForm glu;         // EPI_SWIGLU
@@ -60,6 +61,12 @@ struct GemmParams {
 // (mat,row-tile) items.
 int run_gemm(const GemmParams &p, bool gather, int epi, int rows_per_tile, int max_tiles,
              hipStream_t s);
+// gemm_few.hip: tiles of at most 32 rows, one wave per 32 columns (bf16 weights; gather + SwiGLU, or no gather and
+// EPI_F32, EPI_MIXED, EPI_PARTIAL).  The rows of A lie within a 31-bit byte offset.
+int run_gemm_few(const GemmParams &p, bool gather, int epi, int max_tiles, hipStream_t s);
+inline bool gemm_few_applies(const GemmParams &p, int rows_per_tile, int max_tiles) {
+  return rows_per_tile == 32 && (p.tiles ? (long long)max_tiles * 32 : p.dense_rows) * p.K * 2 < (1ll << 31);
+}
 // gemm_dense.cpp: bf16 weights, no gather (run_gemm comes here for that form)
 int run_gemm_dense(const GemmParams &p, int epi, int rows_per_tile, int max_tiles, hipStream_t s);
 // gemm_tall.hip: tiles of 256 x 256 with both operands through LDS, for launches of thousands of rows,

@@ -85,6 +85,7 @@ int run_gemm_dense(const GemmParams &p, int epi, int rows_per_tile, int max_tile
   GPTOSS_REQUIRE(max_rows * p.N < (1ll << 32) && max_rows * p.K < (1ll << 32), GPTOSS_ERR_DIM,
                  "run_gemm: rows x columns must stay below 2^32 elements (rows<=%lld N=%d K=%d)", max_rows, p.N, p.K);
   if (rows_per_tile == 256) return run_gemm_tall(p, epi, max_tiles, max_rows, s);
+  if (epi != EPI_ARGMAX && gemm_few_applies(p, rows_per_tile, max_tiles)) return run_gemm_few(p, false, epi, max_tiles, s);
   int prc = gemm_prepare_device();
   if (prc != GPTOSS_OK) return prc;
   if (epi == EPI_F32) return dispatch_rows<EPI_F32>(p, rows_per_tile, max_tiles, s);
@@ -149,7 +150,7 @@ static GemmParams dense_params(const bf16_t *A, const bf16_t *W, const float *bi
   g.bias = bias;
   g.out = out;
   g.tiles = nullptr;
-  g.dense_rows = B;
+  g.dense_rows = g.max_tile_rows = B;
   g.N = N;
   g.K = K;
   g.n_col_tiles = gemm_col_tiles(N);

@@ -1,0 +1,227 @@
+// GEMMs of a few rows for gfx950: the same products as gemm_kernel.hpp for row tiles of at most 32 rows.
+//
+//   C[rows, N] = A[rows, K] . W[N, K]^T      rows <= 32: a decoding step of few sequences, or an expert's few tokens
+//
+// Nothing but reading W takes time here, so what counts is how many bytes of W are on their way at any moment, from how
+// many CUs.  The streaming kernels give 256 columns to a workgroup of eight waves with two 4 KB slabs of W in flight
+// each, on a grid of one workgroup per CU: one token's four experts are then 92 (first product) and 48 (second) work
+// items on 256 CUs.  Here a workgroup is 128 columns, or 32 where no tile has more than eight rows, the grid has one for
+// every work item, and a wave has eight slabs in flight (MXFP4: sixteen).  To have the registers for that, A does not
+// pass through them slab by slab: chunks of eight slabs are staged in LDS, one barrier each, and W's loads stay in
+// flight across it.  Operand roles, order of the sum over K and epilogues are those of the streaming kernels, so a row
+// has the same bits whichever kernel computes it.
+// Measured, 2880 x 2880 experts, streaming kernels -> these (us): one token, both products 36 + 32 -> 24 + 14, MXFP4
+// block 60 -> 43; a dense projection of one row 38 -> 13; 27 tokens 156 + 91 -> 157 + 81 (5.9-6.8 TB/s either way);
+// 12 tokens on MXFP4 60 + 32 -> 49 + 29.  32 columns per workgroup instead of 128: one token's block 68 -> 59, eight
+// tokens 178 -> 176.  (A read straight from memory in operand order, without LDS: one token 60, but 12 tokens on MXFP4
+// 127 instead of 99, because A is then four times the bytes of W.)
+#pragma once
+#include "gemm_kernel.hpp"
+
+namespace gptoss {
+
+// WAVES: 32-column blocks of a workgroup, one per wave; the waves share the staged rows of A, eight rows per wave.
+
+// 64-k slabs of W that a wave keeps in flight: 16 bytes per lane and k-step with bf16 weights, 16 per slab with MXFP4
+constexpr int few_ring(bool fp4) { return fp4 ? 16 : 8; }
+constexpr int FEW_CHUNK = 8;                          // slabs of A that are staged together: one barrier each
+constexpr int FEW_ROW = FEW_CHUNK * BK + 8;           // padded row of a staged chunk in bf16 elements (1040 B)
+
+typedef __amdgpu_buffer_rsrc_t few_rsrc_t;
+// cache policy of a buffer load: the non-temporal bit
+constexpr int FEW_NT = 2;
+// A's buffer: offsets from here on read as zeros
+constexpr uint32_t FEW_A_BYTES = 0x80000000u;
+
+__device__ __forceinline__ few_rsrc_t few_buffer(const void *base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);
+}
+
+template <int WAVES, bool GATHER, int EPI, bool FP4, bool ONCE>
+__device__ __forceinline__ void few_block(const GemmParams &p, bf16_t *lds, int mat, int row0, int rows, int cb, int slab0,
+                                          int nslab, void *out) {
+  constexpr int RING = few_ring(FP4);
+  constexpr int ROWS = WAVES * 8;   // rows of A that are staged
+  constexpr int WQ = FP4 ? 1 : 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int K = p.K, N = p.N, kslab = K / BK;
+  const bool live = cb * 32 < N;   // the last workgroup of a row tile may have waves to spare
+
+  // W: the block's slabs lie one behind the other.  Slabs past the end are requested all the same (every load of the
+  // loop is unconditional) and read as zeros without touching memory: they lie outside the buffer.  (The part of an
+  // offset that is checked against the buffer's size is the one in the vector register, so the slab goes there.)
+  const size_t mat_bytes = FP4 ? (size_t)N * K / 2 + (size_t)N * K / 32 : (size_t)N * K * 2;
+  const char *mb = reinterpret_cast<const char *>(p.W) + (size_t)mat * mat_bytes;
+  constexpr int SLAB = FP4 ? 1024 : 4096;
+  const few_rsrc_t wb = few_buffer(mb + ((size_t)cb * kslab + slab0) * SLAB, live ? nslab * SLAB : 0);
+  const few_rsrc_t sb = few_buffer(FP4 ? mb + (size_t)N * K / 2 + ((size_t)cb * kslab + slab0) * 64 : mb,   // MXFP4 scales
+                                   FP4 && live ? nslab * 64 : 0);
+  u32x4 w[RING][WQ];
+  uint32_t sc[RING];
+  auto load_w = [&](int s, auto r) {
+    constexpr int R = decltype(r)::value;
+#pragma unroll
+    for (int q = 0; q < WQ; q++)
+      w[R][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wb, lane * 16 + s * SLAB + q * 1024, 0, ONCE ? FEW_NT : 0));
+    if constexpr (FP4) sc[R] = __builtin_amdgcn_raw_buffer_load_b16(sb, (lane & 31) * 2 + s * 64, 0, ONCE ? FEW_NT : 0);
+  };
+  // which rows of A the tile's rows are: before W, because loads return in order
+  int id = row0 + min(lane & 31, rows - 1);
+  if (GATHER) id = p.row_ids[id];
+  static_for<0, RING>([&](auto r) { load_w(decltype(r)::value, r); });
+  const few_rsrc_t bb = few_buffer(p.bias && live ? p.bias + (size_t)mat * N + cb * 32 : nullptr, p.bias && live ? 128 : 0);
+  const int bias = __builtin_amdgcn_raw_buffer_load_b32(bb, (lane & 31) * 4, 0, 0);
+
+  // A: the workgroup copies chunks of ROWS rows x FEW_CHUNK slabs, a wave one row (1 KB) per load.  Rows beyond the
+  // tile's and k beyond K are zeros, again from outside the buffer.
+  const few_rsrc_t ab = few_buffer(p.A + (size_t)slab0 * BK, FEW_A_BYTES);
+  if (GATHER) id = (uint32_t)id / (uint32_t)p.top_k;
+  uint32_t a_off[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const int r = wave + WAVES * i;
+    a_off[i] = r < rows ? (uint32_t)__builtin_amdgcn_readlane(id, r) * (uint32_t)K * 2u : FEW_A_BYTES;
+  }
+  u32x4 areg[8];
+  auto load_a = [&](int c) {
+    const int k = c * (FEW_CHUNK * BK) + lane * 8;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      areg[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ab, k < nslab * BK ? a_off[i] + k * 2 : FEW_A_BYTES, 0, 0));
+  };
+  auto store_a = [&](int c) {
+    bf16_t *d = lds + (c & 1) * (ROWS * FEW_ROW) + wave * FEW_ROW + lane * 8;
+#pragma unroll
+    for (int i = 0; i < 8; i++) *reinterpret_cast<u32x4 *>(d + WAVES * i * FEW_ROW) = areg[i];
+  };
+  load_a(0);
+  store_a(0);
+  __syncthreads();
+
+  f32x16 acc[1];
+#pragma unroll
+  for (int i = 0; i < 16; i++) acc[0][i] = 0.f;
+  const bf16_t *a_src = lds + min(lane & 31, ROWS - 1) * FEW_ROW + (lane >> 5) * 8;
+  bf16x8 af[2][4];   // a slab's operands are read while the slab before is multiplied
+  auto read_a = [&](int c, auto rr) {
+    constexpr int R = decltype(rr)::value;
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++)
+      af[R & 1][kk] = as_bf16x8(*reinterpret_cast<const u32x4 *>(a_src + (c & 1) * (ROWS * FEW_ROW) + R % FEW_CHUNK * BK + kk * 16));
+  };
+  read_a(0, std::integral_constant<int, 0>{});
+  for (int s = 0; s < nslab; s += RING)
+    static_for<0, RING>([&](auto rr) {
+      constexpr int R = decltype(rr)::value;
+      const int c = (s + R) / FEW_CHUNK;
+      if constexpr (R % FEW_CHUNK == 0) load_a(c + 1);
+      if constexpr (R % FEW_CHUNK != FEW_CHUNK - 1) read_a(c, std::integral_constant<int, R + 1>{});
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++) {
+        bf16x8 b;
+        if constexpr (FP4) b = as_bf16x8(fp4_expand(w[R][0][kk], fp4_scale((sc[R] >> (8 * (kk >> 1))) & 0xffu)));
+        else b = as_bf16x8(w[R][kk % WQ]);
+        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, af[R & 1][kk], acc[0], 0, 0, 0);
+      }
+      load_w(s + R + RING, rr);
+      __builtin_amdgcn_sched_barrier(0);   // the order of the loads is the order of their uses
+      if constexpr (R % FEW_CHUNK == FEW_CHUNK - 1) {
+        store_a(c + 1);
+        __syncthreads();
+        read_a(c + 1, std::integral_constant<int, (R + 1) % RING>{});
+      }
+    });
+  if (!live) return;
+  auto bias_of = [&](int j) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(bias, j)); };
+  if constexpr (EPI == EPI_PARTIAL) {
+    GemmParams q = p;
+    q.out = out;
+    epilogue_rows<1, EPI_F32>(q, row0, rows, cb * 32, lane, acc, bias_of);
+  } else {
+    epilogue_rows<1, EPI>(p, row0, rows, cb * 32, lane, acc, bias_of);
+  }
+}
+
+// Work items are (row tile, 32-column block) pairs; every XCD has a contiguous part of them, so that the row tiles of
+// one expert, which multiply the same blocks of W one after the other, find them in that XCD's L2.
+template <int WAVES, bool GATHER, int EPI, bool FP4>
+__global__ __launch_bounds__(WAVES * 64, 2) void few_gemm_kernel(GemmParams p) {
+  __shared__ __attribute__((aligned(16))) bf16_t lds[2 * WAVES * 8 * FEW_ROW];
+  const const_as<int> tiles = constant_ptr(p.tiles);
+  const int n_tiles = p.tiles ? tiles[0] : (p.dense_rows + 31) / 32;
+  const int n_blk = (p.N / 32 + WAVES - 1) / WAVES;
+  const int tile_items = n_tiles * n_blk;
+  const int total = EPI == EPI_PARTIAL ? tile_items * p.k_splits : tile_items;
+  const int chunk = (total + 7) >> 3;
+  const int j = blockIdx.x >> 3;
+  int work = (blockIdx.x & 7) * chunk + j;
+  if (j >= chunk || work >= total) return;
+  int part = 0;
+  if (EPI == EPI_PARTIAL) {
+    part = work / tile_items;
+    work -= part * tile_items;
+  }
+  int tile, cb, mat = 0, row0, rows;
+  bool once;
+  if (p.tiles) {
+    if (p.xcd_bounds) {   // the tiles of an expert's block are walked column block by column block
+      const int info = constant_ptr(p.xcd_bounds)[XCD_BOUNDS_INTS + work / n_blk];
+      const int first = info >> 8, th = info & 255;
+      const int v = work - first * n_blk;
+      cb = v / th;
+      tile = first + (v - cb * th);
+      once = th == 1;
+    } else {
+      tile = work / n_blk;
+      cb = work - tile * n_blk;
+      once = false;
+    }
+    mat = tiles[1 + 3 * tile];
+    row0 = tiles[2 + 3 * tile];
+    rows = tiles[3 + 3 * tile];
+  } else {
+    cb = work / n_tiles;
+    tile = work - cb * n_tiles;
+    row0 = tile * 32;
+    rows = min(32, p.dense_rows - row0);
+    once = n_tiles == 1;
+  }
+  int slab0 = 0, nslab = p.K / BK;
+  void *out = p.out;
+  if (EPI == EPI_PARTIAL) {
+    slab0 = part * p.split_slabs;
+    nslab = min(p.split_slabs, nslab - slab0);
+    out = reinterpret_cast<float *>(p.out) + (size_t)part * p.dense_rows * p.N;
+  }
+  // wave-uniform, and known to be: buffer resources live in scalar registers
+  mat = __builtin_amdgcn_readfirstlane(mat);
+  cb = __builtin_amdgcn_readfirstlane(cb * WAVES + (threadIdx.x >> 6));
+  row0 = __builtin_amdgcn_readfirstlane(row0), rows = __builtin_amdgcn_readfirstlane(rows);
+  slab0 = __builtin_amdgcn_readfirstlane(slab0), nslab = __builtin_amdgcn_readfirstlane(nslab);
+  if (once) few_block<WAVES, GATHER, EPI, FP4, true>(p, lds, mat, row0, rows, cb, slab0, nslab, out);
+  else few_block<WAVES, GATHER, EPI, FP4, false>(p, lds, mat, row0, rows, cb, slab0, nslab, out);
+}
+
+template <int WAVES, bool GATHER, int EPI, bool FP4>
+int launch_few_waves(const GemmParams &p, int max_tiles, hipStream_t s) {
+  const long long total = (long long)max_tiles * cdiv(p.N / 32, WAVES) * (EPI == EPI_PARTIAL ? p.k_splits : 1);
+  if (total == 0) return GPTOSS_OK;
+  {
+    TraceScope ts(FP4 ? (GATHER ? "gemm1_gather_swiglu_mxfp4" : "gemm_f32_mxfp4")
+                      : (GATHER ? "gemm1_gather_swiglu" : "gemm_f32"), s);
+    few_gemm_kernel<WAVES, GATHER, EPI, FP4><<<(unsigned)(((total + 7) / 8) * 8), WAVES * 64, 0, s>>>(p);
+  }
+  GPTOSS_LAUNCH_CHECK("few_gemm_kernel");
+  return GPTOSS_OK;
+}
+
+// Up to eight rows per tile one wave can stage them by itself, and the launch has four times as many workgroups to fill
+// the chip with; beyond that the rows are shared by four waves.
+template <bool GATHER, int EPI, bool FP4>
+int launch_few_gemm(const GemmParams &p, int max_tiles, hipStream_t s) {
+  if (p.max_tile_rows && p.max_tile_rows <= 8) return launch_few_waves<1, GATHER, EPI, FP4>(p, max_tiles, s);
+  return launch_few_waves<4, GATHER, EPI, FP4>(p, max_tiles, s);
+}
+
+}  // namespace gptoss

@@ -138,19 +138,18 @@ __device__ __forceinline__ void w_load(WRing<NRING, FP4> &ring, const WStream &s
 // would otherwise turn these loads into vector loads.
 // hold != nullptr (SwiGLU form only): the tile goes to LDS instead of memory, row r of the tile at
 // hold + r * HOLD_ROW, this wave's 16 outputs from column hold_col on.
-template <int MB, int EPI, bool CONST_BIAS = false>
-__device__ __forceinline__ void epilogue_store(const GemmParams &p, int mat, int row0, int rows, int n0,
-                                               int lane, const f32x16 (&acc)[MB], bf16_t *hold = nullptr,
-                                               int hold_col = 0) {
+// epilogue_rows: bias_of(c) is the bias of the block's column c, wave-uniform.
+template <int MB, int EPI, typename BIAS>
+__device__ __forceinline__ void epilogue_rows(const GemmParams &p, int row0, int rows, int n0, int lane,
+                                              const f32x16 (&acc)[MB], const BIAS &bias_of, bf16_t *hold = nullptr,
+                                              int hold_col = 0) {
   const int N = p.N;
   const int tok = lane & 31;
   const bool hi = lane >= 32;
   const int h4 = hi ? 4 : 0;
-  using BiasPtr = std::conditional_t<CONST_BIAS, const_as<float>, const float *>;
-  const BiasPtr bp = (BiasPtr)(p.bias ? p.bias + (size_t)mat * N + n0 : nullptr);
   if (EPI == EPI_SWIGLU) {
     // channels 0-15 of the wave are the gates of pairs j0..j0+15, channels 16-31 their ups; in the
-    // unpacked matrix pair j is rows 2j (gate) and 2j+1 (up), so its biases are bp[2jj], bp[2jj+1]
+    // unpacked matrix pair j is rows 2j (gate) and 2j+1 (up), so its biases are those of columns 2jj, 2jj+1
     const int half_n = N >> 1;
     float bg[8], bu[8];
 #pragma unroll
@@ -158,8 +157,8 @@ __device__ __forceinline__ void epilogue_store(const GemmParams &p, int mat, int
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         const int jlo = g * 8 + q, jhi = jlo + 4;
-        const float g_lo = bp ? bp[2 * jlo] : 0.f, g_hi = bp ? bp[2 * jhi] : 0.f;
-        const float u_lo = bp ? bp[2 * jlo + 1] : 0.f, u_hi = bp ? bp[2 * jhi + 1] : 0.f;
+        const float g_lo = bias_of(2 * jlo), g_hi = bias_of(2 * jhi);
+        const float u_lo = bias_of(2 * jlo + 1), u_hi = bias_of(2 * jhi + 1);
         bg[g * 4 + q] = hi ? g_hi : g_lo;
         bu[g * 4 + q] = hi ? u_hi : u_lo;
       }
@@ -198,7 +197,7 @@ __device__ __forceinline__ void epilogue_store(const GemmParams &p, int mat, int
     for (int g = 0; g < 4; g++)
 #pragma unroll
       for (int q = 0; q < 4; q++) {
-        const float lo = bp ? bp[g * 8 + q] : 0.f, hi_v = bp ? bp[g * 8 + 4 + q] : 0.f;
+        const float lo = bias_of(g * 8 + q), hi_v = bias_of(g * 8 + 4 + q);
         bv[g * 4 + q] = hi ? hi_v : lo;
       }
     if constexpr (EPI == EPI_MIXED) {
@@ -250,6 +249,15 @@ __device__ __forceinline__ void epilogue_store(const GemmParams &p, int mat, int
       }
     }
   }
+}
+
+template <int MB, int EPI, bool CONST_BIAS = false>
+__device__ __forceinline__ void epilogue_store(const GemmParams &p, int mat, int row0, int rows, int n0,
+                                               int lane, const f32x16 (&acc)[MB], bf16_t *hold = nullptr,
+                                               int hold_col = 0) {
+  using BiasPtr = std::conditional_t<CONST_BIAS, const_as<float>, const float *>;
+  const BiasPtr bp = (BiasPtr)(p.bias ? p.bias + (size_t)mat * p.N + n0 : nullptr);
+  epilogue_rows<MB, EPI>(p, row0, rows, n0, lane, acc, [&](int c) { return bp ? bp[c] : 0.f; }, hold, hold_col);
 }
 
 // One (row tile, column tile) work item with a compile-time number of 32-row blocks, so every

@@ -1,7 +1,7 @@
 // MXFP4-weight instantiations of the grouped GEMM kernel, and their dispatch.
 #include <mutex>
 
-#include "gemm_kernel.hpp"
+#include "gemm_few_kernel.hpp"
 
 namespace gptoss {
 GPTOSS_GEMM_EACH_TILE(GPTOSS_GEMM_INSTANTIATE, true, EPI_SWIGLU, true)
@@ -16,6 +16,7 @@ static hipError_t set_attrs() {
 
 template <bool GATHER, int EPI>
 static int dispatch_rows(const GemmParams &p, int rows_per_tile, int max_tiles, hipStream_t s) {
+  if (gemm_few_applies(p, rows_per_tile, max_tiles)) return launch_few_gemm<GATHER, EPI, true>(p, max_tiles, s);
   switch (rows_per_tile) {
     case 32: return launch_gemm<1, GATHER, EPI, true>(p, max_tiles, s);
     case 64: return launch_gemm<2, GATHER, EPI, true>(p, max_tiles, s);

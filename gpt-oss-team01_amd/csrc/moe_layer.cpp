@@ -151,7 +151,8 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
   if (!mxfp4 && (long long)B * k >= (long long)moe_tall_min_rows() * E && gemm_tall_shape_ok(2 * I, H, tall_rows) &&
       gemm_tall_shape_ok(H, I, tall_rows))
     rpt = 256;
-  const int max_tiles = gptoss_moe_max_tiles(B, k, E, rpt);
+  // (no more experts have a row than there are rows)
+  const int max_tiles = gptoss_moe_max_tiles(B, k, std::min(E, B * k), rpt);
   // Each expert's row tiles are walked in blocks of up to MOE_TILE_BLOCK, column tile by column
   // tile, so the workgroups of an XCD share a column tile of the expert's weights among the block's
   // row tiles instead of streaming it once per row tile.  With one tile per expert (a decode step
@@ -189,6 +190,7 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
   g1.tiles = ws.tiles;
   g1.tile_block = tile_block;
   g1.xcd_bounds = bounds;
+  g1.max_tile_rows = B;   // a token takes an expert once
   g1.N = 2 * I;
   g1.K = H;
   g1.n_col_tiles = gemm_col_tiles(2 * I);
@@ -206,6 +208,7 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
   g2.tiles = ws.tiles;
   g2.tile_block = tile_block;
   g2.xcd_bounds = bounds;
+  g2.max_tile_rows = B;
   g2.N = H;
   g2.K = I;
   g2.n_col_tiles = gemm_col_tiles(H);

@@ -1,0 +1,70 @@
+"""The few-row GEMM kernels (tiles of at most 32 rows): every row must have the bits that the streaming kernels give it
+in a larger batch, at the edges of row tiles, column blocks and staged chunks of K."""
+import pytest
+import torch
+
+from conftest import load_pkg
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    return load_pkg("ops")
+
+
+def _n(g, *shape, std=1.0):
+    return (torch.randn(*shape, generator=g, device="cuda") * std).to(torch.bfloat16)
+
+
+# K: one slab, one short of a chunk of eight slabs, a chunk, one more, the 20B model's; N: part of a workgroup's 128
+# columns, one workgroup and a block, the 20B model's 22.5 workgroups
+@pytest.mark.parametrize("K", [64, 448, 512, 576, 2880])
+@pytest.mark.parametrize("N", [32, 160, 2880])
+def test_dense_rows_equal_those_of_a_larger_batch(ops, K, N):
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    a, w, bias = _n(g, 150, K), ops.pack_weight(_n(g, N, K, std=0.05)), _n(g, N).float()
+    for b in (bias, None):
+        want = ops.dense_gemm(a, w, N, bias=b)     # 150 rows: the streaming kernel
+        for rows in (1, 2, 7, 8, 9, 31, 32):
+            for first in (0, 150 - rows):
+                got = ops.dense_gemm(a[first:first + rows].contiguous(), w, N, bias=b)
+                assert torch.equal(got, want[first:first + rows]), (rows, first)
+
+
+def _codes(g, *shape):
+    return torch.randint(0, 256, shape, generator=g, device="cuda", dtype=torch.uint8)
+
+
+@pytest.mark.parametrize("H,I,E,k", [(64, 64, 4, 2), (320, 576, 8, 4), (2880, 2880, 8, 4)])
+@pytest.mark.parametrize("mxfp4", [False, True])
+def test_moe_rows_equal_those_of_a_larger_batch(ops, H, I, E, k, mxfp4):
+    g = torch.Generator(device="cuda").manual_seed(H + I + mxfp4)
+    router = (_n(g, E, H, std=H ** -0.5), _n(g, E))
+    if mxfp4:
+        sc = lambda *s: (127 - torch.randint(6, 10, s, generator=g, device="cuda")).to(torch.uint8)
+        layer = ops.MoeLayerMxfp4(*router, _codes(g, E, 2 * I, H // 2), sc(E, 2 * I, H // 32), _n(g, E, 2 * I),
+                                  _codes(g, E, H, I // 2), sc(E, H, I // 32), _n(g, E, H), top_k=k, max_tokens=512)
+    else:
+        layer = ops.MoeLayer(*router, _n(g, E, 2 * I, H, std=0.05), _n(g, E, 2 * I), _n(g, E, H, I, std=0.05), _n(g, E, H),
+                             top_k=k, max_tokens=512)
+    t = _n(g, 400, H)
+    want = layer.forward(t).clone()                # 400 tokens: 200 rows per expert
+    for tokens in (1, 2, 8, 9, 17, 31):            # 9: the largest tile may have more rows than one wave stages
+        got = layer.forward(t[40:40 + tokens].contiguous())
+        assert torch.equal(got, want[40:40 + tokens]), tokens
+
+
+def test_a_tile_list_of_one_expert_and_of_several_tiles(ops):
+    """All tokens on the same experts: tiles of 32 rows with a remainder, the other experts empty."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    H = I = 256
+    E, k = 16, 2
+    b = torch.zeros(E, device="cuda")
+    b[3], b[11] = 50.0, 40.0
+    layer = ops.MoeLayer(_n(g, E, H, std=0.01), b, _n(g, E, 2 * I, H, std=0.05), _n(g, E, 2 * I), _n(g, E, H, I, std=0.05),
+                         _n(g, E, H), top_k=k, max_tokens=512)
+    t = _n(g, 512, H)
+    want = layer.forward(t).clone()
+    for tokens in (5, 33, 64, 70, 100):
+        assert torch.equal(layer.forward(t[:tokens].contiguous()), want[:tokens]), tokens
