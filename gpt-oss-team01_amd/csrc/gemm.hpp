@@ -61,11 +61,18 @@ struct GemmParams {
 // (mat,row-tile) items.
 int run_gemm(const GemmParams &p, bool gather, int epi, int rows_per_tile, int max_tiles,
              hipStream_t s);
-// gemm_few.hip: tiles of at most 32 rows, one wave per 32 columns (bf16 weights; gather + SwiGLU, or no gather and
+// gemm_few.hip: tiles of at most 32 or 64 rows, one wave per 32 columns (bf16 weights; gather + SwiGLU, or no gather and
 // EPI_F32, EPI_MIXED, EPI_PARTIAL).  The rows of A lie within a 31-bit byte offset.
-int run_gemm_few(const GemmParams &p, bool gather, int epi, int max_tiles, hipStream_t s);
+int run_gemm_few(const GemmParams &p, bool gather, int epi, int rows_per_tile, int max_tiles, hipStream_t s);
+constexpr int FEW_SOLO_BLOCKS = 512;   // up to so many 32-column blocks a workgroup is one block
 inline bool gemm_few_applies(const GemmParams &p, int rows_per_tile, int max_tiles) {
-  return rows_per_tile == 32 && (p.tiles ? (long long)max_tiles * 32 : p.dense_rows) * p.K * 2 < (1ll << 31);
+  return rows_per_tile <= 64 && (p.tiles ? (long long)max_tiles * rows_per_tile : p.dense_rows) * p.K * 2 < (1ll << 31);
+}
+// Grouped problems, tiles of 64 rows: the few-row kernels while the launch leaves CUs without work (the block with 4
+// experts of 33 rows, 2880 x 2880: 94 -> 70 us); with more work than that the streaming kernels follow HBM as well or
+// better (16 experts of 25 rows on average: 160 against 167 us; 32 experts, 200-400 tokens: equal within 1 %).
+inline bool grouped_few(const GemmParams &p, int rows_per_tile, int max_tiles) {
+  return rows_per_tile == 32 || (long long)max_tiles * (p.N / 32) <= 1280;
 }
 // gemm_dense.cpp: bf16 weights, no gather (run_gemm comes here for that form)
 int run_gemm_dense(const GemmParams &p, int epi, int rows_per_tile, int max_tiles, hipStream_t s);

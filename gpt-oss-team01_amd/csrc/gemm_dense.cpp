@@ -85,7 +85,7 @@ int run_gemm_dense(const GemmParams &p, int epi, int rows_per_tile, int max_tile
   GPTOSS_REQUIRE(max_rows * p.N < (1ll << 32) && max_rows * p.K < (1ll << 32), GPTOSS_ERR_DIM,
                  "run_gemm: rows x columns must stay below 2^32 elements (rows<=%lld N=%d K=%d)", max_rows, p.N, p.K);
   if (rows_per_tile == 256) return run_gemm_tall(p, epi, max_tiles, max_rows, s);
-  if (epi != EPI_ARGMAX && gemm_few_applies(p, rows_per_tile, max_tiles)) return run_gemm_few(p, false, epi, max_tiles, s);
+  if (epi != EPI_ARGMAX && gemm_few_applies(p, rows_per_tile, max_tiles) && (!p.tiles || grouped_few(p, rows_per_tile, max_tiles))) return run_gemm_few(p, false, epi, rows_per_tile, max_tiles, s);
   int prc = gemm_prepare_device();
   if (prc != GPTOSS_OK) return prc;
   if (epi == EPI_F32) return dispatch_rows<EPI_F32>(p, rows_per_tile, max_tiles, s);
@@ -117,28 +117,44 @@ static int argmax_tall_min_rows() {
   return v;
 }
 
-// Row tile of a dense GEMM on the streaming kernels.  Up to 96 rows: the smallest size that holds every
-// row, so the weights are requested once.  A prompt pass (thousands of rows): 160 rows, every weight
-// fragment feeds five MFMAs.  In between the launch is a handful of rounds of work items on 256 CUs, and
-// an item of MB 32-row blocks takes (0.39 + 0.115 MB) us per 64-k slab (measured at 1024 rows: 0.50 /
-// 0.64 / 0.76 / 0.85 us for 32 / 64 / 96 / 128 rows), so the tile that needs the least rounds x slab time
-// wins: 96 rows for the QKV projection of 1024 rows (220 items, one round), 64 for the output
-// projection (192 items instead of 132: 48 -> 41 us).
-static double slab_us(int mb) { return 0.39 + 0.115 * mb; }
+// Estimated us of a launch, for choosing its row tile and its parts.  `blocks`: 32-column blocks of all its work items,
+// `slabs`: 64-k slabs an item walks.
+// Streaming kernels (gemm_kernel.hpp), items of MB 32-row blocks x 256 columns on 256 CUs, (0.39 + 0.115 MB) us per slab
+// (measured at 1024 rows: 0.50 / 0.64 / 0.76 / 0.85 us for 32 / 64 / 96 / 128 rows).
+// Few-row kernels (gemm_few_kernel.hpp), 128 columns per workgroup, two workgroups per CU: 0.25 us per slab and round of
+// 256 workgroups for 32 rows, 0.32 for 64; up to 512 blocks a workgroup is one block, two per CU.  (Measured on weights
+// that come from HBM, 2048-16384 columns, K 2048-4096, 65-2000 rows: within a fifth of the estimate up to four rounds.)
+static double streaming_us(int mb, long long blocks, int slabs) {
+  return 5.0 + (double)((blocks + 2047) / 2048) * slabs * (0.39 + 0.115 * mb);
+}
 
-static int dense_rows_per_tile(int B, int n_col_tiles) {
-  if (B <= 96) return align_up(B, 32);
-  if (B < 2048 && n_col_tiles >= 64) return 128;  // the unembedding: hundreds of column tiles, measured best at 1024 rows
+static double few_us(int mb, long long blocks, int slabs) {
+  if (blocks <= FEW_SOLO_BLOCKS) return 5.0 + slabs * (mb == 1 ? (blocks <= 256 ? 0.13 : 0.20) : (blocks <= 256 ? 0.28 : 0.33));
+  return 6.5 + (double)((blocks + 1023) / 1024) * slabs * (mb == 1 ? 0.25 : 0.32);
+}
+
+// Row tile of a dense GEMM below the 256-row kernels: the one with the least estimated time; ties go to the larger tile
+// (fewer re-reads of the weights).  Against the streaming kernels alone (96 rows for the QKV projection of 1024 rows, 64
+// for the output projection): 5120 x 2880, 96 / 200 / 400 rows 39 / 32 / 34 -> 16 / 21 / 30 us; 2880 x 4096 52 / 41 / 42
+// -> 17 / 22 / 26; from about 500 rows and 5000 columns on they are the better ones.  Hundreds of column tiles (an
+// unembedding) fill the chip at any size: the smallest tile that holds every row up to 96, then 128, measured best at 1024.
+static int dense_rows_per_tile(int B, int n_col_tiles, int N, int K, int epi) {
   if (B >= 2048) return 160;
+  if (n_col_tiles >= 128 || epi == EPI_ARGMAX) {
+    if (B <= 96) return align_up(B, 32);
+    if (n_col_tiles >= 64) return 128;
+  }
   double best = 0.0;
   int rpt = 160;
   for (int mb = 1; mb <= 5; mb++) {
-    const long long items = (long long)cdiv(B, 32 * mb) * n_col_tiles;
-    const double cost = (double)((items + 255) / 256) * slab_us(mb);
-    if (mb == 1 || cost <= best) {  // ties go to the larger tile: fewer re-reads of the weights
-      best = cost;
+    const long long tiles = cdiv(B, 32 * mb);
+    const double us = mb <= 2 && epi != EPI_ARGMAX ? few_us(mb, tiles * (N / 32), K / 64)
+                                                   : streaming_us(mb, tiles * n_col_tiles * 8, K / 64);
+    if (mb == 1 || us <= best) {
+      best = us;
       rpt = 32 * mb;
     }
+    if (tiles == 1) break;
   }
   return rpt;
 }
@@ -164,7 +180,7 @@ int dense_gemm(const bf16_t *A, const bf16_t *W, const float *bias, void *out, i
   GemmParams g = dense_params(A, W, bias, out, B, N, K);
   g.amax_val = amax_val;
   g.amax_idx = amax_idx;
-  int rpt = dense_rows_per_tile(B, g.n_col_tiles);
+  int rpt = dense_rows_per_tile(B, g.n_col_tiles, N, K, epi);
   if (B >= (epi == EPI_ARGMAX ? argmax_tall_min_rows() : dense_tall_min_rows()) && gemm_tall_applies(g, false, epi) &&
       gemm_tall_shape_ok(N, K, B))
     rpt = 256;
@@ -184,7 +200,7 @@ int dense_gemm_mixed(const bf16_t *A, const bf16_t *W, float *out, const GemmBf1
     GPTOSS_REQUIRE(ranges[i].from % 32 == 0 && ranges[i].to % 32 == 0 && ranges[i].ld % 4 == 0 && aligned(ranges[i].out, 8),
                    GPTOSS_ERR_DIM, "dense_gemm_mixed: ranges are whole 32-column blocks of aligned rows");
   }
-  int rpt = dense_rows_per_tile(B, g.n_col_tiles);
+  int rpt = dense_rows_per_tile(B, g.n_col_tiles, N, K, EPI_MIXED);
   if (B >= dense_tall_min_rows() && gemm_tall_applies(g, false, EPI_MIXED) && gemm_tall_shape_ok(N, K, B)) rpt = 256;
   return run_gemm_dense(g, EPI_MIXED, rpt, cdiv(B, rpt), s);
 }
@@ -206,8 +222,9 @@ int dense_gemm_partial(const bf16_t *A, const bf16_t *W, float *out, size_t max_
       const int per = cdiv(nslab, want), n = cdiv(nslab, per);
       // (an item prefetches two slabs of the next one, so no part may have fewer)
       if (n != want || (n > 1 && (per < 4 || nslab - per * (n - 1) < 2 || (size_t)n * B * N > max_elems))) continue;
-      const long long items = (long long)cdiv(B, 32 * mb) * g.n_col_tiles * n;
-      const double cost = (double)((items + 255) / 256) * (per * slab_us(mb) + 5.0) + (n - 1) * (double)B * N * 8 / 5e6;
+      const long long tiles = cdiv(B, 32 * mb);
+      const double cost = (mb <= 2 ? few_us(mb, tiles * (N / 32) * n, per) : streaming_us(mb, tiles * g.n_col_tiles * 8 * n, per)) +
+                          (n - 1) * (double)B * N * 8 / 5e6;
       if ((mb == 1 && n == 1) || cost < best) {
         best = cost;
         rpt = 32 * mb;

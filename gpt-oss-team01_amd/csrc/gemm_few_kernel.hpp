@@ -1,31 +1,38 @@
-// GEMMs of a few rows for gfx950: the same products as gemm_kernel.hpp for row tiles of at most 32 rows.
+// GEMMs of a few rows for gfx950: the same products as gemm_kernel.hpp for row tiles of at most 32 or 64 rows.
 //
-//   C[rows, N] = A[rows, K] . W[N, K]^T      rows <= 32: a decoding step of few sequences, or an expert's few tokens
+//   C[rows, N] = A[rows, K] . W[N, K]^T      a decoding step of few sequences, a short prompt, an expert's few tokens
 //
 // Nothing but reading W takes time here, so what counts is how many bytes of W are on their way at any moment, from how
 // many CUs.  The streaming kernels give 256 columns to a workgroup of eight waves with two 4 KB slabs of W in flight
 // each, on a grid of one workgroup per CU: one token's four experts are then 92 (first product) and 48 (second) work
-// items on 256 CUs.  Here a workgroup is 128 columns, or 32 where no tile has more than eight rows, the grid has one for
-// every work item, and a wave has eight slabs in flight (MXFP4: sixteen).  To have the registers for that, A does not
-// pass through them slab by slab: chunks of eight slabs are staged in LDS, one barrier each, and W's loads stay in
-// flight across it.  Operand roles, order of the sum over K and epilogues are those of the streaming kernels, so a row
-// has the same bits whichever kernel computes it.
+// items on 256 CUs.  Here a workgroup is 128 columns, or 32 (below), the grid has one for every work item, and a wave
+// has eight slabs in flight (MXFP4: sixteen).  To have the registers for that, A does not pass through them slab by
+// slab: chunks of eight slabs (64 rows: four) are staged in LDS, one barrier each, and W's loads stay in flight across
+// it.  Operand roles, order of the sum over K and epilogues are those of the streaming kernels, so a row has the same
+// bits whichever kernel computes it.
 // Measured, 2880 x 2880 experts, streaming kernels -> these (us): one token, both products 36 + 32 -> 24 + 14, MXFP4
-// block 60 -> 43; a dense projection of one row 38 -> 13; 27 tokens 156 + 91 -> 157 + 81 (5.9-6.8 TB/s either way);
-// 12 tokens on MXFP4 60 + 32 -> 49 + 29.  32 columns per workgroup instead of 128: one token's block 68 -> 59, eight
-// tokens 178 -> 176.  (A read straight from memory in operand order, without LDS: one token 60, but 12 tokens on MXFP4
-// 127 instead of 99, because A is then four times the bytes of W.)
+// block 60 -> 43; 27 tokens 156 + 91 -> 157 + 81 (5.9-6.8 TB/s either way); 12 tokens on MXFP4 60 + 32 -> 49 + 29.
+// Dense 5120 x 2880: one row 31 -> 9, 32 rows 33 -> 11, 64 rows 37 -> 16, 200 rows 32 -> 21.
+// (A read straight from memory in operand order, without LDS: one token 60, but 12 tokens on MXFP4 127 instead of 99,
+// because A is then four times the bytes of W.)
 #pragma once
 #include "gemm_kernel.hpp"
 
 namespace gptoss {
 
-// WAVES: 32-column blocks of a workgroup, one per wave; the waves share the staged rows of A, eight rows per wave.
+// A workgroup: WAVES 32-column blocks, one per wave, times tiles of at most ROWS rows.
+//   4 x 32, 4 x 64   the waves share the staged rows
+//   1 x 8            one wave can stage so few rows by itself, and four times as many workgroups fill the chip: one
+//                    token's block 68 -> 59 us, eight tokens' 178 -> 176
+//   1 x 32, 1 x 64   the same for launches of at most FEW_SOLO_BLOCKS blocks, on the registers of two waves
 
 // 64-k slabs of W that a wave keeps in flight: 16 bytes per lane and k-step with bf16 weights, 16 per slab with MXFP4
 constexpr int few_ring(bool fp4) { return fp4 ? 16 : 8; }
-constexpr int FEW_CHUNK = 8;                          // slabs of A that are staged together: one barrier each
-constexpr int FEW_ROW = FEW_CHUNK * BK + 8;           // padded row of a staged chunk in bf16 elements (1040 B)
+constexpr int few_chunk(int rows) { return rows <= 32 ? 8 : 4; }   // slabs of A that are staged together: one barrier each
+constexpr int few_row(int rows) { return few_chunk(rows) * BK + 8; }   // padded row of a staged chunk in bf16 elements
+constexpr int few_ahead(int rows) { return rows <= 32 ? 4 : 2; }       // k-steps whose operands are read from LDS ahead
+// waves per SIMD: a single wave that stages 32 rows or more needs the registers of two
+constexpr int few_occupancy(int waves, int rows) { return waves == 1 && rows > 8 ? 1 : 2; }
 
 typedef __amdgpu_buffer_rsrc_t few_rsrc_t;
 // cache policy of a buffer load: the non-temporal bit
@@ -37,11 +44,11 @@ __device__ __forceinline__ few_rsrc_t few_buffer(const void *base, uint32_t byte
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);
 }
 
-template <int WAVES, bool GATHER, int EPI, bool FP4, bool ONCE>
+template <int WAVES, int ROWS, bool GATHER, int EPI, bool FP4, bool ONCE>
 __device__ __forceinline__ void few_block(const GemmParams &p, bf16_t *lds, int mat, int row0, int rows, int cb, int slab0,
                                           int nslab, void *out) {
   constexpr int RING = few_ring(FP4);
-  constexpr int ROWS = WAVES * 8;   // rows of A that are staged
+  constexpr int RB = (ROWS + 31) / 32, CHUNK = few_chunk(ROWS), ROW = few_row(ROWS), AHEAD = few_ahead(ROWS);
   constexpr int WQ = FP4 ? 1 : 4;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int K = p.K, N = p.N, kslab = K / BK;
@@ -66,70 +73,86 @@ __device__ __forceinline__ void few_block(const GemmParams &p, bf16_t *lds, int 
     if constexpr (FP4) sc[R] = __builtin_amdgcn_raw_buffer_load_b16(sb, (lane & 31) * 2 + s * 64, 0, ONCE ? FEW_NT : 0);
   };
   // which rows of A the tile's rows are: before W, because loads return in order
-  int id = row0 + min(lane & 31, rows - 1);
+  int id = row0 + min(lane, rows - 1);
   if (GATHER) id = p.row_ids[id];
   static_for<0, RING>([&](auto r) { load_w(decltype(r)::value, r); });
   const few_rsrc_t bb = few_buffer(p.bias && live ? p.bias + (size_t)mat * N + cb * 32 : nullptr, p.bias && live ? 128 : 0);
   const int bias = __builtin_amdgcn_raw_buffer_load_b32(bb, (lane & 31) * 4, 0, 0);
 
-  // A: the workgroup copies chunks of ROWS rows x FEW_CHUNK slabs, a wave one row (1 KB) per load.  Rows beyond the
+  // A: the workgroup copies chunks of ROWS rows x CHUNK slabs, a wave 1 KB (one row or two) per load.  Rows beyond the
   // tile's and k beyond K are zeros, again from outside the buffer.
+  constexpr int PIECES = CHUNK * 8, PER = 64 / PIECES;   // 16-byte pieces of a row; rows of a load instruction
+  constexpr int NA = ROWS / PER / WAVES;
   const few_rsrc_t ab = few_buffer(p.A + (size_t)slab0 * BK, FEW_A_BYTES);
   if (GATHER) id = (uint32_t)id / (uint32_t)p.top_k;
-  uint32_t a_off[8];
+  uint32_t a_off[NA];
 #pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const int r = wave + WAVES * i;
-    a_off[i] = r < rows ? (uint32_t)__builtin_amdgcn_readlane(id, r) * (uint32_t)K * 2u : FEW_A_BYTES;
+  for (int i = 0; i < NA; i++) {
+    const int r = (wave + WAVES * i) * PER + lane / PIECES;
+    int src = __builtin_amdgcn_readlane(id, (wave + WAVES * i) * PER);
+    if (PER == 2) src = lane < PIECES ? src : __builtin_amdgcn_readlane(id, (wave + WAVES * i) * PER + 1);
+    a_off[i] = r < rows ? (uint32_t)src * (uint32_t)K * 2u : FEW_A_BYTES;
   }
-  u32x4 areg[8];
+  u32x4 areg[NA];
   auto load_a = [&](int c) {
-    const int k = c * (FEW_CHUNK * BK) + lane * 8;
+    const int k = c * (CHUNK * BK) + lane % PIECES * 8;
 #pragma unroll
-    for (int i = 0; i < 8; i++)
+    for (int i = 0; i < NA; i++)
       areg[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ab, k < nslab * BK ? a_off[i] + k * 2 : FEW_A_BYTES, 0, 0));
   };
   auto store_a = [&](int c) {
-    bf16_t *d = lds + (c & 1) * (ROWS * FEW_ROW) + wave * FEW_ROW + lane * 8;
+    bf16_t *d = lds + (c & 1) * (ROWS * ROW) + (wave * PER + lane / PIECES) * ROW + lane % PIECES * 8;
 #pragma unroll
-    for (int i = 0; i < 8; i++) *reinterpret_cast<u32x4 *>(d + WAVES * i * FEW_ROW) = areg[i];
+    for (int i = 0; i < NA; i++) *reinterpret_cast<u32x4 *>(d + WAVES * PER * i * ROW) = areg[i];
   };
   load_a(0);
   store_a(0);
   __syncthreads();
 
-  f32x16 acc[1];
+  f32x16 acc[RB];
 #pragma unroll
-  for (int i = 0; i < 16; i++) acc[0][i] = 0.f;
-  const bf16_t *a_src = lds + min(lane & 31, ROWS - 1) * FEW_ROW + (lane >> 5) * 8;
-  bf16x8 af[2][4];   // a slab's operands are read while the slab before is multiplied
-  auto read_a = [&](int c, auto rr) {
-    constexpr int R = decltype(rr)::value;
+  for (int i = 0; i < RB; i++)
 #pragma unroll
-    for (int kk = 0; kk < 4; kk++)
-      af[R & 1][kk] = as_bf16x8(*reinterpret_cast<const u32x4 *>(a_src + (c & 1) * (ROWS * FEW_ROW) + R % FEW_CHUNK * BK + kk * 16));
+    for (int x = 0; x < 16; x++) acc[i][x] = 0.f;
+  const bf16_t *a_src = lds + min(lane & 31, ROWS - 1) * ROW + (lane >> 5) * 8;
+  // the operands of AHEAD k-steps are read while the AHEAD before them are multiplied: group G of them into set G & 1
+  bf16x8 af[2][AHEAD][RB];
+  auto read_a = [&](int c, auto gg) {
+    constexpr int G = decltype(gg)::value;
+#pragma unroll
+    for (int x = 0; x < AHEAD; x++)
+#pragma unroll
+      for (int i = 0; i < RB; i++)
+        af[G & 1][x][i] = as_bf16x8(*reinterpret_cast<const u32x4 *>(a_src + (c & 1) * (ROWS * ROW) + i * 32 * ROW +
+                                                                     (G * AHEAD + x) % (CHUNK * 4) * 16));
   };
   read_a(0, std::integral_constant<int, 0>{});
   for (int s = 0; s < nslab; s += RING)
     static_for<0, RING>([&](auto rr) {
       constexpr int R = decltype(rr)::value;
-      const int c = (s + R) / FEW_CHUNK;
-      if constexpr (R % FEW_CHUNK == 0) load_a(c + 1);
-      if constexpr (R % FEW_CHUNK != FEW_CHUNK - 1) read_a(c, std::integral_constant<int, R + 1>{});
-      __builtin_amdgcn_sched_barrier(0);
+      const int c = (s + R) / CHUNK;
+      if constexpr (R % CHUNK == 0) load_a(c + 1);
+      static_for<0, 4 / AHEAD>([&](auto hh) {
+        constexpr int G = R * 4 / AHEAD + decltype(hh)::value;
+        if constexpr ((G + 1) * AHEAD % (CHUNK * 4) != 0) read_a(c, std::integral_constant<int, G + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int kk = 0; kk < 4; kk++) {
-        bf16x8 b;
-        if constexpr (FP4) b = as_bf16x8(fp4_expand(w[R][0][kk], fp4_scale((sc[R] >> (8 * (kk >> 1))) & 0xffu)));
-        else b = as_bf16x8(w[R][kk % WQ]);
-        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, af[R & 1][kk], acc[0], 0, 0, 0);
-      }
+        for (int x = 0; x < AHEAD; x++) {
+          constexpr int K0 = decltype(hh)::value * AHEAD;
+          bf16x8 b;
+          if constexpr (FP4) b = as_bf16x8(fp4_expand(w[R][0][K0 + x], fp4_scale((sc[R] >> (8 * ((K0 + x) >> 1))) & 0xffu)));
+          else b = as_bf16x8(w[R][(K0 + x) % WQ]);
+#pragma unroll
+          for (int i = 0; i < RB; i++)
+            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, af[G & 1][x][i], acc[i], 0, 0, 0);
+        }
+      });
       load_w(s + R + RING, rr);
       __builtin_amdgcn_sched_barrier(0);   // the order of the loads is the order of their uses
-      if constexpr (R % FEW_CHUNK == FEW_CHUNK - 1) {
+      if constexpr (R % CHUNK == CHUNK - 1) {
         store_a(c + 1);
         __syncthreads();
-        read_a(c + 1, std::integral_constant<int, (R + 1) % RING>{});
+        read_a(c + 1, std::integral_constant<int, (R + 1) % RING * 4 / AHEAD>{});
       }
     });
   if (!live) return;
@@ -137,19 +160,20 @@ __device__ __forceinline__ void few_block(const GemmParams &p, bf16_t *lds, int 
   if constexpr (EPI == EPI_PARTIAL) {
     GemmParams q = p;
     q.out = out;
-    epilogue_rows<1, EPI_F32>(q, row0, rows, cb * 32, lane, acc, bias_of);
+    epilogue_rows<RB, EPI_F32>(q, row0, rows, cb * 32, lane, acc, bias_of);
   } else {
-    epilogue_rows<1, EPI>(p, row0, rows, cb * 32, lane, acc, bias_of);
+    epilogue_rows<RB, EPI>(p, row0, rows, cb * 32, lane, acc, bias_of);
   }
 }
 
 // Work items are (row tile, 32-column block) pairs; every XCD has a contiguous part of them, so that the row tiles of
 // one expert, which multiply the same blocks of W one after the other, find them in that XCD's L2.
-template <int WAVES, bool GATHER, int EPI, bool FP4>
-__global__ __launch_bounds__(WAVES * 64, 2) void few_gemm_kernel(GemmParams p) {
-  __shared__ __attribute__((aligned(16))) bf16_t lds[2 * WAVES * 8 * FEW_ROW];
+template <int WAVES, int ROWS, bool GATHER, int EPI, bool FP4>
+__global__ __launch_bounds__(WAVES * 64, few_occupancy(WAVES, ROWS)) void few_gemm_kernel(GemmParams p) {
+  constexpr int BM = ROWS <= 32 ? 32 : 64;   // rows of a dense problem's tile
+  __shared__ __attribute__((aligned(16))) bf16_t lds[2 * ROWS * few_row(ROWS)];
   const const_as<int> tiles = constant_ptr(p.tiles);
-  const int n_tiles = p.tiles ? tiles[0] : (p.dense_rows + 31) / 32;
+  const int n_tiles = p.tiles ? tiles[0] : (p.dense_rows + BM - 1) / BM;
   const int n_blk = (p.N / 32 + WAVES - 1) / WAVES;
   const int tile_items = n_tiles * n_blk;
   const int total = EPI == EPI_PARTIAL ? tile_items * p.k_splits : tile_items;
@@ -183,8 +207,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void few_gemm_kernel(GemmParams p) {
   } else {
     cb = work / n_tiles;
     tile = work - cb * n_tiles;
-    row0 = tile * 32;
-    rows = min(32, p.dense_rows - row0);
+    row0 = tile * BM;
+    rows = min(BM, p.dense_rows - row0);
     once = n_tiles == 1;
   }
   int slab0 = 0, nslab = p.K / BK;
@@ -199,29 +223,33 @@ __global__ __launch_bounds__(WAVES * 64, 2) void few_gemm_kernel(GemmParams p) {
   cb = __builtin_amdgcn_readfirstlane(cb * WAVES + (threadIdx.x >> 6));
   row0 = __builtin_amdgcn_readfirstlane(row0), rows = __builtin_amdgcn_readfirstlane(rows);
   slab0 = __builtin_amdgcn_readfirstlane(slab0), nslab = __builtin_amdgcn_readfirstlane(nslab);
-  if (once) few_block<WAVES, GATHER, EPI, FP4, true>(p, lds, mat, row0, rows, cb, slab0, nslab, out);
-  else few_block<WAVES, GATHER, EPI, FP4, false>(p, lds, mat, row0, rows, cb, slab0, nslab, out);
+  if (once) few_block<WAVES, ROWS, GATHER, EPI, FP4, true>(p, lds, mat, row0, rows, cb, slab0, nslab, out);
+  else few_block<WAVES, ROWS, GATHER, EPI, FP4, false>(p, lds, mat, row0, rows, cb, slab0, nslab, out);
 }
 
-template <int WAVES, bool GATHER, int EPI, bool FP4>
+template <int WAVES, int ROWS, bool GATHER, int EPI, bool FP4>
 int launch_few_waves(const GemmParams &p, int max_tiles, hipStream_t s) {
   const long long total = (long long)max_tiles * cdiv(p.N / 32, WAVES) * (EPI == EPI_PARTIAL ? p.k_splits : 1);
   if (total == 0) return GPTOSS_OK;
   {
     TraceScope ts(FP4 ? (GATHER ? "gemm1_gather_swiglu_mxfp4" : "gemm_f32_mxfp4")
                       : (GATHER ? "gemm1_gather_swiglu" : "gemm_f32"), s);
-    few_gemm_kernel<WAVES, GATHER, EPI, FP4><<<(unsigned)(((total + 7) / 8) * 8), WAVES * 64, 0, s>>>(p);
+    few_gemm_kernel<WAVES, ROWS, GATHER, EPI, FP4><<<(unsigned)(((total + 7) / 8) * 8), WAVES * 64, 0, s>>>(p);
   }
   GPTOSS_LAUNCH_CHECK("few_gemm_kernel");
   return GPTOSS_OK;
 }
 
-// Up to eight rows per tile one wave can stage them by itself, and the launch has four times as many workgroups to fill
-// the chip with; beyond that the rows are shared by four waves.
 template <bool GATHER, int EPI, bool FP4>
-int launch_few_gemm(const GemmParams &p, int max_tiles, hipStream_t s) {
-  if (p.max_tile_rows && p.max_tile_rows <= 8) return launch_few_waves<1, GATHER, EPI, FP4>(p, max_tiles, s);
-  return launch_few_waves<4, GATHER, EPI, FP4>(p, max_tiles, s);
+int launch_few_gemm(const GemmParams &p, int rows_per_tile, int max_tiles, hipStream_t s) {
+  // few blocks: workgroups of four would leave most CUs without one (2880 x 5120, 32 rows: 20 us on 40 CUs, 11 on 160)
+  const long long blocks = (long long)max_tiles * (p.N / 32) * (EPI == EPI_PARTIAL ? p.k_splits : 1);
+  const bool solo = blocks <= FEW_SOLO_BLOCKS;
+  if constexpr (!FP4)
+    if (rows_per_tile == 64)
+      return solo ? launch_few_waves<1, 64, GATHER, EPI, FP4>(p, max_tiles, s) : launch_few_waves<4, 64, GATHER, EPI, FP4>(p, max_tiles, s);
+  if (p.max_tile_rows && p.max_tile_rows <= 8) return launch_few_waves<1, 8, GATHER, EPI, FP4>(p, max_tiles, s);
+  return solo ? launch_few_waves<1, 32, GATHER, EPI, FP4>(p, max_tiles, s) : launch_few_waves<4, 32, GATHER, EPI, FP4>(p, max_tiles, s);
 }
 
 }  // namespace gptoss

@@ -16,7 +16,7 @@ static hipError_t set_attrs() {
 
 template <bool GATHER, int EPI>
 static int dispatch_rows(const GemmParams &p, int rows_per_tile, int max_tiles, hipStream_t s) {
-  if (gemm_few_applies(p, rows_per_tile, max_tiles)) return launch_few_gemm<GATHER, EPI, true>(p, max_tiles, s);
+  if (rows_per_tile == 32 && gemm_few_applies(p, rows_per_tile, max_tiles)) return launch_few_gemm<GATHER, EPI, true>(p, rows_per_tile, max_tiles, s);
   switch (rows_per_tile) {
     case 32: return launch_gemm<1, GATHER, EPI, true>(p, max_tiles, s);
     case 64: return launch_gemm<2, GATHER, EPI, true>(p, max_tiles, s);

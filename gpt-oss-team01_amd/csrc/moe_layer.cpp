@@ -67,7 +67,7 @@ int moe_tall_min_rows() {
 
 int moe_rows_per_tile(int B, int k, int E, bool mxfp4) {
   double avg = (double)B * k / E;
-  double need = avg + 2.5 * sqrt(avg);
+  double need = k == E ? avg : avg + 2.5 * sqrt(avg);   // (every token on every expert: nothing to deviate)
 
   if (need <= 32) return 32;
   if (need <= 64) return 64;

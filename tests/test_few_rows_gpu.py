@@ -1,4 +1,4 @@
-"""The few-row GEMM kernels (tiles of at most 32 rows): every row must have the bits that the streaming kernels give it
+"""The few-row GEMM kernels (tiles of at most 64 rows): every row must have the bits that the streaming kernels give it
 in a larger batch, at the edges of row tiles, column blocks and staged chunks of K."""
 import pytest
 import torch
@@ -20,14 +20,14 @@ def _n(g, *shape, std=1.0):
 # K: one slab, one short of a chunk of eight slabs, a chunk, one more, the 20B model's; N: part of a workgroup's 128
 # columns, one workgroup and a block, the 20B model's 22.5 workgroups
 @pytest.mark.parametrize("K", [64, 448, 512, 576, 2880])
-@pytest.mark.parametrize("N", [32, 160, 2880])
+@pytest.mark.parametrize("N", [32, 160, 2880, 17408])   # 17408: 544 blocks in one row tile, so never a block each
 def test_dense_rows_equal_those_of_a_larger_batch(ops, K, N):
     g = torch.Generator(device="cuda").manual_seed(K + N)
-    a, w, bias = _n(g, 150, K), ops.pack_weight(_n(g, N, K, std=0.05)), _n(g, N).float()
+    a, w, bias = _n(g, 2100, K), ops.pack_weight(_n(g, N, K, std=0.05)), _n(g, N).float()
     for b in (bias, None):
-        want = ops.dense_gemm(a, w, N, bias=b)     # 150 rows: the streaming kernel
-        for rows in (1, 2, 7, 8, 9, 31, 32):
-            for first in (0, 150 - rows):
+        want = ops.dense_gemm(a, w, N, bias=b)     # 2100 rows: the streaming kernels, or those of 256 rows
+        for rows in (1, 2, 7, 8, 9, 31, 32, 33, 63, 64, 65, 96, 130, 330):
+            for first in (0, 2100 - rows):
                 got = ops.dense_gemm(a[first:first + rows].contiguous(), w, N, bias=b)
                 assert torch.equal(got, want[first:first + rows]), (rows, first)
 
@@ -36,7 +36,7 @@ def _codes(g, *shape):
     return torch.randint(0, 256, shape, generator=g, device="cuda", dtype=torch.uint8)
 
 
-@pytest.mark.parametrize("H,I,E,k", [(64, 64, 4, 2), (320, 576, 8, 4), (2880, 2880, 8, 4)])
+@pytest.mark.parametrize("H,I,E,k", [(64, 64, 4, 2), (320, 576, 8, 4), (512, 448, 4, 4), (2880, 2880, 8, 4)])
 @pytest.mark.parametrize("mxfp4", [False, True])
 def test_moe_rows_equal_those_of_a_larger_batch(ops, H, I, E, k, mxfp4):
     g = torch.Generator(device="cuda").manual_seed(H + I + mxfp4)
@@ -50,7 +50,7 @@ def test_moe_rows_equal_those_of_a_larger_batch(ops, H, I, E, k, mxfp4):
                              top_k=k, max_tokens=512)
     t = _n(g, 400, H)
     want = layer.forward(t).clone()                # 400 tokens: 200 rows per expert
-    for tokens in (1, 2, 8, 9, 17, 31):            # 9: the largest tile may have more rows than one wave stages
+    for tokens in (1, 2, 8, 9, 17, 31, 33, 60, 90):   # 9: the largest tile may have more rows than one wave stages
         got = layer.forward(t[40:40 + tokens].contiguous())
         assert torch.equal(got, want[40:40 + tokens]), tokens
 
