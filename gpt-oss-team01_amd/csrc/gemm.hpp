@@ -119,12 +119,22 @@ constexpr int MOE_MAX_TOP = 32;
 // norm_out = norm(out), in the same kernel as the combine.
 int moe_forward_glu(const gptoss_moe_weights *w, const GluForm &glu, const void *t, int B, float *out, void *workspace,
                     size_t workspace_bytes, hipStream_t s, const TanhNorm &norm, bf16_t *norm_out);
+// The grouping of a batch's pairs by expert, for the router kernel to do as well where one workgroup holds every token:
+// saves a launch that takes 5 us for any small batch.  nbits: bits of an expert id.
+struct RouterGroup {
+  int *expert_offsets = nullptr, *sorted_pair_ids, *inv_perm, *tiles;
+  int *xcd_bounds, nbits;
+};
+constexpr int ROUTER_GROUP_TOKENS = 16;   // the rows of one MFMA
+// (behind a norm in the same kernel, whose rows go two at a time: ROUTER_GROUP_NORM_TOKENS)
+constexpr int ROUTER_GROUP_NORM_TOKENS = 4;
+inline bool router_groups(int B, int k) { return B <= ROUTER_GROUP_TOKENS && k <= 8; }
 // moe_route.hip: residual add + RMSNorm + router GEMM + gating in one launch
 bool norm_router_applies(int B, int H, int E, const float *x, const float *residual, const float *weight,
                          const void *t_out);
 int run_norm_router(float *x, const float *residual, const float *weight, void *t_out, const void *w_router,
                     const float *b_router, float *logits, int B, int H, int E, int k, float *topk_w, int *topk_i,
-                    hipStream_t s);
+                    hipStream_t s, const RouterGroup *group = nullptr);
 int moe_rows_per_tile(int B, int k, int E, bool mxfp4);
 // dense C = A . W^T (+ bias) with the epilogue `epi`; EPI_ARGMAX fills amax_val / amax_idx [B, *amax_tiles]
 // EPI_ARGMAX: *amax_tiles (required) receives the number of (value, column) pairs written per row,
@@ -143,7 +153,7 @@ int gemm_col_tiles(int N);  // column tiles of one workgroup's width
 inline int gemm_argmax_tiles(int N) { return 2 * gemm_col_tiles(N); }  // pairs per row to allocate for EPI_ARGMAX
 // moe_route.hip
 int run_router(const void *t, const void *w_router, const float *b_router, float *logits, int B,
-               int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s);
+               int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group = nullptr);
 int run_topk_softmax(const float *logits, int B, int E, int k, float *topk_w, int *topk_i, hipStream_t s);
 // xcd_bounds (optional, XCD_BOUNDS_INTS + max_tiles ints): see GemmParams; tile_cost0_x2 = twice the fixed part of a tile's
 // cost in units of one 32-row block of arithmetic (cost = fixed + number of 32-row blocks);

@@ -160,24 +160,33 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
   // experts, seven of them above 160 rows) runs the layer 7 % faster, prompt passes 2-4 %.
   const int tile_block = MOE_TILE_BLOCK;
 
-  // router GEMM with the gating of its own 16 tokens fused in, then the stable grouping
-  // (with `pre`, the residual add and RMSNorm that produce t run in the same launch)
-  if (pre && norm_router_applies(B, H, E, pre->x, pre->residual, pre->weight, t))
+  // router GEMM with the gating of its own 16 tokens fused in, then the stable grouping, in the same launch for a few
+  // tokens (with `pre`, the residual add and RMSNorm that produce t run in it as well)
+  const int cost0 = mxfp4 ? MOE_TILE_COST0_X2_MXFP4 : MOE_TILE_COST0_X2_BF16;
+  RouterGroup grp;
+  grp.sorted_pair_ids = ws.sorted_pair_ids;
+  grp.inv_perm = ws.inv_perm;
+  grp.tiles = ws.tiles;
+  grp.xcd_bounds = ws.xcd_bounds;
+  grp.nbits = 0;
+  while ((1 << grp.nbits) < E) grp.nbits++;
+  if (pre && norm_router_applies(B, H, E, pre->x, pre->residual, pre->weight, t)) {
+    if (router_groups(B, k) && B <= ROUTER_GROUP_NORM_TOKENS) grp.expert_offsets = ws.expert_offsets;
     rc = run_norm_router(pre->x, pre->residual, pre->weight, const_cast<void *>(t), w->w_router, w->b_router,
-                         ws.logits, B, H, E, k, ws.topk_w, ws.topk_i, s);
-  else {
+                         ws.logits, B, H, E, k, ws.topk_w, ws.topk_i, s, &grp);
+  } else {
     if (pre) {
       rc = run_rmsnorm(pre->x, pre->residual, pre->weight, (bf16_t *)const_cast<void *>(t), nullptr, B, H, s);
       if (rc != GPTOSS_OK) return rc;
     }
-    rc = run_router(t, w->w_router, w->b_router, ws.logits, B, H, E, k, ws.topk_w, ws.topk_i, s);
+    if (router_groups(B, k)) grp.expert_offsets = ws.expert_offsets;
+    rc = run_router(t, w->w_router, w->b_router, ws.logits, B, H, E, k, ws.topk_w, ws.topk_i, s, &grp);
   }
+  if (rc == GPTOSS_OK && !grp.expert_offsets)
+    rc = run_group(B, E, k, ws.topk_w, ws.topk_i, ws.expert_offsets, ws.sorted_pair_ids, ws.inv_perm,
+                   ws.tiles, rpt, ws.xcd_bounds, cost0, s, ws.sort_scratch);
   if (rc != GPTOSS_OK) return rc;
-  rc = run_group(B, E, k, ws.topk_w, ws.topk_i, ws.expert_offsets, ws.sorted_pair_ids, ws.inv_perm,
-                 ws.tiles, rpt, ws.xcd_bounds, mxfp4 ? MOE_TILE_COST0_X2_MXFP4 : MOE_TILE_COST0_X2_BF16, s,
-                 ws.sort_scratch);
   const int *bounds = max_tiles < 32768 ? ws.xcd_bounds : nullptr;
-  if (rc != GPTOSS_OK) return rc;
 
   GemmParams g1{};
   g1.A = (const bf16_t *)t;

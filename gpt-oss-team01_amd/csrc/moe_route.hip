@@ -18,7 +18,7 @@ namespace gptoss {
 template <int NJ, int KMAX = 8>
 __device__ __forceinline__ void topk_softmax_group(const float (&v)[NJ], int sub, int E, int k,
                                                    bool live, float *__restrict__ w_out,
-                                                   int *__restrict__ i_out) {
+                                                   int *__restrict__ i_out, int *i_copy = nullptr) {
   uint32_t used = 0;
   float pick_v[KMAX];
   int pick_i[KMAX];
@@ -66,183 +66,11 @@ __device__ __forceinline__ void topk_softmax_group(const float (&v)[NJ], int sub
       if (s < k) {
         w_out[s] = (float)((double)ex[s] / sum);
         i_out[s] = pick_i[s];
+        if (i_copy) i_copy[s] = pick_i[s];
       }
     }
   }
 }
-
-// ------------------------------------------------------------------------------------------------
-// Router GEMM: logits[B,E] = t[B,H] . Wr[E,H]^T + br.  One workgroup = 16 token rows x all experts;
-// its 8 waves split the K loop (k-steps of 32, interleaved), request all their operands up front
-// and reduce through LDS.  With topk_w != nullptr the workgroup also gates its 16 tokens (32
-// lanes per token) while the logits are still in LDS.
-// ------------------------------------------------------------------------------------------------
-constexpr int ROUTER_WAVES = 8;
-// k-steps whose operands a wave requests before its first MFMA: as many as ~150 registers hold,
-// so that a hidden size of 2880 with up to 32 experts is a single round of loads
-constexpr int router_steps(int nb) { return nb <= 2 ? 12 : (nb <= 4 ? 7 : (nb <= 8 ? 4 : 2)); }
-
-// What the NORM form of the router kernel does first: x += residual, t = RMSNorm(x) * weight for the
-// workgroup's own token rows.
-struct RouterNorm {
-  float *x;               // [B,H] residual stream, updated in place
-  const float *residual;  // [B,H] or nullptr
-  const float *weight;    // [H]
-  bf16_t *t_out;          // [B,H]
-};
-
-// NB: number of 16-expert column blocks held per wave.  NORM: the workgroup first normalises its
-// rows (the arithmetic of rmsnorm_rows_kernel: 256 threads per row, the same element-to-thread
-// assignment and summation order, so t is the same to the bit), writes x and t to memory, keeps t in
-// LDS and multiplies from there: one launch and one read of t less than norm kernel + router kernel.
-template <int NB, bool NORM>
-__global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
-    const bf16_t *__restrict__ t, const bf16_t *__restrict__ wr, const float *__restrict__ br,
-    float *__restrict__ logits, int B, int H, int E, int k, float *__restrict__ topk_w,
-    int *__restrict__ topk_i, int rows_per_wg, RouterNorm nrm) {
-  __shared__ float red[ROUTER_WAVES][16][NB * 16 + 1];
-  extern __shared__ __attribute__((aligned(16))) unsigned char t_rows_raw[];  // NORM: [rows_per_wg][H] bf16
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // rows_per_wg <= 16 token rows are this workgroup's; the other MFMA rows repeat the last of them
-  const int r0 = blockIdx.x * rows_per_wg;
-  const int arow = min(r0 + min(lane & 15, rows_per_wg - 1), B - 1);
-  const int kq = (lane >> 4) * 8;
-  const bf16_t *ap = t + (size_t)arow * H + kq;
-  if constexpr (NORM) {
-    constexpr int VPT = 4;  // rows of up to 4096 floats
-    __shared__ double nred[2][4];
-    bf16_t *t_rows = reinterpret_cast<bf16_t *>(t_rows_raw);
-    const int grp = threadIdx.x >> 8, tg = threadIdx.x & 255;  // two groups of 256 threads, a row each
-    for (int rr = 0; rr < rows_per_wg; rr += 2) {
-      const int lr = rr + grp;
-      const bool live = lr < rows_per_wg && r0 + lr < B;
-      const size_t row = (size_t)(r0 + lr) * H;
-      f32x4 v[VPT];
-      double ss = 0.0;
-#pragma unroll
-      for (int i = 0; i < VPT; i++) {
-        const int h = (tg + 256 * i) * 4;
-        v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (live && h < H) {
-          v[i] = *reinterpret_cast<const f32x4 *>(nrm.x + row + h);
-          if (nrm.residual) {
-            const f32x4 r = *reinterpret_cast<const f32x4 *>(nrm.residual + row + h);
-#pragma unroll
-            for (int q = 0; q < 4; q++) v[i][q] = __fadd_rn(v[i][q], r[q]);
-            *reinterpret_cast<f32x4 *>(nrm.x + row + h) = v[i];
-          }
-#pragma unroll
-          for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[i][q], v[i][q]);
-        }
-      }
-      for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
-      if (lane == 0) nred[grp][(threadIdx.x >> 6) & 3] = ss;
-      __syncthreads();
-      ss = nred[grp][0] + nred[grp][1] + nred[grp][2] + nred[grp][3];
-      ss /= H;
-      ss += 1e-5f;
-      const double inv = (double)(1.0f / sqrtf((float)ss));
-#pragma unroll
-      for (int i = 0; i < VPT; i++) {
-        const int h = (tg + 256 * i) * 4;
-        if (live && h < H) {
-          const f32x4 w = *reinterpret_cast<const f32x4 *>(nrm.weight + h);
-          f32x4 o;
-#pragma unroll
-          for (int q = 0; q < 4; q++) o[q] = (float)((double)w[q] * (inv * (double)v[i][q]));
-          const u32x2 pk = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-          *reinterpret_cast<u32x2 *>(nrm.t_out + row + h) = pk;
-          *reinterpret_cast<u32x2 *>(t_rows + (size_t)lr * H + h) = pk;
-        }
-      }
-      __syncthreads();   // nred is reused by the next pair of rows; after the last pair: t_rows complete
-    }
-    ap = t_rows + (size_t)(arow - r0) * H + kq;
-  }
-  f32x4 acc[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; nb++) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr int ROUTER_MAX_STEPS = router_steps(NB);
-  const int ksteps = H / 32;
-  for (int ks0 = wave; ks0 < ksteps; ks0 += ROUTER_WAVES * ROUTER_MAX_STEPS) {
-    u32x4 a[ROUTER_MAX_STEPS], b[ROUTER_MAX_STEPS][NB];
-#pragma unroll
-    for (int u = 0; u < ROUTER_MAX_STEPS; u++) {
-      const int ks = min(ks0 + u * ROUTER_WAVES, ksteps - 1);
-      a[u] = *reinterpret_cast<const u32x4 *>(ap + ks * 32);
-#pragma unroll
-      for (int nb = 0; nb < NB; nb++) {
-        int e = min(nb * 16 + (lane & 15), E - 1);
-        b[u][nb] = *reinterpret_cast<const u32x4 *>(wr + (size_t)e * H + ks * 32 + kq);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < ROUTER_MAX_STEPS; u++) {
-      if (ks0 + u * ROUTER_WAVES < ksteps) {
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++)
-          acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[u]), as_bf16x8(b[u][nb]), acc[nb], 0, 0, 0);
-      }
-    }
-  }
-#pragma unroll
-  for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) red[wave][(lane >> 4) * 4 + i][nb * 16 + (lane & 15)] = acc[nb][i];
-  __syncthreads();
-  // 32 lanes per token row: sum the partial products, add the bias, publish, gate
-  const int row = threadIdx.x >> 5, sub = threadIdx.x & 31;
-  const bool live = row < rows_per_wg && r0 + row < B;
-  constexpr int NJ = (NB + 1) / 2;
-  float v[NJ];
-#pragma unroll
-  for (int j = 0; j < NJ; j++) {
-    const int e = sub + 32 * j;
-    float x = -INFINITY;
-    if (e < E) {
-      x = 0.f;
-#pragma unroll
-      for (int w = 0; w < ROUTER_WAVES; w++) x += red[w][row][e];
-      if (br) x += br[e];
-      if (live) logits[(size_t)(r0 + row) * E + e] = x;
-    }
-    v[j] = x;
-  }
-  if (topk_w != nullptr) {
-    const size_t o = (size_t)(live ? r0 + row : 0) * k;
-    topk_softmax_group<NJ>(v, sub, E, k, live, topk_w + o, topk_i + o);
-  }
-}
-
-// ------------------------------------------------------------------------------------------------
-// Stand-alone gating from logits in memory: 32 lanes per token, two tokens per wave.
-// ------------------------------------------------------------------------------------------------
-template <int NJ, int KMAX = 8>
-__global__ __launch_bounds__(256) void topk_softmax_kernel(const float *__restrict__ logits, int B,
-                                                           int E, int k, float *__restrict__ topk_w,
-                                                           int *__restrict__ topk_i) {
-  const int sub = threadIdx.x & 31;
-  const int token = (blockIdx.x * 256 + threadIdx.x) >> 5;
-  const bool live = token < B;
-  const float *row = logits + (size_t)(live ? token : 0) * E;
-  float v[NJ];
-#pragma unroll
-  for (int j = 0; j < NJ; j++) {
-    int e = sub + 32 * j;
-    v[j] = (live && e < E) ? row[e] : -INFINITY;
-  }
-  const size_t o = (size_t)(live ? token : 0) * k;
-  topk_softmax_group<NJ, KMAX>(v, sub, E, k, live, topk_w + o, topk_i + o);
-}
-
-// ------------------------------------------------------------------------------------------------
-// Stable counting sort of P = B*k pairs by expert in ONE workgroup of 1024 threads (16 waves).
-// Each wave owns a contiguous range of pairs.  Inside a 64-pair step the lanes holding the same
-// expert are found with log2(E) ballots; the lowest such lane adds their count to the wave's own
-// LDS histogram row, so no atomics are needed and the order is the pair order (stable).
-// ------------------------------------------------------------------------------------------------
-constexpr int SORT_THREADS = 1024;
-constexpr int SORT_WAVES = SORT_THREADS / 64;
 
 __device__ __forceinline__ uint64_t same_expert_mask(int e, bool valid, int nbits) {
   uint64_t mask = __ballot(valid);
@@ -253,8 +81,6 @@ __device__ __forceinline__ uint64_t same_expert_mask(int e, bool valid, int nbit
   }
   return mask;
 }
-
-constexpr int SORT_CHUNK = 8;  // 64-pair steps whose expert ids a wave requests at once
 
 // Exclusive prefix sum over up to 256 values held 4 per lane by one wave (lane l owns entries
 // 4l..4l+3); returns the lane's own exclusive prefixes through ex[] and the grand total.
@@ -369,6 +195,254 @@ __device__ __forceinline__ void group_finish(const int *total, int *offs, int *c
     if (lane == 0) xcd_bounds[8] = n_tiles << 16;
   }
 }
+
+constexpr int ROUTER_GROUP_PAIRS = ROUTER_GROUP_TOKENS * 8;
+
+// Stable grouping of at most ROUTER_GROUP_PAIRS pairs by one wave: what group_sort_kernel writes for them.  No expert has
+// more than ROUTER_GROUP_TOKENS rows, so every expert that has any is one tile and a block of its own, and the work list
+// is cut into eight parts of equal length.
+__device__ __forceinline__ void group_by_one_wave(const int *topk_i, int P, int E, int *lds, const RouterGroup &g) {
+  int *total = lds, *offs = total + 256;   // [256] each
+  const int lane = threadIdx.x & 63;
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+  for (int i = 0; i < 4; i++) total[lane * 4 + i] = 0;
+  constexpr int STEPS = ROUTER_GROUP_PAIRS / 64;
+  int e[STEPS], rank[STEPS];
+#pragma unroll
+  for (int u = 0; u < STEPS; u++) {
+    if (u * 64 < P) {
+      const int p = u * 64 + lane;
+      const bool valid = p < P;
+      e[u] = valid ? topk_i[p] : 0;
+      const uint64_t mask = same_expert_mask(e[u], valid, g.nbits);
+      rank[u] = valid ? total[e[u]] + __popcll(mask & lt_mask) : 0;
+      // all lanes have read the counts before the lowest lane of each expert updates them (wave-ordered LDS operations)
+      if (valid && (mask & lt_mask) == 0) total[e[u]] += __popcll(mask);
+    }
+  }
+  // one scan for both prefixes: rows in the low half, experts with rows (= tiles) in the high half
+  int v[4], ex[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int c = total[lane * 4 + i];
+    v[i] = c | (c > 0 ? 1 << 16 : 0);
+  }
+  const int n_tiles = wave_scan4(v, ex) >> 16;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int x = lane * 4 + i, off = ex[i] & 0xffff, t = ex[i] >> 16;
+    offs[x] = off;
+    if (x <= E) g.expert_offsets[x] = off;
+    if (v[i]) {
+      int *tp = g.tiles + 1 + 3 * t;
+      tp[0] = x;
+      tp[1] = off;
+      tp[2] = v[i] & 0xffff;
+      g.xcd_bounds[XCD_BOUNDS_INTS + t] = (t << 8) | 1;
+    }
+  }
+  if (lane < 9) g.xcd_bounds[lane] = (lane * n_tiles) << 13;   // tile << 16 | fraction
+  if (lane == 0) g.tiles[0] = n_tiles;
+  if (lane == 0 && E == 256) g.expert_offsets[E] = P;
+#pragma unroll
+  for (int u = 0; u < STEPS; u++) {
+    const int p = u * 64 + lane;
+    if (p < P) {
+      const int dst = offs[e[u]] + rank[u];
+      g.sorted_pair_ids[dst] = p;
+      g.inv_perm[p] = dst;
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Router GEMM: logits[B,E] = t[B,H] . Wr[E,H]^T + br.  One workgroup = 16 token rows x all experts;
+// its 8 waves split the K loop (k-steps of 32, interleaved), request all their operands up front
+// and reduce through LDS.  With topk_w != nullptr the workgroup also gates its 16 tokens (32
+// lanes per token) while the logits are still in LDS.
+// ------------------------------------------------------------------------------------------------
+constexpr int ROUTER_WAVES = 8;
+// k-steps whose operands a wave requests before its first MFMA: as many as ~150 registers hold,
+// so that a hidden size of 2880 with up to 32 experts is a single round of loads
+constexpr int router_steps(int nb) { return nb <= 2 ? 12 : (nb <= 4 ? 7 : (nb <= 8 ? 4 : 2)); }
+
+// What the NORM form of the router kernel does first: x += residual, t = RMSNorm(x) * weight for the
+// workgroup's own token rows.
+struct RouterNorm {
+  float *x;               // [B,H] residual stream, updated in place
+  const float *residual;  // [B,H] or nullptr
+  const float *weight;    // [H]
+  bf16_t *t_out;          // [B,H]
+};
+
+// NB: number of 16-expert column blocks held per wave.  NORM: the workgroup first normalises its
+// rows (the arithmetic of rmsnorm_rows_kernel: 256 threads per row, the same element-to-thread
+// assignment and summation order, so t is the same to the bit), writes x and t to memory, keeps t in
+// LDS and multiplies from there: one launch and one read of t less than norm kernel + router kernel.
+template <int NB, bool NORM>
+__global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
+    const bf16_t *__restrict__ t, const bf16_t *__restrict__ wr, const float *__restrict__ br,
+    float *__restrict__ logits, int B, int H, int E, int k, float *__restrict__ topk_w,
+    int *__restrict__ topk_i, int rows_per_wg, RouterNorm nrm, RouterGroup grp) {
+  __shared__ float red[ROUTER_WAVES][16][NB * 16 + 1];
+  extern __shared__ __attribute__((aligned(16))) unsigned char t_rows_raw[];  // NORM: [rows_per_wg][H] bf16
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // rows_per_wg <= 16 token rows are this workgroup's; the other MFMA rows repeat the last of them
+  const int r0 = blockIdx.x * rows_per_wg;
+  const int arow = min(r0 + min(lane & 15, rows_per_wg - 1), B - 1);
+  const int kq = (lane >> 4) * 8;
+  const bf16_t *ap = t + (size_t)arow * H + kq;
+  constexpr int ROUTER_MAX_STEPS = router_steps(NB);
+  const int ksteps = H / 32;
+  u32x4 a[ROUTER_MAX_STEPS], b[ROUTER_MAX_STEPS][NB];
+  auto load_b = [&](int ks0) {
+#pragma unroll
+    for (int u = 0; u < ROUTER_MAX_STEPS; u++) {
+      const int ks = min(ks0 + u * ROUTER_WAVES, ksteps - 1);
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) {
+        int e = min(nb * 16 + (lane & 15), E - 1);
+        b[u][nb] = *reinterpret_cast<const u32x4 *>(wr + (size_t)e * H + ks * 32 + kq);
+      }
+    }
+  };
+  // the router's weights do not wait for the norm (more than 128 experts: no registers to hold them meanwhile)
+  constexpr bool EARLY = !NORM || NB <= 8;
+  if constexpr (EARLY) load_b(min(wave, ksteps - 1));
+  if constexpr (NORM) {
+    constexpr int VPT = 4;  // rows of up to 4096 floats
+    __shared__ double nred[2][4];
+    bf16_t *t_rows = reinterpret_cast<bf16_t *>(t_rows_raw);
+    const int grp = threadIdx.x >> 8, tg = threadIdx.x & 255;  // two groups of 256 threads, a row each
+    for (int rr = 0; rr < rows_per_wg; rr += 2) {
+      const int lr = rr + grp;
+      const bool live = lr < rows_per_wg && r0 + lr < B;
+      const size_t row = (size_t)(r0 + lr) * H;
+      f32x4 v[VPT];
+      double ss = 0.0;
+#pragma unroll
+      for (int i = 0; i < VPT; i++) {
+        const int h = (tg + 256 * i) * 4;
+        v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (live && h < H) {
+          v[i] = *reinterpret_cast<const f32x4 *>(nrm.x + row + h);
+          if (nrm.residual) {
+            const f32x4 r = *reinterpret_cast<const f32x4 *>(nrm.residual + row + h);
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[i][q] = __fadd_rn(v[i][q], r[q]);
+            *reinterpret_cast<f32x4 *>(nrm.x + row + h) = v[i];
+          }
+#pragma unroll
+          for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[i][q], v[i][q]);
+        }
+      }
+      for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+      if (lane == 0) nred[grp][(threadIdx.x >> 6) & 3] = ss;
+      __syncthreads();
+      ss = nred[grp][0] + nred[grp][1] + nred[grp][2] + nred[grp][3];
+      ss /= H;
+      ss += 1e-5f;
+      const double inv = (double)(1.0f / sqrtf((float)ss));
+#pragma unroll
+      for (int i = 0; i < VPT; i++) {
+        const int h = (tg + 256 * i) * 4;
+        if (live && h < H) {
+          const f32x4 w = *reinterpret_cast<const f32x4 *>(nrm.weight + h);
+          f32x4 o;
+#pragma unroll
+          for (int q = 0; q < 4; q++) o[q] = (float)((double)w[q] * (inv * (double)v[i][q]));
+          const u32x2 pk = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+          *reinterpret_cast<u32x2 *>(nrm.t_out + row + h) = pk;
+          *reinterpret_cast<u32x2 *>(t_rows + (size_t)lr * H + h) = pk;
+        }
+      }
+      __syncthreads();   // nred is reused by the next pair of rows; after the last pair: t_rows complete
+    }
+    ap = t_rows + (size_t)(arow - r0) * H + kq;
+  }
+  f32x4 acc[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; nb++) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int ks0 = wave; ks0 < ksteps; ks0 += ROUTER_WAVES * ROUTER_MAX_STEPS) {
+    if (!EARLY || ks0 != wave) load_b(ks0);
+#pragma unroll
+    for (int u = 0; u < ROUTER_MAX_STEPS; u++)
+      a[u] = *reinterpret_cast<const u32x4 *>(ap + min(ks0 + u * ROUTER_WAVES, ksteps - 1) * 32);
+#pragma unroll
+    for (int u = 0; u < ROUTER_MAX_STEPS; u++) {
+      if (ks0 + u * ROUTER_WAVES < ksteps) {
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++)
+          acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[u]), as_bf16x8(b[u][nb]), acc[nb], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) red[wave][(lane >> 4) * 4 + i][nb * 16 + (lane & 15)] = acc[nb][i];
+  __syncthreads();
+  // 32 lanes per token row: sum the partial products, add the bias, publish, gate
+  const int row = threadIdx.x >> 5, sub = threadIdx.x & 31;
+  const bool live = row < rows_per_wg && r0 + row < B;
+  constexpr int NJ = (NB + 1) / 2;
+  float v[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; j++) {
+    const int e = sub + 32 * j;
+    float x = -INFINITY;
+    if (e < E) {
+      x = 0.f;
+#pragma unroll
+      for (int w = 0; w < ROUTER_WAVES; w++) x += red[w][row][e];
+      if (br) x += br[e];
+      if (live) logits[(size_t)(r0 + row) * E + e] = x;
+    }
+    v[j] = x;
+  }
+  if (topk_w != nullptr) {
+    const size_t o = (size_t)(live ? r0 + row : 0) * k;
+    __shared__ int ids[ROUTER_GROUP_PAIRS];
+    topk_softmax_group<NJ>(v, sub, E, k, live, topk_w + o, topk_i + o, grp.expert_offsets ? ids + row * k : nullptr);
+    if (grp.expert_offsets != nullptr) {   // one workgroup holds every token
+      __syncthreads();
+      if (wave == 0) group_by_one_wave(ids, B * k, E, reinterpret_cast<int *>(&red[0][0][0]), grp);
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Stand-alone gating from logits in memory: 32 lanes per token, two tokens per wave.
+// ------------------------------------------------------------------------------------------------
+template <int NJ, int KMAX = 8>
+__global__ __launch_bounds__(256) void topk_softmax_kernel(const float *__restrict__ logits, int B,
+                                                           int E, int k, float *__restrict__ topk_w,
+                                                           int *__restrict__ topk_i) {
+  const int sub = threadIdx.x & 31;
+  const int token = (blockIdx.x * 256 + threadIdx.x) >> 5;
+  const bool live = token < B;
+  const float *row = logits + (size_t)(live ? token : 0) * E;
+  float v[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; j++) {
+    int e = sub + 32 * j;
+    v[j] = (live && e < E) ? row[e] : -INFINITY;
+  }
+  const size_t o = (size_t)(live ? token : 0) * k;
+  topk_softmax_group<NJ, KMAX>(v, sub, E, k, live, topk_w + o, topk_i + o);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Stable counting sort of P = B*k pairs by expert in ONE workgroup of 1024 threads (16 waves).
+// Each wave owns a contiguous range of pairs.  Inside a 64-pair step the lanes holding the same
+// expert are found with log2(E) ballots; the lowest such lane adds their count to the wave's own
+// LDS histogram row, so no atomics are needed and the order is the pair order (stable).
+// ------------------------------------------------------------------------------------------------
+constexpr int SORT_THREADS = 1024;
+constexpr int SORT_WAVES = SORT_THREADS / 64;
+
+constexpr int SORT_CHUNK = 8;  // 64-pair steps whose expert ids a wave requests at once
 
 __global__ __launch_bounds__(SORT_THREADS) void group_sort_kernel(
     const int *__restrict__ topk_i, int P, int E, int nbits, int *__restrict__ expert_offsets,
@@ -551,12 +625,14 @@ static int router_rows_per_wg(int B) {
 
 // logits (+ optional gating of the same tokens) in one launch
 int run_router(const void *t, const void *w_router, const float *b_router, float *logits, int B,
-               int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s) {
+               int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group) {
   // 16 token rows per workgroup fill the MFMA, but a thousand tokens are then only 64 workgroups;
   // with fewer rows each (the rest of the MFMA rows idle) all CUs take part in what is a
   // latency-bound launch: every workgroup reads the whole router matrix from L2 either way
   // (1024 tokens over 32 experts: 19.7 us with 16 rows, 16.7 with 8, 15.6 with 4, 27 with 2)
-  const int rows_per_wg = router_rows_per_wg(B);
+  const RouterGroup grp = group ? *group : RouterGroup{};
+  const int rows_per_wg = grp.expert_offsets ? ROUTER_GROUP_TOKENS : router_rows_per_wg(B);
+  GPTOSS_REQUIRE(!grp.expert_offsets || (topk_w && router_groups(B, k)), GPTOSS_ERR_DIM, "router: %d tokens are not grouped here", B);
   dim3 grid(cdiv(B, rows_per_wg)), block(ROUTER_WAVES * 64);
   const bf16_t *tp = (const bf16_t *)t, *wp = (const bf16_t *)w_router;
   int nb = cdiv(E, 16);
@@ -566,11 +642,11 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
     return rc != GPTOSS_OK ? rc : run_topk_softmax(logits, B, E, k, topk_w, topk_i, s);
   }
   TraceScope ts(topk_w ? "router_gemm_topk" : "router_gemm", s);
-  if (nb <= 1) router_gemm_kernel<1, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none);
-  else if (nb <= 2) router_gemm_kernel<2, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none);
-  else if (nb <= 4) router_gemm_kernel<4, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none);
-  else if (nb <= 8) router_gemm_kernel<8, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none);
-  else router_gemm_kernel<16, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none);
+  if (nb <= 1) router_gemm_kernel<1, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none, grp);
+  else if (nb <= 2) router_gemm_kernel<2, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none, grp);
+  else if (nb <= 4) router_gemm_kernel<4, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none, grp);
+  else if (nb <= 8) router_gemm_kernel<8, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none, grp);
+  else router_gemm_kernel<16, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none, grp);
   GPTOSS_LAUNCH_CHECK("router_gemm_kernel");
   return GPTOSS_OK;
 }
@@ -578,7 +654,8 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
 
 template <int NB>
 static int launch_norm_router(const RouterNorm &nrm, const bf16_t *wp, const float *b_router, float *logits, int B, int H,
-                              int E, int k, float *topk_w, int *topk_i, int rows_per_wg, size_t dyn, hipStream_t s) {
+                              int E, int k, float *topk_w, int *topk_i, int rows_per_wg, size_t dyn, hipStream_t s,
+                              const RouterGroup &grp) {
   // the kernel's LDS (router partial sums + the rows of t) exceeds what a launch gets by default
   constexpr int MAX_DEV = 64;
   static std::mutex mu;
@@ -597,7 +674,7 @@ static int launch_norm_router(const RouterNorm &nrm, const bf16_t *wp, const flo
   }
   TraceScope ts("norm_router_gemm_topk", s);
   hipLaunchKernelGGL(kern, dim3(cdiv(B, rows_per_wg)), dim3(ROUTER_WAVES * 64), dyn, s, nrm.t_out, wp, b_router, logits, B,
-                     H, E, k, topk_w, topk_i, rows_per_wg, nrm);
+                     H, E, k, topk_w, topk_i, rows_per_wg, nrm, grp);
   GPTOSS_LAUNCH_CHECK("router_gemm_kernel (with norm)");
   return GPTOSS_OK;
 }
@@ -605,7 +682,7 @@ static int launch_norm_router(const RouterNorm &nrm, const bf16_t *wp, const flo
 bool norm_router_applies(int B, int H, int E, const float *x, const float *residual, const float *weight,
                          const void *t_out) {
   const int nb = cdiv(E, 16) <= 1 ? 1 : cdiv(E, 16) <= 2 ? 2 : cdiv(E, 16) <= 4 ? 4 : cdiv(E, 16) <= 8 ? 8 : 16;
-  const size_t lds = (size_t)ROUTER_WAVES * 16 * (nb * 16 + 1) * 4 + (size_t)router_rows_per_wg(B) * H * 2 + 256;
+  const size_t lds = (size_t)ROUTER_WAVES * 16 * (nb * 16 + 1) * 4 + (size_t)router_rows_per_wg(B) * H * 2 + 640;   // (and the pair ids)
   // With more than four rows per workgroup (batches of more than ~1000 rows) the rows a workgroup
   // normalises one after the other cost more than the launch the fusion saves (8192 rows: 2.58 ms
   // per 24 layers against 2.23 ms for the two kernels; 1024 rows: 0.63 against 0.71 ms).
@@ -616,7 +693,10 @@ bool norm_router_applies(int B, int H, int E, const float *x, const float *resid
 // x += residual; t_out = RMSNorm(x) * weight; logits = t_out . Wr^T + br; gating: one launch
 int run_norm_router(float *x, const float *residual, const float *weight, void *t_out, const void *w_router,
                     const float *b_router, float *logits, int B, int H, int E, int k, float *topk_w, int *topk_i,
-                    hipStream_t s) {
+                    hipStream_t s, const RouterGroup *group) {
+  const RouterGroup grp = group ? *group : RouterGroup{};
+  GPTOSS_REQUIRE(!grp.expert_offsets || (router_groups(B, k) && B <= ROUTER_GROUP_NORM_TOKENS), GPTOSS_ERR_DIM,
+                 "norm + router: %d tokens are not grouped here", B);
   GPTOSS_REQUIRE(norm_router_applies(B, H, E, x, residual, weight, t_out), GPTOSS_ERR_DIM,
                  "norm + router: shape or alignment outside the fused kernel's range (H=%d E=%d)", H, E);
   const int rows_per_wg = router_rows_per_wg(B);
@@ -624,11 +704,11 @@ int run_norm_router(float *x, const float *residual, const float *weight, void *
   const bf16_t *wp = (const bf16_t *)w_router;
   const size_t dyn = (size_t)rows_per_wg * H * 2;
   const int nb = cdiv(E, 16);
-  if (nb <= 1) return launch_norm_router<1>(nrm, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, dyn, s);
-  if (nb <= 2) return launch_norm_router<2>(nrm, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, dyn, s);
-  if (nb <= 4) return launch_norm_router<4>(nrm, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, dyn, s);
-  if (nb <= 8) return launch_norm_router<8>(nrm, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, dyn, s);
-  return launch_norm_router<16>(nrm, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, dyn, s);
+  if (nb <= 1) return launch_norm_router<1>(nrm, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, dyn, s, grp);
+  if (nb <= 2) return launch_norm_router<2>(nrm, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, dyn, s, grp);
+  if (nb <= 4) return launch_norm_router<4>(nrm, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, dyn, s, grp);
+  if (nb <= 8) return launch_norm_router<8>(nrm, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, dyn, s, grp);
+  return launch_norm_router<16>(nrm, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, dyn, s, grp);
 }
 
 }  // namespace gptoss

@@ -68,3 +68,20 @@ def test_a_tile_list_of_one_expert_and_of_several_tiles(ops):
     want = layer.forward(t).clone()
     for tokens in (5, 33, 64, 70, 100):
         assert torch.equal(layer.forward(t[:tokens].contiguous()), want[:tokens]), tokens
+
+
+@pytest.mark.parametrize("E,k", [(1, 1), (4, 4), (8, 3), (32, 4), (40, 8), (128, 4), (256, 8)])
+@pytest.mark.parametrize("ties", [False, True])
+def test_grouping_of_a_few_tokens_equals_the_sorting_kernel(ops, E, k, ties):
+    """Up to 16 tokens are grouped by the router's own workgroup, beyond that by a kernel of its own."""
+    g = torch.Generator(device="cuda").manual_seed(E + k)
+    H = I = 64
+    router = _n(g, E, H) if not ties else torch.ones(E, H, device="cuda").bfloat16()   # ties: every expert scores the same
+    layer = ops.MoeLayer(router, torch.zeros(E, device="cuda"), _n(g, E, 2 * I, H), _n(g, E, 2 * I), _n(g, E, H, I),
+                         _n(g, E, H), top_k=k, max_tokens=32)
+    for tokens in (1, 2, 7, 15, 16, 17):
+        layer.forward(_n(g, tokens, H))
+        logits, w, i, off, srt, inv = layer.routing_views()
+        w2, i2, off2, srt2, inv2, _ = ops.moe_route(logits, k)
+        for got, want in ((w, w2), (i, i2), (off, off2), (srt, srt2), (inv, inv2)):
+            assert torch.equal(got, want), tokens
