@@ -195,13 +195,15 @@ int dense_gemm_mixed(const bf16_t *A, const bf16_t *W, float *out, const GemmBf1
                      int N, int K, hipStream_t s) {
   GPTOSS_REQUIRE(n_ranges >= 0 && n_ranges <= 2, GPTOSS_ERR_DIM, "dense_gemm_mixed: %d ranges", n_ranges);
   GemmParams g = dense_params(A, W, nullptr, out, B, N, K);
+  bool wide = true;   // rows that the 256-row kernel can write 16 bytes at a time
   for (int i = 0; i < n_ranges; i++) {
     g.range[i] = ranges[i];
+    wide = wide && ranges[i].ld % 8 == 0 && aligned(ranges[i].out, 16);
     GPTOSS_REQUIRE(ranges[i].from % 32 == 0 && ranges[i].to % 32 == 0 && ranges[i].ld % 4 == 0 && aligned(ranges[i].out, 8),
                    GPTOSS_ERR_DIM, "dense_gemm_mixed: ranges are whole 32-column blocks of aligned rows");
   }
   int rpt = dense_rows_per_tile(B, g.n_col_tiles, N, K, EPI_MIXED);
-  if (B >= dense_tall_min_rows() && gemm_tall_applies(g, false, EPI_MIXED) && gemm_tall_shape_ok(N, K, B)) rpt = 256;
+  if (B >= dense_tall_min_rows() && wide && gemm_tall_applies(g, false, EPI_MIXED) && gemm_tall_shape_ok(N, K, B)) rpt = 256;
   return run_gemm_dense(g, EPI_MIXED, rpt, cdiv(B, rpt), s);
 }
 

@@ -125,6 +125,15 @@ __device__ __forceinline__ void w_load(WRing<NRING, FP4> &ring, const WStream &s
   }
 }
 
+// gate * sigmoid(rate gate) * (up + shift) of the clamped pair; exp2 and the hardware reciprocal are accurate to a few
+// ulp of fp32, far inside the bf16 rounding of the result
+__device__ __forceinline__ float glu(const GluForm &f, float gate, float up) {
+  gate = fminf(gate, f.limit);
+  up = fminf(fmaxf(up, -f.limit), f.limit);
+  const float e = __builtin_amdgcn_exp2f(-f.rate * 1.4426950408889634f * gate);
+  return gate * __builtin_amdgcn_rcpf(1.0f + e) * (up + f.shift);
+}
+
 // Epilogue of one wave's 32-column block at column n0: MB accumulator blocks of 32 rows starting
 // at row0, of which `rows` are real (rows <= 0: nothing is stored).
 // The MFMAs take the W fragment as their first operand, i.e. they compute the transposed tile:
@@ -165,7 +174,6 @@ __device__ __forceinline__ void epilogue_rows(const GemmParams &p, int row0, int
     // address = wave-uniform base (scalar registers) + a 32-bit per-lane element offset
     bf16_t *o = reinterpret_cast<bf16_t *>(p.out) + (size_t)row0 * half_n + (n0 >> 1);
     const uint32_t lane_off = (uint32_t)tok * (uint32_t)half_n + (uint32_t)h4;
-    const float L = p.glu.limit, shift = p.glu.shift, rate = -p.glu.rate * 1.4426950408889634f;
     const int row_lim = rows - tok;  // block i of this lane is a real row iff i*32 < row_lim
 #pragma unroll
     for (int i = 0; i < MB; i++) {
@@ -176,14 +184,7 @@ __device__ __forceinline__ void epilogue_rows(const GemmParams &p, int row0, int
           float v[4];
 #pragma unroll
           for (int q = 0; q < 4; q++) {
-            float gate = acc[i][g * 4 + q] + bg[g * 4 + q];
-            float up = acc[i][(g + 2) * 4 + q] + bu[g * 4 + q];
-            gate = fminf(gate, L);
-            up = fminf(fmaxf(up, -L), L);
-            // gate * sigmoid(rate gate) * (up + shift); exp2 and the hardware reciprocal are accurate
-            // to a few ulp of fp32, far inside the bf16 rounding of the result
-            const float e = __builtin_amdgcn_exp2f(rate * gate);
-            v[q] = gate * __builtin_amdgcn_rcpf(1.0f + e) * (up + shift);
+            v[q] = glu(p.glu, acc[i][g * 4 + q] + bg[g * 4 + q], acc[i][(g + 2) * 4 + q] + bu[g * 4 + q]);
           }
           const u32x2 pk = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
           if (hold) *reinterpret_cast<u32x2 *>(hold + (i * 32 + tok) * HOLD_ROW + hold_col + h4 + g * 8) = pk;

@@ -79,6 +79,107 @@ struct TallSrc {
   int mat, row0, rows, ct;
 };
 
+// Epilogue of a wave's CB x RB blocks.  A lane holds one row and four consecutive columns per register quad, so stored
+// from where they lie an instruction's 64 pieces of 16 bytes go to 32 rows, and with a row of a multiple of 4 KB (8192
+// or 16384 columns) to one and the same memory channel.  fp32 and bf16 columns go through LDS instead, 32 rows of a
+// column block at a time, and leave in whole lines: 8000 x 8192 x 2048 262 -> 236 us, 8192 x 16384 x 2048 678 -> 490,
+// 8192 x 5120 x 2880 235 -> 222.  (Not the gated form: rows of a quarter of the bytes, and its biases read once per row
+// block instead of once cost more than the stores gain: block of 5999 tokens 1318 -> 1403 us.)
+// buf: 8 KB of the A buffer that the next item's first stage fills again.  It is the part that this wave's own loads go
+// to, and they are issued after its reads here; the other waves read it after a barrier.  Pieces of 16 bytes are
+// XOR-swizzled by their row.
+template <class SH, int EPI>
+__device__ __forceinline__ void tall_epilogue(const GemmParams &p, unsigned char *buf, int mat, int row0, int rows, int c0,
+                                              int lane, f32x16 (&acc)[SH::CB][SH::RB]) {
+  constexpr int RB = SH::RB, CB = SH::CB;
+  static_assert(SH::LA * 1024 >= 32 * 128, "32 rows of a column block in fp32");
+  const int N = p.N, tok = lane & 31, h = lane >> 5;
+  const const_as<float> bp = constant_ptr(p.bias ? p.bias + (size_t)mat * N + c0 : nullptr);
+  // a row of the staged block is P pieces of 16 bytes
+  auto put = [&](auto pieces, int piece, auto v) {
+    constexpr int P = decltype(pieces)::value;
+    unsigned char *d = buf + tok * (P * 16) + ((piece ^ (tok & (P - 1))) << 4);
+    if constexpr (sizeof(v) == 8) d += h * 8;   // two lanes share a piece
+    *reinterpret_cast<decltype(v) *>(d) = v;
+  };
+  // rows r * 32 .. of the tile: `width` 16-byte pieces of them are real, out = first byte of the first row
+  auto flush = [&](auto pieces, int r, int width, unsigned char *out, size_t ld) {
+    constexpr int P = decltype(pieces)::value, PER = 64 / P;   // rows of a store instruction
+#pragma unroll
+    for (int i = 0; i < 32 / PER; i++) {
+      const int row = i * PER + lane / P, piece = lane % P;
+      const u32x4 v = *reinterpret_cast<const u32x4 *>(buf + row * (P * 16) + ((piece ^ (row & (P - 1))) << 4));
+      if (r * 32 + row < rows && piece < width) *reinterpret_cast<u32x4 *>(out + (size_t)(r * 32 + row) * ld + piece * 16) = v;
+    }
+  };
+  // the compiler copies accumulators out of their AGPRs early, and spills, unless they are pinned until they are used
+  auto pin = [&](int i, int r) { asm volatile("" : "+a"(acc[i][r])); };
+  using P8 = std::integral_constant<int, 8>;
+  using P4 = std::integral_constant<int, 4>;
+  if constexpr (EPI == EPI_SWIGLU) {
+#pragma unroll
+    for (int i = 0; i < CB; i++) {
+#pragma unroll
+      for (int r = 0; r < RB; r++) pin(i, r);
+      if (c0 + i * 32 < N) epilogue_store<RB, EPI, true>(p, mat, row0, rows, c0 + i * 32, lane, acc[i]);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < CB; i++) {
+      const int n0 = c0 + i * 32;
+#pragma unroll
+      for (int r = 0; r < RB; r++) pin(i, r);
+      if (n0 < N) {
+        float bv[16];
+#pragma unroll
+        for (int x = 0; x < 16; x++) {
+          const int c = i * 32 + (x >> 2) * 8 + (x & 3);
+          const float lo = bp ? bp[c] : 0.f, hi = bp ? bp[c + 4] : 0.f;
+          bv[x] = h ? hi : lo;
+        }
+        bool half = false;
+        GemmBf16Range to;
+        if constexpr (EPI == EPI_MIXED) {
+          const bool in0 = n0 >= p.range[0].from && n0 < p.range[0].to, in1 = n0 >= p.range[1].from && n0 < p.range[1].to;
+          half = in0 || in1;
+          to.from = in1 ? p.range[1].from : p.range[0].from;
+          to.out = in1 ? p.range[1].out : p.range[0].out;
+          to.ld = in1 ? p.range[1].ld : p.range[0].ld;
+          to.relu_squared = in1 ? p.range[1].relu_squared : p.range[0].relu_squared;
+        }
+        if (EPI == EPI_MIXED && half) {
+#pragma unroll
+          for (int r = 0; r < RB; r++) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+              float v[4];
+#pragma unroll
+              for (int q = 0; q < 4; q++) {
+                v[q] = acc[i][r][g * 4 + q] + bv[g * 4 + q];
+                if (to.relu_squared) {
+                  v[q] = fmaxf(v[q], 0.f);
+                  v[q] *= v[q];
+                }
+              }
+              put(P4{}, g, u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])});
+            }
+            flush(P4{}, r, 4, reinterpret_cast<unsigned char *>(to.out + (size_t)row0 * to.ld + (n0 - to.from)), (size_t)to.ld * 2);
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < RB; r++) {
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+              put(P8{}, g * 2 + h, f32x4{acc[i][r][g * 4] + bv[g * 4], acc[i][r][g * 4 + 1] + bv[g * 4 + 1],
+                                         acc[i][r][g * 4 + 2] + bv[g * 4 + 2], acc[i][r][g * 4 + 3] + bv[g * 4 + 3]});
+            flush(P8{}, r, 8, reinterpret_cast<unsigned char *>(p.out) + ((size_t)row0 * N + n0) * 4, (size_t)N * 4);
+          }
+        }
+      }
+    }
+  }
+}
+
 template <class SH, bool GATHER, int EPI>
 __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p) {
   constexpr int RB = SH::RB, CB = SH::CB, LW = SH::LW, LA = SH::LA, LW1 = SH::LW / 2, LA1 = SH::LA / 4;
@@ -126,8 +227,13 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
       tile = work / p.n_col_tiles;
       t.ct = work - tile * p.n_col_tiles;
     } else {
-      t.ct = work / n_tiles;
-      tile = work - t.ct * n_tiles;
+      // dense: blocks of eight row tiles are walked column tile by column tile, so that what an XCD's 32 workgroups read
+      // at a time are the rows of eight tiles and the weights of four, not of 32 and one (8000 x 8192 x 2048: 315 -> 262
+      // us, 8192 x 16384 x 2048: 806 -> 678, 8192 x 5120 x 2880: 241 -> 235)
+      const int grp = work / (8 * p.n_col_tiles), v = work - grp * 8 * p.n_col_tiles;
+      const int th = min(8, n_tiles - grp * 8);
+      t.ct = v / th;
+      tile = grp * 8 + (v - t.ct * th);
     }
     if (p.tiles) {
       t.mat = tiles[1 + 3 * tile];
@@ -361,15 +467,9 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
         }
       }
     } else {
-#pragma unroll
-      for (int i = 0; i < CB; i++) {
-#pragma unroll
-        for (int r = 0; r < RB; r++) asm volatile("" : "+a"(acc[i][r]));
-        const int n0 = cur.ct * SH::BN + (wc * CB + i) * 32;
-        if (n0 < N)
-          epilogue_store<RB, EPI, true>(p, cur.mat, cur.row0 + wr * RB * 32, cur.rows - wr * RB * 32, n0, lane,
-                                        acc[i]);
-      }
+      unsigned char *buf = lds + SH::A_OFF + (ab == 0 ? 2 : ab - 1) * SH::A_BYTES + w * LA * 1024;
+      tall_epilogue<SH, EPI>(p, buf, cur.mat, cur.row0 + wr * RB * 32, cur.rows - wr * RB * 32,
+                             cur.ct * SH::BN + wc * CB * 32, lane, acc);
     }
     if (!more) break;
     j = jn;
