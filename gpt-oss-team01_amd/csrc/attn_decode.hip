@@ -41,6 +41,59 @@ namespace gptoss {
 constexpr int ATT_BLOCK = 64;   // slots per inner iteration
 constexpr float NEG_BIG = -1.0e30f;
 
+// The hardware's exponential by itself: a weight below 2^-126 of its row's largest is zero.  (The library function scales
+// such arguments first, five more instructions per score where a block step has about 300 in all; a row's largest weight
+// is 1, so a sum in fp32 is the same with them or without.)
+__device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// A score's weight against the running maximum m (in powers of two).  Scaling and difference are one fused operation, in
+// every form of the kernels and in blocks with and without masked slots alike: a row's result must not depend on what
+// its partner row in a wave forces.
+__device__ __forceinline__ float weight_of(float score, float scale, float m) {
+  return exp2_hw(__builtin_fmaf(score, scale, -m));
+}
+
+// The largest value of the four lanes n, n + 16, n + 32, n + 48, in all of them, without a trip through LDS.
+__device__ __forceinline__ float max_over_quarters(float v) {
+  const uint32_t u = __float_as_uint(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const float m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const uint32_t w = __float_as_uint(m);
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// Two weights in [0, 1] as bf16 hi + lo parts: truncation to bf16 plus the truncated remainder keeps 16 mantissa bits.
+__device__ __forceinline__ void split_weights(float p0, float p1, uint32_t &h, uint32_t &l) {
+  const uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
+  h = __builtin_amdgcn_perm(u1, u0, 0x07060302u);   // the upper halves
+  const float r0 = p0 - __uint_as_float(u0 & 0xffff0000u), r1 = p1 - __uint_as_float(u1 & 0xffff0000u);
+  l = __builtin_amdgcn_perm(__float_as_uint(r1), __float_as_uint(r0), 0x07060302u);
+}
+
+// A lane's KS * 8 values of a query row as bf16 hi + lo operands; a column without a row or head is zero.  qp points to a
+// real row whether the column has one or not, so that the loads are whole and unconditional (sixteen conditional ones of
+// four bytes: 64 prompts of 125 positions 104 instead of 73 us, eight of 1000 195 instead of 181).
+template <int KS>
+__device__ __forceinline__ void split_query(const float *qp, bool live, bf16x8 (&qh)[KS], bf16x8 (&ql)[KS]) {
+  f32x4 x[2 * KS];
+#pragma unroll
+  for (int i = 0; i < 2 * KS; i++) x[i] = *reinterpret_cast<const f32x4 *>(qp + i * 4);
+#pragma unroll
+  for (int s = 0; s < KS; s++) {
+    uint32_t h[4], l[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float x0 = live ? x[2 * s + (j >> 1)][(j & 1) * 2] : 0.f, x1 = live ? x[2 * s + (j >> 1)][(j & 1) * 2 + 1] : 0.f;
+      const bf16_t h0 = f32_to_bf16(x0), h1 = f32_to_bf16(x1);
+      h[j] = (uint32_t)h0 | ((uint32_t)h1 << 16);
+      l[j] = pack_bf16x2(x0 - bf16_to_f32(h0), x1 - bf16_to_f32(h1));
+    }
+    qh[s] = as_bf16x8(u32x4{h[0], h[1], h[2], h[3]});
+    ql[s] = as_bf16x8(u32x4{l[0], l[1], l[2], l[3]});
+  }
+}
+
 struct AttnParams {
   const float *q;      // [B, n_q, D]
   const bf16_t *kv;    // [B, n_kv, cap/64] blocks of K [64, D] + V [2, D/16, 64, 8]
@@ -278,24 +331,8 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
   using R1 = std::integral_constant<int, 1>;
   if (c1 > c0) load_kv(c0, R0{});
 
-  // ---- Q^T operand, split into bf16 hi and lo parts -----------------------------------------
   bf16x8 qh[KS], ql[KS];
-  {
-    const float *qp = p.q + ((size_t)bn * p.n_q + head) * D + c * KS * 8;
-#pragma unroll
-    for (int s = 0; s < KS; s++) {
-      uint32_t h[4], l[4];
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        float x0 = col_live ? qp[s * 8 + 2 * j] : 0.f, x1 = col_live ? qp[s * 8 + 2 * j + 1] : 0.f;
-        bf16_t h0 = f32_to_bf16(x0), h1 = f32_to_bf16(x1);
-        h[j] = (uint32_t)h0 | ((uint32_t)h1 << 16);
-        l[j] = pack_bf16x2(x0 - bf16_to_f32(h0), x1 - bf16_to_f32(h1));
-      }
-      qh[s] = as_bf16x8(u32x4{h[0], h[1], h[2], h[3]});
-      ql[s] = as_bf16x8(u32x4{l[0], l[1], l[2], l[3]});
-    }
-  }
+  split_query<KS>(p.q + ((size_t)bn * p.n_q + head) * D + c * KS * 8, col_live, qh, ql);
 
   f32x4 o[DB];
 #pragma unroll
@@ -322,28 +359,20 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
       }
       s4[tb] = acc;
     }
-    float bmax = NEG_BIG;
+    float bmax = -INFINITY;   // of the scores as they leave the product
 #pragma unroll
     for (int tb = 0; tb < 4; tb++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        float v = s4[tb][i] * p.scale_log2e;
-        // keep the product a rounded value of its own in both variants of this block (the unmasked
-        // one would otherwise fuse it into the subtraction below): a row's result must not depend
-        // on which variant its partner row forces
-        asm volatile("" : "+v"(v));
         if (EDGE) {
           const int slot = blk + tb * 16 + c * 4 + i;
           const bool ok = PAIR ? (slot >= lane_lo && slot < lane_hi) : (slot < c1 && slot_pos(slot) >= r.t_lo);
-          v = ok ? v : -INFINITY;
+          s4[tb][i] = ok ? s4[tb][i] : -INFINITY;
         }
-        s4[tb][i] = v;
-        bmax = fmaxf(bmax, v);
+        bmax = fmaxf(bmax, s4[tb][i]);
       }
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
-    const float m_new = fmaxf(m_run, bmax);
-    const float alpha = exp2f(m_run - m_new);
+    const float m_new = fmaxf(m_run, max_over_quarters(bmax) * p.scale_log2e);
+    const float alpha = exp2_hw(m_run - m_new);
     m_run = m_new;
     float psum = 0.f;
     bf16x8 ph[2], pl[2];
@@ -353,14 +382,10 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         // operand k index (c, jj): jj<4 -> slot c*4+jj of the first 16, jj>=4 -> of the second 16
-        float p0 = exp2f(s4[grp * 2 + (j >> 1)][(j & 1) * 2] - m_new);
-        float p1 = exp2f(s4[grp * 2 + (j >> 1)][(j & 1) * 2 + 1] - m_new);
+        float p0 = weight_of(s4[grp * 2 + (j >> 1)][(j & 1) * 2], p.scale_log2e, m_new);
+        float p1 = weight_of(s4[grp * 2 + (j >> 1)][(j & 1) * 2 + 1], p.scale_log2e, m_new);
         psum += p0 + p1;
-        // p is in [0,1]: truncation to bf16 plus the bf16 remainder keeps 16 mantissa bits
-        uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
-        h[j] = (u0 >> 16) | (u1 & 0xffff0000u);
-        float r0 = p0 - __uint_as_float(u0 & 0xffff0000u), r1 = p1 - __uint_as_float(u1 & 0xffff0000u);
-        l[j] = (__float_as_uint(r0) >> 16) | (__float_as_uint(r1) & 0xffff0000u);
+        split_weights(p0, p1, h[j], l[j]);
       }
       ph[grp] = as_bf16x8(u32x4{h[0], h[1], h[2], h[3]});
       pl[grp] = as_bf16x8(u32x4{l[0], l[1], l[2], l[3]});
@@ -450,11 +475,11 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
     float M = sink2;
 #pragma unroll
     for (int w = 0; w < 4; w++) M = fmaxf(M, lds_ml[(w * 16 + hm) * 2]);
-    float denom = exp2f(sink2 - M);
+    float denom = exp2_hw(sink2 - M);
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < 4; w++) {
-      const float wgt = exp2f(lds_ml[(w * 16 + hm) * 2] - M);
+      const float wgt = exp2_hw(lds_ml[(w * 16 + hm) * 2] - M);
       denom += lds_ml[(w * 16 + hm) * 2 + 1] * wgt;
       const f32x4 ow = *reinterpret_cast<const f32x4 *>(&lds_o[(w * 16 + hm) * D + d4]);
 #pragma unroll
@@ -472,8 +497,8 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
   if (row_chunks == 1) {
     float sink2 = sink_logit * 1.4426950408889634f;  // lanes that get here have head == hq
     float M = fmaxf(m_run, sink2);
-    float w = exp2f(m_run - M);
-    float denom = l_run * w + exp2f(sink2 - M);
+    float w = exp2_hw(m_run - M);
+    float denom = l_run * w + exp2_hw(sink2 - M);
     float inv = (denom > 0.f) ? w / denom : 0.f;
     bf16_t *op = HOLD ? hold + hn * D : p.out + ((size_t)bn * p.n_q + hq) * D;
     if (HOLD && lane == 0) *hold_row = b * p.n_q + g * G;
@@ -588,7 +613,7 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 #pragma unroll
     for (int u = 0; u < ATT_RED_UNROLL; u++) M = fmaxf(M, m[u]);
   }
-  float denom = exp2f(sink2 - M);
+  float denom = exp2_hw(sink2 - M);
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int c0 = 0; c0 < r.nchunks; c0 += ATT_RED_UNROLL) {
     float m[ATT_RED_UNROLL], l[ATT_RED_UNROLL];
@@ -605,7 +630,7 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 #pragma unroll
     for (int u = 0; u < ATT_RED_UNROLL; u++) {
       if (c0 + u < r.nchunks) {
-        const float w = exp2f(m[u] - M);
+        const float w = exp2_hw(m[u] - M);
         denom += l[u] * w;
 #pragma unroll
         for (int q = 0; q < 4; q++) acc[q] += o[u][q] * w;
@@ -622,13 +647,24 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 // and walks the K/V blocks any of them needs ONCE: every block goes from global memory into LDS
 // (two buffers, one barrier per block) and the eight waves take their operands from there.  The
 // pair form reads a sequence's cache once per row pair, which is quadratic traffic for long
-// prompts; here it is read once per 16 rows, and the pass is bound by the matrix instructions.
+// prompts; here it is read once per 16 rows.  What bounds it is the vector units (70 % busy, the matrix cores 34 %): per
+// 64 x 16 scores a wave issues about 170 of their instructions, a tenth of them exponentials.  Eight prompts of 1000
+// positions, 64 heads: 237 -> 211 us with the exponential, the maximum and the splitting of weights in fewer instructions
+// (exp2_hw, max_over_quarters, split_weights), -> 195 with the scale fused into the exponent's difference (weight_of),
+// one range check per masked slot and blocks straight into LDS, -> 181 with whole loads of q (split_query).
 // Every row sees the arithmetic of the one-wave kernel over its own blocks in ascending order (a
 // block outside a row's range is a no-op for its columns), so rows of up to ATT_CHUNK positions
 // equal the decode call bit for bit; longer rows are summed in one pass instead of chunk by
 // chunk.  Needs slot == position (no wrapped ring) and at most 8 query heads per kv head.
 constexpr int TILE_WAVES = 8;
 constexpr int TILE_ROWS = 2 * TILE_WAVES;
+
+// 16 bytes per lane, from sbase + voff to LDS address lds + 16 * lane
+__device__ __forceinline__ void load_to_lds(unsigned lds, uint32_t voff, const void *sbase) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
+               "v"(voff), "s"(sbase)
+               : "memory");
+}
 
 template <int D>
 __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(AttnParams p) {
@@ -676,58 +712,38 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
   const int cache_seq = p.seq_map ? __builtin_amdgcn_readfirstlane(p.seq_map[seq]) : seq;
   const unsigned char *plane =
       reinterpret_cast<const unsigned char *>(p.kv + kv_block_off(cache_seq, g, p.n_kv, p.cap, D, 0));
-  // the workgroup's copy of a block: piece i of thread t is bytes (i * 512 + t) * 16; a K piece is
-  // chunk j of row r and lands at chunk position j ^ swz(r) of its row, so that the 16 lanes of a
-  // fragment read (16 rows, one chunk) hit 16 different 16-byte slots modulo 256 bytes
+  // The workgroup's copy of a block goes from memory straight into LDS, in pieces of 16 bytes: thread t's load i lands at
+  // piece i * 512 + t.  Position j of K row r is to hold chunk j ^ swz(r), so that the 16 lanes of a fragment read (16
+  // rows, one chunk) hit 16 different 16-byte slots modulo 256 bytes: the lane fetches that chunk.  (Through registers,
+  // the loop's eight of them and the store's addresses do not fit the 128 of two workgroups per CU beside the rest.)
   auto swz = [](int r) { return D == 64 ? ((r >> 1) & 7) : ((r >> 2) & 3); };
-  u32x4 stage[PASSES];
-  auto load_block = [&](int blk) {
+  uint32_t src_off[PASSES];
+#pragma unroll
+  for (int i = 0; i < PASSES; i++) {
+    const int piece = i * TILE_WAVES * 64 + tid, r = piece / ROW_CHUNKS, j = piece % ROW_CHUNKS;
+    src_off[i] = (piece * 16 < K_BYTES ? r * ROW_CHUNKS + (j ^ swz(r)) : piece) * 16;
+  }
+  const unsigned lds_base =
+      __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)&lds[0][0]);
+  auto request_block = [&](int blk, int buf) {
     const unsigned char *src = plane + (size_t)(blk >> 6) * BLOCK_BYTES;
 #pragma unroll
     for (int i = 0; i < PASSES; i++)
-      stage[i] = *reinterpret_cast<const u32x4 *>(src + (size_t)(i * TILE_WAVES * 64 + tid) * 16);
+      load_to_lds(lds_base + buf * BLOCK_BYTES + (i * TILE_WAVES + wave) * 1024, src_off[i], src);
   };
-  auto store_block = [&](int buf) {
-    // the destination is recomputed at every block from a thread id the optimiser cannot see through:
-    // hoisted out of the loop it costs a register that the 128-register budget of two workgroups per
-    // CU does not have, and a spilled register's reload in the loop waits for the block in flight
-    int t_opaque = tid;
-    asm volatile("" : "+v"(t_opaque));
-#pragma unroll
-    for (int i = 0; i < PASSES; i++) {
-      const int piece = i * TILE_WAVES * 64 + t_opaque;
-      int dst = piece * 16;
-      if (piece * 16 < K_BYTES) {
-        const int r = piece / ROW_CHUNKS, j = piece % ROW_CHUNKS;
-        dst = r * (D * 2) + ((j ^ swz(r)) << 4);
-      }
-      *reinterpret_cast<u32x4 *>(&lds[buf][dst]) = stage[i];
-    }
-  };
-  if (blk_end > blk_begin) load_block(blk_begin);
+  if (blk_end > blk_begin) request_block(blk_begin, 0);
 
   bf16x8 qh[KS], ql[KS];
-  {
-    const float *qp = p.q + ((size_t)bn * p.n_q + head) * D + c * KS * 8;
-#pragma unroll
-    for (int s = 0; s < KS; s++) {
-      uint32_t h[4], l[4];
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        float x0 = col_live ? qp[s * 8 + 2 * j] : 0.f, x1 = col_live ? qp[s * 8 + 2 * j + 1] : 0.f;
-        bf16_t h0 = f32_to_bf16(x0), h1 = f32_to_bf16(x1);
-        h[j] = (uint32_t)h0 | ((uint32_t)h1 << 16);
-        l[j] = pack_bf16x2(x0 - bf16_to_f32(h0), x1 - bf16_to_f32(h1));
-      }
-      qh[s] = as_bf16x8(u32x4{h[0], h[1], h[2], h[3]});
-      ql[s] = as_bf16x8(u32x4{l[0], l[1], l[2], l[3]});
-    }
-  }
+  split_query<KS>(p.q + ((size_t)bn * p.n_q + head) * D + c * KS * 8, col_live, qh, ql);
+
   f32x4 o[DB];
 #pragma unroll
   for (int db = 0; db < DB; db++) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_run = NEG_BIG, l_run = 0.f;
-  const int lane_lo = second ? lo1 : lo0, lane_hi = second ? hi1 : hi0;
+  const int lane_lo = second ? lo1 : lo0;
+  const uint32_t lane_n = (second ? hi1 : hi0) - lane_lo;
+  const int any_lo = lo0;
+  const uint32_t any_n = (two ? hi1 : hi0) - any_lo;
 
   // one 64-slot block from LDS buffer `buf`: the arithmetic of the one-wave kernel's block step
   auto process = [&](int blk, int buf, auto edge_sel) {
@@ -747,24 +763,21 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
       }
       s4[tb] = acc;
     }
-    float bmax = NEG_BIG;
+    // the lane's first slot of the block, within its row's range and within either row's; derived per block from an opaque
+    // thread index, as the compiler would keep what it can compute ahead in registers that the loop does not have
+    int tid_here = tid;
+    if (EDGE) asm volatile("" : "+v"(tid_here));
+    const int slot0 = blk + ((tid_here & 63) >> 4) * 4, s0 = slot0 - lane_lo, a0 = slot0 - any_lo;
+    float bmax = -INFINITY;   // of the scores as they leave the product
 #pragma unroll
     for (int tb = 0; tb < 4; tb++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        float v = s4[tb][i] * p.scale_log2e;
-        asm volatile("" : "+v"(v));   // a rounded product of its own, as in the one-wave kernel
-        if (EDGE) {
-          const int slot = blk + tb * 16 + c * 4 + i;
-          v = (slot >= lane_lo && slot < lane_hi) ? v : -INFINITY;
-        }
-        s4[tb][i] = v;
-        bmax = fmaxf(bmax, v);
+        if (EDGE) s4[tb][i] = (uint32_t)(s0 + tb * 16 + i) < lane_n ? s4[tb][i] : -INFINITY;
+        bmax = fmaxf(bmax, s4[tb][i]);
       }
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
-    const float m_new = fmaxf(m_run, bmax);
-    const float alpha = exp2f(m_run - m_new);
+    const float m_new = fmaxf(m_run, max_over_quarters(bmax) * p.scale_log2e);
+    const float alpha = exp2_hw(m_run - m_new);
     m_run = m_new;
     float psum = 0.f;
     bf16x8 ph[2], pl[2];
@@ -773,13 +786,10 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
       uint32_t h[4], l[4];
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        float p0 = exp2f(s4[grp * 2 + (j >> 1)][(j & 1) * 2] - m_new);
-        float p1 = exp2f(s4[grp * 2 + (j >> 1)][(j & 1) * 2 + 1] - m_new);
+        float p0 = weight_of(s4[grp * 2 + (j >> 1)][(j & 1) * 2], p.scale_log2e, m_new);
+        float p1 = weight_of(s4[grp * 2 + (j >> 1)][(j & 1) * 2 + 1], p.scale_log2e, m_new);
         psum += p0 + p1;
-        uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
-        h[j] = (u0 >> 16) | (u1 & 0xffff0000u);
-        float r0 = p0 - __uint_as_float(u0 & 0xffff0000u), r1 = p1 - __uint_as_float(u1 & 0xffff0000u);
-        l[j] = (__float_as_uint(r0) >> 16) | (__float_as_uint(r1) & 0xffff0000u);
+        split_weights(p0, p1, h[j], l[j]);
       }
       ph[grp] = as_bf16x8(u32x4{h[0], h[1], h[2], h[3]});
       pl[grp] = as_bf16x8(u32x4{l[0], l[1], l[2], l[3]});
@@ -798,9 +808,9 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
         if (EDGE) {
 #pragma unroll
           for (int w = 0; w < 4; w++) {
-            const int s_lo = blk + grp * 32 + (w >> 1) * 16 + c * 4 + (w & 1) * 2;
-            auto used = [&](int sl) { return (sl >= lo0 && sl < hi0) || (sl >= lo1 && sl < hi1); };
-            const uint32_t keep = (used(s_lo) ? 0x0000ffffu : 0u) | (used(s_lo + 1) ? 0xffff0000u : 0u);
+            // the two rows are neighbours: what either of them sees is one range
+            const uint32_t sl = a0 + grp * 32 + (w >> 1) * 16 + (w & 1) * 2;
+            const uint32_t keep = (sl < any_n ? 0x0000ffffu : 0u) | (sl + 1 < any_n ? 0xffff0000u : 0u);
             vv[w] &= keep;
           }
         }
@@ -812,9 +822,12 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
 
   int buf = 0;
   for (int blk = blk_begin; blk < blk_end; blk += ATT_BLOCK, buf ^= 1) {
-    store_block(buf);
-    __syncthreads();   // block `blk` is complete in lds[buf]; every wave is done with the other buffer's previous use
-    if (blk + ATT_BLOCK < blk_end) load_block(blk + ATT_BLOCK);
+    // Block `blk` is complete in lds[buf] once every wave's loads of it have landed, and behind the barrier every wave is
+    // done with the other buffer.  (The compiler does not count these loads; the loop has no others.)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (blk + ATT_BLOCK < blk_end) request_block(blk + ATT_BLOCK, buf ^ 1);
     // the wave's rows: first block that holds an active position of either row .. their last one
     const bool mine = (have0 && blk < hi0 && blk + ATT_BLOCK > lo0) || (two && blk < hi1 && blk + ATT_BLOCK > lo1);
     if (mine) {
@@ -830,8 +843,8 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
   const int hq = g * G + hn;
   const float sink2 = sink_logit * 1.4426950408889634f;
   const float M = fmaxf(m_run, sink2);
-  const float w = exp2f(m_run - M);
-  const float denom = l_run * w + exp2f(sink2 - M);
+  const float w = exp2_hw(m_run - M);
+  const float denom = l_run * w + exp2_hw(sink2 - M);
   const float inv = (denom > 0.f) ? w / denom : 0.f;
   bf16_t *op = p.out + ((size_t)bn * p.n_q + hq) * D;
 #pragma unroll
