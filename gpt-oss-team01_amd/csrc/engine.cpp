@@ -9,6 +9,9 @@ using namespace gptoss;
 gptoss_engine::~gptoss_engine() {
   for (void *p : allocs) (void)hipFree(p);
   if (h_next) (void)hipHostFree(h_next);
+  if (h_logits) (void)hipHostFree(h_logits);
+  for (hipEvent_t e : logits_there)
+    if (e) (void)hipEventDestroy(e);
   if (h_rows) (void)hipHostFree(h_rows);
   if (stream) (void)hipStreamDestroy(stream);
 }
@@ -33,6 +36,44 @@ int gptoss_engine::create_rows(int rows_cap) {
   return GPTOSS_OK;
 }
 
+constexpr size_t LOGITS_HALF = 2 << 20;
+
+int gptoss_engine::create_logits_staging() {
+  GPTOSS_HIP(hipHostMalloc((void **)&h_logits, 2 * LOGITS_HALF, hipHostMallocDefault));
+  for (hipEvent_t &e : logits_there) GPTOSS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  return GPTOSS_OK;
+}
+
+// The first m rows of the logits to the caller's array, through the pinned halves in turn: a half travels while the one
+// before is copied out.  (Into the caller's own pages the runtime pins them, or bounces, at every call: one row of a
+// vocabulary of 201088 took 180 us behind its step.)
+int gptoss_engine::copy_logits(int m, float *host_logits) {
+  const size_t row = sizeof(float) * vocab, total = row * m;
+  struct Piece {
+    char *to;
+    size_t bytes;
+  } piece[2] = {};
+  auto take = [&](int half) -> int {
+    GPTOSS_HIP(hipEventSynchronize(logits_there[half]));
+    memcpy(piece[half].to, (char *)h_logits + half * LOGITS_HALF, piece[half].bytes);
+    return GPTOSS_OK;
+  };
+  int n = 0;
+  for (size_t at = 0; at < total; n++) {
+    const size_t r = at / row, within = at % row;
+    // rows that lie one behind the other go together
+    const size_t bytes = std::min(LOGITS_HALF, vocab == vocab_rows ? total - at : row - within);
+    if (n >= 2) GPTOSS_STEP(take(n & 1));
+    piece[n & 1] = {(char *)host_logits + at, bytes};
+    GPTOSS_HIP(hipMemcpyAsync((char *)h_logits + (n & 1) * LOGITS_HALF, (char *)(logits + r * vocab_rows) + within, bytes,
+                              hipMemcpyDeviceToHost, stream));
+    GPTOSS_HIP(hipEventRecord(logits_there[n & 1], stream));
+    at += bytes;
+  }
+  for (int i = std::max(0, n - 2); i < n; i++) GPTOSS_STEP(take(i & 1));
+  return GPTOSS_OK;
+}
+
 int gptoss_engine::create_sampling() {
   const size_t B = max_batch;
   GPTOSS_STEP(device_alloc((void **)&d_next, B * sizeof(int)));
@@ -42,6 +83,7 @@ int gptoss_engine::create_sampling() {
   if (precise()) GPTOSS_STEP(device_alloc((void **)&t_f32, B * hidden * sizeof(float)));
   if (precise() || (flags & GPTOSS_ENGINE_LOGITS)) {
     GPTOSS_STEP(device_alloc((void **)&logits, B * vocab_rows * sizeof(float)));
+    GPTOSS_STEP(create_logits_staging());
   } else {
     const size_t pairs = B * gemm_argmax_tiles(vocab_rows);
     GPTOSS_STEP(device_alloc((void **)&amax_val, pairs * sizeof(float)));
@@ -167,9 +209,7 @@ int gptoss_engine::run_rows(int n, const int *tok, const int *slot, const int *p
     if (host_logits) {
       GPTOSS_STEP(class_gemm(0, m, logits));
       if (logit_softcap > 0.f) GPTOSS_STEP(run_softcap(logits, (size_t)m * vocab_rows, logit_softcap, stream));
-      GPTOSS_HIP(hipMemcpy2DAsync(host_logits + (size_t)first * vocab, sizeof(float) * vocab, logits,
-                                  sizeof(float) * vocab_rows, sizeof(float) * vocab, m, hipMemcpyDeviceToHost, stream));
-      GPTOSS_HIP(hipStreamSynchronize(stream));   // the buffer is reused by the next portion
+      GPTOSS_STEP(copy_logits(m, host_logits + (size_t)first * vocab));   // (the buffer is reused by the next portion)
     } else {
       GPTOSS_STEP(sample_rows(r, sample, slot, first, m));
       GPTOSS_HIP(hipMemcpyAsync(h_next, d_next, sizeof(int) * m, hipMemcpyDeviceToHost, stream));

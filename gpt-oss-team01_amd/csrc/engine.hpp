@@ -64,6 +64,8 @@ struct gptoss_engine {
   gptoss::bf16_t *t = nullptr;   // [max_batch, hidden]
   float *t_f32 = nullptr;        // likewise, GPTOSS_ENGINE_PRECISE
   float *logits = nullptr;       // [max_batch, vocab_rows], only with GPTOSS_ENGINE_LOGITS
+  float *h_logits = nullptr;     // pinned, two halves of LOGITS_HALF bytes: logits on their way to the caller
+  hipEvent_t logits_there[2] = {nullptr, nullptr};   // a half's copy has ended
   float *amax_val = nullptr;     // [max_batch, column tiles of the classifier]: fused arg-max partials
   int *amax_idx = nullptr;
   // rows of a step
@@ -109,11 +111,13 @@ struct gptoss_engine {
   // the rows of a step, and what sampling needs.
   int create_rows(int rows_cap);
   int create_sampling();
+  int create_logits_staging();
   int device_alloc(void **p, size_t bytes);
 
  private:
   int upload_rows(int n, const int *tok, const int *slot, const int *pos, int n_sample, const int *sample,
                   gptoss::StepRows *out);
+  int copy_logits(int m, float *host_logits);
   int class_gemm(int row0, int count, float *out);
   int sample_rows(const gptoss::StepRows &r, const int *sample, const int *slot, int first, int count);
 };

@@ -296,6 +296,7 @@ extern "C" int gptoss_engine_create(const gptoss_config *cfg, const float *host_
   b.hip(hipStreamCreate(&e->stream), "hipStreamCreate");
   b.hip(hipHostMalloc((void **)&e->h_tokens, sizeof(int) * max_batch, hipHostMallocDefault), "hipHostMalloc");
   b.hip(hipHostMalloc((void **)&e->h_next, sizeof(int) * max_batch, hipHostMallocDefault), "hipHostMalloc");
+  if ((flags & GPTOSS_ENGINE_LOGITS) && b.rc == GPTOSS_OK) b.rc = e->create_logits_staging();
   b.hip(hipHostMalloc((void **)&e->h_lens, sizeof(int) * max_batch, hipHostMallocDefault), "hipHostMalloc");
   if (precise) {
     int rc = create_precise(e, b, host_weights);

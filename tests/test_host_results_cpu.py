@@ -1,0 +1,53 @@
+"""Memory of results in host arrays: kept for reuse only when no array uses it, bounded, safe across threads."""
+import gc
+import threading
+
+import numpy as np
+
+from conftest import load_pkg
+
+
+def test_memory_comes_back_with_the_last_array_over_it_only():
+    pool = load_pkg("engine")._HostPool(1 << 20)
+    a = pool.empty(3, 1000)
+    assert a.shape == (3, 1000) and a.dtype == np.float32 and a.flags.writeable and a.flags.c_contiguous
+    view, where = a[1, 5:], a.ctypes.data
+    a[:] = 7.0
+    del a
+    gc.collect()
+    b = pool.empty(3, 1000)
+    assert b.ctypes.data != where      # the view still uses it
+    b[:] = 1.0
+    assert (view == 7.0).all()
+    del view
+    gc.collect()
+    assert pool.empty(3, 1000).ctypes.data == where
+
+
+def test_no_more_is_kept_than_the_limit():
+    pool = load_pkg("engine")._HostPool(1 << 20)
+    arrays = [pool.empty(100, 1000) for _ in range(8)]     # 400 KB each
+    del arrays
+    gc.collect()
+    assert pool._kept <= 1 << 20 and sum(len(v) for v in pool._free.values()) == 2
+    big = pool.empty(1000, 1000)                           # beyond the limit: an array of its own
+    assert big.flags.owndata
+    assert pool.empty(0, 5).shape == (0, 5)
+
+
+def test_threads_never_share_memory_in_use():
+    pool, wrong = load_pkg("engine")._HostPool(1 << 22), []
+
+    def work(k):
+        for i in range(300):
+            a = pool.empty(20, 1000)
+            a[:] = k * 1000 + i
+            b = pool.empty(20, 1000)
+            b[:] = -1.0
+            if not (a == k * 1000 + i).all():
+                wrong.append((k, i))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not wrong
