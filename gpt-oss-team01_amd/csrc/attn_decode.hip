@@ -587,10 +587,186 @@ __global__ __launch_bounds__(256, 2) void attn_decode_resident_kernel(AttnParams
   flush();
 }
 
+// Few rows: one workgroup per (row, kv head, chunk), so that a chunk's eight blocks are all on their way at once and
+// only what has to follow the order of the blocks does.  One wave alone (attn_decode_body) requests a block ahead and
+// takes 2.5 us per block of a row by itself, almost all of it latency.
+//   1. wave w multiplies the queries with the keys of blocks w and w + 4 and publishes the blocks' maxima;
+//   2. every wave runs through the maxima (running maximum, rescale factors), turns its own scores into weights and
+//      publishes them as operands of the second product, with the lanes' sums;
+//   3. wave w accumulates output columns [16 w, 16 w + 16) over all blocks in order.
+// Every value comes from the operations, on the operands and in the order of the one-wave kernel: the same bits.
+// Calls of 16 sequences of up to 500 positions, 64 heads: 20.2 -> 13.3 us, of 3 of up to 8000: 25.0 -> 18.3 (13 of them
+// this kernel, before 21).
+template <int D>
+__global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
+  constexpr int KS = D / 32, DB = D / 16, NBLK = ATT_CHUNK / ATT_BLOCK;
+  static_assert(NBLK == 8 && DB <= 4, "two blocks and at most 16 output columns per wave");
+  __shared__ __attribute__((aligned(16))) u32x4 lds_p[NBLK][4][64];   // weights: hi and lo parts of 32 slots each
+  __shared__ float lds_sum[NBLK][64], lds_max[NBLK][16];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 15, c = lane >> 4, G = p.G;
+  const int g = blockIdx.x % p.n_kv, rest = blockIdx.x / p.n_kv;
+  const int b = rest % p.B, chunk_id = p.max_chunks - 1 - rest / p.B;
+  const SeqRange r = seq_range(__builtin_amdgcn_readfirstlane(row_len(p, b)), p.cap, p.window, p.max_len);
+  if (chunk_id >= r.nchunks) return;
+  const int c0 = r.s_begin + chunk_id * r.chunk, c1 = min(r.s_end, c0 + r.chunk);
+  const int nb = (max(0, c1 - c0) + ATT_BLOCK - 1) / ATT_BLOCK;
+  const int pos_base = (r.len > 0) ? ((r.len - 1) / p.cap) * p.cap : 0;
+  auto active = [&](int slot) {   // see attn_decode_body
+    int pp = slot + pos_base;
+    if (pp > r.len - 1) pp -= p.cap;
+    return slot < c1 && pp >= r.t_lo;
+  };
+  const bool wrapped = r.len > p.cap;
+  const bool ring_all_active = wrapped && (p.window <= 0 || p.window >= p.cap);
+  auto is_edge = [&](int blk) { return blk + ATT_BLOCK > c1 || (!ring_all_active && (wrapped || blk < r.t_lo)); };
+  const int head = g * G + min(n, G - 1);
+  const float sink_logit = p.sinks ? p.sinks[head] : -INFINITY;
+  int seq = (p.rows_per_seq > 1) ? b / p.rows_per_seq : b;
+  if (p.seq_map) seq = __builtin_amdgcn_readfirstlane(p.seq_map[seq]);
+  const bf16_t *plane = p.kv + kv_block_off(seq, g, p.n_kv, p.cap, D, 0);
+
+  // All loads at once; blocks beyond the last repeat it.  (Plain loads: so few rows stay in the caches for the next step.)
+  auto block_at = [&](int j) { return plane + (size_t)((c0 >> 6) + min(j, max(nb - 1, 0))) * (2 * KV_BLOCK * D); };
+  u32x4 kreg[2][4][KS], vreg[NBLK][2];
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int tb = 0; tb < 4; tb++)
+#pragma unroll
+      for (int s = 0; s < KS; s++)
+        kreg[u][tb][s] = *reinterpret_cast<const u32x4 *>(block_at(wave + 4 * u) + (tb * 16 + n) * D + c * KS * 8 + s * 8);
+  bf16x8 qh[KS], ql[KS];
+  split_query<KS>(p.q + ((size_t)b * p.n_q + head) * D + c * KS * 8, n < G, qh, ql);
+  const int db = min(wave, DB - 1);   // head size 32: two waves are done after their weights
+#pragma unroll
+  for (int j = 0; j < NBLK; j++)
+#pragma unroll
+    for (int grp = 0; grp < 2; grp++)
+      vreg[j][grp] = *reinterpret_cast<const u32x4 *>(block_at(j) + KV_BLOCK * D + (grp * DB + db) * 512 + lane * 8);
+
+  f32x4 s4[2][4];
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int j = wave + 4 * u, blk = c0 + j * ATT_BLOCK;
+    if (j < nb) {
+#pragma unroll
+      for (int tb = 0; tb < 4; tb++) {
+        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+          const bf16x8 kf = as_bf16x8(kreg[u][tb][s]);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qh[s], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, ql[s], acc, 0, 0, 0);
+        }
+        s4[u][tb] = acc;
+      }
+      if (is_edge(blk)) {
+#pragma unroll
+        for (int tb = 0; tb < 4; tb++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) s4[u][tb][i] = active(blk + tb * 16 + c * 4 + i) ? s4[u][tb][i] : -INFINITY;
+      }
+      float bmax = -INFINITY;
+#pragma unroll
+      for (int tb = 0; tb < 4; tb++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) bmax = fmaxf(bmax, s4[u][tb][i]);
+      bmax = max_over_quarters(bmax) * p.scale_log2e;
+      if (c == 0) lds_max[j][n] = bmax;
+    }
+  }
+  __syncthreads();
+  float alpha[NBLK], m_own[2] = {NEG_BIG, NEG_BIG}, m_run = NEG_BIG;
+#pragma unroll
+  for (int j = 0; j < NBLK; j++) {
+    alpha[j] = 1.f;
+    if (j < nb) {
+      const float m_new = fmaxf(m_run, lds_max[j][n]);
+      alpha[j] = exp2_hw(m_run - m_new);
+      m_run = m_new;
+    }
+    if (j % 4 == wave) m_own[j / 4] = m_run;
+  }
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int j = wave + 4 * u;
+    if (j < nb) {
+      float psum = 0.f;
+#pragma unroll
+      for (int grp = 0; grp < 2; grp++) {
+        uint32_t h[4], l[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float p0 = weight_of(s4[u][grp * 2 + (i >> 1)][(i & 1) * 2], p.scale_log2e, m_own[u]);
+          const float p1 = weight_of(s4[u][grp * 2 + (i >> 1)][(i & 1) * 2 + 1], p.scale_log2e, m_own[u]);
+          psum += p0 + p1;
+          split_weights(p0, p1, h[i], l[i]);
+        }
+        lds_p[j][grp * 2][lane] = u32x4{h[0], h[1], h[2], h[3]};
+        lds_p[j][grp * 2 + 1][lane] = u32x4{l[0], l[1], l[2], l[3]};
+      }
+      lds_sum[j][lane] = psum;
+    }
+  }
+  __syncthreads();
+  if (wave >= DB) return;
+  f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+  float l_run = 0.f;
+#pragma unroll
+  for (int j = 0; j < NBLK; j++) {
+    if (j < nb) {
+      const int blk = c0 + j * ATT_BLOCK;
+      l_run = l_run * alpha[j] + lds_sum[j][lane];
+#pragma unroll
+      for (int i = 0; i < 4; i++) o[i] *= alpha[j];
+      if (is_edge(blk)) {   // never-written cache memory may hold NaN bit patterns
+#pragma unroll
+        for (int grp = 0; grp < 2; grp++)
+#pragma unroll
+          for (int w = 0; w < 4; w++) {
+            const int s_lo = blk + grp * 32 + (w >> 1) * 16 + c * 4 + (w & 1) * 2;
+            vreg[j][grp][w] &= (active(s_lo) ? 0x0000ffffu : 0u) | (active(s_lo + 1) ? 0xffff0000u : 0u);
+          }
+      }
+#pragma unroll
+      for (int grp = 0; grp < 2; grp++) {
+        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vreg[j][grp]), as_bf16x8(lds_p[j][grp * 2][lane]), o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vreg[j][grp]), as_bf16x8(lds_p[j][grp * 2 + 1][lane]), o, 0, 0, 0);
+      }
+    }
+  }
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (n >= G) return;
+  const int hq = g * G + n;
+  if (r.nchunks == 1) {
+    const float sink2 = sink_logit * 1.4426950408889634f;
+    const float M = fmaxf(m_run, sink2);
+    const float w = exp2_hw(m_run - M);
+    const float denom = l_run * w + exp2_hw(sink2 - M);
+    const float inv = (denom > 0.f) ? w / denom : 0.f;
+    *reinterpret_cast<u32x2 *>(p.out + ((size_t)b * p.n_q + hq) * D + db * 16 + c * 4) =
+        u32x2{pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv)};
+  } else {
+    const size_t slot = ((size_t)b * p.max_chunks + chunk_id) * p.n_q + hq;
+    *reinterpret_cast<f32x4 *>(p.part_o + slot * D + db * 16 + c * 4) = o;
+    if (wave == 0 && c == 0) {
+      p.part_ml[slot * 2] = m_run;
+      p.part_ml[slot * 2 + 1] = l_run;
+    }
+  }
+}
+// Rows of one chunk: up to so many (row, kv head) pairs (16 sequences of 200 positions and 8 kv heads 11.9 -> 10.2 us, 60 of
+// 500 23.0 -> 17.9, 128 of 500 26.7 / 26.2; 256 of 100: 16.0 with a wave each, 25.6).  Chunks of longer rows: always (63
+// sequences of up to 1500 positions 41 -> 33 us, of up to 8000 142 -> 126; from 512 pairs on they take another form).
+constexpr long long ATT_FEW_PAIRS = 1024;
+
 // Merge the chunk partials of one (sequence, q head) with the sink logit.  One thread owns four
 // consecutive output elements; the chunk loop is unrolled in groups of ATT_RED_UNROLL whose loads
 // are all requested before the first use.
-constexpr int ATT_RED_UNROLL = 4;
+constexpr int ATT_RED_UNROLL = 16;
 
 template <int D>
 __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
@@ -1044,12 +1220,16 @@ static int attn_launch(const float *q, const void *kv_cache, const int *lens,
     // one row per sequence: a resident grid that keeps its output rows in LDS until the end (it
     // writes them 16 bytes at a time; an output that is only 8-byte aligned gets the plain launch)
     const bool hold_rows = !pair && aligned(out, 16);
+    const bool few = !pair && !pl.wide && (pl.max_chunks > 1 || items <= ATT_FEW_PAIRS);
     int resident = 0;
-    if (hold_rows) {
+    if (hold_rows && !few) {
       const int rc = head_dim == 64 ? attn_resident_wgs<64>(&resident) : attn_resident_wgs<32>(&resident);
       if (rc != GPTOSS_OK) return rc;
     }
-    if (head_dim == 64) {
+    if (few) {
+      if (head_dim == 64) attn_few_kernel<64><<<(int)items, 256, 0, s>>>(p);
+      else attn_few_kernel<32><<<(int)items, 256, 0, s>>>(p);
+    } else if (head_dim == 64) {
       if (pair) attn_decode_kernel<64, true><<<grid, 256, 0, s>>>(p);
       else if (hold_rows) attn_decode_resident_kernel<64><<<std::min(grid, resident), 256, 0, s>>>(p, grid);
       else attn_decode_kernel<64, false><<<grid, 256, 0, s>>>(p);

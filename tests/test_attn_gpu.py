@@ -276,3 +276,29 @@ def test_attn_prefill_refuses_a_wrapped_window_ring(ops):
     pre = ops.AttnPrefill(1, 200, 64, 8, 64, 200)
     with pytest.raises(lib.GptossError):
         pre.forward(torch.zeros(1, 200, 64, 64).cuda(), cache, window=128)
+
+
+@pytest.mark.parametrize("n_q,n_kv,D,cap,window", [
+    (64, 8, 64, 512, 0), (64, 8, 64, 512, 128), (64, 8, 64, 128, 128),   # 20B heads; window; a ring that has wrapped
+    (64, 8, 64, 192, 128),                                               # a wrapped ring longer than its window
+    (8, 8, 64, 512, 0), (32, 8, 32, 512, 0), (96, 8, 64, 512, 200),      # 1, 4 and 12 query heads per kv head
+])
+def test_a_few_rows_have_the_bits_of_the_same_rows_among_many(ops, n_q, n_kv, D, cap, window):
+    """Rows of up to 512 slots: a workgroup each where few are served, a wave each where many are."""
+    B = 160                                              # 1280 (row, kv head) pairs
+    g = torch.Generator(device="cuda").manual_seed(n_q + cap + window)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    longest = cap if not (window and cap < 512) else cap + 100
+    edges = [0, 1, 2, 63, 64, 65, 127, 128, 129, 255, 257, 448, 449, 511, 512]
+    lens = [min(x, longest) for x in edges] + torch.randint(1, longest + 1, (B - len(edges),), generator=g, device="cuda").tolist()
+    lens = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    cache = ops.KVCache(B, n_kv, D, cap)
+    cache.kv.view(torch.int16).fill_(0x7FC1)             # NaN patterns where nothing is written
+    filled = min(int(lens.max()), cap)
+    cache.write(rnd(B, filled, n_kv, D).bfloat16(), rnd(B, filled, n_kv, D).bfloat16(), 0)
+    q, sinks = rnd(B, n_q, D) * 2, rnd(n_q)
+    many = ops.AttnDecode(B, n_q, n_kv, D, longest).forward(q, cache, lens, sinks, window=window)
+    for rows in (1, 7, 15, 100):
+        few = ops.AttnDecode(rows, n_q, n_kv, D, longest).forward(q[:rows].contiguous(), cache.first(rows), lens[:rows], sinks,
+                                                                  window=window)
+        assert torch.equal(few.view(torch.int16), many[:rows].view(torch.int16)), rows
