@@ -540,8 +540,10 @@ int run_short_conv(const ShortConv &c, const StepRows &r, const float *in, int l
 template <int NI, int KIND>
 static void launch_scan_kind(const Scan &p, const StepRows &r, hipStream_t s) {
   auto grid = [&](int cols) { return dim3((unsigned)(r.n_seg * (p.heads + (KIND == SCAN_RETENTION ? 0 : 1)) * cdiv(p.V, cols))); };
-  // stretches of few heads and sequences: with two columns per lane half of the chip would be idle
-  const bool few = (long long)r.n_seg * p.heads * cdiv(p.V, 64) <= 128;
+  // Stretches of few heads and sequences: with two columns per lane half of the chip would be idle, or every SIMD have
+  // one wave, which issues an instruction every seven cycles (8 prompts of 1000 and 16 heads of 128 x 128, 256 workgroups
+  // against 512: delta rule 455 -> 409 us, per key channel 544 -> 521; 32 heads of 128 x 64, state space 383 -> 342).
+  const bool few = (long long)r.n_seg * p.heads * cdiv(p.V, 64) <= 256;
   if (r.longest == 1) scan_kernel<NI, KIND, true, 2><<<grid(64), 256, 0, s>>>(p, r.segs, r.n_seg);
   else if (few) scan_kernel<NI, KIND, false, 1><<<grid(32), 256, 0, s>>>(p, r.segs, r.n_seg);
   else scan_kernel<NI, KIND, false, 2><<<grid(64), 256, 0, s>>>(p, r.segs, r.n_seg);
