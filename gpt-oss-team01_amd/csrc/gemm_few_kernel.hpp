@@ -6,15 +6,16 @@
 // many CUs.  The streaming kernels give 256 columns to a workgroup of eight waves with two 4 KB slabs of W in flight
 // each, on a grid of one workgroup per CU: one token's four experts are then 92 (first product) and 48 (second) work
 // items on 256 CUs.  Here a workgroup is 128 columns, or 32 (below), the grid has one for every work item, and a wave
-// has eight slabs in flight (MXFP4: sixteen).  To have the registers for that, A does not pass through them slab by
-// slab: chunks of eight slabs (64 rows: four) are staged in LDS, one barrier each, and W's loads stay in flight across
-// it.  Operand roles, order of the sum over K and epilogues are those of the streaming kernels, so a row has the same
-// bits whichever kernel computes it.
+// has eight slabs in flight.  To have the registers for that, A does not pass through them slab by slab: chunks of eight
+// slabs (64 rows, MXFP4: four) are staged in LDS, one barrier each, and W's loads stay in flight across it.  Operand
+// roles, order of the sum over K and epilogues are those of the streaming kernels, so a row has the same bits whichever
+// kernel computes it.
 // Measured, 2880 x 2880 experts, streaming kernels -> these (us): one token, both products 36 + 32 -> 24 + 14, MXFP4
-// block 60 -> 43; 27 tokens 156 + 91 -> 157 + 81 (5.9-6.8 TB/s either way); 12 tokens on MXFP4 60 + 32 -> 49 + 29.
+// block 60 -> 43; 27 tokens 156 + 91 -> 157 + 81 (5.9-6.8 TB/s either way); MXFP4 block of 12 tokens 114 -> 87.
 // Dense 5120 x 2880: one row 31 -> 9, 32 rows 33 -> 11, 64 rows 37 -> 16, 200 rows 32 -> 21.
-// (A read straight from memory in operand order, without LDS: one token 60, but 12 tokens on MXFP4 127 instead of 99,
-// because A is then four times the bytes of W.)
+// (A read straight from memory in operand order, without LDS: one token 60, but 12 tokens on MXFP4 127,
+// because A is then four times the bytes of W.  One wave with 16 rows for MXFP4's small tiles: nine tokens 86.0 -> 87.6,
+// twelve 87.8 -> 93.5.)
 #pragma once
 #include "gemm_kernel.hpp"
 
@@ -26,13 +27,14 @@ namespace gptoss {
 //                    token's block 68 -> 59 us, eight tokens' 178 -> 176
 //   1 x 32, 1 x 64   the same for launches of at most FEW_SOLO_BLOCKS blocks, on the registers of two waves
 
-// 64-k slabs of W that a wave keeps in flight: 16 bytes per lane and k-step with bf16 weights, 16 per slab with MXFP4
-constexpr int few_ring(bool fp4) { return fp4 ? 16 : 8; }
-constexpr int few_chunk(int rows) { return rows <= 32 ? 8 : 4; }   // slabs of A that are staged together: one barrier each
-constexpr int few_row(int rows) { return few_chunk(rows) * BK + 8; }   // padded row of a staged chunk in bf16 elements
+constexpr int FEW_RING = 8;   // 64-k slabs of W that a wave keeps in flight
+constexpr int few_chunk(int rows, bool fp4) { return rows <= 32 && !fp4 ? 8 : 4; }   // slabs of A that are staged together: one barrier each
+constexpr int few_row(int rows, bool fp4) { return few_chunk(rows, fp4) * BK + 8; }   // padded row of a staged chunk in bf16 elements
 constexpr int few_ahead(int rows) { return rows <= 32 ? 4 : 2; }       // k-steps whose operands are read from LDS ahead
-// waves per SIMD: a single wave that stages 32 rows or more needs the registers of two
-constexpr int few_occupancy(int waves, int rows) { return waves == 1 && rows > 8 ? 1 : 2; }
+// Waves per SIMD.  A single wave that stages 32 rows or more needs the registers of two.  MXFP4: expanding the codes takes
+// as long as the products, and a third wave fills in for it (a slab of W is five registers); with two waves, sixteen slabs
+// in flight and chunks of eight, 12 tokens took 95 us instead of 87, 600 on 128 experts 410 instead of 394.
+constexpr int few_occupancy(int waves, int rows, bool fp4) { return waves == 1 && rows > 8 ? 1 : fp4 ? 3 : 2; }
 
 typedef __amdgpu_buffer_rsrc_t few_rsrc_t;
 // cache policy of a buffer load: the non-temporal bit
@@ -47,8 +49,8 @@ __device__ __forceinline__ few_rsrc_t few_buffer(const void *base, uint32_t byte
 template <int WAVES, int ROWS, bool GATHER, int EPI, bool FP4, bool ONCE>
 __device__ __forceinline__ void few_block(const GemmParams &p, bf16_t *lds, int mat, int row0, int rows, int cb, int slab0,
                                           int nslab, void *out) {
-  constexpr int RING = few_ring(FP4);
-  constexpr int RB = (ROWS + 31) / 32, CHUNK = few_chunk(ROWS), ROW = few_row(ROWS), AHEAD = few_ahead(ROWS);
+  constexpr int RING = FEW_RING;
+  constexpr int RB = (ROWS + 31) / 32, CHUNK = few_chunk(ROWS, FP4), ROW = few_row(ROWS, FP4), AHEAD = few_ahead(ROWS);
   constexpr int WQ = FP4 ? 1 : 4;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int K = p.K, N = p.N, kslab = K / BK;
@@ -169,9 +171,9 @@ __device__ __forceinline__ void few_block(const GemmParams &p, bf16_t *lds, int 
 // Work items are (row tile, 32-column block) pairs; every XCD has a contiguous part of them, so that the row tiles of
 // one expert, which multiply the same blocks of W one after the other, find them in that XCD's L2.
 template <int WAVES, int ROWS, bool GATHER, int EPI, bool FP4>
-__global__ __launch_bounds__(WAVES * 64, few_occupancy(WAVES, ROWS)) void few_gemm_kernel(GemmParams p) {
+__global__ __launch_bounds__(WAVES * 64, few_occupancy(WAVES, ROWS, FP4)) void few_gemm_kernel(GemmParams p) {
   constexpr int BM = ROWS <= 32 ? 32 : 64;   // rows of a dense problem's tile
-  __shared__ __attribute__((aligned(16))) bf16_t lds[2 * ROWS * few_row(ROWS)];
+  __shared__ __attribute__((aligned(16))) bf16_t lds[2 * ROWS * few_row(ROWS, FP4)];
   const const_as<int> tiles = constant_ptr(p.tiles);
   const int n_tiles = p.tiles ? tiles[0] : (p.dense_rows + BM - 1) / BM;
   const int n_blk = (p.N / 32 + WAVES - 1) / WAVES;
