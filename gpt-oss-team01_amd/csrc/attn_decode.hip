@@ -53,16 +53,6 @@ __device__ __forceinline__ float weight_of(float score, float scale, float m) {
   return exp2_hw(__builtin_fmaf(score, scale, -m));
 }
 
-// The largest value of the four lanes n, n + 16, n + 32, n + 48, in all of them, without a trip through LDS.
-__device__ __forceinline__ float max_over_quarters(float v) {
-  const uint32_t u = __float_as_uint(v);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  const float m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const uint32_t w = __float_as_uint(m);
-  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-
 // Two weights in [0, 1] as bf16 hi + lo parts: truncation to bf16 plus the truncated remainder keeps 16 mantissa bits.
 __device__ __forceinline__ void split_weights(float p0, float p1, uint32_t &h, uint32_t &l) {
   const uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
@@ -450,8 +440,8 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
   }
 
   // ---- per-head totals: sum the partial denominators of the 4 lanes that share a head --------
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run += lane_xor<16>(l_run);
+  l_run += lane_xor<32>(l_run);
   if constexpr (WG) {
     // the four waves' states (a wave without a block holds the neutral one: max -1e30, sum 0, O 0)
     // meet in LDS and are merged with the sink in wave order, by the formula of attn_reduce_kernel
@@ -737,8 +727,8 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
       }
     }
   }
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run += lane_xor<16>(l_run);
+  l_run += lane_xor<32>(l_run);
   if (n >= G) return;
   const int hq = g * G + n;
   if (r.nchunks == 1) {
@@ -1013,8 +1003,8 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
     }
   }
 
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run += lane_xor<16>(l_run);
+  l_run += lane_xor<32>(l_run);
   if (!col_live) return;
   const int hq = g * G + hn;
   const float sink2 = sink_logit * 1.4426950408889634f;

@@ -5,6 +5,8 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <type_traits>
+
 #include "../../include/gptoss_mi355.h"
 
 namespace gptoss {
@@ -91,6 +93,64 @@ __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) {
 }
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
+
+// ---- exchanges between lanes ---------------------------------------------------------------------
+// The value of lane (own ^ M), every lane active: moves inside a row of 16 lanes and swaps of rows, in registers.  A
+// shuffle goes through LDS and takes over a hundred cycles, and a reduction waits for six of them one after the other,
+// which is what the small kernels of a decoding step did for a good part of their few microseconds.
+template <int M>
+__device__ __forceinline__ uint32_t lane_xor_bits(uint32_t v) {
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8 || M == 16 || M == 32);
+  if constexpr (M == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true);    // quad_perm [1,0,3,2]
+  if constexpr (M == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true);    // quad_perm [2,3,0,1]
+  if constexpr (M == 4)   // half a row mirrored (^ 7), then every quad mirrored (^ 3)
+    return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, true), 0x1B, 0xf, 0xf, true);
+  if constexpr (M == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xf, 0xf, true);   // row_ror 8
+  if constexpr (M == 16) {
+    const auto s = __builtin_amdgcn_permlane16_swap(v, v, false, false);   // [0]: rows 0 0 2 2, [1]: rows 1 1 3 3
+    return (threadIdx.x & 16) ? s[0] : s[1];
+  }
+  if constexpr (M == 32) {
+    const auto s = __builtin_amdgcn_permlane32_swap(v, v, false, false);   // [0]: the lower half twice, [1]: the upper
+    return (threadIdx.x & 32) ? s[0] : s[1];
+  }
+}
+template <int M, typename T>
+__device__ __forceinline__ T lane_xor(T v) {
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8);
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(T, lane_xor_bits<M>(__builtin_bit_cast(uint32_t, v)));
+  } else {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    return __builtin_bit_cast(T, (uint64_t)lane_xor_bits<M>((uint32_t)(u >> 32)) << 32 | lane_xor_bits<M>((uint32_t)u));
+  }
+}
+
+// f(integral_constant<M>) for M = N / 2, N / 4, .. 1: the steps of a butterfly over N lanes
+template <int N, typename F>
+__device__ __forceinline__ void butterfly(F &&f) {
+  if constexpr (N > 1) {
+    f(std::integral_constant<int, N / 2>{});
+    butterfly<N / 2>(f);
+  }
+}
+
+// The sum over N consecutive lanes (N a power of two), in all of them.
+template <int N = WAVE, typename T>
+__device__ __forceinline__ T lanes_sum(T v) {
+  butterfly<N>([&](auto m) { v += lane_xor<decltype(m)::value>(v); });
+  return v;
+}
+
+// The largest value of the four lanes n, n + 16, n + 32, n + 48, in all of them, without a trip through LDS.
+__device__ __forceinline__ float max_over_quarters(float v) {
+  const uint32_t u = __float_as_uint(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const float m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const uint32_t w = __float_as_uint(m);
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
 
 // ---- KV cache layout ---------------------------------------------------------------------------
 // One array per layer: for every (sequence, kv head) capacity/64 blocks of 64 slots; a block holds

@@ -488,8 +488,8 @@ __device__ __forceinline__ void gemm_tile(const GemmParams &p, bf16_t *lds, int 
             }
           }
       }
-      const float ov = __shfl_xor(bv, 32, 64);
-      const int oi = __shfl_xor(bi, 32, 64);
+      const float ov = lane_xor<32>(bv);
+      const int oi = lane_xor<32>(bi);
       if (ov > bv || (ov == bv && oi < bi)) {
         bv = ov;
         bi = oi;

@@ -453,8 +453,8 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
       }
 #pragma unroll
       for (int r = 0; r < RB; r++) {
-        const float ov = __shfl_xor(bv[r], 32, 64);
-        const int oi = __shfl_xor(bi[r], 32, 64);
+        const float ov = lane_xor<32>(bv[r]);
+        const int oi = lane_xor<32>(bi[r]);
         if (ov > bv[r] || (ov == bv[r] && oi < bi[r])) {
           bv[r] = ov;
           bi[r] = oi;

@@ -54,7 +54,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(float *__restrict__ x,
     }
     ss += (double)__fmul_rn(v, v);
   }
-  for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+  ss = lanes_sum(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
   ss = red[0] + red[1] + red[2] + red[3];
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(float *__restrict__ x
       for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[i][q], v[i][q]);
     }
   }
-  for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+  ss = lanes_sum(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
   ss = red[0] + red[1] + red[2] + red[3];
@@ -217,11 +217,11 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ 
         if (row[i + q] > bv || bi == 0x7fffffff) { bv = row[i + q]; bi = i + q; }
     }
   }
-  for (int m = 32; m >= 1; m >>= 1) {
-    float ov = __shfl_xor(bv, m, 64);
-    int oi = __shfl_xor(bi, m, 64);
+  butterfly<64>([&](auto m) {
+    const float ov = lane_xor<decltype(m)::value>(bv);
+    const int oi = lane_xor<decltype(m)::value>(bi);
     if (oi != 0x7fffffff && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi))) { bv = ov; bi = oi; }
-  }
+  });
   if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -437,14 +437,14 @@ __global__ __launch_bounds__(256) void argmax_tiles_kernel(const float *__restri
       bi = i;
     }
   }
-  for (int m = 32; m >= 1; m >>= 1) {
-    const float ov = __shfl_xor(bv, m, 64);
-    const int oi = __shfl_xor(bi, m, 64);
+  butterfly<64>([&](auto m) {
+    const float ov = lane_xor<decltype(m)::value>(bv);
+    const int oi = lane_xor<decltype(m)::value>(bi);
     if (ov > bv || (ov == bv && oi < bi)) {
       bv = ov;
       bi = oi;
     }
-  }
+  });
   if ((threadIdx.x & 63) == 0) {
     sv[threadIdx.x >> 6] = bv;
     si[threadIdx.x >> 6] = bi;
@@ -581,7 +581,7 @@ __global__ __launch_bounds__(256) void depth_average_norm_kernel(float *__restri
     }
   }
   if (!norm_w) return;
-  for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+  ss = lanes_sum(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
   ss = red[0] + red[1] + red[2] + red[3];

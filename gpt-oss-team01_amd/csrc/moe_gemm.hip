@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256) void combine_norm_kernel(const float *__restri
       for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[i][q], v[i][q]);
     }
   }
-  for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+  ss = lanes_sum(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
   ss = red[0] + red[1] + red[2] + red[3];

@@ -39,15 +39,14 @@ __device__ __forceinline__ void topk_softmax_group(const float (&v)[NJ], int sub
           bi = e;
         }
       }
-#pragma unroll
-      for (int m = 16; m >= 1; m >>= 1) {
-        float ov = __shfl_xor(bv, m, 64);
-        int oi = __shfl_xor(bi, m, 64);
+      butterfly<32>([&](auto m) {
+        const float ov = lane_xor<decltype(m)::value>(bv);
+        const int oi = lane_xor<decltype(m)::value>(bi);
         if (oi != NONE && (bi == NONE || ov > bv || (ov == bv && oi < bi))) {
           bv = ov;
           bi = oi;
         }
-      }
+      });
       if (bi != NONE && (bi & 31) == sub) used |= 1u << (bi >> 5);
       pick_v[s] = bv;
       pick_i[s] = bi;
@@ -87,19 +86,22 @@ __device__ __forceinline__ uint64_t same_expert_mask(int e, bool valid, int nbit
 __device__ __forceinline__ int wave_scan4(const int (&v)[4], int (&ex)[4]) {
   const int lane = threadIdx.x & 63;
   int sum = v[0] + v[1] + v[2] + v[3];
+  // inside the rows of 16 lanes (row_shr 1, 2, 4, 8; nothing enters from outside), then the last lane of rows 0 and 2 to
+  // rows 1 and 3, then lane 31 to the upper half
   int inc = sum;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    int o = __shfl_up(inc, d, 64);
-    if (lane >= d) inc += o;
-  }
+  inc += __builtin_amdgcn_mov_dpp(inc, 0x111, 0xf, 0xf, true);
+  inc += __builtin_amdgcn_mov_dpp(inc, 0x112, 0xf, 0xf, true);
+  inc += __builtin_amdgcn_mov_dpp(inc, 0x114, 0xf, 0xf, true);
+  inc += __builtin_amdgcn_mov_dpp(inc, 0x118, 0xf, 0xf, true);
+  inc += __builtin_amdgcn_update_dpp(0, inc, 0x142, 0xa, 0xf, false);
+  inc += __builtin_amdgcn_update_dpp(0, inc, 0x143, 0xc, 0xf, false);
   int run = inc - sum;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     ex[i] = run;
     run += v[i];
   }
-  return __shfl(inc, 63, 64);
+  return __builtin_amdgcn_readlane(inc, 63);
 }
 
 // From the experts' pair counts total[E] (LDS): the experts' offsets into offs[E+1] (LDS), and, when
@@ -337,7 +339,7 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
           for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[i][q], v[i][q]);
         }
       }
-      for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+      ss = lanes_sum(ss);
       if (lane == 0) nred[grp][(threadIdx.x >> 6) & 3] = ss;
       __syncthreads();
       ss = nred[grp][0] + nred[grp][1] + nred[grp][2] + nred[grp][3];

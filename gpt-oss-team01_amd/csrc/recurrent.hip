@@ -29,9 +29,7 @@ __device__ __forceinline__ float softplus_f(float z) {
 }
 
 __device__ __forceinline__ float wave_sum_f(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-  return v;
+  return lanes_sum(v);
 }
 
 // sum over 8 consecutive lanes: two exchanges inside a quad, then the mirrored half row
@@ -479,8 +477,7 @@ __global__ __launch_bounds__(256) void gated_norm_vec_kernel(GatedNorm g) {
       v[i][e] = gated_value(g, v[i][e], z[i][e]);
       ss = fmaf(v[i][e], v[i][e], ss);
     }
-#pragma unroll
-  for (int m = LANES / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+  ss = lanes_sum<LANES>(ss);
   const float inv = 1.f / sqrtf(ss / g.size + g.eps);
   if (!live) return;
   OUT *out = (OUT *)g.out + (size_t)row * g.ld_out + g.out_col + at;

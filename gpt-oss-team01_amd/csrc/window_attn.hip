@@ -60,8 +60,7 @@ __global__ __launch_bounds__(256) void window_store_kernel(WindowAttn a, const i
     float inv[RT];
 #pragma unroll
     for (int r = 0; r < RT; r++) {
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) ss[r] += __shfl_xor(ss[r], m, 64);
+      ss[r] = lanes_sum(ss[r]);
       inv[r] = 1.f / sqrtf(ss[r] / a.dim + a.eps);
     }
 #pragma unroll
@@ -156,8 +155,7 @@ __global__ __launch_bounds__(256) void window_store_rows_kernel(WindowAttn a, co
     }
 #pragma unroll
     for (int k = 0; k < 2; k++) {
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) ss[k] += __shfl_xor(ss[k], m, 64);
+      ss[k] = lanes_sum(ss[k]);
       if ((tid & 63) == 0) red[r][k][tid >> 6] = ss[k];
     }
   }
@@ -214,8 +212,7 @@ __global__ __launch_bounds__(256) void window_store_row_kernel(WindowAttn a, con
   for (int i = tid; i < G * D; i += 256) ss[1] = fmaf(k[i], k[i], ss[1]);
 #pragma unroll
   for (int x = 0; x < 2; x++) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) ss[x] += __shfl_xor(ss[x], m, 64);
+    ss[x] = lanes_sum(ss[x]);
     if ((tid & 63) == 0) red[x][tid >> 6] = ss[x];
   }
   __syncthreads();
@@ -328,9 +325,7 @@ __device__ __forceinline__ void block_output(f32x4 (&s)[4], int db_n, int pos0, 
       s[tb][e] = (pos >= lo && pos <= hi) ? s[tb][e] : WNEG;
       mx = fmaxf(mx, s[tb][e]);
     }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-  const float m_new = fmaxf(m, mx);
+  const float m_new = fmaxf(m, max_over_quarters(mx));
   const float fade = __builtin_amdgcn_exp2f(m - m_new);
   m = m_new;
   float sum = 0.f;
@@ -377,8 +372,8 @@ __device__ __forceinline__ void attend_block(const QFrag<KS> &q, int ks_n, int d
 
 // Row sums over the four lane groups of a column (each lane has summed its own key rows).
 __device__ __forceinline__ float column_sum(float l) {
-  l += __shfl_xor(l, 16, 64);
-  return l + __shfl_xor(l, 32, 64);
+  l += lane_xor<16>(l);
+  return l + lane_xor<32>(l);
 }
 
 // lane (n, c) stores dimensions 16 db + 4 c .. + 4 of its column
@@ -598,14 +593,13 @@ __global__ __launch_bounds__(256) void window_f32_kernel(WindowAttn a, const int
       s *= a.scale;
     }
     float mx = s;
-    for (int x = 32; x >= 1; x >>= 1) mx = fmaxf(mx, __shfl_xor(mx, x, 64));
+    butterfly<64>([&](auto x) { mx = fmaxf(mx, lane_xor<decltype(x)::value>(mx)); });
     if (lane == 0) red[wave] = mx;
     __syncthreads();
     const float m_new = fmaxf(m, fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
     const float e = pos <= hi ? expf(s - m_new) : 0.f;
     sp[tid] = e;
-    float sum = e;
-    for (int x = 32; x >= 1; x >>= 1) sum += __shfl_xor(sum, x, 64);
+    const float sum = lanes_sum(e);
     if (lane == 0) red[4 + wave] = sum;
     __syncthreads();
     const float fade = expf(m - m_new);   // 0 on the first tile
