@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(float *__restrict__ x
                                                            int n_mean) {
   __shared__ double red[4];
   const size_t row = (size_t)blockIdx.x * H;
-  f32x4 v[VPT];
+  f32x4 v[VPT], w[VPT];   // the weights are requested with the row, not when its sum is known
   double ss = 0.0;
 #pragma unroll
   for (int i = 0; i < VPT; i++) {
@@ -87,6 +87,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(float *__restrict__ x
     v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (h < H) {
       v[i] = *reinterpret_cast<const f32x4 *>(x + row + h);
+      w[i] = *reinterpret_cast<const f32x4 *>(weight + h);
       if (residual) {
         const f32x4 r = *reinterpret_cast<const f32x4 *>(residual + row + h);
 #pragma unroll
@@ -108,10 +109,9 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(float *__restrict__ x
   for (int i = 0; i < VPT; i++) {
     const int h = (threadIdx.x + 256 * i) * 4;
     if (h < H) {
-      const f32x4 w = *reinterpret_cast<const f32x4 *>(weight + h);
       f32x4 o;
 #pragma unroll
-      for (int q = 0; q < 4; q++) o[q] = (float)((double)w[q] * (inv * (double)v[i][q]));
+      for (int q = 0; q < 4; q++) o[q] = (float)((double)w[i][q] * (inv * (double)v[i][q]));
       *reinterpret_cast<u32x2 *>(t_bf16 + row + h) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
       if (t_f32) *reinterpret_cast<f32x4 *>(t_f32 + row + h) = o;
     }

@@ -32,12 +32,27 @@ struct TokenExperts {
   }
   __device__ __forceinline__ f32x4 sum(const float *__restrict__ y2, int H, int h, int k) const {
     f32x4 agg = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (KMAX <= 8) {
+      // No load under a condition, so that all of them are on their way together (places beyond k read the first row
+      // again): with a branch for each, a token's rows came one after the other, 3 us of the MoE block of one token.
+      f32x4 v[KMAX];
 #pragma unroll
-    for (int s = 0; s < KMAX; s++) {
-      if (s < k) {
-        const f32x4 v = *reinterpret_cast<const f32x4 *>(y2 + (size_t)rows[s] * H + h);
+      for (int s = 0; s < KMAX; s++) v[s] = *reinterpret_cast<const f32x4 *>(y2 + (size_t)rows[s < k ? s : 0] * H + h);
 #pragma unroll
-        for (int q = 0; q < 4; q++) agg[q] = __fadd_rn(agg[q], __fmul_rn(v[q], w[s]));
+      for (int s = 0; s < KMAX; s++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const float next = __fadd_rn(agg[q], __fmul_rn(v[s][q], w[s]));
+          agg[q] = s < k ? next : agg[q];
+        }
+    } else {
+#pragma unroll
+      for (int s = 0; s < KMAX; s++) {
+        if (s < k) {
+          const f32x4 v = *reinterpret_cast<const f32x4 *>(y2 + (size_t)rows[s] * H + h);
+#pragma unroll
+          for (int q = 0; q < 4; q++) agg[q] = __fadd_rn(agg[q], __fmul_rn(v[q], w[s]));
+        }
       }
     }
     return agg;
@@ -45,8 +60,8 @@ struct TokenExperts {
 };
 
 // Weighted combine: out[b,:] (+)= sum over the token's k experts, in ascending expert order (the
-// order of the reference CPU loop, run.cpp:642-704), of w * y2[row of that pair].  Products and
-// sums are rounded separately, as that loop rounds them.
+// order of the reference CPU loop, run.cpp:642-704), of w * y2[row of that pair].  The compiler
+// fuses every product into its sum, in all forms of the kernel alike.
 // KMAX: room for a token's experts.
 template <int VPT, int KMAX = 8>  // float4 chunks per thread: rows of at most 1024 * VPT floats (0: any length, a loop)
 __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ y2,
@@ -57,8 +72,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
   const int b = blockIdx.x;
   TokenExperts<KMAX> x;
   x.load(topk_w, inv_perm, b, k);
-  auto chunk = [&](int h) {
-    f32x4 agg = x.sum(y2, H, h, k);
+  auto store = [&](int h, f32x4 agg) {
     f32x4 *op = reinterpret_cast<f32x4 *>(out + (size_t)b * H + h);
     if (accumulate) {
       f32x4 prev = *op;
@@ -68,14 +82,17 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
     *op = agg;
   };
   if constexpr (VPT > 0) {
-    // unrolled: the loads of every chunk are in flight before the first sum needs one
+    // no chunk under a condition: the loads of all of them are in flight before the first sum needs one
+    f32x4 agg[VPT];
+#pragma unroll
+    for (int i = 0; i < VPT; i++) agg[i] = x.sum(y2, H, min((int)(threadIdx.x + 256 * i) * 4, H - 4), k);
 #pragma unroll
     for (int i = 0; i < VPT; i++) {
       const int h = (threadIdx.x + 256 * i) * 4;
-      if (h < H) chunk(h);
+      if (h < H) store(h, agg[i]);
     }
   } else {
-    for (int h = threadIdx.x * 4; h < H; h += 256 * 4) chunk(h);
+    for (int h = threadIdx.x * 4; h < H; h += 256 * 4) store(h, x.sum(y2, H, h, k));
   }
 }
 
@@ -84,7 +101,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
 // steps.  Element-to-thread mapping, the double-precision sum of squares and the scaling are those
 // of rmsnorm_rows_kernel (glue.hip), so the result equals running the two kernels one after the
 // other bit for bit.
-template <int VPT>
+template <int VPT, int KMAX>
 __global__ __launch_bounds__(256) void combine_norm_kernel(const float *__restrict__ y2,
                                                            const float *__restrict__ topk_w,
                                                            const int *__restrict__ inv_perm,
@@ -93,21 +110,30 @@ __global__ __launch_bounds__(256) void combine_norm_kernel(const float *__restri
                                                            bf16_t *__restrict__ t_bf16) {
   __shared__ double red[4];
   const int b = blockIdx.x;
-  TokenExperts<8> x;
-  x.load(topk_w, inv_perm, b, k);
-  f32x4 v[VPT];
-  double ss = 0.0;
+  // what does not depend on the routing is requested before it
+  f32x4 v[VPT], nw[VPT];
 #pragma unroll
   for (int i = 0; i < VPT; i++) {
     const int h = (threadIdx.x + 256 * i) * 4;
     v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (h < H) {
-      const f32x4 agg = x.sum(y2, H, h, k);
-      f32x4 *op = reinterpret_cast<f32x4 *>(out + (size_t)b * H + h);
-      const f32x4 prev = *op;
+      v[i] = *reinterpret_cast<const f32x4 *>(out + (size_t)b * H + h);
+      nw[i] = *reinterpret_cast<const f32x4 *>(norm_w + h);
+    }
+  }
+  TokenExperts<KMAX> x;
+  x.load(topk_w, inv_perm, b, k);
+  f32x4 agg[VPT];
 #pragma unroll
-      for (int q = 0; q < 4; q++) v[i][q] = __fadd_rn(prev[q], agg[q]);
-      *op = v[i];
+  for (int i = 0; i < VPT; i++) agg[i] = x.sum(y2, H, min((int)(threadIdx.x + 256 * i) * 4, H - 4), k);
+  double ss = 0.0;
+#pragma unroll
+  for (int i = 0; i < VPT; i++) {
+    const int h = (threadIdx.x + 256 * i) * 4;
+    if (h < H) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) v[i][q] = __fadd_rn(v[i][q], agg[i][q]);
+      *reinterpret_cast<f32x4 *>(out + (size_t)b * H + h) = v[i];
 #pragma unroll
       for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[i][q], v[i][q]);
     }
@@ -123,10 +149,9 @@ __global__ __launch_bounds__(256) void combine_norm_kernel(const float *__restri
   for (int i = 0; i < VPT; i++) {
     const int h = (threadIdx.x + 256 * i) * 4;
     if (h < H) {
-      const f32x4 nw = *reinterpret_cast<const f32x4 *>(norm_w + h);
       f32x4 o;
 #pragma unroll
-      for (int q = 0; q < 4; q++) o[q] = (float)((double)nw[q] * (inv * (double)v[i][q]));
+      for (int q = 0; q < 4; q++) o[q] = (float)((double)nw[i][q] * (inv * (double)v[i][q]));
       *reinterpret_cast<u32x2 *>(t_bf16 + (size_t)b * H + h) =
           u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
     }
@@ -261,7 +286,8 @@ int run_combine(const float *y2, const float *topk_w, const int *inv_perm, float
     GPTOSS_REQUIRE(accumulate && norm_out && H % 4 == 0, GPTOSS_ERR_DIM, "combine: the tanh norm follows an accumulation");
     TraceScope ts("combine_tanh_norm", s);
     const dim3 grid(B, cdiv(H, 1024));
-    if (k <= 8) combine_tanh_norm_kernel<8><<<grid, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, *tanh_norm, norm_out);
+    if (k <= 4) combine_tanh_norm_kernel<4><<<grid, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, *tanh_norm, norm_out);
+    else if (k <= 8) combine_tanh_norm_kernel<8><<<grid, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, *tanh_norm, norm_out);
     else combine_tanh_norm_kernel<MOE_MAX_TOP><<<grid, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, *tanh_norm, norm_out);
     GPTOSS_LAUNCH_CHECK("combine_tanh_norm_kernel");
     return GPTOSS_OK;
@@ -269,18 +295,23 @@ int run_combine(const float *y2, const float *topk_w, const int *inv_perm, float
   // out += combine, then norm_out = RMSNorm(out) * norm_w in the same kernel, when asked for
   if (norm_w && norm_out && accumulate && k <= 8 && H % 4 == 0 && H <= 4096 && aligned(norm_w, 16) && aligned(norm_out, 8)) {
     TraceScope ts("combine_rmsnorm", s);
-    if (H <= 1024) combine_norm_kernel<1><<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, norm_w, norm_out);
-    else if (H <= 2048) combine_norm_kernel<2><<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, norm_w, norm_out);
-    else if (H <= 3072) combine_norm_kernel<3><<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, norm_w, norm_out);
-    else combine_norm_kernel<4><<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, norm_w, norm_out);
+    auto launch = [&](auto kernel) { kernel<<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, norm_w, norm_out); };
+    const bool few = k <= 4;
+    if (H <= 1024) launch(few ? combine_norm_kernel<1, 4> : combine_norm_kernel<1, 8>);
+    else if (H <= 2048) launch(few ? combine_norm_kernel<2, 4> : combine_norm_kernel<2, 8>);
+    else if (H <= 3072) launch(few ? combine_norm_kernel<3, 4> : combine_norm_kernel<3, 8>);
+    else launch(few ? combine_norm_kernel<4, 4> : combine_norm_kernel<4, 8>);
     GPTOSS_LAUNCH_CHECK("combine_norm_kernel");
     return GPTOSS_OK;
   }
   {
     TraceScope ts("combine", s);
     if (k > 8) combine_kernel<0, MOE_MAX_TOP><<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, accumulate);
+    else if (H <= 3072 && H > 2048 && k <= 4) combine_kernel<3, 4><<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, accumulate);
     else if (H <= 3072 && H > 2048) combine_kernel<3><<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, accumulate);
+    else if (H <= 1024 && k <= 4) combine_kernel<1, 4><<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, accumulate);
     else if (H <= 1024) combine_kernel<1><<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, accumulate);
+    else if (k <= 4) combine_kernel<0, 4><<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, accumulate);
     else combine_kernel<0><<<B, 256, 0, s>>>(y2, topk_w, inv_perm, out, H, k, accumulate);
   }
   GPTOSS_LAUNCH_CHECK("combine_kernel");

@@ -318,3 +318,28 @@ def test_moe_forward_of_a_prompt_pass_equals_the_same_tokens_in_small_batches(op
     assert same.mean() > 0.9
     mx, mean = rel_errors(full.cpu().numpy()[rows][same], want[same])
     assert mx <= TOL_MAX and mean <= TOL_MEAN, (mx, mean)
+
+
+# k: one of four places, three, all four, five of eight places, all eight; H: a piece of a thread's chunk, one chunk, the next
+# remainder, three chunks short of the end and whole, a loop
+@pytest.mark.parametrize("k", [1, 3, 4, 5, 8])
+@pytest.mark.parametrize("H", [64, 1024, 1088, 2880, 3072, 4096])
+def test_combine_adds_every_product_in_expert_order(ops, k, H):
+    """With a second product of zeros an expert's row is its bias: what is left is the rounding of at most k products and k
+    sums."""
+    E, B = 16, 19
+    g = torch.Generator(device="cuda").manual_seed(k * H)
+    n = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    layer = ops.MoeLayer(n(E, H), n(E), n(E, 128, H), n(E, 128), torch.zeros(E, H, 64, device="cuda").bfloat16(), n(E, H),
+                         top_k=k, max_tokens=64)
+    t, out = n(B, H), torch.randn(B, H, generator=g, device="cuda")
+    before = out.clone()
+    layer.forward(t, out=out, accumulate=True)
+    fresh = layer.forward(t)
+    _, w, ids = layer.routing_views()[:3]
+    ids, order = ids.long().sort(dim=1)
+    w = w.gather(1, order)
+    terms = torch.stack([layer.b2[ids[:, s]].double() * w[:, s, None].double() for s in range(k)])
+    bound = 2 * k * 2.0 ** -24 * terms.abs().sum(0)
+    assert bool(((fresh - terms.sum(0)).abs() <= bound).all())
+    assert torch.equal(out, before + fresh)
