@@ -289,7 +289,10 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
     int *__restrict__ topk_i, int rows_per_wg, RouterNorm nrm, RouterGroup grp) {
   __shared__ float red[ROUTER_WAVES][16][NB * 16 + 1];
   extern __shared__ __attribute__((aligned(16))) unsigned char t_rows_raw[];  // NORM: [rows_per_wg][H] bf16
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // The wave's number has to be a scalar: matrix instructions do not look at the mask of active lanes, so a wave skips the
+  // k-steps that are not its own only by a branch, and for a condition on a lane's value the compiler leaves the branch
+  // out where masking looks cheaper (one matrix instruction under it, no wait: its products were added all the same).
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // rows_per_wg <= 16 token rows are this workgroup's; the other MFMA rows repeat the last of them
   const int r0 = blockIdx.x * rows_per_wg;
   const int arow = min(r0 + min(lane & 15, rows_per_wg - 1), B - 1);

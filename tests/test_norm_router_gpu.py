@@ -1,0 +1,59 @@
+"""The MoE block that runs the residual add and RMSNorm in front of it by itself, as the engine calls it: every result
+must have the bits of the norm, the router, the grouping and the block called one after the other."""
+import ctypes as C
+
+import pytest
+import torch
+
+from conftest import load_pkg
+
+pytestmark = pytest.mark.gpu
+
+
+class _PreNorm(C.Structure):   # MoePreNorm of gemm.hpp
+    _fields_ = [("x", C.c_void_p), ("residual", C.c_void_p), ("weight", C.c_void_p)]
+
+
+def _forward_norm(layer, x, residual, weight, out):
+    """gptoss::moe_forward_norm, which has no C entry point, by its linker name; -> its t, bf16 [B, H]."""
+    f = getattr(layer.L, "_ZN6gptoss16moe_forward_normEPK18gptoss_moe_weightsPKviPfPvmP12ihipStream_tiPKfPtPKNS_10MoePreNormE")
+    f.restype = C.c_int
+    f.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p, C.c_int, C.c_void_p,
+                  C.c_void_p, C.c_void_p]
+    B, H = x.shape
+    assert B <= layer.max_tokens and all(v.is_contiguous() for v in (x, weight, out))
+    assert residual is None or (residual.shape == x.shape and residual.is_contiguous())
+    t = torch.empty(B, H, dtype=torch.bfloat16, device="cuda")
+    pre = _PreNorm(x.data_ptr(), residual.data_ptr() if residual is not None else None, weight.data_ptr())
+    load_pkg("lib").check(f(C.byref(layer.desc), t.data_ptr(), B, out.data_ptr(), layer.ws.data_ptr(), layer.ws_bytes,
+                            torch.cuda.current_stream().cuda_stream, 0, None, None, C.byref(pre)))
+    layer._last_B = B
+    return t
+
+
+# H: a part of a thread's first chunk, three chunks short of the end, four whole chunks; E: one column block, two, eight, nine
+@pytest.mark.parametrize("H", [64, 2880, 4096])
+@pytest.mark.parametrize("E", [4, 32, 128, 129])
+@pytest.mark.parametrize("with_residual", [False, True])
+def test_a_block_with_its_norm_equals_its_parts(ops, H, E, with_residual):
+    g = torch.Generator(device="cuda").manual_seed(H + E)
+    rnd = lambda *s, std=1.0: torch.randn(*s, generator=g, device="cuda") * std
+    n = lambda *s, **k: rnd(*s, **k).bfloat16()
+    I = 64
+    layer = ops.MoeLayer(n(E, H, std=H ** -0.5), n(E), n(E, 2 * I, H, std=0.05), n(E, 2 * I), n(E, H, I, std=0.05), n(E, H),
+                         top_k=4, max_tokens=301)
+    weight = 1 + rnd(H, std=0.1)
+    # 1, 2, 3, 4 rows: one workgroup groups them; 5, 16, 17: several, and a launch that sorts; 301: a last one of one row
+    for B in (1, 2, 3, 4, 5, 16, 17, 301):
+        x, residual = rnd(B, H) * 3, rnd(B, H) if with_residual else None
+        x_want, out = x.clone(), rnd(B, H)
+        out_want = out.clone()
+        t = _forward_norm(layer, x, residual, weight, out)
+        got = [x, t, out] + layer.routing_views()
+        t_want = ops.rmsnorm(x_want, weight, residual)
+        logits = ops.router_gemm(t_want, layer.w_router, layer.b_router)
+        w, ids, offsets, order, place, _ = ops.moe_route(logits, 4)
+        layer.forward(t_want, out=out_want, accumulate=True)
+        want = [x_want, t_want, out_want, logits, w, ids, offsets, order, place]
+        for name, a, b in zip("x t out logits weights ids offsets order place".split(), got, want):
+            assert torch.equal(a, b), (B, name)
