@@ -14,12 +14,21 @@ namespace gptoss {
 // Selection = k rounds of (local best, 5-step butterfly) ordered by (value desc, expert id asc);
 // softmax over the k picked values with exp in float and the sum and division in double
 // (run.cpp:319-337).  Every lane of the group must call; lane 0 of the group writes.
+// A logit that is no number ranks as -infinity: whatever a token's row holds, its picks are k different experts, so that
+// its pairs cannot displace those of other tokens.  The weights of a token that picks one are no numbers.
 // ------------------------------------------------------------------------------------------------
 template <int NJ, int KMAX = 8>
 __device__ __forceinline__ void topk_softmax_group(const float (&v)[NJ], int sub, int E, int k,
                                                    bool live, float *__restrict__ w_out,
                                                    int *__restrict__ i_out, int *i_copy = nullptr) {
-  uint32_t used = 0;
+  uint32_t used = 0, nan = 0;
+  float rank[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; j++) {
+    const bool no_number = v[j] != v[j];
+    rank[j] = no_number ? -INFINITY : v[j];
+    nan |= (no_number ? 1u : 0u) << j;
+  }
   float pick_v[KMAX];
   int pick_i[KMAX];
   constexpr int NONE = 0x7fffffff;
@@ -34,8 +43,8 @@ __device__ __forceinline__ void topk_softmax_group(const float (&v)[NJ], int sub
       for (int j = 0; j < NJ; j++) {
         int e = sub + 32 * j;
         bool ok = !((used >> j) & 1u) && e < E;
-        if (ok && (bi == NONE || v[j] > bv || (v[j] == bv && e < bi))) {
-          bv = v[j];
+        if (ok && (bi == NONE || rank[j] > bv || (rank[j] == bv && e < bi))) {
+          bv = rank[j];
           bi = e;
         }
       }
@@ -52,6 +61,7 @@ __device__ __forceinline__ void topk_softmax_group(const float (&v)[NJ], int sub
       pick_i[s] = bi;
     }
   }
+  const bool no_numbers = (uint32_t)(__ballot((used & nan) != 0) >> (threadIdx.x & 32)) != 0;
   if (live && sub == 0) {
     float ex[KMAX];
     double sum = 0.0;
@@ -63,7 +73,7 @@ __device__ __forceinline__ void topk_softmax_group(const float (&v)[NJ], int sub
 #pragma unroll
     for (int s = 0; s < KMAX; s++) {
       if (s < k) {
-        w_out[s] = (float)((double)ex[s] / sum);
+        w_out[s] = no_numbers ? NAN : (float)((double)ex[s] / sum);
         i_out[s] = pick_i[s];
         if (i_copy) i_copy[s] = pick_i[s];
       }

@@ -343,3 +343,42 @@ def test_combine_adds_every_product_in_expert_order(ops, k, H):
     bound = 2 * k * 2.0 ** -24 * terms.abs().sum(0)
     assert bool(((fresh - terms.sum(0)).abs() <= bound).all())
     assert torch.equal(out, before + fresh)
+
+
+@pytest.mark.parametrize("E,k", [(4, 4), (32, 4), (40, 3), (256, 8)])
+def test_routing_of_rows_that_are_no_numbers(ops, orc, E, k):
+    """Rows of NaN, a row with one, and one of which only k - 1 values are numbers: k different experts each, weights of NaN
+    where a NaN is picked; the rows between them as if they were alone."""
+    B = 12
+    logits = np.random.default_rng(E).standard_normal((B, E)).astype(np.float32)
+    logits[[0, 7]] = np.nan
+    logits[3, E // 2] = np.nan
+    logits[5, k - 1:] = np.nan
+    tw, ti, off, srt, inv, _ = [x.cpu().numpy() if x is not None else None for x in ops.moe_route(torch.from_numpy(logits).cuda(), k)]
+    ranked = np.where(np.isnan(logits), -np.inf, logits).astype(np.float32)
+    ov, oi = orc.topk_softmax(ranked, k)
+    np.testing.assert_array_equal(ti, oi)
+    picked_nan = np.isnan(np.take_along_axis(logits, oi.astype(np.int64), axis=1)).any(axis=1)
+    assert np.isnan(tw[picked_nan]).all()
+    np.testing.assert_allclose(tw[~picked_nan], ov[~picked_nan], rtol=2e-6, atol=1e-7)
+    for got, want in zip((off, srt, inv), orc.group(oi, E)):
+        np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("B", [3, 16, 17, 100])       # grouped by the router's own workgroup, and by a kernel behind it
+@pytest.mark.parametrize("E", [4, 32, 128])
+def test_tokens_that_are_no_numbers_leave_the_others_alone(ops, B, E):
+    g = torch.Generator(device="cuda").manual_seed(B + E)
+    n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    H = I = 128
+    layer = ops.MoeLayer(n(E, H, std=0.1), n(E), n(E, 2 * I, H, std=0.1), n(E, 2 * I), n(E, H, I, std=0.1), n(E, H), top_k=4,
+                         max_tokens=128)
+    t = n(B, H)
+    want = layer.forward(t).clone()
+    bad = list(range(0, B, 2)) if B <= 16 else list(range(0, B, 7))
+    broken = t.clone()
+    broken[bad] = float("nan")
+    got = layer.forward(broken)
+    rest = [b for b in range(B) if b not in bad]
+    assert bool(torch.isnan(got[bad]).all())
+    assert torch.equal(got[rest], want[rest])
