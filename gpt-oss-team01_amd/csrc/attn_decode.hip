@@ -46,14 +46,32 @@ constexpr float NEG_BIG = -1.0e30f;
 // is 1, so a sum in fp32 is the same with them or without.)
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// A score's weight against the running maximum m (in powers of two).  Scaling and difference are one fused operation, in
-// every form of the kernels and in blocks with and without masked slots alike: a row's result must not depend on what
-// its partner row in a wave forces.
-__device__ __forceinline__ float weight_of(float score, float scale, float m) {
-  return exp2_hw(__builtin_fmaf(score, scale, -m));
+// What the exponential of a block's scores is taken of: the distance of score * scale (powers of two) from the row's running
+// maximum m.  Scaling and difference are one fused operation, in every form of the kernels and in blocks with and without
+// masked slots alike: a row's result must not depend on what its partner row in a wave forces.  The maximum is a rounded
+// product, so its own distance is that rounding error and its weight within 2^(|m| 2^-24) of 1, a factor that all weights
+// of the row share.  From 2^24 on the error is a power of two and more (beyond 2^31 the maximum's weight would overflow or
+// vanish): such rows take the difference of rounded products, the maximum's distance is 0.
+__device__ __forceinline__ void weight_exponents(f32x4 (&s4)[4], float scale, float m) {
+#pragma clang fp contract(off)
+  const bool huge = fabsf(m) >= 16777216.f && m != NEG_BIG;
+  if (__builtin_expect(__ballot(huge) != 0, 0)) {
+#pragma unroll
+    for (int tb = 0; tb < 4; tb++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float fused = __builtin_fmaf(s4[tb][i], scale, -m), product = s4[tb][i] * scale;
+        s4[tb][i] = huge ? product - m : fused;
+      }
+  } else {
+#pragma unroll
+    for (int tb = 0; tb < 4; tb++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) s4[tb][i] = __builtin_fmaf(s4[tb][i], scale, -m);
+  }
 }
 
-// Two weights in [0, 1] as bf16 hi + lo parts: truncation to bf16 plus the truncated remainder keeps 16 mantissa bits.
+// Two weights, positive, as bf16 hi + lo parts: truncation to bf16 plus the truncated remainder keeps 16 mantissa bits.
 __device__ __forceinline__ void split_weights(float p0, float p1, uint32_t &h, uint32_t &l) {
   const uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
   h = __builtin_amdgcn_perm(u1, u0, 0x07060302u);   // the upper halves
@@ -364,6 +382,7 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
     const float m_new = fmaxf(m_run, max_over_quarters(bmax) * p.scale_log2e);
     const float alpha = exp2_hw(m_run - m_new);
     m_run = m_new;
+    weight_exponents(s4, p.scale_log2e, m_new);
     float psum = 0.f;
     bf16x8 ph[2], pl[2];
 #pragma unroll
@@ -372,8 +391,8 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         // operand k index (c, jj): jj<4 -> slot c*4+jj of the first 16, jj>=4 -> of the second 16
-        float p0 = weight_of(s4[grp * 2 + (j >> 1)][(j & 1) * 2], p.scale_log2e, m_new);
-        float p1 = weight_of(s4[grp * 2 + (j >> 1)][(j & 1) * 2 + 1], p.scale_log2e, m_new);
+        float p0 = exp2_hw(s4[grp * 2 + (j >> 1)][(j & 1) * 2]);
+        float p1 = exp2_hw(s4[grp * 2 + (j >> 1)][(j & 1) * 2 + 1]);
         psum += p0 + p1;
         split_weights(p0, p1, h[j], l[j]);
       }
@@ -683,14 +702,15 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
   for (int u = 0; u < 2; u++) {
     const int j = wave + 4 * u;
     if (j < nb) {
+      weight_exponents(s4[u], p.scale_log2e, m_own[u]);
       float psum = 0.f;
 #pragma unroll
       for (int grp = 0; grp < 2; grp++) {
         uint32_t h[4], l[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          const float p0 = weight_of(s4[u][grp * 2 + (i >> 1)][(i & 1) * 2], p.scale_log2e, m_own[u]);
-          const float p1 = weight_of(s4[u][grp * 2 + (i >> 1)][(i & 1) * 2 + 1], p.scale_log2e, m_own[u]);
+          const float p0 = exp2_hw(s4[u][grp * 2 + (i >> 1)][(i & 1) * 2]);
+          const float p1 = exp2_hw(s4[u][grp * 2 + (i >> 1)][(i & 1) * 2 + 1]);
           psum += p0 + p1;
           split_weights(p0, p1, h[i], l[i]);
         }
@@ -816,8 +836,9 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 // prompts; here it is read once per 16 rows.  What bounds it is the vector units (70 % busy, the matrix cores 34 %): per
 // 64 x 16 scores a wave issues about 170 of their instructions, a tenth of them exponentials.  Eight prompts of 1000
 // positions, 64 heads: 237 -> 211 us with the exponential, the maximum and the splitting of weights in fewer instructions
-// (exp2_hw, max_over_quarters, split_weights), -> 195 with the scale fused into the exponent's difference (weight_of),
-// one range check per masked slot and blocks straight into LDS, -> 181 with whole loads of q (split_query).
+// (exp2_hw, max_over_quarters, split_weights), -> 195 with the scale fused into the exponent's difference
+// (weight_exponents), one range check per masked slot and blocks straight into LDS, -> 181 with whole loads of q
+// (split_query).
 // Every row sees the arithmetic of the one-wave kernel over its own blocks in ascending order (a
 // block outside a row's range is a no-op for its columns), so rows of up to ATT_CHUNK positions
 // equal the decode call bit for bit; longer rows are summed in one pass instead of chunk by
@@ -945,6 +966,7 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
     const float m_new = fmaxf(m_run, max_over_quarters(bmax) * p.scale_log2e);
     const float alpha = exp2_hw(m_run - m_new);
     m_run = m_new;
+    weight_exponents(s4, p.scale_log2e, m_new);
     float psum = 0.f;
     bf16x8 ph[2], pl[2];
 #pragma unroll
@@ -952,8 +974,8 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
       uint32_t h[4], l[4];
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        float p0 = weight_of(s4[grp * 2 + (j >> 1)][(j & 1) * 2], p.scale_log2e, m_new);
-        float p1 = weight_of(s4[grp * 2 + (j >> 1)][(j & 1) * 2 + 1], p.scale_log2e, m_new);
+        float p0 = exp2_hw(s4[grp * 2 + (j >> 1)][(j & 1) * 2]);
+        float p1 = exp2_hw(s4[grp * 2 + (j >> 1)][(j & 1) * 2 + 1]);
         psum += p0 + p1;
         split_weights(p0, p1, h[j], l[j]);
       }

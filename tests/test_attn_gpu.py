@@ -1,5 +1,7 @@
 """GPU parity of decode attention (sinks, sliding window, GQA, ragged lengths, ring cache)
 against the CPU oracle, through the C ABI."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -302,3 +304,41 @@ def test_a_few_rows_have_the_bits_of_the_same_rows_among_many(ops, n_q, n_kv, D,
         few = ops.AttnDecode(rows, n_q, n_kv, D, longest).forward(q[:rows].contiguous(), cache.first(rows), lens[:rows], sinks,
                                                                   window=window)
         assert torch.equal(few.view(torch.int16), many[:rows].view(torch.int16)), rows
+
+
+# (sequences, positions, new positions per sequence or 0 for decoding): a workgroup per chunk without and with a merge, a
+# wave per row, a workgroup per row, the prompt kernel
+FORMS = [(3, 300, 0), (3, 1200, 0), (200, 300, 0), (70, 1200, 0), (2, 300, 40)]
+
+
+def _attend(ops, form, q, k, v, sinks):
+    B, n, T = form
+    n_q, D = q.shape[-2:]
+    cache = ops.KVCache(B, k.shape[2], D, (n + 63) // 64 * 64)
+    cache.write(k, v)
+    if T:
+        return ops.AttnPrefill(B, T, n_q, k.shape[2], D, n).forward(q, cache, pos0=n - T, sinks=sinks)
+    lens = torch.full((B,), n, dtype=torch.int32, device="cuda")
+    return ops.AttnDecode(B, n_q, k.shape[2], D, n).forward(q, cache, lens, sinks)
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_scores_of_any_size(ops, form, D, sign):
+    """Scores of about +-2^34 and 2^60 in powers of two, one of them larger than the others by a tenth: it takes all."""
+    B, n, T = form
+    n_q, n_kv = 16, 8
+    g = torch.Generator(device="cuda").manual_seed(D)
+    direction = torch.randn(D, generator=g, device="cuda").sign()
+    for size in (2.0 ** 34, 2.0 ** 60):
+        q = (direction * sign * size / math.sqrt(D)).expand(*((B, T) if T else (B,)), n_q, D).contiguous()
+        level = 1.0 + 0.5 * torch.rand(B, n, n_kv, 1, generator=g, device="cuda")
+        best = torch.randint(0, n - T if T else n, (B, n_kv), generator=g, device="cuda")
+        level.scatter_(1, best[:, None, :, None], 1.75 if sign > 0 else 0.75)
+        k = (level * direction).bfloat16()
+        v = torch.randn(B, n, n_kv, D, generator=g, device="cuda").bfloat16()
+        got = _attend(ops, form, q, k, v, None)
+        want = v.gather(1, best[:, None, :, None].expand(B, 1, n_kv, D)).squeeze(1).repeat_interleave(n_q // n_kv, 1)
+        want = want[:, None].expand_as(got) if T else want
+        assert torch.equal(got, want), size
