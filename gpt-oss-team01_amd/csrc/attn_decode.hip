@@ -41,9 +41,10 @@ namespace gptoss {
 constexpr int ATT_BLOCK = 64;   // slots per inner iteration
 constexpr float NEG_BIG = -1.0e30f;
 
-// The hardware's exponential by itself: a weight below 2^-126 of its row's largest is zero.  (The library function scales
-// such arguments first, five more instructions per score where a block step has about 300 in all; a row's largest weight
-// is 1, so a sum in fp32 is the same with them or without.)
+// The hardware's exponential by itself, for weights against a running maximum: one below 2^-126 is zero.  (The library
+// function scales such arguments first, five more instructions per score where a block step has about 300 in all; the
+// row's largest weight is about 1, so a sum in fp32 is the same with them or without.)  Where a row's sum meets its sink
+// nothing of that size need be in it: a sink may lie more than 126 above every score, and those few factors take exp2f.
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // What the exponential of a block's scores is taken of: the distance of score * scale (powers of two) from the row's running
@@ -484,11 +485,11 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
     float M = sink2;
 #pragma unroll
     for (int w = 0; w < 4; w++) M = fmaxf(M, lds_ml[(w * 16 + hm) * 2]);
-    float denom = exp2_hw(sink2 - M);
+    float denom = exp2f(sink2 - M);
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < 4; w++) {
-      const float wgt = exp2_hw(lds_ml[(w * 16 + hm) * 2] - M);
+      const float wgt = exp2f(lds_ml[(w * 16 + hm) * 2] - M);
       denom += lds_ml[(w * 16 + hm) * 2 + 1] * wgt;
       const f32x4 ow = *reinterpret_cast<const f32x4 *>(&lds_o[(w * 16 + hm) * D + d4]);
 #pragma unroll
@@ -506,8 +507,8 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
   if (row_chunks == 1) {
     float sink2 = sink_logit * 1.4426950408889634f;  // lanes that get here have head == hq
     float M = fmaxf(m_run, sink2);
-    float w = exp2_hw(m_run - M);
-    float denom = l_run * w + exp2_hw(sink2 - M);
+    float w = exp2f(m_run - M);
+    float denom = l_run * w + exp2f(sink2 - M);
     float inv = (denom > 0.f) ? w / denom : 0.f;
     bf16_t *op = HOLD ? hold + hn * D : p.out + ((size_t)bn * p.n_q + hq) * D;
     if (HOLD && lane == 0) *hold_row = b * p.n_q + g * G;
@@ -754,8 +755,8 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
   if (r.nchunks == 1) {
     const float sink2 = sink_logit * 1.4426950408889634f;
     const float M = fmaxf(m_run, sink2);
-    const float w = exp2_hw(m_run - M);
-    const float denom = l_run * w + exp2_hw(sink2 - M);
+    const float w = exp2f(m_run - M);
+    const float denom = l_run * w + exp2f(sink2 - M);
     const float inv = (denom > 0.f) ? w / denom : 0.f;
     *reinterpret_cast<u32x2 *>(p.out + ((size_t)b * p.n_q + hq) * D + db * 16 + c * 4) =
         u32x2{pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv)};
@@ -799,7 +800,7 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 #pragma unroll
     for (int u = 0; u < ATT_RED_UNROLL; u++) M = fmaxf(M, m[u]);
   }
-  float denom = exp2_hw(sink2 - M);
+  float denom = exp2f(sink2 - M);
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int c0 = 0; c0 < r.nchunks; c0 += ATT_RED_UNROLL) {
     float m[ATT_RED_UNROLL], l[ATT_RED_UNROLL];
@@ -816,7 +817,7 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 #pragma unroll
     for (int u = 0; u < ATT_RED_UNROLL; u++) {
       if (c0 + u < r.nchunks) {
-        const float w = exp2_hw(m[u] - M);
+        const float w = exp2f(m[u] - M);
         denom += l[u] * w;
 #pragma unroll
         for (int q = 0; q < 4; q++) acc[q] += o[u][q] * w;
@@ -1031,8 +1032,8 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
   const int hq = g * G + hn;
   const float sink2 = sink_logit * 1.4426950408889634f;
   const float M = fmaxf(m_run, sink2);
-  const float w = exp2_hw(m_run - M);
-  const float denom = l_run * w + exp2_hw(sink2 - M);
+  const float w = exp2f(m_run - M);
+  const float denom = l_run * w + exp2f(sink2 - M);
   const float inv = (denom > 0.f) ? w / denom : 0.f;
   bf16_t *op = p.out + ((size_t)bn * p.n_q + hq) * D;
 #pragma unroll

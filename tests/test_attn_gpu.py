@@ -342,3 +342,26 @@ def test_scores_of_any_size(ops, form, D, sign):
         want = v.gather(1, best[:, None, :, None].expand(B, 1, n_kv, D)).squeeze(1).repeat_interleave(n_q // n_kv, 1)
         want = want[:, None].expand_as(got) if T else want
         assert torch.equal(got, want), size
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("D", [32, 64])
+def test_a_sink_far_above_every_score(ops, form, D):
+    """The sink lies 125 to 145 powers of two above the scores, which are all equal: what is left is the mean of the values
+    times 2^-shift, of values large enough for bf16 to hold it."""
+    B, n, T = form
+    n_q, n_kv = 16, 8
+    g = torch.Generator(device="cuda").manual_seed(D)
+    q = torch.zeros(*((B, T) if T else (B,)), n_q, D, device="cuda")
+    k = torch.randn(B, n, n_kv, D, generator=g, device="cuda").bfloat16()
+    v = (2.0 ** 40 * (1 + torch.rand(B, n, n_kv, D, generator=g, device="cuda"))).bfloat16()
+    shift = torch.linspace(125, 145, n_q, device="cuda")
+    sinks = shift * math.log(2.0)
+    shift = sinks.double() / math.log(2.0)
+    got = _attend(ops, form, q, k, v, sinks).double()
+    seen = torch.arange(n - T + 1, n + 1, device="cuda") if T else torch.tensor([n], device="cuda")
+    total = v.double().cumsum(1)[:, seen - 1]                                        # [B, T or 1, n_kv, D]
+    want = total.repeat_interleave(n_q // n_kv, 2) * torch.exp2(-shift)[:, None]
+    want = want if T else want[:, 0]
+    # bf16: 2^-9; the exponent as a float near 145: 2^-17; its factor near 2^-145 has 2^-5 of itself as its last bit
+    assert bool(((got - want).abs() <= want * (2.0 ** -8 + torch.exp2(shift - 149)[:, None])).all())
