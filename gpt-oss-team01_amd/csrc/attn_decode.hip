@@ -597,7 +597,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_resident_kernel(AttnParams
   flush();
 }
 
-// Few rows: one workgroup per (row, kv head, chunk), so that a chunk's eight blocks are all on their way at once and
+// Few items: one workgroup per (row, kv head, chunk), so that a chunk's eight blocks are all on their way at once and
 // only what has to follow the order of the blocks does.  One wave alone (attn_decode_body) requests a block ahead and
 // takes 2.5 us per block of a row by itself, almost all of it latency.
 //   1. wave w multiplies the queries with the keys of blocks w and w + 4 and publishes the blocks' maxima;
@@ -769,10 +769,18 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
     }
   }
 }
-// Rows of one chunk: up to so many (row, kv head) pairs (16 sequences of 200 positions and 8 kv heads 11.9 -> 10.2 us, 60 of
-// 500 23.0 -> 17.9, 128 of 500 26.7 / 26.2; 256 of 100: 16.0 with a wave each, 25.6).  Chunks of longer rows: always (63
-// sequences of up to 1500 positions 41 -> 33 us, of up to 8000 142 -> 126; from 512 pairs on they take another form).
-constexpr long long ATT_FEW_PAIRS = 1024;
+// The launches that take it: where every row is as long as the longest may be, up to 512 (row, kv head, chunk) items, two
+// per CU; 384 with heads of 32 values; 256 of rows that cannot fill half a chunk (it requests eight blocks whatever a row
+// has).  64 heads of 64 on 8 kv heads, full rows, caches cold, a wave per item -> this kernel (us): 4 of 8000 positions
+// (512 items) 29.0 -> 25.4, 32 of 1000 29.6 -> 25.4, 63 of 448 22.7 -> 18.9; 40 of 128 (320) 12.1 -> 12.1.  Beyond that a
+// wave per item fills the chip as well and follows HBM better: 5 of 8000 (640 items) 29.8 -> 29.7, 16 of 3000 (768) 30.5 ->
+// 32.6, 8 of 8000 (1024) 33.4 -> 37.5, 48 of 4000 (3072) 74.5 -> 85.1, 96 of 300 20.2 -> 23.2, and 1000 rows of a prompt
+// over 8 kv heads 141 -> 196.  (Rows of very different length are another matter: 63 of 500 to 4000 79 -> 70.  The host
+// does not know the lengths.)
+static bool attn_few(long long pairs, int span, int head_dim) {
+  const long long items = pairs * ((span + ATT_CHUNK - 1) / ATT_CHUNK);
+  return items <= (span * head_dim < 256 * 64 ? 256 : head_dim == 32 ? 384 : 512);
+}
 
 // Merge the chunk partials of one (sequence, q head) with the sink logit.  One thread owns four
 // consecutive output elements; the chunk loop is unrolled in groups of ATT_RED_UNROLL whose loads
@@ -1229,11 +1237,11 @@ static int attn_launch(const float *q, const void *kv_cache, const int *lens,
   long long items = (long long)(pair ? (B / rows_per_seq) * ((rows_per_seq + 1) / 2) : B) * n_kv * p.max_chunks;
   int grid = (int)((items + 3) / 4) + (pl.wide ? 1 : 0);
   {
-    TraceScope ts("attn_decode", s);
     // one row per sequence: a resident grid that keeps its output rows in LDS until the end (it
     // writes them 16 bytes at a time; an output that is only 8-byte aligned gets the plain launch)
     const bool hold_rows = !pair && aligned(out, 16);
-    const bool few = !pair && !pl.wide && (pl.max_chunks > 1 || items <= ATT_FEW_PAIRS);
+    const bool few = !pair && !pl.wide && attn_few((long long)B * n_kv, span, head_dim);
+    TraceScope ts(few ? "attn_decode_few" : "attn_decode", s);
     int resident = 0;
     if (hold_rows && !few) {
       const int rc = head_dim == 64 ? attn_resident_wgs<64>(&resident) : attn_resident_wgs<32>(&resident);

@@ -306,6 +306,73 @@ def test_a_few_rows_have_the_bits_of_the_same_rows_among_many(ops, n_q, n_kv, D,
         assert torch.equal(few.view(torch.int16), many[:rows].view(torch.int16)), rows
 
 
+def _kernels(ops, call):
+    with ops.KernelTrace(capacity=16) as trace:
+        call()
+    return [name for name, _ in trace.results()]
+
+
+# longest: rows of one chunk or of up to five; a window over them; a ring that has wrapped
+@pytest.mark.parametrize("longest,cap,window", [(2000, 2048, 0), (700, 768, 0), (2000, 2048, 700), (3000, 1024, 600)])
+@pytest.mark.parametrize("n_q,n_kv,D", [(64, 8, 64), (96, 8, 64), (64, 8, 32)])
+def test_few_rows_of_several_chunks_have_the_bits_of_the_same_rows_among_more(ops, n_q, n_kv, D, longest, cap, window):
+    """A workgroup per chunk where few are served, a wave per chunk where more are (60 rows: too few for a workgroup each)."""
+    B = 60
+    g = torch.Generator(device="cuda").manual_seed(longest + window)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    edges = [longest, 513, 512, 511, 1024, 1025, 64, 1, 0]
+    lens = [min(x, longest) for x in edges] + torch.randint(1, longest + 1, (B - len(edges),), generator=g, device="cuda").tolist()
+    lens = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    cache = ops.KVCache(B, n_kv, D, cap)
+    cache.write(rnd(B, cap, n_kv, D).bfloat16(), rnd(B, cap, n_kv, D).bfloat16(), 0)
+    q, sinks = rnd(B, n_q, D) * 2, rnd(n_q)
+    out = {}
+    def attend(rows):
+        attn = ops.AttnDecode(rows, n_q, n_kv, D, longest)
+        out[rows] = attn.forward(q[:rows].contiguous(), cache.first(rows), lens[:rows], sinks, window=window)
+    assert _kernels(ops, lambda: attend(B)) == ["attn_decode", "attn_reduce"]
+    for rows in (1, 2, 5, 9):
+        assert _kernels(ops, lambda: attend(rows)) == ["attn_decode_few", "attn_reduce"], rows
+        assert torch.equal(out[rows].view(torch.int16), out[B][:rows].view(torch.int16)), rows
+
+
+@pytest.mark.parametrize("pos0,T", [(0, 130), (500, 70), (900, 9)])
+def test_prompt_rows_of_more_than_eight_heads_per_kv_head(ops, pos0, T):
+    """They go row by row: thousands of rows are many, however few the sequences are."""
+    n_q, n_kv, D = 96, 8, 64
+    n = pos0 + T
+    g = torch.Generator(device="cuda").manual_seed(T)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    k, v, q, sinks = rnd(1, n, n_kv, D).bfloat16(), rnd(1, n, n_kv, D).bfloat16(), rnd(1, T, n_q, D), rnd(n_q)
+    cache = ops.KVCache(1, n_kv, D, (n + 63) // 64 * 64)
+    cache.write(k, v)
+    prefill, out = ops.AttnPrefill(1, T, n_q, n_kv, D, n), []
+    names = _kernels(ops, lambda: out.append(prefill.forward(q, cache, pos0=pos0, sinks=sinks)))
+    # up to 512 items: T rows of 8 kv heads and one or two chunks
+    assert names[0] == ("attn_decode_few" if T * 8 * -(-n // 512) <= 512 else "attn_decode"), names
+    one = ops.AttnDecode(1, n_q, n_kv, D, n)
+    for t in (0, 1, T // 2, T - 1):
+        lens = torch.tensor([pos0 + t + 1], dtype=torch.int32, device="cuda")
+        want = one.forward(q[:, t].contiguous(), cache, lens, sinks)
+        assert torch.equal(out[0][:, t].view(torch.int16), want.view(torch.int16)), t
+
+
+@pytest.mark.parametrize("B", [70, 250])       # 560 and 2000 (row, kv head) pairs: less than a round of the resident grid's waves
+def test_attn_output_rows_kept_back_in_less_than_one_round(ops, B):
+    """As above, where every wave has one row at most and the rows are still too many for a workgroup each."""
+    n_q, n_kv, D, S = 16, 8, 64, 192
+    q, K, V, sinks = _mk(B, S, n_q, n_kv, D, seed=34)
+    cache = ops.KVCache(B, n_kv, D, S)
+    cache.write(K.cuda(), V.cuda(), 0)
+    attn = ops.AttnDecode(B, n_q, n_kv, D, S)
+    lens = torch.randint(0, S + 1, (B,), generator=torch.Generator().manual_seed(7), dtype=torch.int32).cuda()
+    flat, out = torch.zeros(B * n_q * D + 8, dtype=torch.bfloat16, device="cuda"), []
+    assert _kernels(ops, lambda: out.append(attn.forward(q.cuda(), cache, lens, sinks.cuda()))) == ["attn_decode"]
+    off = flat[4:4 + B * n_q * D].view(B, n_q, D)
+    attn.forward(q.cuda(), cache, lens, sinks.cuda(), out=off)
+    assert torch.equal(out[0], off)
+
+
 # (sequences, positions, new positions per sequence or 0 for decoding): a workgroup per chunk without and with a merge, a
 # wave per row, a workgroup per row, the prompt kernel
 FORMS = [(3, 300, 0), (3, 1200, 0), (200, 300, 0), (70, 1200, 0), (2, 300, 40)]
