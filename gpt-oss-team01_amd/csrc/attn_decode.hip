@@ -41,11 +41,14 @@ namespace gptoss {
 constexpr int ATT_BLOCK = 64;   // slots per inner iteration
 constexpr float NEG_BIG = -1.0e30f;
 
-// The hardware's exponential by itself, for weights against a running maximum: one below 2^-126 is zero.  (The library
-// function scales such arguments first, five more instructions per score where a block step has about 300 in all; the
-// row's largest weight is about 1, so a sum in fp32 is the same with them or without.)  Where a row's sum meets its sink
-// nothing of that size need be in it: a sink may lie more than 126 above every score, and those few factors take exp2f.
+// The hardware's exponential by itself: a weight below 2^-126 of its row's largest is zero.  (The library function scales
+// such arguments first, five more instructions per score where a block step has about 300 in all; the row's largest weight
+// is about 1, so a sum in fp32 is the same with them or without.)
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// What a row's sum, of maximum m, and its sink are weighed against: the larger of the two, but not so far above m that
+// exp2_hw has no weight left for the sum.  (A sink may lie more than 126 above every score, and bf16 still hold the output.)
+__device__ __forceinline__ float sink_reference(float m, float sink2) { return fminf(fmaxf(m, sink2), m + 100.f); }
 
 // What the exponential of a block's scores is taken of: the distance of score * scale (powers of two) from the row's running
 // maximum m.  Scaling and difference are one fused operation, in every form of the kernels and in blocks with and without
@@ -482,14 +485,15 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
     if (hm >= G) return;
     const int hq = g * G + hm;
     const float sink2 = p.sinks ? p.sinks[hq] * 1.4426950408889634f : -INFINITY;
-    float M = sink2;
+    float M = NEG_BIG;
 #pragma unroll
     for (int w = 0; w < 4; w++) M = fmaxf(M, lds_ml[(w * 16 + hm) * 2]);
-    float denom = exp2f(sink2 - M);
+    M = sink_reference(M, sink2);
+    float denom = exp2_hw(sink2 - M);
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < 4; w++) {
-      const float wgt = exp2f(lds_ml[(w * 16 + hm) * 2] - M);
+      const float wgt = exp2_hw(lds_ml[(w * 16 + hm) * 2] - M);
       denom += lds_ml[(w * 16 + hm) * 2 + 1] * wgt;
       const f32x4 ow = *reinterpret_cast<const f32x4 *>(&lds_o[(w * 16 + hm) * D + d4]);
 #pragma unroll
@@ -506,9 +510,9 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
   const int row_chunks = second ? r1.nchunks : r.nchunks;
   if (row_chunks == 1) {
     float sink2 = sink_logit * 1.4426950408889634f;  // lanes that get here have head == hq
-    float M = fmaxf(m_run, sink2);
-    float w = exp2f(m_run - M);
-    float denom = l_run * w + exp2f(sink2 - M);
+    float M = sink_reference(m_run, sink2);
+    float w = exp2_hw(m_run - M);
+    float denom = l_run * w + exp2_hw(sink2 - M);
     float inv = (denom > 0.f) ? w / denom : 0.f;
     bf16_t *op = HOLD ? hold + hn * D : p.out + ((size_t)bn * p.n_q + hq) * D;
     if (HOLD && lane == 0) *hold_row = b * p.n_q + g * G;
@@ -754,9 +758,9 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
   const int hq = g * G + n;
   if (r.nchunks == 1) {
     const float sink2 = sink_logit * 1.4426950408889634f;
-    const float M = fmaxf(m_run, sink2);
-    const float w = exp2f(m_run - M);
-    const float denom = l_run * w + exp2f(sink2 - M);
+    const float M = sink_reference(m_run, sink2);
+    const float w = exp2_hw(m_run - M);
+    const float denom = l_run * w + exp2_hw(sink2 - M);
     const float inv = (denom > 0.f) ? w / denom : 0.f;
     *reinterpret_cast<u32x2 *>(p.out + ((size_t)b * p.n_q + hq) * D + db * 16 + c * 4) =
         u32x2{pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv)};
@@ -799,7 +803,7 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
   const float sink2 = p.sinks ? p.sinks[hq] * 1.4426950408889634f : -INFINITY;
   const size_t slot0 = (size_t)b * p.max_chunks * p.n_q + hq;
   const size_t slot_stride = p.n_q;
-  float M = sink2;
+  float M = NEG_BIG;
   for (int c0 = 0; c0 < r.nchunks; c0 += ATT_RED_UNROLL) {
     float m[ATT_RED_UNROLL];
 #pragma unroll
@@ -808,7 +812,8 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 #pragma unroll
     for (int u = 0; u < ATT_RED_UNROLL; u++) M = fmaxf(M, m[u]);
   }
-  float denom = exp2f(sink2 - M);
+  M = sink_reference(M, sink2);
+  float denom = exp2_hw(sink2 - M);
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int c0 = 0; c0 < r.nchunks; c0 += ATT_RED_UNROLL) {
     float m[ATT_RED_UNROLL], l[ATT_RED_UNROLL];
@@ -825,7 +830,7 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 #pragma unroll
     for (int u = 0; u < ATT_RED_UNROLL; u++) {
       if (c0 + u < r.nchunks) {
-        const float w = exp2f(m[u] - M);
+        const float w = exp2_hw(m[u] - M);
         denom += l[u] * w;
 #pragma unroll
         for (int q = 0; q < 4; q++) acc[q] += o[u][q] * w;
@@ -1039,9 +1044,9 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
   if (!col_live) return;
   const int hq = g * G + hn;
   const float sink2 = sink_logit * 1.4426950408889634f;
-  const float M = fmaxf(m_run, sink2);
-  const float w = exp2f(m_run - M);
-  const float denom = l_run * w + exp2f(sink2 - M);
+  const float M = sink_reference(m_run, sink2);
+  const float w = exp2_hw(m_run - M);
+  const float denom = l_run * w + exp2_hw(sink2 - M);
   const float inv = (denom > 0.f) ? w / denom : 0.f;
   bf16_t *op = p.out + ((size_t)bn * p.n_q + hq) * D;
 #pragma unroll
