@@ -46,29 +46,31 @@ int gptoss_engine::create_logits_staging() {
 
 // The first m rows of the logits to the caller's array, through the pinned halves in turn: a half travels while the one
 // before is copied out.  (Into the caller's own pages the runtime pins them, or bounces, at every call: one row of a
-// vocabulary of 201088 took 180 us behind its step.)
+// vocabulary of 201088 took 180 us behind its step.)  Rows travel with their padding, one behind the other, and lose it on
+// the host: a copy for each row of a padded vocabulary costs 8 us (512 rows of 1000 logits: 4.1 ms instead of 0.2).
 int gptoss_engine::copy_logits(int m, float *host_logits) {
-  const size_t row = sizeof(float) * vocab, total = row * m;
+  const size_t row = sizeof(float) * vocab, stride = sizeof(float) * vocab_rows, total = stride * m;
   struct Piece {
-    char *to;
-    size_t bytes;
+    size_t at, bytes;   // of the device's rows
   } piece[2] = {};
   auto take = [&](int half) -> int {
     GPTOSS_HIP(hipEventSynchronize(logits_there[half]));
-    memcpy(piece[half].to, (char *)h_logits + half * LOGITS_HALF, piece[half].bytes);
+    const size_t begin = piece[half].at, end = begin + piece[half].bytes;
+    const char *there = (const char *)h_logits + half * LOGITS_HALF;
+    for (size_t r = begin / stride; r * stride < end; r++) {
+      const size_t from = std::max(begin, r * stride), to = std::min(end, r * stride + row);
+      if (from < to) memcpy((char *)host_logits + r * row + (from - r * stride), there + (from - begin), to - from);
+    }
     return GPTOSS_OK;
   };
   int n = 0;
   for (size_t at = 0; at < total; n++) {
-    const size_t r = at / row, within = at % row;
-    // rows that lie one behind the other go together
-    const size_t bytes = std::min(LOGITS_HALF, vocab == vocab_rows ? total - at : row - within);
     if (n >= 2) GPTOSS_STEP(take(n & 1));
-    piece[n & 1] = {(char *)host_logits + at, bytes};
-    GPTOSS_HIP(hipMemcpyAsync((char *)h_logits + (n & 1) * LOGITS_HALF, (char *)(logits + r * vocab_rows) + within, bytes,
+    piece[n & 1] = {at, std::min(LOGITS_HALF, total - at)};
+    GPTOSS_HIP(hipMemcpyAsync((char *)h_logits + (n & 1) * LOGITS_HALF, (char *)logits + at, piece[n & 1].bytes,
                               hipMemcpyDeviceToHost, stream));
     GPTOSS_HIP(hipEventRecord(logits_there[n & 1], stream));
-    at += bytes;
+    at += piece[n & 1].bytes;
   }
   for (int i = std::max(0, n - 2); i < n; i++) GPTOSS_STEP(take(i & 1));
   return GPTOSS_OK;
