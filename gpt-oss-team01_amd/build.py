@@ -25,7 +25,7 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-Wno-u
 DEVICE = ["--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 #: sources every model class links
-CORE = ("common.cpp", "engine.cpp", "model_registry.cpp", "glue.hip", "precise.hip", "gemm_dense.cpp",
+CORE = ("common.cpp", "engine.cpp", "host_pool.cpp", "model_registry.cpp", "glue.hip", "precise.hip", "gemm_dense.cpp",
         "gemm_bf16.hip", "gemm_few.hip", "gemm_mixed_bf16.hip", "gemm_tall.hip")
 #: architecture -> sources of its class beside CORE (None: all of them)
 MODELS = {"gpt-oss": None, "Nezavik": ("model_nezavik.cpp", "recurrent.hip", "window_attn.hip"),

@@ -15,41 +15,74 @@ def _ptr(a):
     return a.ctypes.data_as(C.c_void_p)
 
 
-class _Block:
-    """Host memory of an array that was handed out; goes back to its pool with the last array over it."""
-
-    def __init__(self, pool, memory, shape):
-        self._pool, self._memory = pool, memory
-        self.__array_interface__ = {"version": 3, "typestr": "<f4", "shape": shape, "data": (memory.ctypes.data, False)}
-
-    def __del__(self):
-        self._pool.give(self._memory)
+def _numpy_set_handler():
+    """numpy's PyDataMem_SetHandler (of its C API since 1.22, per context): who allocates the arrays made from now on."""
+    try:
+        from numpy._core import _multiarray_umath as core
+    except ImportError:
+        from numpy.core import _multiarray_umath as core
+    pointer = C.pythonapi.PyCapsule_GetPointer
+    pointer.restype, pointer.argtypes = C.c_void_p, [C.py_object, C.c_char_p]
+    api = C.cast(pointer(core._ARRAY_API, None), C.POINTER(C.c_void_p))
+    return C.PYFUNCTYPE(C.py_object, C.py_object)(api[304])
 
 
 class _HostPool:
-    """Memory for results in host arrays, kept where the caller has dropped the array it was last used for: the first
-    touch of fresh pages costs ten times the copy into them (3 MB of logits: 700 us of page faults, 40 us of copying).
-    At most `limit` bytes are kept; what is more is freed."""
+    """Result arrays whose memory is kept for reuse when the last array over it is gone (csrc/host_pool.cpp): at most
+    `limit` bytes, the longest unused given up first."""
 
     def __init__(self, limit):
-        self._limit, self._free, self._kept, self._lock = limit, {}, 0, threading.RLock()
+        self._limit, self._pool, self._lock = limit, None, threading.Lock()
+
+    def _open(self):
+        with self._lock:
+            if self._pool is None:
+                self._L = L = _l.load()
+                L.gptoss_host_pool_create.restype, L.gptoss_host_pool_create.argtypes = C.c_void_p, [C.c_size_t]
+                L.gptoss_host_pool_release.restype, L.gptoss_host_pool_release.argtypes = None, [C.c_void_p]
+                L.gptoss_host_pool_kept.restype = C.c_size_t
+                L.gptoss_host_pool_kept.argtypes = [C.c_void_p, C.POINTER(C.c_size_t), C.c_size_t, C.POINTER(C.c_size_t)]
+                pool = L.gptoss_host_pool_create(self._limit)
+                if not pool:
+                    raise MemoryError("result arrays")
+                new = C.pythonapi.PyCapsule_New
+                new.restype, new.argtypes = C.py_object, [C.c_void_p, C.c_char_p, C.c_void_p]
+                self._handler, self._set_handler = new(pool, b"mem_handler", None), _numpy_set_handler()
+                self._pool = pool
 
     def empty(self, *shape):
-        n = -(-4 * math.prod(shape) // 4096) * 4096
-        if not 4096 <= n <= self._limit:
+        """An array as numpy.empty gives it, on memory of the pool where that is worth it."""
+        if not 0 < 4 * math.prod(shape) <= self._limit:
             return np.empty(shape, np.float32)
-        with self._lock:   # (re-entrant: a block may be collected, and given back, while it is held)
-            free = self._free.get(n)
-            memory = free.pop() if free else None
-            if memory is not None:
-                self._kept -= n
-        return np.asarray(_Block(self, np.empty(n, np.uint8) if memory is None else memory, shape))
+        if self._pool is None:
+            self._open()
+        before = self._set_handler(self._handler)
+        try:
+            return np.empty(shape, np.float32)
+        finally:
+            self._set_handler(before)
 
-    def give(self, memory):
-        with self._lock:
-            if self._kept + memory.nbytes <= self._limit:
-                self._free.setdefault(memory.nbytes, []).append(memory)
-                self._kept += memory.nbytes
+    def _kept_blocks(self):
+        if self._pool is None:
+            return 0, []
+        n, sizes = C.c_size_t(), (C.c_size_t * 65536)()
+        kept = self._L.gptoss_host_pool_kept(self._pool, sizes, 65536, C.byref(n))
+        return kept, list(sizes[:n.value])
+
+    @property
+    def _kept(self):
+        """Bytes that are kept."""
+        return self._kept_blocks()[0]
+
+    @property
+    def _free(self):
+        """Kept blocks by size."""
+        sizes = self._kept_blocks()[1]
+        return {n: [n] * sizes.count(n) for n in set(sizes)}
+
+    def __del__(self):
+        if self._pool is not None:
+            self._L.gptoss_host_pool_release(self._pool)
 
 
 _results = _HostPool(64 << 20)

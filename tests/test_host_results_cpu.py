@@ -51,3 +51,52 @@ def test_threads_never_share_memory_in_use():
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not wrong
+
+
+def test_arrays_own_their_memory():
+    """Resized in place like any array: smaller, within its pages, beyond them, and with the memory back in the pool after."""
+    pool = load_pkg("engine")._HostPool(1 << 20)
+    a = pool.empty(3, 1000)
+    assert a.flags.owndata and a.base is None
+    a[:] = np.arange(3000).reshape(3, 1000)
+    for rows in (2, 3, 50, 1):
+        a.resize((rows, 1000))
+        keep = min(rows, 2)
+        assert (a[:keep].ravel() == np.arange(1000 * keep)).all()
+    assert (a.size, a.flags.owndata) == (1000, True)
+    del a
+    gc.collect()
+    assert pool._kept > 0
+    kept = np.empty(1000)
+    assert kept.flags.owndata and np.zeros(10).sum() == 0      # arrays made elsewhere are numpy's own
+
+
+def test_sizes_that_are_no_longer_asked_for_make_room():
+    """A batch that shrinks: what the larger results left must not keep the smaller ones from being reused."""
+    pool = load_pkg("engine")._HostPool(1 << 20)
+    for rows in range(100, 10, -1):
+        pool.empty(rows, 1000)
+    gc.collect()
+    assert pool._kept <= 1 << 20
+    where = set()
+    for _ in range(5):
+        a = pool.empty(8, 1000)
+        where.add(a.ctypes.data)
+        del a
+        gc.collect()
+    assert len(where) == 1 and 8 * 4096 in pool._free
+
+
+def test_arrays_outlive_their_pool():
+    engine = load_pkg("engine")
+    pool = engine._HostPool(1 << 20)
+    a, b = pool.empty(20, 1000), pool.empty(20, 1000)
+    a[:], view = 3.0, b[2:]
+    view[:] = 4.0
+    del pool, b
+    gc.collect()
+    assert (a == 3.0).all() and (view == 4.0).all()
+    a.resize((40, 1000))
+    assert (a[:20] == 3.0).all()
+    del a, view
+    gc.collect()
