@@ -42,7 +42,7 @@ struct TokenExperts {
       for (int s = 0; s < KMAX; s++)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-          const float next = __fadd_rn(agg[q], __fmul_rn(v[s][q], w[s]));
+          const float next = __builtin_fmaf(v[s][q], w[s], agg[q]);
           agg[q] = s < k ? next : agg[q];
         }
     } else {
@@ -51,7 +51,7 @@ struct TokenExperts {
         if (s < k) {
           const f32x4 v = *reinterpret_cast<const f32x4 *>(y2 + (size_t)rows[s] * H + h);
 #pragma unroll
-          for (int q = 0; q < 4; q++) agg[q] = __fadd_rn(agg[q], __fmul_rn(v[q], w[s]));
+          for (int q = 0; q < 4; q++) agg[q] = __builtin_fmaf(v[q], w[s], agg[q]);
         }
       }
     }
@@ -60,8 +60,8 @@ struct TokenExperts {
 };
 
 // Weighted combine: out[b,:] (+)= sum over the token's k experts, in ascending expert order (the
-// order of the reference CPU loop, run.cpp:642-704), of w * y2[row of that pair].  The compiler
-// fuses every product into its sum, in all forms of the kernel alike.
+// order of the reference CPU loop, run.cpp:642-704), of w * y2[row of that pair], every product
+// fused into the sum (one rounding each), in all forms of the kernel alike.
 // KMAX: room for a token's experts.
 template <int VPT, int KMAX = 8>  // float4 chunks per thread: rows of at most 1024 * VPT floats (0: any length, a loop)
 __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ y2,

@@ -14,8 +14,9 @@ class _PreNorm(C.Structure):   # MoePreNorm of gemm.hpp
     _fields_ = [("x", C.c_void_p), ("residual", C.c_void_p), ("weight", C.c_void_p)]
 
 
-def _forward_norm(layer, x, residual, weight, out):
-    """gptoss::moe_forward_norm, which has no C entry point, by its linker name; -> its t, bf16 [B, H]."""
+def _forward_norm(layer, x, residual, weight, out, next_weight=None, next_t=None):
+    """gptoss::moe_forward_norm, which has no C entry point, by its linker name; -> its t, bf16 [B, H].  With next_weight
+    the norm of the updated rows goes to next_t."""
     f = getattr(layer.L, "_ZN6gptoss16moe_forward_normEPK18gptoss_moe_weightsPKviPfPvmP12ihipStream_tiPKfPtPKNS_10MoePreNormE")
     f.restype = C.c_int
     f.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p, C.c_int, C.c_void_p,
@@ -25,8 +26,9 @@ def _forward_norm(layer, x, residual, weight, out):
     assert residual is None or (residual.shape == x.shape and residual.is_contiguous())
     t = torch.empty(B, H, dtype=torch.bfloat16, device="cuda")
     pre = _PreNorm(x.data_ptr(), residual.data_ptr() if residual is not None else None, weight.data_ptr())
+    behind = (None, None) if next_weight is None else (next_weight.data_ptr(), next_t.data_ptr())
     load_pkg("lib").check(f(C.byref(layer.desc), t.data_ptr(), B, out.data_ptr(), layer.ws.data_ptr(), layer.ws_bytes,
-                            torch.cuda.current_stream().cuda_stream, 0, None, None, C.byref(pre)))
+                            torch.cuda.current_stream().cuda_stream, 0, *behind, C.byref(pre)))
     layer._last_B = B
     return t
 
@@ -57,3 +59,23 @@ def test_a_block_with_its_norm_equals_its_parts(ops, H, E, with_residual):
         want = [x_want, t_want, out_want, logits, w, ids, offsets, order, place]
         for name, a, b in zip("x t out logits weights ids offsets order place".split(), got, want):
             assert torch.equal(a, b), (B, name)
+
+
+# k: places for four experts and for eight; H: every number of chunks per thread that the fused kernel has
+@pytest.mark.parametrize("k", [1, 4, 5, 8])
+@pytest.mark.parametrize("H", [64, 1024, 2048, 2880, 4096])
+def test_a_block_with_the_norm_behind_it_equals_its_parts(ops, k, H):
+    g = torch.Generator(device="cuda").manual_seed(H + k)
+    rnd = lambda *s, std=1.0: torch.randn(*s, generator=g, device="cuda") * std
+    n = lambda *s, **kw: rnd(*s, **kw).bfloat16()
+    E, I, B = 16, 64, 23
+    layer = ops.MoeLayer(n(E, H, std=H ** -0.5), n(E), n(E, 2 * I, H, std=0.05), n(E, 2 * I), n(E, H, I, std=0.05), n(E, H),
+                         top_k=k, max_tokens=B)
+    weight, next_weight = 1 + rnd(H, std=0.1), 1 + rnd(H, std=0.1)
+    x, residual = rnd(B, H) * 3, rnd(B, H)
+    want = x.clone()
+    got_t = torch.empty(B, H, dtype=torch.bfloat16, device="cuda")
+    _forward_norm(layer, x, residual, weight, x, next_weight, got_t)       # accumulates into x, as the engine has it
+    layer.forward(ops.rmsnorm(want, weight, residual), out=want, accumulate=True)
+    assert torch.equal(x, want)
+    assert torch.equal(got_t, ops.rmsnorm(want, next_weight))
