@@ -79,13 +79,26 @@ static int gemm_prepare_device() {
   return GPTOSS_OK;
 }
 
+// Dense problems with tiles of 64 rows: the few-row kernel for one tile (65536 x 2048, 64 rows 55 -> 53 us, 24576 x 2880 45
+// -> 33), for up to 1152 of its 32-column blocks, one round and a little, and where ten row tiles or more share each of
+// them up to 1536 (4096 x 4096, 640 rows 52 -> 43) or, with a long K, 1856 (2048 x 8192, 1800 rows 97 -> 87, 2880 x 4096,
+// 1280 rows 53 -> 49; 2048 x 2048, 1800 rows 27.7 -> 29.2).  Beyond that the streaming kernel of that size: 2048 x 2048,
+// 2047 rows 35.3 -> 31.0, 10240 x 2048, 257 rows 34.0 -> 31.6, 5120 x 2880, 768 rows 41.6 -> 39.5.
+// With tiles of 32 rows the few-row kernel is the better one wherever they are chosen.
+static bool dense_few(int rows_per_tile, int tiles, int N, int K) {
+  return rows_per_tile == 32 || tiles == 1 ||
+         (long long)tiles * (N / 32) <= (tiles < 10 ? 1152 : K < 4096 ? 1536 : 1856);
+}
+
 int run_gemm_dense(const GemmParams &p, int epi, int rows_per_tile, int max_tiles, hipStream_t s) {
   // output and operand offsets inside the kernels are 32-bit element counts
   const long long max_rows = p.tiles ? (long long)max_tiles * rows_per_tile : p.dense_rows;
   GPTOSS_REQUIRE(max_rows * p.N < (1ll << 32) && max_rows * p.K < (1ll << 32), GPTOSS_ERR_DIM,
                  "run_gemm: rows x columns must stay below 2^32 elements (rows<=%lld N=%d K=%d)", max_rows, p.N, p.K);
   if (rows_per_tile == 256) return run_gemm_tall(p, epi, max_tiles, max_rows, s);
-  if (epi != EPI_ARGMAX && gemm_few_applies(p, rows_per_tile, max_tiles) && (!p.tiles || grouped_few(p, rows_per_tile, max_tiles))) return run_gemm_few(p, false, epi, rows_per_tile, max_tiles, s);
+  if (epi != EPI_ARGMAX && gemm_few_applies(p, rows_per_tile, max_tiles) &&
+      (p.tiles ? grouped_few(p, rows_per_tile, max_tiles) : epi == EPI_PARTIAL || dense_few(rows_per_tile, max_tiles, p.N, p.K)))
+    return run_gemm_few(p, false, epi, rows_per_tile, max_tiles, s);
   int prc = gemm_prepare_device();
   if (prc != GPTOSS_OK) return prc;
   if (epi == EPI_F32) return dispatch_rows<EPI_F32>(p, rows_per_tile, max_tiles, s);
@@ -136,20 +149,27 @@ static double few_us(int mb, long long blocks, int slabs) {
 // Row tile of a dense GEMM below the 256-row kernels: the one with the least estimated time; ties go to the larger tile
 // (fewer re-reads of the weights).  Against the streaming kernels alone (96 rows for the QKV projection of 1024 rows, 64
 // for the output projection): 5120 x 2880, 96 / 200 / 400 rows 39 / 32 / 34 -> 16 / 21 / 30 us; 2880 x 4096 52 / 41 / 42
-// -> 17 / 22 / 26; from about 500 rows and 5000 columns on they are the better ones.  Hundreds of column tiles (an
-// unembedding) fill the chip at any size: the smallest tile that holds every row up to 96, then 128, measured best at 1024.
+// -> 17 / 22 / 26; from about 500 rows and 5000 columns on they are the better ones.  The estimates leave out what a second
+// row tile costs in reads of the weights, so from 65 column tiles on up to 128 rows are one tile: 24576 x 2880, 65 / 128
+// rows 65 / 69 us with tiles of 64, 46 / 54 with one.  Hundreds of column tiles (an unembedding) fill the chip at any size:
+// one tile up to 96 rows, then 128, measured best at 1024.
 static int dense_rows_per_tile(int B, int n_col_tiles, int N, int K, int epi) {
   if (B >= 2048) return 160;
-  if (n_col_tiles >= 128 || epi == EPI_ARGMAX) {
+  if (n_col_tiles >= 128 || epi == EPI_ARGMAX || (n_col_tiles > 64 && B <= 128)) {
     if (B <= 96) return align_up(B, 32);
     if (n_col_tiles >= 64) return 128;
   }
   double best = 0.0;
   int rpt = 160;
   for (int mb = 1; mb <= 5; mb++) {
-    const long long tiles = cdiv(B, 32 * mb);
-    const double us = mb <= 2 && epi != EPI_ARGMAX ? few_us(mb, tiles * (N / 32), K / 64)
-                                                   : streaming_us(mb, tiles * n_col_tiles * 8, K / 64);
+    const int tiles = cdiv(B, 32 * mb);
+    double us = streaming_us(mb, (long long)tiles * n_col_tiles * 8, K / 64);
+    if (epi != EPI_ARGMAX && mb <= 2 && dense_few(32 * mb, tiles, N, K)) {
+      const long long blocks = (long long)tiles * (N / 32);
+      us = few_us(mb, blocks, K / 64);
+      // (one wave staging 64 rows starts late, which shows where K is short: 512 x 512, 2047 rows 13.0 us, 10.1 with 32)
+      if (mb == 2 && blocks <= FEW_SOLO_BLOCKS) us += 2.0;
+    }
     if (mb == 1 || us <= best) {
       best = us;
       rpt = 32 * mb;
