@@ -860,13 +860,6 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 constexpr int TILE_WAVES = 8;
 constexpr int TILE_ROWS = 2 * TILE_WAVES;
 
-// 16 bytes per lane, from sbase + voff to LDS address lds + 16 * lane
-__device__ __forceinline__ void load_to_lds(unsigned lds, uint32_t voff, const void *sbase) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
-               "v"(voff), "s"(sbase)
-               : "memory");
-}
-
 template <int D>
 __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(AttnParams p) {
   constexpr int KS = D / 32;

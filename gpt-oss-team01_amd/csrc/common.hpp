@@ -83,6 +83,14 @@ __device__ __forceinline__ const_as<T> constant_ptr(const T *q) {
   return (const_as<T>)(q);
 }
 
+// 16 bytes per lane, from sbase + voff to LDS address lds + 16 * lane.  The compiler does not count these loads: whoever
+// reads what they bring waits for the vector-memory counter by itself first.
+__device__ __forceinline__ void load_to_lds(unsigned lds, uint32_t voff, const void *sbase) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
+               "v"(voff), "s"(sbase)
+               : "memory");
+}
+
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) {
   union {
     u32x4 u;

@@ -54,12 +54,6 @@ struct TallShape {
   static_assert(NM >= NR + 2 * (LA / 4 + LW / 2), "room for a k-step's reads and loads between its MFMAs");
 };
 
-__device__ __forceinline__ void tall_dma(unsigned lds_addr, uint32_t voff, const void *sbase) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(
-                   __builtin_amdgcn_readfirstlane(lds_addr)),
-               "v"(voff), "s"(sbase)
-               : "memory");
-}
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -287,11 +281,11 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
   // W load instruction q of this wave for stage s of an item, into W buffer buf
   const uint32_t voff_w = lane * 16;
   auto issue_w = [&](const TallSrc<SH> &t, int s, int buf, int q) {
-    tall_dma(lds_base + buf * SH::W_BYTES + (w * LW + q) * 1024, voff_w, t.w[q] + (size_t)s * 2048);
+    load_to_lds(lds_base + buf * SH::W_BYTES + (w * LW + q) * 1024, voff_w, t.w[q] + (size_t)s * 2048);
   };
   // A load instruction q of this wave for chunk c of an item, into A buffer buf
   auto issue_a = [&](const TallSrc<SH> &t, int c, int buf, int q) {
-    tall_dma(lds_base + SH::A_OFF + buf * SH::A_BYTES + (w * LA + q) * 1024, t.a[q], abase + (size_t)c * 128);
+    load_to_lds(lds_base + SH::A_OFF + buf * SH::A_BYTES + (w * LA + q) * 1024, t.a[q], abase + (size_t)c * 128);
   };
 
   f32x16 acc[CB][RB];   // [column block][row block]
