@@ -67,7 +67,9 @@ int moe_tall_min_rows() {
 
 int moe_rows_per_tile(int B, int k, int E, bool mxfp4) {
   double avg = (double)B * k / E;
-  double need = k == E ? avg : avg + 2.5 * sqrt(avg);   // (every token on every expert: nothing to deviate)
+  // Every token on every expert: nothing to deviate.  Short of that the deviation is sqrt(avg (1 - k / E)), but a margin cut
+  // to that is too small: 380 tokens, 4 of 32 experts, 312 -> 361 us with tiles of 64; 166 tokens, 2 of 16, 74 -> 81.
+  double need = k == E ? avg : avg + 2.5 * sqrt(avg);
 
   if (need <= 32) return 32;
   if (need <= 64) return 64;

@@ -1,5 +1,5 @@
-// MoE routing for gfx950: router GEMM (bf16 MFMA 16x16x32), top-k + softmax gating with wave
-// shuffles, and a stable counting sort of the (token,slot) pairs by expert built from wave
+// MoE routing for gfx950: router GEMM (bf16 MFMA 16x16x32), top-k + softmax gating with exchanges
+// between lanes in registers, and a stable counting sort of the (token,slot) pairs by expert built from wave
 // ballots and an LDS histogram (no global atomics), which also emits the tile list that the
 // grouped GEMMs schedule from.
 #include <mutex>

@@ -540,6 +540,8 @@ static void launch_scan_kind(const Scan &p, const StepRows &r, hipStream_t s) {
   // Stretches of few heads and sequences: with two columns per lane half of the chip would be idle, or every SIMD have
   // one wave, which issues an instruction every seven cycles (8 prompts of 1000 and 16 heads of 128 x 128, 256 workgroups
   // against 512: delta rule 455 -> 409 us, per key channel 544 -> 521; 32 heads of 128 x 64, state space 383 -> 342).
+  // Beyond 256 a lane's second column costs less than a second workgroup: 12 prompts of 500, delta rule 336 against 360 us
+  // with one column, per key channel 403 / 450, state space 249 / 228; 16 prompts 359 / 429, 444 / 539, 279 / 346.
   const bool few = (long long)r.n_seg * p.heads * cdiv(p.V, 64) <= 256;
   if (r.longest == 1) scan_kernel<NI, KIND, true, 2><<<grid(64), 256, 0, s>>>(p, r.segs, r.n_seg);
   else if (few) scan_kernel<NI, KIND, false, 1><<<grid(32), 256, 0, s>>>(p, r.segs, r.n_seg);
