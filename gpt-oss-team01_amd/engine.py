@@ -80,12 +80,15 @@ class _HostPool:
         sizes = self._kept_blocks()[1]
         return {n: [n] * sizes.count(n) for n in set(sizes)}
 
+    def release(self):
+        """Give back what is kept; memory of arrays that are still there goes with them."""
+        with self._lock:
+            pool, self._pool = self._pool, None
+        if pool is not None:
+            self._L.gptoss_host_pool_release(pool)
+
     def __del__(self):
-        if self._pool is not None:
-            self._L.gptoss_host_pool_release(self._pool)
-
-
-_results = _HostPool(64 << 20)
+        self.release()
 
 
 class Engine:
@@ -129,6 +132,7 @@ class Engine:
 
     def _adopt(self, handle):
         self._h = handle
+        self._results = _HostPool(64 << 20)
         self.info = _l.ModelInfo()
         _l.check(self.L.gptoss_engine_info(handle, C.byref(self.info)))
         self.max_batch, self.max_seq = self.info.max_batch, self.info.max_seq
@@ -197,7 +201,7 @@ class Engine:
         slot = np.ascontiguousarray(slots, dtype=np.int32)
         pos = np.ascontiguousarray(positions, dtype=np.int32)
         want = np.ascontiguousarray(want, dtype=np.int32)
-        out = _results.empty(want.size, self.info.vocab)
+        out = self._results.empty(want.size, self.info.vocab)
         _l.check(self.L.gptoss_engine_step_logits(self._h, tok.size, _ptr(tok), _ptr(slot), _ptr(pos), want.size,
                                                   _ptr(want), _ptr(out)))
         return out
@@ -219,6 +223,7 @@ class Engine:
         if getattr(self, "_h", None):
             self.L.gptoss_engine_destroy(self._h)
             self._h = None
+            self._results.release()
 
     def __del__(self):
         self.close()

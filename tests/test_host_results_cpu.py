@@ -1,6 +1,7 @@
 """Memory of results in host arrays: kept for reuse only when no array uses it, bounded, safe across threads."""
 import gc
 import threading
+import types
 
 import numpy as np
 
@@ -100,3 +101,21 @@ def test_arrays_outlive_their_pool():
     assert (a[:20] == 3.0).all()
     del a, view
     gc.collect()
+
+
+def test_a_closed_engine_gives_back_what_its_results_left():
+    mod = load_pkg("engine")
+    e = mod.Engine.__new__(mod.Engine)
+    e.L = types.SimpleNamespace(gptoss_engine_info=lambda *a: 0, gptoss_engine_destroy=lambda h: None)
+    e._adopt(1)
+    pool = e._results
+    a, b = pool.empty(20, 1000), pool.empty(20, 1000)
+    a[:] = 3.0
+    del b
+    gc.collect()
+    assert pool._kept > 0
+    e.close()
+    assert pool._kept == 0 and (a == 3.0).all()
+    del a                                                  # the pool is released: its memory goes, nothing is kept
+    gc.collect()
+    assert pool._kept == 0 and pool.empty(20, 1000).flags.owndata
