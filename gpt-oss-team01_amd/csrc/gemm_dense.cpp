@@ -79,15 +79,38 @@ static int gemm_prepare_device() {
   return GPTOSS_OK;
 }
 
-// Dense problems with tiles of 64 rows: the few-row kernel for one tile (65536 x 2048, 64 rows 55 -> 53 us, 24576 x 2880 45
-// -> 33), for up to 1152 of its 32-column blocks, one round and a little, and where ten row tiles or more share each of
-// them up to 1536 (4096 x 4096, 640 rows 52 -> 43) or, with a long K, 1856 (2048 x 8192, 1800 rows 97 -> 87, 2880 x 4096,
-// 1280 rows 53 -> 49; 2048 x 2048, 1800 rows 27.7 -> 29.2).  Beyond that the streaming kernel of that size: 2048 x 2048,
-// 2047 rows 35.3 -> 31.0, 10240 x 2048, 257 rows 34.0 -> 31.6, 5120 x 2880, 768 rows 41.6 -> 39.5.
-// With tiles of 32 rows the few-row kernel is the better one wherever they are chosen.
+// Estimated us of a launch, for choosing its kernel, row tile and parts.  `blocks`: 32-column blocks of all its work items,
+// `slabs`: 64-k slabs an item walks.  A round of work items takes a part of its own (first loads, epilogue) beside its slabs,
+// and both take longer the more CUs are at it: terms per round and terms per full round's worth of items.
+// Streaming kernels (gemm_kernel.hpp): items of MB 32-row blocks x 256 columns, 256 to a round.
+// Few-row kernels (gemm_few_kernel.hpp): 128 columns per workgroup, 256 to a round; up to 512 blocks a workgroup is one block.
+// Fitted to every tile and every number of parts that a launch could have, weights from HBM: 27 shapes of 512-16384 columns
+// and K 256-8192 at 34 row counts of 8-2047, and 12 shapes at 26 with their K cut as well; 4 to 12 % rms (64 rows in several
+// rounds: 5 % on top, as what they gain at a tie is less than what they lose).  With one fixed part per launch, products of
+// short K or narrow N took up to 37 % longer than on streaming kernels alone (us: 1280 x 1280 with its K cut, 257 rows
+// 11.1 instead of 8.1; 2048 x 256, 257 rows 8.0 instead of 6.3).
+static double streaming_us(int mb, long long blocks, int slabs) {
+  // [mb - 1]: launch; per round, and per slab of it; per full round's items, and per slab of them
+  static const double t[5][5] = {{3.2, 0.63, 0.496, 1.8, 0.028}, {3.5, 1.35, 0.533, 3.3, 0.106}, {4.0, 2.5, 0.578, 3.8, 0.145},
+                                 {4.3, 3.7, 0.635, 3.9, 0.222}, {5.0, 5.0, 0.724, 3.5, 0.303}};
+  const double *c = t[mb - 1];
+  return c[0] + (double)((blocks + 2047) / 2048) * (c[1] + c[2] * slabs) + blocks / 2048.0 * (c[3] + c[4] * slabs);
+}
+
+static double few_us(int mb, long long blocks, int slabs) {
+  if (blocks <= FEW_SOLO_BLOCKS) {
+    const double full = (double)blocks / FEW_SOLO_BLOCKS;
+    return mb == 1 ? 3.6 + 0.078 * slabs + full * (1.3 + 0.142 * slabs) : 5.0 + 0.239 * slabs + full * (1.8 + 0.079 * slabs);
+  }
+  const double rounds = (double)((blocks + 1023) / 1024), full = blocks / 1024.0;
+  return mb == 1 ? 3.4 + rounds * (1.1 + 0.175 * slabs) + full * (0.7 + 0.071 * slabs)
+                 : 3.9 + rounds * (1.58 + 0.191 * slabs) + full * (1.15 + 0.147 * slabs);
+}
+
+// Uncut dense problems: the kernel that is estimated to be the faster one with this row tile.
 static bool dense_few(int rows_per_tile, int tiles, int N, int K) {
-  return rows_per_tile == 32 || tiles == 1 ||
-         (long long)tiles * (N / 32) <= (tiles < 10 ? 1152 : K < 4096 ? 1536 : 1856);
+  const int mb = rows_per_tile / 32;
+  return mb <= 2 && few_us(mb, (long long)tiles * (N / 32), K / 64) < streaming_us(mb, (long long)tiles * gemm_col_tiles(N) * 8, K / 64);
 }
 
 int run_gemm_dense(const GemmParams &p, int epi, int rows_per_tile, int max_tiles, hipStream_t s) {
@@ -130,29 +153,12 @@ static int argmax_tall_min_rows() {
   return v;
 }
 
-// Estimated us of a launch, for choosing its row tile and its parts.  `blocks`: 32-column blocks of all its work items,
-// `slabs`: 64-k slabs an item walks.
-// Streaming kernels (gemm_kernel.hpp), items of MB 32-row blocks x 256 columns on 256 CUs, (0.39 + 0.115 MB) us per slab
-// (measured at 1024 rows: 0.50 / 0.64 / 0.76 / 0.85 us for 32 / 64 / 96 / 128 rows).
-// Few-row kernels (gemm_few_kernel.hpp), 128 columns per workgroup, two workgroups per CU: 0.25 us per slab and round of
-// 256 workgroups for 32 rows, 0.32 for 64; up to 512 blocks a workgroup is one block, two per CU.  (Measured on weights
-// that come from HBM, 2048-16384 columns, K 2048-4096, 65-2000 rows: within a fifth of the estimate up to four rounds.)
-static double streaming_us(int mb, long long blocks, int slabs) {
-  return 5.0 + (double)((blocks + 2047) / 2048) * slabs * (0.39 + 0.115 * mb);
-}
-
-static double few_us(int mb, long long blocks, int slabs) {
-  if (blocks <= FEW_SOLO_BLOCKS) return 5.0 + slabs * (mb == 1 ? (blocks <= 256 ? 0.13 : 0.20) : (blocks <= 256 ? 0.28 : 0.33));
-  return 6.5 + (double)((blocks + 1023) / 1024) * slabs * (mb == 1 ? 0.25 : 0.32);
-}
-
 // Row tile of a dense GEMM below the 256-row kernels: the one with the least estimated time; ties go to the larger tile
-// (fewer re-reads of the weights).  Against the streaming kernels alone (96 rows for the QKV projection of 1024 rows, 64
-// for the output projection): 5120 x 2880, 96 / 200 / 400 rows 39 / 32 / 34 -> 16 / 21 / 30 us; 2880 x 4096 52 / 41 / 42
-// -> 17 / 22 / 26; from about 500 rows and 5000 columns on they are the better ones.  The estimates leave out what a second
-// row tile costs in reads of the weights, so from 65 column tiles on up to 128 rows are one tile: 24576 x 2880, 65 / 128
-// rows 65 / 69 us with tiles of 64, 46 / 54 with one.  Hundreds of column tiles (an unembedding) fill the chip at any size:
-// one tile up to 96 rows, then 128, measured best at 1024.
+// (fewer re-reads of the weights).  Timed with every tile at the 918 sizes above: 1 % slower than the best one on average
+// and 16 % faster than the streaming kernels alone (5120 x 2880, 97 / 200 / 364 rows 32 / 32 / 33 -> 19 / 21 / 22 us).  The estimates leave
+// out what a second row tile costs in reads of the weights, so from 65 column tiles on up to 128 rows are one tile:
+// 24576 x 2880, 65 / 128 rows 65 / 69 us with tiles of 64, 46 / 54 with one.  Hundreds of column tiles (an unembedding) fill
+// the chip at any size: one tile up to 96 rows, then 128, measured best at 1024.
 static int dense_rows_per_tile(int B, int n_col_tiles, int N, int K, int epi) {
   if (B >= 2048) return 160;
   if (n_col_tiles >= 128 || epi == EPI_ARGMAX || (n_col_tiles > 64 && B <= 128)) {
@@ -163,13 +169,9 @@ static int dense_rows_per_tile(int B, int n_col_tiles, int N, int K, int epi) {
   int rpt = 160;
   for (int mb = 1; mb <= 5; mb++) {
     const int tiles = cdiv(B, 32 * mb);
-    double us = streaming_us(mb, (long long)tiles * n_col_tiles * 8, K / 64);
-    if (epi != EPI_ARGMAX && mb <= 2 && dense_few(32 * mb, tiles, N, K)) {
-      const long long blocks = (long long)tiles * (N / 32);
-      us = few_us(mb, blocks, K / 64);
-      // (one wave staging 64 rows starts late, which shows where K is short: 512 x 512, 2047 rows 13.0 us, 10.1 with 32)
-      if (mb == 2 && blocks <= FEW_SOLO_BLOCKS) us += 2.0;
-    }
+    const double us = epi != EPI_ARGMAX && dense_few(32 * mb, tiles, N, K)
+                          ? few_us(mb, (long long)tiles * (N / 32), K / 64)
+                          : streaming_us(mb, (long long)tiles * n_col_tiles * 8, K / 64);
     if (mb == 1 || us <= best) {
       best = us;
       rpt = 32 * mb;
@@ -228,8 +230,8 @@ int dense_gemm_mixed(const bf16_t *A, const bf16_t *W, float *out, const GemmBf1
 }
 
 // Few rows and few columns leave most CUs without a work item while those that have one walk all of K.
-// Cutting K makes more items; what it costs is a fixed part per item and the partial sums' way to memory
-// and back.
+// Cutting K makes more items; what it costs is a part per round and the reading of the partial sums.  All row tiles and parts timed at the 312 sizes above: the chosen ones take 2 % longer than the best ones on average
+// and are 15 % faster than with streaming kernels alone (2048 x 2048, 8 / 400 / 1024 rows 7.0 / 14.6 / 21.8 -> 4.7 / 11.5 / 17.5 us).
 int dense_gemm_partial(const bf16_t *A, const bf16_t *W, float *out, size_t max_elems, int *parts, int B, int N, int K,
                        hipStream_t s) {
   *parts = 1;
@@ -244,9 +246,11 @@ int dense_gemm_partial(const bf16_t *A, const bf16_t *W, float *out, size_t max_
       const int per = cdiv(nslab, want), n = cdiv(nslab, per);
       // (an item prefetches two slabs of the next one, so no part may have fewer)
       if (n != want || (n > 1 && (per < 4 || nslab - per * (n - 1) < 2 || (size_t)n * B * N > max_elems))) continue;
-      const long long tiles = cdiv(B, 32 * mb);
-      const double cost = (mb <= 2 ? few_us(mb, tiles * (N / 32) * n, per) : streaming_us(mb, tiles * g.n_col_tiles * 8 * n, per)) +
-                          (n - 1) * (double)B * N * 8 / 5e6;
+      const int tiles = cdiv(B, 32 * mb);
+      const bool few = n == 1 ? dense_few(32 * mb, tiles, N, K) : mb <= 2;   // as run_gemm_dense has it
+      const double cost = (few ? few_us(mb, (long long)tiles * (N / 32) * n, per)
+                               : streaming_us(mb, (long long)tiles * g.n_col_tiles * 8 * n, per)) +
+                          (n - 1) * (double)B * N * 4 / 5e6;
       if ((mb == 1 && n == 1) || cost < best) {
         best = cost;
         rpt = 32 * mb;

@@ -1,5 +1,7 @@
 """The few-row GEMM kernels (tiles of at most 64 rows): every row must have the bits that the streaming kernels give it
 in a larger batch, at the edges of row tiles, column blocks and staged chunks of K."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -85,3 +87,26 @@ def test_grouping_of_a_few_tokens_equals_the_sorting_kernel(ops, E, k, ties):
         w2, i2, off2, srt2, inv2, _ = ops.moe_route(logits, k)
         for got, want in ((w, w2), (i, i2), (off, off2), (srt, srt2), (inv, inv2)):
             assert torch.equal(got, want), tokens
+
+
+# rows on both sides of where the kernel, the row tile or the number of parts changes; K: two slabs, which cannot be cut, to 128
+@pytest.mark.parametrize("N,K", [(512, 128), (768, 768), (1280, 1280), (896, 4864), (2048, 8192)])
+def test_products_with_their_k_cut_add_up(ops, N, K):
+    """gptoss::dense_gemm_partial, which has no C entry point, by its linker name: the parts add up to the product."""
+    lib = load_pkg("lib")
+    f = getattr(lib.load(), "_ZN6gptoss18dense_gemm_partialEPKtS1_PfmPiiiiP12ihipStream_t")
+    f.restype, f.argtypes = C.c_int, [C.c_void_p] * 3 + [C.c_size_t, C.c_void_p] + [C.c_int] * 3 + [C.c_void_p]
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    a, w = _n(g, 2047, K), _n(g, N, K, std=0.05)
+    packed, exact = ops.pack_weight(w), a.double() @ w.double().T
+    bound = K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)     # K sums in fp32, in any order
+    cut = set()
+    for rows in (1, 8, 9, 32, 33, 65, 97, 257, 320, 576, 768, 1024, 1280, 1700, 2047):
+        out, parts = torch.full((8 * rows * N,), float("nan"), device="cuda"), C.c_int()
+        lib.check(f(a.data_ptr(), packed.data_ptr(), out.data_ptr(), out.numel(), C.byref(parts), rows, N, K,
+                    torch.cuda.current_stream().cuda_stream))
+        assert 1 <= parts.value <= 8
+        total = out[:parts.value * rows * N].view(parts.value, rows, N).double().sum(0)
+        assert bool(((total - exact[:rows]).abs() <= bound[:rows]).all()), rows
+        cut.add(parts.value)
+    assert cut == {1} if K == 128 else len(cut) > 1
