@@ -13,11 +13,12 @@
 //     then its V in V^T operand order, common.hpp): a wave reads 16 KB contiguous per block with
 //     128-bit loads, the four waves of a workgroup 64 KB; position p lives in slot p % capacity
 //     (ring buffer for window layers);
-//   * contexts of up to ATT_CHUNK slots are one wave's single pass;
-//   * longer contexts, few sequences: cut into chunks (flash-decoding), one wave each: partial
-//     (max, sum, O) per chunk go to the workspace and a small second kernel merges them with the
-//     sink.  The chunk length is a constant, so a row's result is the same whatever else is in
-//     the launch;
+//   * contexts of up to ATT_CHUNK slots are one wave's single pass, or, where a launch has few of them,
+//     a workgroup's with the same bits (attn_few_kernel);
+//   * longer contexts, few sequences: cut into chunks (flash-decoding), one wave each, or again a
+//     workgroup: partial (max, sum, O) per chunk go to the workspace and a small second kernel merges
+//     them with the sink.  The chunk length is a constant, so a row's result is the same whatever else
+//     is in the launch;
 //   * longer contexts, many sequences (enough to fill the chip with one workgroup per sequence
 //     and kv head): the four waves of a workgroup share one (sequence, kv head), wave w taking the
 //     64-slot blocks w, w+4, ..., and merge their states with the sink in LDS.  Nothing but the
