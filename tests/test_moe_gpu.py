@@ -382,3 +382,21 @@ def test_tokens_that_are_no_numbers_leave_the_others_alone(ops, B, E):
     rest = [b for b in range(B) if b not in bad]
     assert bool(torch.isnan(got[bad]).all())
     assert torch.equal(got[rest], want[rest])
+
+
+@pytest.mark.parametrize("E", [1, 2, 31, 32, 33, 64, 65, 129, 256])   # one to eight experts per lane, lanes without one
+@pytest.mark.parametrize("k", [1, 2, 4, 7, 8])
+def test_routing_of_equal_and_infinite_logits(ops, E, k):
+    """Few different values, zeros of both signs and -infinity among them: the picks are the first k by value, then by expert;
+    the weights are within the rounding of an exponential, a sum of k and a division in fp32."""
+    if k > E:
+        pytest.skip("more picks than experts")
+    rng = np.random.default_rng(E * 8 + k)
+    logits = rng.choice(np.array([-np.inf, -3.5, -0.0, 0.0, 1.25, 1.25, 2.0], np.float32), size=(67, E))
+    logits[:, rng.integers(E)] = 2.0                    # a largest value that is a number
+    tw, ti = [x.cpu().numpy() for x in ops.moe_route(torch.from_numpy(logits).cuda(), k)[:2]]
+    want = np.argsort(-(logits + np.float32(0)), axis=1, kind="stable")[:, :k]
+    np.testing.assert_array_equal(ti, want)
+    picked = np.take_along_axis(logits, want, axis=1).astype(np.float64)
+    e = np.exp(picked - picked[:, :1])
+    np.testing.assert_allclose(tw, e / e.sum(1, keepdims=True), rtol=2e-6, atol=0)
