@@ -5,7 +5,7 @@
 // the tile), which caps it at ~70 % of the MFMA rate before anything else is counted.  Here a
 // workgroup of four waves (one per SIMD) owns a 256 x 256 tile and a wave a 128 x 128 quarter of
 // it: 4 W fragments and 4 A fragments per k-step feed 16 MFMAs, half a fragment per MFMA.  Both
-// operands go from global memory straight into LDS with global_load_lds_dwordx4 (no staging
+// operands go from global memory straight into LDS with buffer_load_dwordx4 .. lds (no staging
 // registers, no LDS store instructions), and the load pipeline runs on from one work item into
 // the next.
 //   W: stages of 32 k in four buffers, three in flight, in the same packed fragment order as
@@ -58,18 +58,33 @@ template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
-template <typename T>
-__device__ __forceinline__ const T *uniform_ptr(const T *q) {
-  const uint64_t v = reinterpret_cast<uint64_t>(q);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return reinterpret_cast<const T *>(((uint64_t)hi << 32) | lo);
+typedef uint32_t tall_rsrc_t __attribute__((ext_vector_type(4)));   // a buffer resource in scalar registers
+__device__ __forceinline__ tall_rsrc_t tall_buffer(const void *base) {
+  const uint64_t v = reinterpret_cast<uint64_t>(base);
+  return tall_rsrc_t{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v),
+                     (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32) & 0xffffu), 0xffffffffu, 0x00020000u};
+}
+
+// 16 bytes per lane, from the buffer's base + voff + soff to LDS address lds + ADD + 16 * lane: load_to_lds (common.hpp) in
+// three instructions.  With one wave per SIMD an instruction takes four cycles of which only those in the shadow of a
+// matrix instruction are free, seven instructions or so: an address of 64 bits per load, added up in scalar registers,
+// made the ten instructions of a load outlast it.  A tile of K = 2880 takes 110 thousand cycles instead of 120 (its matrix
+// instructions alone 92), and the chip, at its power limit, runs them at 1.65 GHz instead of 1.75: block of 5999 tokens
+// 1344 -> 1311 us, of 4500 1152 -> 1120.
+template <int ADD>
+__device__ __forceinline__ void tall_load(unsigned lds, uint32_t voff, tall_rsrc_t base, uint32_t soff) {
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(base),
+               "s"(soff), "n"(ADD)
+               : "memory", "scc");
 }
 
 // where one work item's operands come from, for this wave's share of the loads
 template <class SH>
 struct TallSrc {
-  const unsigned char *w[SH::LW];  // stage 0 of the W fragments this wave loads
-  uint32_t a[SH::LA];              // byte offsets of this lane's piece of the A rows it loads
+  static constexpr int WB = SH::LW / 2;   // column blocks: both k-steps of a stage of each
+  tall_rsrc_t w;       // the tile's first column block
+  uint32_t wo[WB];     // byte offsets of the wave's column blocks from there
+  uint32_t a[SH::LA];  // byte offsets of this lane's piece of the A rows it loads
   int mat, row0, rows, ct;
 };
 
@@ -186,7 +201,6 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
   const int S = K / TALL_BK;                    // even: K % 64 == 0
   const unsigned lds_base =
       __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)lds);
-  const unsigned char *abase = reinterpret_cast<const unsigned char *>(p.A);
 
   // ---- work list: the order of grouped_gemm_kernel (gemm_kernel.hpp), with tiles of BM rows --------
   const const_as<int> tiles = constant_ptr(p.tiles), bounds = constant_ptr(p.xcd_bounds);
@@ -243,13 +257,11 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
     t.row0 = __builtin_amdgcn_readfirstlane(t.row0);
     t.rows = __builtin_amdgcn_readfirstlane(t.rows);
     // W fragment f of a stage = (column block f / 2 of the tile, k-step f % 2); a block beyond N repeats the last one
-    const unsigned char *wm = reinterpret_cast<const unsigned char *>(p.W) + (size_t)t.mat * N * K * 2;
+    const int first = t.ct * (SH::WC * CB);
+    t.w = tall_buffer(reinterpret_cast<const unsigned char *>(p.W) + ((size_t)t.mat * N + (size_t)first * 32) * K * 2);
 #pragma unroll
-    for (int q = 0; q < LW; q++) {
-      const int f = w * LW + q;
-      const int cb = min(t.ct * (SH::WC * CB) + (f >> 1), N / 32 - 1);
-      t.w[q] = uniform_ptr(wm + ((size_t)cb * (K / 16) + (f & 1)) * 1024);
-    }
+    for (int q = 0; q < TallSrc<SH>::WB; q++)
+      t.wo[q] = (uint32_t)min(w * TallSrc<SH>::WB + q, N / 32 - 1 - first) * (uint32_t)K * 64u;
   };
   // A: load instruction q of this wave moves 8 tile rows, eight lanes per row and one 16-byte piece
   // per lane: the lane at position p of row r fetches piece p ^ ((r >> 1) & 7).  Rows past the
@@ -278,15 +290,11 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
     }
   };
 
-  // W load instruction q of this wave for stage s of an item, into W buffer buf
   const uint32_t voff_w = lane * 16;
-  auto issue_w = [&](const TallSrc<SH> &t, int s, int buf, int q) {
-    load_to_lds(lds_base + buf * SH::W_BYTES + (w * LW + q) * 1024, voff_w, t.w[q] + (size_t)s * 2048);
-  };
-  // A load instruction q of this wave for chunk c of an item, into A buffer buf
-  auto issue_a = [&](const TallSrc<SH> &t, int c, int buf, int q) {
-    load_to_lds(lds_base + SH::A_OFF + buf * SH::A_BYTES + (w * LA + q) * 1024, t.a[q], abase + (size_t)c * 128);
-  };
+  const tall_rsrc_t abuf = tall_buffer(p.A);
+  // the wave's parts of W buffer `buf` and of A buffer `buf`
+  auto w_dst = [&](int buf) { return lds_base + buf * SH::W_BYTES + w * LW * 1024; };
+  auto a_dst = [&](int buf) { return lds_base + SH::A_OFF + buf * SH::A_BYTES + w * LA * 1024; };
 
   f32x16 acc[CB][RB];   // [column block][row block]
   const int sw = ((lane & 31) >> 1) & 7, h = lane >> 5;
@@ -325,17 +333,23 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
   // The first loads go out in the order the stage loop would have issued them, so that its waits
   // count right from the first stage on: chunk 0 and W stage 0, then a quarter of chunk 1 with
   // every half of W stages 1 and 2.
-#pragma unroll
-  for (int q = 0; q < LA; q++) issue_a(cur, 0, 0, q);
-#pragma unroll
-  for (int q = 0; q < LW; q++) issue_w(cur, 0, 0, q);
-#pragma unroll
-  for (int x = 0; x < 4; x++) {
-#pragma unroll
-    for (int q = 0; q < LA1; q++) issue_a(cur, 1, 1, x * LA1 + q);
-#pragma unroll
-    for (int q = 0; q < LW1; q++) issue_w(cur, 1 + (x >> 1), 1 + (x >> 1), (x & 1) * LW1 + q);
-  }
+  static_assert(LW1 == 2 && TallSrc<SH>::WB == 2, "half a W stage is one column block of the wave");
+  static_for<0, LA>([&](auto q) { tall_load<decltype(q)::value * 1024>(a_dst(0), cur.a[decltype(q)::value], abuf, 0); });
+  static_for<0, LW>([&](auto q) {
+    constexpr int Q = decltype(q)::value;
+    tall_load<Q * 1024>(w_dst(0), voff_w + (Q & 1) * 1024, cur.w, cur.wo[Q >> 1]);
+  });
+  static_for<0, 4>([&](auto xx) {
+    constexpr int X = decltype(xx)::value;
+    static_for<0, LA1>([&](auto q) {
+      constexpr int Q = X * LA1 + decltype(q)::value;
+      tall_load<Q * 1024>(a_dst(1), cur.a[Q], abuf, 128);
+    });
+    static_for<0, LW1>([&](auto q) {
+      constexpr int Q = (X & 1) * LW1 + decltype(q)::value;
+      tall_load<Q * 1024>(w_dst(1 + (X >> 1)), voff_w + (Q & 1) * 1024, cur.w, cur.wo[Q >> 1] + (1 + (X >> 1)) * 2048);
+    });
+  });
   wait_vmcnt<4 * (LA1 + LW1)>();   // chunk 0 and stage 0 have landed; the loads behind them may be on their way
   __builtin_amdgcn_s_barrier();
 #pragma unroll
@@ -343,6 +357,10 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
   __builtin_amdgcn_sched_barrier(0);
   int g = 0;   // running stage count (even at the start of every item): W buffer g & 3
   int ab = 0;  // A buffer of the current chunk: the running chunk count modulo 3
+  // what the loop requests next: a W stage, of the current item or the next one, and an A chunk
+  tall_rsrc_t ws = cur.w;
+  uint32_t wo[2] = {cur.wo[0] + 3 * 2048, cur.wo[1] + 3 * 2048}, ao = 2 * 128;
+  const uint32_t voff_w1 = voff_w + 1024;
   while (true) {
     const int jn = j + per_xcd;
     const bool more = valid(jn);
@@ -360,46 +378,52 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
     for (int s = 0; s < S; s += 2, g += 2) {
       // ---- even stage s: the first half of A chunk s / 2 --------------------------------------
       const int ab1 = ab == 2 ? 0 : ab + 1, ab2 = ab1 == 2 ? 0 : ab1 + 1;
-      const bool wrap_a = s + 4 >= S;             // the chunk requested now: two ahead, or one of the next item's first two
-      const bool wrap_w0 = s + 3 >= S, wrap_w1 = s + 4 >= S;
-      TallSrc<SH> sa, s0, s1;
-#pragma unroll
-      for (int q = 0; q < LA; q++) sa.a[q] = wrap_a ? nxt.a[q] : cur.a[q];
-#pragma unroll
-      for (int q = 0; q < LW; q++) {
-        s0.w[q] = wrap_w0 ? nxt.w[q] : cur.w[q];
-        s1.w[q] = wrap_w1 ? nxt.w[q] : cur.w[q];
-      }
-      const int ca = (wrap_a ? s + 4 - S : s + 4) >> 1;
-      const int sw0 = wrap_w0 ? s + 3 - S : s + 3, sw1 = wrap_w1 ? s + 4 - S : s + 4;
-      __builtin_amdgcn_sched_barrier(0);
+      // from here on the A chunks that are requested (two ahead) are the next item's, and so is every W stage from the
+      // middle of this round on
+      const bool wrap = s + 4 >= S;
+      if (s + 4 == S) ao = 0;
+      const unsigned ad = a_dst(ab2);
       // Every k-step issues a quarter of A chunk s / 2 + 2, into the buffer that chunk s / 2 - 1 left
       // (every wave is past the barrier of the stage that read it last), and half of a W stage,
       // behind the fragment reads: loads(x, ...) places them after MFMAs NR, NR + 2, ...
-      auto loads = [&](int m, int x, const TallSrc<SH> &sw_, int st, int wbuf, int half) {
-#pragma unroll
-        for (int q = 0; q < LA1; q++)
-          if (m == NR + 2 * q) issue_a(sa, ca, ab2, x * LA1 + q);
-#pragma unroll
-        for (int q = 0; q < LW1; q++)
-          if (m == NR + 2 * (LA1 + q)) issue_w(sw_, st, wbuf, half * LW1 + q);
+      auto loads = [&](int m, auto xx, int wbuf, auto hh) {
+        constexpr int X = decltype(xx)::value, H = decltype(hh)::value;
+        static_for<0, LA1>([&](auto q) {
+          constexpr int Q = X * LA1 + decltype(q)::value;
+          if (m == NR + 2 * decltype(q)::value) tall_load<Q * 1024>(ad, wrap ? nxt.a[Q] : cur.a[Q], abuf, ao);
+        });
+        if (m == NR + 2 * LA1) tall_load<2 * H * 1024>(w_dst(wbuf), voff_w, ws, wo[H]);
+        if (m == NR + 2 * LA1 + 2) {
+          tall_load<(2 * H + 1) * 1024>(w_dst(wbuf), voff_w1, ws, wo[H]);
+          wo[H] += 2048;
+        }
       };
-      kstep(0, g & 3, 1, ab, 1, [&](int m) { loads(m, 0, s0, sw0, (g + 3) & 3, 0); });
+      using I0 = std::integral_constant<int, 0>;
+      using I1 = std::integral_constant<int, 1>;
+      using I2 = std::integral_constant<int, 2>;
+      using I3 = std::integral_constant<int, 3>;
+      kstep(0, g & 3, 1, ab, 1, [&](int m) { loads(m, I0{}, (g + 3) & 3, I0{}); });
       // behind W stage s+1 were issued the loads of two k-steps of stage s-1 and of one of stage s
       wait_vmcnt<3 * (LA1 + LW1)>();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      kstep(1, (g + 1) & 3, 0, ab, 2, [&](int m) { loads(m, 1, s0, sw0, (g + 3) & 3, 1); });
+      kstep(1, (g + 1) & 3, 0, ab, 2, [&](int m) { loads(m, I1{}, (g + 3) & 3, I1{}); });
+      if (s + 4 == S) {   // W stage s + 3 was this item's last
+        ws = nxt.w;
+        wo[0] = nxt.wo[0];
+        wo[1] = nxt.wo[1];
+      }
       // ---- odd stage s+1: the second half of the chunk -----------------------------------------
-      kstep(0, (g + 1) & 3, 1, ab, 3, [&](int m) { loads(m, 2, s1, sw1, (g + 4) & 3, 0); });
+      kstep(0, (g + 1) & 3, 1, ab, 3, [&](int m) { loads(m, I2{}, (g + 4) & 3, I0{}); });
       // W stage s+2, and with it the A chunk that the next stage starts (its last loads went out in
       // front of that stage's), must have landed
       wait_vmcnt<3 * (LA1 + LW1)>();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      kstep(1, (g + 2) & 3, 0, ab1, 0, [&](int m) { loads(m, 3, s1, sw1, (g + 4) & 3, 1); });
+      kstep(1, (g + 2) & 3, 0, ab1, 0, [&](int m) { loads(m, I3{}, (g + 4) & 3, I1{}); });
+      ao += 128;
       ab = ab1;
     }
     // epilogue: the wave's column blocks, each with its row blocks.  The empty asm pins a column
