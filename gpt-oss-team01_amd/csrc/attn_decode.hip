@@ -57,10 +57,12 @@ __device__ __forceinline__ float sink_reference(float m, float sink2) { return f
 // product, so its own distance is that rounding error and its weight within 2^(|m| 2^-24) of 1, a factor that all weights
 // of the row share.  From 2^24 on the error is a power of two and more (beyond 2^31 the maximum's weight would overflow or
 // vanish): such rows take the difference of rounded products, the maximum's distance is 0.
-__device__ __forceinline__ void weight_exponents(f32x4 (&s4)[4], float scale, float m) {
+// any_huge: whether the wave has one.
+__device__ __forceinline__ bool huge_maximum(float m) { return fabsf(m) >= 16777216.f && m != NEG_BIG; }
+__device__ __forceinline__ void weight_exponents(f32x4 (&s4)[4], float scale, float m, bool any_huge) {
 #pragma clang fp contract(off)
-  const bool huge = fabsf(m) >= 16777216.f && m != NEG_BIG;
-  if (__builtin_expect(__ballot(huge) != 0, 0)) {
+  if (__builtin_expect(any_huge, 0)) {
+    const bool huge = huge_maximum(m);
 #pragma unroll
     for (int tb = 0; tb < 4; tb++)
 #pragma unroll
@@ -387,7 +389,7 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
     const float m_new = fmaxf(m_run, max_over_quarters(bmax) * p.scale_log2e);
     const float alpha = exp2_hw(m_run - m_new);
     m_run = m_new;
-    weight_exponents(s4, p.scale_log2e, m_new);
+    weight_exponents(s4, p.scale_log2e, m_new, __ballot(huge_maximum(m_new)) != 0);
     float psum = 0.f;
     bf16x8 ph[2], pl[2];
 #pragma unroll
@@ -708,7 +710,7 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
   for (int u = 0; u < 2; u++) {
     const int j = wave + 4 * u;
     if (j < nb) {
-      weight_exponents(s4[u], p.scale_log2e, m_own[u]);
+      weight_exponents(s4[u], p.scale_log2e, m_own[u], __ballot(huge_maximum(m_own[u])) != 0);
       float psum = 0.f;
 #pragma unroll
       for (int grp = 0; grp < 2; grp++) {
@@ -853,7 +855,10 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 // positions, 64 heads: 237 -> 211 us with the exponential, the maximum and the splitting of weights in fewer instructions
 // (exp2_hw, max_over_quarters, split_weights), -> 195 with the scale fused into the exponent's difference
 // (weight_exponents), one range check per masked slot and blocks straight into LDS, -> 181 with whole loads of q
-// (split_query).
+// (split_query), and, on another box, 160 -> 151 with one instance of a block's step, whose masks and rescaling are branches
+// (one prompt of 2048: 74 -> 72, window of 128: 76 -> 70, three of 33 positions behind 450: 14.6 -> 13.7).  Two blocks to a
+// barrier are as fast; 80 registers for six waves per SIMD spill (180); the remainders of the split weights by dot
+// products, half the instructions: as fast.
 // Every row sees the arithmetic of the one-wave kernel over its own blocks in ascending order (a
 // block outside a row's range is a no-op for its columns), so rows of up to ATT_CHUNK positions
 // equal the decode call bit for bit; longer rows are summed in one pass instead of chunk by
@@ -935,14 +940,17 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
 #pragma unroll
   for (int db = 0; db < DB; db++) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_run = NEG_BIG, l_run = 0.f;
+  bool any_huge = false;
   const int lane_lo = second ? lo1 : lo0;
   const uint32_t lane_n = (second ? hi1 : hi0) - lane_lo;
-  const int any_lo = lo0;
-  const uint32_t any_n = (two ? hi1 : hi0) - any_lo;
+  // what either row sees, and what both see (nothing, where there is no second row)
+  const int any_lo = lo0, any_hi = two ? hi1 : hi0, whole_lo = lo1, whole_hi = two ? hi0 : 0;
+  const uint32_t any_n = any_hi - any_lo;
 
-  // one 64-slot block from LDS buffer `buf`: the arithmetic of the one-wave kernel's block step
-  auto process = [&](int blk, int buf, auto edge_sel) {
-    constexpr bool EDGE = decltype(edge_sel)::value;
+  // One 64-slot block from LDS buffer `buf`: the arithmetic of the one-wave kernel's block step.  `edge` (wave-uniform) only
+  // masks, between the products: as two instances of all of it the accumulators came out in different registers, and every
+  // block copied them.
+  auto process = [&](int blk, int buf, bool edge) {
     const unsigned char *kb = lds[buf];
     const unsigned char *vb = lds[buf] + K_BYTES;
     f32x4 s4[4];
@@ -958,23 +966,34 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
       }
       s4[tb] = acc;
     }
-    // the lane's first slot of the block, within its row's range and within either row's; derived per block from an opaque
-    // thread index, as the compiler would keep what it can compute ahead in registers that the loop does not have
-    int tid_here = tid;
-    if (EDGE) asm volatile("" : "+v"(tid_here));
-    const int slot0 = blk + ((tid_here & 63) >> 4) * 4, s0 = slot0 - lane_lo, a0 = slot0 - any_lo;
+    const int slot0 = blk + c * 4;   // the lane's first slot of the block
+    if (edge) {
+      const int s0 = slot0 - lane_lo;
+#pragma unroll
+      for (int tb = 0; tb < 4; tb++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) s4[tb][i] = (uint32_t)(s0 + tb * 16 + i) < lane_n ? s4[tb][i] : -INFINITY;
+    }
     float bmax = -INFINITY;   // of the scores as they leave the product
 #pragma unroll
     for (int tb = 0; tb < 4; tb++)
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        if (EDGE) s4[tb][i] = (uint32_t)(s0 + tb * 16 + i) < lane_n ? s4[tb][i] : -INFINITY;
-        bmax = fmaxf(bmax, s4[tb][i]);
-      }
-    const float m_new = fmaxf(m_run, max_over_quarters(bmax) * p.scale_log2e);
-    const float alpha = exp2_hw(m_run - m_new);
-    m_run = m_new;
-    weight_exponents(s4, p.scale_log2e, m_new);
+      for (int i = 0; i < 4; i++) bmax = fmaxf(bmax, s4[tb][i]);
+    // Only a block with a larger score for one of the wave's columns exchanges maxima between lanes and rescales: a factor
+    // of 1 otherwise.
+    const float top = bmax * p.scale_log2e;
+    float alpha = 1.f;
+    if (__ballot(top > m_run) != 0) {
+      const float m_new = fmaxf(m_run, max_over_quarters(top));
+      alpha = exp2_hw(m_run - m_new);
+      m_run = m_new;
+#pragma unroll
+      for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[db][i] *= alpha;
+      any_huge = __ballot(huge_maximum(m_run)) != 0;
+    }
+    weight_exponents(s4, p.scale_log2e, m_run, any_huge);
     float psum = 0.f;
     bf16x8 ph[2], pl[2];
 #pragma unroll
@@ -992,28 +1011,26 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
     }
     l_run = l_run * alpha + psum;
 #pragma unroll
-    for (int db = 0; db < DB; db++) {
+    for (int grp = 0; grp < 2; grp++) {
+      u32x4 vv[DB];
 #pragma unroll
-      for (int i = 0; i < 4; i++) o[db][i] *= alpha;
-    }
+      for (int db = 0; db < DB; db++) vv[db] = *reinterpret_cast<const u32x4 *>(vb + (grp * DB + db) * 1024 + lane * 16);
+      if (edge) {
 #pragma unroll
-    for (int grp = 0; grp < 2; grp++)
+        for (int w = 0; w < 4; w++) {
+          // the two rows are neighbours: what either of them sees is one range
+          const uint32_t sl = slot0 - any_lo + grp * 32 + (w >> 1) * 16 + (w & 1) * 2;
+          const uint32_t keep = (sl < any_n ? 0x0000ffffu : 0u) | (sl + 1 < any_n ? 0xffff0000u : 0u);
+#pragma unroll
+          for (int db = 0; db < DB; db++) vv[db][w] &= keep;
+        }
+      }
 #pragma unroll
       for (int db = 0; db < DB; db++) {
-        u32x4 vv = *reinterpret_cast<const u32x4 *>(vb + (grp * DB + db) * 1024 + lane * 16);
-        if (EDGE) {
-#pragma unroll
-          for (int w = 0; w < 4; w++) {
-            // the two rows are neighbours: what either of them sees is one range
-            const uint32_t sl = a0 + grp * 32 + (w >> 1) * 16 + (w & 1) * 2;
-            const uint32_t keep = (sl < any_n ? 0x0000ffffu : 0u) | (sl + 1 < any_n ? 0xffff0000u : 0u);
-            vv[w] &= keep;
-          }
-        }
-        bf16x8 vf = as_bf16x8(vv);
-        o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph[grp], o[db], 0, 0, 0);
-        o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[grp], o[db], 0, 0, 0);
+        o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vv[db]), ph[grp], o[db], 0, 0, 0);
+        o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vv[db]), pl[grp], o[db], 0, 0, 0);
       }
+    }
   };
 
   int buf = 0;
@@ -1025,11 +1042,12 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
     __builtin_amdgcn_sched_barrier(0);
     if (blk + ATT_BLOCK < blk_end) request_block(blk + ATT_BLOCK, buf ^ 1);
     // the wave's rows: first block that holds an active position of either row .. their last one
-    const bool mine = (have0 && blk < hi0 && blk + ATT_BLOCK > lo0) || (two && blk < hi1 && blk + ATT_BLOCK > lo1);
-    if (mine) {
-      const bool edge = !(two && blk >= lo0 && blk + ATT_BLOCK <= hi0 && blk >= lo1 && blk + ATT_BLOCK <= hi1);
-      if (edge) process(blk, buf, std::true_type{});
-      else process(blk, buf, std::false_type{});
+    // (rows are neighbours and ranges of a row that is not there are empty: [lo0, any_hi) is what either of them sees)
+    if (blk < any_hi && blk + ATT_BLOCK > lo0) {
+      // all 64 slots are active for both rows (known to be wave-uniform: otherwise the masks' results get registers of
+      // their own, and blocks without masks copy theirs there)
+      const int edge = __builtin_amdgcn_readfirstlane(blk < whole_lo || blk + ATT_BLOCK > whole_hi);
+      process(blk, buf, edge != 0);
     }
   }
 

@@ -432,3 +432,30 @@ def test_a_sink_far_above_every_score(ops, form, D):
     want = want if T else want[:, 0]
     # bf16: 2^-9; the exponent as a float near 145: 2^-17; its factor near 2^-145 has 2^-5 of itself as its last bit
     assert bool(((got - want).abs() <= want * (2.0 ** -8 + torch.exp2(shift - 149)[:, None])).all())
+
+
+@pytest.mark.parametrize("form", FORMS + [(1, 300, 300)])
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("step", [-12.0, 0.0, 3.0, 7.75, 8.25, 40.0])
+def test_scores_that_climb_from_block_to_block(ops, form, D, step):
+    """The largest score of a 64-slot block is `step` powers of two above the block before: references that stay, that are
+    raised in every block, and in every second or third one.  And a row alone has the bits it has in any other form."""
+    B, n, T = form
+    n_q, n_kv = 16, 8
+    g = torch.Generator(device="cuda").manual_seed(int(step * 4) + D)
+    direction = torch.randn(D, generator=g, device="cuda").sign()
+    q = direction.expand(*((B, T) if T else (B,)), n_q, D) / math.log2(math.e) / math.sqrt(D)
+    level = (torch.arange(n, device="cuda") // 64 * step)[None, :, None, None] - 2 * torch.rand(B, n, n_kv, 1, generator=g, device="cuda")
+    k = (level * direction).bfloat16()                      # scores: about `level` powers of two
+    v = torch.randn(B, n, n_kv, D, generator=g, device="cuda").bfloat16()
+    sinks = torch.randn(n_q, generator=g, device="cuda")
+    got = _attend(ops, form, q.contiguous(), k, v, sinks)
+    rows = got[:, -1] if T else got                         # the last position sees everything
+    s = (q[:, -1] if T else q).double().view(B, n_kv, 2, D) @ k.double().permute(0, 2, 3, 1) / math.sqrt(D)
+    w = torch.softmax(torch.cat([s, sinks.double().view(1, n_kv, 2, 1).expand(B, -1, -1, 1)], -1), -1)[..., :-1]
+    want = (w @ v.double().transpose(1, 2)).view(B, n_q, D)
+    size = (w @ v.double().abs().transpose(1, 2)).view(B, n_q, D)
+    # bf16: 2^-9 of the result; scores of up to 2^8 in fp32, and their sums: 2^-15; weights and queries of 16 bits: 2^-15
+    assert bool(((rows.double() - want).abs() <= want.abs() * 2.0 ** -8 + size * 2.0 ** -13).all())
+    if n <= 512:
+        assert torch.equal(rows[:1], _attend(ops, (1, n, 0), (q[:1, -1] if T else q[:1]).contiguous(), k[:1], v[:1], sinks))
