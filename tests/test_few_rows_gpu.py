@@ -110,3 +110,28 @@ def test_products_with_their_k_cut_add_up(ops, N, K):
         assert bool(((total - exact[:rows]).abs() <= bound[:rows]).all()), rows
         cut.add(parts.value)
     assert cut == {1} if K == 128 else len(cut) > 1
+
+
+class _Range(C.Structure):   # gptoss::GemmBf16Range
+    _fields_ = [("first", C.c_int), ("end", C.c_int), ("out", C.c_void_p), ("ld", C.c_int), ("relu_squared", C.c_int)]
+
+
+# rows at the edges of the 8-, 16- and 32-row kernels; N: half blocks (3 and 320 of them), whole blocks, a workgroup of four
+@pytest.mark.parametrize("N,K", [(96, 64), (96, 1088), (5120, 576), (17408, 64)])
+def test_columns_that_leave_as_bf16_are_the_rounded_fp32_ones(ops, N, K):
+    """gptoss::dense_gemm_mixed by its linker name: a plain and a relu-squared range beside the fp32 columns."""
+    lib = load_pkg("lib")
+    f = getattr(lib.load(), "_ZN6gptoss16dense_gemm_mixedEPKtS1_PfPKNS_13GemmBf16RangeEiiiiP12ihipStream_t")
+    f.restype, f.argtypes = C.c_int, [C.c_void_p] * 4 + [C.c_int] * 4 + [C.c_void_p]
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    a, w = _n(g, 33, K), ops.pack_weight(_n(g, N, K, std=0.05))
+    for rows in (1, 8, 9, 16, 17, 32, 33):
+        want = ops.dense_gemm(a[:rows].contiguous(), w, N)
+        out = torch.zeros(rows, N, device="cuda")
+        plain, squared = (torch.zeros(rows, 40, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+        ranges = (_Range * 2)(_Range(0, 32, plain.data_ptr(), 40, 0), _Range(N - 32, N, squared.data_ptr(), 40, 1))
+        lib.check(f(a.data_ptr(), w.data_ptr(), out.data_ptr(), ranges, 2, rows, N, K, torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(out[:, 32:N - 32], want[:, 32:N - 32]), rows
+        assert torch.equal(plain[:, :32], want[:, :32].bfloat16()), rows
+        assert torch.equal(squared[:, :32], want[:, N - 32:].relu().square().bfloat16()), rows
+        assert not plain[:, 32:].any() and not squared[:, 32:].any(), rows
