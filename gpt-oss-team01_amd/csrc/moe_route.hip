@@ -298,6 +298,9 @@ struct RouterNorm {
 // rows (the arithmetic of rmsnorm_rows_kernel: 256 threads per row, the same element-to-thread
 // assignment and summation order, so t is the same to the bit), writes x and t to memory, keeps t in
 // LDS and multiplies from there: one launch and one read of t less than norm kernel + router kernel.
+// A small launch is a chain of waits for memory, so all that does not depend on each other is requested at once: the
+// router's weights and biases, a row's elements, its residual and the norm's weights.  (With a branch for each of the
+// row's parts they came one behind the other.)  One row of 2880, 4 experts 8.4 -> 7.3 us, 33 rows 10.6 -> 8.4.
 template <int NB, bool NORM>
 __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
     const bf16_t *__restrict__ t, const bf16_t *__restrict__ wr, const float *__restrict__ br,
@@ -331,27 +334,43 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
   // the router's weights do not wait for the norm (more than 128 experts: no registers to hold them meanwhile)
   constexpr bool EARLY = !NORM || NB <= 8;
   if constexpr (EARLY) load_b(min(wave, ksteps - 1));
+  // nor does the bias of the experts that the lane sums up in the end
+  const int row = threadIdx.x >> 5, sub = threadIdx.x & 31;
+  constexpr int NJ = (NB + 1) / 2;
+  float bias[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; j++) bias[j] = br ? br[min(sub + 32 * j, E - 1)] : 0.f;
   if constexpr (NORM) {
     constexpr int VPT = 4;  // rows of up to 4096 floats
     __shared__ double nred[2][4];
     bf16_t *t_rows = reinterpret_cast<bf16_t *>(t_rows_raw);
     const int grp = threadIdx.x >> 8, tg = threadIdx.x & 255;  // two groups of 256 threads, a row each
+    constexpr bool W_EARLY = NB < 8;   // requested with the first rows, where registers allow
+    f32x4 nw[VPT];
+#pragma unroll
+    for (int i = 0; i < VPT; i++)
+      if (W_EARLY) nw[i] = *reinterpret_cast<const f32x4 *>(nrm.weight + min((tg + 256 * i) * 4, H - 4));
     for (int rr = 0; rr < rows_per_wg; rr += 2) {
       const int lr = rr + grp;
       const bool live = lr < rows_per_wg && r0 + lr < B;
       const size_t row = (size_t)(r0 + lr) * H;
-      f32x4 v[VPT];
+      // no load under a condition, so that a row's are all on their way together (lanes past its end read its last elements)
+      const size_t src = (size_t)min(r0 + min(lr, rows_per_wg - 1), B - 1) * H;
+      f32x4 v[VPT], res[VPT];
+#pragma unroll
+      for (int i = 0; i < VPT; i++) {
+        const int h = min((tg + 256 * i) * 4, H - 4);
+        v[i] = *reinterpret_cast<const f32x4 *>(nrm.x + src + h);
+        res[i] = *reinterpret_cast<const f32x4 *>((nrm.residual ? nrm.residual : nrm.x) + src + h);
+      }
       double ss = 0.0;
 #pragma unroll
       for (int i = 0; i < VPT; i++) {
         const int h = (tg + 256 * i) * 4;
-        v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (live && h < H) {
-          v[i] = *reinterpret_cast<const f32x4 *>(nrm.x + row + h);
           if (nrm.residual) {
-            const f32x4 r = *reinterpret_cast<const f32x4 *>(nrm.residual + row + h);
 #pragma unroll
-            for (int q = 0; q < 4; q++) v[i][q] = __fadd_rn(v[i][q], r[q]);
+            for (int q = 0; q < 4; q++) v[i][q] = __fadd_rn(v[i][q], res[i][q]);
             *reinterpret_cast<f32x4 *>(nrm.x + row + h) = v[i];
           }
 #pragma unroll
@@ -369,10 +388,10 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
       for (int i = 0; i < VPT; i++) {
         const int h = (tg + 256 * i) * 4;
         if (live && h < H) {
-          const f32x4 w = *reinterpret_cast<const f32x4 *>(nrm.weight + h);
+          if (!W_EARLY) nw[i] = *reinterpret_cast<const f32x4 *>(nrm.weight + h);
           f32x4 o;
 #pragma unroll
-          for (int q = 0; q < 4; q++) o[q] = (float)((double)w[q] * (inv * (double)v[i][q]));
+          for (int q = 0; q < 4; q++) o[q] = (float)((double)nw[i][q] * (inv * (double)v[i][q]));
           const u32x2 pk = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
           *reinterpret_cast<u32x2 *>(nrm.t_out + row + h) = pk;
           *reinterpret_cast<u32x2 *>(t_rows + (size_t)lr * H + h) = pk;
@@ -405,9 +424,7 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
     for (int i = 0; i < 4; i++) red[wave][(lane >> 4) * 4 + i][nb * 16 + (lane & 15)] = acc[nb][i];
   __syncthreads();
   // 32 lanes per token row: sum the partial products, add the bias, publish, gate
-  const int row = threadIdx.x >> 5, sub = threadIdx.x & 31;
   const bool live = row < rows_per_wg && r0 + row < B;
-  constexpr int NJ = (NB + 1) / 2;
   float v[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; j++) {
@@ -417,7 +434,7 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
       x = 0.f;
 #pragma unroll
       for (int w = 0; w < ROUTER_WAVES; w++) x += red[w][row][e];
-      if (br) x += br[e];
+      if (br) x += bias[j];
       if (live) logits[(size_t)(r0 + row) * E + e] = x;
     }
     v[j] = x;
