@@ -89,11 +89,13 @@ __device__ __forceinline__ void split_weights(float p0, float p1, uint32_t &h, u
 // A lane's KS * 8 values of a query row as bf16 hi + lo operands; a column without a row or head is zero.  qp points to a
 // real row whether the column has one or not, so that the loads are whole and unconditional (sixteen conditional ones of
 // four bytes: 64 prompts of 125 positions 104 instead of 73 us, eight of 1000 195 instead of 181).
-template <int KS>
-__device__ __forceinline__ void split_query(const float *qp, bool live, bf16x8 (&qh)[KS], bf16x8 (&ql)[KS]) {
-  f32x4 x[2 * KS];
+template <int N>
+__device__ __forceinline__ void load_query(const float *qp, f32x4 (&x)[N]) {
 #pragma unroll
-  for (int i = 0; i < 2 * KS; i++) x[i] = *reinterpret_cast<const f32x4 *>(qp + i * 4);
+  for (int i = 0; i < N; i++) x[i] = *reinterpret_cast<const f32x4 *>(qp + i * 4);
+}
+template <int KS>
+__device__ __forceinline__ void split_query(const f32x4 (&x)[2 * KS], bool live, bf16x8 (&qh)[KS], bf16x8 (&ql)[KS]) {
 #pragma unroll
   for (int s = 0; s < KS; s++) {
     uint32_t h[4], l[4];
@@ -107,6 +109,12 @@ __device__ __forceinline__ void split_query(const float *qp, bool live, bf16x8 (
     qh[s] = as_bf16x8(u32x4{h[0], h[1], h[2], h[3]});
     ql[s] = as_bf16x8(u32x4{l[0], l[1], l[2], l[3]});
   }
+}
+template <int KS>
+__device__ __forceinline__ void split_query(const float *qp, bool live, bf16x8 (&qh)[KS], bf16x8 (&ql)[KS]) {
+  f32x4 x[2 * KS];
+  load_query(qp, x);
+  split_query<KS>(x, live, qh, ql);
 }
 
 struct AttnParams {
@@ -644,24 +652,33 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
   if (p.seq_map) seq = __builtin_amdgcn_readfirstlane(p.seq_map[seq]);
   const bf16_t *plane = p.kv + kv_block_off(seq, g, p.n_kv, p.cap, D, 0);
 
-  // All loads at once; blocks beyond the last repeat it.  (Plain loads: so few rows stay in the caches for the next step.)
-  auto block_at = [&](int j) { return plane + (size_t)((c0 >> 6) + min(j, max(nb - 1, 0))) * (2 * KV_BLOCK * D); };
+  // All loads at once, the query first, because they return in order.  (Plain loads: so few rows stay in the caches for
+  // the next step.)  Blocks that a row does not have are left out by one jump to behind the last: even loads that hit the
+  // cache are time on the CU's only path to it, and jumps over each are as many misses in the instruction cache.  One row
+  // of 60 6.0 -> 4.8 us, 8 of 100 6.5 -> 5.3, of 300 7.8 -> 7.0.
+  auto block_at = [&](int j) { return plane + (size_t)((c0 >> 6) + j) * (2 * KV_BLOCK * D); };
+  f32x4 qx[2 * KS];
+  load_query(p.q + ((size_t)b * p.n_q + head) * D + c * KS * 8, qx);
   u32x4 kreg[2][4][KS], vreg[NBLK][2];
 #pragma unroll
-  for (int u = 0; u < 2; u++)
+  for (int u = 0; u < 2; u++) {
+    if (wave + 4 * u >= nb) break;
 #pragma unroll
     for (int tb = 0; tb < 4; tb++)
 #pragma unroll
       for (int s = 0; s < KS; s++)
         kreg[u][tb][s] = *reinterpret_cast<const u32x4 *>(block_at(wave + 4 * u) + (tb * 16 + n) * D + c * KS * 8 + s * 8);
-  bf16x8 qh[KS], ql[KS];
-  split_query<KS>(p.q + ((size_t)b * p.n_q + head) * D + c * KS * 8, n < G, qh, ql);
+  }
   const int db = min(wave, DB - 1);   // head size 32: two waves are done after their weights
 #pragma unroll
-  for (int j = 0; j < NBLK; j++)
+  for (int j = 0; j < NBLK; j++) {
+    if (j >= nb) break;
 #pragma unroll
     for (int grp = 0; grp < 2; grp++)
       vreg[j][grp] = *reinterpret_cast<const u32x4 *>(block_at(j) + KV_BLOCK * D + (grp * DB + db) * 512 + lane * 8);
+  }
+  bf16x8 qh[KS], ql[KS];
+  split_query<KS>(qx, n < G, qh, ql);
 
   f32x4 s4[2][4];
 #pragma unroll
@@ -698,12 +715,10 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
   float alpha[NBLK], m_own[2] = {NEG_BIG, NEG_BIG}, m_run = NEG_BIG;
 #pragma unroll
   for (int j = 0; j < NBLK; j++) {
-    alpha[j] = 1.f;
-    if (j < nb) {
-      const float m_new = fmaxf(m_run, lds_max[j][n]);
-      alpha[j] = exp2_hw(m_run - m_new);
-      m_run = m_new;
-    }
+    if (j >= nb) break;
+    const float m_new = fmaxf(m_run, lds_max[j][n]);
+    alpha[j] = exp2_hw(m_run - m_new);
+    m_run = m_new;
     if (j % 4 == wave) m_own[j / 4] = m_run;
   }
 #pragma unroll
@@ -734,25 +749,24 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
   float l_run = 0.f;
 #pragma unroll
   for (int j = 0; j < NBLK; j++) {
-    if (j < nb) {
-      const int blk = c0 + j * ATT_BLOCK;
-      l_run = l_run * alpha[j] + lds_sum[j][lane];
+    if (j >= nb) break;
+    const int blk = c0 + j * ATT_BLOCK;
+    l_run = l_run * alpha[j] + lds_sum[j][lane];
 #pragma unroll
-      for (int i = 0; i < 4; i++) o[i] *= alpha[j];
-      if (is_edge(blk)) {   // never-written cache memory may hold NaN bit patterns
+    for (int i = 0; i < 4; i++) o[i] *= alpha[j];
+    if (is_edge(blk)) {   // never-written cache memory may hold NaN bit patterns
 #pragma unroll
-        for (int grp = 0; grp < 2; grp++)
+      for (int grp = 0; grp < 2; grp++)
 #pragma unroll
-          for (int w = 0; w < 4; w++) {
-            const int s_lo = blk + grp * 32 + (w >> 1) * 16 + c * 4 + (w & 1) * 2;
-            vreg[j][grp][w] &= (active(s_lo) ? 0x0000ffffu : 0u) | (active(s_lo + 1) ? 0xffff0000u : 0u);
-          }
-      }
+        for (int w = 0; w < 4; w++) {
+          const int s_lo = blk + grp * 32 + (w >> 1) * 16 + c * 4 + (w & 1) * 2;
+          vreg[j][grp][w] &= (active(s_lo) ? 0x0000ffffu : 0u) | (active(s_lo + 1) ? 0xffff0000u : 0u);
+        }
+    }
 #pragma unroll
-      for (int grp = 0; grp < 2; grp++) {
-        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vreg[j][grp]), as_bf16x8(lds_p[j][grp * 2][lane]), o, 0, 0, 0);
-        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vreg[j][grp]), as_bf16x8(lds_p[j][grp * 2 + 1][lane]), o, 0, 0, 0);
-      }
+    for (int grp = 0; grp < 2; grp++) {
+      o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vreg[j][grp]), as_bf16x8(lds_p[j][grp * 2][lane]), o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vreg[j][grp]), as_bf16x8(lds_p[j][grp * 2 + 1][lane]), o, 0, 0, 0);
     }
   }
   l_run += lane_xor<16>(l_run);
@@ -790,55 +804,64 @@ static bool attn_few(long long pairs, int span, int head_dim) {
 }
 
 // Merge the chunk partials of one (sequence, q head) with the sink logit.  One thread owns four
-// consecutive output elements; the chunk loop is unrolled in groups of ATT_RED_UNROLL whose loads
-// are all requested before the first use.
-constexpr int ATT_RED_UNROLL = 16;
-
-template <int D>
+// consecutive output elements.  It is a chain of waits for memory at any size, so the partials of the first
+// U chunks are requested together with the row's length, before it is known how many there are (what lies in
+// the others is left out).  Longer rows go on in groups of that many, maxima first.  Both kernels of 3 rows of 8000
+// 16.5 -> 15.2 us, of 8 of 3000 15.8 -> 14.8 (of which attn_few_kernel 0.3).
+template <int D, int U>  // U: chunks requested at once
 __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
   constexpr int TPP = D / 4;  // threads per (b, head)
   const int pair = blockIdx.x * (256 / TPP) + threadIdx.x / TPP;
   const int d4 = (threadIdx.x % TPP) * 4;
   if (pair >= p.B * p.n_q) return;
   const int b = pair / p.n_q, hq = pair - b * p.n_q;
-  const SeqRange r = seq_range(row_len(p, b), p.cap, p.window, p.max_len);
-  if (r.nchunks <= 1) return;  // already finished by the first kernel
-  const float sink2 = p.sinks ? p.sinks[hq] * 1.4426950408889634f : -INFINITY;
   const size_t slot0 = (size_t)b * p.max_chunks * p.n_q + hq;
-  const size_t slot_stride = p.n_q;
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  f32x2 ml[U];
+  f32x4 o[U];
+  auto load = [&](int c0) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const size_t slot = slot0 + (size_t)min(c0 + u, p.max_chunks - 1) * p.n_q;
+      ml[u] = *reinterpret_cast<const f32x2 *>(p.part_ml + slot * 2);
+      o[u] = *reinterpret_cast<const f32x4 *>(p.part_o + slot * D + d4);
+    }
+  };
+  const int len = row_len(p, b);
+  const float sink = p.sinks ? p.sinks[hq] : -INFINITY;
+  load(0);
+  const SeqRange r = seq_range(len, p.cap, p.window, p.max_len);
+  if (r.nchunks <= 1) return;  // already finished by the first kernel
+  const float sink2 = p.sinks ? sink * 1.4426950408889634f : -INFINITY;
   float M = NEG_BIG;
-  for (int c0 = 0; c0 < r.nchunks; c0 += ATT_RED_UNROLL) {
-    float m[ATT_RED_UNROLL];
 #pragma unroll
-    for (int u = 0; u < ATT_RED_UNROLL; u++)
-      m[u] = (c0 + u < r.nchunks) ? p.part_ml[(slot0 + (size_t)(c0 + u) * slot_stride) * 2] : -INFINITY;
+  for (int u = 0; u < U; u++) M = u < r.nchunks ? fmaxf(M, ml[u][0]) : M;
+  for (int c0 = U; c0 < r.nchunks; c0 += U) {
+    float m[U];
 #pragma unroll
-    for (int u = 0; u < ATT_RED_UNROLL; u++) M = fmaxf(M, m[u]);
+    for (int u = 0; u < U; u++) m[u] = p.part_ml[(slot0 + (size_t)min(c0 + u, r.nchunks - 1) * p.n_q) * 2];
+#pragma unroll
+    for (int u = 0; u < U; u++) M = fmaxf(M, m[u]);
   }
   M = sink_reference(M, sink2);
   float denom = exp2_hw(sink2 - M);
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int c0 = 0; c0 < r.nchunks; c0 += ATT_RED_UNROLL) {
-    float m[ATT_RED_UNROLL], l[ATT_RED_UNROLL];
-    f32x4 o[ATT_RED_UNROLL];
+  // chunks are merged in ascending order, so the result does not depend on the unroll width
+  auto merge = [&](int c0) {
 #pragma unroll
-    for (int u = 0; u < ATT_RED_UNROLL; u++) {
-      const bool ok = c0 + u < r.nchunks;
-      const size_t slot = slot0 + (size_t)(ok ? c0 + u : 0) * slot_stride;
-      m[u] = ok ? p.part_ml[slot * 2] : -INFINITY;
-      l[u] = ok ? p.part_ml[slot * 2 + 1] : 0.f;
-      o[u] = *reinterpret_cast<const f32x4 *>(p.part_o + slot * D + d4);
-    }
-    // chunks are merged in ascending order, so the result does not depend on the unroll width
-#pragma unroll
-    for (int u = 0; u < ATT_RED_UNROLL; u++) {
+    for (int u = 0; u < U; u++) {
       if (c0 + u < r.nchunks) {
-        const float w = exp2_hw(m[u] - M);
-        denom += l[u] * w;
+        const float w = exp2_hw(ml[u][0] - M);
+        denom += ml[u][1] * w;
 #pragma unroll
         for (int q = 0; q < 4; q++) acc[q] += o[u][q] * w;
       }
     }
+  };
+  merge(0);
+  for (int c0 = U; c0 < r.nchunks; c0 += U) {
+    load(c0);
+    merge(c0);
   }
   u32x2 pk = u32x2{pack_bf16x2(denom > 0.f ? acc[0] / denom : 0.f, denom > 0.f ? acc[1] / denom : 0.f),
                    pack_bf16x2(denom > 0.f ? acc[2] / denom : 0.f, denom > 0.f ? acc[3] / denom : 0.f)};
@@ -1292,8 +1315,10 @@ static int attn_launch(const float *q, const void *kv_cache, const int *lens,
     int per_block = 256 / (head_dim / 4);
     int rgrid = (B * n_q + per_block - 1) / per_block;
     TraceScope ts("attn_reduce", s);
-    if (head_dim == 64) attn_reduce_kernel<64><<<rgrid, 256, 0, s>>>(p);
-    else attn_reduce_kernel<32><<<rgrid, 256, 0, s>>>(p);
+    auto launch = [&](auto kernel) { kernel<<<rgrid, 256, 0, s>>>(p); };
+    if (pl.max_chunks <= 4) launch(head_dim == 64 ? attn_reduce_kernel<64, 4> : attn_reduce_kernel<32, 4>);
+    else if (pl.max_chunks <= 8) launch(head_dim == 64 ? attn_reduce_kernel<64, 8> : attn_reduce_kernel<32, 8>);
+    else launch(head_dim == 64 ? attn_reduce_kernel<64, 16> : attn_reduce_kernel<32, 16>);
     GPTOSS_LAUNCH_CHECK("attn_reduce_kernel");
   }
   return GPTOSS_OK;

@@ -459,3 +459,27 @@ def test_scores_that_climb_from_block_to_block(ops, form, D, step):
     assert bool(((rows.double() - want).abs() <= want.abs() * 2.0 ** -8 + size * 2.0 ** -13).all())
     if n <= 512:
         assert torch.equal(rows[:1], _attend(ops, (1, n, 0), (q[:1, -1] if T else q[:1]).contiguous(), k[:1], v[:1], sinks))
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("longest", [1000, 2000, 3500, 7000, 16500])   # room for up to 3, 4, 7, 14 and 33 chunks of 512 positions
+def test_rows_of_few_chunks_where_the_launch_has_room_for_many(ops, longest, D):
+    """The partials of chunks that a row does not have are never written: whatever lies there does not reach its result,
+    and neither does how many of them there are."""
+    lens = [n for c in (0, 1, 2, 3, 4, 7, 8, 9, 15, 16, 17, 32) for n in (512 * c, 512 * c + 1) if n <= longest] + [longest]
+    B, n_q, n_kv = len(lens), 16, 2
+    g = torch.Generator(device="cuda").manual_seed(longest + D)
+    q = torch.randn(B, n_q, D, generator=g, device="cuda")
+    k, v = (torch.randn(B, longest, n_kv, D, generator=g, device="cuda").bfloat16() for _ in range(2))
+    sinks = torch.randn(n_q, generator=g, device="cuda")
+    cache = ops.KVCache(B, n_kv, D, (longest + 63) // 64 * 64)
+    cache.write(k, v)
+    attn = ops.AttnDecode(B, n_q, n_kv, D, longest)
+    attn.ws.fill_(0xFF)   # NaN
+    got = attn.forward(q, cache, torch.tensor(lens, dtype=torch.int32, device="cuda"), sinks)
+    for b, n in enumerate(lens):
+        s = q[b].double().view(n_kv, n_q // n_kv, D) @ k[b, :n].double().permute(1, 2, 0) / math.sqrt(D)
+        w = torch.softmax(torch.cat([s, sinks.double().view(n_kv, -1, 1)], -1), -1)[..., :-1]
+        want, size = ((w @ x.double().transpose(0, 1)).view(n_q, D) for x in (v[b, :n], v[b, :n].abs()))
+        # bf16: 2^-9 of the result; weights and queries of 16 bits, scores and sums in fp32: 2^-14
+        assert bool(((got[b].double() - want).abs() <= want.abs() * 2.0 ** -8 + size * 2.0 ** -13).all()), n
