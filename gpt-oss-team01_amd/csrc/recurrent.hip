@@ -144,18 +144,28 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ShortConv c, const int 
 // ---- recurrence ----------------------------------------------------------------------------------
 constexpr int SCAN_TOKENS = 16;   // tokens staged at a time
 
-// The convolution's last taps - 1 inputs after the stretch; one thread owns a channel.
+// The convolution's last taps - 1 inputs after the stretch; one thread owns a channel.  All are read before the first is
+// written (they move within the same memory).
 __device__ __forceinline__ void advance_conv_state(const Scan &p, const RowSeg &seg, int part, int parts) {
   const ShortConv &c = p.conv_desc;
   const int keep = c.taps - 1;
   for (int ch = part * 256 + threadIdx.x; ch < c.channels; ch += parts * 256) {
     float *st = p.conv_state + (size_t)seg.slot * keep * c.channels + ch;
-    for (int i = 0; i < keep; i++) {
+    auto value = [&](int i) {
       const int t = seg.n - keep + i;   // row of the stretch whose input belongs here; negative: an older one
-      float v = 0.f;
-      if (t >= 0) v = p.in[(size_t)(seg.row0 + t) * p.ld_in + c.col + ch];
-      else if (seg.pos0 + t >= 0) v = st[(size_t)(i + seg.n) * c.channels];
-      st[(size_t)i * c.channels] = v;
+      if (t >= 0) return p.in[(size_t)(seg.row0 + t) * p.ld_in + c.col + ch];
+      return seg.pos0 + t >= 0 ? st[(size_t)(i + seg.n) * c.channels] : 0.f;
+    };
+    constexpr int ROOM = 8;
+    if (keep <= ROOM) {
+      float v[ROOM];
+#pragma unroll
+      for (int i = 0; i < ROOM; i++) v[i] = i < keep ? value(i) : 0.f;
+#pragma unroll
+      for (int i = 0; i < ROOM; i++)
+        if (i < keep) st[(size_t)i * c.channels] = v[i];
+    } else {
+      for (int i = 0; i < keep; i++) st[(size_t)i * c.channels] = value(i);   // (each is read before an earlier place is written)
     }
   }
 }
@@ -185,7 +195,7 @@ __global__ __launch_bounds__(256) void scan_kernel(Scan p, const RowSeg *__restr
   const int seg_id = blockIdx.x % n_seg, unit = blockIdx.x / n_seg;
   const RowSeg seg = segs[seg_id];
   if (unit >= p.heads * blocks) {
-    advance_conv_state(p, seg, unit - p.heads * blocks, blocks);
+    advance_conv_state(p, seg, unit - p.heads * blocks, gridDim.x / n_seg - p.heads * blocks);
     return;
   }
   const int h = unit / blocks;
@@ -459,15 +469,17 @@ __global__ __launch_bounds__(256) void gated_norm_vec_kernel(GatedNorm g) {
   const int at = (live ? group : 0) * g.size;
   const float *y = g.y + (size_t)row * g.ld_y + at, *gate = g.gate + (size_t)row * g.ld_gate + at;
   const float *w = g.weight ? g.weight + (g.weight_per_group ? at : 0) : nullptr;
-  f32x4 v[VPT], z[VPT];
+  f32x4 v[VPT], z[VPT], wv[VPT];
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < VPT; i++) {
     const int d = (l + LANES * i) * 4;
     v[i] = z[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    wv[i] = f32x4{1.f, 1.f, 1.f, 1.f};
     if (d < g.size) {
       v[i] = *reinterpret_cast<const f32x4 *>(y + d);
       z[i] = *reinterpret_cast<const f32x4 *>(gate + d);
+      if (w) wv[i] = *reinterpret_cast<const f32x4 *>(w + d);
     }
   }
 #pragma unroll
@@ -485,11 +497,10 @@ __global__ __launch_bounds__(256) void gated_norm_vec_kernel(GatedNorm g) {
   for (int i = 0; i < VPT; i++) {
     const int d = (l + LANES * i) * 4;
     if (d < g.size) {
-      const f32x4 wv = w ? *reinterpret_cast<const f32x4 *>(w + d) : f32x4{1.f, 1.f, 1.f, 1.f};
       f32x4 o;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        o[e] = v[i][e] * inv * wv[e];
+        o[e] = v[i][e] * inv * wv[i][e];
         if (!g.gate_first) o[e] *= g.sigmoid_gate ? sigmoid_f(z[i][e]) : silu_f(z[i][e]);
         o[e] *= g.scale;
       }
@@ -536,7 +547,10 @@ int run_short_conv(const ShortConv &c, const StepRows &r, const float *in, int l
 
 template <int NI, int KIND>
 static void launch_scan_kind(const Scan &p, const StepRows &r, hipStream_t s) {
-  auto grid = [&](int cols) { return dim3((unsigned)(r.n_seg * (p.heads + (KIND == SCAN_RETENTION ? 0 : 1)) * cdiv(p.V, cols))); };
+  // The convolutions' states: a thread per channel.  With as many workgroups as a head has column blocks, one or two, a
+  // decoding step waited for them: four sequences, 4096 channels and 32 heads of 128 x 64 15.6 -> 5.2 us.
+  const int conv = KIND == SCAN_RETENTION ? 0 : cdiv(p.conv_desc.channels, 256);
+  auto grid = [&](int cols) { return dim3((unsigned)(r.n_seg * (p.heads * cdiv(p.V, cols) + conv))); };
   // Stretches of few heads and sequences: with two columns per lane half of the chip would be idle, or every SIMD have
   // one wave, which issues an instruction every seven cycles (8 prompts of 1000 and 16 heads of 128 x 128, 256 workgroups
   // against 512: delta rule 455 -> 409 us, per key channel 544 -> 521; 32 heads of 128 x 64, state space 383 -> 342).
@@ -567,7 +581,7 @@ int run_scan(const Scan &scan, const StepRows &r, hipStream_t s) {
   GPTOSS_REQUIRE(p.K >= 1 && p.K <= SCAN_MAX_KEY && p.V >= 1 && p.key_heads >= 1 && p.heads % p.key_heads == 0,
                  GPTOSS_ERR_DIM, "scan: key dimension %d (at most %d), %d heads over %d", p.K, SCAN_MAX_KEY, p.heads,
                  p.key_heads);
-  GPTOSS_REQUIRE((long long)r.n_seg * (p.heads + 1) * cdiv(p.V, 32) < (1ll << 31), GPTOSS_ERR_DIM,
+  GPTOSS_REQUIRE(r.n_seg * ((long long)p.heads * cdiv(p.V, 32) + cdiv(p.conv_desc.channels, 256)) < (1ll << 31), GPTOSS_ERR_DIM,
                  "scan: too many workgroups");
   static const char *names[] = {"scan_delta", "scan_channel_delta", "scan_state_space", "scan_retention"};
   TraceScope ts(names[p.kind], s);

@@ -420,3 +420,15 @@ def test_command_line_generates_and_replays(open_model, tmp_path):
     for i, places in enumerate(wanted):
         lg = np.fromfile(tmp_path / f"{i}.f32", "<f4").reshape(len(places), cfg["vocab"])
         check(lg, np.stack([want[n][p] for n, p in places]), True)
+
+
+# taps - 1 inputs are state: as many as are moved at once, one more; channels: one workgroup's, one more, several
+@pytest.mark.parametrize("conv", [9, 10])
+@pytest.mark.parametrize("dim", [64, 65, 200])
+def test_long_convolutions_of_many_channels(open_model, conv, dim):
+    cfg = nm.config([nm.delta(heads=2, kv=1, dim=dim, vdim=dim, conv=conv), nm.channel_delta(heads=1, kv=1, dim=dim, conv=conv)])
+    w = nm.weights(cfg, 79)
+    tok = nm.tokens(cfg, 60, 10)
+    e = open_model(cfg, w, True, max_batch=2)
+    check_model(e, 0, cfg, w, tok, True)
+    check_model(e, 1, cfg, w, tok, True, [5, 1, 2, 20, 1, 9, 1, 8, 1])
