@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void rope_store_kernel(const float *__restrict
   const int b = seq_map ? seq_map[bi] : bi;
   const int pos = lens ? lens[r] - 1 : pos0 + (r - bi * T);
   if (pos < 0) {  // an empty sequence (lens[r] == 0): nothing to rotate or store, its q row is zero
-    if (q_out != nullptr)
+    if (q_out != nullptr && blockIdx.y == 0)
       for (int p = threadIdx.x; p < n_q * D; p += 256) q_out[(size_t)r * n_q * D + p] = 0.f;
     return;
   }
@@ -160,8 +160,10 @@ __global__ __launch_bounds__(256) void rope_store_kernel(const float *__restrict
       hi[q] = __fadd_rn(__fmul_rn(x2[q], c[q]), __fmul_rn(x1[q], s[q]));
     }
   };
+  // the row's workgroups (a few where there are few rows) share its rotations, and its values
+  const int t0 = blockIdx.y * 256 + threadIdx.x, step = gridDim.y * 256;
   if (q_out != nullptr) {
-    for (int p = threadIdx.x; p < n_q * quads; p += 256) {
+    for (int p = t0; p < n_q * quads; p += step) {
       const int h = p / quads, j4 = (p - h * quads) * 4;
       f32x4 lo, hi;
       rotate(row + h * D, j4, lo, hi);
@@ -182,17 +184,19 @@ __global__ __launch_bounds__(256) void rope_store_kernel(const float *__restrict
     }
   }
   if (pos < store_from) return;  // a ring cache keeps only the last positions of a prefill
-  for (int p = threadIdx.x; p < n_kv * quads; p += 256) {
-    const int g = p / quads, j4 = (p - g * quads) * 4;
-    f32x4 lo, hi;
-    rotate(row + q_dim + g * D, j4, lo, hi);
-    bf16_t *krow = kv + kv_block_off(b, g, n_kv, cap, D, slot) + kv_k_elem(slot, 0, D);
-    *reinterpret_cast<u32x2 *>(krow + j4) = u32x2{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3])};
-    *reinterpret_cast<u32x2 *>(krow + half + j4) = u32x2{pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
-  }
-  for (int p = threadIdx.x; p < kv_dim; p += 256) {
-    int g = p / D, d = p - g * D;
-    kv[kv_block_off(b, g, n_kv, cap, D, slot) + kv_v_elem(slot, d, D)] = f32_to_bf16(row[q_dim + kv_dim + p]);
+  // keys, then values, from the row's last workgroup backwards
+  for (int p = (gridDim.y - 1 - blockIdx.y) * 256 + threadIdx.x; p < n_kv * quads + kv_dim; p += step) {
+    if (p < n_kv * quads) {
+      const int g = p / quads, j4 = (p - g * quads) * 4;
+      f32x4 lo, hi;
+      rotate(row + q_dim + g * D, j4, lo, hi);
+      bf16_t *krow = kv + kv_block_off(b, g, n_kv, cap, D, slot) + kv_k_elem(slot, 0, D);
+      *reinterpret_cast<u32x2 *>(krow + j4) = u32x2{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3])};
+      *reinterpret_cast<u32x2 *>(krow + half + j4) = u32x2{pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+    } else {
+      const int e = p - n_kv * quads, g = e / D, d = e - g * D;
+      kv[kv_block_off(b, g, n_kv, cap, D, slot) + kv_v_elem(slot, d, D)] = f32_to_bf16(row[q_dim + kv_dim + e]);
+    }
   }
 }
 
@@ -390,6 +394,13 @@ int run_gather_rows(const float *src, float *dst, int rows, int n, int stride, i
   return GPTOSS_OK;
 }
 
+// Workgroups of a row: one for every 256 of its items while all of them together leave half of the chip idle.
+// (64 + 16 heads of 64: one row 3.8 -> 2.3 us, six 4.8 -> 4.1.)
+static dim3 rope_grid(int rows, int n_q, int n_kv, int D) {
+  const int each = cdiv(n_q * D / 8, 256) + cdiv(n_kv * D / 8 + n_kv * D, 256);
+  return dim3(rows, (long long)rows * each <= 128 ? each : 1);
+}
+
 int run_rope_store(const float *qkv, float *q_out, bf16_t *kv, const float *cos_t,
                    const float *sin_t, int B, int n_q, int n_kv, int D, int cap, int pos,
                    hipStream_t s) {
@@ -400,7 +411,7 @@ int run_rope_store_lens(const float *qkv, float *q_out, bf16_t *kv, const float 
                         const float *sin_t, int B, int n_q, int n_kv, int D, int cap, const int *lens,
                         hipStream_t s, const int *seq_map) {
   TraceScope ts("rope_store", s);
-  rope_store_kernel<true><<<B, 256, 0, s>>>(qkv, q_out, kv, cos_t, sin_t, n_q, n_kv, D, cap, 0, 1, 0, lens, seq_map);
+  rope_store_kernel<true><<<rope_grid(B, n_q, n_kv, D), 256, 0, s>>>(qkv, q_out, kv, cos_t, sin_t, n_q, n_kv, D, cap, 0, 1, 0, lens, seq_map);
   GPTOSS_LAUNCH_CHECK("rope_store_kernel");
   return GPTOSS_OK;
 }
@@ -410,10 +421,10 @@ int run_rope_store_rows(const float *qkv, float *q_out, bf16_t *kv, const float 
                         int store_from, hipStream_t s) {
   TraceScope ts("rope_store", s);
   if (T == 1)
-    rope_store_kernel<true><<<rows, 256, 0, s>>>(qkv, q_out, kv, cos_t, sin_t, n_q, n_kv, D, cap, pos0, T, store_from,
+    rope_store_kernel<true><<<rope_grid(rows, n_q, n_kv, D), 256, 0, s>>>(qkv, q_out, kv, cos_t, sin_t, n_q, n_kv, D, cap, pos0, T, store_from,
                                                  nullptr, nullptr);
   else
-    rope_store_kernel<false><<<rows, 256, 0, s>>>(qkv, q_out, kv, cos_t, sin_t, n_q, n_kv, D, cap, pos0, T, store_from,
+    rope_store_kernel<false><<<rope_grid(rows, n_q, n_kv, D), 256, 0, s>>>(qkv, q_out, kv, cos_t, sin_t, n_q, n_kv, D, cap, pos0, T, store_from,
                                                   nullptr, nullptr);
   GPTOSS_LAUNCH_CHECK("rope_store_kernel");
   return GPTOSS_OK;
@@ -514,13 +525,34 @@ __global__ __launch_bounds__(256) void embedding_position_kernel(const T *__rest
                                                                  const int *__restrict__ tokens,
                                                                  const int *__restrict__ lens,
                                                                  float *__restrict__ x, float *__restrict__ x0,
-                                                                 int H, int ld, int V, int n_pos) {
+                                                                 int H, int ld, int V, int n_pos, bool wide) {
   const int b = blockIdx.x;
   const int tok = min(max(tokens[b], 0), V - 1), pos = min(max(lens[b] - 1, 0), n_pos - 1);
   auto value = [](T v) {
     if constexpr (sizeof(T) == 2) return bf16_to_f32(v);
     else return v;
   };
+  if (H % 8 == 0 && ld % 8 == 0 && wide) {
+    // eight elements at a time: one round of loads for a row of 2048
+    typedef T v8 __attribute__((ext_vector_type(8)));
+    for (int h = threadIdx.x * 8; h < ld; h += 256 * 8) {
+      float v[8] = {};
+      if (h < H) {
+        const v8 t = *reinterpret_cast<const v8 *>(table + (size_t)tok * H + h);
+        v8 q = {};
+        if (positions) q = *reinterpret_cast<const v8 *>(positions + (size_t)pos * H + h);
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = positions ? value(t[i]) + value(q[i]) : value(t[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; i += 4) {
+        const f32x4 o = f32x4{v[i], v[i + 1], v[i + 2], v[i + 3]};
+        *reinterpret_cast<f32x4 *>(x + (size_t)b * ld + h + i) = o;
+        if (x0) *reinterpret_cast<f32x4 *>(x0 + (size_t)b * ld + h + i) = o;
+      }
+    }
+    return;
+  }
   for (int h = threadIdx.x; h < ld; h += 256) {
     float v = h < H ? value(table[(size_t)tok * H + h]) : 0.f;
     if (positions && h < H) v += value(positions[(size_t)pos * H + h]);
@@ -543,41 +575,62 @@ __global__ __launch_bounds__(256) void depth_average_norm_kernel(float *__restri
                                                                  int n_mean) {
   __shared__ double red[4];
   const size_t row = (size_t)blockIdx.x * H;
-  f32x4 v[VPT];
+  // All that does not wait for another load is requested at once, for two of a thread's pieces together: a launch of few
+  // rows is as long as its loads that come one behind the other (four rows of 2048, up to 8 layers: 7.2 -> 6.1 us).  Pieces
+  // past the row's end read its last elements.
+  constexpr int G = VPT < 2 ? VPT : 2;
+  f32x4 v[VPT], nw[VPT];
   double ss = 0.0;
 #pragma unroll
-  for (int i = 0; i < VPT; i++) {
-    const int h = (threadIdx.x + 256 * i) * 4;
-    v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (h < H) {
-      // sums in order of their index, four loads in flight at a time
-      f32x4 own = *reinterpret_cast<const f32x4 *>(y + row + h);
-      const f32x4 before = *reinterpret_cast<const f32x4 *>(x + row + h);
-      int k = 1;
-      for (; k + 4 <= parts; k += 4) {
-        f32x4 part[4];
+  for (int i0 = 0; i0 < VPT; i0 += G) {
+    auto at = [&](int i) { return row + min((threadIdx.x + 256u * (i0 + i)) * 4, H - 4u); };
+    f32x4 own[G], before[G], old[4][G], a[G];
 #pragma unroll
-        for (int q = 0; q < 4; q++) part[q] = *reinterpret_cast<const f32x4 *>(y + (k + q) * part_stride + row + h);
+    for (int i = 0; i < G; i++) {
+      own[i] = *reinterpret_cast<const f32x4 *>(y + at(i));
+      before[i] = *reinterpret_cast<const f32x4 *>(x + at(i));
+      if (norm_w) nw[i0 + i] = *reinterpret_cast<const f32x4 *>(norm_w + (at(i) - row));
+      a[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    auto load_old = [&](int j) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) own += part[q];
+      for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int i = 0; i < G; i++) old[q][i] = *reinterpret_cast<const f32x4 *>(history + (size_t)min(j + q, layer) * plane + at(i));
+    };
+    load_old(0);
+    // sums in order of their index, four at a time
+    for (int k = 1; k < parts; k += 4) {
+      f32x4 part[4][G];
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int i = 0; i < G; i++) part[q][i] = *reinterpret_cast<const f32x4 *>(y + min(k + q, parts - 1) * part_stride + at(i));
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (k + q < parts)
+#pragma unroll
+          for (int i = 0; i < G; i++) own[i] += part[q][i];
+    }
+#pragma unroll
+    for (int i = 0; i < G; i++) own[i] += before[i];
+    for (int j = 0; j <= layer; j += 4) {
+      if (j > 0) load_old(j);
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (j + q <= layer)
+#pragma unroll
+          for (int i = 0; i < G; i++) a[i] += weights[j + q] * old[q][i];
+    }
+#pragma unroll
+    for (int i = 0; i < G; i++) {
+      v[i0 + i] = a[i] + weights[layer + 1] * own[i];
+      if ((threadIdx.x + 256 * (i0 + i)) * 4 < H) {
+        *reinterpret_cast<f32x4 *>(history + (size_t)(layer + 1) * plane + at(i)) = own[i];
+        *reinterpret_cast<f32x4 *>(x + at(i)) = v[i0 + i];
+#pragma unroll
+        for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[i0 + i][q], v[i0 + i][q]);
       }
-      for (; k < parts; k++) own += *reinterpret_cast<const f32x4 *>(y + k * part_stride + row + h);
-      own += before;
-      *reinterpret_cast<f32x4 *>(history + (size_t)(layer + 1) * plane + row + h) = own;
-      f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
-      int j = 0;
-      for (; j + 4 <= layer + 1; j += 4) {
-        f32x4 old[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) old[q] = *reinterpret_cast<const f32x4 *>(history + (size_t)(j + q) * plane + row + h);
-#pragma unroll
-        for (int q = 0; q < 4; q++) a += weights[j + q] * old[q];
-      }
-      for (; j <= layer; j++) a += weights[j] * *reinterpret_cast<const f32x4 *>(history + (size_t)j * plane + row + h);
-      v[i] = a + weights[layer + 1] * own;
-      *reinterpret_cast<f32x4 *>(x + row + h) = v[i];
-#pragma unroll
-      for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[i][q], v[i][q]);
     }
   }
   if (!norm_w) return;
@@ -592,10 +645,9 @@ __global__ __launch_bounds__(256) void depth_average_norm_kernel(float *__restri
   for (int i = 0; i < VPT; i++) {
     const int h = (threadIdx.x + 256 * i) * 4;
     if (h < H) {
-      const f32x4 w = *reinterpret_cast<const f32x4 *>(norm_w + h);
       f32x4 o;
 #pragma unroll
-      for (int q = 0; q < 4; q++) o[q] = (float)((double)w[q] * (inv * (double)v[i][q]));
+      for (int q = 0; q < 4; q++) o[q] = (float)((double)nw[i][q] * (inv * (double)v[i][q]));
       *reinterpret_cast<u32x2 *>(t_bf16 + row + h) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
       if (t_f32) *reinterpret_cast<f32x4 *>(t_f32 + row + h) = o;
     }
@@ -609,25 +661,28 @@ __global__ __launch_bounds__(256) void residual_tanh_norm_kernel(float *__restri
                                                                  int H) {
   const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (at >= part_stride) return;
-  f32x4 v = *reinterpret_cast<const f32x4 *>(x + at);
+  // all that does not wait for another load at once
+  f32x4 v = *reinterpret_cast<const f32x4 *>(x + at), w, b;
+  if (norm.weight) {
+    const int h = (int)(at % (unsigned)H);
+    w = *reinterpret_cast<const f32x4 *>(norm.weight + h);
+    b = *reinterpret_cast<const f32x4 *>(norm.bias + h);
+  }
   if (parts > 0) {
-    // sums in order of their index, four loads in flight at a time
+    // sums in order of their index, four at a time
     f32x4 own = *reinterpret_cast<const f32x4 *>(y + at);
-    int k = 1;
-    for (; k + 4 <= parts; k += 4) {
+    for (int k = 1; k < parts; k += 4) {
       f32x4 part[4];
 #pragma unroll
-      for (int q = 0; q < 4; q++) part[q] = *reinterpret_cast<const f32x4 *>(y + (k + q) * part_stride + at);
+      for (int q = 0; q < 4; q++) part[q] = *reinterpret_cast<const f32x4 *>(y + min(k + q, parts - 1) * part_stride + at);
 #pragma unroll
-      for (int q = 0; q < 4; q++) own += part[q];
+      for (int q = 0; q < 4; q++)
+        if (k + q < parts) own += part[q];
     }
-    for (; k < parts; k++) own += *reinterpret_cast<const f32x4 *>(y + k * part_stride + at);
     v += own;
     *reinterpret_cast<f32x4 *>(x + at) = v;
   }
   if (!norm.weight) return;
-  const int h = (int)(at % (unsigned)H);
-  const f32x4 w = *reinterpret_cast<const f32x4 *>(norm.weight + h), b = *reinterpret_cast<const f32x4 *>(norm.bias + h);
   f32x4 o;
 #pragma unroll
   for (int q = 0; q < 4; q++) o[q] = fmaf(tanhf(norm.alpha * v[q]), w[q], b[q]);
@@ -661,7 +716,8 @@ template <typename T>
 static int launch_embedding_position(const T *table, const T *positions, const int *tokens, const int *lens, float *x,
                                      float *x0, int rows, int H, int ld, int V, int n_pos, hipStream_t s) {
   TraceScope ts("embedding", s);
-  embedding_position_kernel<T><<<rows, 256, 0, s>>>(table, positions, tokens, lens, x, x0, H, ld, V, n_pos);
+  embedding_position_kernel<T><<<rows, 256, 0, s>>>(table, positions, tokens, lens, x, x0, H, ld, V, n_pos,
+                                                    aligned(table, 32) && aligned(positions, 32) && aligned(x, 16) && aligned(x0, 16));
   GPTOSS_LAUNCH_CHECK("embedding_position_kernel");
   return GPTOSS_OK;
 }

@@ -166,13 +166,14 @@ __global__ __launch_bounds__(256) void combine_tanh_norm_kernel(const float *__r
                                                                 float *__restrict__ out, int H, int k, TanhNorm norm,
                                                                 bf16_t *__restrict__ t_bf16) {
   const int b = blockIdx.x, h = (blockIdx.y * 256 + threadIdx.x) * 4;
-  TokenExperts<KMAX> x;
-  x.load(topk_w, inv_perm, b, k);
   if (h >= H) return;
-  const f32x4 agg = x.sum(y2, H, h, k);
+  // what does not depend on the routing is requested before it
   f32x4 *op = reinterpret_cast<f32x4 *>(out + (size_t)b * H + h);
   const f32x4 prev = *op, w = *reinterpret_cast<const f32x4 *>(norm.weight + h),
               c = *reinterpret_cast<const f32x4 *>(norm.bias + h);
+  TokenExperts<KMAX> x;
+  x.load(topk_w, inv_perm, b, k);
+  const f32x4 agg = x.sum(y2, H, h, k);
   f32x4 v, o;
 #pragma unroll
   for (int q = 0; q < 4; q++) {

@@ -188,3 +188,23 @@ def test_rope_kv_store_skips_empty_sequences(ops, orc, synth):
     assert (kv1[1] != 0x1234).any()                                   # the same row with a length does store
     for b in (0, 2):
         assert np.array_equal(q0[b], q1[b]) and np.array_equal(kv0[b], kv1[b])
+
+
+@pytest.mark.parametrize("D,n_q,n_kv", [(32, 4, 4), (32, 8, 2), (64, 64, 8), (64, 6, 3)])
+def test_rotation_of_few_rows_equals_that_of_many(ops, D, n_q, n_kv):
+    """Few rows have several workgroups each; at 300 a row has one."""
+    g = torch.Generator(device="cuda").manual_seed(D + n_q)
+    B, n = 300, 70
+    qkv = torch.randn(B, (n_q + 2 * n_kv) * D, generator=g, device="cuda")
+    cs, sn = (torch.randn(n, D // 2, generator=g, device="cuda") for _ in range(2))
+    lens = torch.randint(0, n + 1, (B,), generator=g, device="cuda", dtype=torch.int32)
+
+    def rotate(rows):
+        cache = ops.KVCache(rows, n_kv, D, 128)
+        cache.kv.view(torch.int16).fill_(0x1234)
+        return ops.rope_kv_store(qkv[:rows].contiguous(), cache, cs, sn, lens[:rows].contiguous(), n_q), cache.kv.view(torch.int16).view(rows, -1)
+
+    q, kv = rotate(B)
+    for rows in (1, 2, 25, 26, 42, 43, 64, 65, 128, 129):
+        q_few, kv_few = rotate(rows)
+        assert torch.equal(q_few.view(rows, -1), q[:rows].view(rows, -1)) and torch.equal(kv_few, kv[:rows]), rows
