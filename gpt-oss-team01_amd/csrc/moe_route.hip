@@ -306,6 +306,7 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
     const bf16_t *__restrict__ t, const bf16_t *__restrict__ wr, const float *__restrict__ br,
     float *__restrict__ logits, int B, int H, int E, int k, float *__restrict__ topk_w,
     int *__restrict__ topk_i, int rows_per_wg, RouterNorm nrm, RouterGroup grp) {
+  const int e0 = blockIdx.y * (NB * 16);   // first expert of the workgroup; it gates only if it has them all
   __shared__ float red[ROUTER_WAVES][16][NB * 16 + 1];
   extern __shared__ __attribute__((aligned(16))) unsigned char t_rows_raw[];  // NORM: [rows_per_wg][H] bf16
   // The wave's number has to be a scalar: matrix instructions do not look at the mask of active lanes, so a wave skips the
@@ -326,7 +327,7 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
       const int ks = min(ks0 + u * ROUTER_WAVES, ksteps - 1);
 #pragma unroll
       for (int nb = 0; nb < NB; nb++) {
-        int e = min(nb * 16 + (lane & 15), E - 1);
+        int e = min(e0 + nb * 16 + (lane & 15), E - 1);
         b[u][nb] = *reinterpret_cast<const u32x4 *>(wr + (size_t)e * H + ks * 32 + kq);
       }
     }
@@ -339,7 +340,7 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
   constexpr int NJ = (NB + 1) / 2;
   float bias[NJ];
 #pragma unroll
-  for (int j = 0; j < NJ; j++) bias[j] = br ? br[min(sub + 32 * j, E - 1)] : 0.f;
+  for (int j = 0; j < NJ; j++) bias[j] = br ? br[min(e0 + sub + 32 * j, E - 1)] : 0.f;
   if constexpr (NORM) {
     constexpr int VPT = 4;  // rows of up to 4096 floats
     __shared__ double nred[2][4];
@@ -428,12 +429,12 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
   float v[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; j++) {
-    const int e = sub + 32 * j;
+    const int col = sub + 32 * j, e = e0 + col;
     float x = -INFINITY;
-    if (e < E) {
+    if (e < E && col < NB * 16) {
       x = 0.f;
 #pragma unroll
-      for (int w = 0; w < ROUTER_WAVES; w++) x += red[w][row][e];
+      for (int w = 0; w < ROUTER_WAVES; w++) x += red[w][row][col];
       if (br) x += bias[j];
       if (live) logits[(size_t)(r0 + row) * E + e] = x;
     }
@@ -642,6 +643,32 @@ __global__ __launch_bounds__(SORT_THREADS) void group_scatter_kernel(
 
 
 // gating only: logits [B,E] -> top-k weights and ids
+// Gating of at most ROUTER_GROUP_TOKENS tokens from their logits, and their grouping: the end of router_gemm_kernel, for
+// experts that several workgroups shared.
+template <int NJ>
+__global__ __launch_bounds__(512) void topk_group_kernel(const float *__restrict__ logits, int B, int E, int k,
+                                                         float *__restrict__ topk_w, int *__restrict__ topk_i, RouterGroup grp) {
+  __shared__ int ids[ROUTER_GROUP_PAIRS], lds[512];
+  const int row = threadIdx.x >> 5, sub = threadIdx.x & 31;
+  const bool live = row < B;
+  float v[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; j++) {
+    const float x = logits[(size_t)min(row, B - 1) * E + min(sub + 32 * j, E - 1)];
+    v[j] = sub + 32 * j < E ? x : -INFINITY;
+  }
+  const size_t o = (size_t)(live ? row : 0) * k;
+  topk_softmax_group<NJ>(v, sub, E, k, live, topk_w + o, topk_i + o, ids + row * k);
+  __syncthreads();
+  if (threadIdx.x < 64) group_by_one_wave(ids, B * k, E, lds, grp);
+}
+
+// Behind a norm in the router's kernel, where no workgroup holds every token: 5.2 us by group_sort_kernel, 2.1 by one wave.
+__global__ __launch_bounds__(64) void group_few_kernel(const int *__restrict__ topk_i, int P, int E, RouterGroup g) {
+  __shared__ int lds[512];
+  group_by_one_wave(topk_i, P, E, lds, g);
+}
+
 int run_topk_softmax(const float *logits, int B, int E, int k, float *topk_w, int *topk_i, hipStream_t s) {
   dim3 grid(cdiv(B * 32, 256)), block(256);
   int nj = cdiv(E, 32);
@@ -661,7 +688,15 @@ static int router_rows_per_wg(int B) {
   return rows_per_wg;
 }
 
-// logits (+ optional gating of the same tokens) in one launch
+// One workgroup reads all experts' weights through its CU's own 64 bytes a cycle, 27 us for 128 experts whatever the number
+// of tokens.  From 33 experts on up to 512 tokens share them out, 16 experts a workgroup, and are gated (up to 16 tokens:
+// and grouped) by a second launch: MoE block of 1 / 33 / 512 tokens, 64 experts 8.6 / 8.0 / 5.1 us less, 128 experts 16.7 /
+// 17.3 / 7.4, 256 experts 35 / 36 / 26; 40 experts 5.2 / 5.7 / 2.7.  With 1000 tokens one workgroup for all experts is as
+// fast or faster (128 experts 115 against 122 us), and so it is with 32 experts (9.3 us, gated and grouped).
+constexpr int ROUTER_SPLIT_TOKENS = 512;
+static bool router_splits(int B, int E) { return E > 32 && B <= ROUTER_SPLIT_TOKENS; }
+
+// logits (+ optional gating of the same tokens), in one launch unless many experts are shared out
 int run_router(const void *t, const void *w_router, const float *b_router, float *logits, int B,
                int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group) {
   // 16 token rows per workgroup fill the MFMA, but a thousand tokens are then only 64 workgroups;
@@ -678,6 +713,22 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
   if (topk_w && k > 8) {   // more experts per token than the fused gating holds
     const int rc = run_router(t, w_router, b_router, logits, B, H, E, k, nullptr, nullptr, s);
     return rc != GPTOSS_OK ? rc : run_topk_softmax(logits, B, E, k, topk_w, topk_i, s);
+  }
+  if (router_splits(B, E) && topk_w) {
+    const int rows = router_rows_per_wg(B);
+    {
+      TraceScope ts("router_gemm", s);
+      router_gemm_kernel<1, false><<<dim3(cdiv(B, rows), nb), block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, nullptr,
+                                                                           nullptr, rows, none, RouterGroup{});
+      GPTOSS_LAUNCH_CHECK("router_gemm_kernel");
+    }
+    if (!grp.expert_offsets) return run_topk_softmax(logits, B, E, k, topk_w, topk_i, s);
+    TraceScope ts("topk_group", s);
+    if (nb <= 4) topk_group_kernel<2><<<1, 512, 0, s>>>(logits, B, E, k, topk_w, topk_i, grp);
+    else if (nb <= 8) topk_group_kernel<4><<<1, 512, 0, s>>>(logits, B, E, k, topk_w, topk_i, grp);
+    else topk_group_kernel<8><<<1, 512, 0, s>>>(logits, B, E, k, topk_w, topk_i, grp);
+    GPTOSS_LAUNCH_CHECK("topk_group_kernel");
+    return GPTOSS_OK;
   }
   TraceScope ts(topk_w ? "router_gemm_topk" : "router_gemm", s);
   if (nb <= 1) router_gemm_kernel<1, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none, grp);
@@ -724,7 +775,8 @@ bool norm_router_applies(int B, int H, int E, const float *x, const float *resid
   // With more than four rows per workgroup (batches of more than ~1000 rows) the rows a workgroup
   // normalises one after the other cost more than the launch the fusion saves (8192 rows: 2.58 ms
   // per 24 layers against 2.23 ms for the two kernels; 1024 rows: 0.63 against 0.71 ms).
-  return B > 0 && router_rows_per_wg(B) <= 4 && H % 32 == 0 && H <= 4096 && lds <= 160 * 1024 && aligned(x, 16) && aligned(weight, 16) &&
+  // (Experts that are shared out have their norm in a kernel of its own: every workgroup would repeat it.)
+  return B > 0 && !router_splits(B, E) && router_rows_per_wg(B) <= 4 && H % 32 == 0 && H <= 4096 && lds <= 160 * 1024 && aligned(x, 16) && aligned(weight, 16) &&
          aligned(t_out, 16) && (!residual || aligned(residual, 16));
 }
 
@@ -737,7 +789,11 @@ int run_norm_router(float *x, const float *residual, const float *weight, void *
                  "norm + router: %d tokens are not grouped here", B);
   GPTOSS_REQUIRE(norm_router_applies(B, H, E, x, residual, weight, t_out), GPTOSS_ERR_DIM,
                  "norm + router: shape or alignment outside the fused kernel's range (H=%d E=%d)", H, E);
-  const int rows_per_wg = router_rows_per_wg(B);
+  // A workgroup norms two rows at a time, so up to 512 rows are two each, unless one workgroup groups them all: with four,
+  // 4 experts, 6 / 33 / 500 rows 7.4 / 7.6 / 8.7 us, with two 5.8 / 5.9 / 7.2; 32 experts 11.6 / 11.9 / 12.9 and 10.1 /
+  // 10.2 / 11.4.
+  const bool grouped = group && group->expert_offsets;
+  const int rows_per_wg = !grouped && cdiv(B, 2) <= 256 ? 2 : router_rows_per_wg(B);
   const RouterNorm nrm{x, residual, weight, (bf16_t *)t_out};
   const bf16_t *wp = (const bf16_t *)w_router;
   const size_t dyn = (size_t)rows_per_wg * H * 2;
@@ -781,6 +837,20 @@ int gptoss::run_group(int B, int E, int k, float *topk_w, int *topk_i, int *expe
                       int *xcd_bounds, int tile_cost0_x2, hipStream_t s, int *sort_scratch) {
   // the cut positions hold the tile index in 15 bits
   if (gptoss_moe_max_tiles(B, k, E, rows_per_tile) >= 32768) xcd_bounds = nullptr;
+  if (B > 0 && router_groups(B, k) && xcd_bounds && tiles && rows_per_tile >= ROUTER_GROUP_TOKENS && E >= 1 && E <= 256) {
+    RouterGroup g;
+    g.expert_offsets = expert_offsets;
+    g.sorted_pair_ids = sorted_pair_ids;
+    g.inv_perm = inv_perm;
+    g.tiles = tiles;
+    g.xcd_bounds = xcd_bounds;
+    g.nbits = 0;
+    while ((1 << g.nbits) < E) g.nbits++;
+    TraceScope ts("group_sort", s);
+    group_few_kernel<<<1, 64, 0, s>>>(topk_i, B * k, E, g);
+    GPTOSS_LAUNCH_CHECK("group_few_kernel");
+    return GPTOSS_OK;
+  }
   return moe_route_impl(nullptr, B, E, k, topk_w, topk_i, expert_offsets, sorted_pair_ids, inv_perm,
                         tiles, rows_per_tile, xcd_bounds, tile_cost0_x2, s, false, sort_scratch);
 }

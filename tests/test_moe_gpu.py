@@ -400,3 +400,44 @@ def test_routing_of_equal_and_infinite_logits(ops, E, k):
     picked = np.take_along_axis(logits, want, axis=1).astype(np.float64)
     e = np.exp(picked - picked[:, :1])
     np.testing.assert_allclose(tw, e / e.sum(1, keepdims=True), rtol=2e-6, atol=0)
+
+
+@pytest.mark.parametrize("E", [33, 48, 64, 100, 128, 256])
+@pytest.mark.parametrize("H", [64, 2880])
+def test_experts_shared_out_among_workgroups_score_and_gate_the_same(ops, E, H):
+    """From 33 experts on up to 512 tokens have 16 experts per workgroup and are gated by another launch; 600 have one
+    workgroup for all experts.  Same bits."""
+    g = torch.Generator(device="cuda").manual_seed(E + H)
+    n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    layer = ops.MoeLayer(n(E, H, std=H ** -0.5), n(E).float(), n(E, 128, H, std=0.05), n(E, 128).float(), n(E, H, 64), n(E, H).float(),
+                         top_k=4, max_tokens=600)
+    t = n(600, H)
+    out = layer.forward(t).clone()
+    want = [v.clone() for v in layer.routing_views()[:3]]
+    for tokens in (1, 3, 16, 17, 65, 512):
+        got = layer.forward(t[:tokens].contiguous())
+        for have, all_of_them in zip(layer.routing_views()[:3], want):
+            assert torch.equal(have, all_of_them[:tokens]), tokens
+        assert torch.equal(got, out[:tokens]), tokens
+
+
+@pytest.mark.parametrize("E,k", [(1, 1), (4, 4), (32, 4), (33, 8), (128, 4), (256, 8)])
+def test_grouping_of_a_few_tokens_by_one_wave(ops, E, k):
+    """gptoss::run_group, which has no C entry point, by its linker name, against gptoss_moe_route's kernels."""
+    import ctypes as C
+    from conftest import load_pkg
+    lib = load_pkg("lib")
+    f = getattr(lib.load(), "_ZN6gptoss9run_groupEiiiPfPiS1_S1_S1_S1_iS1_iP12ihipStream_tS1_")
+    f.restype, f.argtypes = C.c_int, [C.c_int] * 3 + [C.c_void_p] * 6 + [C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p]
+    g = torch.Generator(device="cuda").manual_seed(E + k)
+    for tokens in (1, 2, 5, 15, 16, 17):
+        logits = torch.randn(tokens, E, generator=g, device="cuda")
+        w, i, off, srt, inv, tiles = ops.moe_route(logits, k, rows_per_tile=32)
+        got = [torch.full_like(x, -1) for x in (off, srt, inv, tiles)]
+        bounds = torch.full((16 + tokens * k + E,), -1, dtype=torch.int32, device="cuda")
+        lib.check(f(tokens, E, k, w.data_ptr(), i.data_ptr(), *[x.data_ptr() for x in got], 32, bounds.data_ptr(), 32,
+                    torch.cuda.current_stream().cuda_stream, None))
+        n_tiles = int(tiles[0])
+        for have, want in zip(got[:3] + [got[3][:1 + 3 * n_tiles]], (off, srt, inv, tiles[:1 + 3 * n_tiles])):
+            assert torch.equal(have, want), tokens
+        assert bounds[0] == 0 and bounds[8] == n_tiles << 16 and bool((bounds[:9].diff() >= 0).all())
