@@ -268,25 +268,45 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
   // tile's last one repeat it (their results are not stored).  The pair ids of a gathered tile are
   // read through the constant address space: scalar loads, which the vector-memory counter of the
   // hand-counted waits does not see.
+  // Eight ids are one scalar load, four of which are requested together: id by id, with a wait for each group of rows, an
+  // item began with 3.6 us of its 87 (block of 4500 tokens 1081 -> 1073 us, of 5999 1260 -> 1254).  A tile of fewer than
+  // eight rows reads on behind them, into what follows in the workspace, and does not use it.  id / top_k is a
+  // multiplication, exact for ids below 2^32 / top_k^2 (they stay below 2^31 / 64, top_k at most 32).
+  const uint32_t inv_k = 0xffffffffu / (uint32_t)p.top_k + 1u;   // 2^32 / top_k rounded up; 1: 0
   auto a_offsets = [&](TallSrc<SH> &t) {
-    const const_as<int> ids = constant_ptr(p.row_ids);
-#pragma unroll
-    for (int q = 0; q < LA; q++) {
-      const int r0 = (w * LA + q) * 8, r = r0 + (lane >> 3);
-      int src;
-      if (GATHER) {
-        src = ids[t.row0 + min(r0, t.rows - 1)];
-#pragma unroll
-        for (int i = 1; i < 8; i++) {
-          const int id = ids[t.row0 + min(r0 + i, t.rows - 1)];
-          src = (lane >> 3) == i ? id : src;
-        }
-        src /= p.top_k;
-      } else {
-        src = t.row0 + min(r, t.rows - 1);
-      }
+    typedef int ids_t __attribute__((ext_vector_type(8), aligned(4)));
+    const int last = t.rows - 1, group = lane >> 3;
+    auto offset = [&](int src, int r) {
       const int c = (lane & 7) ^ ((r >> 1) & 7);
-      t.a[q] = ((uint32_t)src * (uint32_t)K) * 2u + (uint32_t)c * 16u;
+      return ((uint32_t)src * (uint32_t)K) * 2u + (uint32_t)c * 16u;
+    };
+    if constexpr (GATHER) {
+      static_assert(LA % 4 == 0, "four row groups at a time");
+#pragma unroll
+      for (int q0 = 0; q0 < LA; q0 += 4) {
+        ids_t v[4];
+        int base[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          base[q] = max(min((w * LA + q0 + q) * 8, last - 7), 0);
+          v[q] = *(const_as<ids_t>)(p.row_ids + t.row0 + base[q]);
+        }
+        asm volatile("" : "+s"(v[0]), "+s"(v[1]), "+s"(v[2]), "+s"(v[3]));
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int r = (w * LA + q0 + q) * 8 + group, j = min(r, last) - base[q];
+          int src = v[q][0];
+#pragma unroll
+          for (int i = 1; i < 8; i++) src = j == i ? v[q][i] : src;
+          t.a[q0 + q] = offset(inv_k ? (int)__umulhi((uint32_t)src, inv_k) : src, r);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < LA; q++) {
+        const int r = (w * LA + q) * 8 + group;
+        t.a[q] = offset(t.row0 + min(r, last), r);
+      }
     }
   };
 

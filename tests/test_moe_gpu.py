@@ -441,3 +441,34 @@ def test_grouping_of_a_few_tokens_by_one_wave(ops, E, k):
         for have, want in zip(got[:3] + [got[3][:1 + 3 * n_tiles]], (off, srt, inv, tiles[:1 + 3 * n_tiles])):
             assert torch.equal(have, want), tokens
         assert bounds[0] == 0 and bounds[8] == n_tiles << 16 and bool((bounds[:9].diff() >= 0).all())
+
+
+def _prompt_pass_equals_small_batches(ops, g, router, b_router, t, k):
+    n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    E, H = router.shape
+    layer = ops.MoeLayer(router, b_router, n(E, 512, H, std=0.05), n(E, 512).float(), n(E, H, 256, std=0.05), n(E, H).float(),
+                         top_k=k, max_tokens=len(t))
+    out = layer.forward(t).clone()                      # 512 rows per expert on average: tiles of 256
+    for i in range(0, len(t), 100):
+        assert torch.equal(layer.forward(t[i:i + 100].contiguous()), out[i:i + 100]), i
+
+
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 250, 255, 256, 257, 263, 264, 520])
+def test_last_row_tiles_of_a_prompt_pass(ops, rows):
+    """Two experts, one per token: `rows` tokens take the first one."""
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    t = torch.randn(1100, 256, generator=g, device="cuda").bfloat16()
+    t[:, 0] = -1.0
+    t[torch.randperm(1100, generator=g, device="cuda")[:rows], 0] = 1.0
+    router = torch.zeros(2, 256, device="cuda").bfloat16()
+    router[0, 0] = 1.0
+    _prompt_pass_equals_small_batches(ops, g, router, torch.zeros(2, device="cuda"), t, 1)
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 7, 8])
+def test_tokens_of_pairs_in_a_prompt_pass(ops, k):
+    """Every token on all k experts: the token of a pair is the pair's number over k."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    t = torch.randn(519, 256, generator=g, device="cuda").bfloat16()
+    _prompt_pass_equals_small_batches(ops, g, torch.randn(k, 256, generator=g, device="cuda").bfloat16(),
+                                      torch.zeros(k, device="cuda"), t, k)
