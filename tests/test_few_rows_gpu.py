@@ -112,6 +112,19 @@ def test_products_with_their_k_cut_add_up(ops, N, K):
     assert cut == {1} if K == 128 else len(cut) > 1
 
 
+@pytest.mark.parametrize("H,I,E,k", [(320, 2880, 8, 4), (2880, 576, 32, 4)])
+def test_mxfp4_rows_of_9_to_16_tokens_equal_those_of_a_larger_batch(ops, H, I, E, k):
+    g = torch.Generator(device="cuda").manual_seed(H + I)
+    # exponents over the range of checkpoints, each column and each 32 inputs their own
+    sc = lambda *s: (127 - torch.randint(4, 12, s, generator=g, device="cuda")).to(torch.uint8)
+    layer = ops.MoeLayerMxfp4(_n(g, E, H, std=H ** -0.5), _n(g, E), _codes(g, E, 2 * I, H // 2), sc(E, 2 * I, H // 32), _n(g, E, 2 * I),
+                              _codes(g, E, H, I // 2), sc(E, H, I // 32), _n(g, E, H), top_k=k, max_tokens=512)
+    t = _n(g, 400, H)
+    want = layer.forward(t).clone()
+    for tokens in (8, 9, 10, 13, 15, 16, 17):
+        assert torch.equal(layer.forward(t[50:50 + tokens].contiguous()), want[50:50 + tokens]), tokens
+
+
 class _Range(C.Structure):   # gptoss::GemmBf16Range
     _fields_ = [("first", C.c_int), ("end", C.c_int), ("out", C.c_void_p), ("ld", C.c_int), ("relu_squared", C.c_int)]
 
