@@ -33,7 +33,8 @@ namespace gptoss {
 
 // A workgroup: WAVES 32-column blocks, one per wave, times tiles of at most ROWS rows.
 //   4 x 32, 4 x 64   the waves share the staged rows
-//   4 x 16           the same for 9 to 16 rows
+//   4 x 16           the same for 9 to 16 rows, half the staging: MXFP4 block of 9 / 12 / 16 tokens 77.5 / 79.9 / 81.9 -> 73.6 /
+//                    75.8 / 77.8 us, 128 experts 95.6 / 112 / 135 -> 89.2 / 105 / 126
 //   1 x 8            one wave can stage so few rows by itself, and four times as many workgroups fill the chip: one
 //                    token's block 68 -> 59 us, eight tokens' 178 -> 176
 //   1 x 16, 1 x 32, 1 x 64   the same for launches of at most FEW_SOLO_BLOCKS blocks, on the registers of two waves
@@ -52,11 +53,10 @@ constexpr int few_ahead(int rows) { return rows <= 32 ? 4 : 2; }       // k-step
 constexpr int few_occupancy(int waves, int rows, bool fp4) { return waves == 1 && rows > 8 ? 1 : fp4 ? 3 : 2; }
 
 // Products by 16x16x32 instructions.  Not for whole blocks of 32 rows on one wave: with four accumulators and twice the
-// operand sets, 5120 x 2880 takes 11.7 instead of 10.9 us at 24 rows.  MXFP4's codes have to be exchanged between lanes for
-// it, which pays where four waves share 16 rows (block of 9 / 12 / 16 tokens 77.5 / 79.9 / 81.9 -> 74.6 / 77.1 / 79.1 us,
-// 128 experts 95.6 / 112 / 135 -> 91.0 / 106 / 128) and not for one wave and 8 rows (one token 30.7 -> 33.7, four 48.6 -> 50.7).
+// operand sets, 5120 x 2880 takes 11.7 instead of 10.9 us at 24 rows.  Not for MXFP4, whose codes have to be exchanged between
+// lanes for it (four waves: 12 tokens 75.8 -> 76.9 us, 27 93.1 -> 96.6; one wave: one token 30.7 -> 33.7).
 constexpr bool few_narrow(int waves, int rows, int cols, bool fp4) {
-  return fp4 ? rows > 8 && rows <= 16 : rows <= 16 || cols == 16 || (waves == 4 && rows <= 32);
+  return !fp4 && (rows <= 16 || cols == 16 || (waves == 4 && rows <= 32));
 }
 constexpr int FEW_CUS = 256;   // compute units
 
@@ -141,8 +141,8 @@ __device__ __forceinline__ void few_block(const GemmParams &p, bf16_t *lds, int 
   uint32_t sc[RING];
   // a lane's first 16 bytes of a slab, and how far apart they are: narrow, fragment q & 1 of a k-step is its column half
   const int group = lane >> 4;
-  const uint32_t w_lane = NARROW && !FP4 ? (group >> 1) * 1024 + (group & 1) * 512 + (lane & 15) * 16 + (COLS == 16 ? (cb & 1) * 256 : 0) : lane * 16;
-  auto w_at = [](int q) { return NARROW && !FP4 ? q / NH * 2048 + q % NH * 256 : q * 1024; };
+  const uint32_t w_lane = NARROW ? (group >> 1) * 1024 + (group & 1) * 512 + (lane & 15) * 16 + (COLS == 16 ? (cb & 1) * 256 : 0) : lane * 16;
+  auto w_at = [](int q) { return NARROW ? q / NH * 2048 + q % NH * 256 : q * 1024; };
   auto load_w = [&](int s, auto r) {
     constexpr int R = decltype(r)::value;
 #pragma unroll
@@ -234,24 +234,11 @@ __device__ __forceinline__ void few_block(const GemmParams &p, bf16_t *lds, int 
         for (int x = 0; x < AHEAD; x++) {
           constexpr int K0 = decltype(hh)::value * AHEAD;
           if constexpr (NARROW) {
-            bf16x8 b[NH];
-            if constexpr (FP4) {
-              // A lane has 8 codes of a column for each 16 k, of the column's half lane >> 4 & 1 and the k's half lane >> 5,
-              // and is to have those of its group's 8 of 32 k for both column halves: two exchanges of rows of lanes.
-              const auto k = __builtin_amdgcn_permlane32_swap(w[R][0][2 * (K0 + x)], w[R][0][2 * (K0 + x) + 1], false, false);
-              const auto c = __builtin_amdgcn_permlane16_swap(k[0], k[1], false, false);
-              const auto e = __builtin_amdgcn_permlane16_swap(sc[R], sc[R], false, false);
-#pragma unroll
-              for (int h = 0; h < NH; h++) b[h] = as_bf16x8(fp4_expand(c[h], fp4_scale((e[h] >> (8 * (K0 + x))) & 0xffu)));
-            } else {
-#pragma unroll
-              for (int h = 0; h < NH; h++) b[h] = as_bf16x8(w[R][((K0 + x) * NH + h) % WQ]);
-            }
 #pragma unroll
             for (int h = 0; h < NH; h++)
 #pragma unroll
               for (int i = 0; i < RB; i++)
-                acc4[i][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[h], af[G & 1][x][i], acc4[i][h], 0, 0, 0);
+                acc4[i][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(w[R][((K0 + x) * NH + h) % WQ]), af[G & 1][x][i], acc4[i][h], 0, 0, 0);
             continue;
           }
           bf16x8 b;
