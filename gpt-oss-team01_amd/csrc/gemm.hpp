@@ -61,7 +61,7 @@ struct GemmParams {
 // (mat,row-tile) items.
 int run_gemm(const GemmParams &p, bool gather, int epi, int rows_per_tile, int max_tiles,
              hipStream_t s);
-// gemm_few.hip: tiles of at most 32 or 64 rows, one wave per 32 columns (bf16 weights; gather + SwiGLU, or no gather and
+// gemm_few.hip: tiles of at most 32 or 64 rows, one wave per 32 columns or 16 (bf16 weights; gather + SwiGLU, or no gather and
 // EPI_F32, EPI_MIXED, EPI_PARTIAL).  The rows of A lie within a 31-bit byte offset.
 int run_gemm_few(const GemmParams &p, bool gather, int epi, int rows_per_tile, int max_tiles, hipStream_t s);
 constexpr int FEW_SOLO_BLOCKS = 512;   // up to so many 32-column blocks a workgroup is one block

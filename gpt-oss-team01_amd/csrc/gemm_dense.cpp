@@ -89,6 +89,8 @@ static int gemm_prepare_device() {
 // rounds: 5 % on top, as what they gain at a tie is less than what they lose).  With one fixed part per launch, products of
 // short K or narrow N took up to 37 % longer than on streaming kernels alone (us: 1280 x 1280 with its K cut, 257 rows
 // 11.1 instead of 8.1; 2048 x 256, 257 rows 8.0 instead of 6.3).
+// (Few-row tiles of up to 16 rows have become up to a third faster since, gemm_few_kernel.hpp; the estimates leave that out, and
+// err towards the streaming kernels and more parts there.)
 static double streaming_us(int mb, long long blocks, int slabs) {
   // [mb - 1]: launch; per round, and per slab of it; per full round's items, and per slab of them
   static const double t[5][5] = {{3.2, 0.63, 0.496, 1.8, 0.028}, {3.5, 1.35, 0.533, 3.3, 0.106}, {4.0, 2.5, 0.578, 3.8, 0.145},

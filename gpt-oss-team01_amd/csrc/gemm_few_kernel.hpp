@@ -10,7 +10,7 @@
 // slabs (64 rows, MXFP4: four) are staged in LDS, one barrier each, and W's loads stay in flight across it.  Operand
 // roles, order of the sum over K and epilogues are those of the streaming kernels, so a row has the same bits whichever
 // kernel computes it.
-// Measured, 2880 x 2880 experts, streaming kernels -> these (us): one token, both products 36 + 32 -> 24 + 14, MXFP4
+// Measured, 2880 x 2880 experts, streaming kernels -> these (us): one token, both products 36 + 32 -> 24 + 14 (21 + 13 with what follows), MXFP4
 // block 60 -> 43; 27 tokens 156 + 91 -> 157 + 81 (5.9-6.8 TB/s either way); MXFP4 block of 12 tokens 114 -> 87.
 // Dense 5120 x 2880: one row 31 -> 9, 32 rows 33 -> 11, 64 rows 37 -> 16, 200 rows 32 -> 21.
 //

@@ -300,7 +300,8 @@ struct RouterNorm {
 // LDS and multiplies from there: one launch and one read of t less than norm kernel + router kernel.
 // A small launch is a chain of waits for memory, so all that does not depend on each other is requested at once: the
 // router's weights and biases, a row's elements, its residual and the norm's weights.  (With a branch for each of the
-// row's parts they came one behind the other.)  One row of 2880, 4 experts 8.4 -> 7.3 us, 33 rows 10.6 -> 8.4.
+// row's parts they came one behind the other.)  One row of 2880, 4 experts 8.4 -> 7.3 us, 33 rows 10.6 -> 8.4
+// (6.1 with two rows per workgroup, run_norm_router).
 template <int NB, bool NORM>
 __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
     const bf16_t *__restrict__ t, const bf16_t *__restrict__ wr, const float *__restrict__ br,
