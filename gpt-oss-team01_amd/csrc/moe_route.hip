@@ -645,7 +645,6 @@ __global__ __launch_bounds__(SORT_THREADS) void group_scatter_kernel(
 }
 
 
-// gating only: logits [B,E] -> top-k weights and ids
 // Gating of at most ROUTER_GROUP_TOKENS tokens from their logits, and their grouping: the end of router_gemm_kernel, for
 // experts that several workgroups shared.
 template <int NJ>
@@ -672,6 +671,7 @@ __global__ __launch_bounds__(64) void group_few_kernel(const int *__restrict__ t
   group_by_one_wave(topk_i, P, E, lds, g);
 }
 
+// gating only: logits [B,E] -> top-k weights and ids
 int run_topk_softmax(const float *logits, int B, int E, int k, float *topk_w, int *topk_i, hipStream_t s) {
   dim3 grid(cdiv(B * 32, 256)), block(256);
   int nj = cdiv(E, 32);
@@ -691,15 +691,42 @@ static int router_rows_per_wg(int B) {
   return rows_per_wg;
 }
 
-// One workgroup reads all experts' weights through its CU's own 64 bytes a cycle, 27 us for 128 experts whatever the number
-// of tokens.  From 33 experts on up to 512 tokens share them out, 16 experts a workgroup, and are gated (up to 16 tokens:
-// and grouped) by a second launch: MoE block of 1 / 33 / 512 tokens, 64 experts 8.6 / 8.0 / 5.1 us less, 128 experts 16.7 /
-// 17.3 / 7.4, 256 experts 35 / 36 / 26; 40 experts 5.2 / 5.7 / 2.7.  With 1000 tokens one workgroup for all experts is as
-// fast or faster (128 experts 115 against 122 us), and so it is with 32 experts (9.3 us, gated and grouped).
-constexpr int ROUTER_SPLIT_TOKENS = 512;
-static bool router_splits(int B, int E) { return E > 32 && B <= ROUTER_SPLIT_TOKENS; }
+// 16-expert column blocks of the kernel instance that holds all experts
+static int router_col_blocks(int E) {
+  const int nb = cdiv(E, 16);
+  return nb <= 1 ? 1 : nb <= 2 ? 2 : nb <= 4 ? 4 : nb <= 8 ? 8 : 16;
+}
 
-// logits (+ optional gating of the same tokens), in one launch unless many experts are shared out
+// Whether a workgroup takes 16 experts instead of all of them.  What one takes is its rounds of loads: 190 to 260 loads of
+// 16 rows x 64 bytes, which its CU returns at 36 KB a us, whatever of them is needed (one token, 128 experts of 1024 / 2048 /
+// 2880 / 4096 inputs 9.7 / 16.7 / 23.8 / 31.0 us; 32 experts of 512 to 2880 inputs 7.7, one round).  Sharing the experts out
+// saves loads and costs a second launch, which gates (up to 16 tokens: and groups).  All experts in one workgroup -> shared
+// out, MoE block with narrow experts (us):
+//   more than one round  2880 inputs, 64 experts, 1 / 512 tokens 29.9 / 80.2 -> 20.7 / 71.3, 128 39.0 / 104 -> 22.0 / 87.0, 33 experts,
+//                        17 / 512 tokens 39.0 / 86.0 -> 34.8 / 82.4; 1024 inputs, 256 experts, 512 tokens 62.6 -> 57.6
+//   one round            1024 inputs, 64 experts, 1 / 256 tokens 19.5 / 36.3 -> 17.2 / 34.3; but 48 experts, 256 tokens 36.9 -> 36.5,
+//                        33 experts 35.9 -> 36.6, 96 experts, 400 tokens 44.5 -> 46.0, 512 inputs, 192 experts, 400 tokens
+//                        38.1 -> 43.1, and 64 inputs, 128 experts, 1 / 256 tokens 14.9 / 26.4 -> 15.2 / 26.6
+// Beyond 512 tokens one workgroup for all is as fast or faster (2880 inputs, 128 experts, 1000 tokens 115 against 122).  A norm
+// in front runs in the router's kernel only if that has all experts: its launch is saved as well there, about 1 us to the
+// other side from 17 tokens on (1024 inputs, 64 experts, 256 tokens 38.1 -> 37.3, 96 experts, 200 tokens +0.8).
+static bool router_splits(int B, int H, int E) {
+  if (E <= 32) return false;
+  const bool one_round = H / 32 <= ROUTER_WAVES * router_steps(router_col_blocks(E));
+  return one_round ? E > 48 && H >= 256 && B <= 256 : B <= 512;
+}
+
+// Rows of a workgroup of 16 experts: four where that is no more than a workgroup per CU.  With four whatever their number,
+// 512 tokens over 128 experts took 59.8 instead of 50.1 us at 1024 inputs, 96.5 instead of 87.0 at 2880, and with 16 rows
+// one token or 16 up to 2 us longer.
+static int router_split_rows(int B, int E) {
+  int rows = 4;
+  while (rows < 16 && cdiv(B, rows) * cdiv(E, 16) > 256) rows *= 2;
+  return rows;
+}
+
+// logits (+ optional gating of the same tokens), in one launch unless many experts are shared out (only with the gating of at
+// most 8 experts per token: logits alone come from one workgroup for all experts)
 int run_router(const void *t, const void *w_router, const float *b_router, float *logits, int B,
                int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group) {
   // 16 token rows per workgroup fill the MFMA, but a thousand tokens are then only 64 workgroups;
@@ -717,8 +744,8 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
     const int rc = run_router(t, w_router, b_router, logits, B, H, E, k, nullptr, nullptr, s);
     return rc != GPTOSS_OK ? rc : run_topk_softmax(logits, B, E, k, topk_w, topk_i, s);
   }
-  if (router_splits(B, E) && topk_w) {
-    const int rows = router_rows_per_wg(B);
+  if (router_splits(B, H, E) && topk_w) {
+    const int rows = router_split_rows(B, E);
     {
       TraceScope ts("router_gemm", s);
       router_gemm_kernel<1, false><<<dim3(cdiv(B, rows), nb), block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, nullptr,
@@ -773,13 +800,13 @@ static int launch_norm_router(const RouterNorm &nrm, const bf16_t *wp, const flo
 
 bool norm_router_applies(int B, int H, int E, const float *x, const float *residual, const float *weight,
                          const void *t_out) {
-  const int nb = cdiv(E, 16) <= 1 ? 1 : cdiv(E, 16) <= 2 ? 2 : cdiv(E, 16) <= 4 ? 4 : cdiv(E, 16) <= 8 ? 8 : 16;
+  const int nb = router_col_blocks(E);
   const size_t lds = (size_t)ROUTER_WAVES * 16 * (nb * 16 + 1) * 4 + (size_t)router_rows_per_wg(B) * H * 2 + 640;   // (and the pair ids)
   // With more than four rows per workgroup (batches of more than ~1000 rows) the rows a workgroup
   // normalises one after the other cost more than the launch the fusion saves (8192 rows: 2.58 ms
   // per 24 layers against 2.23 ms for the two kernels; 1024 rows: 0.63 against 0.71 ms).
   // (Experts that are shared out have their norm in a kernel of its own: every workgroup would repeat it.)
-  return B > 0 && !router_splits(B, E) && router_rows_per_wg(B) <= 4 && H % 32 == 0 && H <= 4096 && lds <= 160 * 1024 && aligned(x, 16) && aligned(weight, 16) &&
+  return B > 0 && !router_splits(B, H, E) && router_rows_per_wg(B) <= 4 && H % 32 == 0 && H <= 4096 && lds <= 160 * 1024 && aligned(x, 16) && aligned(weight, 16) &&
          aligned(t_out, 16) && (!residual || aligned(residual, 16));
 }
 

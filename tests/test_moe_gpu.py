@@ -403,10 +403,10 @@ def test_routing_of_equal_and_infinite_logits(ops, E, k):
 
 
 @pytest.mark.parametrize("E", [33, 48, 64, 100, 128, 256])
-@pytest.mark.parametrize("H", [64, 2880])
+@pytest.mark.parametrize("H", [64, 256, 2880])
 def test_experts_shared_out_among_workgroups_score_and_gate_the_same(ops, E, H):
-    """From 33 experts on up to 512 tokens have 16 experts per workgroup and are gated by another launch; 600 have one
-    workgroup for all experts.  Same bits."""
+    """From 33 experts on up to 512 tokens (H = 256: from 49, up to 256; H = 64: none) have 16 experts per workgroup and are
+    gated by another launch; 600 have one workgroup for all experts.  Same bits."""
     g = torch.Generator(device="cuda").manual_seed(E + H)
     n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
     layer = ops.MoeLayer(n(E, H, std=H ** -0.5), n(E).float(), n(E, 128, H, std=0.05), n(E, 128).float(), n(E, H, 64), n(E, H).float(),
@@ -414,11 +414,28 @@ def test_experts_shared_out_among_workgroups_score_and_gate_the_same(ops, E, H):
     t = n(600, H)
     out = layer.forward(t).clone()
     want = [v.clone() for v in layer.routing_views()[:3]]
-    for tokens in (1, 3, 16, 17, 65, 512):
+    for tokens in (1, 3, 16, 17, 65, 256, 257, 512):
         got = layer.forward(t[:tokens].contiguous())
         for have, all_of_them in zip(layer.routing_views()[:3], want):
             assert torch.equal(have, all_of_them[:tokens]), tokens
         assert torch.equal(got, out[:tokens]), tokens
+
+
+# up to 64 experts a round of loads is 1792 inputs, up to 128 1024, beyond 512; more than that: shared out up to 512 tokens,
+# less: 256 inputs and 49 experts or more, up to 256 tokens
+@pytest.mark.parametrize("H,E,tokens,shared", [
+    (4096, 32, 1, False), (1856, 33, 1, True), (1792, 33, 1, False), (1792, 48, 16, False), (1792, 49, 16, True), (1088, 128, 257, True),
+    (1024, 128, 257, False), (1024, 65, 256, True), (576, 129, 512, True), (576, 129, 513, False), (512, 256, 257, False),
+    (512, 256, 256, True), (256, 64, 17, True), (192, 256, 17, False), (64, 256, 1, False)])
+def test_which_calls_share_their_experts_out(ops, H, E, tokens, shared):
+    g = torch.Generator(device="cuda").manual_seed(H)
+    n = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    layer = ops.MoeLayer(n(E, H), n(E).float(), n(E, 128, H), n(E, 128).float(), n(E, H, 64), n(E, H).float(), top_k=4, max_tokens=tokens)
+    t = n(tokens, H)
+    with ops.KernelTrace(16) as trace:
+        layer.forward(t)
+    launches = [name for name, _ in trace.results()]
+    assert ("router_gemm" in launches) == shared and ("router_gemm_topk" in launches) != shared
 
 
 @pytest.mark.parametrize("E,k", [(1, 1), (4, 4), (32, 4), (33, 8), (128, 4), (256, 8)])
