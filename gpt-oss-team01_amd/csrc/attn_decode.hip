@@ -804,10 +804,11 @@ static bool attn_few(long long pairs, int span, int head_dim) {
 }
 
 // Merge the chunk partials of one (sequence, q head) with the sink logit.  One thread owns four
-// consecutive output elements.  It is a chain of waits for memory at any size, so the partials of the first
-// U chunks are requested together with the row's length, before it is known how many there are (what lies in
-// the others is left out).  Longer rows go on in groups of that many, maxima first.  Both kernels of 3 rows of 8000
-// 16.5 -> 15.2 us, of 8 of 3000 15.8 -> 14.8 (of which attn_few_kernel 0.3).
+// consecutive output elements.  It is a chain of waits for memory at any size: the row's length, then the partials of up to U
+// chunks together, maxima, sums and outputs (longer rows go on in groups of U, maxima first).  Both kernels of 3 rows of 8000
+// 18.3 -> 16.3 us, of one long row among 63 34.5 -> 33.2, against maxima first and partials after them.  Places past the row's
+// last chunk read that again: reading on through the workspace, which the caches do not hold, 16 / 63 rows of 4000 positions
+// with room for 8000 took 30.5 / 100.6 us instead of 29.1 / 98.6.
 template <int D, int U>  // U: chunks requested at once
 __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
   constexpr int TPP = D / 4;  // threads per (b, head)
@@ -819,20 +820,18 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   f32x2 ml[U];
   f32x4 o[U];
+  const SeqRange r = seq_range(row_len(p, b), p.cap, p.window, p.max_len);
+  if (r.nchunks <= 1) return;  // already finished by the first kernel
   auto load = [&](int c0) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const size_t slot = slot0 + (size_t)min(c0 + u, p.max_chunks - 1) * p.n_q;
+      const size_t slot = slot0 + (size_t)min(c0 + u, r.nchunks - 1) * p.n_q;
       ml[u] = *reinterpret_cast<const f32x2 *>(p.part_ml + slot * 2);
       o[u] = *reinterpret_cast<const f32x4 *>(p.part_o + slot * D + d4);
     }
   };
-  const int len = row_len(p, b);
-  const float sink = p.sinks ? p.sinks[hq] : -INFINITY;
   load(0);
-  const SeqRange r = seq_range(len, p.cap, p.window, p.max_len);
-  if (r.nchunks <= 1) return;  // already finished by the first kernel
-  const float sink2 = p.sinks ? sink * 1.4426950408889634f : -INFINITY;
+  const float sink2 = p.sinks ? p.sinks[hq] * 1.4426950408889634f : -INFINITY;
   float M = NEG_BIG;
 #pragma unroll
   for (int u = 0; u < U; u++) M = u < r.nchunks ? fmaxf(M, ml[u][0]) : M;
