@@ -123,7 +123,9 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(float *__restrict__ x
 // reference: qkv_split_rope_store_kernel, layer_hip_batch.cpp:686-776
 // Q_ONCE: q is stored with the non-temporal hint (a compile-time choice: the compiler merges a plain
 // and a hinted store of the same value under a run-time condition into one plain store).
-template <bool Q_ONCE>
+// SHARED: a row has several workgroups (rope_grid).  One alone walks keys and values in loops of their own: in the shared
+// loop, whose stride is no constant, 300 rows of 128 + 32 heads took 7.4 instead of 6.5 us, 1000 18.3 instead of 16.8.
+template <bool Q_ONCE, bool SHARED>
 __global__ __launch_bounds__(256) void rope_store_kernel(const float *__restrict__ qkv,
                                                          float *__restrict__ q_out,
                                                          bf16_t *__restrict__ kv,
@@ -140,7 +142,7 @@ __global__ __launch_bounds__(256) void rope_store_kernel(const float *__restrict
   const int b = seq_map ? seq_map[bi] : bi;
   const int pos = lens ? lens[r] - 1 : pos0 + (r - bi * T);
   if (pos < 0) {  // an empty sequence (lens[r] == 0): nothing to rotate or store, its q row is zero
-    if (q_out != nullptr && blockIdx.y == 0)
+    if (q_out != nullptr && (!SHARED || blockIdx.y == 0))
       for (int p = threadIdx.x; p < n_q * D; p += 256) q_out[(size_t)r * n_q * D + p] = 0.f;
     return;
   }
@@ -161,7 +163,7 @@ __global__ __launch_bounds__(256) void rope_store_kernel(const float *__restrict
     }
   };
   // the row's workgroups (a few where there are few rows) share its rotations, and its values
-  const int t0 = blockIdx.y * 256 + threadIdx.x, step = gridDim.y * 256;
+  const int t0 = SHARED ? blockIdx.y * 256 + threadIdx.x : threadIdx.x, step = SHARED ? gridDim.y * 256 : 256;
   if (q_out != nullptr) {
     for (int p = t0; p < n_q * quads; p += step) {
       const int h = p / quads, j4 = (p - h * quads) * 4;
@@ -184,19 +186,27 @@ __global__ __launch_bounds__(256) void rope_store_kernel(const float *__restrict
     }
   }
   if (pos < store_from) return;  // a ring cache keeps only the last positions of a prefill
-  // keys, then values, from the row's last workgroup backwards
-  for (int p = (gridDim.y - 1 - blockIdx.y) * 256 + threadIdx.x; p < n_kv * quads + kv_dim; p += step) {
-    if (p < n_kv * quads) {
-      const int g = p / quads, j4 = (p - g * quads) * 4;
-      f32x4 lo, hi;
-      rotate(row + q_dim + g * D, j4, lo, hi);
-      bf16_t *krow = kv + kv_block_off(b, g, n_kv, cap, D, slot) + kv_k_elem(slot, 0, D);
-      *reinterpret_cast<u32x2 *>(krow + j4) = u32x2{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3])};
-      *reinterpret_cast<u32x2 *>(krow + half + j4) = u32x2{pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
-    } else {
-      const int e = p - n_kv * quads, g = e / D, d = e - g * D;
-      kv[kv_block_off(b, g, n_kv, cap, D, slot) + kv_v_elem(slot, d, D)] = f32_to_bf16(row[q_dim + kv_dim + e]);
+  auto store_key = [&](int p) {
+    const int g = p / quads, j4 = (p - g * quads) * 4;
+    f32x4 lo, hi;
+    rotate(row + q_dim + g * D, j4, lo, hi);
+    bf16_t *krow = kv + kv_block_off(b, g, n_kv, cap, D, slot) + kv_k_elem(slot, 0, D);
+    *reinterpret_cast<u32x2 *>(krow + j4) = u32x2{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3])};
+    *reinterpret_cast<u32x2 *>(krow + half + j4) = u32x2{pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+  };
+  auto store_value = [&](int p) {
+    const int g = p / D, d = p - g * D;
+    kv[kv_block_off(b, g, n_kv, cap, D, slot) + kv_v_elem(slot, d, D)] = f32_to_bf16(row[q_dim + kv_dim + p]);
+  };
+  if constexpr (SHARED) {
+    // keys, then values, from the row's last workgroup backwards
+    for (int p = (gridDim.y - 1 - blockIdx.y) * 256 + threadIdx.x; p < n_kv * quads + kv_dim; p += step) {
+      if (p < n_kv * quads) store_key(p);
+      else store_value(p - n_kv * quads);
     }
+  } else {
+    for (int p = threadIdx.x; p < n_kv * quads; p += 256) store_key(p);
+    for (int p = threadIdx.x; p < kv_dim; p += 256) store_value(p);
   }
 }
 
@@ -411,7 +421,9 @@ int run_rope_store_lens(const float *qkv, float *q_out, bf16_t *kv, const float 
                         const float *sin_t, int B, int n_q, int n_kv, int D, int cap, const int *lens,
                         hipStream_t s, const int *seq_map) {
   TraceScope ts("rope_store", s);
-  rope_store_kernel<true><<<rope_grid(B, n_q, n_kv, D), 256, 0, s>>>(qkv, q_out, kv, cos_t, sin_t, n_q, n_kv, D, cap, 0, 1, 0, lens, seq_map);
+  const dim3 grid = rope_grid(B, n_q, n_kv, D);
+  (grid.y > 1 ? rope_store_kernel<true, true> : rope_store_kernel<true, false>)<<<grid, 256, 0, s>>>(
+      qkv, q_out, kv, cos_t, sin_t, n_q, n_kv, D, cap, 0, 1, 0, lens, seq_map);
   GPTOSS_LAUNCH_CHECK("rope_store_kernel");
   return GPTOSS_OK;
 }
@@ -420,12 +432,12 @@ int run_rope_store_rows(const float *qkv, float *q_out, bf16_t *kv, const float 
                         const float *sin_t, int rows, int T, int n_q, int n_kv, int D, int cap, int pos0,
                         int store_from, hipStream_t s) {
   TraceScope ts("rope_store", s);
-  if (T == 1)
-    rope_store_kernel<true><<<rope_grid(rows, n_q, n_kv, D), 256, 0, s>>>(qkv, q_out, kv, cos_t, sin_t, n_q, n_kv, D, cap, pos0, T, store_from,
-                                                 nullptr, nullptr);
-  else
-    rope_store_kernel<false><<<rope_grid(rows, n_q, n_kv, D), 256, 0, s>>>(qkv, q_out, kv, cos_t, sin_t, n_q, n_kv, D, cap, pos0, T, store_from,
-                                                  nullptr, nullptr);
+  const dim3 grid = rope_grid(rows, n_q, n_kv, D);
+  auto launch = [&](auto kernel) {
+    kernel<<<grid, 256, 0, s>>>(qkv, q_out, kv, cos_t, sin_t, n_q, n_kv, D, cap, pos0, T, store_from, nullptr, nullptr);
+  };
+  if (grid.y > 1) launch(T == 1 ? rope_store_kernel<true, true> : rope_store_kernel<false, true>);
+  else launch(T == 1 ? rope_store_kernel<true, false> : rope_store_kernel<false, false>);
   GPTOSS_LAUNCH_CHECK("rope_store_kernel");
   return GPTOSS_OK;
 }
