@@ -673,28 +673,25 @@ __global__ __launch_bounds__(256) void residual_tanh_norm_kernel(float *__restri
                                                                  int H) {
   const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (at >= part_stride) return;
-  // all that does not wait for another load at once
-  f32x4 v = *reinterpret_cast<const f32x4 *>(x + at), w, b;
-  if (norm.weight) {
-    const int h = (int)(at % (unsigned)H);
-    w = *reinterpret_cast<const f32x4 *>(norm.weight + h);
-    b = *reinterpret_cast<const f32x4 *>(norm.bias + h);
-  }
+  f32x4 v = *reinterpret_cast<const f32x4 *>(x + at);
   if (parts > 0) {
-    // sums in order of their index, four at a time
+    // sums in order of their index, four loads in flight at a time
     f32x4 own = *reinterpret_cast<const f32x4 *>(y + at);
-    for (int k = 1; k < parts; k += 4) {
+    int k = 1;
+    for (; k + 4 <= parts; k += 4) {
       f32x4 part[4];
 #pragma unroll
-      for (int q = 0; q < 4; q++) part[q] = *reinterpret_cast<const f32x4 *>(y + min(k + q, parts - 1) * part_stride + at);
+      for (int q = 0; q < 4; q++) part[q] = *reinterpret_cast<const f32x4 *>(y + (k + q) * part_stride + at);
 #pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (k + q < parts) own += part[q];
+      for (int q = 0; q < 4; q++) own += part[q];
     }
+    for (; k < parts; k++) own += *reinterpret_cast<const f32x4 *>(y + k * part_stride + at);
     v += own;
     *reinterpret_cast<f32x4 *>(x + at) = v;
   }
   if (!norm.weight) return;
+  const int h = (int)(at % (unsigned)H);
+  const f32x4 w = *reinterpret_cast<const f32x4 *>(norm.weight + h), b = *reinterpret_cast<const f32x4 *>(norm.bias + h);
   f32x4 o;
 #pragma unroll
   for (int q = 0; q < 4; q++) o[q] = fmaf(tanhf(norm.alpha * v[q]), w[q], b[q]);
