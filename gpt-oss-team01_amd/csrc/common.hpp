@@ -91,6 +91,14 @@ __device__ __forceinline__ void load_to_lds(unsigned lds, uint32_t voff, const v
                : "memory");
 }
 
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
+
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) {
   union {
     u32x4 u;

@@ -58,14 +58,6 @@ __device__ __forceinline__ u32x4 fp4_expand(uint32_t w, float scale) {
                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 3))};
 }
 
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
-}
-
 // Where one wave's W fragment stream of a work item starts (wave-uniform; each lane adds its own
 // 16 bytes, or 2 scale bytes, when loading).
 struct WStream {

@@ -590,63 +590,77 @@ __global__ __launch_bounds__(256) void depth_average_norm_kernel(float *__restri
   __shared__ double red[4];
   const size_t row = (size_t)blockIdx.x * H;
   // All that does not wait for another load is requested at once, for two of a thread's pieces together: a launch of few
-  // rows is as long as its loads that come one behind the other (four rows of 2048, up to 8 layers: 7.2 -> 6.1 us).  Pieces
-  // past the row's end read its last elements.
-  constexpr int G = VPT < 2 ? VPT : 2;
+  // rows is as long as its loads that come one behind the other.  As many loads as there are sums, addresses counted up: with
+  // four loads for any remainder and a product per address, 24 layers took longer than without any of this.  Four rows
+  // in the caches, (own sums, layers) before -> now (us): 2048 elements (1, 4) 3.4 -> 3.1, (4, 24) 5.3 -> 4.7; 4096, (2, 4) 5.0 ->
+  // 4.4, (2, 24) 7.8 -> 6.7; 1024, (2, 24) 3.4 -> 3.6; 8000 rows of 2048, (1, 4) 101 -> 95, (4, 24) 415 -> 401.  Lanes past the row's
+  // end read its last elements; a wave without any of a piece leaves it out.
+  const int first = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 256;   // of the wave's elements
+  const float *y_row = y + row, *old_row = history + row;
   f32x4 v[VPT], nw[VPT];
   double ss = 0.0;
-#pragma unroll
-  for (int i0 = 0; i0 < VPT; i0 += G) {
-    auto at = [&](int i) { return row + min((threadIdx.x + 256u * (i0 + i)) * 4, H - 4u); };
-    f32x4 own[G], before[G], old[4][G], a[G];
+  auto pieces = [&](auto i0_, auto n_) {
+    constexpr int I0 = decltype(i0_)::value, G = decltype(n_)::value;
+    unsigned at[G];
+    f32x4 own[G], before[G], old[4][G], part[4][G], a[G];
 #pragma unroll
     for (int i = 0; i < G; i++) {
-      own[i] = *reinterpret_cast<const f32x4 *>(y + at(i));
-      before[i] = *reinterpret_cast<const f32x4 *>(x + at(i));
-      if (norm_w) nw[i0 + i] = *reinterpret_cast<const f32x4 *>(norm_w + (at(i) - row));
+      at[i] = min((threadIdx.x + 256u * (I0 + i)) * 4, H - 4u);
+      own[i] = *reinterpret_cast<const f32x4 *>(y_row + at[i]);
+      before[i] = *reinterpret_cast<const f32x4 *>(x + row + at[i]);
+      if (norm_w) nw[I0 + i] = *reinterpret_cast<const f32x4 *>(norm_w + at[i]);
       a[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    auto load_old = [&](int j) {
+    auto request = [&](const float *p, size_t stride, f32x4 (&dst)[4][G]) {
 #pragma unroll
       for (int q = 0; q < 4; q++)
 #pragma unroll
-        for (int i = 0; i < G; i++) old[q][i] = *reinterpret_cast<const f32x4 *>(history + (size_t)min(j + q, layer) * plane + at(i));
+        for (int i = 0; i < G; i++) dst[q][i] = *reinterpret_cast<const f32x4 *>(p + q * stride + at[i]);
     };
-    load_old(0);
-    // sums in order of their index, four at a time
-    for (int k = 1; k < parts; k += 4) {
-      f32x4 part[4][G];
+    if (layer >= 3) request(old_row, plane, old);
+    // sums in order of their index, four loads in flight at a time
+    int k = 1, j = 0;
+    const float *p = y_row + part_stride;
+    for (; k + 4 <= parts; k += 4, p += 4 * part_stride) {
+      request(p, part_stride, part);
 #pragma unroll
       for (int q = 0; q < 4; q++)
 #pragma unroll
-        for (int i = 0; i < G; i++) part[q][i] = *reinterpret_cast<const f32x4 *>(y + min(k + q, parts - 1) * part_stride + at(i));
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (k + q < parts)
-#pragma unroll
-          for (int i = 0; i < G; i++) own[i] += part[q][i];
+        for (int i = 0; i < G; i++) own[i] += part[q][i];
     }
+    for (; k < parts; k++, p += part_stride)
+#pragma unroll
+      for (int i = 0; i < G; i++) own[i] += *reinterpret_cast<const f32x4 *>(p + at[i]);
 #pragma unroll
     for (int i = 0; i < G; i++) own[i] += before[i];
-    for (int j = 0; j <= layer; j += 4) {
-      if (j > 0) load_old(j);
+    p = old_row;
+    for (; j + 4 <= layer + 1; j += 4, p += 4 * plane) {
+      if (j > 0) request(p, plane, old);
 #pragma unroll
       for (int q = 0; q < 4; q++)
-        if (j + q <= layer)
 #pragma unroll
-          for (int i = 0; i < G; i++) a[i] += weights[j + q] * old[q][i];
+        for (int i = 0; i < G; i++) a[i] += weights[j + q] * old[q][i];
     }
+    for (; j <= layer; j++, p += plane)
+#pragma unroll
+      for (int i = 0; i < G; i++) a[i] += weights[j] * *reinterpret_cast<const f32x4 *>(p + at[i]);
 #pragma unroll
     for (int i = 0; i < G; i++) {
-      v[i0 + i] = a[i] + weights[layer + 1] * own[i];
-      if ((threadIdx.x + 256 * (i0 + i)) * 4 < H) {
-        *reinterpret_cast<f32x4 *>(history + (size_t)(layer + 1) * plane + at(i)) = own[i];
-        *reinterpret_cast<f32x4 *>(x + at(i)) = v[i0 + i];
+      v[I0 + i] = a[i] + weights[layer + 1] * own[i];
+      if ((threadIdx.x + 256 * (I0 + i)) * 4 < H) {
+        *reinterpret_cast<f32x4 *>(history + (size_t)(layer + 1) * plane + row + at[i]) = own[i];
+        *reinterpret_cast<f32x4 *>(x + row + at[i]) = v[I0 + i];
 #pragma unroll
-        for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[i0 + i][q], v[i0 + i][q]);
+        for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[I0 + i][q], v[I0 + i][q]);
       }
     }
-  }
+  };
+  static_for<0, (VPT + 1) / 2>([&](auto g) {
+    constexpr int I0 = 2 * decltype(g)::value;
+    using I = std::integral_constant<int, I0>;
+    if (I0 + 1 < VPT && first + 1024 * (I0 + 1) < H) pieces(I{}, std::integral_constant<int, I0 + 1 < VPT ? 2 : 1>{});
+    else if (first + 1024 * I0 < H) pieces(I{}, std::integral_constant<int, 1>{});
+  });
   if (!norm_w) return;
   ss = lanes_sum(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
