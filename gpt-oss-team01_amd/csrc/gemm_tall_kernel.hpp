@@ -78,6 +78,25 @@ __device__ __forceinline__ void tall_load(unsigned lds, uint32_t voff, tall_rsrc
                : "memory", "scc");
 }
 
+// The token of a pair: id / top_k by a multiplication.  inv = 2^32 / k rounded up (k = 1: 0) is off by e / k with e = inv k -
+// 2^32 < k, which adds id e / (k 2^32) to the quotient: less than the 1 / k that can be missing to the next whole number while
+// id e < 2^32.  A call has fewer than 2^31 / 64 pairs (a row has at least 64 elements) and k <= MOE_MAX_TOP.
+__host__ __device__ constexpr uint32_t pair_inverse(uint32_t k) { return 0xffffffffu / k + 1u; }
+__host__ __device__ constexpr uint32_t pair_token(uint32_t id, uint32_t inv) { return inv ? (uint32_t)((uint64_t)id * inv >> 32) : id; }
+constexpr bool pair_tokens_exact() {
+  constexpr uint64_t pairs = (1ull << 31) / 64;
+  for (uint32_t k = 1; k <= MOE_MAX_TOP; k++) {
+    const uint32_t inv = pair_inverse(k);
+    if (k > 1 && (pairs - 1) * ((uint64_t)inv * k - (1ull << 32)) >= 1ull << 32) return false;
+    for (uint64_t id = k; id < pairs; id *= 2) {
+      const uint32_t m = (uint32_t)(id / k * k);
+      if (pair_token(m, inv) != m / k || pair_token(m - 1, inv) != (m - 1) / k || pair_token(m + k - 1, inv) != m / k) return false;
+    }
+  }
+  return true;
+}
+static_assert(pair_tokens_exact(), "a pair's token by multiplication");
+
 // where one work item's operands come from, for this wave's share of the loads
 template <class SH>
 struct TallSrc {
@@ -270,9 +289,9 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
   // hand-counted waits does not see.
   // Eight ids are one scalar load, four of which are requested together: id by id, with a wait for each group of rows, an
   // item began with 3.6 us of its 87 (block of 4500 tokens 1081 -> 1073 us, of 5999 1260 -> 1254).  A tile of fewer than
-  // eight rows reads on behind them, into what follows in the workspace, and does not use it.  id / top_k is a
-  // multiplication, exact for ids below 2^32 / top_k^2 (they stay below 2^31 / 64, top_k at most 32).
-  const uint32_t inv_k = 0xffffffffu / (uint32_t)p.top_k + 1u;   // 2^32 / top_k rounded up; 1: 0
+  // eight rows reads on behind them, into what follows in the workspace, and does not use it.
+  uint32_t inv_k = 0;
+  if constexpr (GATHER) inv_k = pair_inverse(p.top_k);
   auto a_offsets = [&](TallSrc<SH> &t) {
     typedef int ids_t __attribute__((ext_vector_type(8), aligned(4)));
     const int last = t.rows - 1, group = lane >> 3;
@@ -298,7 +317,7 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
           int src = v[q][0];
 #pragma unroll
           for (int i = 1; i < 8; i++) src = j == i ? v[q][i] : src;
-          t.a[q0 + q] = offset(inv_k ? (int)__umulhi((uint32_t)src, inv_k) : src, r);
+          t.a[q0 + q] = offset((int)pair_token(src, inv_k), r);
         }
       }
     } else {
