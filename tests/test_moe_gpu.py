@@ -458,6 +458,9 @@ def test_grouping_of_a_few_tokens_by_one_wave(ops, E, k):
         for have, want in zip(got[:3] + [got[3][:1 + 3 * n_tiles]], (off, srt, inv, tiles[:1 + 3 * n_tiles])):
             assert torch.equal(have, want), tokens
         assert bounds[0] == 0 and bounds[8] == n_tiles << 16 and bool((bounds[:9].diff() >= 0).all())
+        if tokens <= 16:   # one wave: eight parts of equal length, every tile a block of its own (first tile << 8 | height)
+            assert bounds[:9].tolist() == [(x * n_tiles) << 13 for x in range(9)]
+            assert bounds[16:16 + n_tiles].tolist() == [t << 8 | 1 for t in range(n_tiles)]
 
 
 def _prompt_pass_equals_small_batches(ops, g, router, b_router, t, k):

@@ -33,9 +33,10 @@ def _forward_norm(layer, x, residual, weight, out, next_weight=None, next_t=None
     return t
 
 
-# H: a part of a thread's first chunk, three chunks short of the end, four whole chunks; E: one column block, two, eight, nine
+# H: a part of a thread's first chunk, three chunks short of the end, four whole chunks; E: one column block, two, four, eight,
+# sixteen of the kernel's instances
 @pytest.mark.parametrize("H", [64, 2880, 4096])
-@pytest.mark.parametrize("E", [4, 32, 128, 129])
+@pytest.mark.parametrize("E", [4, 32, 33, 64, 128, 129])
 @pytest.mark.parametrize("with_residual", [False, True])
 def test_a_block_with_its_norm_equals_its_parts(ops, H, E, with_residual):
     g = torch.Generator(device="cuda").manual_seed(H + E)
@@ -43,10 +44,12 @@ def test_a_block_with_its_norm_equals_its_parts(ops, H, E, with_residual):
     n = lambda *s, **k: rnd(*s, **k).bfloat16()
     I = 64
     layer = ops.MoeLayer(n(E, H, std=H ** -0.5), n(E), n(E, 2 * I, H, std=0.05), n(E, 2 * I), n(E, H, I, std=0.05), n(E, H),
-                         top_k=4, max_tokens=301)
+                         top_k=4, max_tokens=601)
     weight = 1 + rnd(H, std=0.1)
-    # 1, 2, 3, 4 rows: one workgroup groups them; 5, 16, 17: several, and a launch that sorts; 301: a last one of one row
-    for B in (1, 2, 3, 4, 5, 16, 17, 301):
+    # 1, 2, 3, 4 rows: one workgroup groups them; 5, 16, 17: several, and a launch that sorts; 301: a last one of one row.  33 and
+    # more experts of H = 2880 and 4096 are shared out among workgroups, behind a norm of its own, up to 512 rows; from 513
+    # on, and at H = 64 always, the norm runs in the router's kernel for them too, with four rows per workgroup
+    for B in (1, 2, 3, 4, 5, 16, 17, 301, 513, 601):
         x, residual = rnd(B, H) * 3, rnd(B, H) if with_residual else None
         x_want, out = x.clone(), rnd(B, H)
         out_want = out.clone()
