@@ -791,13 +791,14 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
   }
 }
 // The launches that take it: where every row is as long as the longest may be, up to 512 (row, kv head, chunk) items, two
-// per CU; 384 with heads of 32 values; 256 of rows that cannot fill half a chunk (it requests eight blocks whatever a row
-// has).  64 heads of 64 on 8 kv heads, full rows, caches cold, a wave per item -> this kernel (us): 4 of 8000 positions
-// (512 items) 29.0 -> 25.4, 32 of 1000 29.6 -> 25.4, 63 of 448 22.7 -> 18.9; 40 of 128 (320) 12.1 -> 12.1.  Beyond that a
-// wave per item fills the chip as well and follows HBM better: 5 of 8000 (640 items) 29.8 -> 29.7, 16 of 3000 (768) 30.5 ->
-// 32.6, 8 of 8000 (1024) 33.4 -> 37.5, 48 of 4000 (3072) 74.5 -> 85.1, 96 of 300 20.2 -> 23.2, and 1000 rows of a prompt
-// over 8 kv heads 141 -> 196.  (Rows of very different length are another matter: 63 of 500 to 4000 79 -> 70.  The host
-// does not know the lengths.)
+// per CU; 384 with heads of 32 values; 256 of rows that cannot fill half a chunk.  64 heads of 64 on 8 kv heads, full rows, caches
+// cold, a wave per item -> this kernel (us): 4 of 8000 positions (512 items) 29.0 -> 25.4, 32 of 1000 29.6 -> 25.4, 63 of 448
+// 22.7 -> 18.9.  Beyond that a wave per item fills the chip as well and follows HBM better: 5 of 8000 (640 items) 29.8 -> 29.7,
+// 16 of 3000 (768) 30.5 -> 32.6, 8 of 8000 (1024) 33.4 -> 37.5, 48 of 4000 (3072) 74.5 -> 85.1, 96 of 300 20.2 -> 23.2, and 1000
+// rows of a prompt over 8 kv heads 141 -> 196.  (Rows of very different length are another matter: 63 of 500 to 4000 79 -> 70.
+// The host does not know the lengths.)  The 256 date from when this kernel requested eight blocks whatever a row has; since it
+// requests the row's own, 512 would do for short rows as well: 40 of 100 (320 items) 9.1 -> 7.2, 63 of 40 / 255 (504) 7.2 / 13.5 ->
+// 6.3 / 9.9, with heads of 32 values 63 of 40 / 100 / 200 5.1 / 6.3 / 8.2 -> 5.5 / 6.1 / 7.7.
 static bool attn_few(long long pairs, int span, int head_dim) {
   const long long items = pairs * ((span + ATT_CHUNK - 1) / ATT_CHUNK);
   return items <= (span * head_dim < 256 * 64 ? 256 : head_dim == 32 ? 384 : 512);
@@ -820,7 +821,9 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   f32x2 ml[U];
   f32x4 o[U];
-  const SeqRange r = seq_range(row_len(p, b), p.cap, p.window, p.max_len);
+  const int len = row_len(p, b);
+  const float sink = p.sinks ? p.sinks[hq] : -INFINITY;   // with the length (behind the partials: 3 rows of 8000 15.8 -> 16.1 us)
+  const SeqRange r = seq_range(len, p.cap, p.window, p.max_len);
   if (r.nchunks <= 1) return;  // already finished by the first kernel
   auto load = [&](int c0) {
 #pragma unroll
@@ -831,7 +834,7 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
     }
   };
   load(0);
-  const float sink2 = p.sinks ? p.sinks[hq] * 1.4426950408889634f : -INFINITY;
+  const float sink2 = p.sinks ? sink * 1.4426950408889634f : -INFINITY;
   float M = NEG_BIG;
 #pragma unroll
   for (int u = 0; u < U; u++) M = u < r.nchunks ? fmaxf(M, ml[u][0]) : M;
@@ -872,7 +875,7 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 // and walks the K/V blocks any of them needs ONCE: every block goes from global memory into LDS
 // (two buffers, one barrier per block) and the eight waves take their operands from there.  The
 // pair form reads a sequence's cache once per row pair, which is quadratic traffic for long
-// prompts; here it is read once per 16 rows.  What bounds it is the vector units (70 % busy, the matrix cores 34 %): per
+// prompts; here it is read once per 16 rows.  What bounds it is the vector units (68 % busy, the matrix cores 36 %): per
 // 64 x 16 scores a wave issues about 170 of their instructions, a tenth of them exponentials.  Eight prompts of 1000
 // positions, 64 heads: 237 -> 211 us with the exponential, the maximum and the splitting of weights in fewer instructions
 // (exp2_hw, max_over_quarters, split_weights), -> 195 with the scale fused into the exponent's difference

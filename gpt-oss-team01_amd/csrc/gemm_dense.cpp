@@ -89,8 +89,9 @@ static int gemm_prepare_device() {
 // rounds: 5 % on top, as what they gain at a tie is less than what they lose).  With one fixed part per launch, products of
 // short K or narrow N took up to 37 % longer than on streaming kernels alone (us: 1280 x 1280 with its K cut, 257 rows
 // 11.1 instead of 8.1; 2048 x 256, 257 rows 8.0 instead of 6.3).
-// (Few-row tiles of up to 16 rows have become up to a third faster since, gemm_few_kernel.hpp; the estimates leave that out, and
-// err towards the streaming kernels and more parts there.)
+// The few-row kernels have become faster since, tiles of up to 16 rows by up to a third (gemm_few_kernel.hpp), which the fit leaves
+// out: uncut products of up to 8 / 16 rows take 0.79 / 0.85 of few_us' time, where the streaming kernels take 1.12 of streaming_us', so
+// these and more parts look better there than they are.  What that costs is stated at the two rules that use it.
 static double streaming_us(int mb, long long blocks, int slabs) {
   // [mb - 1]: launch; per round, and per slab of it; per full round's items, and per slab of them
   static const double t[5][5] = {{3.2, 0.63, 0.496, 1.8, 0.028}, {3.5, 1.35, 0.533, 3.3, 0.106}, {4.0, 2.5, 0.578, 3.8, 0.145},
@@ -156,8 +157,10 @@ static int argmax_tall_min_rows() {
 }
 
 // Row tile of a dense GEMM below the 256-row kernels: the one with the least estimated time; ties go to the larger tile
-// (fewer re-reads of the weights).  Timed with every tile at the 918 sizes above: 1 % slower than the best one on average
-// and 16 % faster than the streaming kernels alone (5120 x 2880, 97 / 200 / 364 rows 32 / 32 / 33 -> 19 / 21 / 22 us).  The estimates leave
+// (fewer re-reads of the weights).  Timed with every tile at the 918 sizes above, with the kernels that the estimates were fitted to:
+// 1 % slower than the best one on average and 16 % faster than the streaming kernels alone (5120 x 2880, 97 / 200 / 364 rows 32 / 32 /
+// 33 -> 19 / 21 / 22 us).  With the present ones, 53 shapes of 512-16384 columns and K 256-8192, 1 to 32 rows: less than 1 % slower than the
+// better of both kernels, which is the few-row one at all of them.  The estimates leave
 // out what a second row tile costs in reads of the weights, so from 65 column tiles on up to 128 rows are one tile:
 // 24576 x 2880, 65 / 128 rows 65 / 69 us with tiles of 64, 46 / 54 with one.  Hundreds of column tiles (an unembedding) fill
 // the chip at any size: one tile up to 96 rows, then 128, measured best at 1024.
@@ -232,8 +235,10 @@ int dense_gemm_mixed(const bf16_t *A, const bf16_t *W, float *out, const GemmBf1
 }
 
 // Few rows and few columns leave most CUs without a work item while those that have one walk all of K.
-// Cutting K makes more items; what it costs is a part per round and the reading of the partial sums.  All row tiles and parts timed at the 312 sizes above: the chosen ones take 2 % longer than the best ones on average
-// and are 15 % faster than with streaming kernels alone (2048 x 2048, 8 / 400 / 1024 rows 7.0 / 14.6 / 21.8 -> 4.7 / 11.5 / 17.5 us).
+// Cutting K makes more items; what it costs is a part per round and the reading of the partial sums.  All row tiles and parts timed at the 312 sizes above, with the kernels that the estimates were fitted to:
+// the chosen ones take 2 % longer than the best ones on average and are 15 % faster than with streaming kernels alone (2048 x 2048,
+// 8 / 400 / 1024 rows 7.0 / 14.6 / 21.8 -> 4.7 / 11.5 / 17.5 us).  With the present ones, 53 shapes, up to 8 / 16 / 32 rows: 9 / 8 / 6 % longer, as
+// fewer parts would do (8192 x 1024, 8 rows 7.2 us in four parts, 5.4 uncut; 2048 x 4096 7.2 in sixteen, 5.6 in four).
 int dense_gemm_partial(const bf16_t *A, const bf16_t *W, float *out, size_t max_elems, int *parts, int B, int N, int K,
                        hipStream_t s) {
   *parts = 1;
