@@ -208,3 +208,76 @@ def test_rotation_of_few_rows_equals_that_of_many(ops, D, n_q, n_kv):
     for rows in (1, 2, 25, 26, 42, 43, 64, 65, 128, 129):
         q_few, kv_few = rotate(rows)
         assert torch.equal(q_few.view(rows, -1), q[:rows].view(rows, -1)) and torch.equal(kv_few, kv[:rows]), rows
+
+
+def _internal(name, argtypes):
+    """A function of namespace gptoss without a C entry point, by its linker name."""
+    import ctypes as C
+    from conftest import load_pkg
+    lib = load_pkg("lib")
+    f = getattr(lib.load(), name)
+    f.restype, f.argtypes = C.c_int, argtypes
+    return lambda *a: lib.check(f(*a, torch.cuda.current_stream().cuda_stream))
+
+
+# H: one 16-byte piece, part of a wave, one wave short of / just past a piece of 256 threads, an odd number of pieces, the last
+# instance; sums: one, a group of four behind it and one more, ...
+@pytest.mark.parametrize("H", [4, 64, 252, 1020, 1024, 1028, 2044, 2052, 2880, 4096, 4100, 8192, 8196, 16384])
+@pytest.mark.parametrize("parts,layer", [(1, 0), (2, 2), (5, 3), (6, 4), (16, 8)])
+def test_depth_average_and_norm(ops, H, parts, layer):
+    import ctypes as C
+    P, I = C.c_void_p, C.c_int
+    run = _internal("_ZN6gptoss22run_depth_average_normEPfPKfiS0_mS2_iS2_PtS0_iifiP12ihipStream_t",
+                    [P, P, I, P, C.c_size_t, P, I, P, P, P, I, I, C.c_float, I, P])
+    g = torch.Generator(device="cuda").manual_seed(H + parts)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    rows, plane = 3, 5 * H
+    x, y, w = rnd(rows, H), rnd(parts, rows, H), rnd(H)
+    history, weights = rnd(layer + 3, 5, H), rnd(layer + 2)
+    before, own = history.clone(), x.double() + y.double().sum(0)
+    size = x.double().abs() + y.double().abs().sum(0)
+    t16, t32 = torch.empty(rows, H, device="cuda", dtype=torch.bfloat16), torch.empty(rows, H, device="cuda")
+    run(x.data_ptr(), y.data_ptr(), parts, history.data_ptr(), plane, weights.data_ptr(), layer, w.data_ptr(), t16.data_ptr(),
+        t32.data_ptr(), rows, H, 1e-5, H)
+    # a sum of n fp32 terms: each of up to n roundings is at most 2^-24 of the sum of their sizes
+    assert bool(((history[layer + 1, :rows].double() - own).abs() <= size * (parts + 1) * 2.0 ** -24).all())
+    terms = weights[:layer + 1, None, None].double() * before[:layer + 1, :rows].double()
+    want = terms.sum(0) + weights[layer + 1].double() * own
+    bound = (terms.abs().sum(0) + weights[layer + 1].double().abs() * size) * (layer + parts + 4) * 2.0 ** -24
+    assert bool(((x.double() - want).abs() <= bound).all())
+    scale = w.double() / torch.sqrt((x.double() ** 2).mean(-1, keepdim=True) + 1e-5)
+    # squares, their root and its reciprocal in fp32, one more rounding: 2^-21 of the result; bf16: 2^-8
+    assert bool(((t32.double() - x.double() * scale).abs() <= (x.double() * scale).abs() * 2.0 ** -21 + 1e-30).all())
+    assert torch.equal(t16, t32.bfloat16())
+    history[layer + 1, :rows] = before[layer + 1, :rows]
+    assert torch.equal(history, before)      # nothing else is written
+
+
+# bf16 rows from 1024 elements on and fp32 rows from 512 on go 16 bytes at a time, if whole and aligned
+@pytest.mark.parametrize("dtype,H,ld", [("bf16", 1016, 1016), ("bf16", 1024, 1024), ("bf16", 1020, 1024), ("bf16", 1024, 1028), ("bf16", 2048, 2112),
+                                        ("bf16", 64, 1024), ("f32", 508, 508), ("f32", 512, 512), ("f32", 510, 512), ("f32", 1028, 1088)])
+@pytest.mark.parametrize("with_positions", [False, True])
+def test_embedding_rows(ops, dtype, H, ld, with_positions):
+    import ctypes as C
+    name = {"bf16": "_ZN6gptoss22run_embedding_positionEPKtS1_PKiS3_PfS4_iiiiiP12ihipStream_t",
+            "f32": "_ZN6gptoss26run_embedding_position_f32EPKfS1_PKiS3_PfS4_iiiiiP12ihipStream_t"}[dtype]
+    run = _internal(name, [C.c_void_p] * 6 + [C.c_int] * 5 + [C.c_void_p])
+    g = torch.Generator(device="cuda").manual_seed(H)
+    cast = (lambda v: v.bfloat16()) if dtype == "bf16" else (lambda v: v)
+    V, n_pos, rows = 37, 11, 5
+    flat = cast(torch.randn(V * H + 1, generator=g, device="cuda"))
+    positions = cast(torch.randn(n_pos, H, generator=g, device="cuda"))
+    tokens = torch.tensor([0, V - 1, 5, V + 3, -1], dtype=torch.int32, device="cuda")   # outside: clamped
+    lens = torch.tensor([1, n_pos, n_pos + 4, 3, 0], dtype=torch.int32, device="cuda")
+    for shift in (0, 1):   # a table that no wide load may touch
+        table = flat[shift:shift + V * H].view(V, H)
+        x = torch.full((rows, ld), 7.0, device="cuda")
+        x0 = torch.full_like(x, 7.0)
+        run(table.data_ptr(), positions.data_ptr() if with_positions else None, tokens.data_ptr(), lens.data_ptr(), x.data_ptr(),
+            x0.data_ptr() if with_positions else None, rows, H, ld, V, n_pos)
+        want = torch.zeros(rows, ld, device="cuda")
+        want[:, :H] = table[tokens.long().clamp(0, V - 1)].float()
+        if with_positions:
+            want[:, :H] += positions[(lens.long() - 1).clamp(0, n_pos - 1)].float()
+            assert torch.equal(x0, want)
+        assert torch.equal(x, want), shift
