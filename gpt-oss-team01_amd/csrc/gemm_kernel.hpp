@@ -15,7 +15,7 @@
 //   * a workgroup = 8 waves = 256 columns x up to 160 rows, each wave keeping at most 80
 //     accumulator registers, so two waves share a SIMD: one wave's MFMAs, epilogue or prologue
 //     overlap the other's waits on memory;
-//   * the kernel is persistent (one workgroup per CU, two for the small-tile MXFP4 kernels); its
+//   * the kernel is persistent (one workgroup per CU, two with MXFP4 weights); its
 //     work items come from the device-built tile list (expert,row0,rows), mapped so that the workgroups of one XCD walk consecutive
 //     column tiles of the same expert (A stays in that XCD's L2), and the register ring of W keeps
 //     streaming across work items;
@@ -524,21 +524,12 @@ __device__ __forceinline__ void gemm_tile(const GemmParams &p, bf16_t *lds, int 
 // behind the A stages of one workgroup per CU (156 KB at 160 rows).
 constexpr bool gemm_holds_output(bool gather, int epi, bool fp4) { return gather && epi == EPI_SWIGLU && !fp4; }
 
-// NRING: slabs of W held in registers per wave, NRING-1 of them in flight.  Three everywhere
-// except the 64-row MXFP4 kernels, where a slab costs 5 registers and two more ring slots fit under
-// the 128 registers of two workgroups per CU: four slabs in flight measured 4-10 % faster there
-// (1024 tokens on 32 experts: 192 + 110 -> 178 + 104 us), nothing or worse for the other tile sizes.
+// NRING: slabs of W held in registers per wave, NRING-1 of them in flight.  Three, except with MXFP4 weights (tiles of up to
+// 64 rows, in launches of at most an item per CU; gemm_mxfp4.hip), where a slab costs 5 registers and two more ring slots fit
+// under the 128 registers that leave room for a second workgroup.
 constexpr int GEMM_NRING = 3;
-constexpr int gemm_nring(int mbmax, bool fp4) { return (fp4 && mbmax == 2) ? 5 : GEMM_NRING; }
-
-// MXFP4 kernels for tiles of up to 96 rows are compiled for 128 registers, so that two workgroups
-// (four waves per SIMD) share a CU: with a quarter of the weight bytes per MFMA the kernel is no
-// longer bound by the W stream but by everything around the MFMAs (load latency, LDS round trips,
-// prologues and epilogues), and a second workgroup fills those gaps better than larger tiles do
-// (64-row tiles on 16 waves: -6 % on a 4096-token layer of 128 experts, -9 % / -14 % on GEMM1 /
-// GEMM2 of a 1024-token layer of 32 experts against 160-row tiles on 8 waves).  With bf16 weights
-// the same change measured nothing: those kernels follow the W stream.
-constexpr bool gemm_two_per_cu(int mbmax, bool fp4) { return fp4 && mbmax <= 3; }
+constexpr int gemm_nring(bool fp4) { return fp4 ? 5 : GEMM_NRING; }
+constexpr bool gemm_two_per_cu(bool fp4) { return fp4; }
 
 // Persistent kernel: the grid is one workgroup of 8 waves per CU; workgroups are dealt round-robin
 // to the 8 XCDs, XCD x owns the x-th contiguous part of the work list (consecutive column tiles
@@ -547,9 +538,9 @@ constexpr bool gemm_two_per_cu(int mbmax, bool fp4) { return fp4 && mbmax <= 3; 
 // or, when the grouping kernel supplied cut positions, equal estimated cost (experts with many
 // rows next to experts with few would otherwise leave some XCDs idle early).
 template <int MBMAX, bool GATHER, int EPI, bool FP4>
-__global__ __launch_bounds__(GEMM_THREADS, (gemm_two_per_cu(MBMAX, FP4) ? 4 : 2)) void grouped_gemm_kernel(GemmParams p) {
+__global__ __launch_bounds__(GEMM_THREADS, (gemm_two_per_cu(FP4) ? 4 : 2)) void grouped_gemm_kernel(GemmParams p) {
   constexpr int BM = MBMAX * 32;
-  constexpr int NRING = gemm_nring(MBMAX, FP4);
+  constexpr int NRING = gemm_nring(FP4);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   bf16_t *lds = reinterpret_cast<bf16_t *>(smem_raw);  // [3][BM][LDS_ROW], then [2][BM][HOLD_ROW] where outputs are held
   const int lane = threadIdx.x & 63;
@@ -733,7 +724,7 @@ int launch_gemm(const GemmParams &p, int max_tiles, hipStream_t s) {
   int total = max_tiles * p.n_col_tiles * (EPI == EPI_PARTIAL ? p.k_splits : 1);
   int grid = ((total + 7) / 8) * 8;
   // resident workgroups: one of 8 waves (2 per SIMD) per CU, or two where the registers allow
-  const int resident = gemm_two_per_cu(MBMAX, FP4) ? 512 : 256;
+  const int resident = gemm_two_per_cu(FP4) ? 512 : 256;
   if (grid > resident) grid = resident;
   if (grid == 0) return GPTOSS_OK;
   {

@@ -48,12 +48,9 @@ static MoeWorkspace carve(void *base, int B, int E, int k, int H, int I) {
 // bf16 weights (32, 64, 128 or 160 rows): the smallest tile that holds an average expert's rows
 // plus 2.5 standard deviations of a uniform routing, so that nearly every expert is a single tile
 // and its weights are streamed exactly once; the kernel is bound by that stream.
-// MXFP4 weights (32 or 64 rows): tiles of at most 64 rows, whose kernels run two workgroups per
-// CU within 128 registers; an expert's few row tiles are walked column tile by column tile
-// (tile_block), so its weights still come from HBM once.  The 96-row kernel does not fit that
-// budget (it spills 12-97 registers, and every reload in its slab loop waits for the loads in
-// flight): 384 / 512 tokens on 32 experts, where 96 rows would hold a whole expert, GEMM1 108 /
-// 119 us and GEMM2 141 / 150 us with it against 91 / 115 and 56 / 78 us with 64-row tiles.
+// MXFP4 weights (32 or 64 rows): tiles of at most 64 rows, three or four workgroups of which share a CU
+// (gemm_mxfp4_kernel.hpp); an expert's few row tiles are walked column tile by column tile
+// (tile_block), so its weights still come from HBM once.
 static int env_int(const char *name, int dflt) {
   const char *e = getenv(name);
   const int n = e ? atoi(e) : 0;

@@ -98,3 +98,24 @@ def test_mxfp4_every_code_and_scale_expands_exactly(ops, orc):
                      torch.from_numpy(w2d).to(torch.bfloat16).cuda(), z2.cuda(), top_k=1, max_tokens=B)
     assert torch.equal(a.forward(t.cuda()), b.forward(t.cuda()))
     assert fp4_w2.numel() == H * I // 2 + H * I // 32 and bf_w2.numel() == H * I
+
+
+# Launches of more work items than CUs, first in either product: 513 items (three workgroups a CU) of one slab, 3248 (four)
+# of two and three slabs, columns that fill a quarter of the last tile, tiles of 1 to 64 rows, experts without any.
+@pytest.mark.parametrize("B,E,H,I,skew", [(700, 128, 64, 320, False), (700, 128, 640, 64, True), (1200, 128, 128, 2048, True),
+                                          (1200, 128, 4096, 192, False), (2000, 32, 576, 448, True)])
+def test_many_tiles_have_the_bits_of_the_bf16_path(ops, orc, B, E, H, I, skew):
+    rng = np.random.default_rng(B + H)
+    w1b, w1s = _rand_mxfp4(rng, E, 2 * I, H)
+    w2b, w2s = _rand_mxfp4(rng, E, H, I)
+    bf = lambda x: torch.from_numpy(x).to(torch.bfloat16).cuda()
+    t, wr = bf(rng.standard_normal((B, H)) * 0.05), bf(rng.standard_normal((E, H)) * 0.02)
+    br = torch.from_numpy(-1.1 * np.log(rng.permutation(E) + 1.0) if skew else np.zeros(E)).float().cuda()
+    b1, b2 = bf(rng.standard_normal((E, 2 * I)) * 0.02), bf(rng.standard_normal((E, H)) * 0.02)
+    cuda = lambda x: torch.from_numpy(x).cuda()
+    fp4 = ops.MoeLayerMxfp4(wr, br, cuda(w1b), cuda(w1s), b1, cuda(w2b), cuda(w2s), b2, max_tokens=B)
+    ref = ops.MoeLayer(wr, br, bf(_dequant(orc, w1b, w1s)), b1, bf(_dequant(orc, w2b, w2s)), b2, max_tokens=B)
+    for n in (B, B - 1):
+        assert torch.equal(fp4.forward(t[:n]), ref.forward(t[:n]))
+    counts = np.diff(fp4.routing_views()[3].cpu().numpy())
+    assert not skew or E < 128 or counts.min() <= 1
