@@ -135,14 +135,34 @@ int run_gemm_dense(const GemmParams &p, int epi, int rows_per_tile, int max_tile
   return fail(GPTOSS_ERR_DIM, "run_gemm: unsupported combination (dense, epi=%d)", epi);
 }
 
-// rows from which a dense fp32-output GEMM uses the 256-row kernel of gemm_tall.hip
+// The same for the 256-row kernel (gemm_tall_kernel.hpp): rounds of 32 tiles per XCD, the last one in halves of a tile where
+// they leave half of its workgroups idle.  A CU's slab takes longer the more CUs multiply (the chip is at its power limit).
+// Within 6 % of 63 products: 9 shapes of 1024-24576 columns and K 512-10240 at 7 row counts of 2048-8000, at fewer rows within 8 %.
+static double tall_us(int B, int N, int K) {
+  const int mine = (cdiv(B, 256) * cdiv(N, 256) + 7) / 8, rest = mine % 32, slabs = K / 64;
+  double us = 4.0 + mine / 32 * (11.5 + 1.44 * slabs);
+  if (rest && 2 * rest <= 32) us += 9.0 + (0.39 + 0.45 * rest / 16.0) * slabs;
+  else if (rest) us += 11.5 + (0.54 + 0.9 * rest / 32.0) * slabs;
+  return us;
+}
+
+// GPTOSS_DENSE_TALL_MIN_ROWS: rows from which a dense fp32-output GEMM uses the 256-row kernel, in place of the estimates
 static int dense_tall_min_rows() {
   static const int v = [] {
     const char *e = getenv("GPTOSS_DENSE_TALL_MIN_ROWS");
-    const int n = e ? atoi(e) : 0;
-    return n > 0 ? n : 2048;
+    return e ? atoi(e) : 0;
   }();
   return v;
+}
+
+// Whether a dense product is one for the 256-row kernel, given the best estimate of the others, which is up to a fifth too high
+// for products of a thousand rows: below 2048 rows the 256-row kernel has to be clearly ahead, above clearly behind.  Timed with
+// both at 792 products (10 shapes of 512-65536 columns, K 256-10240, 256-8000 rows): 6 % faster on average than 256-row tiles from
+// 2048 rows on, nothing more than 5 % slower (8192 x 2048, 2047 rows 86 -> 62 us, 16640 x 2048, 1500 rows 123 -> 106; 1024 x
+// 10240, 4100 rows 118 -> 105; missed by the estimates: 65536 x 1024, 600 rows, 124 instead of 101).
+static bool dense_tall(int B, int N, int K, double other_us) {
+  if (dense_tall_min_rows() > 0) return B >= dense_tall_min_rows();
+  return tall_us(B, N, K) < (B < 2048 ? 0.88 : 1.1) * other_us;
 }
 
 // rows from which the classifier's arg-max GEMM uses it (measured, vocabulary 201088 x 2880: 256 rows
@@ -164,24 +184,27 @@ static int argmax_tall_min_rows() {
 // out what a second row tile costs in reads of the weights, so from 65 column tiles on up to 128 rows are one tile:
 // 24576 x 2880, 65 / 128 rows 65 / 69 us with tiles of 64, 46 / 54 with one.  Hundreds of column tiles (an unembedding) fill
 // the chip at any size: one tile up to 96 rows, then 128, measured best at 1024.
-static int dense_rows_per_tile(int B, int n_col_tiles, int N, int K, int epi) {
-  if (B >= 2048) return 160;
+static int dense_rows_per_tile(int B, int n_col_tiles, int N, int K, int epi, double *us) {
+  auto estimate = [&](int mb) {
+    const int tiles = cdiv(B, 32 * mb);
+    return epi != EPI_ARGMAX && dense_few(32 * mb, tiles, N, K) ? few_us(mb, (long long)tiles * (N / 32), K / 64)
+                                                                : streaming_us(mb, (long long)tiles * n_col_tiles * 8, K / 64);
+  };
   if (n_col_tiles >= 128 || epi == EPI_ARGMAX || (n_col_tiles > 64 && B <= 128)) {
-    if (B <= 96) return align_up(B, 32);
-    if (n_col_tiles >= 64) return 128;
+    const int rpt = B <= 96 ? (int)align_up(B, 32) : n_col_tiles >= 64 ? 128 : 0;
+    if (rpt) {
+      *us = estimate(rpt / 32);
+      return rpt;
+    }
   }
-  double best = 0.0;
   int rpt = 160;
   for (int mb = 1; mb <= 5; mb++) {
-    const int tiles = cdiv(B, 32 * mb);
-    const double us = epi != EPI_ARGMAX && dense_few(32 * mb, tiles, N, K)
-                          ? few_us(mb, (long long)tiles * (N / 32), K / 64)
-                          : streaming_us(mb, (long long)tiles * n_col_tiles * 8, K / 64);
-    if (mb == 1 || us <= best) {
-      best = us;
+    const double t = estimate(mb);
+    if (mb == 1 || t <= *us) {
+      *us = t;
       rpt = 32 * mb;
     }
-    if (tiles == 1) break;
+    if (B <= 32 * mb) break;
   }
   return rpt;
 }
@@ -207,8 +230,9 @@ int dense_gemm(const bf16_t *A, const bf16_t *W, const float *bias, void *out, i
   GemmParams g = dense_params(A, W, bias, out, B, N, K);
   g.amax_val = amax_val;
   g.amax_idx = amax_idx;
-  int rpt = dense_rows_per_tile(B, g.n_col_tiles, N, K, epi);
-  if (B >= (epi == EPI_ARGMAX ? argmax_tall_min_rows() : dense_tall_min_rows()) && gemm_tall_applies(g, false, epi) &&
+  double us = 0.0;
+  int rpt = dense_rows_per_tile(B, g.n_col_tiles, N, K, epi, &us);
+  if ((epi == EPI_ARGMAX ? B >= argmax_tall_min_rows() : dense_tall(B, N, K, us)) && gemm_tall_applies(g, false, epi) &&
       gemm_tall_shape_ok(N, K, B))
     rpt = 256;
   if (epi == EPI_ARGMAX) {
@@ -229,8 +253,9 @@ int dense_gemm_mixed(const bf16_t *A, const bf16_t *W, float *out, const GemmBf1
     GPTOSS_REQUIRE(ranges[i].from % 32 == 0 && ranges[i].to % 32 == 0 && ranges[i].ld % 4 == 0 && aligned(ranges[i].out, 8),
                    GPTOSS_ERR_DIM, "dense_gemm_mixed: ranges are whole 32-column blocks of aligned rows");
   }
-  int rpt = dense_rows_per_tile(B, g.n_col_tiles, N, K, EPI_MIXED);
-  if (B >= dense_tall_min_rows() && wide && gemm_tall_applies(g, false, EPI_MIXED) && gemm_tall_shape_ok(N, K, B)) rpt = 256;
+  double us = 0.0;
+  int rpt = dense_rows_per_tile(B, g.n_col_tiles, N, K, EPI_MIXED, &us);
+  if (dense_tall(B, N, K, us) && wide && gemm_tall_applies(g, false, EPI_MIXED) && gemm_tall_shape_ok(N, K, B)) rpt = 256;
   return run_gemm_dense(g, EPI_MIXED, rpt, cdiv(B, rpt), s);
 }
 
@@ -243,7 +268,7 @@ int dense_gemm_partial(const bf16_t *A, const bf16_t *W, float *out, size_t max_
                        hipStream_t s) {
   *parts = 1;
   GemmParams g = dense_params(A, W, nullptr, out, B, N, K);
-  if (B >= dense_tall_min_rows()) return dense_gemm(A, W, nullptr, out, EPI_F32, B, N, K, s);
+  if (B >= 2048) return dense_gemm(A, W, nullptr, out, EPI_F32, B, N, K, s);
   const int nslab = K / 64;
   double best = 0.0;
   int rpt = 32, splits = 1, slabs = nslab;

@@ -140,7 +140,8 @@ __device__ __forceinline__ float glu(const GluForm &f, float gate, float up) {
 // hold != nullptr (SwiGLU form only): the tile goes to LDS instead of memory, row r of the tile at
 // hold + r * HOLD_ROW, this wave's 16 outputs from column hold_col on.
 // epilogue_rows: bias_of(c) is the bias of the block's column c, wave-uniform.
-template <int MB, int EPI, typename BIAS>
+// STEP: rows from one block to the next.
+template <int MB, int EPI, int STEP = 32, typename BIAS>
 __device__ __forceinline__ void epilogue_rows(const GemmParams &p, int row0, int rows, int n0, int lane,
                                               const f32x16 (&acc)[MB], const BIAS &bias_of, bf16_t *hold = nullptr,
                                               int hold_col = 0) {
@@ -166,11 +167,11 @@ __device__ __forceinline__ void epilogue_rows(const GemmParams &p, int row0, int
     // address = wave-uniform base (scalar registers) + a 32-bit per-lane element offset
     bf16_t *o = reinterpret_cast<bf16_t *>(p.out) + (size_t)row0 * half_n + (n0 >> 1);
     const uint32_t lane_off = (uint32_t)tok * (uint32_t)half_n + (uint32_t)h4;
-    const int row_lim = rows - tok;  // block i of this lane is a real row iff i*32 < row_lim
+    const int row_lim = rows - tok;  // block i of this lane is a real row iff i * STEP < row_lim
 #pragma unroll
     for (int i = 0; i < MB; i++) {
-      if (i * 32 < row_lim) {
-        bf16_t *orow = o + (size_t)((uint32_t)(i * 32) * (uint32_t)half_n);
+      if (i * STEP < row_lim) {
+        bf16_t *orow = o + (size_t)((uint32_t)(i * STEP) * (uint32_t)half_n);
 #pragma unroll
         for (int g = 0; g < 2; g++) {
           float v[4];
@@ -179,7 +180,7 @@ __device__ __forceinline__ void epilogue_rows(const GemmParams &p, int row0, int
             v[q] = glu(p.glu, acc[i][g * 4 + q] + bg[g * 4 + q], acc[i][(g + 2) * 4 + q] + bu[g * 4 + q]);
           }
           const u32x2 pk = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-          if (hold) *reinterpret_cast<u32x2 *>(hold + (i * 32 + tok) * HOLD_ROW + hold_col + h4 + g * 8) = pk;
+          if (hold) *reinterpret_cast<u32x2 *>(hold + (i * STEP + tok) * HOLD_ROW + hold_col + h4 + g * 8) = pk;
           else *reinterpret_cast<u32x2 *>(orow + lane_off + g * 8) = pk;
         }
       }
@@ -201,7 +202,7 @@ __device__ __forceinline__ void epilogue_rows(const GemmParams &p, int row0, int
           bf16_t *o = rg.out + (size_t)(row0 + tok) * rg.ld + (n0 - rg.from) + h4;
 #pragma unroll
           for (int i = 0; i < MB; i++)
-            if (i * 32 < rows - tok) {
+            if (i * STEP < rows - tok) {
 #pragma unroll
               for (int g = 0; g < 4; g++) {
                 float v[4];
@@ -213,7 +214,7 @@ __device__ __forceinline__ void epilogue_rows(const GemmParams &p, int row0, int
                     v[q] *= v[q];
                   }
                 }
-                *reinterpret_cast<u32x2 *>(o + (size_t)(i * 32) * rg.ld + g * 8) =
+                *reinterpret_cast<u32x2 *>(o + (size_t)(i * STEP) * rg.ld + g * 8) =
                     u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
               }
             }
@@ -225,8 +226,8 @@ __device__ __forceinline__ void epilogue_rows(const GemmParams &p, int row0, int
     const int row_lim = rows - tok;
 #pragma unroll
     for (int i = 0; i < MB; i++) {
-      if (i * 32 < row_lim) {
-        const size_t row_off = (size_t)((uint32_t)(row0 + i * 32) * (uint32_t)N) + n0;
+      if (i * STEP < row_lim) {
+        const size_t row_off = (size_t)((uint32_t)(row0 + i * STEP) * (uint32_t)N) + n0;
 #pragma unroll
         for (int g = 0; g < 4; g++) {
           float v[4];
@@ -244,13 +245,13 @@ __device__ __forceinline__ void epilogue_rows(const GemmParams &p, int row0, int
   }
 }
 
-template <int MB, int EPI, bool CONST_BIAS = false>
+template <int MB, int EPI, bool CONST_BIAS = false, int STEP = 32>
 __device__ __forceinline__ void epilogue_store(const GemmParams &p, int mat, int row0, int rows, int n0,
                                                int lane, const f32x16 (&acc)[MB], bf16_t *hold = nullptr,
                                                int hold_col = 0) {
   using BiasPtr = std::conditional_t<CONST_BIAS, const_as<float>, const float *>;
   const BiasPtr bp = (BiasPtr)(p.bias ? p.bias + (size_t)mat * p.N + n0 : nullptr);
-  epilogue_rows<MB, EPI>(p, row0, rows, n0, lane, acc, [&](int c) { return bp ? bp[c] : 0.f; }, hold, hold_col);
+  epilogue_rows<MB, EPI, STEP>(p, row0, rows, n0, lane, acc, [&](int c) { return bp ? bp[c] : 0.f; }, hold, hold_col);
 }
 
 // One (row tile, column tile) work item with a compile-time number of 32-row blocks, so every

@@ -23,8 +23,18 @@
 // the same epilogue code as gemm_kernel.hpp, so the results are bit-identical to it.  Three forms:
 // gather + SwiGLU (GEMM1 of a prompt pass), plain fp32 output (GEMM2, the projections), and the row
 // arg-max of the classifier, which writes no products at all and is the fastest of the three.
+//
+// A tile costs what its rows are worth: its row blocks go to the two wave rows in turn, and the loop has a form for 1, 2, 3 and
+// 4 blocks of a wave.  One block takes about 0.55 of a full tile (fragment reads and the same loads), two 0.6, three 0.75.  And
+// where an XCD's last round of work items leaves half of its workgroups idle, its items are cut into halves of their rows.
+// Before -> now (us): 2880 x 4096, 2048 rows (12 tiles per XCD for 32 workgroups) 77 -> 57, 2048 x 10240 164 -> 111, 5120 x
+// 2880, 3100 rows 129 -> 112, 8000 (2.5 rounds) 211 -> 199; 16640 x 2048, 8000 rows (8.1) 485 -> 469; 8192 x 2048 (whole rounds)
+// 227 -> 228; MoE block of 4500 tokens 1104 -> 1020, 5000 1129 -> 1070, 5999 1268 -> 1252, 4096 and 5000 under Zipf 1.1
+// 1003 -> 922 and 1173 -> 1109.  (Idle CUs at the end of a launch leave the others power, so a round saved is worth less than
+// its share.)
 // gemm_tall.hip instantiates the forms without the gather, gemm_tall_grouped.hip the one with it.
 #pragma once
+#include <algorithm>
 #include <mutex>
 
 #include "gemm_kernel.hpp"
@@ -52,6 +62,7 @@ struct TallShape {
   static constexpr int NM = RB * CB, NR = RB + CB;      // MFMAs and fragment reads of a k-step
   static_assert(LW % 2 == 0 && LA % 4 == 0, "a k-step issues half a W stage and a quarter of an A chunk");
   static_assert(NM >= NR + 2 * (LA / 4 + LW / 2), "room for a k-step's reads and loads between its MFMAs");
+  static constexpr int STEP = WR * 32;                  // rows from one of a wave's blocks to the next: the waves take them in turn
 };
 
 template <int N>
@@ -130,14 +141,14 @@ __device__ __forceinline__ void tall_epilogue(const GemmParams &p, unsigned char
     if constexpr (sizeof(v) == 8) d += h * 8;   // two lanes share a piece
     *reinterpret_cast<decltype(v) *>(d) = v;
   };
-  // rows r * 32 .. of the tile: `width` 16-byte pieces of them are real, out = first byte of the first row
+  // rows of the wave's block r: `width` 16-byte pieces of them are real, out = first byte of the first row
   auto flush = [&](auto pieces, int r, int width, unsigned char *out, size_t ld) {
     constexpr int P = decltype(pieces)::value, PER = 64 / P;   // rows of a store instruction
 #pragma unroll
     for (int i = 0; i < 32 / PER; i++) {
       const int row = i * PER + lane / P, piece = lane % P;
       const u32x4 v = *reinterpret_cast<const u32x4 *>(buf + row * (P * 16) + ((piece ^ (row & (P - 1))) << 4));
-      if (r * 32 + row < rows && piece < width) *reinterpret_cast<u32x4 *>(out + (size_t)(r * 32 + row) * ld + piece * 16) = v;
+      if (r * SH::STEP + row < rows && piece < width) *reinterpret_cast<u32x4 *>(out + (size_t)(r * SH::STEP + row) * ld + piece * 16) = v;
     }
   };
   // the compiler copies accumulators out of their AGPRs early, and spills, unless they are pinned until they are used
@@ -149,7 +160,7 @@ __device__ __forceinline__ void tall_epilogue(const GemmParams &p, unsigned char
     for (int i = 0; i < CB; i++) {
 #pragma unroll
       for (int r = 0; r < RB; r++) pin(i, r);
-      if (c0 + i * 32 < N) epilogue_store<RB, EPI, true>(p, mat, row0, rows, c0 + i * 32, lane, acc[i]);
+      if (c0 + i * 32 < N) epilogue_store<RB, EPI, true, SH::STEP>(p, mat, row0, rows, c0 + i * 32, lane, acc[i]);
     }
   } else {
 #pragma unroll
@@ -211,7 +222,7 @@ __device__ __forceinline__ void tall_epilogue(const GemmParams &p, unsigned char
 template <class SH, bool GATHER, int EPI>
 __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p) {
   constexpr int RB = SH::RB, CB = SH::CB, LW = SH::LW, LA = SH::LA, LW1 = SH::LW / 2, LA1 = SH::LA / 4;
-  constexpr int NM = SH::NM, NR = SH::NR, NSTW = SH::NSTW;
+  constexpr int NR = SH::NR;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -237,12 +248,17 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
     lo = xcd * chunk;
     hi = min(total, lo + chunk);
   }
+  // An XCD's items in its last round, if they leave half of its workgroups without one, are cut into two halves of their rows
+  const int whole = (hi - lo) - (hi - lo) % per_xcd, rest = hi - lo - whole;
+  const bool halves = 2 * rest <= per_xcd;
+  const int mine = halves ? whole + 2 * rest : hi - lo;
   int j = blockIdx.x >> 3;
-  auto valid = [&](int jj) { return lo + jj < hi; };
+  auto valid = [&](int jj) { return jj < mine; };
   if (!valid(j)) return;
   // which tile, which matrix, and this wave's share of the W loads
   auto decode = [&](int jj, TallSrc<SH> &t) {
-    const int work = lo + jj;
+    const bool part = halves && jj >= whole;
+    const int work = lo + (part ? whole + ((jj - whole) >> 1) : jj);
     int tile;
     if (p.tiles && p.tile_block > 1 && p.xcd_bounds) {
       const int info = bounds[XCD_BOUNDS_INTS + work / p.n_col_tiles];
@@ -271,6 +287,14 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
       t.row0 = tile * SH::BM;
       t.rows = min(SH::BM, p.dense_rows - t.row0);
     }
+    if (part) {   // whole row blocks; where there is but one the second half has no rows
+      const int first = min(t.rows, ((t.rows + 63) >> 6) * 32);
+      if (((jj - whole) & 1) == 0) t.rows = first;
+      else {
+        t.row0 += t.rows > first ? first : 0;
+        t.rows -= first;
+      }
+    }
     t.ct = __builtin_amdgcn_readfirstlane(t.ct);
     t.mat = __builtin_amdgcn_readfirstlane(t.mat);
     t.row0 = __builtin_amdgcn_readfirstlane(t.row0);
@@ -294,7 +318,7 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
   if constexpr (GATHER) inv_k = pair_inverse(p.top_k);
   auto a_offsets = [&](TallSrc<SH> &t) {
     typedef int ids_t __attribute__((ext_vector_type(8), aligned(4)));
-    const int last = t.rows - 1, group = lane >> 3;
+    const int last = max(t.rows - 1, 0), group = lane >> 3;
     auto offset = [&](int src, int r) {
       const int c = (lane & 7) ^ ((r >> 1) & 7);
       return ((uint32_t)src * (uint32_t)K) * 2u + (uint32_t)c * 16u;
@@ -337,31 +361,39 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
 
   f32x16 acc[CB][RB];   // [column block][row block]
   const int sw = ((lane & 31) >> 1) & 7, h = lane >> 5;
-  const unsigned a_rd = SH::A_OFF + (wr * RB * 32 + (lane & 31)) * 128;
+  const unsigned a_rd = SH::A_OFF + (wr * 32 + (lane & 31)) * 128;
   unsigned a_k[4];      // where the lane finds its piece of k-step x of a chunk
 #pragma unroll
   for (int x = 0; x < 4; x++) a_k[x] = (unsigned)(((2 * x + h) ^ sw) << 4);
   const unsigned w_rd = (wc * CB) * 2 * 1024 + lane * 16;
   bf16x8 F[2][NR];      // two fragment sets: [0, CB) W column blocks, [CB, CB + RB) A row blocks
   // fragment read number i of a k-step, in the order the MFMAs want them: W0, every A, the other W;
-  // x = the k-step's number inside its A chunk
-  auto rd = [&](int wbuf, int kk, int abuf, int x, int set, int i) {
-    const int f = i == 0 ? 0 : (i <= RB ? CB + i - 1 : i - RB);
+  // x = the k-step's number inside its A chunk, NB = row blocks of the wave
+  auto rd = [&](auto nb, int wbuf, int kk, int abuf, int x, int set, int i) {
+    constexpr int NB = decltype(nb)::value;
+    const int f = i == 0 ? 0 : (i <= NB ? CB + i - 1 : i - NB);
     if (f < CB)
       F[set][f] = as_bf16x8(*reinterpret_cast<const u32x4 *>(lds + wbuf * SH::W_BYTES + w_rd + (f * 2 + kk) * 1024));
     else
       F[set][f] = as_bf16x8(
-          *reinterpret_cast<const u32x4 *>(lds + abuf * SH::A_BYTES + a_rd + (f - CB) * 32 * 128 + a_k[x]));
+          *reinterpret_cast<const u32x4 *>(lds + abuf * SH::A_BYTES + a_rd + (f - CB) * SH::STEP * 128 + a_k[x]));
   };
-  // one k-step: NM MFMAs out of fragment set `set`; with the first NR of them the fragment reads of
-  // the next k-step (into the other set), behind those whatever loads `loads(m)` issues
-  auto kstep = [&](int set, int wbuf, int kk, int abuf, int x, auto &&loads) {
+  // One k-step: NB * CB MFMAs out of fragment set `set`; with the first of them the fragment reads of
+  // the next k-step (into the other set), behind those its loads, loads(0), loads(1), ...
+  auto kstep = [&](auto nb, int set, int wbuf, int kk, int abuf, int x, auto &&loads) {
+    constexpr int NB = decltype(nb)::value, M = NB * CB, R = NB + CB, L = LA1 + LW1;
+    constexpr int PER = (R + L <= M) ? 1 : 2;                                // reads per MFMA
+    constexpr int FIRST = PER == 1 ? R : (M - L > 0 ? M - L : 0);            // MFMA that the first load stands behind
+    constexpr int APART = FIRST + 2 * (L - 1) < M ? 2 : 1;
+    static_assert(FIRST + APART * (L - 1) < M && PER * M >= R, "every read and load has its place");
 #pragma unroll
-    for (int m = 0; m < NM; m++) {
-      acc[m / RB][m % RB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(F[set][m / RB], F[set][CB + m % RB],
-                                                                    acc[m / RB][m % RB], 0, 0, 0);
-      if (m < NR) rd(wbuf, kk, abuf, x, set ^ 1, m);
-      loads(m);
+    for (int m = 0; m < M; m++) {
+      acc[m / NB][m % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(F[set][m / NB], F[set][CB + m % NB],
+                                                                    acc[m / NB][m % NB], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < PER; i++)
+        if (m * PER + i < R) rd(nb, wbuf, kk, abuf, x, set ^ 1, m * PER + i);
+      if (m >= FIRST && (m - FIRST) % APART == 0) loads((m - FIRST) / APART);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -391,9 +423,6 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
   });
   wait_vmcnt<4 * (LA1 + LW1)>();   // chunk 0 and stage 0 have landed; the loads behind them may be on their way
   __builtin_amdgcn_s_barrier();
-#pragma unroll
-  for (int i = 0; i < NR; i++) rd(0, 0, 0, 0, 0, i);
-  __builtin_amdgcn_sched_barrier(0);
   int g = 0;   // running stage count (even at the start of every item): W buffer g & 3
   int ab = 0;  // A buffer of the current chunk: the running chunk count modulo 3
   // what the loop requests next: a W stage, of the current item or the next one, and an A chunk
@@ -414,57 +443,71 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
       for (int r = 0; r < RB; r++)
 #pragma unroll
         for (int x = 0; x < 16; x++) acc[i][r][x] = 0.f;
-    for (int s = 0; s < S; s += 2, g += 2) {
-      // ---- even stage s: the first half of A chunk s / 2 --------------------------------------
-      const int ab1 = ab == 2 ? 0 : ab + 1, ab2 = ab1 == 2 ? 0 : ab1 + 1;
-      // from here on the A chunks that are requested (two ahead) are the next item's, and so is every W stage from the
-      // middle of this round on
-      const bool wrap = s + 4 >= S;
-      if (s + 4 == S) ao = 0;
-      const unsigned ad = a_dst(ab2);
-      // Every k-step issues a quarter of A chunk s / 2 + 2, into the buffer that chunk s / 2 - 1 left
-      // (every wave is past the barrier of the stage that read it last), and half of a W stage,
-      // behind the fragment reads: loads(x, ...) places them after MFMAs NR, NR + 2, ...
-      auto loads = [&](int m, auto xx, int wbuf, auto hh) {
-        constexpr int X = decltype(xx)::value, H = decltype(hh)::value;
-        static_for<0, LA1>([&](auto q) {
-          constexpr int Q = X * LA1 + decltype(q)::value;
-          if (m == NR + 2 * decltype(q)::value) tall_load<Q * 1024>(ad, wrap ? nxt.a[Q] : cur.a[Q], abuf, ao);
-        });
-        if (m == NR + 2 * LA1) tall_load<2 * H * 1024>(w_dst(wbuf), voff_w, ws, wo[H]);
-        if (m == NR + 2 * LA1 + 2) {
-          tall_load<(2 * H + 1) * 1024>(w_dst(wbuf), voff_w1, ws, wo[H]);
-          wo[H] += 2048;
+    // the loop over K for NB row blocks of the wave
+    auto walk = [&](auto nb) {
+      for (int s = 0; s < S; s += 2, g += 2) {
+        // ---- even stage s: the first half of A chunk s / 2 --------------------------------------
+        const int ab1 = ab == 2 ? 0 : ab + 1, ab2 = ab1 == 2 ? 0 : ab1 + 1;
+        // from here on the A chunks that are requested (two ahead) are the next item's, and so is every W stage from the
+        // middle of this round on
+        const bool wrap = s + 4 >= S;
+        if (s + 4 == S) ao = 0;
+        const unsigned ad = a_dst(ab2);
+        // Every k-step issues a quarter of A chunk s / 2 + 2, into the buffer that chunk s / 2 - 1 left
+        // (every wave is past the barrier of the stage that read it last), and half of a W stage,
+        // behind the fragment reads
+        auto loads = [&](int m, auto xx, int wbuf, auto hh) {
+          constexpr int X = decltype(xx)::value, H = decltype(hh)::value;
+          static_for<0, LA1>([&](auto q) {
+            constexpr int Q = X * LA1 + decltype(q)::value;
+            if (m == decltype(q)::value) tall_load<Q * 1024>(ad, wrap ? nxt.a[Q] : cur.a[Q], abuf, ao);
+          });
+          if (m == LA1) tall_load<2 * H * 1024>(w_dst(wbuf), voff_w, ws, wo[H]);
+          if (m == LA1 + 1) {
+            tall_load<(2 * H + 1) * 1024>(w_dst(wbuf), voff_w1, ws, wo[H]);
+            wo[H] += 2048;
+          }
+        };
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        using I3 = std::integral_constant<int, 3>;
+        kstep(nb, 0, g & 3, 1, ab, 1, [&](int m) { loads(m, I0{}, (g + 3) & 3, I0{}); });
+        // behind W stage s+1 were issued the loads of two k-steps of stage s-1 and of one of stage s
+        wait_vmcnt<3 * (LA1 + LW1)>();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        kstep(nb, 1, (g + 1) & 3, 0, ab, 2, [&](int m) { loads(m, I1{}, (g + 3) & 3, I1{}); });
+        if (s + 4 == S) {   // W stage s + 3 was this item's last
+          ws = nxt.w;
+          wo[0] = nxt.wo[0];
+          wo[1] = nxt.wo[1];
         }
-      };
-      using I0 = std::integral_constant<int, 0>;
-      using I1 = std::integral_constant<int, 1>;
-      using I2 = std::integral_constant<int, 2>;
-      using I3 = std::integral_constant<int, 3>;
-      kstep(0, g & 3, 1, ab, 1, [&](int m) { loads(m, I0{}, (g + 3) & 3, I0{}); });
-      // behind W stage s+1 were issued the loads of two k-steps of stage s-1 and of one of stage s
-      wait_vmcnt<3 * (LA1 + LW1)>();
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      kstep(1, (g + 1) & 3, 0, ab, 2, [&](int m) { loads(m, I1{}, (g + 3) & 3, I1{}); });
-      if (s + 4 == S) {   // W stage s + 3 was this item's last
-        ws = nxt.w;
-        wo[0] = nxt.wo[0];
-        wo[1] = nxt.wo[1];
+        // ---- odd stage s+1: the second half of the chunk -----------------------------------------
+        kstep(nb, 0, (g + 1) & 3, 1, ab, 3, [&](int m) { loads(m, I2{}, (g + 4) & 3, I0{}); });
+        // W stage s+2, and with it the A chunk that the next stage starts (its last loads went out in
+        // front of that stage's), must have landed
+        wait_vmcnt<3 * (LA1 + LW1)>();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        kstep(nb, 1, (g + 2) & 3, 0, ab1, 0, [&](int m) { loads(m, I3{}, (g + 4) & 3, I1{}); });
+        ao += 128;
+        ab = ab1;
       }
-      // ---- odd stage s+1: the second half of the chunk -----------------------------------------
-      kstep(0, (g + 1) & 3, 1, ab, 3, [&](int m) { loads(m, I2{}, (g + 4) & 3, I0{}); });
-      // W stage s+2, and with it the A chunk that the next stage starts (its last loads went out in
-      // front of that stage's), must have landed
-      wait_vmcnt<3 * (LA1 + LW1)>();
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      kstep(1, (g + 2) & 3, 0, ab1, 0, [&](int m) { loads(m, I3{}, (g + 4) & 3, I1{}); });
-      ao += 128;
-      ab = ab1;
-    }
+    };
+    // The first fragments (those that the item before has read with its last k-step are not kept across its epilogue, and
+    // may be of fewer blocks).
+#pragma unroll
+    for (int i = 0; i < NR; i++) rd(std::integral_constant<int, RB>{}, g & 3, 0, ab, 0, 0, i);
+    __builtin_amdgcn_sched_barrier(0);
+    // A wave takes every second row block of the tile, so a tile of few rows has few for each of them.
+    const int nb = (cur.rows + SH::STEP - 1) / SH::STEP;
+    if (nb >= RB) walk(std::integral_constant<int, RB>{});
+    else if (nb == 3) walk(std::integral_constant<int, 3>{});
+    else if (nb == 2) walk(std::integral_constant<int, 2>{});
+    else walk(std::integral_constant<int, 1>{});
     // epilogue: the wave's column blocks, each with its row blocks.  The empty asm pins a column
     // block's accumulators in their AGPRs until the block before it has been stored: left alone,
     // the compiler copies every accumulator to VGPRs where the stage loop ends, and spills.
@@ -516,7 +559,7 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
           bv[r] = ov;
           bi[r] = oi;
         }
-        const int row = (wr * RB + r) * 32 + lane;
+        const int row = r * SH::STEP + wr * 32 + lane;
         if (lane < 32 && row < cur.rows) {
           const size_t o = (size_t)(cur.row0 + row) * (SH::WC * p.n_col_tiles) + cur.ct * SH::WC + wc;
           p.amax_val[o] = bv[r];
@@ -525,7 +568,7 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
       }
     } else {
       unsigned char *buf = lds + SH::A_OFF + (ab == 0 ? 2 : ab - 1) * SH::A_BYTES + w * LA * 1024;
-      tall_epilogue<SH, EPI>(p, buf, cur.mat, cur.row0 + wr * RB * 32, cur.rows - wr * RB * 32,
+      tall_epilogue<SH, EPI>(p, buf, cur.mat, cur.row0 + wr * 32, cur.rows - wr * 32,
                              cur.ct * SH::BN + wc * CB * 32, lane, acc);
     }
     if (!more) break;
@@ -555,9 +598,8 @@ static int launch_tall(const GemmParams &p, int max_tiles, hipStream_t s) {
   }
   GemmParams q = p;
   q.n_col_tiles = cdiv(p.N, SH::BN);
-  const int total = max_tiles * q.n_col_tiles;
-  int grid = ((total + 7) / 8) * 8;
-  if (grid > 256) grid = 256;
+  const long long items = (long long)max_tiles * q.n_col_tiles;
+  int grid = (int)std::min<long long>(16 * ((items + 7) / 8), 256);   // room for the halves of an XCD's items
   if (grid == 0) return GPTOSS_OK;
   {
     TraceScope ts(EPI == EPI_ARGMAX ? "gemm_argmax" : GATHER ? "gemm1_gather_swiglu" : "gemm_f32", s);

@@ -70,6 +70,13 @@ def test_dense_gemm_of_a_prompt_pass_equals_the_same_rows_in_small_batches(ops, 
         assert torch.equal(full[r0:r0 + step], ops.dense_gemm(a[r0:r0 + step].contiguous(), wp, N, b)), r0
 
 
+# Tiles of 256 rows per XCD, 32 of which are a round: 12 (halves only), 74 (two rounds and halves; of the last tile's 52 rows, 33
+# and 1, whose second half is 20, 1 and 0), 83 (two rounds, the rest whole)
+@pytest.mark.parametrize("B,N,K", [(2048, 2880, 4096), (2100, 16640, 256), (2081, 16640, 256), (2049, 16640, 256), (2369, 16672, 320)])
+def test_halves_of_the_tiles_in_a_last_round(ops, B, N, K):
+    test_dense_gemm_of_a_prompt_pass_equals_the_same_rows_in_small_batches(ops, B, N, K)
+
+
 @pytest.mark.parametrize("B,V,K", [(5, 4096, 256), (130, 201088, 2880), (1024, 50304, 512), (515, 9984, 256),
                                    (256, 9984, 512), (255, 4128, 320)])
 def test_classifier_argmax_equals_argmax_of_logits(ops, B, V, K):

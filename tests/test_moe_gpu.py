@@ -485,6 +485,12 @@ def test_last_row_tiles_of_a_prompt_pass(ops, rows):
     _prompt_pass_equals_small_batches(ops, g, router, torch.zeros(2, device="cuda"), t, 1)
 
 
+@pytest.mark.parametrize("rows", [32, 33, 64, 65, 96, 97, 128, 129, 160, 192, 193, 224, 225, 385])
+def test_row_blocks_of_a_prompt_pass(ops, rows):
+    """Tiles of one to four row blocks per wave, whole and in halves (the launch has fewer tiles than workgroups)."""
+    test_last_row_tiles_of_a_prompt_pass(ops, rows)
+
+
 @pytest.mark.parametrize("k", [1, 2, 3, 5, 7, 8])
 def test_tokens_of_pairs_in_a_prompt_pass(ops, k):
     """Every token on all k experts: the token of a pair is the pair's number over k."""
