@@ -28,7 +28,7 @@ DEVICE = ["--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-pa
 CORE = ("common.cpp", "engine.cpp", "host_pool.cpp", "model_registry.cpp", "glue.hip", "precise.hip", "gemm_dense.cpp",
         "gemm_bf16.hip", "gemm_few.hip", "gemm_mixed_bf16.hip", "gemm_tall.hip")
 #: architecture -> sources of its class beside CORE (None: all of them)
-MODELS = {"gpt-oss": None, "Nezavik": ("model_nezavik.cpp", "recurrent.hip", "window_attn.hip"),
+MODELS = {"gpt-oss": None, "Nezavik": ("model_nezavik.cpp", "recurrent.hip", "scan_chunks.hip", "window_attn.hip"),
           "Netinex": ("model_netinex.cpp", "retention.hip", "recurrent.hip", "window_attn.hip", "rotary.hip", "moe_layer.cpp",
                       "moe_route.hip", "moe_gemm.hip", "gemm_gather_bf16.hip", "gemm_tall_grouped.hip")}
 

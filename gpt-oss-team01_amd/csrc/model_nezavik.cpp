@@ -122,7 +122,7 @@ int Nezavik::forward_rows(const StepRows &r) {
     sc.out = y_rows;
     sc.ld_out = sc.heads * sc.V;
     sc.conv_desc = w.conv;
-    GPTOSS_STEP(run_scan(sc, r, s));
+    GPTOSS_STEP(!f32 && scan_chunks_apply(sc, r) ? run_scan_chunks(sc, r, s) : run_scan(sc, r, s));
     GatedNorm g = w.gated;
     g.y = y_rows;
     g.ld_y = sc.ld_out;

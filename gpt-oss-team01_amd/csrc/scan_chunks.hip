@@ -1,0 +1,408 @@
+// The gated delta rule with one decay per head and the state-space recurrence over stretches of a prompt on gfx950, in
+// chunks of 32 tokens on the matrix cores, in fp32 throughout (v_mfma_f32_16x16x4).  With t, s counting from the chunk's
+// first token, S the state in front of it, c_t the sum of the logarithms of the decays up to and with token t and
+// u_s what token s writes,
+//   o_t = e^(c_t) S^T q_t + sum_{s <= t} e^(c_t - c_s) (k_s . q_t) u_s
+//   S  <- e^(c_31) S + sum_s e^(c_31 - c_s) k_s u_s^T
+// State space: u_s = dt_s v_s.  Delta rule: u_t = beta_t (v_t - e^(c_t) S^T k_t - sum_{s < t} e^(c_t - c_s) (k_s . k_t) u_s), a
+// triangular system whose diagonal blocks of 16 are inverted by forward substitution.
+//
+// The sums c are kept in double, so that a difference of two is as exact as one decay's logarithm; every weight is
+// e^(difference) <= 1, whatever the decays.
+//
+// A workgroup of four waves has 64 columns of one head's state of one sequence, a wave 16 of them, in registers.  Reduction
+// indices are taken four at a time as a 16x16 result lies in its lanes (lane group c = lane >> 4 has rows 4 c .. + 3): state,
+// u and token products are operands of the next product without a shuffle, and an operand's four values are one 16-byte read.
+//
+// Token by token (recurrent.hip) a state element takes three (state space) or four vector instructions a token, and the
+// reads of keys and queries fill LDS at the same time; here it takes two or three products at twice the vector units' rate.
+// Measured, token by token -> here (us): 8 prompts of 1000 tokens, 32 heads of 128 x 64 (state space) 338 -> 152, 16 heads of
+// 128 x 128 (delta rule) 412 -> 222; 16 prompts of 260 150 -> 85, 195 -> 121; one 71 -> 42, 82 -> 60.  The products alone are 70
+// and 113 us of the first two: with one wave per SIMD what lies between them is not hidden (LDS reads are requested a group of
+// products ahead, the tokens' decays two chunks; as the compiler placed them 185 and 270 us), and the second workgroup that a
+// CU has room for, up to 128 keys, is there from 9 sequences of 32 heads on.
+// Errors against 64 bits, six layers of other sizes, 500 tokens, decays of 0.6 to 0.999 and of 0 to 0.9: 0.82 to 1.10 times
+// those of the recurrence token by token, 0.97 on average.
+#include "recurrent_device.hpp"
+
+namespace gptoss {
+
+constexpr int CHUNK = 32;
+
+// floats of LDS
+template <int NI>
+struct ChunkLds {
+  static constexpr int KP = 32 * NI, ROW = KP + 4;
+  static constexpr int Q = 0, K = CHUNK * ROW, STAGE = 2 * CHUNK * ROW;   // two stages
+  // 16x16 tiles, 64 lanes x 4 values: products with the queries, with the keys, inverses of the diagonal blocks
+  static constexpr int P = 2 * STAGE, A = P + 3 * 256, INV = A + 3 * 256;
+  static constexpr int CUM = INV + 2 * 256;                              // [2][CHUNK] doubles, then per token
+  static constexpr int FROM = CUM + 4 * CHUNK, OUT = FROM + 2 * CHUNK, BETA = OUT + 2 * CHUNK, FLOATS = BETA + 2 * CHUNK;
+};
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// inclusive sums over 32 lanes, of both halves of the wave
+__device__ __forceinline__ double prefix32(double v) {
+  auto add = [&](auto ctrl, auto rows) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (uint32_t)u, decltype(ctrl)::value, decltype(rows)::value, 0xf, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (uint32_t)(u >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xf, true);
+    v += __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+  };
+  using All = std::integral_constant<int, 0xf>;
+  add(std::integral_constant<int, 0x111>{}, All{});   // row_shr 1, 2, 4, 8: lanes without a source add nothing
+  add(std::integral_constant<int, 0x112>{}, All{});
+  add(std::integral_constant<int, 0x114>{}, All{});
+  add(std::integral_constant<int, 0x118>{}, All{});
+  add(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});   // the last lane of rows 0 and 2 to rows 1 and 3
+  return v;
+}
+
+template <int NI, int KIND>
+__global__ __launch_bounds__(256, NI <= 4 ? 2 : 1) void scan_chunk_kernel(Scan p, const RowSeg *__restrict__ segs, int n_seg,
+                                                                               int fewest) {
+  using L = ChunkLds<NI>;
+  constexpr bool DELTA = KIND == SCAN_DELTA;
+  constexpr int KP = L::KP, ROW = L::ROW, NB = 2 * NI;   // 16-key blocks of the state
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int seg_id = blockIdx.x % n_seg, unit = blockIdx.x / n_seg, blocks = (p.V + 63) / 64;
+  const RowSeg seg = segs[seg_id];
+  if (seg.n < fewest) return;   // taken elsewhere
+  if (unit >= p.heads * blocks) {   // workgroups of the convolutions' states come last
+    advance_conv_state(p, seg, unit - p.heads * blocks, gridDim.x / n_seg - p.heads * blocks);
+    return;
+  }
+  const int h = unit / blocks, kh = h / (p.heads / p.key_heads);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, c = lane >> 4;
+  const int c0 = (unit - h * blocks) * 64 + wave * 16, col = min(c0 + n, p.V - 1);   // columns c0 .. + 15 of the wave
+  const bool live = c0 + n < p.V;
+  const float rate = expf(p.a_log[h]), bias = p.dt_bias[h], skip = DELTA ? 0.f : p.d_skip[h];
+
+  f32x4 S[NB];   // keys 16 b + 4 c + e of column c0 + n
+  float *st = p.state + (((size_t)seg.slot * p.heads + h) * p.V + col) * KP + 4 * c;
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    S[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (seg.pos0 > 0 && live) S[b] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(st + 16 * b));
+  }
+
+  // The next chunk's inputs travel through registers while the current one is worked on.  Addresses: a base per chunk and a
+  // 32-bit offset per lane, its token's part by a product of 24 bits (a 64-bit product each takes as long as 16 others).
+  f32x4 rk[NI], rq[NI];
+  float rv[2][4];
+  const uint32_t ld4 = 4 * p.ld_conv;
+  auto fetch = [&](int t0) {
+    const int T = min(CHUNK, seg.n - t0);
+    const char *rows = reinterpret_cast<const char *>(p.conv + (size_t)(seg.row0 + t0) * p.ld_conv);
+    const char *ks = rows + 4 * (size_t)(p.k_col + kh * p.K), *qs = rows + 4 * (size_t)(p.q_col + kh * p.K);
+    const char *vs = rows + 4 * (size_t)(p.v_col + h * p.V);
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      const int idx = tid + 256 * i, t = min(idx / (KP / 4), T - 1), d = min(idx % (KP / 4) * 4, p.K - 4);
+      const uint32_t at = __umul24(t, ld4) + 4 * d;
+      rk[i] = *reinterpret_cast<const f32x4 *>(ks + at);
+      rq[i] = *reinterpret_cast<const f32x4 *>(qs + at);
+    }
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        rv[x][e] = *reinterpret_cast<const float *>(vs + __umul24(min(16 * x + 4 * c + e, T - 1), ld4) + 4 * col);
+  };
+  // rows and columns outside the problem are zero: they write nothing
+  auto put = [&](int t0, int stage) {
+    const int T = min(CHUNK, seg.n - t0);
+    float *at = lds + stage * L::STAGE;
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      const int idx = tid + 256 * i, t = idx / (KP / 4), d = idx % (KP / 4) * 4;
+      if (T < CHUNK || p.K < KP) {
+        const bool out = t >= T || d >= p.K;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          rk[i][e] = out ? 0.f : rk[i][e];
+          rq[i][e] = out ? 0.f : rq[i][e];
+        }
+      }
+      *reinterpret_cast<f32x4 *>(at + L::K + t * ROW + d) = rk[i];
+      *reinterpret_cast<f32x4 *>(at + L::Q + t * ROW + d) = rq[i];
+    }
+  };
+  // Decays and strengths of a chunk's tokens, lane t (and t + 32 again) of the last wave, requested two chunks ahead: it has
+  // the least to do while the token products are made.
+  float r_decay = 0.f, r_beta = 0.f;
+  auto fetch_tokens = [&](int t0) {
+    const float *in = p.in + (size_t)(seg.row0 + min(t0 + (tid & 31), seg.n - 1)) * p.ld_in + h;
+    r_decay = in[p.decay_col];
+    if (DELTA) r_beta = in[p.beta_col];
+  };
+  auto put_tokens = [&](int t0, int stage) {
+    const int t = lane & 31;
+    const bool real = t0 + t < seg.n;
+    const float dt = softplus_f(r_decay + bias);
+    const double cum = prefix32(real ? (double)(-rate * dt) : 0.0), all = __shfl(cum, 31);
+    if (lane < 32) {
+      reinterpret_cast<double *>(lds + L::CUM)[stage * CHUNK + t] = cum;
+      lds[L::FROM + stage * CHUNK + t] = exp_f((float)cum);
+      lds[L::OUT + stage * CHUNK + t] = exp_f((float)(all - cum));
+      lds[L::BETA + stage * CHUNK + t] = real ? (DELTA ? sigmoid_f(r_beta) : dt) : 0.f;
+    }
+  };
+
+  if (wave == 3) fetch_tokens(0);
+  fetch(0);
+  put(0, 0);
+  if (wave == 3) {
+    put_tokens(0, 0);
+    fetch_tokens(CHUNK);
+  }
+  int stage = 0;
+  for (int t0 = 0; t0 < seg.n; t0 += CHUNK, stage ^= 1) {
+    const int T = min(CHUNK, seg.n - t0);
+    const bool more = t0 + CHUNK < seg.n;
+    float v[2][4];
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[x][e] = 16 * x + 4 * c + e < T && live ? rv[x][e] : 0.f;
+    __syncthreads();   // this chunk is staged, and nobody reads the other stage or the tiles any more
+    if (more) {
+      if (wave == 3) {
+        put_tokens(t0 + CHUNK, stage ^ 1);
+        fetch_tokens(t0 + 2 * CHUNK);
+      }
+      fetch(t0 + CHUNK);
+    }
+    const float *q = lds + stage * L::STAGE + L::Q + n * ROW + 4 * c, *k = lds + stage * L::STAGE + L::K + n * ROW + 4 * c;
+    const double *cum = reinterpret_cast<const double *>(lds + L::CUM) + stage * CHUNK;
+    auto at4 = [&](const float *a) { return *reinterpret_cast<const f32x4 *>(a); };
+
+    // Products of keys (rows) and queries or keys (columns) of tokens, decayed and masked, in tiles (keys', columns') (0, 0),
+    // (0, 1), (1, 1).  Delta rule: the first two waves have a diagonal tile of the keys each and its inverse.
+    auto product = [&](const float *right, int sx, int tx, bool strict, const float *beta, float *to) {
+      f32x4 even = f32x4{0.f, 0.f, 0.f, 0.f}, odd = even, x[2][2], y[2][2];
+      auto load = [&](int i) {
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+          x[i & 1][b] = at4(k + sx * 16 * ROW + 16 * (2 * i + b));
+          y[i & 1][b] = at4(right + tx * 16 * ROW + 16 * (2 * i + b));
+        }
+      };
+      load(0);
+#pragma unroll
+      for (int i = 0; i < NI; i++) {
+        if (i + 1 < NI) load(i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          even = mfma4(x[i & 1][0][e], y[i & 1][0][e], even);
+          odd = mfma4(x[i & 1][1][e], y[i & 1][1][e], odd);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const int t = tx * 16 + n;
+      const double ct = cum[t];
+      const float scale = beta ? beta[t] : 1.f;
+      f32x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int s = sx * 16 + 4 * c + e;
+        const float x = scale * exp_f((float)(ct - cum[s])) * (even[e] + odd[e]);
+        w[e] = (strict ? s < t : s <= t) ? x : 0.f;
+      }
+      *reinterpret_cast<f32x4 *>(to + lane * 4) = w;
+    };
+    const float *beta = lds + L::BETA + stage * CHUNK;
+    if constexpr (!DELTA) {
+      if (wave < 3) product(q, wave == 2, wave > 0, false, nullptr, lds + L::P + wave * 256);
+    } else if (wave < 2) {
+      float *a = lds + L::A + wave * 512;
+      product(k, wave, wave, true, beta, a);
+      // The inverse of the unit lower triangular block by columns, lane (column).  Row t of the products lies at lanes t, t + 16,
+      // ..: four values each.
+      if (lane < 16) {
+        float x[16];
+#pragma unroll
+        for (int t = 0; t < 16; t++) {
+          float sum = t == n ? 1.f : 0.f;
+#pragma unroll
+          for (int g = 0; 4 * g < t; g++) {
+            const f32x4 w = at4(a + (g * 16 + t) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+              if (4 * g + e < t) sum = fmaf(-w[e], x[4 * g + e], sum);
+          }
+          x[t] = sum;
+        }
+        float *to = lds + L::INV + wave * 256 + (n >> 2) * 64 + (n & 3);
+#pragma unroll
+        for (int t = 0; t < 16; t++) to[t * 4] = x[t];
+      }
+    } else if (wave == 2) {
+      product(q, 0, 0, false, nullptr, lds + L::P);
+      product(q, 0, 1, false, nullptr, lds + L::P + 256);
+    } else {
+      product(q, 1, 1, false, nullptr, lds + L::P + 512);
+      product(k, 0, 1, true, beta, lds + L::A + 256);
+    }
+    __syncthreads();
+
+    // what the state in front of the chunk gives: [token][column]
+    f32x4 o[2], r[2];
+#pragma unroll
+    for (int x = 0; x < 2; x++) o[x] = r[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 qx[3][2], kx[3][2];
+    auto load = [&](int b) {
+#pragma unroll
+      for (int x = 0; x < 2; x++) {
+        qx[b % 3][x] = at4(q + x * 16 * ROW + 16 * b);
+        if (DELTA) kx[b % 3][x] = at4(k + x * 16 * ROW + 16 * b);
+      }
+    };
+    load(0);
+    load(1);
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      if (b + 2 < NB) load(b + 2);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int x = 0; x < 2; x++) {
+          o[x] = mfma4(qx[b % 3][x][e], S[b][e], o[x]);
+          if (DELTA) r[x] = mfma4(kx[b % 3][x][e], S[b][e], r[x]);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // what the tokens write
+    f32x4 u[2];
+#pragma unroll
+    for (int x = 0; x < 2; x++) {
+      const f32x4 from = at4(lds + L::FROM + stage * CHUNK + 16 * x + 4 * c), be = at4(beta + 16 * x + 4 * c);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        o[x][e] *= from[e];
+        u[x][e] = be[e] * (DELTA ? v[x][e] - from[e] * r[x][e] : v[x][e]);
+      }
+    }
+    auto tile = [&](f32x4 acc, const float *a, f32x4 b) {
+      const f32x4 w = at4(a + lane * 4);
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc = mfma4(w[e], b[e], acc);
+      return acc;
+    };
+    const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (DELTA) {
+      u[0] = tile(zero, lds + L::INV, u[0]);
+      u[1] -= tile(zero, lds + L::A + 256, u[0]);
+      u[1] = tile(zero, lds + L::INV + 256, u[1]);
+    }
+    o[0] = tile(o[0], lds + L::P, u[0]);
+    o[1] = tile(o[1], lds + L::P + 256, u[0]);
+    o[1] = tile(o[1], lds + L::P + 512, u[1]);
+    if (!DELTA)
+#pragma unroll
+      for (int x = 0; x < 2; x++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[x][e] = fmaf(skip, v[x][e], o[x][e]);
+    char *out = reinterpret_cast<char *>(p.out + (size_t)(seg.row0 + t0) * p.ld_out + h * p.V);
+    const uint32_t out4 = 4 * p.ld_out, first = __umul24(4 * c, out4) + 4 * (c0 + n);
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        float *to = reinterpret_cast<float *>(out + (16 * x + e) * out4 + first);
+        if (T == CHUNK && c0 + 16 <= p.V) *to = o[x][e];
+        else if (live && 16 * x + 4 * c + e < T) *to = o[x][e];
+      }
+
+    // the state behind the chunk
+    const float faded = lds[L::FROM + stage * CHUNK + CHUNK - 1];
+#pragma unroll
+    for (int x = 0; x < 2; x++) u[x] *= at4(lds + L::OUT + stage * CHUNK + 16 * x + 4 * c);
+    const float *keys = lds + stage * L::STAGE + L::K + 4 * c * ROW + n;   // keys of token 4 c, key n
+    float kt[2][2][2][4];
+    auto load_keys = [&](int i) {
+#pragma unroll
+      for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int x = 0; x < 2; x++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) kt[i & 1][b][x][e] = keys[(16 * x + e) * ROW + 16 * (2 * i + b)];
+    };
+    load_keys(0);
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      if (i + 1 < NI) load_keys(i + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < 2; b++) S[2 * i + b] *= faded;
+#pragma unroll
+      for (int x = 0; x < 2; x++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+          for (int b = 0; b < 2; b++) S[2 * i + b] = mfma4(kt[i & 1][b][x][e], u[x][e], S[2 * i + b]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (more) put(t0 + CHUNK, stage ^ 1);
+  }
+  if (live) {
+#pragma unroll
+    for (int b = 0; b < NB; b++) __builtin_nontemporal_store(S[b], reinterpret_cast<f32x4 *>(st + 16 * b));
+  }
+}
+
+bool scan_chunks_apply(const Scan &p, const StepRows &r) {
+  return (p.kind == SCAN_DELTA || p.kind == SCAN_STATE_SPACE) && r.longest >= SCAN_CHUNK_ROWS && scan_reads_wide(p) &&
+         p.K >= 4 && p.K <= SCAN_MAX_KEY && p.ld_conv < (1 << 22) && p.ld_out < (1 << 22);   // (24-bit row pitches)
+}
+
+template <int NI, int KIND>
+static int launch_chunks(const Scan &p, const StepRows &r, int fewest, hipStream_t s) {
+  constexpr int bytes = ChunkLds<NI>::FLOATS * (int)sizeof(float);
+  auto kern = scan_chunk_kernel<NI, KIND>;
+  GPTOSS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+  TraceScope ts(KIND == SCAN_DELTA ? "scan_delta" : "scan_state_space", s);
+  const size_t grid = (size_t)r.n_seg * (p.heads * cdiv(p.V, 64) + cdiv(p.conv_desc.channels, 256));
+  kern<<<(unsigned)grid, 256, bytes, s>>>(p, r.segs, r.n_seg, fewest);
+  GPTOSS_LAUNCH_CHECK("scan_chunk_kernel");
+  return GPTOSS_OK;
+}
+
+template <int KIND>
+static int launch_kind(const Scan &p, const StepRows &r, int fewest, hipStream_t s) {
+  switch (scan_key_pad(p.K) / 32) {
+    case 1: return launch_chunks<1, KIND>(p, r, fewest, s);
+    case 2: return launch_chunks<2, KIND>(p, r, fewest, s);
+    case 3: return launch_chunks<3, KIND>(p, r, fewest, s);
+    case 4: return launch_chunks<4, KIND>(p, r, fewest, s);
+    case 5: return launch_chunks<5, KIND>(p, r, fewest, s);
+    case 6: return launch_chunks<6, KIND>(p, r, fewest, s);
+    case 7: return launch_chunks<7, KIND>(p, r, fewest, s);
+    default: return launch_chunks<8, KIND>(p, r, fewest, s);
+  }
+}
+
+int run_scan_chunks(const Scan &p, const StepRows &r, hipStream_t s) {
+  GPTOSS_REQUIRE(scan_chunks_apply(p, r) && p.V >= 1 && p.key_heads >= 1 && p.heads % p.key_heads == 0, GPTOSS_ERR_DIM,
+                 "scan: kind %d with keys of %d, %d heads over %d does not go by chunks", (int)p.kind, p.K, p.heads, p.key_heads);
+  GPTOSS_REQUIRE(r.n_seg * ((long long)p.heads * cdiv(p.V, 64) + cdiv(p.conv_desc.channels, 256)) < (1ll << 31), GPTOSS_ERR_DIM,
+                 "scan: too many workgroups");
+  // Decoding rows beside the stretches: a chunk of one token takes a CU as long as a full one, which is nothing while there are
+  // CUs to spare; with more of them than run at a time they go as a step of their own.
+  int fewest = 1;
+  if ((long long)r.n_singles * p.heads * cdiv(p.V, 64) > 512) {
+    StepRows single = r;
+    single.segs = r.singles;
+    single.n_seg = r.n_singles;
+    single.longest = 1;
+    GPTOSS_STEP(run_scan(p, single, s));
+    fewest = 2;
+  }
+  return p.kind == SCAN_DELTA ? launch_kind<SCAN_DELTA>(p, r, fewest, s) : launch_kind<SCAN_STATE_SPACE>(p, r, fewest, s);
+}
+
+}  // namespace gptoss

@@ -1,0 +1,119 @@
+"""The delta rule and the state-space recurrence in chunks on the matrix cores, and token by token, against the recurrence in
+64 bits: gptoss::run_scan_chunks and gptoss::run_scan by their linker names, at the edges of chunks, key and column blocks."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import load_pkg
+
+pytestmark = pytest.mark.gpu
+
+DELTA, STATE_SPACE = 0, 2
+
+
+def _struct(name, *fields):
+    return type(name, (C.Structure,), {"_fields_": [(f, {"i": C.c_int, "f": C.c_float, "p": C.c_void_p}.get(t, t))
+                                                    for t, names in fields for f in names.split()]})
+
+
+Rotary = _struct("Rotary", ("p", "table"), ("i", "dims interleaved"))
+ShortConv = _struct("ShortConv", ("i", "col channels taps"), ("p", "weight bias"), ("i", "n_unit unit_dim"), ("f", "unit_scale"))
+Scan = _struct("Scan", ("i", "kind heads key_heads K V"), ("p", "conv"), ("i", "ld_conv q_col k_col v_col"), ("p", "inp"),
+               ("i", "ld_in beta_col decay_col"), ("p", "channel_decay"), ("i", "ld_decay"),
+               ("p", "a_log dt_bias d_skip head_decay decay_powers"), ("f", "value_scale"), (Rotary, "rot"),
+               ("p", "state out"), ("i", "ld_out"), (ShortConv, "conv_desc"), ("p", "conv_state"), ("i", "vec"))
+StepRows = _struct("StepRows", ("i", "n n_seg max_len"), ("p", "tokens slots lens offset segs sample singles"),
+                   ("i", "n_singles longest"), ("p", "tiles0 tiles1 tiles2"))
+
+
+def _softplus(x):
+    return np.maximum(x, 0) + np.log1p(np.exp(-np.abs(x)))
+
+
+def _exact(kind, q, k, v, b, a, rate, bias, skip, S):
+    """-> outputs [T, H, V], state [H, V, K], from state S, in float64."""
+    T, H, V = v.shape
+    out, dt = np.zeros((T, H, V)), _softplus(a + bias)
+    decay = np.exp(-rate * dt)
+    for t in range(T):
+        S = S * decay[t][:, None, None]
+        if kind == DELTA:
+            u = (v[t] - np.einsum("hvk,hk->hv", S, k[t])) / (1 + np.exp(-b[t]))[:, None]
+        else:
+            u = dt[t][:, None] * v[t]
+        S = S + u[:, :, None] * k[t][:, None, :]
+        out[t] = np.einsum("hvk,hk->hv", S, q[t]) + (skip[:, None] * v[t] if kind == STATE_SPACE else 0)
+    return out, S
+
+
+@pytest.mark.parametrize("strong", [False, True])
+@pytest.mark.parametrize("kind", [DELTA, STATE_SPACE])
+@pytest.mark.parametrize("heads,key_heads,K,V,lengths", [
+    (2, 1, 4, 5 * 4, (48, 1, 49)),          # one key block of which an eighth is there; a token beside the stretches
+    (4, 2, 36, 68, (64, 65, 31)),           # two column blocks, the second of four columns
+    (2, 2, 128, 64, (95, 96, 97, 32, 33)),
+    (1, 1, 132, 128, (50,)),
+    (2, 1, 256, 16, (129, 15, 16, 17)),     # the largest keys
+    (6, 3, 64, 64, (70,) + 100 * (1,)),     # more single tokens than workgroups run at a time
+])
+def test_chunks_equal_the_recurrence(kind, strong, heads, key_heads, K, V, lengths):
+    g = np.random.default_rng(K + V + kind)
+    n, slots, KP = sum(lengths), len(lengths), (K + 31) // 32 * 32
+    unit = lambda x: x / np.sqrt((x * x).sum(-1, keepdims=True))
+    q, k = unit(g.standard_normal((n, key_heads, K))) / np.sqrt(K), unit(g.standard_normal((n, key_heads, K)))
+    v = g.standard_normal((n, heads, V))
+    b, a = g.standard_normal((n, heads)), g.standard_normal((n, heads))
+    a_log, bias, skip = g.uniform(-5, -.5, heads) + 4.5 * strong, g.standard_normal(heads), g.standard_normal(heads)
+    state = np.zeros((slots, heads, V, KP))
+    state[..., :K] = g.standard_normal((slots, heads, V, K)) * 0.1
+    f32 = lambda x: np.ascontiguousarray(x, np.float32)
+    q, k, v, b, a, a_log, bias, skip, state = map(f32, (q, k, v, b, a, a_log, bias, skip, state))
+    conv = np.concatenate([q.reshape(n, -1), k.reshape(n, -1), v.reshape(n, -1)], axis=1)
+    inp = np.concatenate([b, a], axis=1)
+    order = g.permutation(slots)               # slots in another order than the stretches; the first starts from nothing
+    at = np.concatenate([[0], np.cumsum(lengths)])[:-1]
+    segs = np.array([(r, m, s, 0 if i == 0 else 7) for i, (r, m, s) in enumerate(zip(at, lengths, order))], np.int32)
+
+    lib, keep = load_pkg("lib").load(), []
+
+    def dev(x):
+        keep.append(torch.from_numpy(np.ascontiguousarray(x)).cuda())
+        return keep[-1].data_ptr()
+
+    nk = key_heads * K
+    got = []
+    for name in ("_ZN6gptoss15run_scan_chunksERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t",
+                 "_ZN6gptoss8run_scanERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t"):
+        st, out = torch.from_numpy(state).cuda(), torch.full((n, heads * V), np.nan, device="cuda")
+        p = Scan(kind=kind, heads=heads, key_heads=key_heads, K=K, V=V, conv=dev(conv), ld_conv=conv.shape[1], q_col=0, k_col=nk,
+                 v_col=2 * nk, inp=dev(inp), ld_in=2 * heads, beta_col=0, decay_col=heads, a_log=dev(a_log), dt_bias=dev(bias),
+                 d_skip=dev(skip), value_scale=1.0, state=st.data_ptr(), out=out.data_ptr(), ld_out=heads * V)
+        singles = segs[segs[:, 1] == 1]
+        r = StepRows(n=n, n_seg=slots, segs=dev(segs), singles=dev(singles) if len(singles) else None, n_singles=len(singles),
+                     longest=max(lengths))
+        f = getattr(lib, name)
+        f.restype, f.argtypes = C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p]
+        torch.cuda.synchronize()
+        assert f(C.addressof(p), C.addressof(r), None) == 0
+        torch.cuda.synchronize()
+        got.append((out.cpu().numpy().reshape(n, heads, V).astype(np.float64), st.cpu().numpy().astype(np.float64)))
+
+    d = lambda x: x.astype(np.float64)
+    rep = lambda x: np.repeat(d(x), heads // key_heads, axis=1)
+    want, state_want = np.zeros((n, heads, V)), d(state)
+    for r0, m, s, pos0 in segs:
+        rows = slice(r0, r0 + m)
+        S0 = d(state[s, ..., :K]) if pos0 else np.zeros((heads, V, K))
+        want[rows], state_want[s, ..., :K] = _exact(kind, rep(q)[rows], rep(k)[rows], d(v)[rows], d(b)[rows], d(a)[rows],
+                                                    np.exp(d(a_log)), d(bias), d(skip), S0)
+    state_want[order[0], ..., K:] = 0
+    # A sum of K products and of a chunk's tokens, and a decay per token, in fp32: a few hundred roundings of 6e-8 that add up
+    # like their root, 2e-6 of the largest value; the two forms are alike in that.
+    for out, st in got:
+        assert np.isfinite(out).all()
+        assert np.abs(out - want).max() <= 4e-6 * np.abs(want).max()
+        assert np.abs(st - state_want).max() <= 4e-6 * np.abs(state_want).max()
+    rms = [np.sqrt(((out - want) ** 2).mean()) for out, _ in got]
+    assert rms[0] <= 1.5 * rms[1] + 1e-8
