@@ -37,6 +37,8 @@ int gptoss_engine::create_rows(int rows_cap) {
 }
 
 constexpr size_t LOGITS_HALF = 2 << 20;
+constexpr size_t LOGITS_PIECE = 128 << 10;   // what a thread copies out at a time, from LOGITS_SHARED bytes on
+constexpr size_t LOGITS_SHARED = 512 << 10;
 
 int gptoss_engine::create_logits_staging() {
   GPTOSS_HIP(hipHostMalloc((void **)&h_logits, 2 * LOGITS_HALF, hipHostMallocDefault));
@@ -55,12 +57,19 @@ int gptoss_engine::copy_logits(int m, float *host_logits) {
   } piece[2] = {};
   auto take = [&](int half) -> int {
     GPTOSS_HIP(hipEventSynchronize(logits_there[half]));
-    const size_t begin = piece[half].at, end = begin + piece[half].bytes;
+    const size_t at = piece[half].at;
     const char *there = (const char *)h_logits + half * LOGITS_HALF;
-    for (size_t r = begin / stride; r * stride < end; r++) {
-      const size_t from = std::max(begin, r * stride), to = std::min(end, r * stride + row);
-      if (from < to) memcpy((char *)host_logits + r * row + (from - r * stride), there + (from - begin), to - from);
-    }
+    auto copy = [&](size_t begin, size_t end) {
+      for (size_t r = begin / stride; r * stride < end; r++) {
+        const size_t from = std::max(begin, r * stride), to = std::min(end, r * stride + row);
+        if (from < to) memcpy((char *)host_logits + r * row + (from - r * stride), there + (from - at), to - from);
+      }
+    };
+    if (total < LOGITS_SHARED) copy(at, at + piece[half].bytes);
+    else
+      crew.run((int)((piece[half].bytes + LOGITS_PIECE - 1) / LOGITS_PIECE), [&](int i) {
+        copy(at + i * LOGITS_PIECE, at + std::min(piece[half].bytes, (i + 1) * LOGITS_PIECE));
+      });
     return GPTOSS_OK;
   };
   int n = 0;

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "copy_crew.hpp"
 #include "gemm.hpp"
 #include "glue.hpp"
 #include "precise.hpp"
@@ -66,6 +67,7 @@ struct gptoss_engine {
   float *logits = nullptr;       // [max_batch, vocab_rows], only with GPTOSS_ENGINE_LOGITS
   float *h_logits = nullptr;     // pinned, two halves of LOGITS_HALF bytes: logits on their way to the caller
   hipEvent_t logits_there[2] = {nullptr, nullptr};   // a half's copy has ended
+  gptoss::CopyCrew crew;         // copies halves out
   float *amax_val = nullptr;     // [max_batch, column tiles of the classifier]: fused arg-max partials
   int *amax_idx = nullptr;
   // rows of a step
