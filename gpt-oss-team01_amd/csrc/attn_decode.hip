@@ -622,8 +622,21 @@ __global__ __launch_bounds__(256, 2) void attn_decode_resident_kernel(AttnParams
 // Every value comes from the operations, on the operands and in the order of the one-wave kernel: the same bits.
 // Calls of 16 sequences of up to 500 positions, 64 heads: 20.2 -> 13.3 us, of 3 of up to 8000: 25.0 -> 18.3 (13 of them
 // this kernel, before 21).
-template <int D>
-__global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
+//
+// ROPE: the queries, and the key and the value of the row's last position, come from the projections as they are.  A workgroup
+// rotates its own heads' queries where it would read rotated ones, and the one whose chunk has the last position puts the key
+// and the value into its operands and into the cache.  As a kernel of its own in front (rope_store_kernel, same operations,
+// same bits) that took 2.4 us of every layer of a decoding step, a launch and two waits for memory for 20 KB; here it adds 0.9
+// us to attention's 5.6 (gpt-oss-20b's shape, one sequence: 38 us of a step's 2.06 ms).  The value is put in right before the
+// second product: in front of the scores it makes them wait for all of the values too, and nothing is won (7.4 us).
+// No row may read what another of the same call stores: one row per sequence.
+struct RopeInput {
+  const float *qkv;            // [B, (n_q + 2 n_kv) D]
+  const float *cos_t, *sin_t;  // [positions, D / 2]
+  bf16_t *kv;
+};
+template <int D, bool ROPE>
+__global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p, RopeInput rope) {
   constexpr int KS = D / 32, DB = D / 16, NBLK = ATT_CHUNK / ATT_BLOCK;
   static_assert(NBLK == 8 && DB <= 4, "two blocks and at most 16 output columns per wave");
   __shared__ __attribute__((aligned(16))) u32x4 lds_p[NBLK][4][64];   // weights: hi and lo parts of 32 slots each
@@ -633,7 +646,8 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
   const int n = lane & 15, c = lane >> 4, G = p.G;
   const int g = blockIdx.x % p.n_kv, rest = blockIdx.x / p.n_kv;
   const int b = rest % p.B, chunk_id = p.max_chunks - 1 - rest / p.B;
-  const SeqRange r = seq_range(__builtin_amdgcn_readfirstlane(row_len(p, b)), p.cap, p.window, p.max_len);
+  const int length = __builtin_amdgcn_readfirstlane(row_len(p, b));
+  const SeqRange r = seq_range(length, p.cap, p.window, p.max_len);
   if (chunk_id >= r.nchunks) return;
   const int c0 = r.s_begin + chunk_id * r.chunk, c1 = min(r.s_end, c0 + r.chunk);
   const int nb = (max(0, c1 - c0) + ATT_BLOCK - 1) / ATT_BLOCK;
@@ -657,8 +671,28 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
   // cache are time on the CU's only path to it, and jumps over each are as many misses in the instruction cache.  One row
   // of 60 6.0 -> 4.8 us, 8 of 100 6.5 -> 5.3, of 300 7.8 -> 7.0.
   auto block_at = [&](int j) { return plane + (size_t)((c0 >> 6) + j) * (2 * KV_BLOCK * D); };
+  const int db = min(wave, DB - 1);   // head size 32: two waves are done after their weights
   f32x4 qx[2 * KS];
-  load_query(p.q + ((size_t)b * p.n_q + head) * D + c * KS * 8, qx);
+  // ROPE: a lane's dimensions d0 .. of a head (their partners in the rotation are those of the lane 32 further), and those of
+  // the last position's key where the wave multiplies its block
+  const int d0 = c * KS * 8;
+  f32x4 cosine[2 * KS], sine[2 * KS], kx[2 * KS];
+  float v_new = 0.f;
+  const int at = ROPE ? (length > 0 ? (length - 1) % p.cap - c0 : -1) : -1;   // the last position's place in the chunk
+  const bool fresh = ROPE && at >= 0 && c0 + at < c1;
+  if constexpr (ROPE) {
+    const float *row = rope.qkv + (size_t)b * (p.n_q + 2 * p.n_kv) * D;
+    const size_t angle = (size_t)max(length - 1, 0) * (D / 2) + (d0 & (D / 2 - 1));
+    load_query(row + head * D + d0, qx);
+    load_query(rope.cos_t + angle, cosine);
+    load_query(rope.sin_t + angle, sine);
+    if (fresh) {
+      if (at / ATT_BLOCK % 4 == wave) load_query(row + (p.n_q + g) * D + d0, kx);
+      v_new = row[(p.n_q + p.n_kv + g) * D + db * 16 + n];
+    }
+  } else {
+    load_query(p.q + ((size_t)b * p.n_q + head) * D + d0, qx);
+  }
   u32x4 kreg[2][4][KS], vreg[NBLK][2];
 #pragma unroll
   for (int u = 0; u < 2; u++) {
@@ -669,13 +703,48 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
       for (int s = 0; s < KS; s++)
         kreg[u][tb][s] = *reinterpret_cast<const u32x4 *>(block_at(wave + 4 * u) + (tb * 16 + n) * D + c * KS * 8 + s * 8);
   }
-  const int db = min(wave, DB - 1);   // head size 32: two waves are done after their weights
 #pragma unroll
   for (int j = 0; j < NBLK; j++) {
     if (j >= nb) break;
 #pragma unroll
     for (int grp = 0; grp < 2; grp++)
       vreg[j][grp] = *reinterpret_cast<const u32x4 *>(block_at(j) + KV_BLOCK * D + (grp * DB + db) * 512 + lane * 8);
+  }
+  if constexpr (ROPE) {
+    auto rotate = [&](f32x4 (&x)[2 * KS]) {
+#pragma unroll
+      for (int i = 0; i < 2 * KS; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float m = __fmul_rn(lane_xor<32>(x[i][e]), sine[i][e]);
+          x[i][e] = __fadd_rn(__fmul_rn(x[i][e], cosine[i][e]), d0 >= D / 2 ? m : -m);
+        }
+    };
+    rotate(qx);
+    if (fresh && at / ATT_BLOCK % 4 == wave) {
+      rotate(kx);
+      u32x4 key[KS];
+#pragma unroll
+      for (int s = 0; s < KS; s++)
+        key[s] = u32x4{pack_bf16x2(kx[2 * s][0], kx[2 * s][1]), pack_bf16x2(kx[2 * s][2], kx[2 * s][3]),
+                       pack_bf16x2(kx[2 * s + 1][0], kx[2 * s + 1][1]), pack_bf16x2(kx[2 * s + 1][2], kx[2 * s + 1][3])};
+      const bool mine = n == (at & 15);
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int tb = 0; tb < 4; tb++)
+          if (at >> 4 == (wave + 4 * u) * 4 + tb) {
+#pragma unroll
+            for (int s = 0; s < KS; s++)
+#pragma unroll
+              for (int w = 0; w < 4; w++) kreg[u][tb][s][w] = mine ? key[s][w] : kreg[u][tb][s][w];
+          }
+      if (mine) {
+        bf16_t *to = rope.kv + kv_block_off(seq, g, p.n_kv, p.cap, D, c0 + at) + kv_k_elem(at, d0, D);
+#pragma unroll
+        for (int s = 0; s < KS; s++) *reinterpret_cast<u32x4 *>(to + 8 * s) = key[s];
+      }
+    }
   }
   bf16x8 qh[KS], ql[KS];
   split_query<KS>(qx, n < G, qh, ql);
@@ -754,14 +823,24 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) {
     l_run = l_run * alpha[j] + lds_sum[j][lane];
 #pragma unroll
     for (int i = 0; i < 4; i++) o[i] *= alpha[j];
-    if (is_edge(blk)) {   // never-written cache memory may hold NaN bit patterns
+    const bool newest = fresh && at / ATT_BLOCK == j;
+    if (newest || is_edge(blk)) {   // never-written cache memory may hold NaN bit patterns
 #pragma unroll
       for (int grp = 0; grp < 2; grp++)
 #pragma unroll
         for (int w = 0; w < 4; w++) {
           const int s_lo = blk + grp * 32 + (w >> 1) * 16 + c * 4 + (w & 1) * 2;
           vreg[j][grp][w] &= (active(s_lo) ? 0x0000ffffu : 0u) | (active(s_lo + 1) ? 0xffff0000u : 0u);
+          if (ROPE) {
+            const uint32_t value = f32_to_bf16(v_new), x = vreg[j][grp][w];
+            const uint32_t there = x & 0xffff0000u, here = x & 0xffffu;
+            vreg[j][grp][w] = !fresh ? x : s_lo == c0 + at ? there | value : s_lo + 1 == c0 + at ? here | value << 16 : x;
+          }
         }
+      if (newest) {
+        const int d = db * 16 + n;
+        if (c == ((at >> 2) & 3)) rope.kv[kv_block_off(seq, g, p.n_kv, p.cap, D, c0 + at) + kv_v_elem(at, d, D)] = f32_to_bf16(v_new);
+      }
     }
 #pragma unroll
     for (int grp = 0; grp < 2; grp++) {
@@ -1215,7 +1294,7 @@ static int attn_launch(const float *q, const void *kv_cache, const int *lens,
                        const float *sinks, void *out, int B, int rows_per_seq, int n_q, int n_kv,
                        int head_dim, int capacity, int window, int max_len, void *workspace,
                        size_t workspace_bytes, void *stream, int len_base = 0, int len_period = 0,
-                       const int *seq_map = nullptr) {
+                       const int *seq_map = nullptr, const RopeInput *rope = nullptr) {
   GPTOSS_REQUIRE(q && kv_cache && out, GPTOSS_ERR_NULL, "attn_decode: null pointer");
   if (!lens && len_base == 0) len_base = max_len;  // no lengths given: every row has max_len positions
   GPTOSS_REQUIRE(B > 0 && n_q > 0 && n_kv > 0 && n_q % n_kv == 0 && n_q / n_kv <= 16, GPTOSS_ERR_DIM,
@@ -1290,8 +1369,9 @@ static int attn_launch(const float *q, const void *kv_cache, const int *lens,
       if (rc != GPTOSS_OK) return rc;
     }
     if (few) {
-      if (head_dim == 64) attn_few_kernel<64><<<(int)items, 256, 0, s>>>(p);
-      else attn_few_kernel<32><<<(int)items, 256, 0, s>>>(p);
+      auto launch = [&](auto kernel) { kernel<<<(int)items, 256, 0, s>>>(p, rope ? *rope : RopeInput{}); };
+      if (rope) launch(head_dim == 64 ? attn_few_kernel<64, true> : attn_few_kernel<32, true>);
+      else launch(head_dim == 64 ? attn_few_kernel<64, false> : attn_few_kernel<32, false>);
     } else if (head_dim == 64) {
       if (pair) attn_decode_kernel<64, true><<<grid, 256, 0, s>>>(p);
       else if (hold_rows) attn_decode_resident_kernel<64><<<std::min(grid, resident), 256, 0, s>>>(p, grid);
@@ -1333,11 +1413,24 @@ extern "C" int gptoss_attn_decode(const float *q, const void *kv_cache, const in
                      max_len, workspace, workspace_bytes, stream);
 }
 
-int gptoss::attn_decode_mapped(const float *q, const void *kv_cache, const int *lens, const float *sinks, void *out,
-                               int B, int n_q, int n_kv, int head_dim, int capacity, int window, int max_len,
-                               void *workspace, size_t workspace_bytes, void *stream, const int *seq_map) {
+int gptoss::attn_decode_rope(const float *qkv, float *q, const float *cos_t, const float *sin_t, void *kv_cache,
+                             const int *lens, const float *sinks, void *out, int B, bool own_sequences, int n_q, int n_kv,
+                             int head_dim, int capacity, int window, int max_len, void *workspace, size_t workspace_bytes,
+                             void *stream, const int *seq_map) {
+  const int span = max_len > capacity ? capacity : window > 0 && window < max_len ? window : max_len;
+  const bool here = own_sequences && (head_dim == 32 || head_dim == 64) && n_kv > 0 && n_q % n_kv == 0 &&
+                    !attn_plan(B, 1, n_q, n_kv, head_dim, span).wide && attn_few((long long)B * n_kv, span, head_dim) &&
+                    aligned(qkv, 16) && aligned(cos_t, 16) && aligned(sin_t, 16);
+  const RopeInput rope{qkv, cos_t, sin_t, (bf16_t *)kv_cache};
+  if (!here) {
+    const int rc = lens ? run_rope_store_lens(qkv, q, (bf16_t *)kv_cache, cos_t, sin_t, B, n_q, n_kv, head_dim, capacity, lens,
+                                              (hipStream_t)stream, seq_map)
+                        : run_rope_store(qkv, q, (bf16_t *)kv_cache, cos_t, sin_t, B, n_q, n_kv, head_dim, capacity, max_len - 1,
+                                         (hipStream_t)stream);
+    if (rc != GPTOSS_OK) return rc;
+  }
   return attn_launch(q, kv_cache, lens, sinks, out, B, 1, n_q, n_kv, head_dim, capacity, window, max_len, workspace,
-                     workspace_bytes, stream, 0, 0, seq_map);
+                     workspace_bytes, stream, 0, 0, seq_map, here ? &rope : nullptr);
 }
 
 // ---- the same call without a caller workspace ---------------------------------------------------

@@ -42,11 +42,12 @@ int run_rope_store_rows(const float *qkv, float *q_out, bf16_t *kv, const float 
 int run_rope_store_lens(const float *qkv, float *q_out, bf16_t *kv, const float *cos_t,
                         const float *sin_t, int B, int n_q, int n_kv, int D, int cap, const int *lens,
                         hipStream_t s, const int *seq_map = nullptr);
-// attn_decode.hip: gptoss_attn_decode with row b reading the cache of sequence seq_map[b] (device
-// array) up to lens[b]
-int attn_decode_mapped(const float *q, const void *kv_cache, const int *lens, const float *sinks, void *out, int B,
-                       int n_q, int n_kv, int head_dim, int capacity, int window, int max_len, void *workspace,
-                       size_t workspace_bytes, void *stream, const int *seq_map);
+// attn_decode.hip: run_rope_store (lens: run_rope_store_lens) into q and the cache, then gptoss_attn_decode with row b reading
+// the cache of sequence seq_map[b] (device array; nullptr: b) up to lens[b] (nullptr: max_len).  own_sequences: no two rows are
+// of one sequence; both may then be one kernel, which leaves q as it was.
+int attn_decode_rope(const float *qkv, float *q, const float *cos_t, const float *sin_t, void *kv_cache, const int *lens,
+                     const float *sinks, void *out, int B, bool own_sequences, int n_q, int n_kv, int head_dim, int capacity,
+                     int window, int max_len, void *workspace, size_t workspace_bytes, void *stream, const int *seq_map);
 // dst[i, :] = src[idx[i], :]
 int run_gather_rows_idx(const float *src, float *dst, const int *idx, int rows, int n, hipStream_t s);
 // dst[i, :] = src[i * stride + offset, :]

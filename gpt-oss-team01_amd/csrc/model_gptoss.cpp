@@ -522,15 +522,9 @@ int GptOss::step(const int *host_tokens, int pos, const int *host_pos, int B, in
     const LayerWeights &w = e->layers[l];
     if (l == 0) STEP(run_rmsnorm(e->x, nullptr, w.attn_norm, e->t, nullptr, B, H, s));
     STEP(dense_gemm(e->t, w.w_qkv, w.b_qkv, e->qkv, EPI_F32, B, qkv_dim, H, s));
-    if (host_pos)
-      STEP(run_rope_store_lens(e->qkv, e->q, w.kv_cache, e->cos_t, e->sin_t, B, nq, nkv, D,
-                               w.cache_cap, e->d_lens, s));
-    else
-      STEP(run_rope_store(e->qkv, e->q, w.kv_cache, e->cos_t, e->sin_t, B, nq, nkv, D,
-                          w.cache_cap, pos, s));
     // lock step: every sequence has pos + 1 positions, which the call takes from max_len
-    STEP(gptoss_attn_decode(e->q, w.kv_cache, host_pos ? e->d_lens : nullptr, w.sinks, e->attn_out, B, nq, nkv, D,
-                            w.cache_cap, w.window, pos + 1, e->attn_ws, e->attn_ws_bytes, s));
+    STEP(attn_decode_rope(e->qkv, e->q, e->cos_t, e->sin_t, w.kv_cache, host_pos ? e->d_lens : nullptr, w.sinks, e->attn_out, B,
+                          true, nq, nkv, D, w.cache_cap, w.window, pos + 1, e->attn_ws, e->attn_ws_bytes, s, nullptr));
     STEP(dense_gemm(e->attn_out, w.w_o, w.b_o, e->tb2, EPI_F32, B, H, nq * D, s));
     // x += attention branch, then the ffn norm (model.cpp:66)
     const MoePreNorm pre{e->x, e->tb2, w.mlp_norm};   // runs inside the block's router kernel
@@ -689,10 +683,9 @@ int GptOss::forward_rows(const StepRows &r) {
     const LayerWeights &w = e->layers[l];
     if (l == 0) GPTOSS_STEP(run_rmsnorm(rows_x, nullptr, w.attn_norm, pf.t, nullptr, n, H, s));
     GPTOSS_STEP(dense_gemm(pf.t, w.w_qkv, w.b_qkv, pf.qkv, EPI_F32, n, qkv_dim, H, s));
-    GPTOSS_STEP(run_rope_store_lens(pf.qkv, pf.q, w.kv_cache, e->cos_t, e->sin_t, n, nq, nkv, D, w.cache_cap, r.lens, s,
-                             r.slots));
-    GPTOSS_STEP(attn_decode_mapped(pf.q, w.kv_cache, r.lens, w.sinks, pf.attn_out, n, nq, nkv, D, w.cache_cap, w.window,
-                            r.max_len, pf.attn_ws, pf.attn_ws_bytes, s, r.slots));
+    GPTOSS_STEP(attn_decode_rope(pf.qkv, pf.q, e->cos_t, e->sin_t, w.kv_cache, r.lens, w.sinks, pf.attn_out, n,
+                                 r.n_seg == n, nq, nkv, D, w.cache_cap, w.window, r.max_len, pf.attn_ws, pf.attn_ws_bytes, s,
+                                 r.slots));
     GPTOSS_STEP(dense_gemm(pf.attn_out, w.w_o, w.b_o, pf.tb2, EPI_F32, n, H, nq * D, s));
     const MoePreNorm pre{rows_x, pf.tb2, w.mlp_norm};   // runs inside the block's router kernel
     gptoss_moe_weights mw;

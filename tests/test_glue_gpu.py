@@ -288,3 +288,39 @@ def test_embedding_rows(ops, dtype, H, ld, with_positions):
             want[:, :H] += positions[(lens.long() - 1).clamp(0, n_pos - 1)].float()
             assert torch.equal(x0, want)
         assert torch.equal(x, want), shift
+
+
+# lengths at the edges of 16-slot rows, blocks, chunks; one and two chunks; a ring that has wrapped; an empty sequence
+@pytest.mark.parametrize("D,n_q,n_kv,cap,window,lens", [
+    (64, 64, 8, 576, 0, (1, 16, 17, 63, 64)), (64, 16, 2, 1088, 0, (65, 512, 513, 0, 577, 1088)), (64, 4, 4, 192, 128, (128, 129, 190)),
+    (64, 16, 1, 128, 128, (127, 128, 129, 300, 384)), (32, 24, 3, 640, 0, (5, 33, 600)), (32, 8, 8, 64, 64, (64, 65, 200)),
+])
+def test_rotation_within_the_attention_equals_that_in_front_of_it(ops, D, n_q, n_kv, cap, window, lens):
+    """gptoss::attn_decode_rope by its linker name: one kernel where no two rows are of one sequence, two otherwise."""
+    import ctypes as C
+    from conftest import load_pkg
+    f = load_pkg("lib").load()._ZN6gptoss16attn_decode_ropeEPKfPfS1_S1_PvPKiS1_S3_ibiiiiiiS3_mS3_S5_
+    p, i = C.c_void_p, C.c_int
+    f.argtypes = [p, p, p, p, p, p, p, p, i, C.c_bool, i, i, i, i, i, i, p, C.c_size_t, p, p]
+    g = torch.Generator(device="cuda").manual_seed(D + cap)
+    B, slots = len(lens), len(lens) + 2
+    qkv = torch.randn(B, (n_q + 2 * n_kv) * D, device="cuda", generator=g)
+    angle = torch.rand(1200, D // 2, device="cuda", generator=g) * 6.3
+    cos, sin, sinks = angle.cos(), angle.sin(), torch.randn(n_q, device="cuda", generator=g)
+    filled = torch.randn(slots * n_kv * cap * 2 * D, device="cuda", generator=g).to(torch.bfloat16)
+    lens_t = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    seq_map = torch.randperm(slots, device="cuda", generator=g)[:B].to(torch.int32)
+    ws = torch.empty(1 << 24, dtype=torch.uint8, device="cuda")
+    got = []
+    for own in (False, True):
+        kv, out = filled.clone(), torch.zeros(B, n_q, D, dtype=torch.bfloat16, device="cuda")
+        q = torch.full((B, n_q, D), 7.0, device="cuda")
+        torch.cuda.synchronize()
+        assert f(qkv.data_ptr(), q.data_ptr(), cos.data_ptr(), sin.data_ptr(), kv.data_ptr(), lens_t.data_ptr(), sinks.data_ptr(),
+                 out.data_ptr(), B, own, n_q, n_kv, D, cap, window, max(lens), ws.data_ptr(), ws.numel(), None,
+                 seq_map.data_ptr()) == 0
+        torch.cuda.synchronize()
+        assert bool((q == 7.0).all()) == own            # the queries in front of it go through memory
+        got.append((out, kv))
+    assert torch.equal(got[0][0].view(torch.int16), got[1][0].view(torch.int16))
+    assert torch.equal(got[0][1].view(torch.int16), got[1][1].view(torch.int16)) and not torch.equal(filled, got[1][1])
