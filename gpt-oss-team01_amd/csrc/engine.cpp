@@ -10,7 +10,7 @@ gptoss_engine::~gptoss_engine() {
   for (void *p : allocs) (void)hipFree(p);
   if (h_next) (void)hipHostFree(h_next);
   if (h_logits) (void)hipHostFree(h_logits);
-  for (hipEvent_t e : logits_there)
+  for (hipEvent_t e : logits_out)
     if (e) (void)hipEventDestroy(e);
   if (h_rows) (void)hipHostFree(h_rows);
   if (stream) (void)hipStreamDestroy(stream);
@@ -39,47 +39,70 @@ int gptoss_engine::create_rows(int rows_cap) {
 constexpr size_t LOGITS_HALF = 2 << 20;
 constexpr size_t LOGITS_PIECE = 128 << 10;   // what a thread copies out at a time, from LOGITS_SHARED bytes on
 constexpr size_t LOGITS_SHARED = 512 << 10;
+constexpr int LOGITS_CHUNKS = LOGITS_HALF / LOGITS_CHUNK;
+constexpr int LOGITS_SPINS = 20000;   // looks at a chunk's word, about a millisecond, before the thread waits for the kernel's end
 
 int gptoss_engine::create_logits_staging() {
-  GPTOSS_HIP(hipHostMalloc((void **)&h_logits, 2 * LOGITS_HALF, hipHostMallocDefault));
-  for (hipEvent_t &e : logits_there) GPTOSS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  GPTOSS_HIP(hipHostMalloc((void **)&h_logits, 2 * LOGITS_HALF + 2 * LOGITS_CHUNKS * sizeof(uint32_t), hipHostMallocCoherent));
+  logits_there = (uint32_t *)((char *)h_logits + 2 * LOGITS_HALF);
+  for (hipEvent_t &e : logits_out) GPTOSS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   return GPTOSS_OK;
 }
 
-// The first m rows of the logits to the caller's array, through the pinned halves in turn: a half travels while the one
-// before is copied out.  (Into the caller's own pages the runtime pins them, or bounces, at every call: one row of a
-// vocabulary of 201088 took 180 us behind its step.)  Rows travel with their padding, one behind the other, and lose it on
-// the host: a copy for each row of a padded vocabulary costs 8 us (512 rows of 1000 logits: 4.1 ms instead of 0.2).
+// The first m rows of the logits, soft-capped where the model says so, to the caller's array, through the pinned halves in
+// turn: a kernel writes a half chunk by chunk, and a chunk is copied out as soon as its word says that it is there.  (Into the
+// caller's own pages the runtime pins them, or bounces, at every call: one row of a vocabulary of 201088 took 180 us behind its
+// step.  Its copies into pinned memory begin 11 us behind the kernel in front, each of them.)  Rows travel with their padding,
+// one behind the other, and lose it on the host: a copy for each row of a padded vocabulary costs 8 us (512 rows of 1000 logits:
+// 4.1 ms instead of 0.2).
 int gptoss_engine::copy_logits(int m, float *host_logits) {
   const size_t row = sizeof(float) * vocab, stride = sizeof(float) * vocab_rows, total = stride * m;
   struct Piece {
     size_t at, bytes;   // of the device's rows
   } piece[2] = {};
   auto take = [&](int half) -> int {
-    GPTOSS_HIP(hipEventSynchronize(logits_there[half]));
-    const size_t at = piece[half].at;
+    const size_t at = piece[half].at, bytes = piece[half].bytes;
     const char *there = (const char *)h_logits + half * LOGITS_HALF;
-    auto copy = [&](size_t begin, size_t end) {
-      for (size_t r = begin / stride; r * stride < end; r++) {
-        const size_t from = std::max(begin, r * stride), to = std::min(end, r * stride + row);
-        if (from < to) memcpy((char *)host_logits + r * row + (from - r * stride), there + (from - at), to - from);
+    std::atomic<int> failed{hipSuccess};
+    auto wait = [&](size_t chunk) {
+      const uint32_t *word = logits_there + half * LOGITS_CHUNKS + chunk;
+      for (int i = 0; i < LOGITS_SPINS; i++) {
+        if (__atomic_load_n(word, __ATOMIC_ACQUIRE)) return;
+        __builtin_ia32_pause();
+      }
+      const hipError_t err = hipEventSynchronize(logits_out[half]);
+      if (err != hipSuccess) failed = err;
+    };
+    auto copy = [&](int i) {
+      const size_t first = at + i * LOGITS_PIECE, last = at + std::min(bytes, (i + 1) * LOGITS_PIECE);
+      for (size_t begin = first; begin < last && failed == hipSuccess; begin += LOGITS_CHUNK) {
+        const size_t end = std::min(last, begin + LOGITS_CHUNK);
+        wait((begin - at) / LOGITS_CHUNK);
+        for (size_t r = begin / stride; r * stride < end; r++) {
+          const size_t from = std::max(begin, r * stride), to = std::min(end, r * stride + row);
+          if (from < to) memcpy((char *)host_logits + r * row + (from - r * stride), there + (from - at), to - from);
+        }
       }
     };
-    if (total < LOGITS_SHARED) copy(at, at + piece[half].bytes);
+    wait(0);   // (the crew stays asleep until then)
+    const int n = (int)((bytes + LOGITS_PIECE - 1) / LOGITS_PIECE);
+    if (total < LOGITS_SHARED)
+      for (int i = 0; i < n; i++) copy(i);
     else
-      crew.run((int)((piece[half].bytes + LOGITS_PIECE - 1) / LOGITS_PIECE), [&](int i) {
-        copy(at + i * LOGITS_PIECE, at + std::min(piece[half].bytes, (i + 1) * LOGITS_PIECE));
-      });
+      crew.run(n, copy);
+    GPTOSS_HIP((hipError_t)failed.load());
     return GPTOSS_OK;
   };
   int n = 0;
   for (size_t at = 0; at < total; n++) {
-    if (n >= 2) GPTOSS_STEP(take(n & 1));
-    piece[n & 1] = {at, std::min(LOGITS_HALF, total - at)};
-    GPTOSS_HIP(hipMemcpyAsync((char *)h_logits + (n & 1) * LOGITS_HALF, (char *)logits + at, piece[n & 1].bytes,
-                              hipMemcpyDeviceToHost, stream));
-    GPTOSS_HIP(hipEventRecord(logits_there[n & 1], stream));
-    at += piece[n & 1].bytes;
+    const int half = n & 1;
+    if (n >= 2) GPTOSS_STEP(take(half));
+    piece[half] = {at, std::min(LOGITS_HALF, total - at)};
+    std::fill_n(logits_there + half * LOGITS_CHUNKS, LOGITS_CHUNKS, 0u);
+    GPTOSS_STEP(run_logits_out(logits + at / sizeof(float), h_logits + half * (LOGITS_HALF / sizeof(float)),
+                               piece[half].bytes / sizeof(float), logit_softcap, logits_there + half * LOGITS_CHUNKS, stream));
+    GPTOSS_HIP(hipEventRecord(logits_out[half], stream));
+    at += piece[half].bytes;
   }
   for (int i = std::max(0, n - 2); i < n; i++) GPTOSS_STEP(take(i & 1));
   return GPTOSS_OK;
@@ -157,7 +180,7 @@ int gptoss_engine::upload_rows(int n, const int *tok, const int *slot, const int
   const size_t o_smp = take(n_sample);
   if (n_sample) memcpy(h_rows + o_smp, sample, sizeof(int) * n_sample);
   GPTOSS_REQUIRE(used <= row_ints, GPTOSS_ERR_STATE, "engine: row block of %zu ints exceeds %zu", used, row_ints);
-  GPTOSS_HIP(hipMemcpyAsync(d_rows, h_rows, sizeof(int) * used, hipMemcpyHostToDevice, stream));
+  GPTOSS_STEP(run_rows_in(d_rows, h_rows, used, stream));
   r.tokens = d_rows + o_tok;
   r.slots = d_rows + o_slot;
   r.lens = d_rows + o_len;
@@ -219,7 +242,6 @@ int gptoss_engine::run_rows(int n, const int *tok, const int *slot, const int *p
     GPTOSS_STEP(norm_sampled(m));
     if (host_logits) {
       GPTOSS_STEP(class_gemm(0, m, logits));
-      if (logit_softcap > 0.f) GPTOSS_STEP(run_softcap(logits, (size_t)m * vocab_rows, logit_softcap, stream));
       GPTOSS_STEP(copy_logits(m, host_logits + (size_t)first * vocab));   // (the buffer is reused by the next portion)
     } else {
       GPTOSS_STEP(sample_rows(r, sample, slot, first, m));

@@ -65,8 +65,9 @@ struct gptoss_engine {
   gptoss::bf16_t *t = nullptr;   // [max_batch, hidden]
   float *t_f32 = nullptr;        // likewise, GPTOSS_ENGINE_PRECISE
   float *logits = nullptr;       // [max_batch, vocab_rows], only with GPTOSS_ENGINE_LOGITS
-  float *h_logits = nullptr;     // pinned, two halves of LOGITS_HALF bytes: logits on their way to the caller
-  hipEvent_t logits_there[2] = {nullptr, nullptr};   // a half's copy has ended
+  float *h_logits = nullptr;     // pinned, two halves of LOGITS_HALF bytes: logits on their way to the caller; their words
+  uint32_t *logits_there = nullptr;   // pinned: a word for each chunk of the halves, 1 once it can be read
+  hipEvent_t logits_out[2] = {nullptr, nullptr};   // a half's kernel has ended
   gptoss::CopyCrew crew;         // copies halves out
   float *amax_val = nullptr;     // [max_batch, column tiles of the classifier]: fused arg-max partials
   int *amax_idx = nullptr;

@@ -715,6 +715,41 @@ __global__ __launch_bounds__(256) void residual_tanh_norm_kernel(float *__restri
   if (t_f32) *reinterpret_cast<f32x4 *>(t_f32 + at) = o;
 }
 
+// Logits into pinned host memory, LOGITS_CHUNK bytes a workgroup at a time, and behind each chunk its word in `there`: the host
+// copies a chunk out while the next ones travel.  cap > 0: soft-capped on the way, in z as well.  Bound by PCIe.  Netinex, a
+// step of 12 sequences and its 3 MB of logits: 584 us, with the soft-cap's kernel and the runtime's copies 620 (11 us before
+// each); 32 KB a chunk 601, 8 KB 598, 8 / 16 / 64 / 128 workgroups 641 / 590 / 585 / 601.  One sequence 479 -> 461.
+__global__ __launch_bounds__(256) void logits_out_kernel(float *__restrict__ z, float *__restrict__ host, size_t n, float cap,
+                                                         uint32_t *__restrict__ there) {
+  constexpr int ELEMS = LOGITS_CHUNK / sizeof(float), STEPS = ELEMS / 1024;
+  for (size_t chunk = blockIdx.x; chunk * ELEMS < n; chunk += gridDim.x) {
+    f32x4 v[STEPS];
+    const size_t at = chunk * ELEMS + threadIdx.x * 4;
+#pragma unroll
+    for (int i = 0; i < STEPS; i++)
+      if (at + i * 1024 < n) v[i] = *reinterpret_cast<const f32x4 *>(z + at + i * 1024);
+#pragma unroll
+    for (int i = 0; i < STEPS; i++)
+      if (at + i * 1024 < n) {
+        if (cap > 0.f) {
+#pragma unroll
+          for (int q = 0; q < 4; q++) v[i][q] = cap * tanhf(v[i][q] / cap);
+          *reinterpret_cast<f32x4 *>(z + at + i * 1024) = v[i];
+        }
+        *reinterpret_cast<f32x4 *>(host + at + i * 1024) = v[i];
+      }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's own stores, before the word that speaks for them all
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(there + chunk, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// A step's row block from pinned host memory.
+__global__ __launch_bounds__(256) void rows_in_kernel(u32x4 *__restrict__ to, const u32x4 *__restrict__ host, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) to[i] = host[i];
+}
+
 __global__ __launch_bounds__(256) void softcap_kernel(float *__restrict__ z, size_t n, float cap) {
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
     z[i] = cap * tanhf(z[i] / cap);
@@ -734,6 +769,25 @@ int run_softcap(float *z, size_t n, float cap, hipStream_t s) {
   TraceScope ts("softcap", s);
   softcap_kernel<<<grid_for(n), 256, 0, s>>>(z, n, cap);
   GPTOSS_LAUNCH_CHECK("softcap_kernel");
+  return GPTOSS_OK;
+}
+
+int run_logits_out(float *z, float *host, size_t n, float cap, uint32_t *there, hipStream_t s) {
+  GPTOSS_REQUIRE(n % 4 == 0 && aligned(z, 16) && aligned(host, 16), GPTOSS_ERR_DIM, "logits_out: %zu logits (a multiple of 4)", n);
+  TraceScope ts("logits_out", s);
+  constexpr size_t ELEMS = LOGITS_CHUNK / sizeof(float);
+  logits_out_kernel<<<(unsigned)std::min<size_t>(LOGITS_OUT_WGS, (n + ELEMS - 1) / ELEMS), 256, 0, s>>>(z, host, n, cap, there);
+  GPTOSS_LAUNCH_CHECK("logits_out_kernel");
+  return GPTOSS_OK;
+}
+
+int run_rows_in(int *to, const int *host, size_t n, hipStream_t s) {
+  GPTOSS_REQUIRE(n % 4 == 0 && n / 4 < (1u << 30) && aligned(to, 16) && aligned(host, 16), GPTOSS_ERR_DIM,
+                 "rows_in: %zu ints (a multiple of 4)", n);
+  TraceScope ts("rows_in", s);
+  const int quads = (int)(n / 4);
+  rows_in_kernel<<<cdiv(quads, 256), 256, 0, s>>>((u32x4 *)to, (const u32x4 *)host, quads);
+  GPTOSS_LAUNCH_CHECK("rows_in_kernel");
   return GPTOSS_OK;
 }
 

@@ -19,6 +19,12 @@ int run_residual_tanh_norm(float *x, const float *y, int parts, const TanhNorm &
                            int rows, int H, hipStream_t s);
 // z = cap * tanh(z / cap)
 int run_softcap(float *z, size_t n, float cap, hipStream_t s);
+// n logits to pinned host memory, soft-capped (there and in z) where cap > 0; there[i] becomes 1 once chunk i of LOGITS_CHUNK
+// bytes can be read on the host
+constexpr int LOGITS_CHUNK = 16 << 10, LOGITS_OUT_WGS = 32;
+int run_logits_out(float *z, float *host, size_t n, float cap, uint32_t *there, hipStream_t s);
+// a step's row block from pinned host memory (n ints, a multiple of 4)
+int run_rows_in(int *to, const int *host, size_t n, hipStream_t s);
 // x = x0 = table[token] + positions[lens - 1], rows of stride ld (zero from column H on); positions and x0 may be null
 int run_embedding_position(const bf16_t *table, const bf16_t *positions, const int *tokens, const int *lens, float *x,
                            float *x0, int rows, int H, int ld, int V, int n_pos, hipStream_t s);
