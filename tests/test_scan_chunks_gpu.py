@@ -1,4 +1,4 @@
-"""The delta rule and the state-space recurrence in chunks on the matrix cores, and token by token, against the recurrence in
+"""The delta rules and the state-space recurrence in chunks on the matrix cores, and token by token, against the recurrence in
 64 bits: gptoss::run_scan_chunks and gptoss::run_scan by their linker names, at the edges of chunks, key and column blocks."""
 import ctypes as C
 
@@ -10,7 +10,7 @@ from conftest import load_pkg
 
 pytestmark = pytest.mark.gpu
 
-DELTA, STATE_SPACE = 0, 2
+DELTA, CHANNEL_DELTA, STATE_SPACE = 0, 1, 2
 
 
 def _struct(name, *fields):
@@ -36,10 +36,10 @@ def _exact(kind, q, k, v, b, a, rate, bias, skip, S):
     """-> outputs [T, H, V], state [H, V, K], from state S, in float64."""
     T, H, V = v.shape
     out, dt = np.zeros((T, H, V)), _softplus(a + bias)
-    decay = np.exp(-rate * dt)
+    decay = np.exp(-rate.reshape(H, 1) * dt.reshape(T, H, -1))   # one, or one per key channel
     for t in range(T):
-        S = S * decay[t][:, None, None]
-        if kind == DELTA:
+        S = S * decay[t][:, None, :]
+        if kind != STATE_SPACE:
             u = (v[t] - np.einsum("hvk,hk->hv", S, k[t])) / (1 + np.exp(-b[t]))[:, None]
         else:
             u = dt[t][:, None] * v[t]
@@ -49,29 +49,33 @@ def _exact(kind, q, k, v, b, a, rate, bias, skip, S):
 
 
 @pytest.mark.parametrize("strong", [False, True])
-@pytest.mark.parametrize("kind", [DELTA, STATE_SPACE])
+@pytest.mark.parametrize("kind", [DELTA, CHANNEL_DELTA, STATE_SPACE])
 @pytest.mark.parametrize("heads,key_heads,K,V,lengths", [
     (2, 1, 4, 5 * 4, (48, 1, 49)),          # one key block of which an eighth is there; a token beside the stretches
     (4, 2, 36, 68, (64, 65, 31)),           # two column blocks, the second of four columns
     (2, 2, 128, 64, (95, 96, 97, 32, 33)),
     (1, 1, 132, 128, (50,)),
+    (2, 1, 160, 20, (63, 17, 48)),
     (2, 1, 256, 16, (129, 15, 16, 17)),     # the largest keys
     (6, 3, 64, 64, (70,) + 100 * (1,)),     # more single tokens than workgroups run at a time
 ])
 def test_chunks_equal_the_recurrence(kind, strong, heads, key_heads, K, V, lengths):
+    if kind == CHANNEL_DELTA and K > 160:
+        pytest.skip("token by token only")
     g = np.random.default_rng(K + V + kind)
     n, slots, KP = sum(lengths), len(lengths), (K + 31) // 32 * 32
     unit = lambda x: x / np.sqrt((x * x).sum(-1, keepdims=True))
     q, k = unit(g.standard_normal((n, key_heads, K))) / np.sqrt(K), unit(g.standard_normal((n, key_heads, K)))
     v = g.standard_normal((n, heads, V))
-    b, a = g.standard_normal((n, heads)), g.standard_normal((n, heads))
-    a_log, bias, skip = g.uniform(-5, -.5, heads) + 4.5 * strong, g.standard_normal(heads), g.standard_normal(heads)
+    channels = (heads, K) if kind == CHANNEL_DELTA else (heads,)
+    b, a = g.standard_normal((n, heads)), g.standard_normal((n, *channels))
+    a_log, bias, skip = g.uniform(-5, -.5, heads) + 4.5 * strong, g.standard_normal(channels), g.standard_normal(heads)
     state = np.zeros((slots, heads, V, KP))
     state[..., :K] = g.standard_normal((slots, heads, V, K)) * 0.1
     f32 = lambda x: np.ascontiguousarray(x, np.float32)
     q, k, v, b, a, a_log, bias, skip, state = map(f32, (q, k, v, b, a, a_log, bias, skip, state))
     conv = np.concatenate([q.reshape(n, -1), k.reshape(n, -1), v.reshape(n, -1)], axis=1)
-    inp = np.concatenate([b, a], axis=1)
+    inp = np.concatenate([b, a.reshape(n, -1)], axis=1)
     order = g.permutation(slots)               # slots in another order than the stretches; the first starts from nothing
     at = np.concatenate([[0], np.cumsum(lengths)])[:-1]
     segs = np.array([(r, m, s, 0 if i == 0 else 7) for i, (r, m, s) in enumerate(zip(at, lengths, order))], np.int32)
@@ -88,7 +92,8 @@ def test_chunks_equal_the_recurrence(kind, strong, heads, key_heads, K, V, lengt
                  "_ZN6gptoss8run_scanERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t"):
         st, out = torch.from_numpy(state).cuda(), torch.full((n, heads * V), np.nan, device="cuda")
         p = Scan(kind=kind, heads=heads, key_heads=key_heads, K=K, V=V, conv=dev(conv), ld_conv=conv.shape[1], q_col=0, k_col=nk,
-                 v_col=2 * nk, inp=dev(inp), ld_in=2 * heads, beta_col=0, decay_col=heads, a_log=dev(a_log), dt_bias=dev(bias),
+                 v_col=2 * nk, inp=dev(inp), ld_in=inp.shape[1], beta_col=0, decay_col=heads,
+                 channel_decay=dev(a) if kind == CHANNEL_DELTA else None, ld_decay=heads * K, a_log=dev(a_log), dt_bias=dev(bias),
                  d_skip=dev(skip), value_scale=1.0, state=st.data_ptr(), out=out.data_ptr(), ld_out=heads * V)
         singles = segs[segs[:, 1] == 1]
         r = StepRows(n=n, n_seg=slots, segs=dev(segs), singles=dev(singles) if len(singles) else None, n_singles=len(singles),
