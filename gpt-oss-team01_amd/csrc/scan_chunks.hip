@@ -59,6 +59,27 @@ __device__ __forceinline__ double prefix32(double v) {
   return v;
 }
 
+// What tokens write, where some of it is not finite.  A product with a whole tile would take its zeros above the diagonal times
+// an infinity and give every token of the chunk no number, those in front of the infinity too; here only the tokens in front of
+// a token (own: and it itself) give it something.
+__device__ __forceinline__ bool any_not_finite(float sum) { return __ballot(sum * 0.f != 0.f) != 0; }
+__device__ __forceinline__ f32x4 tile_below(f32x4 acc, const float *a, f32x4 b, bool own, int lane) {
+  const int n = lane & 15, c = lane >> 4;
+#pragma unroll 1
+  for (int g = 0; g < 4; g++)
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+      const int s = 4 * g + f;
+      const float from = __shfl(b[f], g * 16 + n);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int t = 4 * c + e;
+        if (s < t || (own && s == t)) acc[e] = fmaf(a[(g * 16 + t) * 4 + f], from, acc[e]);
+      }
+    }
+  return acc;
+}
+
 // The inverse of I + A, A a strictly lower triangular tile of 16x16 ((s >> 2, t, s & 3), s < t), by columns: lane n (< 16) has
 // column n.  What a row of the inverse gives the later ones is taken off all of them at once, four columns of A in registers at
 // a time (AHEAD: the next four requested meanwhile).
@@ -176,7 +197,9 @@ __global__ __launch_bounds__(256, NI <= 4 ? 2 : 1) void scan_chunk_kernel(Scan p
     const int t = lane & 31;
     const bool real = t0 + t < seg.n;
     const float dt = softplus_f(r_decay + bias);
-    const double cum = prefix32(real ? (double)(-rate * dt) : 0.0), all = __shfl(cum, 31);
+    // (Past e^-200, which is zero, no further: the differences behind an infinite sum would be no numbers.)
+    const float log_decay = -rate * dt < -200.f ? -200.f : -rate * dt;
+    const double cum = prefix32(real ? (double)log_decay : 0.0), all = __shfl(cum, 31);
     if (lane < 32) {
       reinterpret_cast<double *>(lds + L::CUM)[stage * CHUNK + t] = cum;
       lds[L::FROM + stage * CHUNK + t] = exp_f((float)cum);
@@ -309,14 +332,26 @@ __global__ __launch_bounds__(256, NI <= 4 ? 2 : 1) void scan_chunk_kernel(Scan p
       return acc;
     };
     const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 w[2] = {u[0], u[1]};
     if constexpr (DELTA) {
-      u[0] = tile(zero, lds + L::INV, u[0]);
-      u[1] -= tile(zero, lds + L::A + 256, u[0]);
-      u[1] = tile(zero, lds + L::INV + 256, u[1]);
+      w[0] = tile(zero, lds + L::INV, u[0]);
+      w[1] = tile(zero, lds + L::INV + 256, u[1] - tile(zero, lds + L::A + 256, w[0]));
     }
-    o[0] = tile(o[0], lds + L::P, u[0]);
-    o[1] = tile(o[1], lds + L::P + 256, u[0]);
-    o[1] = tile(o[1], lds + L::P + 512, u[1]);
+    const f32x4 sum = w[0] + w[1];
+    if (any_not_finite(sum[0] + sum[1] + sum[2] + sum[3])) {
+      if constexpr (DELTA) {
+        w[0] = tile_below(zero, lds + L::INV, u[0], true, lane);
+        w[1] = tile_below(zero, lds + L::INV + 256, u[1] - tile(zero, lds + L::A + 256, w[0]), true, lane);
+      }
+      o[0] = tile_below(o[0], lds + L::P, w[0], true, lane);
+      o[1] = tile_below(tile(o[1], lds + L::P + 256, w[0]), lds + L::P + 512, w[1], true, lane);
+    } else {
+      o[0] = tile(o[0], lds + L::P, w[0]);
+      o[1] = tile(o[1], lds + L::P + 256, w[0]);
+      o[1] = tile(o[1], lds + L::P + 512, w[1]);
+    }
+#pragma unroll
+    for (int x = 0; x < 2; x++) u[x] = w[x];
     if (!DELTA)
 #pragma unroll
       for (int x = 0; x < 2; x++)
@@ -696,6 +731,11 @@ __global__ __launch_bounds__(768, 1) void scan_channel_kernel(Scan p, const RowS
 #pragma unroll
     for (int e = 0; e < 4; e++) w = mfma4(inv[e], u[e], w);
     w += u;
+    const bool careful = any_not_finite(w[0] + w[1] + w[2] + w[3]);
+    if (careful) {
+      w = tile_below(zero, lds + L::INV, u, false, lane) + u;
+      o = tile_below(o, stage + L::P, w, false, lane);
+    }
     // the state behind the chunk, and what its own tokens give
 #pragma unroll
     for (int i = 0; i < NI; i++) {
@@ -707,7 +747,7 @@ __global__ __launch_bounds__(768, 1) void scan_channel_kernel(Scan p, const RowS
       for (int e = 0; e < 4; e++) {
 #pragma unroll
         for (int b = 0; b < 2; b++) S[2 * i + b] = mfma4(kt[i & 1][b][e], w[e], S[2 * i + b]);
-        if (i == 0) o = mfma4(pt[e], w[e], o);
+        if (i == 0 && !careful) o = mfma4(pt[e], w[e], o);
       }
       __builtin_amdgcn_sched_barrier(0);
     }

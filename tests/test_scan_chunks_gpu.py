@@ -48,6 +48,37 @@ def _exact(kind, q, k, v, b, a, rate, bias, skip, S):
     return out, S
 
 
+def _both_forms(kind, heads, key_heads, K, V, conv, inp, a, a_log, bias, skip, state, segs):
+    """-> outputs [T, heads, V] and states in chunks, then token by token, in float64."""
+    n, longest = len(conv), int(segs[:, 1].max())
+    lib, keep = load_pkg("lib").load(), []
+
+    def dev(x):
+        keep.append(torch.from_numpy(np.ascontiguousarray(x)).cuda())
+        return keep[-1].data_ptr()
+
+    nk = key_heads * K
+    got = []
+    for name in ("_ZN6gptoss15run_scan_chunksERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t",
+                 "_ZN6gptoss8run_scanERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t"):
+        st, out = torch.from_numpy(state).cuda(), torch.full((n, heads * V), np.nan, device="cuda")
+        p = Scan(kind=kind, heads=heads, key_heads=key_heads, K=K, V=V, conv=dev(conv), ld_conv=conv.shape[1], q_col=0, k_col=nk,
+                 v_col=2 * nk, inp=dev(inp), ld_in=inp.shape[1], beta_col=0, decay_col=heads,
+                 channel_decay=dev(a) if kind == CHANNEL_DELTA else None, ld_decay=heads * K, a_log=dev(a_log), dt_bias=dev(bias),
+                 d_skip=dev(skip), value_scale=1.0, state=st.data_ptr(), out=out.data_ptr(), ld_out=heads * V)
+        singles = segs[segs[:, 1] == 1]
+        r = StepRows(n=n, n_seg=len(segs), segs=dev(segs), singles=dev(singles) if len(singles) else None, n_singles=len(singles),
+                     longest=longest)
+        f = getattr(lib, name)
+        f.restype, f.argtypes = C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p]
+        torch.cuda.synchronize()
+        assert f(C.addressof(p), C.addressof(r), None) == 0
+        torch.cuda.synchronize()
+        got.append((out.cpu().numpy().reshape(n, heads, V).astype(np.float64), st.cpu().numpy().astype(np.float64)))
+
+    return got
+
+
 @pytest.mark.parametrize("strong", [False, True])
 @pytest.mark.parametrize("kind", [DELTA, CHANNEL_DELTA, STATE_SPACE])
 @pytest.mark.parametrize("heads,key_heads,K,V,lengths", [
@@ -80,30 +111,7 @@ def test_chunks_equal_the_recurrence(kind, strong, heads, key_heads, K, V, lengt
     at = np.concatenate([[0], np.cumsum(lengths)])[:-1]
     segs = np.array([(r, m, s, 0 if i == 0 else 7) for i, (r, m, s) in enumerate(zip(at, lengths, order))], np.int32)
 
-    lib, keep = load_pkg("lib").load(), []
-
-    def dev(x):
-        keep.append(torch.from_numpy(np.ascontiguousarray(x)).cuda())
-        return keep[-1].data_ptr()
-
-    nk = key_heads * K
-    got = []
-    for name in ("_ZN6gptoss15run_scan_chunksERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t",
-                 "_ZN6gptoss8run_scanERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t"):
-        st, out = torch.from_numpy(state).cuda(), torch.full((n, heads * V), np.nan, device="cuda")
-        p = Scan(kind=kind, heads=heads, key_heads=key_heads, K=K, V=V, conv=dev(conv), ld_conv=conv.shape[1], q_col=0, k_col=nk,
-                 v_col=2 * nk, inp=dev(inp), ld_in=inp.shape[1], beta_col=0, decay_col=heads,
-                 channel_decay=dev(a) if kind == CHANNEL_DELTA else None, ld_decay=heads * K, a_log=dev(a_log), dt_bias=dev(bias),
-                 d_skip=dev(skip), value_scale=1.0, state=st.data_ptr(), out=out.data_ptr(), ld_out=heads * V)
-        singles = segs[segs[:, 1] == 1]
-        r = StepRows(n=n, n_seg=slots, segs=dev(segs), singles=dev(singles) if len(singles) else None, n_singles=len(singles),
-                     longest=max(lengths))
-        f = getattr(lib, name)
-        f.restype, f.argtypes = C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p]
-        torch.cuda.synchronize()
-        assert f(C.addressof(p), C.addressof(r), None) == 0
-        torch.cuda.synchronize()
-        got.append((out.cpu().numpy().reshape(n, heads, V).astype(np.float64), st.cpu().numpy().astype(np.float64)))
+    got = _both_forms(kind, heads, key_heads, K, V, conv, inp, a, a_log, bias, skip, state, segs)
 
     d = lambda x: x.astype(np.float64)
     rep = lambda x: np.repeat(d(x), heads // key_heads, axis=1)
@@ -122,3 +130,34 @@ def test_chunks_equal_the_recurrence(kind, strong, heads, key_heads, K, V, lengt
         assert np.abs(st - state_want).max() <= 4e-6 * np.abs(state_want).max()
     rms = [np.sqrt(((out - want) ** 2).mean()) for out, _ in got]
     assert rms[0] <= 1.5 * rms[1] + 1e-8
+
+
+@pytest.mark.parametrize("what", ["value", "decay"])
+@pytest.mark.parametrize("kind", [DELTA, CHANNEL_DELTA, STATE_SPACE])
+def test_an_infinity_reaches_no_earlier_token(kind, what):
+    """A value that is infinite spoils its column from its token on and nothing in front of it; a decay input that is (of a
+    channel, where there is one for each) only empties the state."""
+    g = np.random.default_rng(7 + kind)
+    n, H, K, V, bad = 70, 2, 64, 64, 37
+    unit = lambda x: x / np.sqrt((x * x).sum(-1, keepdims=True))
+    f32 = lambda x: np.ascontiguousarray(x, np.float32)
+    q, k, v = unit(g.standard_normal((n, H, K))), unit(g.standard_normal((n, H, K))), g.standard_normal((n, H, V))
+    b, a = g.standard_normal((n, H)), g.standard_normal((n, H, K) if kind == CHANNEL_DELTA else (n, H))
+    bias, state = g.standard_normal(a.shape[1:]), np.zeros((1, H, V, K), np.float32)
+    if what == "value":
+        v[bad, 1, 5] = np.inf
+    elif kind == STATE_SPACE:   # (the input is its step size too, of what it writes)
+        a[bad, 1] = 1e30
+    else:
+        a[bad, 1] = np.inf
+    conv = f32(np.concatenate([q.reshape(n, -1), k.reshape(n, -1), v.reshape(n, -1)], axis=1))
+    inp = f32(np.concatenate([b, a.reshape(n, -1)], axis=1))
+    (got, _), (want, _) = _both_forms(kind, H, H, K, V, conv, inp, f32(a), f32(g.uniform(-3, -1, H)), f32(bias),
+                                      f32(g.standard_normal(H)), state, np.array([(0, n, 0, 0)], np.int32))
+    fine = np.ones((n, H, V), bool)
+    if what == "value":
+        fine[bad:, 1, 5] = False
+    elif kind == STATE_SPACE:
+        fine[bad:, 1] = False   # 1e30 times as large as the others
+    assert np.isfinite(want[fine]).all() and np.isfinite(got[fine]).all()
+    assert np.abs(got - want)[fine].max() <= 8e-6 * np.abs(want[fine]).max()   # either form's 4e-6
