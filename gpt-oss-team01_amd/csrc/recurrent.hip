@@ -9,7 +9,7 @@
 // the tokens go by, their keys, queries and gates staged in LDS and shared by the workgroup's columns.
 // Everything is fp32, and the tokens are taken one after the other, so a sequence's results are bit for
 // bit the same however it is cut into steps.  Long stretches of a prompt run in retention.hip (retention) and scan_chunks.hip
-// (state space, delta rules) instead, which equal this to rounding.
+// (state space) instead, which equal this to rounding.
 #include <type_traits>
 
 #include "recurrent_device.hpp"

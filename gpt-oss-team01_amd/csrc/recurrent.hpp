@@ -62,10 +62,9 @@ inline bool scan_reads_wide(const Scan &p) {
          (p.kind != SCAN_CHANNEL_DELTA || (p.ld_decay % 4 == 0 && aligned(p.channel_decay, 16)));
 }
 int run_scan(const Scan &p, const StepRows &r, hipStream_t s);
-// The same in chunks of 32 or 16 tokens on the matrix cores (scan_chunks.hip), for steps with a stretch of at least SCAN_CHUNK_ROWS
-// rows: two chunks take as long as 40 to 48 tokens one by one (1 / 4 / 16 sequences of 48 rows, 16 heads of 128 x 128: 18.9 /
-// 21.2 / 33.2 us against 19.5 / 21.3 / 39.4; of 40 rows 20.2 / 20.1 / 32.8 against 17.5 / 19.0 / 34.5; a decay per channel, 48 rows
-// 21.9 / 22.3 / 40.8 against 21.9 / 23.3 / 40.5, 64 rows of 16 48.8 / 51.7).
+// The state-space recurrence in chunks of 32 tokens on the matrix cores (scan_chunks.hip), for steps with a stretch of at least
+// SCAN_CHUNK_ROWS rows: two chunks take less time than 48 tokens one by one (1 / 4 / 16 sequences of 48 rows, 32 heads of 128 x 64:
+// 11.7 / 12.4 / 18.8 us against 14.4 / 15.4 / 25.4; 8 heads of 128 x 16 10.7 / 11.0 / 11.1 against 12.8 / 13.1 / 13.3).
 constexpr int SCAN_CHUNK_ROWS = 48;
 bool scan_chunks_apply(const Scan &p, const StepRows &r);
 int run_scan_chunks(const Scan &p, const StepRows &r, hipStream_t s);

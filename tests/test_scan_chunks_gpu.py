@@ -1,5 +1,6 @@
-"""The delta rules and the state-space recurrence in chunks on the matrix cores, and token by token, against the recurrence in
-64 bits: gptoss::run_scan_chunks and gptoss::run_scan by their linker names, at the edges of chunks, key and column blocks."""
+"""The delta rules and the state-space recurrence over the rows of a step, in the form that a step takes (stretches of a prompt:
+the state-space recurrence in chunks on the matrix cores) and token by token, against the recurrence in 64 bits:
+gptoss::run_scan_chunks and gptoss::run_scan by their linker names, at the edges of chunks, key and column blocks."""
 import ctypes as C
 
 import numpy as np
@@ -28,6 +29,12 @@ StepRows = _struct("StepRows", ("i", "n n_seg max_len"), ("p", "tokens slots len
                    ("i", "n_singles longest"), ("p", "tiles0 tiles1 tiles2"))
 
 
+def _takes_chunks(lib, p, r):
+    f = lib["_ZN6gptoss17scan_chunks_applyERKNS_4ScanERKNS_8StepRowsE"]
+    f.restype, f.argtypes = C.c_bool, [C.c_void_p, C.c_void_p]
+    return f(C.addressof(p), C.addressof(r))
+
+
 def _softplus(x):
     return np.maximum(x, 0) + np.log1p(np.exp(-np.abs(x)))
 
@@ -49,7 +56,7 @@ def _exact(kind, q, k, v, b, a, rate, bias, skip, S):
 
 
 def _both_forms(kind, heads, key_heads, K, V, conv, inp, a, a_log, bias, skip, state, segs):
-    """-> outputs [T, heads, V] and states in chunks, then token by token, in float64."""
+    """-> outputs [T, heads, V] and states in the form that a step takes, then token by token, in float64."""
     n, longest = len(conv), int(segs[:, 1].max())
     lib, keep = load_pkg("lib").load(), []
 
@@ -59,8 +66,9 @@ def _both_forms(kind, heads, key_heads, K, V, conv, inp, a, a_log, bias, skip, s
 
     nk = key_heads * K
     got = []
-    for name in ("_ZN6gptoss15run_scan_chunksERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t",
-                 "_ZN6gptoss8run_scanERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t"):
+    chunks, tokens = (getattr(lib, name) for name in ("_ZN6gptoss15run_scan_chunksERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t",
+                                                      "_ZN6gptoss8run_scanERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t"))
+    for f in (chunks, tokens):
         st, out = torch.from_numpy(state).cuda(), torch.full((n, heads * V), np.nan, device="cuda")
         p = Scan(kind=kind, heads=heads, key_heads=key_heads, K=K, V=V, conv=dev(conv), ld_conv=conv.shape[1], q_col=0, k_col=nk,
                  v_col=2 * nk, inp=dev(inp), ld_in=inp.shape[1], beta_col=0, decay_col=heads,
@@ -69,7 +77,8 @@ def _both_forms(kind, heads, key_heads, K, V, conv, inp, a, a_log, bias, skip, s
         singles = segs[segs[:, 1] == 1]
         r = StepRows(n=n, n_seg=len(segs), segs=dev(segs), singles=dev(singles) if len(singles) else None, n_singles=len(singles),
                      longest=longest)
-        f = getattr(lib, name)
+        if f is chunks and not _takes_chunks(lib, p, r):
+            f = tokens
         f.restype, f.argtypes = C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p]
         torch.cuda.synchronize()
         assert f(C.addressof(p), C.addressof(r), None) == 0
@@ -91,8 +100,6 @@ def _both_forms(kind, heads, key_heads, K, V, conv, inp, a, a_log, bias, skip, s
     (6, 3, 64, 64, (70,) + 100 * (1,)),     # more single tokens than workgroups run at a time
 ])
 def test_chunks_equal_the_recurrence(kind, strong, heads, key_heads, K, V, lengths):
-    if kind == CHANNEL_DELTA and K > 160:
-        pytest.skip("token by token only")
     g = np.random.default_rng(K + V + kind)
     n, slots, KP = sum(lengths), len(lengths), (K + 31) // 32 * 32
     unit = lambda x: x / np.sqrt((x * x).sum(-1, keepdims=True))
@@ -161,3 +168,44 @@ def test_an_infinity_reaches_no_earlier_token(kind, what):
         fine[bad:, 1] = False   # 1e30 times as large as the others
     assert np.isfinite(want[fine]).all() and np.isfinite(got[fine]).all()
     assert np.abs(got - want)[fine].max() <= 8e-6 * np.abs(want[fine]).max()   # either form's 4e-6
+
+
+def _drift(g, *shape):
+    return g.standard_normal((1, *shape[1:])) + 0.1 * np.cumsum(g.standard_normal(shape), axis=0)
+
+
+def _taps_and_silu(g, *shape):
+    taps, x = g.standard_normal((4, *shape[1:])) / 2, g.standard_normal((shape[0] + 3, *shape[1:]))
+    y = sum(taps[i] * x[i:i + shape[0]] for i in range(4))
+    return y / (1 + np.exp(-y))
+
+
+KEYS = {"random": lambda g, *shape: g.standard_normal(shape), "as a model makes them": _taps_and_silu, "drifting": _drift,
+        "with a common part": lambda g, *shape: g.standard_normal((1, *shape[1:])) + 0.3 * g.standard_normal(shape)}
+
+
+@pytest.mark.parametrize("strong", [False, True])
+@pytest.mark.parametrize("keys", KEYS)
+@pytest.mark.parametrize("kind", [DELTA, CHANNEL_DELTA])
+def test_the_form_of_a_prompt_is_as_exact_as_token_by_token(kind, keys, strong):
+    """Errors of the outputs against 64 bits, where keys are random, as the layers make them, or agree (then a delta rule takes off
+    most of what the state holds): three sizes together, within a tenth, by which two correct orders of the sums differ."""
+    ratios = []
+    for heads, K, V in ((4, 128, 64), (4, 64, 64), (2, 256 if kind != CHANNEL_DELTA else 160, 32)):
+        g, n = np.random.default_rng(K), 320
+        unit = lambda x: x / np.sqrt((x * x).sum(-1, keepdims=True))
+        f32 = lambda x: np.ascontiguousarray(x, np.float32)
+        k = unit(KEYS[keys](g, n, heads, K))
+        q = unit(k + 0.3 * unit(g.standard_normal(k.shape)) if keys != "random" else g.standard_normal(k.shape)) / np.sqrt(K)
+        channels = (heads, K) if kind == CHANNEL_DELTA else (heads,)
+        v, b, a = g.standard_normal((n, heads, V)), g.standard_normal((n, heads)), g.standard_normal((n, *channels))
+        q, k, v, b, a, rate, bias, skip = map(f32, (q, k, v, b, a, g.uniform(-5, -.5, heads) + 4.5 * strong,
+                                                    g.standard_normal(channels), g.standard_normal(heads)))
+        state = np.zeros((1, heads, V, (K + 31) // 32 * 32), np.float32)
+        conv = np.concatenate([q.reshape(n, -1), k.reshape(n, -1), v.reshape(n, -1)], axis=1)
+        got = _both_forms(kind, heads, heads, K, V, conv, np.concatenate([b, a.reshape(n, -1)], axis=1), a, rate, bias, skip, state,
+                          np.array([(0, n, 0, 0)], np.int32))
+        d = lambda x: x.astype(np.float64)
+        want, _ = _exact(kind, d(q), d(k), d(v), d(b), d(a), np.exp(d(rate)), d(bias), d(skip), np.zeros((heads, V, K)))
+        ratios.append(np.divide(*(np.sqrt(((out - want) ** 2).mean()) for out, _ in got)))
+    assert np.mean(ratios) <= 1.1, ratios
