@@ -13,10 +13,17 @@
 //
 // Token by token (recurrent.hip) a state element takes three vector instructions a token, and the reads of keys and queries
 // fill LDS at the same time; here it takes two products at twice the vector units' rate.  Measured, token by token -> here (us),
-// 32 heads of 128 x 64: 8 prompts of 1000 tokens 338 -> 152, 16 of 260 150 -> 85, one 71 -> 42.  The products alone are 70 us of
-// the first: with one wave per SIMD what lies between them is not hidden (LDS reads are requested a group of products ahead,
-// the tokens' decays two chunks; as the compiler placed them 185 us), and the second workgroup that a CU has room for, up to
-// 128 keys, is there from 9 sequences of 32 heads on.
+// 32 heads of 128 x 64: 8 prompts of 1000 tokens 281 -> 139, 16 of 260 116 -> 68, one 65 -> 41; 8 heads of 128 x 16, one of 1000
+// 220 -> 133; 4 of 256 x 64 808 -> 251.  With one wave per SIMD what lies between the products is not hidden (LDS reads are
+// requested a group of products ahead, the tokens' decays two chunks); the second workgroup that a CU has room for, up to 128
+// keys, is there from 9 sequences of 32 heads on.
+//
+// A matrix instruction adds its products to a sum one behind the other, so sums over keys are eight, added up in the end, what
+// the chunk's tokens give is summed up by itself, and a token's own key times query, most of its output where decays are strong,
+// is made in double by the wave that has no tile.  Errors of the outputs against 64 bits, times those token by token, five sizes,
+// 500 tokens: random keys 0.69 on average, with decays of 0 to 0.9 0.76, as the layers make them 0.72 and 0.83, of a common
+// direction 0.78 and 1.00, that drift 0.68 and 1.02; of the states 0.5 to 1.0.  With one sum over the state's keys, two over a tile's
+// and no part by itself the outputs had 0.96 and 1.44, 1.18 and 1.49, 1.14 and 1.47, 1.08 and 1.55, in 8 % less time.
 //
 // Not for the delta rules, although a chunk can be made of them as well (u is then the solution of a triangular system; 412 ->
 // 222 us with a decay per head, 449 -> 273 with one per channel).  What a token writes there takes off what the state has along
@@ -37,7 +44,8 @@ struct ChunkLds {
   static constexpr int Q = 0, K = CHUNK * ROW, STAGE = 2 * CHUNK * ROW;   // two stages
   static constexpr int P = 2 * STAGE;         // 16x16 tiles of token products, 64 lanes x 4 values
   static constexpr int CUM = P + 3 * 256;     // [2][CHUNK] doubles, then per token
-  static constexpr int FROM = CUM + 4 * CHUNK, OUT = FROM + 2 * CHUNK, STEP = OUT + 2 * CHUNK, FLOATS = STEP + 2 * CHUNK;
+  static constexpr int FROM = CUM + 4 * CHUNK, OUT = FROM + 2 * CHUNK, STEP = OUT + 2 * CHUNK, OWN = STEP + 2 * CHUNK,
+                       FLOATS = OWN + CHUNK;   // (OWN: of the present chunk)
 };
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
@@ -59,8 +67,12 @@ __device__ __forceinline__ double prefix32(double v) {
   return v;
 }
 
+__device__ __forceinline__ f32x4 sum_of_eight(const f32x4 (&x)[2][4]) {
+  return ((x[0][0] + x[1][0]) + (x[0][1] + x[1][1])) + ((x[0][2] + x[1][2]) + (x[0][3] + x[1][3]));
+}
+
 // What tokens write, where some of it is not finite.  A product with a whole tile would take its zeros above the diagonal times
-// an infinity and give every token of the chunk no number, those in front of the infinity too; here only the tokens up to and with
+// an infinity and give every token of the chunk no number, those in front of the infinity too; here only the tokens in front of
 // a token give it something.
 __device__ __forceinline__ bool any_not_finite(float sum) { return __ballot(sum * 0.f != 0.f) != 0; }
 __device__ __forceinline__ f32x4 tile_below(f32x4 acc, const float *a, f32x4 b, int lane) {
@@ -74,7 +86,7 @@ __device__ __forceinline__ f32x4 tile_below(f32x4 acc, const float *a, f32x4 b, 
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int t = 4 * c + e;
-        if (s <= t) acc[e] = fmaf(a[(g * 16 + t) * 4 + f], from, acc[e]);
+        if (s < t) acc[e] = fmaf(a[(g * 16 + t) * 4 + f], from, acc[e]);
       }
     }
   return acc;
@@ -199,9 +211,14 @@ __global__ __launch_bounds__(256, NI <= 4 ? 2 : 1) void scan_chunk_kernel(Scan p
     const double *cum = reinterpret_cast<const double *>(lds + L::CUM) + stage * CHUNK;
     auto at4 = [&](const float *a) { return *reinterpret_cast<const f32x4 *>(a); };
 
-    // Products of keys (rows) and queries (columns) of tokens, decayed and masked, in tiles (keys', queries') (0, 0), (0, 1), (1, 1)
+    // Products of keys (rows) and queries (columns) of tokens, decayed and masked, in tiles (keys', queries') (0, 0), (0, 1), (1, 1),
+    // and in the last wave a token's own key times query
     auto product = [&](int sx, int tx, float *to) {
-      f32x4 even = f32x4{0.f, 0.f, 0.f, 0.f}, odd = even, x[2][2], y[2][2];
+      f32x4 sum[2][4], x[2][2], y[2][2];
+#pragma unroll
+      for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) sum[b][e] = f32x4{0.f, 0.f, 0.f, 0.f};
       auto load = [&](int i) {
 #pragma unroll
         for (int b = 0; b < 2; b++) {
@@ -215,30 +232,44 @@ __global__ __launch_bounds__(256, NI <= 4 ? 2 : 1) void scan_chunk_kernel(Scan p
         if (i + 1 < NI) load(i + 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          even = mfma4(x[i & 1][0][e], y[i & 1][0][e], even);
-          odd = mfma4(x[i & 1][1][e], y[i & 1][1][e], odd);
-        }
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+          for (int b = 0; b < 2; b++) sum[b][e] = mfma4(x[i & 1][b][e], y[i & 1][b][e], sum[b][e]);
         __builtin_amdgcn_sched_barrier(0);
       }
+      const f32x4 all = sum_of_eight(sum);
       const int t = tx * 16 + n;
       const double ct = cum[t];
       f32x4 w;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int s = sx * 16 + 4 * c + e;
-        const float x = exp_f((float)(ct - cum[s])) * (even[e] + odd[e]);
-        w[e] = s <= t ? x : 0.f;
+        const float x = exp_f((float)(ct - cum[s])) * all[e];
+        w[e] = s < t ? x : 0.f;
       }
       *reinterpret_cast<f32x4 *>(to + lane * 4) = w;
     };
     if (wave < 3) product(wave == 2, wave > 0, lds + L::P + wave * 256);
+    else {
+      const float *kt = lds + stage * L::STAGE + L::K + (lane & 31) * ROW + (lane >> 5) * (KP / 2), *qt = kt + (L::Q - L::K);
+      double own[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+      for (int d = 0; d < KP / 2; d += 4) {
+        const f32x4 a = at4(kt + d), b = at4(qt + d);
+#pragma unroll
+        for (int e = 0; e < 4; e++) own[e] = fma((double)a[e], (double)b[e], own[e]);
+      }
+      const double sum = (own[0] + own[1]) + (own[2] + own[3]), all = sum + lane_xor<32>(sum);
+      if (lane < 32) lds[L::OWN + lane] = (float)all;
+    }
     __syncthreads();
 
     // what the state in front of the chunk gives: [token][column]
-    f32x4 o[2], qx[3][2];
+    f32x4 o8[2][2][4], qx[3][2];
 #pragma unroll
-    for (int x = 0; x < 2; x++) o[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) o8[x][0][e] = o8[x][1][e] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto load = [&](int b) {
 #pragma unroll
       for (int x = 0; x < 2; x++) qx[b % 3][x] = at4(q + x * 16 * ROW + 16 * b);
@@ -252,39 +283,35 @@ __global__ __launch_bounds__(256, NI <= 4 ? 2 : 1) void scan_chunk_kernel(Scan p
 #pragma unroll
       for (int e = 0; e < 4; e++)
 #pragma unroll
-        for (int x = 0; x < 2; x++) o[x] = mfma4(qx[b % 3][x][e], S[b][e], o[x]);
+        for (int x = 0; x < 2; x++) o8[x][b & 1][e] = mfma4(qx[b % 3][x][e], S[b][e], o8[x][b & 1][e]);
       __builtin_amdgcn_sched_barrier(0);
     }
     // what the tokens write
     f32x4 u[2];
 #pragma unroll
-    for (int x = 0; x < 2; x++) {
-      const f32x4 from = at4(lds + L::FROM + stage * CHUNK + 16 * x + 4 * c), step = at4(lds + L::STEP + stage * CHUNK + 16 * x + 4 * c);
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        o[x][e] *= from[e];
-        u[x][e] = step[e] * v[x][e];
-      }
-    }
+    for (int x = 0; x < 2; x++) u[x] = at4(lds + L::STEP + stage * CHUNK + 16 * x + 4 * c) * f32x4{v[x][0], v[x][1], v[x][2], v[x][3]};
     auto tile = [&](f32x4 acc, const float *a, f32x4 b) {
       const f32x4 w = at4(a + lane * 4);
 #pragma unroll
       for (int e = 0; e < 4; e++) acc = mfma4(w[e], b[e], acc);
       return acc;
     };
-    const f32x4 sum = u[0] + u[1];
+    const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f}, sum = u[0] + u[1];
+    f32x4 o[2];   // what the chunk's tokens give later ones
     if (any_not_finite(sum[0] + sum[1] + sum[2] + sum[3])) {
-      o[0] = tile_below(o[0], lds + L::P, u[0], lane);
-      o[1] = tile_below(tile(o[1], lds + L::P + 256, u[0]), lds + L::P + 512, u[1], lane);
+      o[0] = tile_below(zero, lds + L::P, u[0], lane);
+      o[1] = tile_below(tile(zero, lds + L::P + 256, u[0]), lds + L::P + 512, u[1], lane);
     } else {
-      o[0] = tile(o[0], lds + L::P, u[0]);
-      o[1] = tile(o[1], lds + L::P + 256, u[0]);
-      o[1] = tile(o[1], lds + L::P + 512, u[1]);
+      o[0] = tile(zero, lds + L::P, u[0]);
+      o[1] = tile(zero, lds + L::P + 256, u[0]) + tile(zero, lds + L::P + 512, u[1]);
     }
 #pragma unroll
-    for (int x = 0; x < 2; x++)
+    for (int x = 0; x < 2; x++) {
+      const f32x4 from = at4(lds + L::FROM + stage * CHUNK + 16 * x + 4 * c), own = at4(lds + L::OWN + 16 * x + 4 * c);
+      const f32x4 before = sum_of_eight(o8[x]);
 #pragma unroll
-      for (int e = 0; e < 4; e++) o[x][e] = fmaf(skip, v[x][e], o[x][e]);
+      for (int e = 0; e < 4; e++) o[x][e] = fmaf(skip, v[x][e], fmaf(own[e], u[x][e], fmaf(from[e], before[e], o[x][e])));
+    }
     char *out = reinterpret_cast<char *>(p.out + (size_t)(seg.row0 + t0) * p.ld_out + h * p.V);
     const uint32_t out4 = 4 * p.ld_out, first = __umul24(4 * c, out4) + 4 * (c0 + n);
 #pragma unroll

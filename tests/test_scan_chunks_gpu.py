@@ -186,16 +186,16 @@ KEYS = {"random": lambda g, *shape: g.standard_normal(shape), "as a model makes 
 
 @pytest.mark.parametrize("strong", [False, True])
 @pytest.mark.parametrize("keys", KEYS)
-@pytest.mark.parametrize("kind", [DELTA, CHANNEL_DELTA])
+@pytest.mark.parametrize("kind", [DELTA, CHANNEL_DELTA, STATE_SPACE])
 def test_the_form_of_a_prompt_is_as_exact_as_token_by_token(kind, keys, strong):
     """Errors of the outputs against 64 bits, where keys are random, as the layers make them, or agree (then a delta rule takes off
     most of what the state holds): three sizes together, within a tenth, by which two correct orders of the sums differ."""
     ratios = []
     for heads, K, V in ((4, 128, 64), (4, 64, 64), (2, 256 if kind != CHANNEL_DELTA else 160, 32)):
         g, n = np.random.default_rng(K), 320
-        unit = lambda x: x / np.sqrt((x * x).sum(-1, keepdims=True))
+        unit = lambda x: x / np.sqrt((x * x).sum(-1, keepdims=True)) * (np.sqrt(K) if kind == STATE_SPACE else 1)
         f32 = lambda x: np.ascontiguousarray(x, np.float32)
-        k = unit(KEYS[keys](g, n, heads, K))
+        k = unit(KEYS[keys](g, n, heads, K))   # a delta rule's are unit vectors; the state space's channels are of size 1
         q = unit(k + 0.3 * unit(g.standard_normal(k.shape)) if keys != "random" else g.standard_normal(k.shape)) / np.sqrt(K)
         channels = (heads, K) if kind == CHANNEL_DELTA else (heads,)
         v, b, a = g.standard_normal((n, heads, V)), g.standard_normal((n, heads)), g.standard_normal((n, *channels))
