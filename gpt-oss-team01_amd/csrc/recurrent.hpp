@@ -62,9 +62,11 @@ inline bool scan_reads_wide(const Scan &p) {
          (p.kind != SCAN_CHANNEL_DELTA || (p.ld_decay % 4 == 0 && aligned(p.channel_decay, 16)));
 }
 int run_scan(const Scan &p, const StepRows &r, hipStream_t s);
-// The state-space recurrence in chunks of 32 tokens on the matrix cores (scan_chunks.hip), for steps with a stretch of at least
-// SCAN_CHUNK_ROWS rows: two chunks take less time than 48 tokens one by one (1 / 4 / 16 sequences of 48 rows, 32 heads of 128 x 64:
-// 12.2 / 12.9 / 20.1 us against 14.4 / 15.4 / 26.7; 8 heads of 128 x 16 11.1 / 11.4 / 11.6 against 12.8 / 13.1 / 13.3).
+// The same for steps with a stretch of at least SCAN_CHUNK_ROWS rows: such stretches of the state-space recurrence in chunks of 32
+// tokens on the matrix cores (scan_chunks.hip), the others of the step as by run_scan, so that a stretch's form depends on its own
+// length only and a decoding row has the same bits beside a prompt as alone.  Two chunks take less time than 48 tokens one by one
+// (1 / 4 / 16 sequences of 48 rows, 32 heads of 128 x 64: 12.2 / 12.9 / 20.1 us against 14.4 / 15.4 / 26.7; 8 heads of 128 x 16
+// 11.1 / 11.4 / 11.6 against 12.8 / 13.1 / 13.3).
 constexpr int SCAN_CHUNK_ROWS = 48;
 bool scan_chunks_apply(const Scan &p, const StepRows &r);
 int run_scan_chunks(const Scan &p, const StepRows &r, hipStream_t s);

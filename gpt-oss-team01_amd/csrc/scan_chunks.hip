@@ -14,16 +14,17 @@
 // Token by token (recurrent.hip) a state element takes three vector instructions a token, and the reads of keys and queries
 // fill LDS at the same time; here it takes two products at twice the vector units' rate.  Measured, token by token -> here (us),
 // 32 heads of 128 x 64: 8 prompts of 1000 tokens 281 -> 139, 16 of 260 116 -> 68, one 65 -> 41; 8 heads of 128 x 16, one of 1000
-// 220 -> 133; 4 of 256 x 64 808 -> 251.  With one wave per SIMD what lies between the products is not hidden (LDS reads are
+// 220 -> 133; 4 of 256 x 64 424 -> 250.  With one wave per SIMD what lies between the products is not hidden (LDS reads are
 // requested a group of products ahead, the tokens' decays two chunks); the second workgroup that a CU has room for, up to 128
 // keys, is there from 9 sequences of 32 heads on.
 //
-// A matrix instruction adds its products to a sum one behind the other, so sums over keys are eight, added up in the end, what
-// the chunk's tokens give is summed up by itself, and a token's own key times query, most of its output where decays are strong,
-// is made in double by the wave that has no tile.  Errors of the outputs against 64 bits, times those token by token, five sizes,
-// 500 tokens: random keys 0.69 on average, with decays of 0 to 0.9 0.76, as the layers make them 0.72 and 0.83, of a common
-// direction 0.78 and 1.00, that drift 0.68 and 1.02; of the states 0.5 to 1.0.  With one sum over the state's keys, two over a tile's
-// and no part by itself the outputs had 0.96 and 1.44, 1.18 and 1.49, 1.14 and 1.47, 1.08 and 1.55, in 8 % less time.
+// A matrix instruction adds its products to a sum one behind the other, so sums over the state's keys are four and over a tile's
+// eight, added up in the end, what the chunk's tokens give is summed up by itself, and a token's own key times query, most of its
+// output where decays are strong, is made in double by the wave that has no tile.  Errors of the outputs against 64 bits, times
+// those token by token, five sizes, 500 tokens: random keys 0.70 on average, with decays of 0 to 0.9 0.76, as the layers make them
+// 0.74 and 0.83, of a common direction 0.79 and 1.00, that drift 0.70 and 1.02; of the states 0.5 to 1.0.  With one sum over the
+// state's keys, two over a tile's and no part by itself the outputs had 0.96 and 1.44, 1.18 and 1.49, 1.14 and 1.47, 1.08 and 1.55,
+// in 8 % less time.
 //
 // Not for the delta rules, although a chunk can be made of them as well (u is then the solution of a triangular system; 412 ->
 // 222 us with a decay per head, 449 -> 273 with one per channel).  What a token writes there takes off what the state has along
@@ -93,16 +94,26 @@ __device__ __forceinline__ f32x4 tile_below(f32x4 acc, const float *a, f32x4 b, 
 }
 
 template <int NI>
-__global__ __launch_bounds__(256, NI <= 4 ? 2 : 1) void scan_chunk_kernel(Scan p, const RowSeg *__restrict__ segs, int n_seg,
-                                                                               int fewest) {
+__global__ __launch_bounds__(256, NI <= 4 ? 2 : 1) void scan_chunk_kernel(Scan p, const RowSeg *__restrict__ segs, int n_seg) {
   using L = ChunkLds<NI>;
   constexpr int KP = L::KP, ROW = L::ROW, NB = 2 * NI;   // 16-key blocks of the state
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int seg_id = blockIdx.x % n_seg, unit = blockIdx.x / n_seg, blocks = (p.V + 63) / 64;
   const RowSeg seg = segs[seg_id];
-  if (seg.n < fewest) return;   // taken elsewhere
   if (unit >= p.heads * blocks) {   // workgroups of the convolutions' states come last
     advance_conv_state(p, seg, unit - p.heads * blocks, gridDim.x / n_seg - p.heads * blocks);
+    return;
+  }
+  // Shorter ones token by token, as in a step without a long one: the same bits.  In this launch, because one behind the other
+  // takes longer (us, both in one / shorter ones first / all token by token: a prompt of 48 and 7 of 30, 32 heads of 128 x 64
+  // 14.7 / 25.7 / 17.3, 8 heads of 64 x 16 8.8 / 15.9 / 10.3; a prompt of 48 beside 15 / 100 decoding rows, 32 heads 19.7 / 26.6 / 23.9
+  // and 50.3 / 54.1 / 55.0; the exception is hundreds of decoding rows of narrow heads: 500 beside 200 tokens, 32 heads of 128 x 16
+  // 137 / 105 / 162).
+  if (seg.n < SCAN_CHUNK_ROWS) {
+    using Tokens = ScanLds<NI, SCAN_STATE_SPACE, false, 2>;
+    static_assert(sizeof(Tokens) <= L::FLOATS * sizeof(float));
+    const int h = unit / blocks;
+    scan_stretch<NI, SCAN_STATE_SPACE, false, 2>(p, seg, h, (unit - h * blocks) * 64, *reinterpret_cast<Tokens *>(lds));
     return;
   }
   const int h = unit / blocks, kh = h / (p.heads / p.key_heads);
@@ -265,11 +276,11 @@ __global__ __launch_bounds__(256, NI <= 4 ? 2 : 1) void scan_chunk_kernel(Scan p
     __syncthreads();
 
     // what the state in front of the chunk gives: [token][column]
-    f32x4 o8[2][2][4], qx[3][2];
+    f32x4 o4[2][4], qx[3][2];
 #pragma unroll
     for (int x = 0; x < 2; x++)
 #pragma unroll
-      for (int e = 0; e < 4; e++) o8[x][0][e] = o8[x][1][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int e = 0; e < 4; e++) o4[x][e] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto load = [&](int b) {
 #pragma unroll
       for (int x = 0; x < 2; x++) qx[b % 3][x] = at4(q + x * 16 * ROW + 16 * b);
@@ -283,7 +294,7 @@ __global__ __launch_bounds__(256, NI <= 4 ? 2 : 1) void scan_chunk_kernel(Scan p
 #pragma unroll
       for (int e = 0; e < 4; e++)
 #pragma unroll
-        for (int x = 0; x < 2; x++) o8[x][b & 1][e] = mfma4(qx[b % 3][x][e], S[b][e], o8[x][b & 1][e]);
+        for (int x = 0; x < 2; x++) o4[x][e] = mfma4(qx[b % 3][x][e], S[b][e], o4[x][e]);
       __builtin_amdgcn_sched_barrier(0);
     }
     // what the tokens write
@@ -308,7 +319,7 @@ __global__ __launch_bounds__(256, NI <= 4 ? 2 : 1) void scan_chunk_kernel(Scan p
 #pragma unroll
     for (int x = 0; x < 2; x++) {
       const f32x4 from = at4(lds + L::FROM + stage * CHUNK + 16 * x + 4 * c), own = at4(lds + L::OWN + 16 * x + 4 * c);
-      const f32x4 before = sum_of_eight(o8[x]);
+      const f32x4 before = (o4[x][0] + o4[x][1]) + (o4[x][2] + o4[x][3]);
 #pragma unroll
       for (int e = 0; e < 4; e++) o[x][e] = fmaf(skip, v[x][e], fmaf(own[e], u[x][e], fmaf(from[e], before[e], o[x][e])));
     }
@@ -366,42 +377,33 @@ bool scan_chunks_apply(const Scan &p, const StepRows &r) {
 }
 
 template <int NI>
-static int launch_chunks(const Scan &p, const StepRows &r, int fewest, hipStream_t s) {
+static int launch_chunks(const Scan &p, const StepRows &r, hipStream_t s) {
   constexpr int bytes = ChunkLds<NI>::FLOATS * (int)sizeof(float);
   auto kern = scan_chunk_kernel<NI>;
   GPTOSS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
   TraceScope ts("scan_state_space", s);
   const size_t grid = (size_t)r.n_seg * (p.heads * cdiv(p.V, 64) + cdiv(p.conv_desc.channels, 256));
-  kern<<<(unsigned)grid, 256, bytes, s>>>(p, r.segs, r.n_seg, fewest);
+  kern<<<(unsigned)grid, 256, bytes, s>>>(p, r.segs, r.n_seg);
   GPTOSS_LAUNCH_CHECK("scan_chunk_kernel");
   return GPTOSS_OK;
 }
 
-int run_scan_chunks(const Scan &p, const StepRows &r, hipStream_t s) {
+int run_scan_chunks(const Scan &scan, const StepRows &r, hipStream_t s) {
+  Scan p = scan;
+  p.vec = 1;   // (scan_chunks_apply)
   GPTOSS_REQUIRE(scan_chunks_apply(p, r) && p.V >= 1 && p.key_heads >= 1 && p.heads % p.key_heads == 0, GPTOSS_ERR_DIM,
                  "scan: kind %d with keys of %d, %d heads over %d does not go by chunks", (int)p.kind, p.K, p.heads, p.key_heads);
   GPTOSS_REQUIRE(r.n_seg * ((long long)p.heads * cdiv(p.V, 64) + cdiv(p.conv_desc.channels, 256)) < (1ll << 31), GPTOSS_ERR_DIM,
                  "scan: too many workgroups");
-  // Decoding rows beside the stretches: a chunk of one token takes a CU as long as a full one, which is nothing while there are
-  // CUs to spare; with more of them than run at a time they go as a step of their own.
-  int fewest = 1;
-  if ((long long)r.n_singles * p.heads * cdiv(p.V, 64) > 512) {
-    StepRows single = r;
-    single.segs = r.singles;
-    single.n_seg = r.n_singles;
-    single.longest = 1;
-    GPTOSS_STEP(run_scan(p, single, s));
-    fewest = 2;
-  }
   switch (scan_key_pad(p.K) / 32) {
-    case 1: return launch_chunks<1>(p, r, fewest, s);
-    case 2: return launch_chunks<2>(p, r, fewest, s);
-    case 3: return launch_chunks<3>(p, r, fewest, s);
-    case 4: return launch_chunks<4>(p, r, fewest, s);
-    case 5: return launch_chunks<5>(p, r, fewest, s);
-    case 6: return launch_chunks<6>(p, r, fewest, s);
-    case 7: return launch_chunks<7>(p, r, fewest, s);
-    default: return launch_chunks<8>(p, r, fewest, s);
+    case 1: return launch_chunks<1>(p, r, s);
+    case 2: return launch_chunks<2>(p, r, s);
+    case 3: return launch_chunks<3>(p, r, s);
+    case 4: return launch_chunks<4>(p, r, s);
+    case 5: return launch_chunks<5>(p, r, s);
+    case 6: return launch_chunks<6>(p, r, s);
+    case 7: return launch_chunks<7>(p, r, s);
+    default: return launch_chunks<8>(p, r, s);
   }
 }
 

@@ -55,8 +55,9 @@ def _exact(kind, q, k, v, b, a, rate, bias, skip, S):
     return out, S
 
 
-def _both_forms(kind, heads, key_heads, K, V, conv, inp, a, a_log, bias, skip, state, segs):
-    """-> outputs [T, heads, V] and states in the form that a step takes, then token by token, in float64."""
+def _both_forms(kind, heads, key_heads, K, V, conv, inp, a, a_log, bias, skip, state, segs, short_conv=None,
+                conv_state=None):
+    """-> outputs [T, heads, V], states and convolution states in the form that a step takes, then token by token, in float64."""
     n, longest = len(conv), int(segs[:, 1].max())
     lib, keep = load_pkg("lib").load(), []
 
@@ -70,10 +71,12 @@ def _both_forms(kind, heads, key_heads, K, V, conv, inp, a, a_log, bias, skip, s
                                                       "_ZN6gptoss8run_scanERKNS_4ScanERKNS_8StepRowsEP12ihipStream_t"))
     for f in (chunks, tokens):
         st, out = torch.from_numpy(state).cuda(), torch.full((n, heads * V), np.nan, device="cuda")
+        taken = torch.from_numpy(conv_state if conv_state is not None else np.zeros(1, np.float32)).cuda()
         p = Scan(kind=kind, heads=heads, key_heads=key_heads, K=K, V=V, conv=dev(conv), ld_conv=conv.shape[1], q_col=0, k_col=nk,
                  v_col=2 * nk, inp=dev(inp), ld_in=inp.shape[1], beta_col=0, decay_col=heads,
                  channel_decay=dev(a) if kind == CHANNEL_DELTA else None, ld_decay=heads * K, a_log=dev(a_log), dt_bias=dev(bias),
-                 d_skip=dev(skip), value_scale=1.0, state=st.data_ptr(), out=out.data_ptr(), ld_out=heads * V)
+                 d_skip=dev(skip), value_scale=1.0, state=st.data_ptr(), out=out.data_ptr(), ld_out=heads * V,
+                 conv_desc=short_conv or ShortConv(taps=1), conv_state=taken.data_ptr())
         singles = segs[segs[:, 1] == 1]
         r = StepRows(n=n, n_seg=len(segs), segs=dev(segs), singles=dev(singles) if len(singles) else None, n_singles=len(singles),
                      longest=longest)
@@ -83,7 +86,7 @@ def _both_forms(kind, heads, key_heads, K, V, conv, inp, a, a_log, bias, skip, s
         torch.cuda.synchronize()
         assert f(C.addressof(p), C.addressof(r), None) == 0
         torch.cuda.synchronize()
-        got.append((out.cpu().numpy().reshape(n, heads, V).astype(np.float64), st.cpu().numpy().astype(np.float64)))
+        got.append([x.cpu().numpy().astype(np.float64) for x in (out.view(n, heads, V), st, taken)])
 
     return got
 
@@ -97,7 +100,7 @@ def _both_forms(kind, heads, key_heads, K, V, conv, inp, a, a_log, bias, skip, s
     (1, 1, 132, 128, (50,)),
     (2, 1, 160, 20, (63, 17, 48)),
     (2, 1, 256, 16, (129, 15, 16, 17)),     # the largest keys
-    (6, 3, 64, 64, (70,) + 100 * (1,)),     # more single tokens than workgroups run at a time
+    (6, 3, 64, 64, (70,) + 100 * (1,)),
 ])
 def test_chunks_equal_the_recurrence(kind, strong, heads, key_heads, K, V, lengths):
     g = np.random.default_rng(K + V + kind)
@@ -131,11 +134,11 @@ def test_chunks_equal_the_recurrence(kind, strong, heads, key_heads, K, V, lengt
     state_want[order[0], ..., K:] = 0
     # A sum of K products and of a chunk's tokens, and a decay per token, in fp32: a few hundred roundings of 6e-8 that add up
     # like their root, 2e-6 of the largest value; the two forms are alike in that.
-    for out, st in got:
+    for out, st, _ in got:
         assert np.isfinite(out).all()
         assert np.abs(out - want).max() <= 4e-6 * np.abs(want).max()
         assert np.abs(st - state_want).max() <= 4e-6 * np.abs(state_want).max()
-    rms = [np.sqrt(((out - want) ** 2).mean()) for out, _ in got]
+    rms = [np.sqrt(((out - want) ** 2).mean()) for out, _, _ in got]
     assert rms[0] <= 1.5 * rms[1] + 1e-8
 
 
@@ -159,7 +162,7 @@ def test_an_infinity_reaches_no_earlier_token(kind, what):
         a[bad, 1] = np.inf
     conv = f32(np.concatenate([q.reshape(n, -1), k.reshape(n, -1), v.reshape(n, -1)], axis=1))
     inp = f32(np.concatenate([b, a.reshape(n, -1)], axis=1))
-    (got, _), (want, _) = _both_forms(kind, H, H, K, V, conv, inp, f32(a), f32(g.uniform(-3, -1, H)), f32(bias),
+    (got, _, _), (want, _, _) = _both_forms(kind, H, H, K, V, conv, inp, f32(a), f32(g.uniform(-3, -1, H)), f32(bias),
                                       f32(g.standard_normal(H)), state, np.array([(0, n, 0, 0)], np.int32))
     fine = np.ones((n, H, V), bool)
     if what == "value":
@@ -207,5 +210,35 @@ def test_the_form_of_a_prompt_is_as_exact_as_token_by_token(kind, keys, strong):
                           np.array([(0, n, 0, 0)], np.int32))
         d = lambda x: x.astype(np.float64)
         want, _ = _exact(kind, d(q), d(k), d(v), d(b), d(a), np.exp(d(rate)), d(bias), d(skip), np.zeros((heads, V, K)))
-        ratios.append(np.divide(*(np.sqrt(((out - want) ** 2).mean()) for out, _ in got)))
+        ratios.append(np.divide(*(np.sqrt(((out - want) ** 2).mean()) for out, _, _ in got)))
     assert np.mean(ratios) <= 1.1, ratios
+
+
+@pytest.mark.parametrize("kind", [DELTA, CHANNEL_DELTA, STATE_SPACE])
+@pytest.mark.parametrize("lengths", [(48, 1, 47), (1, 300, 1), (2, 64, 1, 49, 31), (70,) + 100 * (1,), (48, 50)])
+def test_short_stretches_beside_a_prompt_are_as_alone(kind, lengths):
+    """A stretch's form depends on its own length only: those of fewer than 48 rows have the bits that they have token by token,
+    whatever else is in the step.  The convolution's state of every stretch is brought up to date once: the last three inputs,
+    those in front of the stretch from the state as it was, or zero where the sequence begins."""
+    g = np.random.default_rng(sum(lengths) + kind)
+    n, slots, H, K, V, taps, channels = sum(lengths), len(lengths), 2, 64, 68, 4, 300
+    f32 = lambda x: np.ascontiguousarray(x, np.float32)
+    unit = lambda x: x / np.sqrt((x * x).sum(-1, keepdims=True))
+    a = g.standard_normal((n, H, K) if kind == CHANNEL_DELTA else (n, H))
+    conv = f32(np.concatenate([unit(g.standard_normal((n, 2 * H, K))).reshape(n, -1), g.standard_normal((n, H * V))], axis=1))
+    before = np.concatenate([g.standard_normal((n, H)), a.reshape(n, -1)], axis=1)
+    x = f32(g.standard_normal((n, channels)))
+    at = np.concatenate([[0], np.cumsum(lengths)])[:-1]
+    segs = np.array([(r, m, s, 0 if i == 1 else 2 + i) for i, (r, m, s) in enumerate(zip(at, lengths, g.permutation(slots)))], np.int32)
+    state, taken = f32(g.standard_normal((slots, H, V, K))), f32(g.standard_normal((slots, taps - 1, channels)))
+    got = _both_forms(kind, H, H, K, V, conv, np.concatenate([f32(before), x], axis=1), f32(a), f32(g.uniform(-3, -1, H)),
+                      f32(g.standard_normal(a.shape[1:])), f32(g.standard_normal(H)), state, segs,
+                      ShortConv(col=before.shape[1], channels=channels, taps=taps), taken)
+    (out, st, left), (out_alone, st_alone, left_alone) = got
+    for r, m, s, pos0 in segs:
+        if m < 48:
+            assert np.array_equal(out[r:r + m], out_alone[r:r + m]) and np.array_equal(st[s], st_alone[s])
+        older = taken[s] if pos0 else np.zeros_like(taken[s])
+        assert np.array_equal(left[s], np.concatenate([older, x[r:r + m]])[-(taps - 1):])
+    assert np.array_equal(left, left_alone)
+    assert np.abs(out - out_alone).max() <= 8e-6 * np.abs(out_alone).max()   # either form's 4e-6
