@@ -636,7 +636,7 @@ struct RopeInput {
   bf16_t *kv;
 };
 template <int D, bool ROPE>
-__global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p, RopeInput rope) {
+__device__ __forceinline__ void attn_few_chunk(const AttnParams &p, const RopeInput &rope) {
   constexpr int KS = D / 32, DB = D / 16, NBLK = ATT_CHUNK / ATT_BLOCK;
   static_assert(NBLK == 8 && DB <= 4, "two blocks and at most 16 output columns per wave");
   __shared__ __attribute__((aligned(16))) u32x4 lds_p[NBLK][4][64];   // weights: hi and lo parts of 32 slots each
@@ -869,6 +869,11 @@ __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p, RopeInpu
     }
   }
 }
+template <int D>
+__global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) { attn_few_chunk<D, false>(p, RopeInput{}); }
+template <int D>
+__global__ __launch_bounds__(256, 1) void attn_few_rope_kernel(AttnParams p, RopeInput rope) { attn_few_chunk<D, true>(p, rope); }
+
 // The launches that take it: where every row is as long as the longest may be, up to 512 (row, kv head, chunk) items, two
 // per CU; 384 with heads of 32 values; 256 of rows that cannot fill half a chunk.  64 heads of 64 on 8 kv heads, full rows, caches
 // cold, a wave per item -> this kernel (us): 4 of 8000 positions (512 items) 29.0 -> 25.4, 32 of 1000 29.6 -> 25.4, 63 of 448
@@ -1369,9 +1374,9 @@ static int attn_launch(const float *q, const void *kv_cache, const int *lens,
       if (rc != GPTOSS_OK) return rc;
     }
     if (few) {
-      auto launch = [&](auto kernel) { kernel<<<(int)items, 256, 0, s>>>(p, rope ? *rope : RopeInput{}); };
-      if (rope) launch(head_dim == 64 ? attn_few_kernel<64, true> : attn_few_kernel<32, true>);
-      else launch(head_dim == 64 ? attn_few_kernel<64, false> : attn_few_kernel<32, false>);
+      auto launch = [&](auto kernel, const auto &...more) { kernel<<<(int)items, 256, 0, s>>>(p, more...); };
+      if (rope) launch(head_dim == 64 ? attn_few_rope_kernel<64> : attn_few_rope_kernel<32>, *rope);
+      else launch(head_dim == 64 ? attn_few_kernel<64> : attn_few_kernel<32>);
     } else if (head_dim == 64) {
       if (pair) attn_decode_kernel<64, true><<<grid, 256, 0, s>>>(p);
       else if (hold_rows) attn_decode_resident_kernel<64><<<std::min(grid, resident), 256, 0, s>>>(p, grid);

@@ -65,7 +65,8 @@ def test_no_matrix_instruction_under_a_lane_mask(tmp_path):
         bad, seen = masked_matrix_instructions(listing)
         found.update(bad)
         kernels |= seen
-    for part in ("router_gemm_kernel", "grouped_gemm_kernel", "few_gemm_kernel", "tall_gemm_kernel", "attn_few_kernel"):
+    for part in ("router_gemm_kernel", "grouped_gemm_kernel", "few_gemm_kernel", "tall_gemm_kernel", "attn_few_kernel",
+                 "attn_few_rope_kernel", "scan_chunk_kernel"):
         assert any(part in k for k in kernels), part      # the listing was read
     assert not found, found
 
