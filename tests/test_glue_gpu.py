@@ -44,8 +44,8 @@ def test_rmsnorm_matches_oracle(ops, orc, B, H):
                                         (600, 2880, 4096, True), (1024, 5120, 2880, False),
                                         (700, 4096, 256, True), (2304, 1056, 512, True)])
 def test_dense_gemm(ops, B, N, K, bias):
-    """Every regime of the dispatch: row tiles of 32..160 rows chosen from the batch size, 256-row
-    tiles from 2048 rows on, ragged last row tile and last column tile."""
+    """Every regime of the dispatch: row tiles of 32..160 rows or 256 by estimated time, ragged last row tile and last column
+    tile.  (The 256-row kernel by itself: test_tall_dense_gpu.py.)"""
     g = torch.Generator(device="cuda").manual_seed(B + N)
     a = torch.randn(B, K, device="cuda", generator=g).to(torch.bfloat16)
     w = (torch.randn(N, K, device="cuda", generator=g) * 0.05).to(torch.bfloat16)
@@ -57,8 +57,8 @@ def test_dense_gemm(ops, B, N, K, bias):
 
 @pytest.mark.parametrize("B,N,K", [(2500, 2880, 4096), (2049, 5120, 2880), (4096, 288, 256)])
 def test_dense_gemm_of_a_prompt_pass_equals_the_same_rows_in_small_batches(ops, B, N, K):
-    """From 2048 rows on the fp32 GEMM runs the kernel with 256-row tiles and both operands through
-    LDS: same bits per row as the streaming kernels, which run the batches of a fifth of the rows."""
+    """Thousands of rows, where most products run the kernel with 256-row tiles and both operands through LDS (here all but the
+    narrow one): same bits per row as the streaming kernels, which run the batches of a fifth of the rows."""
     g = torch.Generator(device="cuda").manual_seed(B + N)
     a = torch.randn(B, K, device="cuda", generator=g).to(torch.bfloat16)
     w = (torch.randn(N, K, device="cuda", generator=g) * 0.05).to(torch.bfloat16)

@@ -311,8 +311,9 @@ def test_rotation_far_from_the_start(open_model, scaling, precise):
 
 @BOTH
 def test_wide_rows_and_passes_of_thousands_of_rows(open_model, precise):
-    """Sizes at which the products cut their sum over K into parts (few rows, many inputs) and run on the
-    256-row tiles (2048 rows and more in a pass, several sequences; hundreds of rows per expert)."""
+    """Sizes at which the products cut their sum over K into parts (few rows, many inputs), and a pass of thousands of rows, of
+    several sequences (the experts' products: hundreds of rows per expert).  (Dense products this narrow stay off the 256-row
+    kernel: test_tall_dense_gpu.py.)"""
     cfg = xm.config([xm.retention(heads=4, dim=64, vdim=128, dims=64, mlp=xm.moe(ff=256, experts=4, top=2)),
                      xm.attention(heads=8, kv=2, dim=64, dims=64, size=300, scale=0.125, mlp=xm.moe(ff=300, experts=3, top=2))],
                     vocab=96, width=320)

@@ -288,8 +288,8 @@ def test_other_sizes(open_model, name, precise):
 
 @BOTH
 def test_wide_rows_and_passes_of_thousands_of_rows(open_model, precise):
-    """Sizes at which the products cut their sum over K into parts (few rows, many inputs) and run on the
-    256-row tiles (2048 rows and more in a pass, several sequences)."""
+    """Sizes at which the products cut their sum over K into parts (few rows, many inputs), and a pass of thousands of rows, of
+    several sequences.  (Products this narrow stay off the 256-row kernel: test_tall_dense_gpu.py.)"""
     cfg = nm.config([nm.channel_delta(heads=2, kv=1, dim=32, vdim=128, ff=1400),
                      nm.parallel(heads=2, kv=1, dim=64, vdim=64, window=100, s_heads=1, groups=1, state=64, s_vdim=64,
                                  norm_groups=1, ff=900)], vocab=96, width=320, max_positions=900)
