@@ -157,9 +157,11 @@ static int dense_tall_min_rows() {
 
 // Whether a dense product is one for the 256-row kernel, given the best estimate of the others, which is up to a fifth too high
 // for products of a thousand rows: below 2048 rows the 256-row kernel has to be clearly ahead, above clearly behind.  Timed with
-// both at 792 products (10 shapes of 512-65536 columns, K 256-10240, 256-8000 rows): 6 % faster on average than 256-row tiles from
-// 2048 rows on, nothing more than 5 % slower (8192 x 2048, 2047 rows 86 -> 62 us, 16640 x 2048, 1500 rows 123 -> 106; 1024 x
-// 10240, 4100 rows 118 -> 105; missed by the estimates: 65536 x 1024, 600 rows, 124 instead of 101).
+// both at 630 products (18 shapes of 512-65536 columns, K 256-10240, 256-8000 rows) against 256-row tiles from 2048 rows on: 5 %
+// less time on average (8192 x 2048, 2047 rows 86 -> 62 us, 16640 x 2048, 1500 rows 123 -> 106; 1024 x 10240, 4100 rows 118 -> 105).
+// Two are slower, 4128 x 256 with 4000 and 4096 rows, 32 -> 33.5: the others' estimate leaves out what writes of short K cost.  A
+// margin of 1.15 instead of 1.1 mends these and costs more elsewhere (5120 x 2880, 3100 rows 97 -> 112, 2560 x 320, 2500 rows
+// 14.7 -> 17.5).  Missed by the estimates: 65536 x 1024, 600 rows, 122 instead of 100.
 static bool dense_tall(int B, int N, int K, double other_us) {
   if (dense_tall_min_rows() > 0) return B >= dense_tall_min_rows();
   return tall_us(B, N, K) < (B < 2048 ? 0.88 : 1.1) * other_us;
