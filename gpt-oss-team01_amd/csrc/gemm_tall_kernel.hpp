@@ -287,7 +287,7 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
       t.row0 = tile * SH::BM;
       t.rows = min(SH::BM, p.dense_rows - t.row0);
     }
-    if (part) {   // whole row blocks; where there is but one the second half has no rows
+    if (part) {   // whole row blocks; where there is but one the second half has no rows, and is no item
       const int first = min(t.rows, ((t.rows + 63) >> 6) * 32);
       if (((jj - whole) & 1) == 0) t.rows = first;
       else {
@@ -318,7 +318,7 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
   if constexpr (GATHER) inv_k = pair_inverse(p.top_k);
   auto a_offsets = [&](TallSrc<SH> &t) {
     typedef int ids_t __attribute__((ext_vector_type(8), aligned(4)));
-    const int last = max(t.rows - 1, 0), group = lane >> 3;
+    const int last = t.rows - 1, group = lane >> 3;
     auto offset = [&](int src, int r) {
       const int c = (lane & 7) ^ ((r >> 1) & 7);
       return ((uint32_t)src * (uint32_t)K) * 2u + (uint32_t)c * 16u;
@@ -400,6 +400,7 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
 
   TallSrc<SH> cur, nxt;
   decode(j, cur);
+  if (cur.rows == 0) return;
   a_offsets(cur);
   // The first loads go out in the order the stage loop would have issued them, so that its waits
   // count right from the first stage on: chunk 0 and W stage 0, then a quarter of chunk 1 with
@@ -431,12 +432,13 @@ __global__ __launch_bounds__(TALL_THREADS, 1) void tall_gemm_kernel(GemmParams p
   const uint32_t voff_w1 = voff_w + 1024;
   while (true) {
     const int jn = j + per_xcd;
-    const bool more = valid(jn);
-    nxt = cur;  // past the last item the pipeline requests this item's first loads again, and drops them
+    bool more = valid(jn);
     if (more) {
       decode(jn, nxt);
-      a_offsets(nxt);
+      more = nxt.rows > 0;   // (an empty half belongs to the last round, so nothing comes behind it)
     }
+    if (more) a_offsets(nxt);
+    else nxt = cur;  // past the last item the pipeline requests this item's first loads again, and drops them
 #pragma unroll
     for (int i = 0; i < CB; i++)
 #pragma unroll
