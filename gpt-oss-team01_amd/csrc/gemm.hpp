@@ -15,6 +15,7 @@ struct GemmBf16Range {
   int ld = 0;             // elements per row, a multiple of 4
   int relu_squared = 0;   // the square of relu instead of the value itself
 };
+static_assert(sizeof(GemmBf16Range) == 24 && __builtin_offsetof(GemmBf16Range, ld) == 16);   // tests lay it out field by field
 
 // The gated activation of an expert's first product (EPI_SWIGLU):
 //   g sigmoid(rate g) (u + shift),  g = min(gate, limit), u = up clamped to [-limit, limit].
@@ -57,8 +58,8 @@ struct GemmParams {
   int split_slabs;     // 64-k slabs; part s is written to out + s * dense_rows * N (no bias)
 };
 
-// rows_per_tile in {32,64,96,128,160}, or 256 where gemm_tall_applies(); max_tiles bounds the number of
-// (mat,row-tile) items.
+// rows_per_tile in {32,64,96,128,160}, or 256 where gemm_tall_applies(); MXFP4 weights: 32 or 64, grouped problems only.
+// max_tiles bounds the number of (mat,row-tile) items.
 int run_gemm(const GemmParams &p, bool gather, int epi, int rows_per_tile, int max_tiles,
              hipStream_t s);
 // gemm_few.hip: tiles of at most 32 or 64 rows, one wave per 32 columns or 16 (bf16 weights; gather + SwiGLU, or no gather and

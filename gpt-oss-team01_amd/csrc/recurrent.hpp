@@ -1,6 +1,8 @@
 // Internal interface of the recurrent mixers (recurrent.hip): short causal convolution, the gated
 // delta rules, the state-space recurrence and retention, and their gated output norms.
 #pragma once
+#include <stddef.h>
+
 #include "engine.hpp"
 #include "rotary.hpp"
 
@@ -53,6 +55,10 @@ struct Scan {
   float *conv_state = nullptr;
   int vec = 0;            // the launch's choice of loads (retention chunks: of stores), 16 bytes at a time
 };
+// tests/test_scan_chunks_gpu.py lays these out field by field
+static_assert(sizeof(ShortConv) == 48 && offsetof(ShortConv, unit_scale) == 40 && sizeof(Scan) == 240 &&
+              offsetof(Scan, channel_decay) == 72 && offsetof(Scan, rot) == 136 && offsetof(Scan, vec) == 232);
+static_assert(sizeof(StepRows) == 104 && offsetof(StepRows, singles) == 64 && offsetof(StepRows, longest) == 76);
 inline int scan_key_pad(int K) { return (K + 31) / 32 * 32; }
 inline size_t scan_state_elems(int heads, int K, int V) { return (size_t)heads * V * scan_key_pad(K); }
 // rows may be read 16 bytes at a time
