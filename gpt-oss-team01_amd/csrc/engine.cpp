@@ -40,7 +40,10 @@ constexpr size_t LOGITS_HALF = 2 << 20;
 constexpr size_t LOGITS_PIECE = 128 << 10;   // what a thread copies out at a time, from LOGITS_SHARED bytes on
 constexpr size_t LOGITS_SHARED = 512 << 10;
 constexpr int LOGITS_CHUNKS = LOGITS_HALF / LOGITS_CHUNK;
-constexpr int LOGITS_SPINS = 20000;   // looks at a chunk's word, about a millisecond, before the thread waits for the kernel's end
+// Looks at a chunk's word, a third of a millisecond to a whole one by the CPU's pause, before the thread waits for the kernel's end.
+// A longer step than that is waited for to the end (GPT-OSS: 2 ms, and 20 us for the kernel with its row of logits); only the
+// calling thread looks for a half's first chunk, the crew's begin with it.
+constexpr int LOGITS_SPINS = 20000;
 
 int gptoss_engine::create_logits_staging() {
   GPTOSS_HIP(hipHostMalloc((void **)&h_logits, 2 * LOGITS_HALF + 2 * LOGITS_CHUNKS * sizeof(uint32_t), hipHostMallocCoherent));
@@ -399,8 +402,9 @@ static int generate_lockstep(gptoss_engine *e, const int *host_prompts, const in
 
 // Continuous batching: max_batch slots; a slot whose sequence ended (stop id or its length limit)
 // takes the next waiting request at once, while the other slots carry on at their own positions.
-// Every request sees the arithmetic it would see alone, so its output is the one the lock-step
-// schedule gives; only the order of the work changes.  host_max_len (optional) limits request r
+// Every request sees the arithmetic it would see alone (sums over K in parts, over attention's chunks and
+// over a prompt's chunks in the recurrences to rounding, which depend on the rows of a step and on where a
+// prompt is cut), so its output is the one the lock-step schedule gives; only the order of the work changes.  host_max_len (optional) limits request r
 // to host_max_len[r] positions in all (prompt included) instead of max_seq_len.
 //
 // Prompts are not forced one token per step (getp_run_submit.cpp:67-72 does that).  The positions

@@ -13,8 +13,8 @@
 // Measured against the streaming kernel with 64-row tiles (both products, 2880 x 2880, us): 128 experts, 4096 tokens
 // 707 + 380 -> 595 + 327 (Zipf 1.1), 700 + 377 -> 576 + 314 (uniform), 850 tokens 275 + 151 -> 234 + 131; 32 experts, 4096
 // tokens 586 + 317 -> 495 + 272, 500 tokens 118 + 77 -> 101 + 62.  4096 tokens on all of 4 experts (no tile with less than
-// 64 rows) 637 + 361 -> 454 + 248: 1.2 PFLOP/s, matrix cores 61 % busy at 1.7 GHz; what is left is waves that wait for each
-// other at the barriers, and tiles and rounds that are not full.
+// 64 rows) 637 + 361 -> 454 + 248: 1.2 PFLOP/s, matrix cores 67 and 57 % busy (775 and 456 thousand cycles), waves waiting 45 %
+// of their cycles; what is left is waves that wait for each other at the barriers, and tiles and rounds that are not full.
 // Not kept: tiles of 128 rows (two workgroups a CU, two waves per SIMD: 4096 tokens 964 -> 1036), 96 rows (1058), W straight
 // into registers a stage ahead (955 -> 995: the registers of a wave more), a higher priority for the waves that multiply
 // (within 1 %).

@@ -402,7 +402,10 @@ int gptoss_engine_prefill(gptoss_engine *e, const int *host_tokens, int B, int T
  * decoding, so they share that step's passes over the weights (on sliding-window layers only
  * while they stay inside the ring's first lap; later prompt positions are forced as before).
  * Every request gets the arithmetic it would get alone, so the output is that of the reference's
- * batch-by-batch lock-step schedule. */
+ * batch-by-batch lock-step schedule.  That is bit for bit but for sums that are equal to rounding only:
+ * over K in parts and over attention's chunks, which depend on the rows of a step; the recurrences of a
+ * prompt, which run in chunks (state space: stretches of 48 rows and more of one sequence; retention:
+ * steps with a stretch of more than 8) and so depend on where the schedule cuts it. */
 int gptoss_engine_generate(gptoss_engine *e, const int *host_prompts, const int *host_n_prompt,
                            int prompt_stride, int n_req, int max_seq_len, int *host_out,
                            long long *n_generated);
