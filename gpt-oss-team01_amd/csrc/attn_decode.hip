@@ -42,21 +42,29 @@ namespace gptoss {
 constexpr int ATT_BLOCK = 64;   // slots per inner iteration
 constexpr float NEG_BIG = -1.0e30f;
 
-// The hardware's exponential by itself: a weight below 2^-126 of its row's largest is zero.  (The library function scales
-// such arguments first, five more instructions per score where a block step has about 300 in all; the row's largest weight
-// is about 1, so a sum in fp32 is the same with them or without.)
+// The hardware's exponential by itself: a weight below 2^-126 is zero.  (The library function scales such arguments first, five
+// more instructions per score where a block step has about 300 in all; the row's largest weight is between 1/2 and 16, so a sum
+// in fp32 is the same with them or without.)
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// The reference that a row's weights are taken against, from a block's largest score: raised only by more than RAISE_FROM, to
+// the next whole number, so that most blocks behind a row's first rescale nothing, and where one does the factor is a power of
+// two, without a rounding.
+constexpr float RAISE_FROM = 4.f;
+__device__ __forceinline__ bool raises_reference(float m, float top) { return top > m + RAISE_FROM; }
+__device__ __forceinline__ float raise_reference(float m, float top) { return raises_reference(m, top) ? ceilf(top) : m; }
 
 // What a row's sum, of maximum m, and its sink are weighed against: the larger of the two, but not so far above m that
 // exp2_hw has no weight left for the sum.  (A sink may lie more than 126 above every score, and bf16 still hold the output.)
 __device__ __forceinline__ float sink_reference(float m, float sink2) { return fminf(fmaxf(m, sink2), m + 100.f); }
 
-// What the exponential of a block's scores is taken of: the distance of score * scale (powers of two) from the row's running
-// maximum m.  Scaling and difference are one fused operation, in every form of the kernels and in blocks with and without
-// masked slots alike: a row's result must not depend on what its partner row in a wave forces.  The maximum is a rounded
-// product, so its own distance is that rounding error and its weight within 2^(|m| 2^-24) of 1, a factor that all weights
-// of the row share.  From 2^24 on the error is a power of two and more (beyond 2^31 the maximum's weight would overflow or
-// vanish): such rows take the difference of rounded products, the maximum's distance is 0.
+// What the exponential of a block's scores is taken of: the distance of score * scale (powers of two) from the row's
+// reference m.  Scaling and difference are one fused operation, in every form of the kernels and in blocks with and without
+// masked slots alike: a row's result must not depend on what its partner row in a wave forces.  The reference comes from a rounded
+// product, so the distance of the score behind it is off by that rounding error, 2^(|m| 2^-24), a factor that all weights
+// of the row share.  From 2^24 on the error is a power of two and more (beyond 2^31 the largest weight would overflow or
+// vanish): such rows take the difference of rounded products, whole numbers both, and the largest score's distance is 0 or
+// what RAISE_FROM lets pass.
 // any_huge: whether the wave has one.
 __device__ __forceinline__ bool huge_maximum(float m) { return fabsf(m) >= 16777216.f && m != NEG_BIG; }
 __device__ __forceinline__ void weight_exponents(f32x4 (&s4)[4], float scale, float m, bool any_huge) {
@@ -86,35 +94,34 @@ __device__ __forceinline__ void split_weights(float p0, float p1, uint32_t &h, u
   l = __builtin_amdgcn_perm(__float_as_uint(r1), __float_as_uint(r0), 0x07060302u);
 }
 
-// A lane's KS * 8 values of a query row as bf16 hi + lo operands; a column without a row or head is zero.  qp points to a
-// real row whether the column has one or not, so that the loads are whole and unconditional (sixteen conditional ones of
-// four bytes: 64 prompts of 125 positions 104 instead of 73 us, eight of 1000 195 instead of 181).
+// A lane's KS * 8 values of a query row as bf16 hi + lo operands.  qp points to a real row whether the column has one or
+// not, so that the loads are whole and unconditional (sixteen conditional ones of four bytes: 64 prompts of 125 positions 104
+// instead of 73 us, eight of 1000 195 instead of 181): a column without a row or head repeats another's, and is not stored.
 template <int N>
 __device__ __forceinline__ void load_query(const float *qp, f32x4 (&x)[N]) {
 #pragma unroll
   for (int i = 0; i < N; i++) x[i] = *reinterpret_cast<const f32x4 *>(qp + i * 4);
 }
 template <int KS>
-__device__ __forceinline__ void split_query(const f32x4 (&x)[2 * KS], bool live, bf16x8 (&qh)[KS], bf16x8 (&ql)[KS]) {
+__device__ __forceinline__ void split_query(const f32x4 (&x)[2 * KS], bf16x8 (&qh)[KS], bf16x8 (&ql)[KS]) {
 #pragma unroll
   for (int s = 0; s < KS; s++) {
     uint32_t h[4], l[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-      const float x0 = live ? x[2 * s + (j >> 1)][(j & 1) * 2] : 0.f, x1 = live ? x[2 * s + (j >> 1)][(j & 1) * 2 + 1] : 0.f;
-      const bf16_t h0 = f32_to_bf16(x0), h1 = f32_to_bf16(x1);
-      h[j] = (uint32_t)h0 | ((uint32_t)h1 << 16);
-      l[j] = pack_bf16x2(x0 - bf16_to_f32(h0), x1 - bf16_to_f32(h1));
+      const float x0 = x[2 * s + (j >> 1)][(j & 1) * 2], x1 = x[2 * s + (j >> 1)][(j & 1) * 2 + 1];
+      h[j] = pack_bf16x2(x0, x1);
+      l[j] = pack_bf16x2(x0 - __uint_as_float(h[j] << 16), x1 - __uint_as_float(h[j] & 0xffff0000u));
     }
     qh[s] = as_bf16x8(u32x4{h[0], h[1], h[2], h[3]});
     ql[s] = as_bf16x8(u32x4{l[0], l[1], l[2], l[3]});
   }
 }
 template <int KS>
-__device__ __forceinline__ void split_query(const float *qp, bool live, bf16x8 (&qh)[KS], bf16x8 (&ql)[KS]) {
+__device__ __forceinline__ void split_query(const float *qp, bf16x8 (&qh)[KS], bf16x8 (&ql)[KS]) {
   f32x4 x[2 * KS];
   load_query(qp, x);
-  split_query<KS>(x, live, qh, ql);
+  split_query<KS>(x, qh, ql);
 }
 
 struct AttnParams {
@@ -128,6 +135,7 @@ struct AttnParams {
   float *part_ml;      // [B, max_chunks, n_q, 2]
   int B, n_q, n_kv, G, cap, window, max_chunks, max_len;
   int rows_per_seq;    // query rows per cached sequence: row b reads the cache of sequence b / rows_per_seq
+  int n_seq, row_groups;   // prompt tiles: sequences, and groups of TILE_ROWS rows of each
   float scale_log2e;   // log2(e) / sqrt(D)
   int only_single;     // chunked kernels: leave rows of more than one chunk to the workgroup-per-row kernel
   const int2 *order;   // workgroup-per-row kernel: (row, its length) by descending slot span (nullptr: row order)
@@ -355,7 +363,7 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
   if (c1 > c0) load_kv(c0, R0{});
 
   bf16x8 qh[KS], ql[KS];
-  split_query<KS>(p.q + ((size_t)bn * p.n_q + head) * D + c * KS * 8, col_live, qh, ql);
+  split_query<KS>(p.q + ((size_t)bn * p.n_q + head) * D + c * KS * 8, qh, ql);
 
   f32x4 o[DB];
 #pragma unroll
@@ -394,7 +402,7 @@ __device__ __forceinline__ void attn_decode_body(const AttnParams &p, const int 
         }
         bmax = fmaxf(bmax, s4[tb][i]);
       }
-    const float m_new = fmaxf(m_run, max_over_quarters(bmax) * p.scale_log2e);
+    const float m_new = raise_reference(m_run, max_over_quarters(bmax) * p.scale_log2e);
     const float alpha = exp2_hw(m_run - m_new);
     m_run = m_new;
     weight_exponents(s4, p.scale_log2e, m_new, __ballot(huge_maximum(m_new)) != 0);
@@ -747,7 +755,7 @@ __device__ __forceinline__ void attn_few_chunk(const AttnParams &p, const RopeIn
     }
   }
   bf16x8 qh[KS], ql[KS];
-  split_query<KS>(qx, n < G, qh, ql);
+  split_query<KS>(qx, qh, ql);
 
   f32x4 s4[2][4];
 #pragma unroll
@@ -785,7 +793,7 @@ __device__ __forceinline__ void attn_few_chunk(const AttnParams &p, const RopeIn
 #pragma unroll
   for (int j = 0; j < NBLK; j++) {
     if (j >= nb) break;
-    const float m_new = fmaxf(m_run, lds_max[j][n]);
+    const float m_new = raise_reference(m_run, lds_max[j][n]);
     alpha[j] = exp2_hw(m_run - m_new);
     m_run = m_new;
     if (j % 4 == wave) m_own[j / 4] = m_run;
@@ -959,15 +967,20 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 // and walks the K/V blocks any of them needs ONCE: every block goes from global memory into LDS
 // (two buffers, one barrier per block) and the eight waves take their operands from there.  The
 // pair form reads a sequence's cache once per row pair, which is quadratic traffic for long
-// prompts; here it is read once per 16 rows.  What bounds it is the vector units (68 % busy, the matrix cores 36 %): per
-// 64 x 16 scores a wave issues about 170 of their instructions, a tenth of them exponentials.  Eight prompts of 1000
-// positions, 64 heads: 237 -> 211 us with the exponential, the maximum and the splitting of weights in fewer instructions
-// (exp2_hw, max_over_quarters, split_weights), -> 195 with the scale fused into the exponent's difference
-// (weight_exponents), one range check per masked slot and blocks straight into LDS, -> 181 with whole loads of q
-// (split_query), and, on another box, 160 -> 151 with one instance of a block's step, whose masks and rescaling are branches
-// (one prompt of 2048: 74 -> 72, window of 128: 76 -> 70, three of 33 positions behind 450: 14.6 -> 13.7).  Two blocks to a
+// prompts; here it is read once per 16 rows.  What bounds it is power, and the vector
+// units next (68 % busy, the matrix cores 36 %): per 64 x 16 scores a wave issues about 150 of their instructions, a tenth of them
+// exponentials.  Eight prompts of 1000 positions, 64 heads: 237 -> 211 us with the exponential, the maximum and the splitting of
+// weights in fewer instructions (exp2_hw, max_over_quarters, split_weights), -> 195 with the scale fused into the exponent's
+// difference (weight_exponents), one range check per masked slot and blocks straight into LDS, -> 181 with whole loads of q
+// (split_query), and, on another box, 160 -> 151 with one instance of a block's step, whose masks and rescaling are branches.
+// On a third, 170 -> 161 with references that are seldom raised (raise_reference: before, a larger score for any of a wave's 16
+// columns made it rescale, as nearly every block of a prompt brings one), K pieces swizzled for the order in which LDS serves a
+// wave (below) and a shorter beginning; prompts of 485 / 700 positions 16.9 / 19.6 -> 15.9 / 18.1, three of 1427 behind 87 122 ->
+// 115, three of 33 behind 450 13.6 -> 12.6, eight of 1000 with a window of 128 75 -> 70.
+// Four rows per wave on 32x32x16 products, the same bits with half of the LDS reads and 11 % fewer cycles: within 2 %, because
+// the clock falls with them (2.06 -> 1.98 GHz), and 5 to 10 % slower where the workgroups do not fill the chip.  Two blocks to a
 // barrier are as fast; 80 registers for six waves per SIMD spill (180); the remainders of the split weights by dot
-// products, half the instructions: as fast.
+// products, half the instructions: 2 % slower.
 // Every row sees the arithmetic of the one-wave kernel over its own blocks in ascending order (a
 // block outside a row's range is a no-op for its columns), so rows of up to ATT_CHUNK positions
 // equal the decode call bit for bit; longer rows are summed in one pass instead of chunk by
@@ -989,14 +1002,10 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int T = p.rows_per_seq;
-  const int groups = (T + TILE_ROWS - 1) / TILE_ROWS;
-  const int n_seq = p.B / T;
   // late row groups first: they walk the most blocks
-  const int g = blockIdx.x % p.n_kv;
-  const int rest = blockIdx.x / p.n_kv;
-  const int seq = rest % n_seq;
-  const int rg = groups - 1 - rest / n_seq;
-  const int t0 = rg * TILE_ROWS;                             // first row of the group within the sequence
+  const int rest = blockIdx.x / p.n_kv, g = blockIdx.x - rest * p.n_kv;
+  const int late = rest / p.n_seq, seq = rest - late * p.n_seq;
+  const int t0 = (p.row_groups - 1 - late) * TILE_ROWS;                             // first row of the group within the sequence
   const int t_last = min(T, t0 + TILE_ROWS) - 1;
   // active positions of row t: [lo(t), hi(t)), hi(t) = len_base + t
   auto row_hi = [&](int t) { return min(p.len_base + t, p.max_len); };
@@ -1022,10 +1031,12 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
   const unsigned char *plane =
       reinterpret_cast<const unsigned char *>(p.kv + kv_block_off(cache_seq, g, p.n_kv, p.cap, D, 0));
   // The workgroup's copy of a block goes from memory straight into LDS, in pieces of 16 bytes: thread t's load i lands at
-  // piece i * 512 + t.  Position j of K row r is to hold chunk j ^ swz(r), so that the 16 lanes of a fragment read (16
-  // rows, one chunk) hit 16 different 16-byte slots modulo 256 bytes: the lane fetches that chunk.  (Through registers,
-  // the loop's eight of them and the store's addresses do not fit the 128 of two workgroups per CU beside the rest.)
-  auto swz = [](int r) { return D == 64 ? ((r >> 1) & 7) : ((r >> 2) & 3); };
+  // piece i * 512 + t.  Position j of K row r is to hold chunk j ^ swz(r), the chunk that the lane fetches: LDS serves lanes 0-3,
+  // 12-15 and 20-27 of a fragment read (16 rows, one chunk per quarter) together, then 4-11, 16-19 and 28-31, and the upper half
+  // alike, and these are to hit 16 different 16-byte slots modulo 256 bytes.  (A third of the cycles of all reads went into
+  // conflicts where 16 lanes in a row did so.)  (Through registers, the loop's eight of them and the store's addresses do not
+  // fit the 128 of two workgroups per CU beside the rest.)
+  auto swz = [](int r) { return D == 64 ? ((r >> 1) & 7) ^ (r & 4) : ((r >> 2) & 3) ^ ((r >> 1) & 2); };
   uint32_t src_off[PASSES];
 #pragma unroll
   for (int i = 0; i < PASSES; i++) {
@@ -1043,7 +1054,7 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
   if (blk_end > blk_begin) request_block(blk_begin, 0);
 
   bf16x8 qh[KS], ql[KS];
-  split_query<KS>(p.q + ((size_t)bn * p.n_q + head) * D + c * KS * 8, col_live, qh, ql);
+  split_query<KS>(p.q + ((size_t)bn * p.n_q + head) * D + c * KS * 8, qh, ql);
 
   f32x4 o[DB];
 #pragma unroll
@@ -1092,8 +1103,8 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
     // of 1 otherwise.
     const float top = bmax * p.scale_log2e;
     float alpha = 1.f;
-    if (__ballot(top > m_run) != 0) {
-      const float m_new = fmaxf(m_run, max_over_quarters(top));
+    if (__ballot(raises_reference(m_run, top)) != 0) {
+      const float m_new = raise_reference(m_run, max_over_quarters(top));
       alpha = exp2_hw(m_run - m_new);
       m_run = m_new;
 #pragma unroll
@@ -1355,6 +1366,8 @@ static int attn_launch(const float *q, const void *kv_cache, const int *lens,
     const long long wgs = (long long)(B / rows_per_seq) * n_kv * ((rows_per_seq + TILE_ROWS - 1) / TILE_ROWS);
     GPTOSS_REQUIRE(wgs < (1ll << 31), GPTOSS_ERR_DIM, "attn_prefill: too many row groups (%lld)", wgs);
     TraceScope ts("attn_prefill_tiles", s);
+    p.n_seq = B / rows_per_seq;
+    p.row_groups = cdiv(rows_per_seq, TILE_ROWS);
     if (head_dim == 64) attn_prefill_tile_kernel<64><<<(int)wgs, TILE_WAVES * 64, 0, s>>>(p);
     else attn_prefill_tile_kernel<32><<<(int)wgs, TILE_WAVES * 64, 0, s>>>(p);
     GPTOSS_LAUNCH_CHECK("attn_prefill_tile_kernel");
