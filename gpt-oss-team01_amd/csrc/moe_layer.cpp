@@ -56,13 +56,22 @@ static int env_int(const char *name, int dflt) {
   const int n = e ? atoi(e) : 0;
   return n > 0 ? n : dflt;
 }
-// Average rows per expert from which a bf16 MoE block uses the 256-row kernels of gemm_tall.hip.  Between 416 and 512 they gain
-// 2-23 % (both routings, uniform and Zipf 1.1; 2880 x 2880, 32 experts of 437 rows 877 -> 790 us; below, the second tile of
-// an expert has too few rows: 290 rows 646 against 709) where there is work for the whole chip: blocks of 1024 x 512 on 16
-// experts lose 13 %, blocks of four times the arithmetic gain.
-static int moe_tall_min_rows(long long pairs, int N, int K) {
+// Whether a bf16 MoE block uses the 256-row kernels of gemm_tall.hip, by its average rows per expert.
+// From 416 on they gain 2-23 % (both routings, uniform and Zipf 1.1; 2880 x 2880, 32 experts of 437 rows 877 -> 790 us) where there
+// is work for the whole chip: blocks of 1024 x 512 on 16 experts lose 13 %, blocks of four times the arithmetic gain, so small ones
+// from 512 on.
+// From 165 to 248 an expert's rows are two 160-row tiles and one of 256 (2880 x 2880, uniform / Zipf 1.1, streaming -> 256-row
+// kernels, us: 32 experts of 160 rows 530 / 541 -> 475 / 564, 175 623 / 577 -> 509 / 578, 200 702 / 622 -> 542 / 608, 240
+// 684 / 698 -> 595 / 669, 248 717 / 693 -> 663 / 683; 64 of 200 1314 / 1164 -> 993 / 1138; 16 of 200 350 / 332 -> 285 / 339).  Below,
+// one of 160 holds them (150 rows 496 / 531 -> 479 / 555, 128 391 / 506 -> 434 / 505), above two of either (275 692 / 737 ->
+// 790 / 704, 325 837 / 802 -> 861 / 784).  Small blocks lose here too: 2048 x 1024, 32 experts of 200 210 / 212 -> 227 / 213, eight of
+// 2880 x 2880 187 / 173 -> 163 / 187.
+static bool moe_tall(long long pairs, int E, int N, int K) {
   static const int v = env_int("GPTOSS_MOE_TALL_MIN_ROWS", 0);
-  return v ? v : (double)pairs * N * K >= (double)(1ll << 34) ? 416 : 512;
+  if (v) return pairs >= (long long)v * E;
+  const double work = (double)pairs * N * K;
+  if (pairs >= (long long)(work >= (double)(1ll << 34) ? 416 : 512) * E) return true;
+  return work >= (double)(1ll << 35) && pairs >= 165ll * E && pairs <= 248ll * E;
 }
 
 int moe_rows_per_tile(int B, int k, int E, bool mxfp4) {
@@ -150,8 +159,7 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
   // a prompt pass, hundreds of rows per expert: bound by the matrix cores, not by streaming W
   // (the kernels address a row of A by a 32-bit byte offset: batches beyond that stay on the streaming kernels)
   const long long tall_rows = ((long long)B * k / 256 + E) * 256;
-  if (!mxfp4 && (long long)B * k >= (long long)moe_tall_min_rows((long long)B * k, 2 * I, H) * E && gemm_tall_shape_ok(2 * I, H, tall_rows) &&
-      gemm_tall_shape_ok(H, I, tall_rows))
+  if (!mxfp4 && moe_tall((long long)B * k, E, 2 * I, H) && gemm_tall_shape_ok(2 * I, H, tall_rows) && gemm_tall_shape_ok(H, I, tall_rows))
     rpt = 256;
   // (no more experts have a row than there are rows)
   const int max_tiles = gptoss_moe_max_tiles(B, k, std::min(E, B * k), rpt);

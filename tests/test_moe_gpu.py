@@ -491,6 +491,20 @@ def test_row_blocks_of_a_prompt_pass(ops, rows):
     test_last_row_tiles_of_a_prompt_pass(ops, rows)
 
 
+@pytest.mark.parametrize("rows", [164, 165, 200, 248, 249])
+def test_large_blocks_of_one_and_two_row_tiles_per_expert(ops, rows):
+    """Every token on all of 4 experts of 4096 x 8640: one 256-row tile from 165 rows to 248, two 160-row tiles outside."""
+    E, H, I = 4, 4096, 8640
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    layer = ops.MoeLayer(n(E, H), n(E).float(), n(E, 2 * I, H, std=0.02), n(E, 2 * I).float(), n(E, H, I, std=0.02),
+                         n(E, H).float(), max_tokens=rows)
+    t = n(rows, H)
+    out = layer.forward(t).clone()
+    for i in range(0, rows, 64):
+        assert torch.equal(layer.forward(t[i:i + 64].contiguous()), out[i:i + 64]), i
+
+
 @pytest.mark.parametrize("k", [1, 2, 3, 5, 7, 8])
 def test_tokens_of_pairs_in_a_prompt_pass(ops, k):
     """Every token on all k experts: the token of a pair is the pair's number over k."""
