@@ -333,18 +333,23 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
   const bf16_t *ap = t + (size_t)arow * H + kq;
   constexpr int ROUTER_MAX_STEPS = router_steps(NB);
   const int ksteps = H / 32;
-  u32x4 a[ROUTER_MAX_STEPS], b[ROUTER_MAX_STEPS][NB];
-  auto load_b = [&](int ks0) {
+  // In two halves: while one is multiplied, the other's loads are on their way (2880 inputs, 64 experts 16.3 -> 13.9 us, a third
+  // round of loads for the second one's last steps less; 128 25.0 -> 24.5).  More than 128 experts leave no registers for it.
+  constexpr int SETS = NB <= 8 ? 2 : 1, HALF = (ROUTER_MAX_STEPS + SETS - 1) / SETS, STRIDE = HALF * ROUTER_WAVES;
+  u32x4 a[SETS][HALF], b[SETS][HALF][NB];
+  auto load_b = [&](int ks0, auto set) {
 #pragma unroll
-    for (int u = 0; u < ROUTER_MAX_STEPS; u++) {
+    for (int u = 0; u < HALF; u++) {
       const int ks = min(ks0 + u * ROUTER_WAVES, ksteps - 1);
 #pragma unroll
       for (int nb = 0; nb < NB; nb++) {
         int e = min(e0 + nb * 16 + (lane & 15), E - 1);
-        b[u][nb] = *reinterpret_cast<const u32x4 *>(wr + (size_t)e * H + ks * 32 + kq);
+        b[decltype(set)::value][u][nb] = *reinterpret_cast<const u32x4 *>(wr + (size_t)e * H + ks * 32 + kq);
       }
     }
   };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, SETS - 1>;
   // the bias of the experts that the lane sums up in the end
   const int row = threadIdx.x >> 5, sub = threadIdx.x & 31;
   constexpr int NJ = (NB + 1) / 2;
@@ -355,7 +360,9 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
   // in order, so the bias is in front of them, and a wave without a k-step requests none: behind twelve steps' loads in each
   // of eight waves, of which H = 64 has work for two, 32 / 128 experts took 7.0 / 9.1 us instead of 3.1 / 3.7.
   constexpr bool EARLY = !NORM || NB <= 8;
-  if (EARLY && wave < ksteps) load_b(wave);
+  static_assert(EARLY || SETS == 1, "two sets are requested early");
+  if (EARLY && wave < ksteps) load_b(wave, S0{});
+  if (SETS == 2 && EARLY && wave + STRIDE < ksteps) load_b(wave + STRIDE, S1{});
   if constexpr (NORM) {
     constexpr int VPT = 4;  // rows of up to 4096 floats
     __shared__ double nred[2][4];
@@ -420,17 +427,42 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
   f32x4 acc[NB];
 #pragma unroll
   for (int nb = 0; nb < NB; nb++) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int ks0 = wave; ks0 < ksteps; ks0 += ROUTER_WAVES * ROUTER_MAX_STEPS) {
-    if (!EARLY || ks0 != wave) load_b(ks0);
+  auto load_a = [&](int ks0, auto set) {
 #pragma unroll
-    for (int u = 0; u < ROUTER_MAX_STEPS; u++)
-      a[u] = *reinterpret_cast<const u32x4 *>(ap + min(ks0 + u * ROUTER_WAVES, ksteps - 1) * 32);
+    for (int u = 0; u < HALF; u++)
+      a[decltype(set)::value][u] = *reinterpret_cast<const u32x4 *>(ap + min(ks0 + u * ROUTER_WAVES, ksteps - 1) * 32);
+  };
+  auto multiply = [&](int ks0, auto set) {
 #pragma unroll
-    for (int u = 0; u < ROUTER_MAX_STEPS; u++) {
+    for (int u = 0; u < HALF; u++) {
       if (ks0 + u * ROUTER_WAVES < ksteps) {
 #pragma unroll
         for (int nb = 0; nb < NB; nb++)
-          acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[u]), as_bf16x8(b[u][nb]), acc[nb], 0, 0, 0);
+          acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[decltype(set)::value][u]),
+                                                            as_bf16x8(b[decltype(set)::value][u][nb]), acc[nb], 0, 0, 0);
+      }
+    }
+  };
+  if constexpr (SETS == 1) {
+    for (int ks0 = wave; ks0 < ksteps; ks0 += STRIDE) {
+      if (!EARLY || ks0 != wave) load_b(ks0, S0{});
+      load_a(ks0, S0{});
+      multiply(ks0, S0{});
+    }
+  } else if (wave < ksteps) {
+    load_a(wave, S0{});
+    if (wave + STRIDE < ksteps) load_a(wave + STRIDE, S1{});
+    for (int ks0 = wave; ks0 < ksteps; ks0 += 2 * STRIDE) {
+      multiply(ks0, S0{});
+      if (ks0 + 2 * STRIDE < ksteps) {
+        load_b(ks0 + 2 * STRIDE, S0{});
+        load_a(ks0 + 2 * STRIDE, S0{});
+      }
+      if (ks0 + STRIDE >= ksteps) break;
+      multiply(ks0 + STRIDE, S1{});
+      if (ks0 + 3 * STRIDE < ksteps) {
+        load_b(ks0 + 3 * STRIDE, S1{});
+        load_a(ks0 + 3 * STRIDE, S1{});
       }
     }
   }
@@ -706,7 +738,16 @@ int run_topk_softmax(const float *logits, int B, int E, int k, float *topk_w, in
   return GPTOSS_OK;
 }
 
+// Token rows of a workgroup: as few as leave no more workgroups than CUs, where a workgroup has a CU to itself (eight waves with
+// the registers of two per SIMD) and takes the time of its share of the experts' weights whatever its rows are.  2880 inputs, 32 / 128 experts: 1100
+// to 2000 tokens in groups of four 15.9 / 48.5 us, of eight 8.8 / 25.0; 2100 to 4000 in groups of eight 16.7 / 49.8, of 16 9.8 / 26.5.
 static int router_rows_per_wg(int B) {
+  int rows_per_wg = 4;
+  while (rows_per_wg < 16 && cdiv(B, rows_per_wg) > 256) rows_per_wg *= 2;
+  return rows_per_wg;
+}
+// With the norm in front (norm_router_applies): two rows at a time by a workgroup, so four even where that is more of them.
+static int norm_router_rows_per_wg(int B) {
   int rows_per_wg = 16;
   while (rows_per_wg > 4 && cdiv(B, rows_per_wg) < 256) rows_per_wg >>= 1;
   return rows_per_wg;
@@ -753,7 +794,7 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
   // 16 token rows per workgroup fill the MFMA, but a thousand tokens are then only 64 workgroups;
   // with fewer rows each (the rest of the MFMA rows idle) all CUs take part in what is a
   // latency-bound launch: every workgroup reads the whole router matrix from L2 either way
-  // (1024 tokens over 32 experts: 19.7 us with 16 rows, 16.7 with 8, 15.6 with 4, 27 with 2)
+  // (with the gating, 1024 tokens over 32 experts: 19.7 us with 16 rows, 16.7 with 8, 15.6 with 4, 27 with 2)
   const RouterGroup grp = group ? *group : RouterGroup{};
   const int rows_per_wg = grp.expert_offsets ? ROUTER_GROUP_TOKENS : router_rows_per_wg(B);
   GPTOSS_REQUIRE(!grp.expert_offsets || (topk_w && router_groups(B, k)), GPTOSS_ERR_DIM, "router: %d tokens are not grouped here", B);
@@ -822,12 +863,12 @@ static int launch_norm_router(const RouterNorm &nrm, const bf16_t *wp, const flo
 bool norm_router_applies(int B, int H, int E, const float *x, const float *residual, const float *weight,
                          const void *t_out) {
   const int nb = router_col_blocks(E);
-  const size_t lds = (size_t)ROUTER_WAVES * 16 * (nb * 16 + 1) * 4 + (size_t)router_rows_per_wg(B) * H * 2 + 640;   // (and the pair ids)
+  const size_t lds = (size_t)ROUTER_WAVES * 16 * (nb * 16 + 1) * 4 + (size_t)norm_router_rows_per_wg(B) * H * 2 + 640;   // (and the pair ids)
   // With more than four rows per workgroup (batches of more than ~1000 rows) the rows a workgroup
   // normalises one after the other cost more than the launch the fusion saves (8192 rows: 2.58 ms
   // per 24 layers against 2.23 ms for the two kernels; 1024 rows: 0.63 against 0.71 ms).
   // (Experts that are shared out have their norm in a kernel of its own: every workgroup would repeat it.)
-  return B > 0 && !router_splits(B, H, E) && router_rows_per_wg(B) <= 4 && H % 32 == 0 && H <= 4096 && lds <= 160 * 1024 && aligned(x, 16) && aligned(weight, 16) &&
+  return B > 0 && !router_splits(B, H, E) && norm_router_rows_per_wg(B) <= 4 && H % 32 == 0 && H <= 4096 && lds <= 160 * 1024 && aligned(x, 16) && aligned(weight, 16) &&
          aligned(t_out, 16) && (!residual || aligned(residual, 16));
 }
 
@@ -844,7 +885,7 @@ int run_norm_router(float *x, const float *residual, const float *weight, void *
   // 4 experts, 6 / 33 / 500 rows 7.4 / 7.6 / 8.7 us, with two 5.8 / 5.9 / 7.2; 32 experts 11.6 / 11.9 / 12.9 and 10.1 /
   // 10.2 / 11.4.
   const bool grouped = group && group->expert_offsets;
-  const int rows_per_wg = !grouped && cdiv(B, 2) <= 256 ? 2 : router_rows_per_wg(B);
+  const int rows_per_wg = !grouped && cdiv(B, 2) <= 256 ? 2 : norm_router_rows_per_wg(B);
   const RouterNorm nrm{x, residual, weight, (bf16_t *)t_out};
   const bf16_t *wp = (const bf16_t *)w_router;
   const size_t dyn = (size_t)rows_per_wg * H * 2;

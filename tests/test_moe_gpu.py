@@ -96,6 +96,21 @@ def test_router_gemm(ops, B, H, E):
 
 
 # ---------------------------------------------------------------- weight packing
+@pytest.mark.parametrize("E", [32, 64, 128, 256])           # two halves of a wave's k-steps, more than 128 experts one
+@pytest.mark.parametrize("H", [32, 320, 1792, 2048, 2080, 3104])   # one k-step in all; around a wave's 7 or 8, and 12
+def test_router_rows_are_the_same_in_groups_of_any_size(ops, E, H):
+    """Workgroups of 4, 8 and 16 token rows: up to 1024 tokens, 2048, more."""
+    g = torch.Generator(device="cuda").manual_seed(E + H)
+    n = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    t, w, b = n(4099, H), n(E, H), n(E).float()
+    want = t.double() @ w.double().T + b.double()
+    for tokens in (1024, 1025, 2048, 2049, 4096, 4099):
+        got = ops.router_gemm(t[:tokens], w, b)
+        # exact products, fp32 sums of H of them: 2^-24 for each of at most H / 8 + 8 roundings, sizes of about sqrt(H)
+        assert bool(((got.double() - want[:tokens]).abs() <= 2.0 ** -24 * (H / 8 + 8) * 8 * H ** 0.5).all()), tokens
+        assert torch.equal(got[-3:], ops.router_gemm(t[tokens - 3:tokens], w, b)), tokens
+
+
 def test_pack_weight_layout(ops):
     n_mat, N, K = 2, 128, 128
     w = torch.arange(n_mat * N * K, dtype=torch.float32).reshape(n_mat, N, K) % 251
