@@ -30,6 +30,34 @@ struct GluForm {
 constexpr int MOE_TILE_BLOCK = 8;
 constexpr int XCD_BOUNDS_INTS = 16;  // ints reserved for the cut positions in front of the block table
 
+// The grouping of a batch's pairs by expert, for the router kernel to do as well where one workgroup holds every token:
+// saves a launch that takes 5 us for any small batch.  nbits: bits of an expert id.
+struct RouterGroup {
+  int *expert_offsets = nullptr, *sorted_pair_ids, *inv_perm, *tiles;
+  int *xcd_bounds, nbits;
+};
+
+// A router's products as router_parts_kernel leaves them: parts[w][row][expert], a wave of router_gemm_kernel each.
+constexpr int ROUTER_WAVES = 8;
+struct RouterParts {
+  const float *parts;
+  const float *bias;   // [E] or nullptr
+  int B, E, k;
+};
+inline size_t router_parts_floats(int B, int E) { return (size_t)ROUTER_WAVES * B * E; }
+
+// Experts' first product of a few tokens that gates and groups them as well (few_routed_kernel): what is left of the routing.
+constexpr int ROUTED_TOKENS = 4, ROUTED_EXPERTS = 128;
+struct RoutedFew {
+  RouterParts router;
+  float *logits, *topk_w;
+  int *topk_i;
+  RouterGroup group;
+  float *x;                // with a norm in front: x += residual, which nothing in front of this kernel has stored
+  const float *residual;   // or nullptr
+  int x_count;             // (a multiple of 4)
+};
+
 struct GemmParams {
   const bf16_t *A;     // activations, row-major [*, K]
   const int *row_ids;  // gather: sorted pair ids (row of A = id / top_k); else unused
@@ -53,6 +81,7 @@ struct GemmParams {
   int N, K;
   int n_col_tiles;     // gemm_col_tiles(N)
   GluForm glu;         // EPI_SWIGLU
+  const RoutedFew *routed;   // (host) gather + EPI_SWIGLU, up to ROUTED_TOKENS tokens: the tile list does not exist yet
   GemmBf16Range range[2];  // EPI_MIXED
   int k_splits;        // EPI_PARTIAL (dense only): the sum over K is cut into k_splits parts of split_slabs
   int split_slabs;     // 64-k slabs; part s is written to out + s * dense_rows * N (no bias)
@@ -110,7 +139,7 @@ struct MoePreNorm {
 // The MoE block with the RMSNorm of the updated residual stream fused into its last kernel
 // (moe_layer.cpp); out is accumulated into.  With `pre`, t is an output of the call as well: the norm
 // that produces it runs inside the router kernel (or in a kernel of its own where that kernel's
-// limits do not allow it).
+// limits do not allow it, or where the router's products are spread over workgroups).
 int moe_forward_norm(const gptoss_moe_weights *w, const void *t, int B, float *out, void *workspace,
                      size_t workspace_bytes, hipStream_t s, int mxfp4, const float *norm_w, bf16_t *norm_out,
                      const MoePreNorm *pre = nullptr);
@@ -120,12 +149,6 @@ constexpr int MOE_MAX_TOP = 32;
 // norm_out = norm(out), in the same kernel as the combine.
 int moe_forward_glu(const gptoss_moe_weights *w, const GluForm &glu, const void *t, int B, float *out, void *workspace,
                     size_t workspace_bytes, hipStream_t s, const TanhNorm &norm, bf16_t *norm_out);
-// The grouping of a batch's pairs by expert, for the router kernel to do as well where one workgroup holds every token:
-// saves a launch that takes 5 us for any small batch.  nbits: bits of an expert id.
-struct RouterGroup {
-  int *expert_offsets = nullptr, *sorted_pair_ids, *inv_perm, *tiles;
-  int *xcd_bounds, nbits;
-};
 constexpr int ROUTER_GROUP_TOKENS = 16;   // the rows of one MFMA
 // (behind a norm in the same kernel, whose rows go two at a time: ROUTER_GROUP_NORM_TOKENS)
 constexpr int ROUTER_GROUP_NORM_TOKENS = 4;
@@ -154,7 +177,13 @@ int gemm_col_tiles(int N);  // column tiles of one workgroup's width
 inline int gemm_argmax_tiles(int N) { return 2 * gemm_col_tiles(N); }  // pairs per row to allocate for EPI_ARGMAX
 // moe_route.hip
 int run_router(const void *t, const void *w_router, const float *b_router, float *logits, int B,
-               int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group = nullptr);
+               int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group = nullptr,
+               float *parts = nullptr);   // parts: room for router_parts_floats(B, E), if there is any
+int run_router_parts(const void *t, const void *w_router, float *parts, int B, int H, int E, hipStream_t s);
+// the same behind a norm of at most ROUTED_TOKENS rows: t_out = RMSNorm(x + residual) * weight; x itself is left as it is
+bool norm_router_parts_apply(int B, int H, const float *x, const float *residual, const float *weight, const void *t_out);
+int run_norm_router_parts(const float *x, const float *residual, const float *weight, void *t_out, const void *w_router,
+                          float *parts, int B, int H, int E, hipStream_t s);
 int run_topk_softmax(const float *logits, int B, int E, int k, float *topk_w, int *topk_i, hipStream_t s);
 // xcd_bounds (optional, XCD_BOUNDS_INTS + max_tiles ints): see GemmParams; tile_cost0_x2 = twice the fixed part of a tile's
 // cost in units of one 32-row block of arithmetic (cost = fixed + number of 32-row blocks);

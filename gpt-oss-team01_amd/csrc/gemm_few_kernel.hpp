@@ -28,6 +28,7 @@
 // twelve 87.8 -> 93.5.)
 #pragma once
 #include "gemm_kernel.hpp"
+#include "moe_gating.hpp"
 
 namespace gptoss {
 
@@ -115,7 +116,7 @@ __device__ __forceinline__ void narrow_epilogue(const GemmParams &p, int row0, i
 
 template <int WAVES, int ROWS, int COLS, bool GATHER, int EPI, bool FP4, bool ONCE>
 __device__ __forceinline__ void few_block(const GemmParams &p, bf16_t *lds, int mat, int row0, int rows, int cb, int slab0,
-                                          int nslab, void *out) {
+                                          int nslab, void *out, const int *row_ids = nullptr) {
   constexpr int RING = few_ring(ROWS, COLS);
   constexpr bool NARROW = few_narrow(WAVES, ROWS, COLS, FP4);
   constexpr int RB = NARROW ? (ROWS + 15) / 16 : (ROWS + 31) / 32, RBLK = NARROW ? 16 : 32, CHUNK = few_chunk(ROWS, FP4), ROW = few_row(ROWS, FP4);
@@ -152,7 +153,7 @@ __device__ __forceinline__ void few_block(const GemmParams &p, bf16_t *lds, int 
   };
   // which rows of A the tile's rows are: before W, because loads return in order
   int id = row0 + min(lane, rows - 1);
-  if (GATHER) id = p.row_ids[id];
+  if (GATHER) id = row_ids ? row_ids[id] : p.row_ids[id];
   static_for<0, RING>([&](auto r) { load_w(decltype(r)::value, r); });
   const few_rsrc_t bb = few_buffer(p.bias && live ? p.bias + (size_t)mat * N + cb * COLS : nullptr, p.bias && live ? COLS * 4 : 0);
   int bias = 0;
@@ -349,6 +350,114 @@ __global__ __launch_bounds__(WAVES * 64, few_occupancy(WAVES, ROWS, FP4)) void f
   else few_block<WAVES, ROWS, COLS, GATHER, EPI, FP4, false>(p, lds, mat, row0, rows, cb, slab0, nslab, out);
 }
 
+// The first product of up to ROUTED_TOKENS tokens, whose workgroups gate and group them from the router's partial products, each
+// for itself: a chain of 2 us in front of a product of 19 (one token, 4 of 32 experts, 2880 x 5760, between events 22.9 -> 24.8 us,
+// MXFP4 12.4 -> 15.0), in place of a launch, whose workgroup everybody waited for, with that chain and 3 us more.  The grid's
+// first row of workgroups has no tile: one leaves the routing's results, and what the kernels behind this one read, the others
+// add a norm's residual to x.
+template <int NJ, bool FP4>   // experts per lane
+__global__ __launch_bounds__(64, few_occupancy(1, 8, FP4)) void few_routed_kernel(GemmParams p, RoutedFew r) {
+  __shared__ __attribute__((aligned(16))) bf16_t lds[2 * 8 * few_row(8, FP4)];
+  __shared__ float weight[ROUTED_TOKENS * 8];
+  __shared__ int expert[ROUTED_TOKENS * 8], sorted[ROUTED_TOKENS * 8];
+  const int lane = threadIdx.x, sub = lane & 31, E = r.router.E, k = r.router.k, B = r.router.B, P = B * k;
+  const bool publish = blockIdx.y == 0;
+  if (publish && blockIdx.x != 0) {
+    if (r.residual)
+      for (int i = ((blockIdx.x - 1) * 64 + lane) * 4; i < r.x_count; i += (gridDim.x - 1) * 64 * 4) {
+        f32x4 v = *reinterpret_cast<const f32x4 *>(r.x + i);
+        const f32x4 d = *reinterpret_cast<const f32x4 *>(r.residual + i);
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[q] = __fadd_rn(v[q], d[q]);
+        *reinterpret_cast<f32x4 *>(r.x + i) = v;
+      }
+    return;
+  }
+  // two tokens at a time
+  constexpr int PASSES = ROUTED_TOKENS / 2;
+  PartialLogit x[PASSES][NJ];
+#pragma unroll
+  for (int i = 0; i < PASSES; i++)
+    if (2 * i < B)
+#pragma unroll
+      for (int j = 0; j < NJ; j++) x[i][j].load(r.router, 2 * i + (lane >> 5), sub + 32 * j);
+#pragma unroll
+  for (int i = 0; i < PASSES; i++)
+    if (2 * i < B) {
+      const int row = 2 * i + (lane >> 5);
+      float v[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; j++) {
+        const int e = sub + 32 * j;
+        v[j] = e < E ? x[i][j].sum(r.router) : -INFINITY;
+        if (publish && row < B && e < E) r.logits[(size_t)row * E + e] = v[j];
+      }
+      const int o = row < B ? row * k : 0;
+      topk_softmax_group<NJ>(v, sub, E, k, row < B, weight + o, expert + o);
+    }
+  __syncthreads();
+  // a pair per lane: pairs of lower experts, earlier ones and all of its own
+  const int e = lane < P ? expert[lane] : 0x7fffffff;
+  int lower = 0, before = 0, same = 0;
+  for (int q = 0; q < P; q++) {
+    const int other = __builtin_amdgcn_readlane(e, q);
+    lower += other < e ? 1 : 0;
+    same += other == e ? 1 : 0;
+    before += other == e && q < lane ? 1 : 0;
+  }
+  const uint64_t firsts = __ballot(lane < P && before == 0);
+  const int n_tiles = __popcll(firsts);
+  int mine = 0;   // the pair's tile: experts before its own
+  for (uint64_t f = firsts; f != 0; f &= f - 1) mine += __builtin_amdgcn_readlane(e, __builtin_ctzll(f)) < e ? 1 : 0;
+  if (publish) {
+    const RouterGroup &g = r.group;
+    if (lane < P) {
+      r.topk_w[lane] = weight[lane];
+      r.topk_i[lane] = e;
+      g.sorted_pair_ids[lower + before] = lane;
+      g.inv_perm[lane] = lower + before;
+      if (before == 0) {
+        int *tp = g.tiles + 1 + 3 * mine;
+        tp[0] = e;
+        tp[1] = lower;
+        tp[2] = same;
+        g.xcd_bounds[XCD_BOUNDS_INTS + mine] = (mine << 8) | 1;
+      }
+    }
+    if (lane < 9) g.xcd_bounds[lane] = (lane * n_tiles) << 13;   // eight parts of equal length, as group_by_one_wave
+    if (lane == 0) g.tiles[0] = n_tiles;
+    for (int x = lane; x <= E; x += 64) {
+      int n = 0;
+      for (int q = 0; q < P; q++) n += expert[q] < x ? 1 : 0;
+      g.expert_offsets[x] = n;
+    }
+    return;
+  }
+  const int tile = blockIdx.y - 1;
+  if (tile >= n_tiles) return;
+  const uint64_t of_tile = __ballot(lane < P && mine == tile);
+  const int one = __builtin_ctzll(of_tile);
+  const int mat = __builtin_amdgcn_readlane(e, one), row0 = __builtin_amdgcn_readlane(lower, one), rows = __popcll(of_tile);
+  if (lane < P) sorted[lower + before] = lane;
+  __syncthreads();
+  few_block<1, 8, 32, true, EPI_SWIGLU, FP4, true>(p, lds, mat, row0, rows, blockIdx.x, 0, p.K / BK, p.out, sorted);
+}
+
+template <bool FP4>
+int launch_few_routed(const GemmParams &p, int max_tiles, hipStream_t s) {
+  const RoutedFew &r = *p.routed;
+  GPTOSS_REQUIRE(r.router.B >= 1 && r.router.B <= ROUTED_TOKENS && r.router.k <= 8 && r.router.E <= ROUTED_EXPERTS && p.N % 32 == 0 && p.N >= 64, GPTOSS_ERR_DIM,
+                 "run_gemm: %d tokens over %d experts are not routed here", r.router.B, r.router.E);
+  {
+    TraceScope ts(FP4 ? "gemm1_gather_swiglu_mxfp4" : "gemm1_gather_swiglu", s);
+    const dim3 grid(p.N / 32, max_tiles + 1);
+    if (r.router.E <= 32) few_routed_kernel<1, FP4><<<grid, 64, 0, s>>>(p, r);
+    else few_routed_kernel<4, FP4><<<grid, 64, 0, s>>>(p, r);
+  }
+  GPTOSS_LAUNCH_CHECK("few_routed_kernel");
+  return GPTOSS_OK;
+}
+
 template <int WAVES, int ROWS, int COLS, bool GATHER, int EPI, bool FP4>
 int launch_few_waves(const GemmParams &p, int max_tiles, hipStream_t s) {
   constexpr int BM = ROWS <= 32 ? 32 : 64;
@@ -371,6 +480,8 @@ int launch_few_waves(const GemmParams &p, int max_tiles, hipStream_t s) {
 
 template <bool GATHER, int EPI, bool FP4>
 int launch_few_gemm(const GemmParams &p, int rows_per_tile, int max_tiles, hipStream_t s) {
+  if constexpr (GATHER && EPI == EPI_SWIGLU)
+    if (p.routed) return launch_few_routed<FP4>(p, max_tiles, s);
   // few blocks: workgroups of four would leave most CUs without one (2880 x 5120, 32 rows: 20 us on 40 CUs, 11 on 160)
   const long long blocks = (long long)max_tiles * (p.N / 32) * (EPI == EPI_PARTIAL ? p.k_splits : 1);
   const bool solo = blocks <= FEW_SOLO_BLOCKS;

@@ -180,7 +180,34 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
   grp.xcd_bounds = ws.xcd_bounds;
   grp.nbits = 0;
   while ((1 << grp.nbits) < E) grp.nbits++;
-  if (pre && norm_router_applies(B, H, E, pre->x, pre->residual, pre->weight, t)) {
+  // A few tokens: the router's products are spread over CUs (router_parts_kernel), if the second product's output, which comes
+  // later, has room for them.
+  float *parts = router_parts_floats(B, E) <= (size_t)B * k * H ? ws.y2 : nullptr;
+  // Up to four are gated and grouped by the workgroups of the first product (few_routed_kernel); the norm in front runs in the
+  // router's kernel.  The block by one launch less, us: 2880 x 2880, one token on 4 of 32 experts 45.9 -> 40.6, two 68.4 -> 63.8,
+  // four 120.5 -> 116.2, in MXFP4 31.6 -> 26.8, 38.2 -> 33.6, 49.6 -> 46.6, one on 128 experts 31.6 -> 27.9, with the norm one on 32
+  // experts 48.5 -> 43.0, on 128 (1024 wide) 30.5 -> 25.5.  Each workgroup repeats the gating, so three and four tokens go this way
+  // only where that is little, up to 32 experts, and where the router's own kernel has a large matrix to read: 128 experts, four
+  // tokens 51.4 -> 54.4, four experts of 2880 inputs 42.8 -> 43.5, eight of 2048 27.9 -> 28.2; 32 of 640 20.6 -> 18.2.
+  RoutedFew routed{RouterParts{parts, w->b_router, B, E, k}, ws.logits, ws.topk_w, ws.topk_i, grp};
+  routed.group.expert_offsets = ws.expert_offsets;
+  if (pre) {
+    routed.x = pre->x;
+    routed.residual = pre->residual;
+    routed.x_count = B * H;
+  }
+  const bool few = (B <= 2 || (B <= ROUTED_TOKENS && E <= 32 && H * E >= 20480)) && k <= 8 && E <= ROUTED_EXPERTS && rpt == 32 && parts &&
+                   (long long)max_tiles * 32 * H * 2 < (1ll << 31) &&
+                   (!pre || norm_router_parts_apply(B, H, pre->x, pre->residual, pre->weight, t));
+  if (few) {
+    rc = pre ? run_norm_router_parts(pre->x, pre->residual, pre->weight, const_cast<void *>(t), w->w_router, parts, B, H, E, s)
+             : run_router_parts(t, w->w_router, parts, B, H, E, s);
+    if (rc != GPTOSS_OK) return rc;
+    // (from 16 experts on, more tokens than that kernel groups have their norm in front of router_parts_kernel: 2880 x 2880, 32
+    // experts, 5 / 12 / 16 tokens 102.8 / 142.1 / 174.6 -> 99.5 / 138.7 / 171.5 us, 1024 wide 25.3 / 31.0 / 30.8 -> 21.0 / 27.1 / 27.2; with
+    // eight experts 18.5 / 19.3 / 19.2 -> 16.9 / 18.9 / 18.9 and four 46.8 / 51.4 / 58.5 -> 47.7 / 52.2 / 59.2)
+  } else if (pre && !(parts && E >= 16 && B > ROUTER_GROUP_NORM_TOKENS && router_groups(B, k)) &&
+             norm_router_applies(B, H, E, pre->x, pre->residual, pre->weight, t)) {
     if (router_groups(B, k) && B <= ROUTER_GROUP_NORM_TOKENS) grp.expert_offsets = ws.expert_offsets;
     rc = run_norm_router(pre->x, pre->residual, pre->weight, const_cast<void *>(t), w->w_router, w->b_router,
                          ws.logits, B, H, E, k, ws.topk_w, ws.topk_i, s, &grp);
@@ -190,9 +217,9 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
       if (rc != GPTOSS_OK) return rc;
     }
     if (router_groups(B, k)) grp.expert_offsets = ws.expert_offsets;
-    rc = run_router(t, w->w_router, w->b_router, ws.logits, B, H, E, k, ws.topk_w, ws.topk_i, s, &grp);
+    rc = run_router(t, w->w_router, w->b_router, ws.logits, B, H, E, k, ws.topk_w, ws.topk_i, s, &grp, parts);
   }
-  if (rc == GPTOSS_OK && !grp.expert_offsets)
+  if (rc == GPTOSS_OK && !few && !grp.expert_offsets)
     rc = run_group(B, E, k, ws.topk_w, ws.topk_i, ws.expert_offsets, ws.sorted_pair_ids, ws.inv_perm,
                    ws.tiles, rpt, ws.xcd_bounds, cost0, s, ws.sort_scratch);
   if (rc != GPTOSS_OK) return rc;
@@ -210,6 +237,7 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
   g1.tile_block = tile_block;
   g1.xcd_bounds = bounds;
   g1.max_tile_rows = B;   // a token takes an expert once
+  g1.routed = few ? &routed : nullptr;
   g1.N = 2 * I;
   g1.K = H;
   g1.n_col_tiles = gemm_col_tiles(2 * I);

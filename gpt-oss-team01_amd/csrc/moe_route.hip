@@ -6,86 +6,9 @@
 
 #include "common.hpp"
 #include "gemm.hpp"
+#include "moe_gating.hpp"
 
 namespace gptoss {
-
-// ------------------------------------------------------------------------------------------------
-// Top-k + softmax for one token held by a group of 32 lanes: lane j holds experts j, j+32, ...
-// Selection = k rounds ordered by (value desc, expert id asc); softmax over the k picked values with exp in float and the
-// sum and division in double (run.cpp:319-337).  Every lane of the group must call; lane s writes pick s.
-// A logit that is no number ranks as -infinity: whatever a token's row holds, its picks are k different experts, so that
-// its pairs cannot displace those of other tokens.  The weights of a token that picks one are no numbers.
-// A small launch waits for this from end to end, so every round is short: values as integers of the same order, their
-// largest by five exchanges, its holder by a ballot, and the exponentials and divisions of all picks at once, one per
-// lane.  The router kernel, one token over 32 experts 10.8 -> 9.2 us, twelve 12.8 -> 10.8 (before, value and expert went
-// through every exchange, and one lane computed all weights).
-// ------------------------------------------------------------------------------------------------
-template <int NJ, int KMAX = 8>
-__device__ __forceinline__ void topk_softmax_group(const float (&v)[NJ], int sub, int E, int k,
-                                                   bool live, float *__restrict__ w_out,
-                                                   int *__restrict__ i_out, int *i_copy = nullptr) {
-  uint32_t key[NJ], nan = 0;   // 0: not to be picked (any longer)
-#pragma unroll
-  for (int j = 0; j < NJ; j++) {
-    const bool no_number = v[j] != v[j];
-    const uint32_t u = __float_as_uint((no_number ? -INFINITY : v[j]) + 0.f);   // (zeros of either sign are equal)
-    key[j] = sub + 32 * j < E ? ((int)u < 0 ? ~u : u | 0x80000000u) : 0u;
-    nan |= (no_number ? 1u : 0u) << j;
-  }
-  float top = 0.f, mine = 0.f;   // the largest value, and pick number `sub`
-  int my_id = 0;
-  bool no_number = false;
-#pragma unroll
-  for (int s = 0; s < KMAX; s++) {
-    if (s < k) {
-      uint32_t best = key[0];
-      int slot = 0;
-#pragma unroll
-      for (int j = 1; j < NJ; j++) {
-        slot = key[j] > best ? j : slot;
-        best = max(best, key[j]);
-      }
-      uint32_t all = best;
-      butterfly<32>([&](auto m) { all = max(all, lane_xor<decltype(m)::value>(all)); });
-      // the lowest expert among those that hold it
-      int id = 0;
-      bool found = false;
-#pragma unroll
-      for (int j = 0; j < NJ; j++) {
-        const uint32_t holders = (uint32_t)(__ballot(best == all && slot == j) >> (threadIdx.x & 32));
-        if (!found && holders != 0) id = __builtin_ctz(holders) + 32 * j;
-        found = found || holders != 0;
-      }
-      const bool won = (id & 31) == sub;
-#pragma unroll
-      for (int j = 0; j < NJ; j++) {
-        const bool taken = won && (id >> 5) == j;
-        no_number = no_number || (taken && ((nan >> j) & 1u));
-        key[j] = taken ? 0u : key[j];
-      }
-      const float value = __uint_as_float((int)all < 0 ? all & 0x7fffffffu : ~all);
-      if (s == 0) top = value;
-      mine = sub == s ? value : mine;
-      my_id = sub == s ? id : my_id;
-    }
-  }
-  const bool no_numbers = (uint32_t)(__ballot(no_number) >> (threadIdx.x & 32)) != 0;
-  const float ex = sub < k ? expf(mine - top) : 0.f;
-  double sum = 0.0;
-#pragma unroll
-  for (int s = 0; s < KMAX; s++) {
-    if (s < k) {
-      const float lower = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__float_as_int(ex), s));
-      const float upper = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__float_as_int(ex), 32 + s));
-      sum += (threadIdx.x & 32) ? upper : lower;
-    }
-  }
-  if (live && sub < k) {
-    w_out[sub] = no_numbers ? NAN : (float)((double)ex / sum);
-    i_out[sub] = my_id;
-    if (i_copy) i_copy[sub] = my_id;
-  }
-}
 
 __device__ __forceinline__ uint64_t same_expert_mask(int e, bool valid, int nbits) {
   uint64_t mask = __ballot(valid);
@@ -292,7 +215,6 @@ __device__ __forceinline__ void group_by_one_wave(const int *topk_i, int P, int 
 // and reduce through LDS.  With topk_w != nullptr the workgroup also gates its 16 tokens (32
 // lanes per token) while the logits are still in LDS.
 // ------------------------------------------------------------------------------------------------
-constexpr int ROUTER_WAVES = 8;
 // k-steps whose operands a wave requests before its first MFMA: as many as ~150 registers hold,
 // so that a hidden size of 2880 with up to 32 experts is a single round of loads
 constexpr int router_steps(int nb) { return nb <= 2 ? 12 : (nb <= 4 ? 7 : (nb <= 8 ? 4 : 2)); }
@@ -306,10 +228,74 @@ struct RouterNorm {
   bf16_t *t_out;          // [B,H]
 };
 
+// x += residual, t = RMSNorm(x) * weight for `rows` rows from r0 on, t to memory and to t_rows in LDS: the arithmetic of
+// rmsnorm_rows_kernel, 256 threads per row, the same element-to-thread assignment and summation order, so t is the same to the
+// bit; as many rows at a time as the workgroup has 256 threads.  SHARED: other workgroups norm the same rows, so x stays as it is,
+// and t is stored by one of them (store_t).  requested(): called once, when the first rows are on their way.
+template <bool W_EARLY, bool SHARED, class Requested>
+__device__ __forceinline__ void norm_rows(const RouterNorm &nrm, bf16_t *t_rows, int r0, int rows, int B, int H, bool store_t,
+                                          Requested &&requested) {
+  constexpr int VPT = 4;  // rows of up to 4096 floats
+  __shared__ double nred[2][4];
+  const int grp = threadIdx.x >> 8, tg = threadIdx.x & 255, groups = blockDim.x >> 8;  // groups of 256 threads, a row each
+  f32x4 nw[VPT];
+#pragma unroll
+  for (int i = 0; i < VPT; i++)
+    if (W_EARLY) nw[i] = *reinterpret_cast<const f32x4 *>(nrm.weight + min((tg + 256 * i) * 4, H - 4));
+  for (int rr = 0; rr < rows; rr += groups) {
+    const int lr = rr + grp;
+    const bool live = lr < rows && r0 + lr < B;
+    const size_t row = (size_t)(r0 + lr) * H;
+    // no load under a condition, so that a row's are all on their way together (lanes past its end read its last elements)
+    const size_t src = (size_t)min(r0 + min(lr, rows - 1), B - 1) * H;
+    f32x4 v[VPT], res[VPT];
+#pragma unroll
+    for (int i = 0; i < VPT; i++) {
+      const int h = min((tg + 256 * i) * 4, H - 4);
+      v[i] = *reinterpret_cast<const f32x4 *>(nrm.x + src + h);
+      res[i] = *reinterpret_cast<const f32x4 *>((nrm.residual ? nrm.residual : nrm.x) + src + h);
+    }
+    if (rr == 0) requested();
+    double ss = 0.0;
+#pragma unroll
+    for (int i = 0; i < VPT; i++) {
+      const int h = (tg + 256 * i) * 4;
+      if (live && h < H) {
+        if (nrm.residual) {
+#pragma unroll
+          for (int q = 0; q < 4; q++) v[i][q] = __fadd_rn(v[i][q], res[i][q]);
+          if (!SHARED) *reinterpret_cast<f32x4 *>(nrm.x + row + h) = v[i];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[i][q], v[i][q]);
+      }
+    }
+    ss = lanes_sum(ss);
+    if ((threadIdx.x & 63) == 0) nred[grp][(threadIdx.x >> 6) & 3] = ss;
+    __syncthreads();
+    ss = nred[grp][0] + nred[grp][1] + nred[grp][2] + nred[grp][3];
+    ss /= H;
+    ss += 1e-5f;
+    const double inv = (double)(1.0f / sqrtf((float)ss));
+#pragma unroll
+    for (int i = 0; i < VPT; i++) {
+      const int h = (tg + 256 * i) * 4;
+      if (live && h < H) {
+        if (!W_EARLY) nw[i] = *reinterpret_cast<const f32x4 *>(nrm.weight + h);
+        f32x4 o;
+#pragma unroll
+        for (int q = 0; q < 4; q++) o[q] = (float)((double)nw[i][q] * (inv * (double)v[i][q]));
+        const u32x2 pk = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+        if (!SHARED || store_t) *reinterpret_cast<u32x2 *>(nrm.t_out + row + h) = pk;
+        *reinterpret_cast<u32x2 *>(t_rows + (size_t)lr * H + h) = pk;
+      }
+    }
+    __syncthreads();   // nred is reused by the next pair of rows; after the last pair: t_rows complete
+  }
+}
+
 // NB: number of 16-expert column blocks held per wave.  NORM: the workgroup first normalises its
-// rows (the arithmetic of rmsnorm_rows_kernel: 256 threads per row, the same element-to-thread
-// assignment and summation order, so t is the same to the bit), writes x and t to memory, keeps t in
-// LDS and multiplies from there: one launch and one read of t less than norm kernel + router kernel.
+// rows (norm_rows) and multiplies them from LDS: one launch and one read of t less than norm kernel + router kernel.
 // A small launch is a chain of waits for memory, so all that does not depend on each other is requested at once: the
 // router's weights and biases, a row's elements, its residual and the norm's weights.  (With a branch for each of the
 // row's parts they came one behind the other.)  One row of 2880, 4 experts 8.4 -> 7.3 us, 33 rows 10.6 -> 8.4
@@ -364,64 +350,8 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
   if (EARLY && wave < ksteps) load_b(wave, S0{});
   if (SETS == 2 && EARLY && wave + STRIDE < ksteps) load_b(wave + STRIDE, S1{});
   if constexpr (NORM) {
-    constexpr int VPT = 4;  // rows of up to 4096 floats
-    __shared__ double nred[2][4];
     bf16_t *t_rows = reinterpret_cast<bf16_t *>(t_rows_raw);
-    const int grp = threadIdx.x >> 8, tg = threadIdx.x & 255;  // two groups of 256 threads, a row each
-    constexpr bool W_EARLY = NB < 8;   // requested with the first rows, where registers allow
-    f32x4 nw[VPT];
-#pragma unroll
-    for (int i = 0; i < VPT; i++)
-      if (W_EARLY) nw[i] = *reinterpret_cast<const f32x4 *>(nrm.weight + min((tg + 256 * i) * 4, H - 4));
-    for (int rr = 0; rr < rows_per_wg; rr += 2) {
-      const int lr = rr + grp;
-      const bool live = lr < rows_per_wg && r0 + lr < B;
-      const size_t row = (size_t)(r0 + lr) * H;
-      // no load under a condition, so that a row's are all on their way together (lanes past its end read its last elements)
-      const size_t src = (size_t)min(r0 + min(lr, rows_per_wg - 1), B - 1) * H;
-      f32x4 v[VPT], res[VPT];
-#pragma unroll
-      for (int i = 0; i < VPT; i++) {
-        const int h = min((tg + 256 * i) * 4, H - 4);
-        v[i] = *reinterpret_cast<const f32x4 *>(nrm.x + src + h);
-        res[i] = *reinterpret_cast<const f32x4 *>((nrm.residual ? nrm.residual : nrm.x) + src + h);
-      }
-      double ss = 0.0;
-#pragma unroll
-      for (int i = 0; i < VPT; i++) {
-        const int h = (tg + 256 * i) * 4;
-        if (live && h < H) {
-          if (nrm.residual) {
-#pragma unroll
-            for (int q = 0; q < 4; q++) v[i][q] = __fadd_rn(v[i][q], res[i][q]);
-            *reinterpret_cast<f32x4 *>(nrm.x + row + h) = v[i];
-          }
-#pragma unroll
-          for (int q = 0; q < 4; q++) ss += (double)__fmul_rn(v[i][q], v[i][q]);
-        }
-      }
-      ss = lanes_sum(ss);
-      if (lane == 0) nred[grp][(threadIdx.x >> 6) & 3] = ss;
-      __syncthreads();
-      ss = nred[grp][0] + nred[grp][1] + nred[grp][2] + nred[grp][3];
-      ss /= H;
-      ss += 1e-5f;
-      const double inv = (double)(1.0f / sqrtf((float)ss));
-#pragma unroll
-      for (int i = 0; i < VPT; i++) {
-        const int h = (tg + 256 * i) * 4;
-        if (live && h < H) {
-          if (!W_EARLY) nw[i] = *reinterpret_cast<const f32x4 *>(nrm.weight + h);
-          f32x4 o;
-#pragma unroll
-          for (int q = 0; q < 4; q++) o[q] = (float)((double)nw[i][q] * (inv * (double)v[i][q]));
-          const u32x2 pk = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-          *reinterpret_cast<u32x2 *>(nrm.t_out + row + h) = pk;
-          *reinterpret_cast<u32x2 *>(t_rows + (size_t)lr * H + h) = pk;
-        }
-      }
-      __syncthreads();   // nred is reused by the next pair of rows; after the last pair: t_rows complete
-    }
+    norm_rows<(NB < 8), false>(nrm, t_rows, r0, rows_per_wg, B, H, true, [] {});   // (W_EARLY where registers allow)
     ap = t_rows + (size_t)(arow - r0) * H + kq;
   }
   f32x4 acc[NB];
@@ -495,6 +425,52 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
       __syncthreads();
       if (wave == 0) group_by_one_wave(ids, B * k, E, reinterpret_cast<int *>(&red[0][0][0]), grp);
     }
+  }
+}
+
+// The partial products that the waves of router_gemm_kernel add up, of at most 16 tokens: a workgroup is one of its waves over
+// 16 experts.  One workgroup for all of them waits for the experts' weights, of which a CU gets 36 KB a us; here 8 to 128 CUs
+// share them.  Whoever gates adds the parts up (PartialLogit).  NORM: every workgroup norms the few rows for itself, in the time
+// that its weights take, and t is an output; what adds the residual to x comes behind (few_routed_kernel).
+// Between events, which add 4 us: 2880 inputs, 32 experts, one token 11.8 us with the gating -> 6.2 without; of 12 tokens the
+// whole routing, in two launches instead of one, takes 4.6 us less.
+template <bool NORM>
+__global__ __launch_bounds__(NORM ? 512 : 64) void router_parts_kernel(const bf16_t *__restrict__ t, const bf16_t *__restrict__ wr,
+                                                                       float *__restrict__ parts, int B, int H, int E, RouterNorm nrm) {
+  constexpr int STEPS = 12;
+  extern __shared__ __attribute__((aligned(16))) unsigned char t_rows_raw[];   // NORM: [B][H] bf16
+  const int lane = threadIdx.x & 63, wave = blockIdx.x, e0 = blockIdx.y * 16;
+  const bool multiplies = !NORM || __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0;
+  const int kq = (lane >> 4) * 8, ksteps = H / 32, arow = min(lane & 15, B - 1);
+  const bf16_t *ap = t + (size_t)arow * H + kq, *bp = wr + (size_t)min(e0 + (lane & 15), E - 1) * H + kq;
+  u32x4 a[STEPS], b[STEPS];
+  auto load = [&](const bf16_t *from, u32x4 (&to)[STEPS], int ks0) {
+#pragma unroll
+    for (int u = 0; u < STEPS; u++) to[u] = *reinterpret_cast<const u32x4 *>(from + min(ks0 + u * ROUTER_WAVES, ksteps - 1) * 32);
+  };
+  if constexpr (NORM) {
+    bf16_t *t_rows = reinterpret_cast<bf16_t *>(t_rows_raw);
+    norm_rows<true, true>(nrm, t_rows, 0, B, B, H, wave == 0 && e0 == 0, [&] {
+      if (multiplies) load(bp, b, wave);
+    });
+    if (!multiplies) return;
+    ap = t_rows + (size_t)arow * H + kq;
+  } else {
+    load(bp, b, wave);
+  }
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int ks0 = wave; ks0 < ksteps; ks0 += ROUTER_WAVES * STEPS) {
+    if (ks0 != wave) load(bp, b, ks0);
+    load(ap, a, ks0);
+#pragma unroll
+    for (int u = 0; u < STEPS; u++)
+      if (ks0 + u * ROUTER_WAVES < ksteps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[u]), as_bf16x8(b[u]), acc, 0, 0, 0);
+  }
+  const int e = e0 + (lane & 15);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int row = (lane >> 4) * 4 + i;
+    if (row < B && e < E) parts[((size_t)wave * B + row) * E + e] = acc[i];
   }
 }
 
@@ -698,19 +674,31 @@ __global__ __launch_bounds__(SORT_THREADS) void group_scatter_kernel(
 }
 
 
-// Gating of at most ROUTER_GROUP_TOKENS tokens from their logits, and their grouping: the end of router_gemm_kernel, for
-// experts that several workgroups shared.
-template <int NJ>
-__global__ __launch_bounds__(512) void topk_group_kernel(const float *__restrict__ logits, int B, int E, int k,
+// Gating of at most ROUTER_GROUP_TOKENS tokens from their logits (PARTS: from the router's partial products, and the logits), and
+// their grouping: the end of router_gemm_kernel, for experts that several workgroups shared.
+template <int NJ, bool PARTS>
+__global__ __launch_bounds__(512) void topk_group_kernel(float *__restrict__ logits, RouterParts parts, int B, int E, int k,
                                                          float *__restrict__ topk_w, int *__restrict__ topk_i, RouterGroup grp) {
   __shared__ int ids[ROUTER_GROUP_PAIRS], lds[512];
   const int row = threadIdx.x >> 5, sub = threadIdx.x & 31;
   const bool live = row < B;
   float v[NJ];
+  if constexpr (PARTS) {
+    PartialLogit x[NJ];
 #pragma unroll
-  for (int j = 0; j < NJ; j++) {
-    const float x = logits[(size_t)min(row, B - 1) * E + min(sub + 32 * j, E - 1)];
-    v[j] = sub + 32 * j < E ? x : -INFINITY;
+    for (int j = 0; j < NJ; j++) x[j].load(parts, row, sub + 32 * j);
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+      const int e = sub + 32 * j;
+      v[j] = e < E ? x[j].sum(parts) : -INFINITY;
+      if (live && e < E) logits[(size_t)row * E + e] = v[j];
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+      const float x = logits[(size_t)min(row, B - 1) * E + min(sub + 32 * j, E - 1)];
+      v[j] = sub + 32 * j < E ? x : -INFINITY;
+    }
   }
   const size_t o = (size_t)(live ? row : 0) * k;
   topk_softmax_group<NJ>(v, sub, E, k, live, topk_w + o, topk_i + o, ids + row * k);
@@ -787,10 +775,35 @@ static int router_split_rows(int B, int E) {
   return rows;
 }
 
+int run_router_parts(const void *t, const void *w_router, float *parts, int B, int H, int E, hipStream_t s) {
+  GPTOSS_REQUIRE(B >= 1 && B <= ROUTER_GROUP_TOKENS, GPTOSS_ERR_DIM, "router: no partial products of %d tokens", B);
+  TraceScope ts(router_splits(B, H, E) ? "router_gemm" : "router_gemm_topk", s);   // (the second with the gating in another kernel than its own)
+  router_parts_kernel<false><<<dim3(ROUTER_WAVES, cdiv(E, 16)), 64, 0, s>>>((const bf16_t *)t, (const bf16_t *)w_router, parts, B, H, E, RouterNorm{});
+  GPTOSS_LAUNCH_CHECK("router_parts_kernel");
+  return GPTOSS_OK;
+}
+
+bool norm_router_parts_apply(int B, int H, const float *x, const float *residual, const float *weight, const void *t_out) {
+  return B >= 1 && B <= ROUTED_TOKENS && H % 32 == 0 && H <= 4096 && aligned(x, 16) && aligned(weight, 16) && aligned(t_out, 16) &&
+         (!residual || aligned(residual, 16));
+}
+
+int run_norm_router_parts(const float *x, const float *residual, const float *weight, void *t_out, const void *w_router,
+                          float *parts, int B, int H, int E, hipStream_t s) {
+  GPTOSS_REQUIRE(norm_router_parts_apply(B, H, x, residual, weight, t_out), GPTOSS_ERR_DIM,
+                 "norm + router: no partial products of this form (B=%d H=%d)", B, H);
+  TraceScope ts("norm_router_gemm", s);
+  const RouterNorm nrm{const_cast<float *>(x), residual, weight, (bf16_t *)t_out};
+  router_parts_kernel<true><<<dim3(ROUTER_WAVES, cdiv(E, 16)), B == 1 ? 256 : 512, (size_t)B * H * 2, s>>>(
+      nrm.t_out, (const bf16_t *)w_router, parts, B, H, E, nrm);
+  GPTOSS_LAUNCH_CHECK("router_parts_kernel (with norm)");
+  return GPTOSS_OK;
+}
+
 // logits (+ optional gating of the same tokens), in one launch unless many experts are shared out (only with the gating of at
 // most 8 experts per token: logits alone come from one workgroup for all experts)
 int run_router(const void *t, const void *w_router, const float *b_router, float *logits, int B,
-               int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group) {
+               int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group, float *parts) {
   // 16 token rows per workgroup fill the MFMA, but a thousand tokens are then only 64 workgroups;
   // with fewer rows each (the rest of the MFMA rows idle) all CUs take part in what is a
   // latency-bound launch: every workgroup reads the whole router matrix from L2 either way
@@ -806,6 +819,23 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
     const int rc = run_router(t, w_router, b_router, logits, B, H, E, k, nullptr, nullptr, s);
     return rc != GPTOSS_OK ? rc : run_topk_softmax(logits, B, E, k, topk_w, topk_i, s);
   }
+  // Few tokens: the products of a kernel of their own for any number of experts, one launch more for those that one workgroup had.
+  // The whole block, us: 32 experts, 5 / 16 tokens 53.4 / 84.2 -> 49.6 / 78.6 (MXFP4, 2880 x 2880), 21.2 / 27.1 -> 17.4 / 22.6 (640 x
+  // 256); 128 61.9 / 126.7 -> 59.4 / 123.9; 256 of 1024 inputs 24.4 / 30.7 -> 22.5 / 29.3; 16 of 4096 32.9 / 41.5 -> 28.6 / 32.4; four and eight
+  // from eight tokens on: 42.5 / 53.5 -> 43.9 / 51.7 and 27.9 / 36.0 -> 28.1 / 34.2.
+  if (grp.expert_offsets && parts && topk_w && (E >= 16 || B >= 8)) {
+    int rc = run_router_parts(t, w_router, parts, B, H, E, s);
+    if (rc != GPTOSS_OK) return rc;
+    const RouterParts rp{parts, b_router, B, E, k};
+    TraceScope ts("topk_group", s);
+    auto launch = [&](auto kern) { kern<<<1, 512, 0, s>>>(logits, rp, B, E, k, topk_w, topk_i, grp); };
+    if (nb <= 2) launch(topk_group_kernel<1, true>);
+    else if (nb <= 4) launch(topk_group_kernel<2, true>);
+    else if (nb <= 8) launch(topk_group_kernel<4, true>);
+    else launch(topk_group_kernel<8, true>);
+    GPTOSS_LAUNCH_CHECK("topk_group_kernel");
+    return GPTOSS_OK;
+  }
   if (router_splits(B, H, E) && topk_w) {
     const int rows = router_split_rows(B, E);
     {
@@ -816,9 +846,10 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
     }
     if (!grp.expert_offsets) return run_topk_softmax(logits, B, E, k, topk_w, topk_i, s);
     TraceScope ts("topk_group", s);
-    if (nb <= 4) topk_group_kernel<2><<<1, 512, 0, s>>>(logits, B, E, k, topk_w, topk_i, grp);
-    else if (nb <= 8) topk_group_kernel<4><<<1, 512, 0, s>>>(logits, B, E, k, topk_w, topk_i, grp);
-    else topk_group_kernel<8><<<1, 512, 0, s>>>(logits, B, E, k, topk_w, topk_i, grp);
+    auto launch = [&](auto kern) { kern<<<1, 512, 0, s>>>(logits, RouterParts{}, B, E, k, topk_w, topk_i, grp); };
+    if (nb <= 4) launch(topk_group_kernel<2, false>);
+    else if (nb <= 8) launch(topk_group_kernel<4, false>);
+    else launch(topk_group_kernel<8, false>);
     GPTOSS_LAUNCH_CHECK("topk_group_kernel");
     return GPTOSS_OK;
   }

@@ -453,6 +453,39 @@ def test_which_calls_share_their_experts_out(ops, H, E, tokens, shared):
     assert ("router_gemm" in launches) == shared and ("router_gemm_topk" in launches) != shared
 
 
+# up to two tokens are gated by the workgroups of the first product, up to four with 16 to 32 experts (of 1280 inputs), up to 128
+# experts; the others by one workgroup.  One expert per lane and four, lanes without one, one to 32 pairs
+@pytest.mark.parametrize("mxfp4", [False, True])
+@pytest.mark.parametrize("E,k", [(1, 1), (2, 2), (15, 8), (16, 1), (31, 5), (32, 8), (33, 4), (128, 8), (129, 8)])
+def test_a_few_tokens_are_routed_as_in_any_batch(ops, E, k, mxfp4):
+    g = torch.Generator(device="cuda").manual_seed(E * 9 + k)
+    H, I = 1280, 192
+    n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    def matrix(rows, cols):
+        if not mxfp4:
+            return [n(E, rows, cols, std=0.05)]
+        codes = torch.randint(0, 256, (E, rows, cols // 2), generator=g, device="cuda", dtype=torch.uint8)
+        return [codes, torch.randint(118, 124, (E, rows, cols // 32), generator=g, device="cuda", dtype=torch.uint8)]
+    bias = (torch.arange(E, device="cuda") % 3).float()   # a token of zeros: many equal logits
+    layer = (ops.MoeLayerMxfp4 if mxfp4 else ops.MoeLayer)(
+        n(E, H, std=H ** -0.5), bias, *matrix(2 * I, H), n(E, 2 * I).float(), *matrix(H, I), n(E, H).float(), top_k=k, max_tokens=40)
+    t = n(40, H)
+    t[2] = 0
+    t[3] = float("nan")
+    t[5] = 1e38           # products and sums that are infinite, or none
+    same = lambda a, b: torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num())
+    all_of_them = layer.forward(t).clone()
+    for tokens in (1, 2, 3, 4, 5, 7, 8, 16):
+        for first in (0, 2, 3, 4):
+            part = t[first:first + tokens].contiguous()
+            got = layer.forward(part)
+            logits = ops.router_gemm(part, layer.w_router, layer.b_router)
+            want = [logits, *ops.moe_route(logits, k)[:5]]
+            for name, a, b in zip("logits weights ids offsets order place".split(), layer.routing_views(), want):
+                assert same(a, b), (tokens, first, name)
+            assert same(got, all_of_them[first:first + tokens]), (tokens, first)
+
+
 @pytest.mark.parametrize("E,k", [(1, 1), (4, 4), (32, 4), (33, 8), (128, 4), (256, 8)])
 def test_grouping_of_a_few_tokens_by_one_wave(ops, E, k):
     """gptoss::run_group, which has no C entry point, by its linker name, against gptoss_moe_route's kernels."""
