@@ -29,13 +29,15 @@ struct StorePlace {
   }
 };
 
-// One wave per (RT rows, head): query heads, key heads, value heads.
+// One wave per (RT rows, head): query heads (left out from unit `first` on), key heads, value heads.  Bound by what it moves:
+// with the queries, 2048 columns of fp32 in and out for 1024 of keys and values, 8000 rows took 71 us; the attention
+// kernels norm the queries themselves where they can (norms_queries), and it takes 35.
 template <bool F32, int RT>
 __global__ __launch_bounds__(256) void window_store_kernel(WindowAttn a, const int *__restrict__ slots,
-                                                           const int *__restrict__ lens, int n) {
+                                                           const int *__restrict__ lens, int n, int first) {
   constexpr int PIECES = WINDOW_ATTN_MAX_DIM / 64;
   const int row0 = blockIdx.y * RT, lane = threadIdx.x & 63, live = min(RT, n - row0);
-  const int unit = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int unit = first + blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int H = a.heads, G = a.kv_heads;
   if (unit >= H + 2 * G) return;
   const int DK = F32 ? a.dim : a.dim_pad(), DV = a.vdim_pad();
@@ -70,6 +72,21 @@ __global__ __launch_bounds__(256) void window_store_kernel(WindowAttn a, const i
       const float wd = d < width ? w[d] : 0.f;
 #pragma unroll
       for (int r = 0; r < RT; r++) v[i][r] = v[i][r] * inv[r] * wd;
+    }
+  }
+  if constexpr (!F32 && RT == 4) {
+    // four positions from a multiple of four on: a value's places are neighbours
+    const int pos = lens[row0] - 1, end = row0 + live - 1;
+    if (is_v && live == 4 && pos % 4 == 0 && lens[end] - 1 == pos + 3 && slots[end] == slots[row0]) {
+      const int cslot = pos % a.cap;
+      const StorePlace at{a.kv + ((size_t)(slots[row0] * G + head) * (a.cap >> 6) + (cslot >> 6)) * a.block_elems(), cslot, DK, DV};
+#pragma unroll
+      for (int i = 0; i < PIECES; i++) {
+        const int d = lane + 64 * i;
+        if (d < DV)
+          *reinterpret_cast<u32x2 *>(at.value(d)) = u32x2{pack_bf16x2(v[i][0], v[i][1]), pack_bf16x2(v[i][2], v[i][3])};
+      }
+      return;
     }
   }
 #pragma unroll
@@ -295,6 +312,33 @@ __device__ __forceinline__ void load_q(QFrag<KS> &f, const float *q, int ks_n, i
   }
 }
 
+// The same from the projection, normed here, where a head is all of the operands: the operations of window_store_kernel, the sum
+// of squares by the four lanes of a column.
+template <int KS>
+__device__ __forceinline__ void load_q_normed(QFrag<KS> &f, const float *q, const float *w, int c, float eps, float scale) {
+  f32x4 x[2 * KS], wx[2 * KS];
+#pragma unroll
+  for (int i = 0; i < 2 * KS; i++) {
+    x[i] = *reinterpret_cast<const f32x4 *>(q + c * KS * 8 + i * 4);
+    wx[i] = *reinterpret_cast<const f32x4 *>(w + c * KS * 8 + i * 4);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2 * KS; i++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) ss = fmaf(x[i][e], x[i][e], ss);
+  ss += lane_xor<16>(ss);
+  ss += lane_xor<32>(ss);
+  const float inv = 1.f / sqrtf(ss / (KS * 32) + eps);
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) {
+    float y[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = x[2 * ks + (e >> 2)][e & 3] * inv * wx[2 * ks + (e >> 2)][e & 3] * scale;
+    split8(y, f.hi[ks], f.lo[ks]);
+  }
+}
+
 // One 64-slot block for 16 query columns, in two halves so that a caller can request the next block's K
 // between them.  kf(tb, ks) and vf(kg, db) return operands; key slot i of the block is position
 // pos0 + i; the column sees positions lo..hi.
@@ -399,7 +443,8 @@ __device__ __forceinline__ void store_column(bf16_t *dst, int vdim, int db_n, in
 // ---- decoding rows -------------------------------------------------------------------------------
 // EXACT: both head sizes are DMAX, so every operand has its place in registers: a wave's K and V of the next
 // block are requested as soon as those of the current one have been used.
-template <int DMAX, bool EXACT>
+// NORM: the queries come from the projection and are normed here.
+template <int DMAX, bool EXACT, bool NORM = false>
 __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttn a, const RowSeg *__restrict__ singles) {
   constexpr int KS = DMAX / 32, DB = DMAX / 16;
   __shared__ float so[3][DMAX][16], sm[3][16], sl[3][16];
@@ -444,7 +489,8 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttn a, const 
       load_v(rb);
     }
     QFrag<KS> q;
-    load_q<KS>(q, a.q + ((size_t)seg.row0 * a.heads + head) * DK, ks_n, c, a.scale * 1.4426950408889634f);
+    if constexpr (NORM) load_q_normed<KS>(q, a.in + (size_t)seg.row0 * a.ld_in + a.q_col + head * DMAX, a.q_norm, c, a.eps, a.scale * 1.4426950408889634f);
+    else load_q<KS>(q, a.q + ((size_t)seg.row0 * a.heads + head) * DK, ks_n, c, a.scale * 1.4426950408889634f);
     while (b <= b_last) {
       const int next = b + 4 <= b_last ? (rb + 4) % ring : rb;   // past the end: this block again, unused
       f32x4 s[4];
@@ -571,6 +617,130 @@ __global__ __launch_bounds__(256, DMAX > 128 ? 1 : 2) void window_tile_kernel(Wi
   }
 }
 
+// Heads of 64 (padded): eight waves of 16 queries each, blocks straight into LDS, two buffers and one barrier per block.  The
+// vector units bound it, so a block that every row of a wave sees whole has no masks, sums are rescaled only for a score more
+// than WRAISE powers of two above the reference (then to a whole number: an exact factor), and four waves per SIMD, not two,
+// cover for each other.  Consecutive pieces, which read the same blocks, go to one XCD.  8 prompts of 1000 rows, 32 query over 8 kv
+// heads, window 512: 139 -> 93 us.
+constexpr int WTILE_WAVES = 8;
+constexpr float WRAISE = 4.f;
+// K rows in LDS: position j of row r holds chunk j ^ window_swizzle(r) of 16 bytes, so that the lanes that LDS serves together
+// (0-3, 12-15 and 20-27 of a fragment's read, then the others) hit different banks
+__device__ __forceinline__ int window_swizzle(int r) { return ((r >> 1) & 7) ^ (r & 4); }
+
+template <bool NORM>
+__global__ __launch_bounds__(WTILE_WAVES * 64, 4) void window_tile64_kernel(WindowAttn a, const RowSeg *__restrict__ tiles, int n_tiles) {
+  constexpr int D = 64, KS = D / 32, DB = D / 16, K_BYTES = KV_BLOCK * D * 2, BLOCK_BYTES = 2 * K_BYTES;
+  static_assert(K_BYTES == WTILE_WAVES * 64 * 16, "a thread copies a piece of K and one of V");
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2][BLOCK_BYTES];
+  const int total = n_tiles * a.kv_heads, chunk = (total + 7) >> 3, item = (blockIdx.x & 7) * chunk + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= chunk || item >= total) return;
+  const int g = item / n_tiles, per = a.heads / a.kv_heads;
+  const RowSeg *seg = tiles + (item - g * n_tiles);
+  const int row0 = __builtin_amdgcn_readfirstlane(seg->row0), rows = __builtin_amdgcn_readfirstlane(seg->n);
+  const int slot = __builtin_amdgcn_readfirstlane(seg->slot), pos0 = __builtin_amdgcn_readfirstlane(seg->pos0);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, c = lane >> 4;
+  const int ring = a.cap >> 6, queries = rows * per;
+  const unsigned char *plane = reinterpret_cast<const unsigned char *>(a.kv) + (size_t)(slot * a.kv_heads + g) * ring * BLOCK_BYTES;
+  const uint32_t k_off = ((tid & ~7) | ((tid & 7) ^ window_swizzle(tid >> 3))) * 16, v_off = K_BYTES + tid * 16;
+  const unsigned lds_base =
+      __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)&lds[0][0]) + wave * 1024;
+  auto request = [&](int rb, int buf) {
+    const unsigned char *src = plane + (size_t)rb * BLOCK_BYTES;
+    load_to_lds(lds_base + buf * BLOCK_BYTES, k_off, src);
+    load_to_lds(lds_base + buf * BLOCK_BYTES + K_BYTES, v_off, src);
+  };
+  for (int q0 = 0; q0 < queries; q0 += WTILE_WAVES * 16) {
+    const int b_lo = a.first(pos0 + q0 / per) >> 6, b_hi = (pos0 + min(q0 + WTILE_WAVES * 16 - 1, queries - 1) / per) >> 6;
+    int rb = b_lo % ring;
+    if (q0) __builtin_amdgcn_s_barrier();   // every wave is done with the blocks of the queries before
+    request(rb, 0);
+    // the wave's queries and what their rows see: some of them [any_lo, any_hi], all of them [whole_lo, whole_hi]
+    const int q_first = q0 + wave * 16, qi = q_first + n;
+    const int any_hi = pos0 + min(q_first + 15, queries - 1) / per, whole_hi = pos0 + min(q_first, queries - 1) / per;
+    const int any_lo = a.first(whole_hi), whole_lo = a.first(any_hi);
+    const int use = min(qi, queries - 1), row = use / per, head = g * per + (use - row * per);
+    const int lo = a.first(pos0 + row);
+    const uint32_t seen = pos0 + row - lo + 1;
+    QFrag<KS> q;
+    const float scale = a.scale * 1.4426950408889634f;
+    if constexpr (NORM) load_q_normed<KS>(q, a.in + (size_t)(row0 + row) * a.ld_in + a.q_col + head * D, a.q_norm, c, a.eps, scale);
+    else load_q<KS>(q, a.q + ((size_t)(row0 + row) * a.heads + head) * D, KS, c, scale);
+    float m = WNEG, l = 0.f;
+    f32x4 o[DB];
+#pragma unroll
+    for (int db = 0; db < DB; db++) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int buf = 0;
+    for (int b = b_lo; b <= b_hi; b++, buf ^= 1) {
+      // The block is complete once every wave's loads of it have landed, and behind the barrier every wave is done with the
+      // other buffer.  (The compiler does not count these loads; the loop has no others.)
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if (b < b_hi) {
+        rb = rb + 1 == ring ? 0 : rb + 1;
+        request(rb, buf ^ 1);
+      }
+      const int first = b << 6;
+      const bool busy = q_first < queries && first <= any_hi && first + 63 >= any_lo;
+      if (!__builtin_amdgcn_readfirstlane(busy)) continue;
+      const int edge = __builtin_amdgcn_readfirstlane(first < whole_lo || first + 63 > whole_hi);
+      const unsigned char *kb = lds[buf], *vb = lds[buf] + K_BYTES;
+      f32x4 s[4];
+      block_scores<KS>(q, KS, s, [&](int tb, int ks) {
+        const int r = tb * 16 + n;
+        return as_bf16x8(*reinterpret_cast<const u32x4 *>(kb + r * (D * 2) + (((c * KS + ks) ^ window_swizzle(r)) << 4)));
+      });
+      if (edge) {
+        const int s0 = first + c * 4 - lo;
+#pragma unroll
+        for (int tb = 0; tb < 4; tb++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) s[tb][e] = (uint32_t)(s0 + tb * 16 + e) < seen ? s[tb][e] : -INFINITY;
+      }
+      float top = -INFINITY;
+#pragma unroll
+      for (int tb = 0; tb < 4; tb++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) top = fmaxf(top, s[tb][e]);
+      if (__ballot(top > m + WRAISE) != 0) {
+        top = max_over_quarters(top);
+        const float m_new = top > m + WRAISE ? ceilf(top) : m, fade = __builtin_amdgcn_exp2f(m - m_new);
+        m = m_new;
+        l *= fade;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) o[db][e] *= fade;
+      }
+      float sum = 0.f;
+#pragma unroll
+      for (int kg = 0; kg < 2; kg++) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          x[e] = __builtin_amdgcn_exp2f(s[2 * kg + (e >> 2)][e & 3] - m);
+          sum += x[e];
+        }
+        bf16x8 hi8, lo8;
+        split8(x, hi8, lo8);
+#pragma unroll
+        for (int db = 0; db < DB; db++) {
+          const bf16x8 v = as_bf16x8(*reinterpret_cast<const u32x4 *>(vb + (kg * DB + db) * 1024 + lane * 16));
+          o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, lo8, o[db], 0, 0, 0);
+          o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, hi8, o[db], 0, 0, 0);
+        }
+      }
+      l += sum;
+    }
+    const float total_l = column_sum(l);
+    if (qi < queries)
+      store_column<DB>((bf16_t *)a.out + (size_t)(row0 + row) * a.ld_out + a.out_col + head * a.vdim, a.vdim, DB, c,
+                       a.out_scale / total_l, o);
+  }
+}
+
 // ---- fp32 ----------------------------------------------------------------------------------------
 // One workgroup per (row, head): online softmax over tiles of 256 positions.
 __global__ __launch_bounds__(256) void window_f32_kernel(WindowAttn a, const int *__restrict__ slots,
@@ -645,6 +815,12 @@ static void launch_store_rows(const WindowAttn &a, const StepRows &r, hipStream_
   }
 }
 
+// Whether the attention kernels take the queries from the projection and norm them: heads of 64 whole, a norm per head.
+static bool norms_queries(const WindowAttn &a) {
+  return !a.k32 && !a.whole_norm && a.dim == 64 && a.vdim_pad() == 64 && a.ld_in % 4 == 0 && a.q_col % 4 == 0 && aligned(a.in, 16) &&
+         aligned(a.q_norm, 16);
+}
+
 int run_window_attn(const WindowAttn &a, const StepRows &r, hipStream_t s) {
   GPTOSS_REQUIRE(a.dim >= 1 && a.dim <= WINDOW_ATTN_MAX_DIM && a.vdim >= 1 && a.vdim <= WINDOW_ATTN_MAX_DIM &&
                      a.kv_heads >= 1 && a.heads % a.kv_heads == 0 && a.window >= 1 && a.cap % 64 == 0,
@@ -660,7 +836,7 @@ int run_window_attn(const WindowAttn &a, const StepRows &r, hipStream_t s) {
     {
       TraceScope ts("window_store", s);
       if (a.whole_norm) launch_store_rows<true>(a, r, s);
-      else window_store_kernel<true, 1><<<dim3(cdiv(units, 4), r.n), 256, 0, s>>>(a, r.slots, r.lens, r.n);
+      else window_store_kernel<true, 1><<<dim3(cdiv(units, 4), r.n), 256, 0, s>>>(a, r.slots, r.lens, r.n, 0);
     }
     GPTOSS_LAUNCH_CHECK("window_store_kernel");
     TraceScope ts("window_attn_f32", s);
@@ -668,11 +844,13 @@ int run_window_attn(const WindowAttn &a, const StepRows &r, hipStream_t s) {
     GPTOSS_LAUNCH_CHECK("window_f32_kernel");
     return GPTOSS_OK;
   }
+  const bool norms_q = norms_queries(a);
   {
     TraceScope ts("window_store", s);
+    const int first = norms_q ? a.heads : 0, blocks = cdiv(units - first, 4);
     if (a.whole_norm) launch_store_rows<false>(a, r, s);
-    else if (r.n >= 1024) window_store_kernel<false, 4><<<dim3(cdiv(units, 4), cdiv(r.n, 4)), 256, 0, s>>>(a, r.slots, r.lens, r.n);
-    else window_store_kernel<false, 1><<<dim3(cdiv(units, 4), r.n), 256, 0, s>>>(a, r.slots, r.lens, r.n);
+    else if (r.n >= 1024) window_store_kernel<false, 4><<<dim3(blocks, cdiv(r.n, 4)), 256, 0, s>>>(a, r.slots, r.lens, r.n, first);
+    else window_store_kernel<false, 1><<<dim3(blocks, r.n), 256, 0, s>>>(a, r.slots, r.lens, r.n, first);
   }
   GPTOSS_LAUNCH_CHECK("window_store_kernel");
   const int widest = std::max(a.dim, a.vdim);
@@ -680,7 +858,8 @@ int run_window_attn(const WindowAttn &a, const StepRows &r, hipStream_t s) {
     TraceScope ts("window_decode", s);
     const dim3 grid(r.n_singles, a.kv_heads, cdiv(a.heads / a.kv_heads, 16));
     const bool both = a.dim_pad() == a.vdim_pad();
-    if (widest <= 64)
+    if (norms_q) window_decode_kernel<64, true, true><<<grid, 256, 0, s>>>(a, r.singles);
+    else if (widest <= 64)
       both && a.dim_pad() == 64 ? window_decode_kernel<64, true><<<grid, 256, 0, s>>>(a, r.singles)
                                 : window_decode_kernel<64, false><<<grid, 256, 0, s>>>(a, r.singles);
     else if (widest <= 128)
@@ -693,7 +872,10 @@ int run_window_attn(const WindowAttn &a, const StepRows &r, hipStream_t s) {
   if (t.n) {
     TraceScope ts("window_tiles", s);
     const dim3 grid(t.n, a.kv_heads);
-    if (widest <= 64) window_tile_kernel<64><<<grid, 256, 0, s>>>(a, t.tiles);
+    const int items = cdiv(t.n * a.kv_heads, 8) * 8;
+    if (norms_q) window_tile64_kernel<true><<<items, WTILE_WAVES * 64, 0, s>>>(a, t.tiles, t.n);
+    else if (a.dim_pad() == 64 && a.vdim_pad() == 64) window_tile64_kernel<false><<<items, WTILE_WAVES * 64, 0, s>>>(a, t.tiles, t.n);
+    else if (widest <= 64) window_tile_kernel<64><<<grid, 256, 0, s>>>(a, t.tiles);
     else if (widest <= 128) window_tile_kernel<128><<<grid, 256, 0, s>>>(a, t.tiles);
     else window_tile_kernel<256><<<grid, 256, 0, s>>>(a, t.tiles);
     GPTOSS_LAUNCH_CHECK("window_tile_kernel");

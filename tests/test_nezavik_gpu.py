@@ -286,6 +286,23 @@ def test_other_sizes(open_model, name, precise):
     check_model(e, 1, cfg, w, tok, precise, [70, 1, 2, 13, 1], factor)
 
 
+# query and kv heads, key and value size, window, scale: three, one, 130 and eight query heads per kv head (a piece of 42 rows, of
+# 128, of one in two passes, of 16), sizes that only the padded cache makes 64, scores that raise the reference often
+HEADS_OF_64 = [(6, 2, 64, 64, 90, 0.125), (4, 4, 64, 50, 65, 0.5), (130, 1, 64, 64, 70, 0.125), (8, 1, 40, 64, 128, 0.2), (4, 2, 64, 64, 300, 3.0)]
+
+
+@pytest.mark.parametrize("heads,kv,dim,vdim,window,scale", HEADS_OF_64)
+def test_windows_over_heads_of_64(open_model, heads, kv, dim, vdim, window, scale):
+    """Stretches whose pieces end inside a block, start in the middle of one and go round the ring, and single rows behind
+    them, both with the queries' norm in the attention."""
+    cfg = nm.config([nm.parallel(heads=heads, kv=kv, dim=dim, vdim=vdim, window=window, scale=scale, ff=None)])
+    w = nm.weights(cfg, 77)
+    tok = nm.tokens(cfg, 460, 6)
+    e = open_model(cfg, w, False, max_batch=2)
+    check_model(e, 0, cfg, w, tok, False)
+    check_model(e, 1, cfg, w, tok, False, [130, 1, 62, 1, 1, 200, 65])
+
+
 @BOTH
 def test_wide_rows_and_passes_of_thousands_of_rows(open_model, precise):
     """Sizes at which the products cut their sum over K into parts (few rows, many inputs), and a pass of thousands of rows, of
