@@ -101,8 +101,8 @@ inline bool gemm_few_applies(const GemmParams &p, int rows_per_tile, int max_til
 // Grouped problems, tiles of 64 rows: the few-row kernels while the launch leaves CUs without work (the block with 4
 // experts of 33 rows, 2880 x 2880: 94 -> 70 us); with more work than that the streaming kernels follow HBM as well or
 // better (16 experts of 25 rows on average: 160 against 167 us; 32 experts, 200-400 tokens: equal within 1 %).
-inline bool grouped_few(const GemmParams &p, int rows_per_tile, int max_tiles) {
-  return rows_per_tile == 32 || (long long)max_tiles * (p.N / 32) <= 1280;
+inline bool grouped_few(int rows_per_tile, int max_tiles, int N) {
+  return rows_per_tile == 32 || (rows_per_tile == 64 && (long long)max_tiles * (N / 32) <= 1280);
 }
 // gemm_dense.cpp: bf16 weights, no gather (run_gemm comes here for that form)
 int run_gemm_dense(const GemmParams &p, int epi, int rows_per_tile, int max_tiles, hipStream_t s);
@@ -173,6 +173,8 @@ int dense_gemm_mixed(const bf16_t *A, const bf16_t *W, float *out, const GemmBf1
 constexpr int GEMM_MAX_PARTS = 16;
 int dense_gemm_partial(const bf16_t *A, const bf16_t *W, float *out, size_t max_elems, int *parts, int B, int N, int K,
                        hipStream_t s);
+// Estimated us of a grouped product in bf16 with `tiles` row tiles (gemm_dense.cpp), by the few-row kernels or not
+double grouped_us(int rows_per_tile, double tiles, bool few, int N, int K);
 int gemm_col_tiles(int N);  // column tiles of one workgroup's width
 inline int gemm_argmax_tiles(int N) { return 2 * gemm_col_tiles(N); }  // pairs per row to allocate for EPI_ARGMAX
 // moe_route.hip

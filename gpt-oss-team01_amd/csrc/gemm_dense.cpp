@@ -1,5 +1,6 @@
 // Host side of the dense bf16 GEMMs (kernel dispatch) and the weight repacking kernel.  The GEMM kernels
 // themselves are in gemm_kernel.hpp and gemm_tall_kernel.hpp.
+#include <math.h>
 #include <stdlib.h>
 
 #include <mutex>
@@ -123,7 +124,7 @@ int run_gemm_dense(const GemmParams &p, int epi, int rows_per_tile, int max_tile
                  "run_gemm: rows x columns must stay below 2^32 elements (rows<=%lld N=%d K=%d)", max_rows, p.N, p.K);
   if (rows_per_tile == 256) return run_gemm_tall(p, epi, max_tiles, max_rows, s);
   if (epi != EPI_ARGMAX && gemm_few_applies(p, rows_per_tile, max_tiles) &&
-      (p.tiles ? grouped_few(p, rows_per_tile, max_tiles) : epi == EPI_PARTIAL || dense_few(rows_per_tile, max_tiles, p.N, p.K)))
+      (p.tiles ? grouped_few(rows_per_tile, max_tiles, p.N) : epi == EPI_PARTIAL || dense_few(rows_per_tile, max_tiles, p.N, p.K)))
     return run_gemm_few(p, false, epi, rows_per_tile, max_tiles, s);
   int prc = gemm_prepare_device();
   if (prc != GPTOSS_OK) return prc;
@@ -138,12 +139,20 @@ int run_gemm_dense(const GemmParams &p, int epi, int rows_per_tile, int max_tile
 // The same for the 256-row kernel (gemm_tall_kernel.hpp): rounds of 32 tiles per XCD, the last one in halves of a tile where
 // they leave half of its workgroups idle.  A CU's slab takes longer the more CUs multiply (the chip is at its power limit).
 // Within 6 % of 63 products: 9 shapes of 1024-24576 columns and K 512-10240 at 7 row counts of 2048-8000, at fewer rows within 8 %.
-static double tall_us(int B, int N, int K) {
-  const int mine = (cdiv(B, 256) * cdiv(N, 256) + 7) / 8, rest = mine % 32, slabs = K / 64;
+static double tall_tiles_us(double tiles, int slabs) {
+  const int mine = (int)ceil(tiles / 8), rest = mine % 32;
   double us = 4.0 + mine / 32 * (11.5 + 1.44 * slabs);
   if (rest && 2 * rest <= 32) us += 9.0 + (0.39 + 0.45 * rest / 16.0) * slabs;
   else if (rest) us += 11.5 + (0.54 + 0.9 * rest / 32.0) * slabs;
   return us;
+}
+static double tall_us(int B, int N, int K) { return tall_tiles_us(cdiv(B, 256) * cdiv(N, 256), K / 64); }
+
+double grouped_us(int rows_per_tile, double tiles, bool few, int N, int K) {
+  // (tiles of several experts share no weights: a tenth more)
+  if (rows_per_tile == 256) return 1.1 * tall_tiles_us(tiles * cdiv(N, 256), K / 64);
+  return few ? few_us(rows_per_tile / 32, (long long)(tiles * (N / 32)), K / 64)
+             : streaming_us(rows_per_tile / 32, (long long)(tiles * gemm_col_tiles(N) * 8), K / 64);
 }
 
 // GPTOSS_DENSE_TALL_MIN_ROWS: rows from which a dense fp32-output GEMM uses the 256-row kernel, in place of the estimates

@@ -271,7 +271,7 @@ int run_gemm(const GemmParams &p, bool gather, int epi, int rows_per_tile, int m
     GPTOSS_REQUIRE(run_gemm_mxfp4, GPTOSS_ERR_STATE, "run_gemm: this library was linked without the MXFP4 kernels");
     return run_gemm_mxfp4(p, gather, epi, rows_per_tile, max_tiles, s);
   }
-  if (gather && epi == EPI_SWIGLU && gemm_few_applies(p, rows_per_tile, max_tiles) && grouped_few(p, rows_per_tile, max_tiles))
+  if (gather && epi == EPI_SWIGLU && gemm_few_applies(p, rows_per_tile, max_tiles) && grouped_few(rows_per_tile, max_tiles, p.N))
     return run_gemm_few(p, true, epi, rows_per_tile, max_tiles, s);
   int prc = gemm_prepare_device();
   if (prc != GPTOSS_OK) return prc;

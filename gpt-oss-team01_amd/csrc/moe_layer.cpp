@@ -66,9 +66,12 @@ static int env_int(const char *name, int dflt) {
 // one of 160 holds them (150 rows 496 / 531 -> 479 / 555, 128 391 / 506 -> 434 / 505), above two of either (275 692 / 737 ->
 // 790 / 704, 325 837 / 802 -> 861 / 784).  Small blocks lose here too: 2048 x 1024, 32 experts of 200 210 / 212 -> 227 / 213, eight of
 // 2880 x 2880 187 / 173 -> 163 / 187.
-static bool moe_tall(long long pairs, int E, int N, int K) {
+static int moe_tall_forced() {
   static const int v = env_int("GPTOSS_MOE_TALL_MIN_ROWS", 0);
-  if (v) return pairs >= (long long)v * E;
+  return v;
+}
+static bool moe_tall(long long pairs, int E, int N, int K) {
+  if (const int v = moe_tall_forced()) return pairs >= (long long)v * E;
   const double work = (double)pairs * N * K;
   if (pairs >= (long long)(work >= (double)(1ll << 34) ? 416 : 512) * E) return true;
   return work >= (double)(1ll << 35) && pairs >= 165ll * E && pairs <= 248ll * E;
@@ -85,6 +88,44 @@ int moe_rows_per_tile(int B, int k, int E, bool mxfp4) {
   if (mxfp4) return 64;
   if (need <= 128) return 128;
   return 160;
+}
+
+// Row tiles of E experts with `avg` rows each on average, spread as a uniform routing spreads them.
+static double expected_tiles(int k, int E, double avg, int rows_per_tile) {
+  if (k == E) return E * ceil(avg / rows_per_tile);
+  const double s = sqrt(2 * avg * (1 - (double)k / E));
+  double n = 1;
+  for (int m = 1; m * rows_per_tile <= 2 * avg + 64; m++) n += 0.5 * erfc((m * rows_per_tile + 0.5 - avg) / s);
+  return E * n;
+}
+
+// The row tile of a bf16 block, given the one that holds an expert's rows: where tiles of that size are work for fewer than two
+// rounds of the CUs, the one that makes both products shortest by the estimates of gemm_dense.cpp.  Smaller tiles put more
+// CUs to work (an item of 160 rows is a CU's for 20 to 50 us), and where every token takes every expert, so that the tiles are known,
+// 256 rows may save a round.  It has to be ahead by a tenth, the estimates' error, or by a quarter where the rows per expert are
+// not known: the estimates are for a uniform routing.  Blocks in us, before -> after: 4 of 4 experts, 2048 x 1024, 70 / 135 /
+// 240 rows each 61 / 73 / 75 -> 39 / 42 / 44, 2880 x 2880, 100 / 330 rows 102 / 192 -> 82 / 131; 4 of 16, 1024 x 512, 60 / 200 rows
+// 45 / 61 -> 35 / 51; two of 4, 4096 x 1536, 70 rows 93 -> 64.  Of 500 blocks of random sizes, uniform and Zipf 1.1, a few lose, up to 6 %.
+static int small_block_rows(int dflt, int B, int k, int E, int H, int I, bool tall) {
+  const double avg = (double)B * k / E;
+  if (dflt <= 64 || dflt == 256 || expected_tiles(k, E, avg, dflt) * gemm_col_tiles(2 * I) >= 512) return dflt;
+  auto us = [&](int rpt) {
+    const int max_tiles = gptoss_moe_max_tiles(B, k, std::min(E, B * k), rpt);
+    const double tiles = expected_tiles(k, E, avg, rpt);
+    return grouped_us(rpt, tiles, grouped_few(rpt, max_tiles, 2 * I), 2 * I, H) + grouped_us(rpt, tiles, grouped_few(rpt, max_tiles, H), H, I);
+  };
+  int best = dflt;
+  double least = (k == E ? 0.9 : 0.75) * us(dflt);
+  for (int rpt : {32, 64, 128, 160, 256}) {
+    // (tiles of 32 rows read the weights again and again: not beyond two rounds of the few-row kernels)
+    if ((rpt == 256 && (!tall || k != E)) || (rpt == 32 && expected_tiles(k, E, avg, 32) * (2 * I / 32) > 2560)) continue;
+    const double t = us(rpt);
+    if (t < least) {
+      least = t;
+      best = rpt;
+    }
+  }
+  return best;
 }
 
 // Fixed part of a work item's cost, in half units of one 32-row block of arithmetic, used to cut
@@ -159,8 +200,11 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
   // a prompt pass, hundreds of rows per expert: bound by the matrix cores, not by streaming W
   // (the kernels address a row of A by a 32-bit byte offset: batches beyond that stay on the streaming kernels)
   const long long tall_rows = ((long long)B * k / 256 + E) * 256;
-  if (!mxfp4 && moe_tall((long long)B * k, E, 2 * I, H) && gemm_tall_shape_ok(2 * I, H, tall_rows) && gemm_tall_shape_ok(H, I, tall_rows))
-    rpt = 256;
+  if (!mxfp4) {
+    const bool tall = gemm_tall_shape_ok(2 * I, H, tall_rows) && gemm_tall_shape_ok(H, I, tall_rows);
+    if (tall && moe_tall((long long)B * k, E, 2 * I, H)) rpt = 256;
+    if (!moe_tall_forced()) rpt = small_block_rows(rpt, B, k, E, H, I, tall);
+  }
   // (no more experts have a row than there are rows)
   const int max_tiles = gptoss_moe_max_tiles(B, k, std::min(E, B * k), rpt);
   // Each expert's row tiles are walked in blocks of up to MOE_TILE_BLOCK, column tile by column

@@ -553,6 +553,21 @@ def test_large_blocks_of_one_and_two_row_tiles_per_expert(ops, rows):
         assert torch.equal(layer.forward(t[i:i + 64].contiguous()), out[i:i + 64]), i
 
 
+@pytest.mark.parametrize("E,k,H,I", [(4, 4, 2048, 1024), (4, 2, 512, 256), (16, 4, 1024, 512), (4, 4, 2880, 2880)])
+@pytest.mark.parametrize("rows", [33, 64, 65, 97, 129, 161, 240, 330])
+def test_blocks_that_leave_cus_idle_give_the_same_in_tiles_of_any_size(ops, E, k, H, I, rows):
+    """Up to 330 rows per expert where tiles of 32 to 256 rows are chosen by estimated time, against batches of 16 tokens."""
+    B = rows * E // k
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    layer = ops.MoeLayer(n(E, H), n(E).float(), n(E, 2 * I, H, std=0.02), n(E, 2 * I).float(), n(E, H, I, std=0.02),
+                         n(E, H).float(), top_k=k, max_tokens=B)
+    t = n(B, H)
+    out = layer.forward(t).clone()
+    for i in range(0, B, 16):
+        assert torch.equal(layer.forward(t[i:i + 16].contiguous()), out[i:i + 16]), i
+
+
 @pytest.mark.parametrize("k", [1, 2, 3, 5, 7, 8])
 def test_tokens_of_pairs_in_a_prompt_pass(ops, k):
     """Every token on all k experts: the token of a pair is the pair's number over k."""
