@@ -13,8 +13,8 @@
 //     then its V in V^T operand order, common.hpp): a wave reads 16 KB contiguous per block with
 //     128-bit loads, the four waves of a workgroup 64 KB; position p lives in slot p % capacity
 //     (ring buffer for window layers);
-//   * contexts of up to ATT_CHUNK slots are one wave's single pass, or, where a launch has few of them,
-//     a workgroup's with the same bits (attn_few_kernel);
+//   * contexts of up to ATT_CHUNK slots are one wave's single pass, or, unless a launch has very many of them,
+//     a workgroup's with the same bits (attn_few_kernel, attn_chunks_kernel);
 //   * longer contexts, few sequences: cut into chunks (flash-decoding), one wave each, or again a
 //     workgroup: partial (max, sum, O) per chunk go to the workspace and a small second kernel merges
 //     them with the sink.  The chunk length is a constant, so a row's result is the same whatever else
@@ -643,7 +643,8 @@ struct RopeInput {
   const float *cos_t, *sin_t;  // [positions, D / 2]
   bf16_t *kv;
 };
-template <int D, bool ROPE>
+// NT: more chunks than the caches hold, read once.  WIDE: in front of the workgroup-per-row kernel, see there.
+template <int D, bool ROPE, bool NT = false, bool WIDE = false>
 __device__ __forceinline__ void attn_few_chunk(const AttnParams &p, const RopeInput &rope) {
   constexpr int KS = D / 32, DB = D / 16, NBLK = ATT_CHUNK / ATT_BLOCK;
   static_assert(NBLK == 8 && DB <= 4, "two blocks and at most 16 output columns per wave");
@@ -651,12 +652,17 @@ __device__ __forceinline__ void attn_few_chunk(const AttnParams &p, const RopeIn
   __shared__ float lds_sum[NBLK][64], lds_max[NBLK][16];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (WIDE && blockIdx.x == gridDim.x - 1) {   // the extra workgroup writes the row order
+    static_assert(sizeof lds_p >= 2 * (ATT_ORDER_BUCKETS + 1) * sizeof(int), "room for the counters");
+    attn_write_order(p, reinterpret_cast<int *>(lds_p));
+    return;
+  }
   const int n = lane & 15, c = lane >> 4, G = p.G;
   const int g = blockIdx.x % p.n_kv, rest = blockIdx.x / p.n_kv;
   const int b = rest % p.B, chunk_id = p.max_chunks - 1 - rest / p.B;
   const int length = __builtin_amdgcn_readfirstlane(row_len(p, b));
   const SeqRange r = seq_range(length, p.cap, p.window, p.max_len);
-  if (chunk_id >= r.nchunks) return;
+  if (chunk_id >= r.nchunks || (WIDE && r.nchunks > 1)) return;
   const int c0 = r.s_begin + chunk_id * r.chunk, c1 = min(r.s_end, c0 + r.chunk);
   const int nb = (max(0, c1 - c0) + ATT_BLOCK - 1) / ATT_BLOCK;
   const int pos_base = (r.len > 0) ? ((r.len - 1) / p.cap) * p.cap : 0;
@@ -674,10 +680,14 @@ __device__ __forceinline__ void attn_few_chunk(const AttnParams &p, const RopeIn
   if (p.seq_map) seq = __builtin_amdgcn_readfirstlane(p.seq_map[seq]);
   const bf16_t *plane = p.kv + kv_block_off(seq, g, p.n_kv, p.cap, D, 0);
 
-  // All loads at once, the query first, because they return in order.  (Plain loads: so few rows stay in the caches for
+  // All loads at once, the query first, because they return in order.  (Plain loads where so few rows stay in the caches for
   // the next step.)  Blocks that a row does not have are left out by one jump to behind the last: even loads that hit the
   // cache are time on the CU's only path to it, and jumps over each are as many misses in the instruction cache.  One row
   // of 60 6.0 -> 4.8 us, 8 of 100 6.5 -> 5.3, of 300 7.8 -> 7.0.
+  auto fetch = [](const bf16_t *x) {
+    if (!NT) return *reinterpret_cast<const u32x4 *>(x);
+    return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x));
+  };
   auto block_at = [&](int j) { return plane + (size_t)((c0 >> 6) + j) * (2 * KV_BLOCK * D); };
   const int db = min(wave, DB - 1);   // head size 32: two waves are done after their weights
   f32x4 qx[2 * KS];
@@ -709,14 +719,14 @@ __device__ __forceinline__ void attn_few_chunk(const AttnParams &p, const RopeIn
     for (int tb = 0; tb < 4; tb++)
 #pragma unroll
       for (int s = 0; s < KS; s++)
-        kreg[u][tb][s] = *reinterpret_cast<const u32x4 *>(block_at(wave + 4 * u) + (tb * 16 + n) * D + c * KS * 8 + s * 8);
+        kreg[u][tb][s] = fetch(block_at(wave + 4 * u) + (tb * 16 + n) * D + c * KS * 8 + s * 8);
   }
 #pragma unroll
   for (int j = 0; j < NBLK; j++) {
     if (j >= nb) break;
 #pragma unroll
     for (int grp = 0; grp < 2; grp++)
-      vreg[j][grp] = *reinterpret_cast<const u32x4 *>(block_at(j) + KV_BLOCK * D + (grp * DB + db) * 512 + lane * 8);
+      vreg[j][grp] = fetch(block_at(j) + KV_BLOCK * D + (grp * DB + db) * 512 + lane * 8);
   }
   if constexpr (ROPE) {
     auto rotate = [&](f32x4 (&x)[2 * KS]) {
@@ -879,6 +889,10 @@ __device__ __forceinline__ void attn_few_chunk(const AttnParams &p, const RopeIn
 }
 template <int D>
 __global__ __launch_bounds__(256, 1) void attn_few_kernel(AttnParams p) { attn_few_chunk<D, false>(p, RopeInput{}); }
+// The same for more chunks than CUs hold at once: three workgroups a CU, and reads with the non-temporal hint or (WIDE) plain ones,
+// which are then 2-5 % faster.
+template <int D, bool WIDE>
+__global__ __launch_bounds__(256, 3) void attn_chunks_kernel(AttnParams p) { attn_few_chunk<D, false, !WIDE, WIDE>(p, RopeInput{}); }
 template <int D>
 __global__ __launch_bounds__(256, 1) void attn_few_rope_kernel(AttnParams p, RopeInput rope) { attn_few_chunk<D, true>(p, rope); }
 
@@ -894,6 +908,31 @@ __global__ __launch_bounds__(256, 1) void attn_few_rope_kernel(AttnParams p, Rop
 static bool attn_few(long long pairs, int span, int head_dim) {
   const long long items = pairs * ((span + ATT_CHUNK - 1) / ATT_CHUNK);
   return items <= (span * head_dim < 256 * 64 ? 256 : head_dim == 32 ? 384 : 512);
+}
+
+struct AttnPlan {
+  int max_chunks;
+  bool wide;          // many sequences: rows of more than one chunk get a workgroup each, no partials
+  size_t order_bytes, part_o_bytes, part_ml_bytes;
+};
+
+// Beyond those, heads of 64: attn_chunks_kernel instead of a wave per item.  Four waves of one workgroup, the chunks of one row and
+// four kv heads, are one CU's 512 KB where another CU has none (a CU reads about 40 KB a us), and a wave takes its blocks one
+// behind the other, 20 us for 512 positions.  64 heads of 64 on 8 kv heads, caches cold, rows of an eighth to all of the length / all
+// of it, a wave per item -> workgroup per item (us):
+//   chunks merged by a kernel behind   17 sequences of 5000 39.3 / 43.4 -> 26.7 / 38.4, 40 of 1000 23.2 / 24.7 -> 20.3 / 24.0, 63 of 4000
+//     76.0 / 94.8 -> 59.1 / 92.7, 32 of 32000 315 / 405 -> 262 / 393; the worst 30 of 4000 40.6 / 46.8 -> 32.5 / 48.5.  Always.
+//   rows of one chunk   80 of 300 15.2 / 16.0 -> 12.6 / 14.8, 150 of 257 21.7 / 27.8 -> 16.8 / 22.2, 255 of 448 25 / 30 -> 23 / 30;
+//     100 of 400 19.1 / 20.9 -> 16.4 / 22.4, 512 of 300 47.5 / 57.3 -> 45.7 / 59.9, 256 of 128 15.8 / 16.1 -> 18.8 / 18.3.
+//     From 256 positions on, up to 2560 items, and not where the host knows that all rows are of one length.
+//   rows of one chunk in front of the workgroup-per-row kernel   64 of 1000 35.8 / 27.9 -> 27.2 / 27.4, 98 of 736 34.8 / 34.5 ->
+//     29.0 / 34.4, 256 of 1000 74.4 / 85.7 -> 61.0 / 85.7, 512 of 1000 124.6 / 166.1 -> 112.2 / 167.4; of 1024 of 600, where
+//     8192 workgroups may have nothing to do, 162.1 / 214.9 -> 149.8 / 218.5.  Up to 4096 items.
+// (Rows of a prompt read the same blocks: those stay with a wave per item.)
+static bool attn_many(long long items, const AttnPlan &pl, int span, int head_dim, bool one_length) {
+  if (head_dim != 64) return false;
+  if (pl.wide) return items <= 4096;
+  return pl.max_chunks > 1 ? items < (1ll << 31) : span >= 256 && items <= 2560 && !one_length;
 }
 
 // Merge the chunk partials of one (sequence, q head) with the sink logit.  One thread owns four
@@ -1220,22 +1259,16 @@ static int attn_tile_min_rows() {
   return v;
 }
 
-struct AttnPlan {
-  int max_chunks;
-  bool wide;          // many sequences: rows of more than one chunk get a workgroup each, no partials
-  size_t order_bytes, part_o_bytes, part_ml_bytes;
-};
-
 // Enough sequences that one workgroup per (sequence, kv head) fills the chip twice over: then long
 // rows are served by the workgroup-per-row kernel.  A property of the launch shape alone, so a
 // row's arithmetic depends on the number of sequences in the call but never on their contents.
 static bool attn_wide(int n_seq, int n_kv) { return (long long)n_seq * n_kv >= 512; }
 
-static AttnPlan attn_plan(int B, int rows_per_seq, int n_q, int n_kv, int D, int span) {
+static AttnPlan attn_plan(int B, int rows_per_seq, int n_q, int n_kv, int D, int span, bool windowed) {
   AttnPlan pl;
-  // most work items any row can have: a slot range can start up to 63 slots before the first
+  // most work items any row can have: the slot range of a window can start up to 63 slots before the first
   // active position
-  const int longest = span + ATT_BLOCK - 1;
+  const int longest = windowed ? span + ATT_BLOCK - 1 : span;
   pl.max_chunks = (longest + ATT_CHUNK - 1) / ATT_CHUNK;
   if (pl.max_chunks < 1) pl.max_chunks = 1;
   pl.wide = pl.max_chunks > 1 && attn_wide(B / std::max(1, rows_per_seq), n_kv);
@@ -1327,7 +1360,7 @@ static int attn_launch(const float *q, const void *kv_cache, const int *lens,
   // longest slot range one sequence can visit: the whole ring once it may have wrapped
   int span = (max_len > capacity) ? capacity
                                   : ((window > 0 && window < max_len) ? window : max_len);
-  AttnPlan pl = attn_plan(B, rows_per_seq, n_q, n_kv, head_dim, span);
+  AttnPlan pl = attn_plan(B, rows_per_seq, n_q, n_kv, head_dim, span, window > 0);
   const size_t need = pl.order_bytes + pl.part_o_bytes + pl.part_ml_bytes;
   GPTOSS_REQUIRE(workspace && aligned(workspace, 256) && workspace_bytes >= need, GPTOSS_ERR_WORKSPACE,
                  "attn_decode: workspace missing, misaligned or smaller than %zu bytes", need);
@@ -1380,9 +1413,10 @@ static int attn_launch(const float *q, const void *kv_cache, const int *lens,
     // writes them 16 bytes at a time; an output that is only 8-byte aligned gets the plain launch)
     const bool hold_rows = !pair && aligned(out, 16);
     const bool few = !pair && !pl.wide && attn_few((long long)B * n_kv, span, head_dim);
+    const bool many = rows_per_seq <= 1 && !few && attn_many(items, pl, span, head_dim, !lens && len_period == 0);
     TraceScope ts(few ? "attn_decode_few" : "attn_decode", s);
     int resident = 0;
-    if (hold_rows && !few) {
+    if (hold_rows && !few && !many) {
       const int rc = head_dim == 64 ? attn_resident_wgs<64>(&resident) : attn_resident_wgs<32>(&resident);
       if (rc != GPTOSS_OK) return rc;
     }
@@ -1390,6 +1424,9 @@ static int attn_launch(const float *q, const void *kv_cache, const int *lens,
       auto launch = [&](auto kernel, const auto &...more) { kernel<<<(int)items, 256, 0, s>>>(p, more...); };
       if (rope) launch(head_dim == 64 ? attn_few_rope_kernel<64> : attn_few_rope_kernel<32>, *rope);
       else launch(head_dim == 64 ? attn_few_kernel<64> : attn_few_kernel<32>);
+    } else if (many) {
+      if (pl.wide) attn_chunks_kernel<64, true><<<(int)items + 1, 256, 0, s>>>(p);
+      else attn_chunks_kernel<64, false><<<(int)items, 256, 0, s>>>(p);
     } else if (head_dim == 64) {
       if (pair) attn_decode_kernel<64, true><<<grid, 256, 0, s>>>(p);
       else if (hold_rows) attn_decode_resident_kernel<64><<<std::min(grid, resident), 256, 0, s>>>(p, grid);
@@ -1437,7 +1474,7 @@ int gptoss::attn_decode_rope(const float *qkv, float *q, const float *cos_t, con
                              void *stream, const int *seq_map) {
   const int span = max_len > capacity ? capacity : window > 0 && window < max_len ? window : max_len;
   const bool here = own_sequences && (head_dim == 32 || head_dim == 64) && n_kv > 0 && n_q % n_kv == 0 &&
-                    !attn_plan(B, 1, n_q, n_kv, head_dim, span).wide && attn_few((long long)B * n_kv, span, head_dim) &&
+                    !attn_plan(B, 1, n_q, n_kv, head_dim, span, window > 0).wide && attn_few((long long)B * n_kv, span, head_dim) &&
                     aligned(qkv, 16) && aligned(cos_t, 16) && aligned(sin_t, 16);
   const RopeInput rope{qkv, cos_t, sin_t, (bf16_t *)kv_cache};
   if (!here) {

@@ -336,6 +336,30 @@ def test_few_rows_of_several_chunks_have_the_bits_of_the_same_rows_among_more(op
         assert torch.equal(out[rows].view(torch.int16), out[B][:rows].view(torch.int16)), rows
 
 
+# rows of one chunk: up to 320 sequences a workgroup each, 330 a wave; of one chunk and of several: up to 512 sequences a
+# workgroup for each of one chunk as well, in front of the kernel that takes the others, 520 a wave
+@pytest.mark.parametrize("sequences,longest,cap,window", [
+    ((330, 65, 200, 320), 256, 256, 0), ((330, 65, 200, 320), 512, 512, 0), ((330, 65, 320), 512, 512, 300),
+    ((520, 64, 65, 300, 512), 700, 704, 0), ((520, 64, 512), 900, 640, 576)])
+def test_rows_have_the_same_bits_a_workgroup_or_a_wave_each(ops, sequences, longest, cap, window):
+    B, n_q, n_kv, D = sequences[0], 64, 8, 64
+    g = torch.Generator(device="cuda").manual_seed(longest + window)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    edges = [longest, 0, 1, 64, 65, 255, 256, 257, 448, 449, 511, 512, 513]
+    lens = [min(x, longest) for x in edges] + torch.randint(1, longest + 1, (B - len(edges),), generator=g, device="cuda").tolist()
+    lens = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    cache = ops.KVCache(B, n_kv, D, cap)
+    cache.kv.view(torch.int16).fill_(0x7FC1)             # NaN patterns where nothing is written
+    cache.write(rnd(B, min(longest, cap), n_kv, D).bfloat16(), rnd(B, min(longest, cap), n_kv, D).bfloat16(), 0)
+    q, sinks = rnd(B, n_q, D) * 2, rnd(n_q)
+    out = {}
+    for rows in sequences:
+        attn = ops.AttnDecode(rows, n_q, n_kv, D, longest)
+        out[rows] = attn.forward(q[:rows].contiguous(), cache.first(rows), lens[:rows], sinks, window=window)
+        assert torch.isfinite(out[rows]).all()
+        assert torch.equal(out[rows].view(torch.int16), out[B][:rows].view(torch.int16)), rows
+
+
 @pytest.mark.parametrize("pos0,T", [(0, 130), (500, 70), (900, 9)])
 def test_prompt_rows_of_more_than_eight_heads_per_kv_head(ops, pos0, T):
     """They go row by row: thousands of rows are many, however few the sequences are."""
