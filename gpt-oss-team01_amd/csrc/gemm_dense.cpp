@@ -92,7 +92,8 @@ static int gemm_prepare_device() {
 // 11.1 instead of 8.1; 2048 x 256, 257 rows 8.0 instead of 6.3).
 // The few-row kernels have become faster since, tiles of up to 16 rows by up to a third (gemm_few_kernel.hpp), which the fit leaves
 // out: uncut products of up to 8 / 16 rows take 0.79 / 0.85 of few_us' time, where the streaming kernels take 1.12 of streaming_us', so
-// these and more parts look better there than they are.  What that costs is stated at the two rules that use it.
+// these look better there than they are.  What that costs is stated at the rules that use it; how often to cut the K of so
+// few rows is by partial_us.
 static double streaming_us(int mb, long long blocks, int slabs) {
   // [mb - 1]: launch; per round, and per slab of it; per full round's items, and per slab of them
   static const double t[5][5] = {{3.2, 0.63, 0.496, 1.8, 0.028}, {3.5, 1.35, 0.533, 3.3, 0.106}, {4.0, 2.5, 0.578, 3.8, 0.145},
@@ -109,6 +110,16 @@ static double few_us(int mb, long long blocks, int slabs) {
   const double rounds = (double)((blocks + 1023) / 1024), full = blocks / 1024.0;
   return mb == 1 ? 3.4 + rounds * (1.1 + 0.175 * slabs) + full * (0.7 + 0.071 * slabs)
                  : 3.9 + rounds * (1.58 + 0.191 * slabs) + full * (1.15 + 0.147 * slabs);
+}
+
+// The few-row kernels on up to 8 or 16 rows, K cut into parts: 59 shapes of 512-16384 columns and K 512-12288 at every number of parts
+// up to 16, weights from HBM, 1 / 6 / 8 / 12 / 16 rows; 4 to 5 % rms (some of 9 to 16 rows beyond 512 blocks 8).  256 blocks to a round.
+static double partial_us(int rows, long long blocks, int slabs) {
+  // [rows > 8][more than FEW_SOLO_BLOCKS]: launch; per round, and per slab of it; per full round's blocks, and per slab of them
+  static const double t[2][2][5] = {{{2.6, 0.76, 0.035, -0.2, 0.1}, {2.6, 0.46, 0.047, -0.048, 0.096}},
+                                    {{2.9, 0.065, 0.056, 0.49, 0.091}, {2.9, 1.0, 0.0021, -0.62, 0.15}}};
+  const double *c = t[rows > 8][blocks > FEW_SOLO_BLOCKS], full = blocks / 256.0;
+  return c[0] + (double)((blocks + 255) / 256) * (c[1] + c[2] * slabs) + full * (c[3] + c[4] * slabs);
 }
 
 // Uncut dense problems: the kernel that is estimated to be the faster one with this row tile.
@@ -271,10 +282,12 @@ int dense_gemm_mixed(const bf16_t *A, const bf16_t *W, float *out, const GemmBf1
 }
 
 // Few rows and few columns leave most CUs without a work item while those that have one walk all of K.
-// Cutting K makes more items; what it costs is a part per round and the reading of the partial sums.  All row tiles and parts timed at the 312 sizes above, with the kernels that the estimates were fitted to:
+// Cutting K makes more items; what it costs is a part per round and the reading of the partial sums.  All row tiles and parts timed
+// at the 312 sizes above, with the kernels that the estimates were fitted to:
 // the chosen ones take 2 % longer than the best ones on average and are 15 % faster than with streaming kernels alone (2048 x 2048,
-// 8 / 400 / 1024 rows 7.0 / 14.6 / 21.8 -> 4.7 / 11.5 / 17.5 us).  With the present ones, 53 shapes, up to 8 / 16 / 32 rows: 9 / 8 / 6 % longer, as
-// fewer parts would do (8192 x 1024, 8 rows 7.2 us in four parts, 5.4 uncut; 2048 x 4096 7.2 in sixteen, 5.6 in four).
+// 8 / 400 / 1024 rows 7.0 / 14.6 / 21.8 -> 4.7 / 11.5 / 17.5 us).  Up to 8 / 16 rows, where partial_us decides, the chosen parts
+// take 1 % longer than the best, by few_us 9 / 7 % (2048 x 12288, 8 rows, 16 parts 11.7 us, four 10.3; 4096 x 2048 eight 6.7, one or two
+// 5.5-5.8; 2880 x 4096 eleven 7.6, two 6.7); 17 to 32 rows 5 %.
 int dense_gemm_partial(const bf16_t *A, const bf16_t *W, float *out, size_t max_elems, int *parts, int B, int N, int K,
                        hipStream_t s) {
   *parts = 1;
@@ -291,7 +304,7 @@ int dense_gemm_partial(const bf16_t *A, const bf16_t *W, float *out, size_t max_
       if (n != want || (n > 1 && (per < 4 || nslab - per * (n - 1) < 2 || (size_t)n * B * N > max_elems))) continue;
       const int tiles = cdiv(B, 32 * mb);
       const bool few = n == 1 ? dense_few(32 * mb, tiles, N, K) : mb <= 2;   // as run_gemm_dense has it
-      const double cost = (few ? few_us(mb, (long long)tiles * (N / 32) * n, per)
+      const double cost = (few ? B <= 16 ? partial_us(B, (long long)(N / 32) * n, per) : few_us(mb, (long long)tiles * (N / 32) * n, per)
                                : streaming_us(mb, (long long)tiles * g.n_col_tiles * 8 * n, per)) +
                           (n - 1) * (double)B * N * 4 / 5e6;
       if ((mb == 1 && n == 1) || cost < best) {
