@@ -210,16 +210,14 @@ __device__ __forceinline__ void group_by_one_wave(const int *topk_i, int P, int 
 }
 
 // ------------------------------------------------------------------------------------------------
-// Router GEMM: logits[B,E] = t[B,H] . Wr[E,H]^T + br.  One workgroup = 16 token rows x all experts;
-// its 8 waves split the K loop (k-steps of 32, interleaved), request all their operands up front
-// and reduce through LDS.  With topk_w != nullptr the workgroup also gates its 16 tokens (32
-// lanes per token) while the logits are still in LDS.
+// Router GEMM: logits[B,E] = t[B,H] . Wr[E,H]^T + br, and the gating of the tokens, 32 lanes per token, while the logits are
+// still in LDS.
 // ------------------------------------------------------------------------------------------------
 // k-steps whose operands a wave requests before its first MFMA: as many as ~150 registers hold,
 // so that a hidden size of 2880 with up to 32 experts is a single round of loads
 constexpr int router_steps(int nb) { return nb <= 2 ? 12 : (nb <= 4 ? 7 : (nb <= 8 ? 4 : 2)); }
 
-// What the NORM form of the router kernel does first: x += residual, t = RMSNorm(x) * weight for the
+// What norm_router_kernel does first: x += residual, t = RMSNorm(x) * weight for the
 // workgroup's own token rows.
 struct RouterNorm {
   float *x;               // [B,H] residual stream, updated in place
@@ -294,20 +292,52 @@ __device__ __forceinline__ void norm_rows(const RouterNorm &nrm, bf16_t *t_rows,
   }
 }
 
-// NB: number of 16-expert column blocks held per wave.  NORM: the workgroup first normalises its
-// rows (norm_rows) and multiplies them from LDS: one launch and one read of t less than norm kernel + router kernel.
+// What follows the products of a workgroup of ROUTER_WAVES waves, 32 lanes per token row (`live`: it is one): the sum of the
+// waves' parts and the bias, published, and gated if the workgroup has all experts.
+template <int NB>
+__device__ __forceinline__ void router_gate(float (*red)[16][NB * 16 + 1], const float (&bias)[(NB + 1) / 2],
+                                            float *__restrict__ logits, int r0, int e0, bool live, bool has_bias, int B, int E, int k,
+                                            float *__restrict__ topk_w, int *__restrict__ topk_i, const RouterGroup &grp) {
+  constexpr int NJ = (NB + 1) / 2;
+  const int row = threadIdx.x >> 5, sub = threadIdx.x & 31;
+  float v[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; j++) {
+    const int col = sub + 32 * j, e = e0 + col;
+    float x = -INFINITY;
+    if (e < E && col < NB * 16) {
+      x = 0.f;
+#pragma unroll
+      for (int w = 0; w < ROUTER_WAVES; w++) x += red[w][row][col];
+      if (has_bias) x += bias[j];
+      if (live) logits[(size_t)(r0 + row) * E + e] = x;
+    }
+    v[j] = x;
+  }
+  if (topk_w != nullptr) {
+    const size_t o = (size_t)(live ? r0 + row : 0) * k;
+    __shared__ int ids[ROUTER_GROUP_PAIRS];
+    topk_softmax_group<NJ>(v, sub, E, k, live, topk_w + o, topk_i + o, grp.expert_offsets ? ids + row * k : nullptr);
+    if (grp.expert_offsets != nullptr) {   // one workgroup holds every token
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0) group_by_one_wave(ids, B * k, E, reinterpret_cast<int *>(red), grp);
+    }
+  }
+}
+
+// The router behind a norm: the workgroup first normalises its
+// rows (norm_rows) and multiplies them from LDS, with the experts' weights, meanwhile requested, from registers: one launch and one read of t less than norm kernel + router kernel.
 // A small launch is a chain of waits for memory, so all that does not depend on each other is requested at once: the
 // router's weights and biases, a row's elements, its residual and the norm's weights.  (With a branch for each of the
 // row's parts they came one behind the other.)  One row of 2880, 4 experts 8.4 -> 7.3 us, 33 rows 10.6 -> 8.4
 // (6.1 with two rows per workgroup, run_norm_router).
-template <int NB, bool NORM>
-__global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
-    const bf16_t *__restrict__ t, const bf16_t *__restrict__ wr, const float *__restrict__ br,
+template <int NB>   // 16-expert column blocks held per wave
+__global__ __launch_bounds__(ROUTER_WAVES * 64) void norm_router_kernel(
+    const bf16_t *__restrict__ wr, const float *__restrict__ br,
     float *__restrict__ logits, int B, int H, int E, int k, float *__restrict__ topk_w,
     int *__restrict__ topk_i, int rows_per_wg, RouterNorm nrm, RouterGroup grp) {
-  const int e0 = blockIdx.y * (NB * 16);   // first expert of the workgroup; it gates only if it has them all
   __shared__ float red[ROUTER_WAVES][16][NB * 16 + 1];
-  extern __shared__ __attribute__((aligned(16))) unsigned char t_rows_raw[];  // NORM: [rows_per_wg][H] bf16
+  extern __shared__ __attribute__((aligned(16))) unsigned char t_rows_raw[];  // [rows_per_wg][H] bf16
   // The wave's number has to be a scalar: matrix instructions do not look at the mask of active lanes, so a wave skips the
   // k-steps that are not its own only by a branch, and for a condition on a lane's value the compiler leaves the branch
   // out where masking looks cheaper (one matrix instruction under it, no wait: its products were added all the same).
@@ -316,7 +346,6 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
   const int r0 = blockIdx.x * rows_per_wg;
   const int arow = min(r0 + min(lane & 15, rows_per_wg - 1), B - 1);
   const int kq = (lane >> 4) * 8;
-  const bf16_t *ap = t + (size_t)arow * H + kq;
   constexpr int ROUTER_MAX_STEPS = router_steps(NB);
   const int ksteps = H / 32;
   // In two halves: while one is multiplied, the other's loads are on their way (2880 inputs, 64 experts 16.3 -> 13.9 us, a third
@@ -329,7 +358,7 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
       const int ks = min(ks0 + u * ROUTER_WAVES, ksteps - 1);
 #pragma unroll
       for (int nb = 0; nb < NB; nb++) {
-        int e = min(e0 + nb * 16 + (lane & 15), E - 1);
+        int e = min(nb * 16 + (lane & 15), E - 1);
         b[decltype(set)::value][u][nb] = *reinterpret_cast<const u32x4 *>(wr + (size_t)e * H + ks * 32 + kq);
       }
     }
@@ -341,19 +370,17 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
   constexpr int NJ = (NB + 1) / 2;
   float bias[NJ];
 #pragma unroll
-  for (int j = 0; j < NJ; j++) bias[j] = br ? br[min(e0 + sub + 32 * j, E - 1)] : 0.f;
+  for (int j = 0; j < NJ; j++) bias[j] = br ? br[min(sub + 32 * j, E - 1)] : 0.f;
   // the router's weights do not wait for the norm (more than 128 experts: no registers to hold them meanwhile).  Loads return
   // in order, so the bias is in front of them, and a wave without a k-step requests none: behind twelve steps' loads in each
   // of eight waves, of which H = 64 has work for two, 32 / 128 experts took 7.0 / 9.1 us instead of 3.1 / 3.7.
-  constexpr bool EARLY = !NORM || NB <= 8;
+  constexpr bool EARLY = NB <= 8;
   static_assert(EARLY || SETS == 1, "two sets are requested early");
   if (EARLY && wave < ksteps) load_b(wave, S0{});
   if (SETS == 2 && EARLY && wave + STRIDE < ksteps) load_b(wave + STRIDE, S1{});
-  if constexpr (NORM) {
-    bf16_t *t_rows = reinterpret_cast<bf16_t *>(t_rows_raw);
-    norm_rows<(NB < 8), false>(nrm, t_rows, r0, rows_per_wg, B, H, true, [] {});   // (W_EARLY where registers allow)
-    ap = t_rows + (size_t)(arow - r0) * H + kq;
-  }
+  bf16_t *t_rows = reinterpret_cast<bf16_t *>(t_rows_raw);
+  norm_rows<(NB < 8), false>(nrm, t_rows, r0, rows_per_wg, B, H, true, [] {});   // (W_EARLY where registers allow)
+  const bf16_t *ap = t_rows + (size_t)(arow - r0) * H + kq;
   f32x4 acc[NB];
 #pragma unroll
   for (int nb = 0; nb < NB; nb++) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -401,31 +428,110 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
 #pragma unroll
     for (int i = 0; i < 4; i++) red[wave][(lane >> 4) * 4 + i][nb * 16 + (lane & 15)] = acc[nb][i];
   __syncthreads();
-  // 32 lanes per token row: sum the partial products, add the bias, publish, gate
-  const bool live = row < rows_per_wg && r0 + row < B;
-  float v[NJ];
+  router_gate<NB>(red, bias, logits, r0, 0, row < rows_per_wg && r0 + row < B, br != nullptr, B, E, k, topk_w, topk_i, grp);
+}
+
+// The router: one workgroup = 16 token rows x all experts (or 16 of them, where they are shared out among workgroups); its 8
+// waves split the K loop (k-steps of 32, interleaved) and reduce through LDS; with topk_w it also gates its tokens.
+// The operands come through LDS.  In operand order a load takes 16 bytes of
+// 16 rows by every four lanes in a row, and a CU reads 36 KB a us that way; of whole rows 64 bytes a cycle (all CUs at work on what
+// their L2s hold: 110 KB a us).  So the workgroup's 16 rows and its experts' come in stages of 512 bytes a row, one k-step for each
+// wave, straight into LDS, and are taken from there.  More than 64 experts come in parts of a stage, so that three
+// buffers have room; 32 experts' three buffers leave room for a second workgroup (6000 tokens 13.2 -> 12.5).  Operands straight into registers in operand order -> this, 2880 inputs (us): 32 experts, 27 / 1024 / 4096 tokens 8.3 /
+// 8.9 / 10.4 -> 5.0 / 5.6 / 6.3, 64 16.0 / 16.7 / 18.2 -> 7.1 / 7.9 / 8.4, 128 27.2 / 26.0 / 27.5 -> 12.3 / 13.0 / 14.3; 2048 inputs and four
+// 4.1 / 4.5 / 6.5 -> 3.9 / 3.9 / 6.1.  Same bits.
+template <int NB>
+struct RouterStages {
+  static constexpr int PARTS = (NB + 3) / 4, BLOCKS = NB / PARTS;   // parts of a stage, 16-expert blocks of a part
+  static constexpr int ROWS = 16 + BLOCKS * 16, BYTES = ROWS * 512, LOADS = ROWS / 16;   // loads: per wave, two rows each
+  static constexpr int COUNT = NB == 1 ? 4 : 3;                       // buffers, all but one of them on their way
+  static constexpr int RED = ROUTER_WAVES * 16 * (NB * 16 + 1) * 4;   // the waves' sums, when the loop is over
+  static constexpr int SMEM = COUNT * BYTES > RED ? COUNT * BYTES : RED;
+  static_assert(SMEM + 1024 <= 160 * 1024, "LDS of a CU");
+};
+
+template <int N>
+__device__ __forceinline__ void router_wait() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+
+template <int NB>
+__global__ __launch_bounds__(ROUTER_WAVES * 64) void router_gemm_kernel(
+    const bf16_t *__restrict__ t, const bf16_t *__restrict__ wr, const float *__restrict__ br, float *__restrict__ logits, int B,
+    int H, int E, int k, float *__restrict__ topk_w, int *__restrict__ topk_i, int rows_per_wg, RouterGroup grp) {
+  const int e0 = blockIdx.y * (NB * 16);   // first expert of the workgroup; it gates only if it has them all
+  using S = RouterStages<NB>;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r0 = blockIdx.x * rows_per_wg, ksteps = H / 32, n_stages = (ksteps + ROUTER_WAVES - 1) / ROUTER_WAVES;
+  const int row = threadIdx.x >> 5, sub = threadIdx.x & 31;
+  constexpr int NJ = (NB + 1) / 2;
+  float bias[NJ];
 #pragma unroll
-  for (int j = 0; j < NJ; j++) {
-    const int col = sub + 32 * j, e = e0 + col;
-    float x = -INFINITY;
-    if (e < E && col < NB * 16) {
-      x = 0.f;
+  for (int j = 0; j < NJ; j++) bias[j] = br ? br[min(e0 + sub + 32 * j, E - 1)] : 0.f;
+  // Load x of the wave moves rows 16 x + 2 wave and the next of a buffer: token rows with x = 0 (those beyond the workgroup's
+  // repeat its last one), then experts'.  Position j of row r holds piece j ^ (r & 15), so that a fragment's lanes hit
+  // different banks.  (The compiler does not count these loads.)
+  const int pair = 2 * wave + (lane >> 5), piece = (lane & 31) ^ pair;
+  const uint32_t a_row = (uint32_t)min(min(pair, rows_per_wg - 1), B - 1 - r0) * (uint32_t)H * 2u;
+  uint32_t e_row[NB];
 #pragma unroll
-      for (int w = 0; w < ROUTER_WAVES; w++) x += red[w][row][col];
-      if (br) x += bias[j];
-      if (live) logits[(size_t)(r0 + row) * E + e] = x;
-    }
-    v[j] = x;
+  for (int nb = 0; nb < NB; nb++) e_row[nb] = (uint32_t)min(e0 + nb * 16 + pair, E - 1) * (uint32_t)H * 2u;
+  const unsigned lds_base =
+      __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)lds) + wave * 1024;
+  const bf16_t *a_src = t + (size_t)r0 * H;
+  auto request = [&](int st, auto part, int buf) {
+    constexpr int P = decltype(part)::value;
+    const uint32_t at = (uint32_t)st * 512u + (st * 256 + piece * 8 < H ? piece * 16 : 0);   // (beyond a row's end: nobody's)
+    const unsigned to = lds_base + buf * S::BYTES;
+    load_to_lds(to, a_row + at, a_src);
+#pragma unroll
+    for (int x = 0; x < S::BLOCKS; x++) load_to_lds(to + (x + 1) * 8192, e_row[P * S::BLOCKS + x] + at, wr);
+  };
+  f32x4 acc[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; nb++) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const unsigned char *frag = lds + (lane & 15) * 512 + (((wave * 4 + (lane >> 4)) ^ (lane & 15)) << 4);
+  // parts are numbered through: part u of the loop is part u % PARTS of stage u / PARTS
+  const int total = n_stages * S::PARTS;
+  static_for<0, S::COUNT - 1>([&](auto u) {
+    constexpr int U = decltype(u)::value;
+    if (U < total) request(U / S::PARTS, std::integral_constant<int, U % S::PARTS>{}, U);
+  });
+  int buf = 0, ahead = S::COUNT - 1;
+  for (int st = 0; st < n_stages; st++) {
+    static_for<0, S::PARTS>([&](auto part) {
+      constexpr int P = decltype(part)::value;
+      const int u = st * S::PARTS + P;
+      // part u has landed when no more than the COUNT - 2 behind it are on their way; behind the barrier it has for every
+      // wave, and nobody reads the buffer of the part before any more
+      if (u + S::COUNT - 1 <= total) router_wait<(S::COUNT - 2) * S::LOADS>();
+      else router_wait<0>();
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      constexpr int Q = P + S::COUNT - 1;
+      if (u + S::COUNT - 1 < total) request(st + Q / S::PARTS, std::integral_constant<int, Q % S::PARTS>{}, ahead);
+      if (st * ROUTER_WAVES + wave < ksteps) {
+        const unsigned char *f = frag + buf * S::BYTES;
+        const bf16x8 a = as_bf16x8(*reinterpret_cast<const u32x4 *>(f));
+#pragma unroll
+        for (int x = 0; x < S::BLOCKS; x++)
+          acc[P * S::BLOCKS + x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a, as_bf16x8(*reinterpret_cast<const u32x4 *>(f + (x + 1) * 8192)), acc[P * S::BLOCKS + x], 0, 0, 0);
+      }
+      buf = buf + 1 == S::COUNT ? 0 : buf + 1;
+      ahead = ahead + 1 == S::COUNT ? 0 : ahead + 1;
+    });
   }
-  if (topk_w != nullptr) {
-    const size_t o = (size_t)(live ? r0 + row : 0) * k;
-    __shared__ int ids[ROUTER_GROUP_PAIRS];
-    topk_softmax_group<NJ>(v, sub, E, k, live, topk_w + o, topk_i + o, grp.expert_offsets ? ids + row * k : nullptr);
-    if (grp.expert_offsets != nullptr) {   // one workgroup holds every token
-      __syncthreads();
-      if (wave == 0) group_by_one_wave(ids, B * k, E, reinterpret_cast<int *>(&red[0][0][0]), grp);
-    }
-  }
+  __syncthreads();   // the buffers have been read
+  typedef float Sums[16][NB * 16 + 1];
+  Sums *red = reinterpret_cast<Sums *>(lds);
+#pragma unroll
+  for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) red[wave][(lane >> 4) * 4 + i][nb * 16 + (lane & 15)] = acc[nb][i];
+  __syncthreads();
+  router_gate<NB>(red, bias, logits, r0, e0, row < rows_per_wg && r0 + row < B, br != nullptr, B, E, k, topk_w, topk_i, grp);
 }
 
 // The partial products that the waves of router_gemm_kernel add up, of at most 16 tokens: a workgroup is one of its waves over
@@ -747,11 +853,10 @@ static int router_col_blocks(int E) {
   return nb <= 1 ? 1 : nb <= 2 ? 2 : nb <= 4 ? 4 : nb <= 8 ? 8 : 16;
 }
 
-// Whether a workgroup takes 16 experts instead of all of them.  What one takes is its rounds of loads: 190 to 260 loads of
-// 16 rows x 64 bytes, which its CU returns at 36 KB a us, whatever of them is needed (one token, 128 experts of 1024 / 2048 /
-// 2880 / 4096 inputs 9.7 / 16.7 / 23.8 / 31.0 us; 32 experts of 512 to 2880 inputs 7.7, one round).  Sharing the experts out
-// saves loads and costs a second launch, which gates (up to 16 tokens: and groups).  All experts in one workgroup -> shared
-// out, MoE block with narrow experts (us):
+// Whether a workgroup takes 16 experts instead of all of them.  Sharing the experts out saves loads and costs a second launch,
+// which gates (up to 16 tokens: and groups).  The lines are where they were worth it while a workgroup's loads came in operand
+// order, in rounds of 190 to 260 at 36 KB a us; now that all experts in one workgroup take half of that time (router_gemm_kernel),
+// the two are closer.  Then, all experts in one workgroup -> shared out, MoE block with narrow experts (us):
 //   more than one round  2880 inputs, 64 experts, 1 / 512 tokens 29.9 / 80.2 -> 20.7 / 71.3, 128 39.0 / 104 -> 22.0 / 87.0, 33 experts,
 //                        17 / 512 tokens 39.0 / 86.0 -> 34.8 / 82.4; 1024 inputs, 256 experts, 512 tokens 62.6 -> 57.6
 //   one round            1024 inputs, 64 experts, 1 / 256 tokens 19.5 / 36.3 -> 17.2 / 34.3; but 48 experts, 256 tokens 36.9 -> 36.5,
@@ -802,6 +907,30 @@ int run_norm_router_parts(const float *x, const float *residual, const float *we
 
 // logits (+ optional gating of the same tokens), in one launch unless many experts are shared out (only with the gating of at
 // most 8 experts per token: logits alone come from one workgroup for all experts)
+template <int NB>
+static int launch_router(const bf16_t *t, const bf16_t *wr, const float *br, float *logits, int B, int H, int E, int k,
+                         float *topk_w, int *topk_i, int rows_per_wg, int shares, const RouterGroup &grp, hipStream_t s) {
+  constexpr int MAX_DEV = 64;
+  static std::mutex mu;
+  static bool raised[MAX_DEV];
+  int dev = 0;
+  GPTOSS_HIP(hipGetDevice(&dev));
+  GPTOSS_REQUIRE(dev >= 0 && dev < MAX_DEV, GPTOSS_ERR_STATE, "router: device ordinal %d outside 0..%d", dev, MAX_DEV - 1);
+  auto kern = router_gemm_kernel<NB>;
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (!raised[dev]) {
+      GPTOSS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     RouterStages<NB>::SMEM));
+      raised[dev] = true;
+    }
+  }
+  hipLaunchKernelGGL(kern, dim3(cdiv(B, rows_per_wg), shares), dim3(ROUTER_WAVES * 64), RouterStages<NB>::SMEM, s, t, wr, br, logits, B, H, E,
+                     k, topk_w, topk_i, rows_per_wg, grp);
+  GPTOSS_LAUNCH_CHECK("router_gemm_kernel");
+  return GPTOSS_OK;
+}
+
 int run_router(const void *t, const void *w_router, const float *b_router, float *logits, int B,
                int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group, float *parts) {
   // 16 token rows per workgroup fill the MFMA, but a thousand tokens are then only 64 workgroups;
@@ -811,10 +940,8 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
   const RouterGroup grp = group ? *group : RouterGroup{};
   const int rows_per_wg = grp.expert_offsets ? ROUTER_GROUP_TOKENS : router_rows_per_wg(B);
   GPTOSS_REQUIRE(!grp.expert_offsets || (topk_w && router_groups(B, k)), GPTOSS_ERR_DIM, "router: %d tokens are not grouped here", B);
-  dim3 grid(cdiv(B, rows_per_wg)), block(ROUTER_WAVES * 64);
   const bf16_t *tp = (const bf16_t *)t, *wp = (const bf16_t *)w_router;
   int nb = cdiv(E, 16);
-  const RouterNorm none{nullptr, nullptr, nullptr, nullptr};
   if (topk_w && k > 8) {   // more experts per token than the fused gating holds
     const int rc = run_router(t, w_router, b_router, logits, B, H, E, k, nullptr, nullptr, s);
     return rc != GPTOSS_OK ? rc : run_topk_softmax(logits, B, E, k, topk_w, topk_i, s);
@@ -840,9 +967,8 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
     const int rows = router_split_rows(B, E);
     {
       TraceScope ts("router_gemm", s);
-      router_gemm_kernel<1, false><<<dim3(cdiv(B, rows), nb), block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, nullptr,
-                                                                           nullptr, rows, none, RouterGroup{});
-      GPTOSS_LAUNCH_CHECK("router_gemm_kernel");
+      const int rc = launch_router<1>(tp, wp, b_router, logits, B, H, E, k, nullptr, nullptr, rows, nb, RouterGroup{}, s);
+      if (rc != GPTOSS_OK) return rc;
     }
     if (!grp.expert_offsets) return run_topk_softmax(logits, B, E, k, topk_w, topk_i, s);
     TraceScope ts("topk_group", s);
@@ -854,13 +980,11 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
     return GPTOSS_OK;
   }
   TraceScope ts(topk_w ? "router_gemm_topk" : "router_gemm", s);
-  if (nb <= 1) router_gemm_kernel<1, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none, grp);
-  else if (nb <= 2) router_gemm_kernel<2, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none, grp);
-  else if (nb <= 4) router_gemm_kernel<4, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none, grp);
-  else if (nb <= 8) router_gemm_kernel<8, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none, grp);
-  else router_gemm_kernel<16, false><<<grid, block, 0, s>>>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, none, grp);
-  GPTOSS_LAUNCH_CHECK("router_gemm_kernel");
-  return GPTOSS_OK;
+  if (nb <= 1) return launch_router<1>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);
+  if (nb <= 2) return launch_router<2>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);
+  if (nb <= 4) return launch_router<4>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);
+  if (nb <= 8) return launch_router<8>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);
+  return launch_router<16>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);
 }
 
 
@@ -875,7 +999,7 @@ static int launch_norm_router(const RouterNorm &nrm, const bf16_t *wp, const flo
   int dev = 0;
   GPTOSS_HIP(hipGetDevice(&dev));
   GPTOSS_REQUIRE(dev >= 0 && dev < MAX_DEV, GPTOSS_ERR_STATE, "router: device ordinal %d outside 0..%d", dev, MAX_DEV - 1);
-  auto kern = router_gemm_kernel<NB, true>;
+  auto kern = norm_router_kernel<NB>;
   {
     std::lock_guard<std::mutex> lock(mu);
     if (raised[dev] < dyn) {
@@ -885,9 +1009,9 @@ static int launch_norm_router(const RouterNorm &nrm, const bf16_t *wp, const flo
     }
   }
   TraceScope ts("norm_router_gemm_topk", s);
-  hipLaunchKernelGGL(kern, dim3(cdiv(B, rows_per_wg)), dim3(ROUTER_WAVES * 64), dyn, s, nrm.t_out, wp, b_router, logits, B,
-                     H, E, k, topk_w, topk_i, rows_per_wg, nrm, grp);
-  GPTOSS_LAUNCH_CHECK("router_gemm_kernel (with norm)");
+  hipLaunchKernelGGL(kern, dim3(cdiv(B, rows_per_wg)), dim3(ROUTER_WAVES * 64), dyn, s, wp, b_router, logits, B, H,
+                     E, k, topk_w, topk_i, rows_per_wg, nrm, grp);
+  GPTOSS_LAUNCH_CHECK("norm_router_kernel");
   return GPTOSS_OK;
 }
 

@@ -95,6 +95,19 @@ def test_router_gemm(ops, B, H, E):
     assert np.abs(got - want).max() <= 1e-4 * max(1.0, np.abs(want).max())
 
 
+@pytest.mark.parametrize("E", [1, 17, 33, 65, 129, 255])    # blocks of 16 experts, whole and not, in one to four parts of a stage
+@pytest.mark.parametrize("H", [32, 224, 256, 288, 768])     # stages of 256 inputs: a piece of one, one, one and a piece, three
+def test_router_stages(ops, E, H):
+    g = torch.Generator(device="cuda").manual_seed(E + H)
+    n = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    t, w, b = n(21, H), n(E, H), n(E).float()
+    want = t.double() @ w.double().T + b.double()
+    for tokens in (1, 5, 16, 21):
+        got = ops.router_gemm(t[:tokens].contiguous(), w, b)
+        # as in test_router_rows_are_the_same_in_groups_of_any_size
+        assert bool(((got.double() - want[:tokens]).abs() <= 2.0 ** -24 * (H / 8 + 8) * 8 * H ** 0.5).all()), tokens
+
+
 # ---------------------------------------------------------------- weight packing
 @pytest.mark.parametrize("E", [32, 64, 128, 256])           # two halves of a wave's k-steps, more than 128 experts one
 @pytest.mark.parametrize("H", [32, 320, 1792, 2048, 2080, 3104])   # one k-step in all; around a wave's 7 or 8, and 12
