@@ -719,7 +719,8 @@ __device__ __forceinline__ void attn_few_chunk(const AttnParams &p, const RopeIn
     for (int tb = 0; tb < 4; tb++)
 #pragma unroll
       for (int s = 0; s < KS; s++)
-        kreg[u][tb][s] = fetch(block_at(wave + 4 * u) + (tb * 16 + n) * D + c * KS * 8 + s * 8);
+        kreg[u][tb][s] = fetch(block_at(wave + 4 * u) + ((tb * KS + s) * 64 + lane) * 8);   // as it lies
+
   }
 #pragma unroll
   for (int j = 0; j < NBLK; j++) {
@@ -728,6 +729,12 @@ __device__ __forceinline__ void attn_few_chunk(const AttnParams &p, const RopeIn
     for (int grp = 0; grp < 2; grp++)
       vreg[j][grp] = fetch(block_at(j) + KV_BLOCK * D + (grp * DB + db) * 512 + lane * 8);
   }
+  // In the wave's part of the weights' LDS, which nobody uses before the barrier below.  Keys in operand order from memory -> this
+  // (us): 17 sequences of 625 to 4999 positions 27.0 -> 25.4, 200 of 38 to 300 21.3 -> 19.4, 45 of 48 to 383 10.4 -> 9.9.
+  static_assert(4 * KV_BLOCK * D * 2 <= (int)sizeof lds_p, "a block of K per wave");
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+    if (wave + 4 * u < nb) keys_to_operands<D>(kreg[u], reinterpret_cast<unsigned char *>(lds_p) + wave * (KV_BLOCK * D * 2));
   if constexpr (ROPE) {
     auto rotate = [&](f32x4 (&x)[2 * KS]) {
 #pragma unroll
@@ -1070,17 +1077,14 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
   const unsigned char *plane =
       reinterpret_cast<const unsigned char *>(p.kv + kv_block_off(cache_seq, g, p.n_kv, p.cap, D, 0));
   // The workgroup's copy of a block goes from memory straight into LDS, in pieces of 16 bytes: thread t's load i lands at
-  // piece i * 512 + t.  Position j of K row r is to hold chunk j ^ swz(r), the chunk that the lane fetches: LDS serves lanes 0-3,
-  // 12-15 and 20-27 of a fragment read (16 rows, one chunk per quarter) together, then 4-11, 16-19 and 28-31, and the upper half
-  // alike, and these are to hit 16 different 16-byte slots modulo 256 bytes.  (A third of the cycles of all reads went into
-  // conflicts where 16 lanes in a row did so.)  (Through registers, the loop's eight of them and the store's addresses do not
+  // piece i * 512 + t.  Position j of K row r is to hold chunk j ^ kv_swizzle(r), the chunk that the lane fetches.  (A third of the
+  // cycles of all reads went into conflicts where 16 lanes in a row hit different slots.)  (Through registers, the loop's eight of them and the store's addresses do not
   // fit the 128 of two workgroups per CU beside the rest.)
-  auto swz = [](int r) { return D == 64 ? ((r >> 1) & 7) ^ (r & 4) : ((r >> 2) & 3) ^ ((r >> 1) & 2); };
   uint32_t src_off[PASSES];
 #pragma unroll
   for (int i = 0; i < PASSES; i++) {
     const int piece = i * TILE_WAVES * 64 + tid, r = piece / ROW_CHUNKS, j = piece % ROW_CHUNKS;
-    src_off[i] = (piece * 16 < K_BYTES ? r * ROW_CHUNKS + (j ^ swz(r)) : piece) * 16;
+    src_off[i] = (piece * 16 < K_BYTES ? r * ROW_CHUNKS + (j ^ kv_swizzle<D>(r)) : piece) * 16;
   }
   const unsigned lds_base =
       __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)&lds[0][0]);
@@ -1119,7 +1123,7 @@ __global__ __launch_bounds__(TILE_WAVES * 64, 4) void attn_prefill_tile_kernel(A
       const int r = tb * 16 + n;
 #pragma unroll
       for (int s = 0; s < KS; s++) {
-        const bf16x8 kf = as_bf16x8(*reinterpret_cast<const u32x4 *>(kb + r * (D * 2) + (((c * KS + s) ^ swz(r)) << 4)));
+        const bf16x8 kf = as_bf16x8(*reinterpret_cast<const u32x4 *>(kb + r * (D * 2) + (((c * KS + s) ^ kv_swizzle<D>(r)) << 4)));
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qh[s], acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, ql[s], acc, 0, 0, 0);
       }

@@ -188,4 +188,34 @@ __device__ __forceinline__ int kv_v_elem(int slot, int d, int D) {
   return KV_BLOCK * D + (((slot & 63) >> 5) * (D >> 4) + (d >> 4)) * 512 + lane * 8 + j;
 }
 
+// K rows of a block in LDS: piece j (16 bytes) of row r is at j ^ kv_swizzle(r).  LDS serves lanes 0-3, 12-15 and 20-27 of a fragment
+// read (16 rows, one piece per quarter) together, then 4-11, 16-19 and 28-31, and the upper half alike, and these hit 16
+// different 16-byte slots modulo 256 bytes.
+template <int D>
+__device__ __forceinline__ int kv_swizzle(int r) {
+  static_assert(D == 32 || D == 64);
+  return D == 64 ? ((r >> 1) & 7) ^ (r & 4) : ((r >> 2) & 3) ^ ((r >> 1) & 2);
+}
+
+// K of a block as it lies, load i / KS, i % KS of a wave its i-th KB, into operands: lane (n, c) of [tb][s] has piece c KS + s of
+// row 16 tb + n.  own: KV_BLOCK * D * 2 bytes of LDS that the wave has to itself.  (In operand order a load takes 16 bytes of each of 16
+// rows, and a CU reads 36 KB a us that way, of whole lines 110.)
+template <int D>
+__device__ __forceinline__ void keys_to_operands(u32x4 (&k)[4][D / 32], unsigned char *own) {
+  constexpr int KS = D / 32, PIECES = D / 8;
+  const int lane = lane_id(), n = lane & 15, c = lane >> 4;
+#pragma unroll
+  for (int i = 0; i < 4 * KS; i++) {
+    const int r = i * (64 / PIECES) + lane / PIECES, j = lane % PIECES;
+    *reinterpret_cast<u32x4 *>(own + r * (D * 2) + ((j ^ kv_swizzle<D>(r)) << 4)) = k[i / KS][i % KS];
+  }
+#pragma unroll
+  for (int tb = 0; tb < 4; tb++)
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+      const int r = tb * 16 + n;
+      k[tb][s] = *reinterpret_cast<const u32x4 *>(own + r * (D * 2) + (((c * KS + s) ^ kv_swizzle<D>(r)) << 4));
+    }
+}
+
 }  // namespace gptoss

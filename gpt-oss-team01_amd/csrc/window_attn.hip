@@ -447,7 +447,9 @@ __device__ __forceinline__ void store_column(bf16_t *dst, int vdim, int db_n, in
 template <int DMAX, bool EXACT, bool NORM = false>
 __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttn a, const RowSeg *__restrict__ singles) {
   constexpr int KS = DMAX / 32, DB = DMAX / 16;
+  constexpr bool LINES = EXACT && DMAX == 64;   // keys in whole lines (keys_to_operands)
   __shared__ float so[3][DMAX][16], sm[3][16], sl[3][16];
+  __shared__ __attribute__((aligned(16))) unsigned char keys[LINES ? 4 : 1][LINES ? KV_BLOCK * DMAX * 2 : 16];
   const RowSeg seg = singles[blockIdx.x];
   const int g = blockIdx.y, per = a.heads / a.kv_heads;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -471,11 +473,11 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttn a, const 
   if constexpr (EXACT) {
     u32x4 kr[4][KS], vr[2][DB];
     auto load_k = [&](int at) {
-      const bf16_t *x = plane + (size_t)at * block + k_lane;
+      const bf16_t *x = plane + (size_t)at * block + (LINES ? (size_t)lane * 8 : k_lane);
 #pragma unroll
       for (int tb = 0; tb < 4; tb++)
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) kr[tb][ks] = fetch(x + tb * 16 * DMAX + ks * 8);
+        for (int ks = 0; ks < KS; ks++) kr[tb][ks] = fetch(x + (LINES ? (tb * KS + ks) * 512 : tb * 16 * DMAX + ks * 8));
     };
     auto load_v = [&](int at) {
       const bf16_t *x = plane + (size_t)at * block + v_lane;
@@ -494,6 +496,7 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttn a, const 
     while (b <= b_last) {
       const int next = b + 4 <= b_last ? (rb + 4) % ring : rb;   // past the end: this block again, unused
       f32x4 s[4];
+      if constexpr (LINES) keys_to_operands<DMAX>(kr, keys[wave]);
       block_scores<KS>(q, KS, s, [&](int tb, int ks) { return as_bf16x8(kr[tb][ks]); });
       load_k(next);
       block_output<DB>(s, DB, b << 6, lo, hi, c, m, l, o, [&](int kg, int db) { return as_bf16x8(vr[kg][db]); });
@@ -624,9 +627,6 @@ __global__ __launch_bounds__(256, DMAX > 128 ? 1 : 2) void window_tile_kernel(Wi
 // heads, window 512: 139 -> 93 us.
 constexpr int WTILE_WAVES = 8;
 constexpr float WRAISE = 4.f;
-// K rows in LDS: position j of row r holds chunk j ^ window_swizzle(r) of 16 bytes, so that the lanes that LDS serves together
-// (0-3, 12-15 and 20-27 of a fragment's read, then the others) hit different banks
-__device__ __forceinline__ int window_swizzle(int r) { return ((r >> 1) & 7) ^ (r & 4); }
 
 template <bool NORM>
 __global__ __launch_bounds__(WTILE_WAVES * 64, 4) void window_tile64_kernel(WindowAttn a, const RowSeg *__restrict__ tiles, int n_tiles) {
@@ -643,7 +643,7 @@ __global__ __launch_bounds__(WTILE_WAVES * 64, 4) void window_tile64_kernel(Wind
   const int n = lane & 15, c = lane >> 4;
   const int ring = a.cap >> 6, queries = rows * per;
   const unsigned char *plane = reinterpret_cast<const unsigned char *>(a.kv) + (size_t)(slot * a.kv_heads + g) * ring * BLOCK_BYTES;
-  const uint32_t k_off = ((tid & ~7) | ((tid & 7) ^ window_swizzle(tid >> 3))) * 16, v_off = K_BYTES + tid * 16;
+  const uint32_t k_off = ((tid & ~7) | ((tid & 7) ^ kv_swizzle<64>(tid >> 3))) * 16, v_off = K_BYTES + tid * 16;
   const unsigned lds_base =
       __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)&lds[0][0]) + wave * 1024;
   auto request = [&](int rb, int buf) {
@@ -690,7 +690,7 @@ __global__ __launch_bounds__(WTILE_WAVES * 64, 4) void window_tile64_kernel(Wind
       f32x4 s[4];
       block_scores<KS>(q, KS, s, [&](int tb, int ks) {
         const int r = tb * 16 + n;
-        return as_bf16x8(*reinterpret_cast<const u32x4 *>(kb + r * (D * 2) + (((c * KS + ks) ^ window_swizzle(r)) << 4)));
+        return as_bf16x8(*reinterpret_cast<const u32x4 *>(kb + r * (D * 2) + (((c * KS + ks) ^ kv_swizzle<64>(r)) << 4)));
       });
       if (edge) {
         const int s0 = first + c * 4 - lo;
