@@ -909,9 +909,7 @@ __global__ __launch_bounds__(256, 1) void attn_few_rope_kernel(AttnParams p, Rop
 // 22.7 -> 18.9.  Beyond that a wave per item fills the chip as well and follows HBM better: 5 of 8000 (640 items) 29.8 -> 29.7,
 // 16 of 3000 (768) 30.5 -> 32.6, 8 of 8000 (1024) 33.4 -> 37.5, 48 of 4000 (3072) 74.5 -> 85.1, 96 of 300 20.2 -> 23.2, and 1000
 // rows of a prompt over 8 kv heads 141 -> 196.  (Rows of very different length are another matter: 63 of 500 to 4000 79 -> 70.
-// The host does not know the lengths.)  The 256 date from when this kernel requested eight blocks whatever a row has; since it
-// requests the row's own, 512 would do for short rows as well: 40 of 100 (320 items) 9.1 -> 7.2, 63 of 40 / 255 (504) 7.2 / 13.5 ->
-// 6.3 / 9.9, with heads of 32 values 63 of 40 / 100 / 200 5.1 / 6.3 / 8.2 -> 5.5 / 6.1 / 7.7.
+// The host does not know the lengths.)  With heads of 64 what is beyond these lines goes by attn_many.
 static bool attn_few(long long pairs, int span, int head_dim) {
   const long long items = pairs * ((span + ATT_CHUNK - 1) / ATT_CHUNK);
   return items <= (span * head_dim < 256 * 64 ? 256 : head_dim == 32 ? 384 : 512);
@@ -929,17 +927,19 @@ struct AttnPlan {
 // of it, a wave per item -> workgroup per item (us):
 //   chunks merged by a kernel behind   17 sequences of 5000 39.3 / 43.4 -> 26.7 / 38.4, 40 of 1000 23.2 / 24.7 -> 20.3 / 24.0, 63 of 4000
 //     76.0 / 94.8 -> 59.1 / 92.7, 32 of 32000 315 / 405 -> 262 / 393; the worst 30 of 4000 40.6 / 46.8 -> 32.5 / 48.5.  Always.
-//   rows of one chunk   80 of 300 15.2 / 16.0 -> 12.6 / 14.8, 150 of 257 21.7 / 27.8 -> 16.8 / 22.2, 255 of 448 25 / 30 -> 23 / 30;
-//     100 of 400 19.1 / 20.9 -> 16.4 / 22.4, 512 of 300 47.5 / 57.3 -> 45.7 / 59.9, 256 of 128 15.8 / 16.1 -> 18.8 / 18.3.
-//     From 256 positions on, up to 2560 items, and not where the host knows that all rows are of one length.
+//   rows of one chunk   200 of 200 20.7 / 24.8 -> 16.8 / 22.2, 100 of 256 13.5 / 13.7 -> 11.8 / 13.3, 400 of 448 57.2 / 70.7 -> 40.8 /
+//     61.3, 512 of 200 36.1 / 47.8 -> 33.6 / 46.3, of 448 62.6 / 75.7 -> 51.5 / 77.2; short ones 70 of 64 7.1 / 6.7 -> 6.9 / 5.9, of 128
+//     9.2 / 8.8 -> 8.0 / 7.4, but 100 of 64 7.5 / 7.1 -> 9.1 / 7.6, 256 of 128 15.7 / 16.3 -> 17.8 / 17.1, 256 of 2000 with a window of 128
+//     21.3 / 20.9 -> 23.2 / 23.1.  From 192 positions on up to 4096 items, shorter ones up to 640.
 //   rows of one chunk in front of the workgroup-per-row kernel   64 of 1000 35.8 / 27.9 -> 27.2 / 27.4, 98 of 736 34.8 / 34.5 ->
-//     29.0 / 34.4, 256 of 1000 74.4 / 85.7 -> 61.0 / 85.7, 512 of 1000 124.6 / 166.1 -> 112.2 / 167.4; of 1024 of 600, where
-//     8192 workgroups may have nothing to do, 162.1 / 214.9 -> 149.8 / 218.5.  Up to 4096 items.
+//     29.0 / 34.4, 256 of 1000 74.4 / 85.7 -> 61.0 / 85.7, 600 of 1000 146.4 / 194.4 -> 128.0 / 195.4; of 1024 of 600, where
+//     8192 workgroups may have nothing to do, 160.4 / 214.2 -> 146.3 / 217.3.  Up to 4096 items, 8192 where the host does not know that
+//     all rows are of one length.
 // (Rows of a prompt read the same blocks: those stay with a wave per item.)
 static bool attn_many(long long items, const AttnPlan &pl, int span, int head_dim, bool one_length) {
   if (head_dim != 64) return false;
-  if (pl.wide) return items <= 4096;
-  return pl.max_chunks > 1 ? items < (1ll << 31) : span >= 256 && items <= 2560 && !one_length;
+  if (pl.wide) return items <= (one_length ? 4096 : 8192);
+  return pl.max_chunks > 1 ? items < (1ll << 31) : items <= (span >= 192 ? 4096 : 640);
 }
 
 // Merge the chunk partials of one (sequence, q head) with the sink logit.  One thread owns four

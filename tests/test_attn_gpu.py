@@ -336,11 +336,12 @@ def test_few_rows_of_several_chunks_have_the_bits_of_the_same_rows_among_more(op
         assert torch.equal(out[rows].view(torch.int16), out[B][:rows].view(torch.int16)), rows
 
 
-# rows of one chunk: up to 320 sequences a workgroup each, 330 a wave; of one chunk and of several: up to 512 sequences a
-# workgroup for each of one chunk as well, in front of the kernel that takes the others, 520 a wave
+# rows of one chunk: up to 512 sequences a workgroup each, 520 a wave, short ones up to 80 and 90; of one chunk and of several: up to
+# 1024 sequences a workgroup for each of one chunk as well, in front of the kernel that takes the others, 1030 a wave
 @pytest.mark.parametrize("sequences,longest,cap,window", [
-    ((330, 65, 200, 320), 256, 256, 0), ((330, 65, 200, 320), 512, 512, 0), ((330, 65, 320), 512, 512, 300),
-    ((520, 64, 65, 300, 512), 700, 704, 0), ((520, 64, 512), 900, 640, 576)])
+    ((90, 33, 64, 65, 80), 128, 128, 0), ((90, 64, 80), 400, 512, 100), ((520, 65, 200, 512), 192, 192, 0),
+    ((520, 65, 200, 512), 512, 512, 0), ((520, 65, 512), 512, 512, 300),
+    ((1030, 64, 65, 300, 1024), 700, 704, 0), ((1030, 64, 1024), 900, 640, 576)])
 def test_rows_have_the_same_bits_a_workgroup_or_a_wave_each(ops, sequences, longest, cap, window):
     B, n_q, n_kv, D = sequences[0], 64, 8, 64
     g = torch.Generator(device="cuda").manual_seed(longest + window)
