@@ -83,11 +83,16 @@ __device__ __forceinline__ const_as<T> constant_ptr(const T *q) {
   return (const_as<T>)(q);
 }
 
-// 16 bytes per lane, from sbase + voff to LDS address lds + 16 * lane.  The compiler does not count these loads: whoever
-// reads what they bring waits for the vector-memory counter by itself first.
+// 16 bytes per lane, from sbase + voff (an unsigned offset) to LDS address lds + 16 * lane.  The compiler does not count these
+// loads: whoever reads what they bring waits for the vector-memory counter by itself first.
 __device__ __forceinline__ void load_to_lds(unsigned lds, uint32_t voff, const void *sbase) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
                "v"(voff), "s"(sbase)
+               : "memory");
+}
+// The same from an address of each lane's own.
+__device__ __forceinline__ void load_to_lds(unsigned lds, const void *from) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(from)
                : "memory");
 }
 

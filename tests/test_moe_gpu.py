@@ -108,6 +108,22 @@ def test_router_stages(ops, E, H):
         assert bool(((got.double() - want[:tokens]).abs() <= 2.0 ** -24 * (H / 8 + 8) * 8 * H ** 0.5).all()), tokens
 
 
+# the last experts' rows, and the last tokens' too, begin 4 GiB and more behind the first one
+@pytest.mark.parametrize("B,H,E", [(3, 8421536, 256), (4, 715827904, 4)])
+def test_router_matrices_of_more_than_four_gib(ops, B, H, E):
+    g = torch.Generator(device="cuda").manual_seed(E)
+    t = torch.zeros(B, H, dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros(E, H, dtype=torch.bfloat16, device="cuda")
+    at = torch.tensor([0, 8, 255, 256, 1000, H // 2, H - 300, H - 33, H - 1], device="cuda")
+    t[:, at] = torch.randint(-3, 4, (B, len(at)), generator=g, device="cuda").bfloat16()
+    w[:, at] = torch.randint(-9, 10, (E, len(at)), generator=g, device="cuda").bfloat16()
+    b = torch.arange(E, device="cuda").float()
+    assert (E - 1) * H * 2 >= 2 ** 32 and H % 32 == 0
+    got = ops.router_gemm(t, w, b)
+    want = (t[:, at].float() @ w[:, at].float().T) + b      # whole numbers, exact in any order
+    assert torch.equal(got, want)
+
+
 # ---------------------------------------------------------------- weight packing
 @pytest.mark.parametrize("E", [32, 64, 128, 256])           # two halves of a wave's k-steps, more than 128 experts one
 @pytest.mark.parametrize("H", [32, 320, 1792, 2048, 2080, 3104])   # one k-step in all; around a wave's 7 or 8, and 12
