@@ -377,7 +377,8 @@ __device__ __forceinline__ void block_output(f32x4 (&s)[4], int db_n, int pos0, 
   for (int tb = 0; tb < 4; tb++)
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      // a masked slot keeps weight 0 also while nothing of the column has been seen (m == WNEG)
+      // a masked slot keeps weight 0 also while nothing of the column has been seen (m == WNEG), and so does a score that is
+      // no number: a key that has overflowed is left out, in a stretch as in a step
       s[tb][e] = s[tb][e] > 0.5f * WNEG ? __builtin_amdgcn_exp2f(s[tb][e] - m_new) : 0.f;
       sum += s[tb][e];
     }
@@ -717,11 +718,21 @@ __global__ __launch_bounds__(WTILE_WAVES * 64, 4) void window_tile64_kernel(Wind
       float sum = 0.f;
 #pragma unroll
       for (int kg = 0; kg < 2; kg++) {
+        const float before = sum;
         float x[8];
 #pragma unroll
         for (int e = 0; e < 8; e++) {
           x[e] = __builtin_amdgcn_exp2f(s[2 * kg + (e >> 2)][e & 3] - m);
           sum += x[e];
+        }
+        if (__ballot(sum != sum) != 0) {   // a score that is no number has no weight (block_output), which the sum shows
+          sum = before;
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            const float score = s[2 * kg + (e >> 2)][e & 3];
+            x[e] = score != score ? 0.f : x[e];
+            sum += x[e];
+          }
         }
         bf16x8 hi8, lo8;
         split8(x, hi8, lo8);

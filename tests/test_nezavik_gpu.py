@@ -303,6 +303,24 @@ def test_windows_over_heads_of_64(open_model, heads, kv, dim, vdim, window, scal
     check_model(e, 1, cfg, w, tok, False, [130, 1, 62, 1, 1, 200, 65])
 
 
+@pytest.mark.parametrize("heads,kv,dim,vdim,window,scale", [(6, 2, 64, 64, 90, 0.125), (8, 1, 40, 64, 128, 0.2), (4, 2, 96, 64, 70, 0.1)])
+def test_a_key_that_is_no_number_has_no_weight(open_model, heads, kv, dim, vdim, window, scale):
+    """Some tokens' keys overflow and are normed to NaN, their queries and values are finite: in stretches and token by token
+    alike they are left out, and a row that sees no other key is none."""
+    cfg = nm.config([nm.parallel(heads=heads, kv=kv, dim=dim, vdim=vdim, window=window, scale=scale, ff=None)])
+    w = nm.weights(cfg, 78)
+    tok = nm.tokens(cfg, 300, 7)
+    bad = tok[[40, 41, 130, 210]]
+    w["embed"][:, 5] = w["pos"][:, 5] = 0
+    w["embed"][bad, 5] = 60.0
+    w["l0.mix.left.k"][:, 5] = 3e38
+    e = open_model(cfg, w, False, max_batch=2)
+    whole, single = feed(e, 0, tok), feed(e, 1, tok, [1])
+    seen = np.array([any(t not in bad for t in tok[max(0, i - window + 1):i + 1]) for i in range(len(tok))])
+    assert seen.sum() > 250 and np.isnan(whole[~seen]).all() and np.isnan(single[~seen]).all()
+    check(whole[seen], single[seen].astype(np.float64), False)
+
+
 @BOTH
 def test_wide_rows_and_passes_of_thousands_of_rows(open_model, precise):
     """Sizes at which the products cut their sum over K into parts (few rows, many inputs), and a pass of thousands of rows, of
