@@ -895,7 +895,7 @@ static int router_split_rows(int B, int E) {
 
 int run_router_parts(const void *t, const void *w_router, float *parts, int B, int H, int E, hipStream_t s) {
   GPTOSS_REQUIRE(B >= 1 && B <= ROUTER_GROUP_TOKENS, GPTOSS_ERR_DIM, "router: no partial products of %d tokens", B);
-  TraceScope ts(router_splits(B, H, E) ? "router_gemm" : "router_gemm_topk", s);   // (the second with the gating in another kernel than its own)
+  TraceScope ts("router_parts", s);
   router_parts_kernel<false><<<dim3(ROUTER_WAVES, cdiv(E, 16)), 64, 0, s>>>((const bf16_t *)t, (const bf16_t *)w_router, parts, B, H, E, RouterNorm{});
   GPTOSS_LAUNCH_CHECK("router_parts_kernel");
   return GPTOSS_OK;
@@ -910,7 +910,7 @@ int run_norm_router_parts(const float *x, const float *residual, const float *we
                           float *parts, int B, int H, int E, hipStream_t s) {
   GPTOSS_REQUIRE(norm_router_parts_apply(B, H, x, residual, weight, t_out), GPTOSS_ERR_DIM,
                  "norm + router: no partial products of this form (B=%d H=%d)", B, H);
-  TraceScope ts("norm_router_gemm", s);
+  TraceScope ts("norm_router_parts", s);
   const RouterNorm nrm{const_cast<float *>(x), residual, weight, (bf16_t *)t_out};
   router_parts_kernel<true><<<dim3(ROUTER_WAVES, cdiv(E, 16)), B == 1 ? 256 : 512, (size_t)B * H * 2, s>>>(
       nrm.t_out, (const bf16_t *)w_router, parts, B, H, E, nrm);

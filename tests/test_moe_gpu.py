@@ -466,12 +466,15 @@ def test_experts_shared_out_among_workgroups_score_and_gate_the_same(ops, E, H):
 
 
 # up to 64 experts a round of loads is 1792 inputs, up to 128 1024, beyond 512; more than that: shared out up to 512 tokens,
-# less: 256 inputs and 49 experts or more, up to 256 tokens
-@pytest.mark.parametrize("H,E,tokens,shared", [
-    (4096, 32, 1, False), (1856, 33, 1, True), (1792, 33, 1, False), (1792, 48, 16, False), (1792, 49, 16, True), (1088, 128, 257, True),
-    (1024, 128, 257, False), (1024, 65, 256, True), (576, 129, 512, True), (576, 129, 513, False), (512, 256, 257, False),
-    (512, 256, 256, True), (256, 64, 17, True), (192, 256, 17, False), (64, 256, 1, False)])
-def test_which_calls_share_their_experts_out(ops, H, E, tokens, shared):
+# less: 256 inputs and 49 experts or more, up to 256 tokens.  Up to 16 tokens: partial products, unless 8 E floats are more
+# than k H, or three to seven tokens have fewer than 16 experts
+@pytest.mark.parametrize("H,E,tokens,router", [
+    (4096, 32, 1, "parts"), (4096, 32, 17, "one"), (1856, 33, 1, "parts"), (1856, 33, 17, "shared"), (1792, 33, 17, "one"),
+    (1792, 48, 16, "parts"), (1792, 48, 17, "one"), (1792, 49, 16, "parts"), (1792, 49, 17, "shared"), (1088, 128, 257, "shared"),
+    (1024, 128, 257, "one"), (1024, 65, 256, "shared"), (576, 129, 512, "shared"), (576, 129, 513, "one"), (512, 256, 257, "one"),
+    (512, 256, 256, "shared"), (512, 256, 16, "parts"), (448, 256, 16, "shared"), (256, 64, 17, "shared"), (192, 256, 17, "one"),
+    (64, 256, 1, "one"), (256, 15, 2, "parts"), (256, 15, 7, "one"), (256, 15, 8, "parts"), (256, 16, 5, "parts")])
+def test_which_calls_share_their_experts_out(ops, H, E, tokens, router):
     g = torch.Generator(device="cuda").manual_seed(H)
     n = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
     layer = ops.MoeLayer(n(E, H), n(E).float(), n(E, 128, H), n(E, 128).float(), n(E, H, 64), n(E, H).float(), top_k=4, max_tokens=tokens)
@@ -479,7 +482,33 @@ def test_which_calls_share_their_experts_out(ops, H, E, tokens, shared):
     with ops.KernelTrace(16) as trace:
         layer.forward(t)
     launches = [name for name, _ in trace.results()]
-    assert ("router_gemm" in launches) == shared and ("router_gemm_topk" in launches) != shared
+    name = {"parts": "router_parts", "one": "router_gemm_topk", "shared": "router_gemm"}
+    assert [x for x in launches if x.startswith("router")] == [name[router]]
+
+
+@pytest.mark.parametrize("E,H", [(49, 256), (64, 320), (65, 256), (128, 960), (129, 512), (256, 1984)])
+def test_a_few_tokens_without_room_for_partial_products(ops, E, H):
+    """One expert per token: 8 E floats are more than its row of the second product's output.  The experts are shared out and one
+    workgroup gates and groups the tokens, as larger batches do in other kernels, to the bit."""
+    g = torch.Generator(device="cuda").manual_seed(E + H)
+    n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    layer = ops.MoeLayer(n(E, H, std=H ** -0.5), n(E).float(), n(E, 128, H, std=0.05), n(E, 128).float(), n(E, H, 64), n(E, H).float(),
+                         top_k=1, max_tokens=600)
+    t = n(600, H)
+    out = layer.forward(t).clone()
+    want = [v.clone() for v in layer.routing_views()[:3]]
+    for tokens in (1, 2, 3, 8, 15, 16):
+        part = t[:tokens].contiguous()
+        with ops.KernelTrace(16) as trace:
+            got = layer.forward(part)
+        launches = [name for name, _ in trace.results()]
+        assert "router_gemm" in launches and "topk_group" in launches
+        have = layer.routing_views()
+        for a, b in zip(have, want):
+            assert torch.equal(a, b[:tokens]), tokens
+        for a, b in zip(have[3:], ops.moe_route(ops.router_gemm(part, layer.w_router, layer.b_router), 1)[2:5]):
+            assert torch.equal(a, b), tokens
+        assert torch.equal(got, out[:tokens]), tokens
 
 
 # up to two tokens are gated by the workgroups of the first product, up to four with 16 to 32 experts (of 1280 inputs), up to 128
