@@ -906,10 +906,9 @@ __global__ __launch_bounds__(256, 1) void attn_few_rope_kernel(AttnParams p, Rop
 // The launches that take it: where every row is as long as the longest may be, up to 512 (row, kv head, chunk) items, two
 // per CU; 384 with heads of 32 values; 256 of rows that cannot fill half a chunk.  64 heads of 64 on 8 kv heads, full rows, caches
 // cold, a wave per item -> this kernel (us): 4 of 8000 positions (512 items) 29.0 -> 25.4, 32 of 1000 29.6 -> 25.4, 63 of 448
-// 22.7 -> 18.9.  Beyond that a wave per item fills the chip as well and follows HBM better: 5 of 8000 (640 items) 29.8 -> 29.7,
-// 16 of 3000 (768) 30.5 -> 32.6, 8 of 8000 (1024) 33.4 -> 37.5, 48 of 4000 (3072) 74.5 -> 85.1, 96 of 300 20.2 -> 23.2, and 1000
-// rows of a prompt over 8 kv heads 141 -> 196.  (Rows of very different length are another matter: 63 of 500 to 4000 79 -> 70.
-// The host does not know the lengths.)  With heads of 64 what is beyond these lines goes by attn_many.
+// 22.7 -> 18.9.  Beyond that this kernel, with its two workgroups per CU, was behind a wave per item: 16 of 3000 (768 items) 30.5 -> 32.6,
+// 8 of 8000 (1024) 33.4 -> 37.5, 96 of 300 20.2 -> 23.2, and 1000 rows of a prompt over 8 kv heads 141 -> 196.  With heads of 64 what
+// is beyond these lines goes by attn_many.
 static bool attn_few(long long pairs, int span, int head_dim) {
   const long long items = pairs * ((span + ATT_CHUNK - 1) / ATT_CHUNK);
   return items <= (span * head_dim < 256 * 64 ? 256 : head_dim == 32 ? 384 : 512);
@@ -925,21 +924,27 @@ struct AttnPlan {
 // four kv heads, are one CU's 512 KB where another CU has none (a CU reads about 40 KB a us), and a wave takes its blocks one
 // behind the other, 20 us for 512 positions.  64 heads of 64 on 8 kv heads, caches cold, rows of an eighth to all of the length / all
 // of it, a wave per item -> workgroup per item (us):
-//   chunks merged by a kernel behind   17 sequences of 5000 39.3 / 43.4 -> 26.7 / 38.4, 40 of 1000 23.2 / 24.7 -> 20.3 / 24.0, 63 of 4000
-//     76.0 / 94.8 -> 59.1 / 92.7, 32 of 32000 315 / 405 -> 262 / 393; the worst 30 of 4000 40.6 / 46.8 -> 32.5 / 48.5.  Always.
-//   rows of one chunk   200 of 200 20.7 / 24.8 -> 16.8 / 22.2, 100 of 256 13.5 / 13.7 -> 11.8 / 13.3, 400 of 448 57.2 / 70.7 -> 40.8 /
-//     61.3, 512 of 200 36.1 / 47.8 -> 33.6 / 46.3, of 448 62.6 / 75.7 -> 51.5 / 77.2; short ones 70 of 64 7.1 / 6.7 -> 6.9 / 5.9, of 128
-//     9.2 / 8.8 -> 8.0 / 7.4, but 100 of 64 7.5 / 7.1 -> 9.1 / 7.6, 256 of 128 15.7 / 16.3 -> 17.8 / 17.1, 256 of 2000 with a window of 128
+//   chunks merged by a kernel behind   17 sequences of 4000 25.2 / 41.0 -> 22.8 / 32.0, 40 of 1000 23.6 / 25.3 -> 18.9 / 22.8, 63 of
+//     4000 75.2 / 95.4 -> 54.0 / 92.5, 63 of 16000 254 / 416 -> 208 / 370.  Items of one length take the waves whole rounds of 1024 and
+//     this kernel rounds of 768: 32 of 2000 24.5 / 28.6 -> 20.9 / 32.4, 30 of 2000 24.2 / 27.8 -> 20.7 / 29.9, 63 of 1000 24.5 / 28.4 ->
+//     21.3 / 29.2, 63 of 2000 41.2 / 49.0 -> 32.5 / 52.8, 63 of 3000 56.1 / 70.0 -> 39.4 / 71.1, 48 of 4000 58.9 / 71.0 -> 46.0 / 72.7; at
+//     more rounds it is ahead there too.  So always, but where the host knows that all rows are of one length (it does not if it is
+//     given lengths) and they nearly fill up to three rounds of waves.
+//   rows of one chunk   200 of 200 20.4 / 24.5 -> 16.5 / 21.9, 100 of 256 14.2 / 14.3 -> 11.8 / 13.2, 400 of 448 54.6 / 71.6 -> 40.8 /
+//     61.0, 512 of 200 37.0 / 49.6 -> 33.4 / 45.8, of 448 62.1 / 76.5 -> 50.2 / 76.7; short ones 70 of 64 7.4 / 6.8 -> 7.0 / 5.9, of 128
+//     9.4 / 8.8 -> 7.9 / 7.4, but 100 of 64 7.5 / 7.1 -> 9.1 / 7.6, 256 of 128 15.7 / 16.3 -> 17.8 / 17.1, 256 of 2000 with a window of 128
 //     21.3 / 20.9 -> 23.2 / 23.1.  From 192 positions on up to 4096 items, shorter ones up to 640.
-//   rows of one chunk in front of the workgroup-per-row kernel   64 of 1000 35.8 / 27.9 -> 27.2 / 27.4, 98 of 736 34.8 / 34.5 ->
-//     29.0 / 34.4, 256 of 1000 74.4 / 85.7 -> 61.0 / 85.7, 600 of 1000 146.4 / 194.4 -> 128.0 / 195.4; of 1024 of 600, where
-//     8192 workgroups may have nothing to do, 160.4 / 214.2 -> 146.3 / 217.3.  Up to 4096 items, 8192 where the host does not know that
+//   rows of one chunk in front of the workgroup-per-row kernel   64 of 1000 35.4 / 28.2 -> 28.4 / 27.6, 98 of 736 35.3 / 34.4 ->
+//     30.8 / 34.6, 256 of 1000 74.5 / 86.1 -> 61.5 / 85.9, 600 of 1000 148 / 195 -> 127 / 196; of 1024 of 576, where
+//     8192 workgroups may have nothing to do, 151.6 / 198 -> 144.5 / 200.5.  Up to 4096 items, 8192 where the host does not know that
 //     all rows are of one length.
 // (Rows of a prompt read the same blocks: those stay with a wave per item.)
 static bool attn_many(long long items, const AttnPlan &pl, int span, int head_dim, bool one_length) {
   if (head_dim != 64) return false;
   if (pl.wide) return items <= (one_length ? 4096 : 8192);
-  return pl.max_chunks > 1 ? items < (1ll << 31) : items <= (span >= 192 ? 4096 : 640);
+  if (pl.max_chunks == 1) return items <= (span >= 192 ? 4096 : 640);
+  const bool full_rounds = items <= 3 * 1024 && (items + 1023) / 1024 * 1024 - items <= 128;
+  return items < (1ll << 31) && !(one_length && full_rounds);
 }
 
 // Merge the chunk partials of one (sequence, q head) with the sink logit.  One thread owns four

@@ -316,7 +316,8 @@ def _kernels(ops, call):
 @pytest.mark.parametrize("longest,cap,window", [(2000, 2048, 0), (700, 768, 0), (2000, 2048, 700), (3000, 1024, 600)])
 @pytest.mark.parametrize("n_q,n_kv,D", [(64, 8, 64), (96, 8, 64), (64, 8, 32)])
 def test_few_rows_of_several_chunks_have_the_bits_of_the_same_rows_among_more(ops, n_q, n_kv, D, longest, cap, window):
-    """A workgroup per chunk where few are served, a wave per chunk where more are (60 rows: too few for a workgroup each)."""
+    """All loads of a chunk at once where few are served; for 60 rows heads of 64 three workgroups per CU, heads of 32 a wave per
+    chunk."""
     B = 60
     g = torch.Generator(device="cuda").manual_seed(longest + window)
     rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
@@ -334,6 +335,23 @@ def test_few_rows_of_several_chunks_have_the_bits_of_the_same_rows_among_more(op
     for rows in (1, 2, 5, 9):
         assert _kernels(ops, lambda: attend(rows)) == ["attn_decode_few", "attn_reduce"], rows
         assert torch.equal(out[rows].view(torch.int16), out[B][:rows].view(torch.int16)), rows
+
+
+# rounds of 1024 (row, kv head, chunk) items that are nearly full, and one that is not (24 of 2000: 768)
+@pytest.mark.parametrize("B,longest", [(32, 2000), (63, 1000), (63, 2000), (48, 3900), (24, 2000)])
+def test_rows_of_one_length_have_the_same_bits_a_workgroup_or_a_wave_per_chunk(ops, B, longest):
+    """Without lengths all rows are known to have the longest one, and go by a wave per chunk where that fills rounds."""
+    n_q, n_kv, D, cap = 64, 8, 64, (longest + 63) // 64 * 64
+    g = torch.Generator(device="cuda").manual_seed(longest + B)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    cache = ops.KVCache(B, n_kv, D, cap)
+    cache.kv.view(torch.int16).fill_(0x7FC1)             # NaN patterns where nothing is written
+    cache.write(rnd(B, longest, n_kv, D).bfloat16(), rnd(B, longest, n_kv, D).bfloat16(), 0)
+    q, sinks = rnd(B, n_q, D) * 2, rnd(n_q)
+    attn = ops.AttnDecode(B, n_q, n_kv, D, longest)
+    known = attn.forward(q, cache, None, sinks)
+    given = attn.forward(q, cache, torch.full((B,), longest, dtype=torch.int32, device="cuda"), sinks)
+    assert torch.isfinite(known).all() and torch.equal(known.view(torch.int16), given.view(torch.int16))
 
 
 # rows of one chunk: up to 512 sequences a workgroup each, 520 a wave, short ones up to 80 and 90; of one chunk and of several: up to
