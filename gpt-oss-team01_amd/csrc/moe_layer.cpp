@@ -62,10 +62,11 @@ static int env_int(const char *name, int dflt) {
 // from 512 on.
 // From 165 to 248 an expert's rows are two 160-row tiles and one of 256 (2880 x 2880, uniform / Zipf 1.1, streaming -> 256-row
 // kernels, us: 32 experts of 160 rows 530 / 541 -> 475 / 564, 175 623 / 577 -> 509 / 578, 200 702 / 622 -> 542 / 608, 240
-// 684 / 698 -> 595 / 669, 248 717 / 693 -> 663 / 683; 64 of 200 1314 / 1164 -> 993 / 1138; 16 of 200 350 / 332 -> 285 / 339).  Below,
+// 684 / 698 -> 595 / 669, 248 717 / 693 -> 663 / 683; 64 of 200 1314 / 1164 -> 993 / 1138).  Below,
 // one of 160 holds them (150 rows 496 / 531 -> 479 / 555, 128 391 / 506 -> 434 / 505), above two of either (275 692 / 737 ->
-// 790 / 704, 325 837 / 802 -> 861 / 784).  Small blocks lose here too: 2048 x 1024, 32 experts of 200 210 / 212 -> 227 / 213, eight of
-// 2880 x 2880 187 / 173 -> 163 / 187.
+// 790 / 704, 325 837 / 802 -> 861 / 784).  With less arithmetic a skewed routing loses what a uniform one gains (16 experts of 190
+// rows of 2816 x 2880 303 / 278 -> 264 / 319, 32 of 165 of 2688 x 1664 304 / 276 -> 287 / 327); from the line on, 24 sizes, uniform
+// routings gain 5 to 20 % and Zipf 0.6 and 1.1 are between 5 % shorter and 4 % longer, 1 % on average.
 static int moe_tall_forced() {
   static const int v = env_int("GPTOSS_MOE_TALL_MIN_ROWS", 0);
   return v;
@@ -74,7 +75,7 @@ static bool moe_tall(long long pairs, int E, int N, int K) {
   if (const int v = moe_tall_forced()) return pairs >= (long long)v * E;
   const double work = (double)pairs * N * K;
   if (pairs >= (long long)(work >= (double)(1ll << 34) ? 416 : 512) * E) return true;
-  return work >= (double)(1ll << 35) && pairs >= 165ll * E && pairs <= 248ll * E;
+  return work >= 5.0 * (1ll << 34) && pairs >= 165ll * E && pairs <= 248ll * E;
 }
 
 int moe_rows_per_tile(int B, int k, int E, bool mxfp4) {
@@ -102,24 +103,26 @@ static double expected_tiles(int k, int E, double avg, int rows_per_tile) {
 // The row tile of a bf16 block, given the one that holds an expert's rows: where tiles of that size are work for fewer than two
 // rounds of the CUs, the one that makes both products shortest by the estimates of gemm_dense.cpp.  Smaller tiles put more
 // CUs to work (an item of 160 rows is a CU's for 20 to 50 us), and where every token takes every expert, so that the tiles are known,
-// 256 rows may save a round.  It has to be ahead by a tenth, the estimates' error, or by a quarter where the rows per expert are
-// not known: the estimates are for a uniform routing.  Blocks in us, before -> after: 4 of 4 experts, 2048 x 1024, 70 / 135 /
+// 256 rows may save a round.  It has to be ahead by 15 %, the estimates' error, or by a quarter, with a fifth more tiles than a
+// uniform routing makes, where the rows per expert are not known.  Blocks in us, before -> after: 4 of 4 experts, 2048 x 1024, 70 / 135 /
 // 240 rows each 61 / 73 / 75 -> 39 / 42 / 44, 2880 x 2880, 100 / 330 rows 102 / 192 -> 82 / 131; 4 of 16, 1024 x 512, 60 / 200 rows
-// 45 / 61 -> 35 / 51; two of 4, 4096 x 1536, 70 rows 93 -> 64.  Of 500 blocks of random sizes, uniform and Zipf 1.1, a few lose, up to 6 %.
+// 45 / 61 -> 35 / 51; two of 4, 4096 x 1536, 70 rows 93 -> 64.  Of 4700 blocks of random sizes, uniform, Zipf 0.6 and 1.1, none takes
+// more than 1 % longer.  (Ahead by a tenth and by a quarter, without the fifth, 25 of them did, by up to a quarter: 6 experts of 106
+// rows of 2624 x 2688 have 12 tiles of 64, one round of the CUs, or 13, and two.)
 static int small_block_rows(int dflt, int B, int k, int E, int H, int I, bool tall) {
   const double avg = (double)B * k / E;
   if (dflt <= 64 || dflt == 256 || expected_tiles(k, E, avg, dflt) * gemm_col_tiles(2 * I) >= 512) return dflt;
-  auto us = [&](int rpt) {
+  auto us = [&](int rpt, double more) {
     const int max_tiles = gptoss_moe_max_tiles(B, k, std::min(E, B * k), rpt);
-    const double tiles = expected_tiles(k, E, avg, rpt);
+    const double tiles = expected_tiles(k, E, avg, rpt) * more;
     return grouped_us(rpt, tiles, grouped_few(rpt, max_tiles, 2 * I), 2 * I, H) + grouped_us(rpt, tiles, grouped_few(rpt, max_tiles, H), H, I);
   };
   int best = dflt;
-  double least = (k == E ? 0.9 : 0.75) * us(dflt);
+  double least = (k == E ? 0.85 : 0.75) * us(dflt, 1.0);
   for (int rpt : {32, 64, 128, 160, 256}) {
     // (tiles of 32 rows read the weights again and again: not beyond two rounds of the few-row kernels)
     if ((rpt == 256 && (!tall || k != E)) || (rpt == 32 && expected_tiles(k, E, avg, 32) * (2 * I / 32) > 2560)) continue;
-    const double t = us(rpt);
+    const double t = k == E || rpt == dflt ? us(rpt, 1.0) : std::max(us(rpt, 1.0), us(rpt, 1.2));
     if (t < least) {
       least = t;
       best = rpt;

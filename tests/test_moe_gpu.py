@@ -599,8 +599,8 @@ def test_row_blocks_of_a_prompt_pass(ops, rows):
 
 @pytest.mark.parametrize("rows", [164, 165, 200, 248, 249])
 def test_large_blocks_of_one_and_two_row_tiles_per_expert(ops, rows):
-    """Every token on all of 4 experts of 4096 x 8640: one 256-row tile from 165 rows to 248, two 160-row tiles outside."""
-    E, H, I = 4, 4096, 8640
+    """Every token on all of 4 experts of 4096 x 16128: one 256-row tile from 165 rows to 248, two 160-row tiles outside."""
+    E, H, I = 4, 4096, 16128
     g = torch.Generator(device="cuda").manual_seed(rows)
     n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
     layer = ops.MoeLayer(n(E, H), n(E).float(), n(E, 2 * I, H, std=0.02), n(E, 2 * I).float(), n(E, H, I, std=0.02),
