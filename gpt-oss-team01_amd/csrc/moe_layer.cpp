@@ -228,14 +228,17 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
   grp.nbits = 0;
   while ((1 << grp.nbits) < E) grp.nbits++;
   // A few tokens: the router's products are spread over CUs (router_parts_kernel), if the second product's output, which comes
-  // later, has room for them.
-  float *parts = router_parts_floats(B, E) <= (size_t)B * k * H ? ws.y2 : nullptr;
+  // later, has room for them.  A router of few inputs is little to spread (block, us: 128 inputs, 8 experts of 1024, 8 / 16 tokens
+  // +6 / +4 %, one of 128 +9 / +7 %; 64 inputs, 16 experts 3 to 11 %; 32 experts of 128 inputs -5 to -15 %).
+  float *parts = router_parts_floats(B, E) <= (size_t)B * k * H && (H >= 256 || E * H >= 4096) ? ws.y2 : nullptr;
   // Up to four are gated and grouped by the workgroups of the first product (few_routed_kernel); the norm in front runs in the
   // router's kernel.  The block by one launch less, us: 2880 x 2880, one token on 4 of 32 experts 45.9 -> 40.6, two 68.4 -> 63.8,
   // four 120.5 -> 116.2, in MXFP4 31.6 -> 26.8, 38.2 -> 33.6, 49.6 -> 46.6, one on 128 experts 31.6 -> 27.9, with the norm one on 32
   // experts 48.5 -> 43.0, on 128 (1024 wide) 30.5 -> 25.5.  Each workgroup repeats the gating, so three and four tokens go this way
   // only where that is little, up to 32 experts, and where the router's own kernel has a large matrix to read: 128 experts, four
   // tokens 51.4 -> 54.4, four experts of 2880 inputs 42.8 -> 43.5, eight of 2048 27.9 -> 28.2; 32 of 640 20.6 -> 18.2.
+  // More than 32 experts take four values a lane, and more workgroups than the chip holds at once gate in a second round: two
+  // tokens on 8 of 48 experts of 768 x 2880, 3060 workgroups, +6 %, one token, 1620, -5 %; up to 2048.
   RoutedFew routed{RouterParts{parts, w->b_router, B, E, k}, ws.logits, ws.topk_w, ws.topk_i, grp};
   routed.group.expert_offsets = ws.expert_offsets;
   if (pre) {
@@ -243,7 +246,8 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
     routed.residual = pre->residual;
     routed.x_count = B * H;
   }
-  const bool few = (B <= 2 || (B <= ROUTED_TOKENS && E <= 32 && H * E >= 20480)) && k <= 8 && E <= ROUTED_EXPERTS && rpt == 32 && parts &&
+  const bool gated_at_once = E <= 32 || (long long)(max_tiles + 1) * (2 * I / 32) <= 2048;
+  const bool few = (B <= 2 || (B <= ROUTED_TOKENS && E <= 32 && H * E >= 20480)) && k <= 8 && E <= ROUTED_EXPERTS && rpt == 32 && parts && gated_at_once &&
                    (long long)max_tiles * 32 * H * 2 < (1ll << 31) &&
                    (!pre || norm_router_parts_apply(B, H, pre->x, pre->residual, pre->weight, t));
   if (few) {

@@ -866,6 +866,12 @@ static int router_col_blocks(int E) {
   return nb <= 1 ? 1 : nb <= 2 ? 2 : nb <= 4 ? 4 : nb <= 8 ? 8 : 16;
 }
 
+// More than 128 experts of so few inputs that a row is a part of one stage (router_gemm_kernel): nothing hides the four parts one
+// behind the other.  Blocks of 64 inputs, one workgroup for all -> shared out, us: 129 experts, 1 / 17 / 300 tokens 21.1 / 29.1 /
+// 32.6 -> 19.8 / 26.7 / 30.9, 256 15.7 / 24.0 / 25.0 -> 14.4 / 22.8 / 24.1; but 4000 tokens 46.3 -> 49.6 and 33.9 -> 39.7.  The logits
+// alone of 256, 1 / 300 tokens 5.4 / 5.7 -> 3.6 / 3.7.
+static bool router_one_stage(int E, int H) { return E > 128 && H <= 128; }
+
 // Whether a workgroup takes 16 experts instead of all of them.  Sharing the experts out saves loads and costs a second launch,
 // which gates (up to 16 tokens: and groups).  The lines are where they were worth it while a workgroup's loads came in operand
 // order, in rounds of 190 to 260 at 36 KB a us; now that all experts in one workgroup take half of that time (router_gemm_kernel),
@@ -880,6 +886,7 @@ static int router_col_blocks(int E) {
 // other side from 17 tokens on (1024 inputs, 64 experts, 256 tokens 38.1 -> 37.3, 96 experts, 200 tokens +0.8).
 static bool router_splits(int B, int H, int E) {
   if (E <= 32) return false;
+  if (router_one_stage(E, H)) return B <= 512;
   const bool one_round = H / 32 <= ROUTER_WAVES * router_steps(router_col_blocks(E));
   return one_round ? E > 48 && H >= 256 && B <= 256 : B <= 512;
 }
@@ -918,8 +925,6 @@ int run_norm_router_parts(const float *x, const float *residual, const float *we
   return GPTOSS_OK;
 }
 
-// logits (+ optional gating of the same tokens), in one launch unless many experts are shared out (only with the gating of at
-// most 8 experts per token: logits alone come from one workgroup for all experts)
 template <int NB, bool LARGE>
 static int launch_router_rows(const bf16_t *t, const bf16_t *wr, const float *br, float *logits, int B, int H, int E, int k,
                          float *topk_w, int *topk_i, int rows_per_wg, int shares, const RouterGroup &grp, hipStream_t s) {
@@ -949,6 +954,8 @@ static int launch_router(const bf16_t *t, const bf16_t *wr, const float *br, flo
   return (large ? launch_router_rows<NB, true> : launch_router_rows<NB, false>)(t, wr, br, logits, B, H, E, more...);
 }
 
+// logits (+ optional gating of the same tokens), in one launch unless many experts are shared out (with the gating of at
+// most 8 experts per token: logits alone come from one workgroup for all experts, or router_one_stage)
 int run_router(const void *t, const void *w_router, const float *b_router, float *logits, int B,
                int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group, float *parts) {
   // 16 token rows per workgroup fill the MFMA, but a thousand tokens are then only 64 workgroups;
@@ -998,6 +1005,8 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
     return GPTOSS_OK;
   }
   TraceScope ts(topk_w ? "router_gemm_topk" : "router_gemm", s);
+  if (!topk_w && router_one_stage(E, H) && B <= 512)
+    return launch_router<1>(tp, wp, b_router, logits, B, H, E, k, nullptr, nullptr, router_split_rows(B, E), nb, RouterGroup{}, s);
   if (nb <= 1) return launch_router<1>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);
   if (nb <= 2) return launch_router<2>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);
   if (nb <= 4) return launch_router<4>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);

@@ -449,7 +449,7 @@ def test_routing_of_equal_and_infinite_logits(ops, E, k):
 @pytest.mark.parametrize("E", [33, 48, 64, 100, 128, 256])
 @pytest.mark.parametrize("H", [64, 256, 2880])
 def test_experts_shared_out_among_workgroups_score_and_gate_the_same(ops, E, H):
-    """From 33 experts on up to 512 tokens (H = 256: from 49, up to 256; H = 64: none) have 16 experts per workgroup and are
+    """From 33 experts on up to 512 tokens (H = 256: from 49, up to 256; H = 64: from 129) have 16 experts per workgroup and are
     gated by another launch; 600 have one workgroup for all experts.  Same bits."""
     g = torch.Generator(device="cuda").manual_seed(E + H)
     n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
@@ -466,14 +466,16 @@ def test_experts_shared_out_among_workgroups_score_and_gate_the_same(ops, E, H):
 
 
 # up to 64 experts a round of loads is 1792 inputs, up to 128 1024, beyond 512; more than that: shared out up to 512 tokens,
-# less: 256 inputs and 49 experts or more, up to 256 tokens.  Up to 16 tokens: partial products, unless 8 E floats are more
-# than k H, or three to seven tokens have fewer than 16 experts
+# less: 256 inputs and 49 experts or more, up to 256 tokens; up to 128 inputs from 129 experts on, up to 512 tokens.  Up to 16
+# tokens: partial products, unless 8 E floats are more than k H, three to seven tokens have fewer than 16 experts, or there are
+# fewer than 256 inputs and 4096 weights
 @pytest.mark.parametrize("H,E,tokens,router", [
     (4096, 32, 1, "parts"), (4096, 32, 17, "one"), (1856, 33, 1, "parts"), (1856, 33, 17, "shared"), (1792, 33, 17, "one"),
     (1792, 48, 16, "parts"), (1792, 48, 17, "one"), (1792, 49, 16, "parts"), (1792, 49, 17, "shared"), (1088, 128, 257, "shared"),
     (1024, 128, 257, "one"), (1024, 65, 256, "shared"), (576, 129, 512, "shared"), (576, 129, 513, "one"), (512, 256, 257, "one"),
     (512, 256, 256, "shared"), (512, 256, 16, "parts"), (448, 256, 16, "shared"), (256, 64, 17, "shared"), (192, 256, 17, "one"),
-    (64, 256, 1, "one"), (256, 15, 2, "parts"), (256, 15, 7, "one"), (256, 15, 8, "parts"), (256, 16, 5, "parts")])
+    (128, 129, 512, "shared"), (128, 129, 513, "one"), (128, 128, 17, "one"), (64, 256, 1, "shared"), (192, 21, 1, "one"),
+    (192, 22, 5, "parts"), (64, 64, 4, "one"), (256, 15, 2, "parts"), (256, 15, 7, "one"), (256, 15, 8, "parts"), (256, 16, 5, "parts")])
 def test_which_calls_share_their_experts_out(ops, H, E, tokens, router):
     g = torch.Generator(device="cuda").manual_seed(H)
     n = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
@@ -484,6 +486,23 @@ def test_which_calls_share_their_experts_out(ops, H, E, tokens, router):
     launches = [name for name, _ in trace.results()]
     name = {"parts": "router_parts", "one": "router_gemm_topk", "shared": "router_gemm"}
     assert [x for x in launches if x.startswith("router")] == [name[router]]
+
+
+# 48 experts of 768 x 2880: 1620 workgroups for one token, 3060 for two; 32 experts: any number
+@pytest.mark.parametrize("E,tokens,by_one", [(48, 1, False), (48, 2, True), (32, 2, False)])
+def test_two_tokens_over_more_workgroups_than_the_chip_holds_are_gated_by_one(ops, E, tokens, by_one):
+    g = torch.Generator(device="cuda").manual_seed(E + tokens)
+    n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    H, I = 768, 2880
+    layer = ops.MoeLayer(n(E, H, std=H ** -0.5), n(E).float(), n(E, 2 * I, H, std=0.05), n(E, 2 * I).float(), n(E, H, I, std=0.05),
+                         n(E, H).float(), top_k=8, max_tokens=40)
+    t = n(40, H)
+    out = layer.forward(t).clone()
+    with ops.KernelTrace(16) as trace:
+        got = layer.forward(t[:tokens].contiguous())
+    launches = [name for name, _ in trace.results()]
+    assert "router_parts" in launches and ("topk_group" in launches) == by_one
+    assert torch.equal(got, out[:tokens])
 
 
 @pytest.mark.parametrize("E,H", [(49, 256), (64, 320), (65, 256), (128, 960), (129, 512), (256, 1984)])
