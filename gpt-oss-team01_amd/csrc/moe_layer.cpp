@@ -60,22 +60,22 @@ static int env_int(const char *name, int dflt) {
 // From 416 on they gain 2-23 % (both routings, uniform and Zipf 1.1; 2880 x 2880, 32 experts of 437 rows 877 -> 790 us) where there
 // is work for the whole chip: blocks of 1024 x 512 on 16 experts lose 13 %, blocks of four times the arithmetic gain, so small ones
 // from 512 on.
-// From 165 to 248 an expert's rows are two 160-row tiles and one of 256 (2880 x 2880, uniform / Zipf 1.1, streaming -> 256-row
-// kernels, us: 32 experts of 160 rows 530 / 541 -> 475 / 564, 175 623 / 577 -> 509 / 578, 200 702 / 622 -> 542 / 608, 240
-// 684 / 698 -> 595 / 669, 248 717 / 693 -> 663 / 683; 64 of 200 1314 / 1164 -> 993 / 1138).  Below,
-// one of 160 holds them (150 rows 496 / 531 -> 479 / 555, 128 391 / 506 -> 434 / 505), above two of either (275 692 / 737 ->
-// 790 / 704, 325 837 / 802 -> 861 / 784).  With less arithmetic a skewed routing loses what a uniform one gains (16 experts of 190
-// rows of 2816 x 2880 303 / 278 -> 264 / 319, 32 of 165 of 2688 x 1664 304 / 276 -> 287 / 327); from the line on, 24 sizes, uniform
-// routings gain 5 to 20 % and Zipf 0.6 and 1.1 are between 5 % shorter and 4 % longer, 1 % on average.
+// From 165 to 248 an expert's rows are two 160-row tiles and one of 256, but only while the routing is uniform (2880 x 2880, 32
+// experts, uniform / Zipf 0.6 / 1.1, streaming kernels = 1: 165 rows 0.90 / 1.03 / 1.05, 177 0.85 / 1.07 / 1.06, 189 0.84 / 1.08 /
+// 1.05, 201 0.82 / 1.03 / 1.05, 213 0.85 / 1.04 / 1.01, 225 0.87 / 1.03 / 0.98, 243 0.92 / 1.02 / 0.99; 500 us at 177, 560 at 213).  So
+// from 213 on, where preferences like a trained router's lose nothing, and with as much arithmetic as that: of smaller blocks those
+// lose up to 18 %, of 7 sizes beyond the line uniform routings gain 5 to 16 %, Zipf 0.6 and 1.1 1 % on average, at most 3 % lost.
+// Where every token takes every expert, so that no expert has more rows than another, from 165 on and with 40 % of that arithmetic.
+// Above 248 two tiles of either (275 rows 692 / - / 737 -> 790 / - / 704 us, 325 837 / - / 802 -> 861 / - / 784).
 static int moe_tall_forced() {
   static const int v = env_int("GPTOSS_MOE_TALL_MIN_ROWS", 0);
   return v;
 }
-static bool moe_tall(long long pairs, int E, int N, int K) {
+static bool moe_tall(long long pairs, int E, int k, int N, int K) {
   if (const int v = moe_tall_forced()) return pairs >= (long long)v * E;
   const double work = (double)pairs * N * K;
   if (pairs >= (long long)(work >= (double)(1ll << 34) ? 416 : 512) * E) return true;
-  return work >= 5.0 * (1ll << 34) && pairs >= 165ll * E && pairs <= 248ll * E;
+  return work >= (k == E ? 2.0 : 5.0) * (1ll << 34) && pairs >= (k == E ? 165ll : 213ll) * E && pairs <= 248ll * E;
 }
 
 int moe_rows_per_tile(int B, int k, int E, bool mxfp4) {
@@ -205,7 +205,7 @@ static int moe_forward_impl(const gptoss_moe_weights *w, const void *t, int B, f
   const long long tall_rows = ((long long)B * k / 256 + E) * 256;
   if (!mxfp4) {
     const bool tall = gemm_tall_shape_ok(2 * I, H, tall_rows) && gemm_tall_shape_ok(H, I, tall_rows);
-    if (tall && moe_tall((long long)B * k, E, 2 * I, H)) rpt = 256;
+    if (tall && moe_tall((long long)B * k, E, k, 2 * I, H)) rpt = 256;
     if (!moe_tall_forced()) rpt = small_block_rows(rpt, B, k, E, H, I, tall);
   }
   // (no more experts have a row than there are rows)

@@ -616,17 +616,19 @@ def test_row_blocks_of_a_prompt_pass(ops, rows):
     test_last_row_tiles_of_a_prompt_pass(ops, rows)
 
 
-@pytest.mark.parametrize("rows", [164, 165, 200, 248, 249])
-def test_large_blocks_of_one_and_two_row_tiles_per_expert(ops, rows):
-    """Every token on all of 4 experts of 4096 x 16128: one 256-row tile from 165 rows to 248, two 160-row tiles outside."""
-    E, H, I = 4, 4096, 16128
+# every token on all experts: one 256-row tile from 165 rows to 248, two 160-row tiles outside; on half of them: from 213
+@pytest.mark.parametrize("k,I,rows", [(4, 8640, 164), (4, 8640, 165), (4, 8640, 200), (4, 8640, 248), (4, 8640, 249),
+                                      (2, 16128, 212), (2, 16128, 213), (2, 16128, 248), (2, 16128, 249)])
+def test_large_blocks_of_one_and_two_row_tiles_per_expert(ops, k, I, rows):
+    E, H = 4, 4096
+    B = rows * E // k
     g = torch.Generator(device="cuda").manual_seed(rows)
     n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
-    layer = ops.MoeLayer(n(E, H), n(E).float(), n(E, 2 * I, H, std=0.02), n(E, 2 * I).float(), n(E, H, I, std=0.02),
-                         n(E, H).float(), max_tokens=rows)
-    t = n(rows, H)
+    layer = ops.MoeLayer(n(E, H, std=0.02), n(E).float(), n(E, 2 * I, H, std=0.02), n(E, 2 * I).float(), n(E, H, I, std=0.02),
+                         n(E, H).float(), top_k=k, max_tokens=B)
+    t = n(B, H)
     out = layer.forward(t).clone()
-    for i in range(0, rows, 64):
+    for i in range(0, B, 64):
         assert torch.equal(layer.forward(t[i:i + 64].contiguous()), out[i:i + 64]), i
 
 
