@@ -350,8 +350,7 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void norm_router_kernel(
   const int kq = (lane >> 4) * 8;
   constexpr int ROUTER_MAX_STEPS = router_steps(NB);
   const int ksteps = H / 32;
-  // In two halves: while one is multiplied, the other's loads are on their way (2880 inputs, 64 experts 16.3 -> 13.9 us, a third
-  // round of loads for the second one's last steps less; 128 25.0 -> 24.5).  More than 128 experts leave no registers for it.
+  // In two halves: while one is multiplied, the other's loads are on their way.  More than 128 experts leave no registers for it.
   constexpr int SETS = NB <= 8 ? 2 : 1, HALF = (ROUTER_MAX_STEPS + SETS - 1) / SETS, STRIDE = HALF * ROUTER_WAVES;
   u32x4 a[SETS][HALF], b[SETS][HALF][NB];
   auto load_b = [&](int ks0, auto set) {
@@ -845,9 +844,10 @@ int run_topk_softmax(const float *logits, int B, int E, int k, float *topk_w, in
   return GPTOSS_OK;
 }
 
-// Token rows of a workgroup: as few as leave no more workgroups than CUs, where a workgroup has a CU to itself (eight waves with
-// the registers of two per SIMD) and takes the time of its share of the experts' weights whatever its rows are.  2880 inputs, 32 / 128 experts: 1100
-// to 2000 tokens in groups of four 15.9 / 48.5 us, of eight 8.8 / 25.0; 2100 to 4000 in groups of eight 16.7 / 49.8, of 16 9.8 / 26.5.
+// Token rows of a workgroup: as few as leave no more workgroups than CUs.  Up to there their number makes little difference (2880
+// inputs, 32 experts, 512 / 1024 tokens in groups of four 5.5 / 5.9 us, of eight 5.5 / 5.6, of 16 5.4 / 5.5), because a workgroup takes the time
+// of its experts' weights whatever its rows are; beyond it they come in rounds: 1400 tokens, 32 / 128 experts, 7.6 / 23.6, 5.7 / 12.6 and
+// 5.6 / 12.6, 3000 11.0 / 34.4, 8.0 / 23.8 and 6.1 / 13.1.
 static int router_rows_per_wg(int B) {
   int rows_per_wg = 4;
   while (rows_per_wg < 16 && cdiv(B, rows_per_wg) > 256) rows_per_wg *= 2;
@@ -866,30 +866,18 @@ static int router_col_blocks(int E) {
   return nb <= 1 ? 1 : nb <= 2 ? 2 : nb <= 4 ? 4 : nb <= 8 ? 8 : 16;
 }
 
-// More than 128 experts of so few inputs that a row is a part of one stage (router_gemm_kernel): nothing hides the four parts one
-// behind the other.  Blocks of 64 inputs, one workgroup for all -> shared out, us: 129 experts, 1 / 17 / 300 tokens 21.1 / 29.1 /
-// 32.6 -> 19.8 / 26.7 / 30.9, 256 15.7 / 24.0 / 25.0 -> 14.4 / 22.8 / 24.1; but 4000 tokens 46.3 -> 49.6 and 33.9 -> 39.7.  The logits
-// alone of 256, 1 / 300 tokens 5.4 / 5.7 -> 3.6 / 3.7.
-static bool router_one_stage(int E, int H) { return E > 128 && H <= 128; }
-
-// Whether a workgroup takes 16 experts instead of all of them.  Sharing the experts out saves loads and costs a second launch,
-// which gates (up to 16 tokens: and groups).  The lines are where they were worth it while a workgroup's loads came in operand
-// order, in rounds of 190 to 260 at 36 KB a us; now that all experts in one workgroup take half of that time (router_gemm_kernel),
-// the two are closer.  Then, all experts in one workgroup -> shared out, MoE block with narrow experts (us):
-//   more than one round  2880 inputs, 64 experts, 1 / 512 tokens 29.9 / 80.2 -> 20.7 / 71.3, 128 39.0 / 104 -> 22.0 / 87.0, 33 experts,
-//                        17 / 512 tokens 39.0 / 86.0 -> 34.8 / 82.4; 1024 inputs, 256 experts, 512 tokens 62.6 -> 57.6
-//   one round            1024 inputs, 64 experts, 1 / 256 tokens 19.5 / 36.3 -> 17.2 / 34.3; but 48 experts, 256 tokens 36.9 -> 36.5,
-//                        33 experts 35.9 -> 36.6, 96 experts, 400 tokens 44.5 -> 46.0, 512 inputs, 192 experts, 400 tokens
-//                        38.1 -> 43.1, and 64 inputs, 128 experts, 1 / 256 tokens 14.9 / 26.4 -> 15.2 / 26.6
-// Beyond 512 tokens one workgroup for all is as fast or faster (2880 inputs, 128 experts, 1000 tokens 115 against 122).  A norm
-// in front runs in the router's kernel only if that has all experts: its launch is saved as well there, about 1 us to the
-// other side from 17 tokens on (1024 inputs, 64 experts, 256 tokens 38.1 -> 37.3, 96 experts, 200 tokens +0.8).
-static bool router_splits(int B, int H, int E) {
-  if (E <= 32) return false;
-  if (router_one_stage(E, H)) return B <= 512;
-  const bool one_round = H / 32 <= ROUTER_WAVES * router_steps(router_col_blocks(E));
-  return one_round ? E > 48 && H >= 256 && B <= 256 : B <= 512;
-}
+// Whether a workgroup takes 16 experts instead of all of them.  That saves the loads and the parts of a stage one behind the other
+// (router_gemm_kernel) and costs a second launch, which gates (up to 16 tokens: and groups).  MoE block with narrow experts, all
+// experts in one workgroup -> shared out, us:
+//   more than 128 experts  2880 inputs, 256 experts, 17 / 512 tokens 77.4 / 168 -> 61.6 / 148, 1024 41.6 / 66.7 -> 35.0 / 61.9, 512 28.3 / 37.7
+//                          -> 25.5 / 35.4, 256 26.7 / 32.5 -> 25.1 / 31.4, 64 24.0 / 25.2 -> 22.8 / 24.9; 192 of 512 28.2 / 37.4 -> 25.5 / 35.2
+//   65 to 128              2880 inputs, 128 experts 46.4 / 97.7 -> 40.4 / 90.4, 1024 27.2 / 44.2 -> 25.5 / 42.6, 96 experts 27.3 / 43.6 -> 26.0 /
+//                          42.2, 512 24.4 / 33.4 -> 24.0 / 33.1; but 256 23.6 / 28.6 -> 23.8 / 29.4
+//   33 to 64               4096 inputs, 64 experts 46.1 / 88.2 -> 44.3 / 85.4, 2880 37.8 / 73.0 -> 36.9 / 71.3, 33 experts 35.8 / 68.4 -> 34.4 /
+//                          67.6; but 2048, 48 experts 30.6 / 49.2 -> 30.4 / 49.3, 1792, 49 30.1 / 48.3 -> 30.1 / 48.6, 1024, 64 24.2 / 35.7 ->
+//                          24.8 / 36.5, 512 22.0 / 31.4 -> 22.9 / 32.3
+// Up to 512 tokens: at 1000 it is 0 to 5 % (256 experts of 64 inputs, 1500 / 4000 tokens 26.9 / 33.9 -> 29.2 / 39.7).
+static bool router_splits(int B, int H, int E) { return E > 32 && B <= 512 && (E > 128 || H >= (E > 64 ? 512 : 2112)); }
 
 // Rows of a workgroup of 16 experts: four where that is no more than a workgroup per CU.  With four whatever their number,
 // 512 tokens over 128 experts took 59.8 instead of 50.1 us at 1024 inputs, 96.5 instead of 87.0 at 2880, and with 16 rows
@@ -955,13 +943,9 @@ static int launch_router(const bf16_t *t, const bf16_t *wr, const float *br, flo
 }
 
 // logits (+ optional gating of the same tokens), in one launch unless many experts are shared out (with the gating of at
-// most 8 experts per token: logits alone come from one workgroup for all experts, or router_one_stage)
+// most 8 experts per token: logits alone come from one workgroup for all experts, but for many experts of few inputs)
 int run_router(const void *t, const void *w_router, const float *b_router, float *logits, int B,
                int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group, float *parts) {
-  // 16 token rows per workgroup fill the MFMA, but a thousand tokens are then only 64 workgroups;
-  // with fewer rows each (the rest of the MFMA rows idle) all CUs take part in what is a
-  // latency-bound launch: every workgroup reads the whole router matrix from L2 either way
-  // (with the gating, 1024 tokens over 32 experts: 19.7 us with 16 rows, 16.7 with 8, 15.6 with 4, 27 with 2)
   const RouterGroup grp = group ? *group : RouterGroup{};
   const int rows_per_wg = grp.expert_offsets ? ROUTER_GROUP_TOKENS : router_rows_per_wg(B);
   GPTOSS_REQUIRE(!grp.expert_offsets || (topk_w && router_groups(B, k)), GPTOSS_ERR_DIM, "router: %d tokens are not grouped here", B);
@@ -998,14 +982,15 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
     if (!grp.expert_offsets) return run_topk_softmax(logits, B, E, k, topk_w, topk_i, s);
     TraceScope ts("topk_group", s);
     auto launch = [&](auto kern) { kern<<<1, 512, 0, s>>>(logits, RouterParts{}, B, E, k, topk_w, topk_i, grp); };
-    if (nb <= 4) launch(topk_group_kernel<2, false>);
-    else if (nb <= 8) launch(topk_group_kernel<4, false>);
+    // (up to 64 experts are shared out only with so many inputs that the products have room as parts)
+    if (nb <= 8) launch(topk_group_kernel<4, false>);
     else launch(topk_group_kernel<8, false>);
     GPTOSS_LAUNCH_CHECK("topk_group_kernel");
     return GPTOSS_OK;
   }
   TraceScope ts(topk_w ? "router_gemm_topk" : "router_gemm", s);
-  if (!topk_w && router_one_stage(E, H) && B <= 512)
+  // (256 experts of 64 inputs, 1 / 300 tokens 5.4 / 5.7 us in one workgroup, 3.6 / 3.7 shared out)
+  if (!topk_w && E > 128 && H <= 128 && B <= 512)
     return launch_router<1>(tp, wp, b_router, logits, B, H, E, k, nullptr, nullptr, router_split_rows(B, E), nb, RouterGroup{}, s);
   if (nb <= 1) return launch_router<1>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);
   if (nb <= 2) return launch_router<2>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);
@@ -1042,6 +1027,16 @@ static int launch_norm_router(const RouterNorm &nrm, const bf16_t *wp, const flo
   return GPTOSS_OK;
 }
 
+// Whether a norm in front of more than 32 experts is a kernel of its own.  Behind it in one kernel (norm_router_kernel) all experts'
+// loads come in operand order, in rounds; behind one of its own the router takes either form.  Block with narrow experts, one kernel ->
+// two and shared out, us: 2880 inputs, 64 experts, 512 tokens 80.2 -> 71.3, 128 104 -> 87.0; one round: 1024 inputs, 64 experts, 256
+// tokens 36.3 -> 34.3, 33 experts 35.9 -> 36.6, 96 experts, 400 tokens 44.5 -> 46.0, 512 inputs, 192 experts, 400 tokens 38.1 -> 43.1.
+static bool norm_apart(int B, int H, int E) {
+  if (E <= 32) return false;
+  const bool one_round = H / 32 <= ROUTER_WAVES * router_steps(router_col_blocks(E));
+  return one_round ? E > 48 && H >= 256 && B <= 256 : B <= 512;
+}
+
 bool norm_router_applies(int B, int H, int E, const float *x, const float *residual, const float *weight,
                          const void *t_out) {
   const int nb = router_col_blocks(E);
@@ -1049,8 +1044,7 @@ bool norm_router_applies(int B, int H, int E, const float *x, const float *resid
   // With more than four rows per workgroup (batches of more than ~1000 rows) the rows a workgroup
   // normalises one after the other cost more than the launch the fusion saves (8192 rows: 2.58 ms
   // per 24 layers against 2.23 ms for the two kernels; 1024 rows: 0.63 against 0.71 ms).
-  // (Experts that are shared out have their norm in a kernel of its own: every workgroup would repeat it.)
-  return B > 0 && !router_splits(B, H, E) && norm_router_rows_per_wg(B) <= 4 && H % 32 == 0 && H <= 4096 && lds <= 160 * 1024 && aligned(x, 16) && aligned(weight, 16) &&
+  return B > 0 && !norm_apart(B, H, E) && norm_router_rows_per_wg(B) <= 4 && H % 32 == 0 && H <= 4096 && lds <= 160 * 1024 && aligned(x, 16) && aligned(weight, 16) &&
          aligned(t_out, 16) && (!residual || aligned(residual, 16));
 }
 

@@ -449,7 +449,7 @@ def test_routing_of_equal_and_infinite_logits(ops, E, k):
 @pytest.mark.parametrize("E", [33, 48, 64, 100, 128, 256])
 @pytest.mark.parametrize("H", [64, 256, 2880])
 def test_experts_shared_out_among_workgroups_score_and_gate_the_same(ops, E, H):
-    """From 33 experts on up to 512 tokens (H = 256: from 49, up to 256; H = 64: from 129) have 16 experts per workgroup and are
+    """From 33 experts on (H = 256 and 64: from 129) up to 512 tokens have 16 experts per workgroup and are
     gated by another launch; 600 have one workgroup for all experts.  Same bits."""
     g = torch.Generator(device="cuda").manual_seed(E + H)
     n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
@@ -465,15 +465,14 @@ def test_experts_shared_out_among_workgroups_score_and_gate_the_same(ops, E, H):
         assert torch.equal(got, out[:tokens]), tokens
 
 
-# up to 64 experts a round of loads is 1792 inputs, up to 128 1024, beyond 512; more than that: shared out up to 512 tokens,
-# less: 256 inputs and 49 experts or more, up to 256 tokens; up to 128 inputs from 129 experts on, up to 512 tokens.  Up to 16
+# 33 to 64 experts of more than 2048 inputs, up to 128 of 512 and more, beyond of any: shared out up to 512 tokens.  Up to 16
 # tokens: partial products, unless 8 E floats are more than k H, three to seven tokens have fewer than 16 experts, or there are
 # fewer than 256 inputs and 4096 weights
 @pytest.mark.parametrize("H,E,tokens,router", [
-    (4096, 32, 1, "parts"), (4096, 32, 17, "one"), (1856, 33, 1, "parts"), (1856, 33, 17, "shared"), (1792, 33, 17, "one"),
-    (1792, 48, 16, "parts"), (1792, 48, 17, "one"), (1792, 49, 16, "parts"), (1792, 49, 17, "shared"), (1088, 128, 257, "shared"),
-    (1024, 128, 257, "one"), (1024, 65, 256, "shared"), (576, 129, 512, "shared"), (576, 129, 513, "one"), (512, 256, 257, "one"),
-    (512, 256, 256, "shared"), (512, 256, 16, "parts"), (448, 256, 16, "shared"), (256, 64, 17, "shared"), (192, 256, 17, "one"),
+    (4096, 32, 1, "parts"), (4096, 32, 17, "one"), (2112, 33, 1, "parts"), (2112, 33, 17, "shared"), (2112, 33, 513, "one"),
+    (2048, 33, 17, "one"), (2048, 64, 16, "parts"), (2048, 64, 17, "one"), (512, 65, 16, "parts"), (512, 65, 17, "shared"),
+    (448, 128, 17, "one"), (1088, 128, 512, "shared"), (1024, 128, 513, "one"), (576, 129, 512, "shared"), (576, 129, 513, "one"),
+    (512, 256, 257, "shared"), (512, 256, 16, "parts"), (448, 256, 16, "shared"), (256, 64, 17, "one"), (192, 256, 17, "shared"),
     (128, 129, 512, "shared"), (128, 129, 513, "one"), (128, 128, 17, "one"), (64, 256, 1, "shared"), (192, 21, 1, "one"),
     (192, 22, 5, "parts"), (64, 64, 4, "one"), (256, 15, 2, "parts"), (256, 15, 7, "one"), (256, 15, 8, "parts"), (256, 16, 5, "parts")])
 def test_which_calls_share_their_experts_out(ops, H, E, tokens, router):
@@ -505,10 +504,10 @@ def test_two_tokens_over_more_workgroups_than_the_chip_holds_are_gated_by_one(op
     assert torch.equal(got, out[:tokens])
 
 
-@pytest.mark.parametrize("E,H", [(49, 256), (64, 320), (65, 256), (128, 960), (129, 512), (256, 1984)])
+@pytest.mark.parametrize("E,H", [(49, 256), (64, 448), (65, 512), (128, 960), (129, 64), (129, 512), (256, 1984)])
 def test_a_few_tokens_without_room_for_partial_products(ops, E, H):
-    """One expert per token: 8 E floats are more than its row of the second product's output.  The experts are shared out and one
-    workgroup gates and groups the tokens, as larger batches do in other kernels, to the bit."""
+    """One expert per token: 8 E floats are more than its row of the second product's output.  Up to 64 experts one workgroup does
+    the whole routing, beyond the experts are shared out and one workgroup gates and groups the tokens; as in larger batches, to the bit."""
     g = torch.Generator(device="cuda").manual_seed(E + H)
     n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
     layer = ops.MoeLayer(n(E, H, std=H ** -0.5), n(E).float(), n(E, 128, H, std=0.05), n(E, 128).float(), n(E, H, 64), n(E, H).float(),
@@ -521,7 +520,7 @@ def test_a_few_tokens_without_room_for_partial_products(ops, E, H):
         with ops.KernelTrace(16) as trace:
             got = layer.forward(part)
         launches = [name for name, _ in trace.results()]
-        assert "router_gemm" in launches and "topk_group" in launches
+        assert ("router_gemm" in launches and "topk_group" in launches) == (E > 64) and "router_parts" not in launches
         have = layer.routing_views()
         for a, b in zip(have, want):
             assert torch.equal(a, b[:tokens]), tokens
