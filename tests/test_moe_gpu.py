@@ -125,8 +125,8 @@ def test_router_matrices_of_more_than_four_gib(ops, B, H, E):
 
 
 # ---------------------------------------------------------------- weight packing
-@pytest.mark.parametrize("E", [32, 64, 128, 256])           # two halves of a wave's k-steps, more than 128 experts one
-@pytest.mark.parametrize("H", [32, 320, 1792, 2048, 2080, 3104])   # one k-step in all; around a wave's 7 or 8, and 12
+@pytest.mark.parametrize("E", [32, 64, 128, 256])           # a stage in one part, one, two and four
+@pytest.mark.parametrize("H", [32, 320, 1792, 2048, 2080, 3104])   # one k-step in all; whole stages of 256 inputs, and a last one of one k-step or two
 def test_router_rows_are_the_same_in_groups_of_any_size(ops, E, H):
     """Workgroups of 4, 8 and 16 token rows: up to 1024 tokens, 2048, more."""
     g = torch.Generator(device="cuda").manual_seed(E + H)

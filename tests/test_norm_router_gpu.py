@@ -39,6 +39,19 @@ def _forward_norm(layer, x, residual, weight, out, next_weight=None, next_t=None
 @pytest.mark.parametrize("E", [4, 32, 33, 64, 128, 129])
 @pytest.mark.parametrize("with_residual", [False, True])
 def test_a_block_with_its_norm_equals_its_parts(ops, H, E, with_residual):
+    check_block_with_its_norm(ops, H, E, with_residual)
+
+
+# the router's two sets of k-steps per wave: up to 32 experts 1536 inputs each, up to 64 1024, up to 128 512 (beyond, one set of
+# 512); just below a set's end, at it and behind it, where the second one begins or the first is filled again
+@pytest.mark.parametrize("E,H", [(E, end + d) for E, ends in ((16, (1536, 3072)), (32, (1536, 3072)), (33, (1024, 2048)), (64, (1024, 2048)),
+                                                              (65, (512, 1024, 1536)), (128, (512, 1024, 1536)), (129, (512, 1024)))
+                                 for end in ends for d in (-64, 0, 64)])
+def test_a_block_with_its_norm_at_the_ends_of_the_routers_sets(ops, E, H):
+    check_block_with_its_norm(ops, H, E, True)
+
+
+def check_block_with_its_norm(ops, H, E, with_residual):
     g = torch.Generator(device="cuda").manual_seed(H + E)
     rnd = lambda *s, std=1.0: torch.randn(*s, generator=g, device="cuda") * std
     n = lambda *s, **k: rnd(*s, **k).bfloat16()
