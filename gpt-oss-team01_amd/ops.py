@@ -17,10 +17,16 @@ def _ptr(t):
     return t.data_ptr() if t is not None else None
 
 
+# (private names of torch: without them the public way)
+_raw_stream, _raw_device = (getattr(torch._C, name, None) for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+
+
 def _stream():
     """The current device's current stream as an address.  (torch.cuda.current_stream() makes a Stream object for it, 2.5 of the
     8.8 us that the host spent on a small attention call; now 5.9.)"""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if _raw_stream is None or _raw_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_raw_device())
 
 
 def _need_gpu():

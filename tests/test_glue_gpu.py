@@ -324,3 +324,17 @@ def test_rotation_within_the_attention_equals_that_in_front_of_it(ops, D, n_q, n
         got.append((out, kv))
     assert torch.equal(got[0][0].view(torch.int16), got[1][0].view(torch.int16))
     assert torch.equal(got[0][1].view(torch.int16), got[1][1].view(torch.int16)) and not torch.equal(filled, got[1][1])
+
+
+def test_calls_go_to_the_current_stream(ops, monkeypatch):
+    def streams():
+        torch.cuda.init()
+        other = torch.cuda.Stream()
+        with torch.cuda.stream(other):
+            inside = ops._stream(), other.cuda_stream
+        return [inside, (ops._stream(), torch.cuda.current_stream().cuda_stream)]
+    for have, want in streams():
+        assert have == want
+    monkeypatch.setattr(ops, "_raw_stream", None)      # a torch without it
+    for have, want in streams():
+        assert have == want
