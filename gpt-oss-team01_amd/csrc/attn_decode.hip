@@ -47,13 +47,6 @@ constexpr float NEG_BIG = -1.0e30f;
 // in fp32 is the same with them or without.)
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// The reference that a row's weights are taken against, from a block's largest score: raised only by more than RAISE_FROM, to
-// the next whole number, so that most blocks behind a row's first rescale nothing, and where one does the factor is a power of
-// two, without a rounding.
-constexpr float RAISE_FROM = 4.f;
-__device__ __forceinline__ bool raises_reference(float m, float top) { return top > m + RAISE_FROM; }
-__device__ __forceinline__ float raise_reference(float m, float top) { return raises_reference(m, top) ? ceilf(top) : m; }
-
 // What a row's sum, of maximum m, and its sink are weighed against: the larger of the two, but not so far above m that
 // exp2_hw has no weight left for the sum.  (A sink may lie more than 126 above every score, and bf16 still hold the output.)
 __device__ __forceinline__ float sink_reference(float m, float sink2) { return fminf(fmaxf(m, sink2), m + 100.f); }

@@ -193,6 +193,13 @@ __device__ __forceinline__ int kv_v_elem(int slot, int d, int D) {
   return KV_BLOCK * D + (((slot & 63) >> 5) * (D >> 4) + (d >> 4)) * 512 + lane * 8 + j;
 }
 
+// Attention: the reference that a row's weights are taken against, from a block's largest score: raised only by more than RAISE_FROM,
+// to the next whole number, so that most blocks behind a row's first rescale nothing, and where one does the factor is a power of
+// two, without a rounding.
+constexpr float RAISE_FROM = 4.f;
+__device__ __forceinline__ bool raises_reference(float m, float top) { return top > m + RAISE_FROM; }
+__device__ __forceinline__ float raise_reference(float m, float top) { return raises_reference(m, top) ? ceilf(top) : m; }
+
 // K rows of a block in LDS: piece j (16 bytes) of row r is at j ^ kv_swizzle(r).  LDS serves lanes 0-3, 12-15 and 20-27 of a fragment
 // read (16 rows, one piece per quarter) together, then 4-11, 16-19 and 28-31, and the upper half alike, and these hit 16
 // different 16-byte slots modulo 256 bytes.

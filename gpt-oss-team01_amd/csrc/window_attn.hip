@@ -8,7 +8,7 @@
 //   * A row that is alone in its sequence: one workgroup per (row, kv head, 16 query heads); its four
 //     waves take the window's blocks in turn and merge their states in LDS.
 //   * A stretch of rows: one workgroup per (piece of a stretch, kv head); every K/V block of the
-//     piece's range goes through LDS once and serves up to 128 queries (rows x heads), 32 per wave.
+//     piece's range goes through LDS once and serves up to 128 queries (rows x heads), 32 per wave, with heads of 64 values 16.
 #include "window_attn.hpp"
 
 namespace gptoss {
@@ -622,12 +622,10 @@ __global__ __launch_bounds__(256, DMAX > 128 ? 1 : 2) void window_tile_kernel(Wi
 }
 
 // Heads of 64 (padded): eight waves of 16 queries each, blocks straight into LDS, two buffers and one barrier per block.  The
-// vector units bound it, so a block that every row of a wave sees whole has no masks, sums are rescaled only for a score more
-// than WRAISE powers of two above the reference (then to a whole number: an exact factor), and four waves per SIMD, not two,
-// cover for each other.  Consecutive pieces, which read the same blocks, go to one XCD.  8 prompts of 1000 rows, 32 query over 8 kv
+// vector units bound it, so a block that every row of a wave sees whole has no masks, sums are rescaled only where a reference is
+// raised (raise_reference), and four waves per SIMD, not two, cover for each other.  Consecutive pieces, which read the same blocks, go to one XCD.  8 prompts of 1000 rows, 32 query over 8 kv
 // heads, window 512: 139 -> 93 us.
 constexpr int WTILE_WAVES = 8;
-constexpr float WRAISE = 4.f;
 
 template <bool NORM>
 __global__ __launch_bounds__(WTILE_WAVES * 64, 4) void window_tile64_kernel(WindowAttn a, const RowSeg *__restrict__ tiles, int n_tiles) {
@@ -705,9 +703,9 @@ __global__ __launch_bounds__(WTILE_WAVES * 64, 4) void window_tile64_kernel(Wind
       for (int tb = 0; tb < 4; tb++)
 #pragma unroll
         for (int e = 0; e < 4; e++) top = fmaxf(top, s[tb][e]);
-      if (__ballot(top > m + WRAISE) != 0) {
+      if (__ballot(raises_reference(m, top)) != 0) {
         top = max_over_quarters(top);
-        const float m_new = top > m + WRAISE ? ceilf(top) : m, fade = __builtin_amdgcn_exp2f(m - m_new);
+        const float m_new = raise_reference(m, top), fade = __builtin_amdgcn_exp2f(m - m_new);
         m = m_new;
         l *= fade;
 #pragma unroll
