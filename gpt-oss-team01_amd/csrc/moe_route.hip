@@ -942,8 +942,7 @@ static int launch_router(const bf16_t *t, const bf16_t *wr, const float *br, flo
   return (large ? launch_router_rows<NB, true> : launch_router_rows<NB, false>)(t, wr, br, logits, B, H, E, more...);
 }
 
-// logits (+ optional gating of the same tokens), in one launch unless many experts are shared out (with the gating of at
-// most 8 experts per token: logits alone come from one workgroup for all experts, but for many experts of few inputs)
+// logits (+ optional gating of the same tokens), in one launch unless many experts are shared out and gated as well
 int run_router(const void *t, const void *w_router, const float *b_router, float *logits, int B,
                int H, int E, int k, float *topk_w, int *topk_i, hipStream_t s, const RouterGroup *group, float *parts) {
   const RouterGroup grp = group ? *group : RouterGroup{};
@@ -989,8 +988,11 @@ int run_router(const void *t, const void *w_router, const float *b_router, float
     return GPTOSS_OK;
   }
   TraceScope ts(topk_w ? "router_gemm_topk" : "router_gemm", s);
-  // (256 experts of 64 inputs, 1 / 300 tokens 5.4 / 5.7 us in one workgroup, 3.6 / 3.7 shared out)
-  if (!topk_w && E > 128 && H <= 128 && B <= 512)
+  // Logits alone need no launch more for experts that are shared out: up to 1024 tokens that is the faster form at every size (us, one
+  // workgroup for all -> shared out: 80 experts of 96 inputs, 9 tokens 3.6 -> 2.3; 136 of 288, 513 tokens 6.6 -> 3.0; 64 of 2880, 1024
+  // tokens 7.5 -> 4.7; 256 of 2880, 1 / 1024 tokens 20.7 / 23.4 -> 4.2 / 11.7).  Beyond, each share reads the tokens again: 1025 tokens over
+  // 64 of 7168 13.4 -> 15.3, 2000 over 256 of 1024 10.5 -> 11.8.
+  if (!topk_w && E > 32 && B <= 1024)
     return launch_router<1>(tp, wp, b_router, logits, B, H, E, k, nullptr, nullptr, router_split_rows(B, E), nb, RouterGroup{}, s);
   if (nb <= 1) return launch_router<1>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);
   if (nb <= 2) return launch_router<2>(tp, wp, b_router, logits, B, H, E, k, topk_w, topk_i, rows_per_wg, 1, grp, s);

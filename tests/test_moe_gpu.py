@@ -108,8 +108,23 @@ def test_router_stages(ops, E, H):
         assert bool(((got.double() - want[:tokens]).abs() <= 2.0 ** -24 * (H / 8 + 8) * 8 * H ** 0.5).all()), tokens
 
 
+@pytest.mark.parametrize("E", [32, 33, 48, 65, 129, 255])   # blocks of 16 experts, whole and not, in one to four parts of a stage
+@pytest.mark.parametrize("H", [32, 96, 256, 288, 768, 2912])
+def test_router_logits_of_shared_experts_and_of_all_in_one_workgroup(ops, E, H):
+    """Without the gating, more than 32 experts are shared out up to 1024 tokens; 1025 have all experts in a workgroup.  Same bits."""
+    g = torch.Generator(device="cuda").manual_seed(E * H)
+    n = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    t, w, b = n(1025, H), n(E, H), n(E).float()
+    want = t.double() @ w.double().T + b.double()
+    whole = ops.router_gemm(t, w, b)
+    # as in test_router_rows_are_the_same_in_groups_of_any_size
+    assert bool(((whole.double() - want).abs() <= 2.0 ** -24 * (H / 8 + 8) * 8 * H ** 0.5).all())
+    for tokens in (1, 17, 511, 1024):
+        assert torch.equal(ops.router_gemm(t[:tokens].contiguous(), w, b), whole[:tokens]), tokens
+
+
 # the last experts' rows, and the last tokens' too, begin 4 GiB and more behind the first one
-@pytest.mark.parametrize("B,H,E", [(3, 8421536, 256), (4, 715827904, 4)])
+@pytest.mark.parametrize("B,H,E", [(3, 8421536, 256), (4, 715827904, 4), (3, 69273696, 32)])
 def test_router_matrices_of_more_than_four_gib(ops, B, H, E):
     g = torch.Generator(device="cuda").manual_seed(E)
     t = torch.zeros(B, H, dtype=torch.bfloat16, device="cuda")
