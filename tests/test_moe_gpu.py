@@ -1,4 +1,6 @@
 """GPU parity of the MoE path against the CPU oracle, through the C ABI."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -659,6 +661,27 @@ def test_blocks_that_leave_cus_idle_give_the_same_in_tiles_of_any_size(ops, E, k
     out = layer.forward(t).clone()
     for i in range(0, B, 16):
         assert torch.equal(layer.forward(t[i:i + 16].contiguous()), out[i:i + 16]), i
+
+
+def _longest_tile(layer, tokens):
+    """Rows of the longest row tile of the last forward call; its tile list is behind the inverse permutation."""
+    ptrs = [C.c_void_p() for _ in range(6)]
+    layer.L.gptoss_moe_workspace_views(layer.ws.data_ptr(), tokens, layer.E, layer.k, layer.H, layer.I, *[C.byref(p) for p in ptrs])
+    at = ptrs[5].value - layer.ws.data_ptr() + (tokens * layer.k * 4 + 255) // 256 * 256
+    tiles = layer.ws[at:at + 4 * (1 + 3 * (tokens * layer.k // 32 + layer.E))].view(torch.int32).tolist()
+    return max(tiles[3:1 + 3 * tiles[0]:3])
+
+
+# every token on all experts: 160-row tiles, or ones that are estimated to be ahead of them by 11 %
+@pytest.mark.parametrize("E,H,I,rows,longest", [(4, 2880, 2880, 150, 150), (4, 2880, 2880, 165, 128), (4, 2880, 2880, 180, 128),
+                                                (6, 2944, 1024, 345, 128), (2, 2816, 5056, 341, 128), (5, 2816, 4800, 70, 70)])
+def test_row_tiles_where_every_token_takes_every_expert(ops, E, H, I, rows, longest):
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    layer = ops.MoeLayer(n(E, H), n(E).float(), n(E, 2 * I, H, std=0.02), n(E, 2 * I).float(), n(E, H, I, std=0.02),
+                         n(E, H).float(), top_k=E, max_tokens=rows)
+    layer.forward(n(rows, H))
+    assert _longest_tile(layer, rows) == longest
 
 
 @pytest.mark.parametrize("k", [1, 2, 3, 5, 7, 8])
