@@ -103,28 +103,33 @@ static double expected_tiles(int k, int E, double avg, int rows_per_tile) {
 // The row tile of a bf16 block, given the one that holds an expert's rows: where tiles of that size are work for fewer than two
 // rounds of the CUs, the one that makes both products shortest by the estimates of gemm_dense.cpp.  Smaller tiles put more
 // CUs to work (an item of 160 rows is a CU's for 20 to 50 us), and where every token takes every expert, so that the tiles are known,
-// 256 rows may save a round.  It has to be ahead by 11 %, the estimates' error, or by a quarter, with a fifth more tiles than a
-// uniform routing makes, where the rows per expert are not known.  Blocks in us, before -> after: 4 of 4 experts, 2048 x 1024, 70 / 135 /
-// 240 rows each 61 / 73 / 75 -> 39 / 42 / 44, 2880 x 2880, 100 / 330 rows 102 / 192 -> 82 / 131; 4 of 16, 1024 x 512, 60 / 200 rows
-// 45 / 61 -> 35 / 51; two of 4, 4096 x 1536, 70 rows 93 -> 64.  Of 890 blocks of random sizes in which every token takes every expert none takes
-// more than 2 % longer; ahead by a tenth, 70 rows of 2816 x 4800 on five lose 3 %, and by 15 %, 21 blocks do without what they gain, four experts of 165 to
-// 190 rows, 2880 x 2880, 177 -> 105 us.  Of 4700 others, uniform, Zipf 0.6 and 1.1, none takes more than 1 % longer.  (Ahead by a tenth and by a quarter, without the fifth, 25 of them did, by up to a quarter: 6 experts of 106
-// rows of 2624 x 2688 have 12 tiles of 64, one round of the CUs, or 13, and two.)
+// 256 rows may save a round.  Blocks in us, before -> after: 4 of 4 experts, 2048 x 1024, 70 / 135 / 240 rows each 61 / 73 / 75 -> 39 / 42 /
+// 44, 2880 x 2880, 100 / 330 rows 102 / 192 -> 82 / 131; 4 of 16, 1024 x 512, 60 / 200 rows 45 / 61 -> 35 / 51; two of 4, 4096 x 1536, 70 rows
+// 93 -> 64.
+// Every token on every expert: it has to be ahead by 11 %, the estimates' error.  Of 890 blocks of random sizes none takes more than 2 %
+// longer; ahead by a tenth, 70 rows of 2816 x 4800 on five lose 3 %, and by 15 %, 21 blocks do without what they gain, four experts of 165 to 190
+// rows, 2880 x 2880, 177 -> 105 us.
+// Experts that are chosen: by a quarter, and by 12 % with a fifth more tiles than a uniform routing makes (or as many as there can be): 6
+// experts of 106 rows of 2624 x 2688 have 12 tiles of 64, one round of the CUs, or 13, and two.  Below 64 rows on average the default's tiles
+// are mostly of no more blocks than one of 64 rows, and cost no more: there by a quarter as well with those more.  188 blocks that the first
+// condition alone sends to other tiles, uniform, Zipf 0.6 and 1.1: half of them are sent there, 20 % faster on average, at worst 3 % slower; all of them,
+// 12 %, and up to 21 %.
 static int small_block_rows(int dflt, int B, int k, int E, int H, int I, bool tall) {
   const double avg = (double)B * k / E;
   if (dflt <= 64 || dflt == 256 || expected_tiles(k, E, avg, dflt) * gemm_col_tiles(2 * I) >= 512) return dflt;
   auto us = [&](int rpt, double more) {
     const int max_tiles = gptoss_moe_max_tiles(B, k, std::min(E, B * k), rpt);
-    const double tiles = expected_tiles(k, E, avg, rpt) * more;
+    const double expected = expected_tiles(k, E, avg, rpt), tiles = std::min(expected * more, std::max(expected, (double)max_tiles));
     return grouped_us(rpt, tiles, grouped_few(rpt, max_tiles, 2 * I), 2 * I, H) + grouped_us(rpt, tiles, grouped_few(rpt, max_tiles, H), H, I);
   };
   int best = dflt;
-  double least = (k == E ? 0.89 : 0.75) * us(dflt, 1.0);
+  const double dflt_us = us(dflt, 1.0), at_most = (avg >= 64 ? 0.88 : 0.75) * dflt_us;
+  double least = (k == E ? 0.89 : 0.75) * dflt_us;
   for (int rpt : {32, 64, 128, 160, 256}) {
     // (tiles of 32 rows read the weights again and again: not beyond two rounds of the few-row kernels)
     if ((rpt == 256 && (!tall || k != E)) || (rpt == 32 && expected_tiles(k, E, avg, 32) * (2 * I / 32) > 2560)) continue;
-    const double t = k == E || rpt == dflt ? us(rpt, 1.0) : std::max(us(rpt, 1.0), us(rpt, 1.2));
-    if (t < least) {
+    const double t = us(rpt, 1.0);
+    if (t < least && (k == E || us(rpt, 1.2) < at_most)) {
       least = t;
       best = rpt;
     }

@@ -684,6 +684,18 @@ def test_row_tiles_where_every_token_takes_every_expert(ops, E, H, I, rows, long
     assert _longest_tile(layer, rows) == longest
 
 
+# some experts per token: 64-row tiles where they are ahead with a fifth more of them too, or with as many as there can be (four experts)
+@pytest.mark.parametrize("E,k,H,I,tokens,tile", [(4, 2, 768, 2048, 845, 64), (12, 4, 512, 4672, 330, 64), (6, 2, 2624, 2688, 318, 160),
+                                                 (24, 1, 2176, 768, 1332, 128)])
+def test_row_tiles_where_experts_are_chosen(ops, E, k, H, I, tokens, tile):
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    n = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    layer = ops.MoeLayer(n(E, H), torch.zeros(E, device="cuda"), n(E, 2 * I, H, std=0.02), n(E, 2 * I).float(), n(E, H, I, std=0.02),
+                         n(E, H).float(), top_k=k, max_tokens=tokens)
+    layer.forward(n(tokens, H))
+    assert _longest_tile(layer, tokens) == min(tile, int(layer.routing_views()[3].diff().max()))
+
+
 @pytest.mark.parametrize("k", [1, 2, 3, 5, 7, 8])
 def test_tokens_of_pairs_in_a_prompt_pass(ops, k):
     """Every token on all k experts: the token of a pair is the pair's number over k."""
