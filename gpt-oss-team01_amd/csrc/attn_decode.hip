@@ -1011,8 +1011,8 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 // and walks the K/V blocks any of them needs ONCE: every block goes from global memory into LDS
 // (two buffers, one barrier per block) and the eight waves take their operands from there.  The
 // pair form reads a sequence's cache once per row pair, which is quadratic traffic for long
-// prompts; here it is read once per 16 rows.  What bounds it is power, and the vector
-// units next (68 % busy, the matrix cores 36 %): per 64 x 16 scores a wave issues about 150 of their instructions, a tenth of them
+// prompts; here it is read once per 16 rows.  What bounds it is the vector
+// units (67 % busy, the matrix cores 40 %, no bank conflicts) at the clock that power leaves them (2.07 GHz): per 64 x 16 scores a wave issues about 150 of their instructions, a tenth of them
 // exponentials.  Eight prompts of 1000 positions, 64 heads: 237 -> 211 us with the exponential, the maximum and the splitting of
 // weights in fewer instructions (exp2_hw, max_over_quarters, split_weights), -> 195 with the scale fused into the exponent's
 // difference (weight_exponents), one range check per masked slot and blocks straight into LDS, -> 181 with whole loads of q

@@ -438,7 +438,8 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64) void norm_router_kernel(
 // 16 rows by every four lanes in a row, and a CU reads 36 KB a us that way; of whole rows 64 bytes a cycle (all CUs at work on what
 // their L2s hold: 110 KB a us).  So the workgroup's 16 rows and its experts' come in stages of 512 bytes a row, one k-step for each
 // wave, straight into LDS, and are taken from there.  More than 64 experts come in parts of a stage, so that three
-// buffers have room; 32 experts' three buffers leave room for a second workgroup (6000 tokens 13.2 -> 12.5).  Operands straight into registers in operand order -> this, 2880 inputs (us): 32 experts, 27 / 1024 / 4096 tokens 8.3 /
+// buffers have room; 32 experts' three buffers leave room for a second workgroup (6000 tokens 13.2 -> 12.5).  Operands straight into registers in operand order -> this,
+// all experts in one workgroup, 2880 inputs (us): 32 experts, 27 / 1024 / 4096 tokens 8.3 /
 // 8.9 / 10.4 -> 5.0 / 5.6 / 6.3, 64 16.0 / 16.7 / 18.2 -> 7.1 / 7.9 / 8.4, 128 27.2 / 26.0 / 27.5 -> 12.3 / 13.0 / 14.3; 2048 inputs and four
 // 4.1 / 4.5 / 6.5 -> 3.9 / 3.9 / 6.1.  Same bits.
 template <int NB>
